@@ -108,6 +108,16 @@ def load() -> C.CDLL:
     return lib
 
 
+def load_host():
+    """The native host side of kernels.py (``_host.so``, csrc/host.cpp), which calls the same library."""
+    load()
+    try:
+        from . import _host
+    except ImportError as e:
+        raise RuntimeError("juliavision_amd/_host.so is missing or does not load: build it with `python -m juliavision_amd.build`") from e
+    return _host
+
+
 _initialised = False
 
 

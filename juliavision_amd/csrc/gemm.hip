@@ -2379,7 +2379,7 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split) {
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split) {
     TilePlan best = {4, 1, false};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
@@ -2397,6 +2397,19 @@ TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_sp
         }
     }
     return best;
+}
+
+// The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
+// thread keeps the last answers.  The key holds everything the estimate reads.
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split) {
+    struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
+    static thread_local Entry table[256] = {};
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0);
+    const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 40;
+    Entry &e = table[(h >> 32) & 255];
+    if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split)};
+    return e.plan;
 }
 
 // Workspace of a planned split: the planes, or the exchanged partials of the peer reduction (never less than the planes,

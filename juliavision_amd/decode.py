@@ -19,7 +19,7 @@ from typing import Callable, List, Optional
 import torch
 
 from . import _lib as L
-from .kernels import Ctx, DeclineError, Workspace, _strides_elbh, layernorm_, ln_matmul_, matmul_, matmul_heads_, relayout_weight, sdpa, sdpa_append
+from .kernels import Ctx, DeclineError, Workspace, _strides_elbh, layernorm_, ln_matmul_, matmul_, matmul_heads_, memo_view, relayout_weight, sdpa, sdpa_append
 
 
 # Fold the cache write into the self-attention launch where the one-launch kernel covers the shape.
@@ -43,6 +43,10 @@ class KVCache:
 
     def reset(self):
         self.length.zero_()
+
+    def layer(self, i: int):
+        """``(self_k, self_v, cross_k, cross_v)`` of layer ``i``, each ``(B, H, n, E)``."""
+        return tuple(memo_view(self, name, i, lambda t: t[i]) for name in ("self_k", "self_v", "cross_k", "cross_v"))
 
     def advance(self, ctx: Ctx, delta: int = 1):
         """length += delta on the device (``c.position += 1``, decode.jl:201).  The counter stops at ``max_target + 1``:
@@ -140,7 +144,9 @@ def decoder_layer_step(ctx: Ctx, W: DecoderLayerWeights, cache: KVCache, layer: 
     run once for this step.  ``x``, ``out``: ``(B, d_model)`` fp16."""
     B, d = x.shape
     H, E = cache.heads, cache.headdim
-    heads = lambda t: t.view(B, H, 1, E)
+    heads = lambda name: memo_view(buf, name, (B, H, E), lambda t: t.view(B, H, 1, E))
+    self_k, self_v, cross_k, cross_v = cache.layer(layer)
+
     def normed_linear(dst, w, src, g, b_, bias, epi="none"):
         # every workgroup of the folded form recomputes the row statistics: worth it for a few rows
         # (one launch less per norm), not for eight
@@ -152,19 +158,19 @@ def decoder_layer_step(ctx: Ctx, W: DecoderLayerWeights, cache: KVCache, layer: 
             matmul_(ctx, dst, w, buf.h, bias, epi=epi)
 
     normed_linear(buf.qkv, W.wqkv, x, W.ln1_g, W.ln1_b, W.bqkv)
-    q, k_new, v_new = (buf.qkv[:, i * d:(i + 1) * d].unflatten(1, (H, 1, E)) for i in range(3))
+    q, k_new, v_new = memo_view(buf, "qkv", (d, H, E), lambda t: tuple(t[:, i * d:(i + 1) * d].unflatten(1, (H, 1, E)) for i in range(3)))
     if FUSE_APPEND and E <= 64 and E % 8 == 0:
         # one launch: the new row is key length - 1 and goes into its cache slot on the way
-        sdpa_append(ctx, q, cache.self_k[layer], cache.self_v[layer], k_new, v_new, cache.length, out=heads(buf.att))
+        sdpa_append(ctx, q, self_k, self_v, k_new, v_new, cache.length, out=heads("att"))
     else:
         cache.append(ctx, layer, k_new, v_new)
         ctx.ws.reset()
-        sdpa(ctx, q, cache.self_k[layer], cache.self_v[layer], out=heads(buf.att), kv_len=cache.length)
+        sdpa(ctx, q, self_k, self_v, out=heads("att"), kv_len=cache.length)
     ctx.ws.reset()
     matmul_(ctx, buf.x1, W.wo, buf.att, W.bo, residual=x)
     normed_linear(buf.qc, W.wq_c, buf.x1, W.ln2_g, W.ln2_b, W.bq_c)
     ctx.ws.reset()
-    sdpa(ctx, heads(buf.qc), cache.cross_k[layer], cache.cross_v[layer], out=heads(buf.catt))
+    sdpa(ctx, heads("qc"), cross_k, cross_v, out=heads("catt"))
     ctx.ws.reset()
     matmul_(ctx, buf.x2, W.wo_c, buf.catt, W.bo_c, residual=buf.x1)
     normed_linear(buf.f, W.w1, buf.x2, W.ln3_g, W.ln3_b, W.b1, epi="gelu")

@@ -21,7 +21,7 @@ from typing import List, Optional
 import torch
 
 from .kernels import (Ctx, LnFoldedLinear, add_, convolution_tokens_, convsize, layernorm_, ln_matmul_, ln_matmul_folds, ln_matmul_pays,
-                      lnfold_matmul_, lnfold_prepare, matmul_, matmul_ln_, matmul_rowstats_, rowstats_, rowstats_new, sdpa)
+                      lnfold_matmul_, lnfold_prepare, matmul_, matmul_ln_, matmul_rowstats_, memo_view, rowstats_, rowstats_new, sdpa)
 
 
 @dataclass
@@ -49,6 +49,13 @@ class EncoderBuffers:
         e = lambda n: torch.empty((tokens, n), dtype=torch.float16, device=device)
         self.h, self.qkv, self.att, self.x1, self.f = e(d_model), e(3 * d_model), e(d_model), e(d_model), e(ffn)
 
+    def heads(self, d: int, heads: int):
+        """q, k, v -- column bands of the projection, heads column bands of those -- and the attention result as (B,H,L,E)
+        views, no copy."""
+        split = lambda t: t.unflatten(1, (heads, d // heads)).permute(1, 0, 2).unsqueeze(0)
+        q, k, v = memo_view(self, "qkv", (d, heads), lambda t: tuple(split(t[:, i * d:(i + 1) * d]) for i in range(3)))
+        return q, k, v, memo_view(self, "att", (d, heads), split)
+
 
 def encoder_layer(ctx: Ctx, W: EncoderLayerWeights, x: torch.Tensor, out: torch.Tensor, buf: EncoderBuffers, heads: int,
                   eps: float = 1e-5, act: str = "gelu", *, normed_in: bool = False, next_norm=None):
@@ -59,7 +66,6 @@ def encoder_layer(ctx: Ctx, W: EncoderLayerWeights, x: torch.Tensor, out: torch.
     encoder's final one) is written to ``dst`` by this layer's last GEMM (``matmul_ln_``).  ``normed_in``: the
     previous layer did that for this one, ``buf.h`` already holds ``LN1(x)``."""
     T, d = x.shape
-    E = d // heads
     # where the norm is cheaper as the prologue of the GEMM that reads it (today: at most 8 token rows), it is one
     fold1 = not normed_in and ln_matmul_folds(T, d, 3 * d) and ln_matmul_pays(T, d, 3 * d)
     fold2 = ln_matmul_folds(T, d, W.w1.shape[1]) and ln_matmul_pays(T, d, W.w1.shape[1])
@@ -70,10 +76,9 @@ def encoder_layer(ctx: Ctx, W: EncoderLayerWeights, x: torch.Tensor, out: torch.
         ln_matmul_(ctx, buf.qkv, W.wqkv, x, W.ln1_g, W.ln1_b, eps, W.bqkv)
     else:
         matmul_(ctx, buf.qkv, W.wqkv, buf.h, W.bqkv)
-    # q, k, v are column bands of the projection, heads are 64-wide column bands of those: (B,H,L,E) views, no copy
-    q, k, v = (buf.qkv[:, i * d:(i + 1) * d].unflatten(1, (heads, E)).permute(1, 0, 2).unsqueeze(0) for i in range(3))
+    q, k, v, att = buf.heads(d, heads)
     ctx.ws.reset()
-    sdpa(ctx, q, k, v, out=buf.att.unflatten(1, (heads, E)).permute(1, 0, 2).unsqueeze(0))
+    sdpa(ctx, q, k, v, out=att)
     ctx.ws.reset()
     matmul_(ctx, buf.x1, W.wo, buf.att, W.bo, residual=x)
     ctx.ws.reset()
@@ -126,12 +131,11 @@ def encoder_layer_folded(ctx: Ctx, W: EncoderLayerFolded, x: torch.Tensor, out: 
     addmm, add, layer_norm, addmm + gelu, addmm, add); held to the parity gate against it, not to the bits of
     ``encoder_layer``."""
     T, d = x.shape
-    E = d // heads
     ctx.ws.reset()
     lnfold_matmul_(ctx, buf.qkv, W.qkv, x, st.x, eps)
-    q, k, v = (buf.qkv[:, i * d:(i + 1) * d].unflatten(1, (heads, E)).permute(1, 0, 2).unsqueeze(0) for i in range(3))
+    q, k, v, att = buf.heads(d, heads)
     ctx.ws.reset()
-    sdpa(ctx, q, k, v, out=buf.att.unflatten(1, (heads, E)).permute(1, 0, 2).unsqueeze(0))
+    sdpa(ctx, q, k, v, out=att)
     ctx.ws.reset()
     matmul_rowstats_(ctx, buf.x1, st.x1, W.wo, buf.att, W.bo, residual=x)
     ctx.ws.reset()

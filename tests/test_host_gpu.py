@@ -1,0 +1,58 @@
+"""The native host side: an exported graph's recorded calls issued again on other inputs, and the calls it leaves to Python."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+class _Net(nn.Module):
+    def __init__(self, d, heads):
+        super().__init__()
+        self.heads, self.norm = heads, nn.LayerNorm(d)
+        self.q, self.k, self.v, self.o, self.fc = (nn.Linear(d, d) for _ in range(5))
+
+    def forward(self, x):
+        B, T, D = x.shape
+        split = lambda t: t.view(B, T, self.heads, D // self.heads).transpose(1, 2)
+        y = self.norm(x)
+        a = F.scaled_dot_product_attention(split(self.q(y)), split(self.k(y)), split(self.v(y)))
+        return x + self.o(a.transpose(1, 2).reshape(B, T, D)), F.gelu(self.fc(x))
+
+
+@pytest.mark.parametrize("T", [5, 130])
+def test_recorded_calls_follow_their_inputs(T):
+    import juliavision_amd as jv
+    from juliavision_amd import graph as G
+    torch.manual_seed(T)
+    m = _Net(128, 2).eval().half()
+    g = G.optimize(G.Graph.load(G.convert(torch.export.export(m, (torch.randn(1, T, 128).half(),)), "net")))
+    run = G.Executor(g, m.state_dict(), jv.Ctx("cuda"))
+    xs = [torch.randn(1, T, 128, device="cuda").half() for _ in range(5)]
+    shifted = torch.randn(8 + T * 128, device="cuda").half()[8:].view(1, T, 128)      # another alignment: not the calls recorded for xs
+    for i, x in enumerate(xs[:3] + [shifted, shifted] + xs[3:]):
+        got = [t.float().clone() for t in run(x)]
+        if i == 4:
+            run.ctx.ws.scratch(4 * run.ctx.ws.buf.numel())                                 # the workspace moves: recorded addresses are stale
+        fresh = G.Executor(g, m.state_dict(), jv.Ctx("cuda"))(x)
+        for a, b in zip(got, fresh):
+            assert torch.equal(a, b.float()), f"run {i}"
+    assert run._calls is not None
+
+
+def test_what_the_native_side_leaves_is_still_refused_by_name():
+    import juliavision_amd as jv
+    ctx = jv.Ctx("cuda")
+    h = lambda *s: torch.zeros(s, dtype=torch.float16, device="cuda")
+    with pytest.raises(jv.DeclineError, match="bias"):
+        jv.matmul_(ctx, h(16, 64), h(64, 64), h(16, 64), torch.zeros(64, device="cuda"))
+    with pytest.raises(jv.DeclineError, match="extent"):
+        jv.matmul_(ctx, h(16, 64), h(64, 64), h(16, 32))
+    with pytest.raises(jv.DeclineError, match="residual"):
+        jv.matmul_(ctx, h(16, 64), h(64, 64), h(16, 64), residual=h(16, 32))
+    with pytest.raises(jv.DeclineError, match="nocoopmat"):
+        jv.matmul_(jv.Ctx("cuda", dev=jv.MI355X._replace(coopmat=False)), h(16, 64), h(64, 64), h(16, 64))
+    with pytest.raises(jv.DeclineError, match="extent"):
+        jv.sdpa(ctx, h(1, 2, 8, 64), h(1, 2, 9, 64), h(1, 2, 8, 64), out=h(1, 2, 8, 64))
+    torch.cuda.synchronize()
