@@ -1,14 +1,13 @@
 // fp16 GEMM for gfx950: MFMA 32x32x16 f16 with fp32 accumulation, LDS
 // double-buffered operand tiles, 128-bit global loads, fused bias / activation /
-// residual store; a split-K bandwidth kernel for decode-sized T; a scalar
-// kernel for operands the tiled kernels cannot address.
+// residual store; a split-K bandwidth kernel for decode-sized T.  The four-wave kernel, the decode-sized kernels, the plans and
+// the C ABI are here; gemm_pipe.hip has the small and gathered tiles, gemm_any.hip what neither can address.
 //
 // Internal problem statement (row-major):  Y[M x N] = A[M x K] . B  (+ bias)
 //   A is K-contiguous.  B is either N-contiguous [K][N] (B_KN) or K-contiguous
 //   [N][K].  For a linear layer M = tokens, N = features, A = X, B = W.
-#include "common.hpp"
+#include "gemm_common.hpp"
 #include "sk_exchange.hpp"
-#include <type_traits>
 #include <atomic>
 
 // Arrival flags of the split-K peer reduction (gemm_w4_kernel, SK): SK_BANKS banks of SK_FLAGS words, and as many
@@ -27,972 +26,6 @@ static __device__ unsigned device_status_words[4];
 static __device__ __align__(256) unsigned char scratch[MI_NOALLOC_SCRATCH_BYTES];
 
 namespace {
-
-struct GemmArgs {
-    void *Y;
-    const half_t *A, *B, *bias, *residual;
-    int M, N, K;
-    int NB;                 // columns addressable in B (>= N; a multiple of 8 for the [K][N] layout)
-    long ldY, ldA, ldB;
-    long sY, sA, sB, sBias; // batch strides (elements)
-    int bias_mode, epi, out_f32;
-    int tiles_m, tiles_n, group_m;
-    int vec_store;          // Y (and residual) rows allow 16-byte accesses
-    ConvGather cv;          // cv.xp != nullptr: B is the im2col matrix of a convolution, gathered on the fly
-    NhwcGather ag;          // ag.x != nullptr: A is the patch matrix of a channels-last convolution, gathered on the fly
-    // Decode-sized kernels only: the rows of A are layer-normalised over K on their way into LDS
-    // (ln_on; gamma, beta may be null), exactly as layernorm_vec_kernel would have written them.
-    const half_t *ln_gamma, *ln_beta;
-    float ln_eps;
-    int ln_on;
-    // Output side: when lnout is set, the rows of Y are also layer-normalised over N into lnout (dense rows of N
-    // halves), as mi_layernorm_f16 on Y would write them (the next block's first norm riding in this GEMM's store).
-    half_t *lnout;
-    const half_t *lnout_gamma, *lnout_beta;
-    float lnout_eps;
-    // Tiled kernels and the split-K plane sums: > 0 clamps the fp16 result to [-clamp, clamp] after the residual add,
-    // as a separate aten::clamp on Y would (the overflow guard of exported fp16 encoder layers).
-    float clamp;
-    // Measurement only (mi_set_clock_probe): workgroup 0 of a four-wave launch stores {shader clock, 100 MHz clock}
-    // here when it starts and again after its last store.  Null in ordinary use.
-    unsigned long long *clk;
-    // Measurement only (mi_set_phase_probe): every matrix wave of the first phase_wgs workgroups of a four-wave launch
-    // stores the shader clocks it spent {before its K loop, in it, issuing its store, waiting for the store to drain}.
-    unsigned long long *phase;
-    int phase_wgs;
-    // Split-K with the partial tiles exchanged between the workgroups of a tile instead of written as planes
-    // (gemm_w4_kernel, SK instance): sk_S = 2 workgroups per tile, tiles dealt sk_tpx per XCD; partials in sk_part,
-    // per-wave arrival flags in sk_flags (they carry sk_epoch; the last reader of a flag clears it).
-    int sk_S, sk_tpx;
-    float *sk_part;
-    unsigned *sk_flags;
-    unsigned sk_epoch;
-    // Layer norm folded away (mi_lnfold_gemm_f16): A holds the raw rows, B carries gamma, and the store turns an
-    // accumulator into r (acc - mu colsum[n]) + biasp[n], with the row's (mu, r) combined from lnf_stats.
-    const float *lnf_stats;           // [lnf_nseg][M][2]: (sum, squares about its own mean) of each 32-column segment of a row
-    const float *lnf_colsum, *lnf_biasp;      // fp32[N], plane stride lnf_svec
-    long lnf_svec;
-    int lnf_nseg;
-    float lnf_eps;
-    // Row statistics of the result for a later folded norm: stats_out[n / 32][m] = (sum, squares about the mean) of the
-    // final fp16 values Y[m][32 (n / 32) .. + 32); stats_nseg segments per row.
-    float *stats_out;
-    int stats_nseg;
-    int sk_spin;                      // polls before a wave gives up on its partners
-    unsigned sk_pub_xor, sk_xcc_xor;  // zero in ordinary use: mi_test_exchange_faults makes the waits fail from the host side
-    unsigned *status;                 // the device's sticky status word
-};
-
-// ------------------------------------------------------------------------------------------
-// Staging of a K-contiguous operand tile ROWS x BK: each thread moves 16-byte
-// chunks global -> registers -> LDS rows of BK+8 halves (the 16-byte pad makes
-// the 32 rows an MFMA operand read touches fall in distinct bank groups).
-template <int ROWS, int BK, int NT>
-struct KcStage {
-    static constexpr int CPR = BK / 8;
-    static constexpr int CHUNKS = ROWS * CPR;
-    static constexpr int PER = (CHUNKS + NT - 1) / NT;
-    static constexpr int LD = BK + 8;
-    u32x4 r[PER];
-
-    __device__ __forceinline__ void load(const half_t *base, long ld, int row0, int nrows, int k0, int K, int tid) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int c = tid + i * NT;
-            int row = c / CPR, kc = c % CPR;
-            int gr = min(row0 + row, nrows - 1);
-            int gk = k0 + kc * 8;
-            u32x4 z = {0u, 0u, 0u, 0u};
-            if (CHUNKS % NT == 0 || c < CHUNKS) r[i] = gk < K ? ldg16(base + (long)gr * ld + gk) : z;
-        }
-    }
-    __device__ __forceinline__ void store(half_t *lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int c = tid + i * NT;
-            int row = c / CPR, kc = c % CPR;
-            if (CHUNKS % NT == 0 || c < CHUNKS) *reinterpret_cast<u32x4 *>(lds + row * LD + kc * 8) = r[i];
-        }
-    }
-};
-
-// Staging of an N-contiguous operand tile [BK][COLS] into the same K-contiguous
-// LDS rows: a thread loads an 8(k) x 8(n) block with eight 16-byte row loads,
-// transposes it in registers (v_perm_b32) and writes eight 16-byte LDS rows.
-template <int COLS, int BK, int NT>
-struct KnStage {
-    static constexpr int KB = BK / 8;
-    static constexpr int BLOCKS = KB * (COLS / 8);
-    static constexpr int PER = (BLOCKS + NT - 1) / NT;
-    static constexpr int LD = BK + 8;
-    u32x4 r[PER][8];
-
-    __device__ __forceinline__ void load(const half_t *base, long ld, int col0, int ncols, int k0, int K, int tid) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int blk = tid + i * NT;
-            int kb = blk % KB, nb = blk / KB;
-            int gn = min(col0 + nb * 8, ncols - 8);
-            if (BLOCKS % NT == 0 || blk < BLOCKS) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    int gk = k0 + kb * 8 + j;
-                    u32x4 z = {0u, 0u, 0u, 0u};
-                    r[i][j] = gk < K ? ldg16(base + (long)gk * ld + gn) : z;
-                }
-            }
-        }
-    }
-    __device__ __forceinline__ void store(half_t *lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int blk = tid + i * NT;
-            int kb = blk % KB, nb = blk / KB;
-            if (BLOCKS % NT == 0 || blk < BLOCKS) {
-#pragma unroll
-                for (int w = 0; w < 4; w++) {   // dword w of each row holds columns 2w, 2w+1
-                    u32x4 lo, hi;
-                    lo.x = pack_lo(r[i][0][w], r[i][1][w]); hi.x = pack_hi(r[i][0][w], r[i][1][w]);
-                    lo.y = pack_lo(r[i][2][w], r[i][3][w]); hi.y = pack_hi(r[i][2][w], r[i][3][w]);
-                    lo.z = pack_lo(r[i][4][w], r[i][5][w]); hi.z = pack_hi(r[i][4][w], r[i][5][w]);
-                    lo.w = pack_lo(r[i][6][w], r[i][7][w]); hi.w = pack_hi(r[i][6][w], r[i][7][w]);
-                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w) * LD + kb * 8) = lo;
-                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w + 1) * LD + kb * 8) = hi;
-                }
-            }
-        }
-    }
-};
-
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<int, N - 1>{});
-    }
-}
-
-// Workgroup id -> output tile.  The hardware deals consecutive workgroups
-// round-robin over the 8 XCDs, each with its own L2; this hands every XCD one
-// contiguous run of the tile order, and the tile order walks GROUP_M row tiles
-// per column tile so a run reuses a small set of A and B panels.
-__device__ __forceinline__ void tile_of(int pid, int nwg, int tiles_m, int tiles_n, int group_m, int &tm, int &tn) {
-    int xcd = pid & 7, idx = pid >> 3;
-    int full = nwg >> 3, rem = nwg & 7;
-    int logical = xcd * full + min(xcd, rem) + idx;
-    int width = group_m * tiles_n;
-    int g = logical / width, in = logical - g * width;
-    int first = g * group_m;
-    int gsz = min(tiles_m - first, group_m);
-    tm = first + in % gsz;
-    tn = in / gsz;
-}
-
-// What the store of a folded norm needs, fetched while the first operand tiles are on their way and parked in `slot`
-// (LDS past everything else the kernel keeps there: BM float2 (r, r mu), then BN column sums, then BN biases).
-//
-// A row's mean and reciprocal standard deviation over its K elements come from the per-segment statistics a producer
-// left (stats[seg][row] = (sum, squares about the segment's own mean)).  LPR lanes share a row, each with every LPR-th
-// segment, many loads in flight at a time (a lane that walked all segments one dependent load after the other held
-// the whole workgroup at its first barrier for 10 us).  One pass: the squares between the segments are taken about the
-// first segment's mean, which lies within a segment mean's spread of the row mean, so the final subtraction cancels
-// nothing that matters -- sum(x^2) - n mean^2 about zero would.  r = 1 / sqrt(var + eps), rmu = r * mean.
-// The caller synchronises the workgroup before anybody reads the slot.
-template <int BM, int BN, int NT, typename Args>
-__device__ __forceinline__ void lnf_stage(const Args &p, float2v *slot, int m0, int n0, long bz, int tid) {
-    if (!p.lnf_stats) return;
-    constexpr int LPR = NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1;
-    static_assert(NT >= BM && (BM * LPR) % 64 == 0, "whole waves work on the rows");
-    if (tid < BM * LPR) {
-        const int row = tid / LPR, q = tid % LPR;
-        const float2v *seg = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + row, p.M - 1);
-        const float ref = seg[0][0] / (float)min(32, p.K);
-        float total = 0.0f, within = 0.0f, between = 0.0f;
-        // U loads in flight per lane: all of a row's segments in one trip to memory for K <= 1536 (2048 with four lanes a
-        // row) -- a trip costs 1 to 2 us here (the statistics were written by another kernel, on other XCDs), and the
-        // first operand tiles, requested before this, take about as long, so one trip is hidden and every further one
-        // is not (two and three batches of eight measured +3.3 and +4.3 us per launch)
-        constexpr int U = LPR == 4 ? 16 : 24;
-        for (int s0 = q; s0 < p.lnf_nseg; s0 += U * LPR) {
-            float2v v[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int sg = s0 + u * LPR;
-                const float2v z = {0.0f, 0.0f};
-                v[u] = sg < p.lnf_nseg ? seg[(long)sg * p.M] : z;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int sg = s0 + u * LPR;
-                if (sg < p.lnf_nseg) {
-                    const int left = p.K - 32 * sg;
-                    const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
-                    const float d = fmaf(v[u][0], inv, -ref);
-                    total += v[u][0];
-                    within += v[u][1];
-                    between = fmaf(cnt * d, d, between);
-                }
-            }
-        }
-        if constexpr (LPR >= 2) { total += lane_xor<1>(total); within += lane_xor<1>(within); between += lane_xor<1>(between); }
-        if constexpr (LPR >= 4) { total += lane_xor<2>(total); within += lane_xor<2>(within); between += lane_xor<2>(between); }
-        if (q == 0) {
-            const float mu = total / (float)p.K, dm = mu - ref;
-            const float m2 = within + fmaxf(between - (float)p.K * dm * dm, 0.0f);
-            const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
-            const float2v o = {r, r * mu};
-            slot[row] = o;
-        }
-    }
-    // the tile's columns of colsum and biasp
-    for (int t = tid; t < BN / 2; t += NT) {
-        const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
-        const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
-        float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
-        else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
-        *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = v;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
-
-// ------------------------------------------------------------------------------------------
-// Accumulator tile -> memory, shared by the tiled kernels.
-// acc[i][j][r]: n = n0 + wn*WTN + 32 i + 8 (r/4) + 4 (lane/32) + r%4,  m = m0 + wm*WTM + 32 j + lane%32.
-// Each wave stages one 32 x WTN sub-tile at a time in its own LDS region (bias
-// joined in fp32, one rounding), then reads it back row-wise so that the
-// activation, the residual add and the global stores run on 16-byte vectors
-// that are contiguous along the output row.  The caller has synchronised the
-// workgroup after its last read of the operand tiles.
-// The column bias of a wave's sub-tile, in the accumulator's order: cb[i][g] covers
-// n = n0 + wn*WTN + 32 i + 8 g + 4 (lane/32) .. +3.  Fetched by the kernels ahead of their last
-// k-step so that the epilogue does not start with a trip to memory.
-template <int TN, int WTN>
-__device__ __forceinline__ void load_col_bias(const GemmArgs &p, half4v (&cb)[TN][4], int n0, int wn, int lane, long bz) {
-    const half4v z = {(half_t)0.0f, (half_t)0.0f, (half_t)0.0f, (half_t)0.0f};
-    const bool on = p.bias_mode == MI_BIAS_COL;
-    const half_t *bias = on ? p.bias + bz * p.sBias : nullptr;
-    const bool vec = (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
-#pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int n = n0 + wn * WTN + 32 * i + 8 * g + 4 * (lane >> 5);
-            cb[i][g] = z;
-            if (on) {
-                if (n + 3 < p.N && vec) cb[i][g] = *reinterpret_cast<const half4v *>(bias + n);
-                else for (int e = 0; e < 4; e++) if (n + e < p.N) cb[i][g][e] = bias[n + e];
-            }
-        }
-}
-
-// What the store of a folded layer norm carries (by value, so that it stays in registers): (r, r mu) of the lane's rows
-// m0 + wm WTM + 32 j + lane % 32, and the LDS copy of the tile's colsum (bn floats) followed by its biasp.
-template <int TM>
-struct LnFold {
-    bool on = false;
-    float r[TM] = {}, rmu[TM] = {};
-    const float *col = nullptr;
-    int bn = 0;
-};
-template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
-__device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                               int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
-    const int frow = lane & 31;
-    const half_t *bias = p.bias ? p.bias + bz * p.sBias : nullptr;
-    constexpr int SLD_H = WTN + 8;                 // halves per staged row (fp16 output)
-    constexpr int SLD_F = WTN + 4;                 // floats per staged row (fp32 output)
-    constexpr int STAGE_BYTES = 32 * SLD_F * 4;
-    static_assert(STAGE_BYTES * NWAVES <= LDS_BYTES, "epilogue staging exceeds the operand LDS");
-    char *stage = smem + wave * STAGE_BYTES;
-    const int hl = lane >> 5;
-    // Row biases for all of the wave's rows before the first store (store_tile_simple says why).
-    float brow_j[TM];
-#pragma unroll
-    for (int j = 0; j < TM; j++) {
-        const int m = m0 + wm * WTM + 32 * j + frow;
-        brow_j[j] = (p.bias_mode == MI_BIAS_ROW && m < p.M) ? (float)bias[m] : 0.0f;
-    }
-    static_for<TM>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        const int mrow = m0 + wm * WTM + 32 * j;
-        const float brow = brow_j[j];
-#pragma unroll
-        for (int i = 0; i < TN; i++) {
-            // folded layer norm: this lane's columns of colsum and biasp from their LDS copy, a 32-column group at a time
-            float4v lc4[4], lb4[4];
-            if (ln.on) {
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int nl = 32 * i + 8 * g + 4 * hl;
-                    lc4[g] = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl);
-                    lb4[g] = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl);
-                }
-            }
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int nl = 32 * i + 8 * g + 4 * hl;
-                const int n = n0 + wn * WTN + nl;
-                float v[4];
-                if (ln.on) {      // uniform: r (acc - mu colsum) + biasp
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = fmaf(acc[i][j][4 * g + e], ln.r[j], fmaf(-ln.rmu[j], lc4[g][e], lb4[g][e]));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e] + brow + (float)cb[i][g][e];
-                }
-                if (p.out_f32) {
-                    float4v o = {v[0], v[1], v[2], v[3]};
-                    *reinterpret_cast<float4v *>(reinterpret_cast<float *>(stage) + frow * SLD_F + nl) = o;
-                } else {
-                    half4v o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-                    *reinterpret_cast<half4v *>(reinterpret_cast<half_t *>(stage) + frow * SLD_H + nl) = o;
-                }
-            }
-        }
-        // A wave reads back only what it staged itself, and its LDS operations complete in order:
-        // no workgroup barrier, only a stop for the compiler.
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (p.out_f32) {
-            constexpr int CPR = WTN / 4;
-            for (int c = lane; c < 32 * CPR; c += 64) {
-                const int row = c / CPR, ch = c % CPR;
-                const int m = mrow + row, n = n0 + wn * WTN + ch * 4;
-                if (m < p.M && n < p.N) {
-                    float4v x = *reinterpret_cast<const float4v *>(reinterpret_cast<const float *>(stage) + row * SLD_F + ch * 4);
-                    float *yp = reinterpret_cast<float *>(p.Y) + bz * p.sY + (long)m * p.ldY + n;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) x[e] = apply_epi_c<EPI>(x[e]);
-                    if (p.vec_store && n + 3 < p.N) *reinterpret_cast<float4v *>(yp) = x;
-                    else for (int e = 0; e < 4; e++) if (n + e < p.N) yp[e] = x[e];
-                }
-            }
-        } else {
-            constexpr int CPR = WTN / 8;
-            static_assert((32 * CPR) % 64 == 0 && CPR % 4 == 0, "whole waves walk the staged tile; four lanes hold a 32-column segment");
-            for (int c = lane; c < 32 * CPR; c += 64) {
-                const int row = c / CPR, ch = c % CPR;
-                const int m = mrow + row, n = n0 + wn * WTN + ch * 8;
-                half8v x = {};
-                if (m < p.M && n < p.N) {
-                    x = *reinterpret_cast<const half8v *>(reinterpret_cast<const half_t *>(stage) + row * SLD_H + ch * 8);
-                    const long off = bz * p.sY + (long)m * p.ldY + n;
-                    half_t *yp = reinterpret_cast<half_t *>(p.Y) + off;
-                    if constexpr (EPI != MI_EPI_NONE) {
-#pragma unroll
-                        for (int e = 0; e < 8; e++) x[e] = (half_t)apply_epi_c<EPI>((float)x[e]);
-                    }
-                    if (p.vec_store && n + 7 < p.N) {
-                        if (p.residual) {
-                            half8v rv = as_half8(ldg16(p.residual + off));
-#pragma unroll
-                            for (int e = 0; e < 8; e++) x[e] = (half_t)((float)x[e] + (float)rv[e]);
-                        }
-                        if (p.clamp > 0.0f) {
-#pragma unroll
-                            for (int e = 0; e < 8; e++) x[e] = (half_t)fminf(fmaxf((float)x[e], -p.clamp), p.clamp);
-                        }
-                        *reinterpret_cast<half8v *>(yp) = x;
-                    } else {
-                        for (int e = 0; e < 8; e++) {
-                            if (n + e < p.N) {
-                                half_t o = x[e];
-                                if (p.residual) o = (half_t)((float)o + (float)p.residual[off + e]);
-                                if (p.clamp > 0.0f) o = (half_t)fminf(fmaxf((float)o, -p.clamp), p.clamp);
-                                yp[e] = o;
-                            }
-                        }
-                    }
-                }
-                if (p.stats_out) {      // uniform; the launcher admits it with 16-byte stores and N % 8 == 0 only
-                    // the four lanes of a quad hold the 32 columns of one segment of one row (chunks that lie past N
-                    // or below M count nothing): sum, then squares about the segment's own mean, both over the quad
-                    const bool have = m < p.M && n < p.N;
-                    float cnt = have ? 8.0f : 0.0f, sum = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) sum += have ? (float)x[e] : 0.0f;
-                    sum += lane_xor<1>(sum); sum += lane_xor<2>(sum);
-                    cnt += lane_xor<1>(cnt); cnt += lane_xor<2>(cnt);
-                    const float mean = sum / fmaxf(cnt, 1.0f);
-                    float sq = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) { const float d = (float)x[e] - mean; sq = have ? fmaf(d, d, sq) : sq; }
-                    sq += lane_xor<1>(sq); sq += lane_xor<2>(sq);
-                    if (have && (ch & 3) == 0) {
-                        const float2v o = {sum, sq};
-                        *reinterpret_cast<float2v *>(p.stats_out + ((long)(n / 32) * p.M + m) * 2) = o;
-                    }
-                }
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    });
-}
-
-// Block j (32 rows) of a wave's accumulators -> its staging area `dst` (32 rows of WTN + 8 halves), rounded to fp16 once
-// with the column bias -- or the folded layer norm's r (acc - mu colsum) + biasp -- joined in fp32.
-template <int j, int TM, int TN, int WTN>
-__device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], const LnFold<TM> &ln, int wn, char *dst, int lane) {
-    constexpr int SLD_H = WTN + 8;
-    const int frow = lane & 31, hl = lane >> 5;
-    half_t *st = reinterpret_cast<half_t *>(dst) + frow * SLD_H + 4 * hl;
-#pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int nl = 32 * i + 8 * g;
-            float v[4];
-            if (ln.on) {      // uniform; the tile's colsum and biasp from their LDS copy
-                const float4v lc = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl + 4 * hl);
-                const float4v lb = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl + 4 * hl);
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = fmaf(acc[i][j][4 * g + e], ln.r[j], fmaf(-ln.rmu[j], lc[e], lb[e]));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e] + (float)cb[i][g][e];
-            }
-            const half4v o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-            *reinterpret_cast<half4v *>(st + nl) = o;
-        }
-}
-
-// The common store: fp16 output in whole 16-byte chunks, column bias (or a folded layer norm), optional activation,
-// residual, clamp and row statistics; no row bias, no fp32 output, no ragged N.
-//
-// Loads and stores of a wave share one counter and complete in order, so a wait for a load -- wherever the compiler
-// places it -- is also a wait for every store issued before that load to be acknowledged: a trip of two microseconds
-// under the burst of all workgroups' stores.  The general store above pays it once per 32-row block of a wave's tile
-// and once per residual chunk (8 000 clocks of a 44 000-clock launch at 1500 x 1280 -> 5120).  Here nothing is fetched
-// behind a store that anybody then waits for: the caller's column bias is pinned in registers ahead of the first store,
-// and the residual chunks of block j + 1 are requested before block j's stores go out.
-// Same arithmetic as the general store (bias joined in fp32, one rounding, activation on the rounded value, residual,
-// clamp), so the two give the same bits.  Two staging areas a wave: block j + 1 is staged while block j's chunks are on
-// their way back from the LDS (a wave's LDS operations complete in order: no wait between staging a block and reading it).
-template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
-__device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                                  int wave, int lane, long bz, const LnFold<TM> ln) {
-    constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;      // halves per staged row; one staging area
-    constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI;     // 16-byte chunks per row; rows a wave covers at a time; chunks per lane and block
-    static_assert(2 * BUF_BYTES * NWAVES <= LDS_BYTES && 64 % CPR == 0 && CPR % 4 == 0, "two staging areas a wave; four lanes hold a 32-column segment");
-    char *const buf = smem + wave * 2 * BUF_BYTES;
-    const int frow = lane & 31, hl = lane >> 5;
-    const int ch = lane % CPR, r0 = lane / CPR;                      // this lane's chunks of a block: rows r0 + RPI t, columns 8 ch ..
-    const int mw = m0 + wm * WTM, n = n0 + wn * WTN + ch * 8;
-    const bool col_ok = n < p.N;                                     // N % 8 == 0: a chunk that starts below N ends below it
-    const long off0 = bz * p.sY + (long)(mw + r0) * p.ldY + n;
-    half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + off0;
-    const half_t *const rbase = p.residual ? p.residual + off0 : nullptr;
-#pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) asm volatile("" ::"v"(cb[i][g]));
-    auto stage = [&](auto J) {
-        constexpr int j = decltype(J)::value;
-        stage_block<j, TM, TN, WTN>(acc, cb, ln, wn, buf + (j & 1) * BUF_BYTES, lane);
-    };
-    half8v res[2][NIT];
-    auto fetch_residual = [&](auto J) {
-        constexpr int j = decltype(J)::value;
-#pragma unroll
-        for (int t = 0; t < NIT; t++) {
-            res[j & 1][t] = half8v{};
-            if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) res[j & 1][t] = as_half8(ldg16(rbase + (long)(32 * j + t * RPI) * p.ldY));
-        }
-    };
-    if (rbase) fetch_residual(std::integral_constant<int, 0>{});
-    stage(std::integral_constant<int, 0>{});
-    static_for<TM>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        const half_t *rd = reinterpret_cast<const half_t *>(buf + (j & 1) * BUF_BYTES) + r0 * SLD_H + ch * 8;
-        half8v x[NIT];
-#pragma unroll
-        for (int t = 0; t < NIT; t++) x[t] = *reinterpret_cast<const half8v *>(rd + t * RPI * SLD_H);
-        if constexpr (j + 1 < TM) {
-            stage(std::integral_constant<int, j + 1>{});
-            if (rbase) fetch_residual(std::integral_constant<int, j + 1>{});
-        }
-#pragma unroll
-        for (int t = 0; t < NIT; t++) {
-            const int m = mw + 32 * j + r0 + t * RPI;
-            const bool have = col_ok && m < p.M;
-            if constexpr (EPI != MI_EPI_NONE) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[t][e] = (half_t)apply_epi_c<EPI>((float)x[t][e]);
-            }
-            if (rbase) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[t][e] = (half_t)((float)x[t][e] + (float)res[j & 1][t][e]);
-            }
-            if (p.clamp > 0.0f) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[t][e] = (half_t)fminf(fmaxf((float)x[t][e], -p.clamp), p.clamp);
-            }
-            if (have) *reinterpret_cast<half8v *>(ybase + (long)(32 * j + t * RPI) * p.ldY) = x[t];
-            if (p.stats_out) {      // uniform
-                // the four lanes of a quad hold the 32 columns of one segment of one row (chunks that lie past N or
-                // below M count nothing): sum, then squares about the segment's own mean, both over the quad
-                float cnt = have ? 8.0f : 0.0f, sum = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += have ? (float)x[t][e] : 0.0f;
-                sum += lane_xor<1>(sum); sum += lane_xor<2>(sum);
-                cnt += lane_xor<1>(cnt); cnt += lane_xor<2>(cnt);
-                const float mean = sum / fmaxf(cnt, 1.0f);
-                float sq = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; e++) { const float d = (float)x[t][e] - mean; sq = have ? fmaf(d, d, sq) : sq; }
-                sq += lane_xor<1>(sq); sq += lane_xor<2>(sq);
-                if (have && (ch & 3) == 0) {
-                    const float2v o = {sum, sq};
-                    *reinterpret_cast<float2v *>(p.stats_out + ((long)(n / 32) * p.M + m) * 2) = o;
-                }
-            }
-        }
-    });
-}
-
-// The four-wave kernel's store, shared between a matrix wave and the helper wave on its SIMD.  One wave issues a vector
-// instruction every eight clocks, a SIMD takes one every four: the erf-GELU of a 128 x 256 tile (a reciprocal, an
-// exponential and thirteen other vector instructions on each of 128 values a lane) cost a lone matrix wave 14 600
-// clocks, 8 100 with a helper, and the plain store gains too (1500 x 1280 -> 5120 + bias: 21.8 us against 22.8).  The
-// matrix wave stages its 32-row blocks as in store_tile_simple and takes the first half of each block's chunks, the
-// helper the second half; a workgroup barrier per block says "block j is staged" (a wave passes barrier j + 1 only
-// when it has block j's chunks in registers, so staging block j + 2 over block j's area after that barrier is safe).
-// Launches without residual, clamp or statistics only: the others keep store_tile_simple on the matrix waves alone.
-__host__ __device__ __forceinline__ bool coop_store_applies(const GemmArgs &p) {
-    return !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW && !p.residual &&
-           !(p.clamp > 0.0f) && !p.stats_out;
-}
-template <int EPI, int TM, int WTN, bool HELPER, typename StageF, typename BarrierF>
-__device__ __forceinline__ void store_coop_epi(const GemmArgs &p, char *buf, int mw, int nw, int lane, long bz, StageF stage, BarrierF barrier) {
-    constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;
-    constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI, T0 = HELPER ? NIT / 2 : 0, T1 = HELPER ? NIT : NIT / 2;
-    static_assert(NIT % 2 == 0, "the chunks of a block split in two");
-    const int ch = lane % CPR, r0 = lane / CPR;
-    const int n = nw + ch * 8;
-    const bool col_ok = n < p.N;
-    half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + bz * p.sY + (long)(mw + r0) * p.ldY + n;
-    if constexpr (!HELPER) stage(std::integral_constant<int, 0>{});
-    static_for<TM>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        barrier();                                             // block j is staged
-        const half_t *rd = reinterpret_cast<const half_t *>(buf + (j & 1) * BUF_BYTES) + r0 * SLD_H + ch * 8;
-        half8v x[T1 - T0];
-#pragma unroll
-        for (int t = T0; t < T1; t++) x[t - T0] = *reinterpret_cast<const half8v *>(rd + t * RPI * SLD_H);
-        if constexpr (!HELPER && j + 1 < TM) stage(std::integral_constant<int, j + 1>{});
-#pragma unroll
-        for (int t = T0; t < T1; t++) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[t - T0][e] = (half_t)apply_epi_c<EPI>((float)x[t - T0][e]);
-            if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) *reinterpret_cast<half8v *>(ybase + (long)(32 * j + t * RPI) * p.ldY) = x[t - T0];
-        }
-    });
-}
-template <int TM, int WTN, bool HELPER, typename StageF, typename BarrierF>
-__device__ __forceinline__ void store_coop(const GemmArgs &p, char *buf, int mw, int nw, int lane, long bz, StageF stage, BarrierF barrier) {
-    switch (p.epi) {
-    case MI_EPI_GELU_ERF: store_coop_epi<MI_EPI_GELU_ERF, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
-    case MI_EPI_GELU_TANH: store_coop_epi<MI_EPI_GELU_TANH, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
-    case MI_EPI_RELU: store_coop_epi<MI_EPI_RELU, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
-    default: store_coop_epi<MI_EPI_NONE, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
-    }
-}
-
-// The activation is a compile-time choice inside the store loops: one uniform branch per tile
-// instead of one per element.
-template <int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
-__device__ __forceinline__ void store_tile(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                           int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
-    const bool simple = !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW;
-    if (simple) {
-        switch (p.epi) {
-        case MI_EPI_GELU_ERF: store_tile_simple<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        case MI_EPI_GELU_TANH: store_tile_simple<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        case MI_EPI_RELU: store_tile_simple<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        default: store_tile_simple<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        }
-        return;
-    }
-    switch (p.epi) {
-    case MI_EPI_GELU_ERF: store_tile_epi<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-    case MI_EPI_GELU_TANH: store_tile_epi<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-    case MI_EPI_RELU: store_tile_epi<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-    default: store_tile_epi<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// The tiled MFMA kernel.  BM x BN output tile per workgroup, WAVES_M x WAVES_N
-// waves, each owning a (BM/WAVES_M) x (BN/WAVES_N) sub-tile as 32x32 MFMA
-// tiles.  The MFMA is issued "transposed" (rows = n, columns = m) so that a
-// lane's four consecutive accumulator registers are four consecutive n of one
-// output row: an 8-byte fp16 store.
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool B_KN>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_mfma_kernel(GemmArgs p) {
-    constexpr int NT = WAVES_M * WAVES_N * 64;
-    constexpr int LD = BK + 8;
-    constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
-    constexpr int TM = WTM / 32, TN = WTN / 32;
-    extern __shared__ __align__(16) char smem[];
-    half_t *As = reinterpret_cast<half_t *>(smem);   // [2][BM][LD]
-    half_t *Bs = As + 2 * BM * LD;                   // [2][BN][LD]
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave % WAVES_M, wn = wave / WAVES_M;
-    int tm_, tn_;
-    tile_of(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, p.group_m, tm_, tn_);
-    const int m0 = tm_ * BM, n0 = tn_ * BN;
-    const long bz = blockIdx.y;
-    const half_t *A = p.A + bz * p.sA;
-    const half_t *B = p.B + bz * p.sB;
-
-    KcStage<BM, BK, NT> sa;
-    KcStage<BN, BK, NT> sbk;
-    KnStage<BN, BK, NT> sbn;
-
-    float16v acc[TN][TM];
-#pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-        for (int j = 0; j < TM; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    const int nk = (p.K + BK - 1) / BK;
-    sa.load(A, p.ldA, m0, p.M, 0, p.K, tid);
-    if (B_KN) sbn.load(B, p.ldB, n0, p.NB, 0, p.K, tid); else sbk.load(B, p.ldB, n0, p.N, 0, p.K, tid);
-    sa.store(As, tid);
-    if (B_KN) sbn.store(Bs, tid); else sbk.store(Bs, tid);
-    __syncthreads();
-
-    const int frow = lane & 31, fk = (lane >> 5) * 8;
-    for (int kt = 0; kt < nk; kt++) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < nk;
-        if (more) {
-            sa.load(A, p.ldA, m0, p.M, (kt + 1) * BK, p.K, tid);
-            if (B_KN) sbn.load(B, p.ldB, n0, p.NB, (kt + 1) * BK, p.K, tid); else sbk.load(B, p.ldB, n0, p.N, (kt + 1) * BK, p.K, tid);
-        }
-        const half_t *as = As + cur * BM * LD + (wm * WTM + frow) * LD + fk;
-        const half_t *bs = Bs + cur * BN * LD + (wn * WTN + frow) * LD + fk;
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ks++) {
-            half8v fa[TM], fb[TN];
-#pragma unroll
-            for (int j = 0; j < TM; j++) fa[j] = *reinterpret_cast<const half8v *>(as + j * 32 * LD + ks * 16);
-#pragma unroll
-            for (int i = 0; i < TN; i++) fb[i] = *reinterpret_cast<const half8v *>(bs + i * 32 * LD + ks * 16);
-#pragma unroll
-            for (int i = 0; i < TN; i++)
-#pragma unroll
-                for (int j = 0; j < TM; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[i], fa[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            sa.store(As + (cur ^ 1) * BM * LD, tid);
-            if (B_KN) sbn.store(Bs + (cur ^ 1) * BN * LD, tid); else sbk.store(Bs + (cur ^ 1) * BN * LD, tid);
-        }
-        __syncthreads();
-    }
-
-    half4v cb[TN][4];
-    load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
-    store_tile<TM, TN, WTM, WTN, WAVES_M * WAVES_N, 2 * (BM + BN) * LD * 2>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz);
-}
-
-// ------------------------------------------------------------------------------------------
-// The software-pipelined kernel for K % 64 == 0 (every linear of the encoder
-// configurations).  Same tiles and LDS layout as gemm_mfma_kernel, but the K loop
-// is written out as a four-phase pipeline per 64-deep tile:
-//   phase 0: read fragments of k-step 1 | MFMAs of k-step 0   (+ issue the global loads of tile kt+2)
-//   phase 1: read fragments of k-step 2 | MFMAs of k-step 1 | write the A part of tile kt+1 to the other LDS buffer
-//   phase 2: read fragments of k-step 3 | MFMAs of k-step 2 | write the B part of tile kt+1
-//   barrier
-//   phase 3: read fragments of k-step 0 of tile kt+1 | MFMAs of k-step 3
-// Global loads run two tiles ahead through two register sets, so a load has a
-// whole tile of MFMAs to land before its LDS write; the only barrier of a tile sits
-// where its successor's first fragment read can be hidden behind the last k-step.
-// Two waves per SIMD (8 waves on a 128 x 256 tile) cover each other's waits.
-// BMODE: 0 = B is [N][K], 1 = B is [K][N], 2 = B is [K][N] gathered from a padded image (implicit-GEMM convolution).
-// AMODE 1: A is gathered from a channels-last image (NhwcGather); B is then an ordinary [N][K] or [K][N] operand.
-// AMODE 2: the rows of A are layer-normalised over K on their way in (K <= 512): before the K loop every wave
-// normalises rows of the tile's A panel -- one wave per row, a lane holding eight consecutive k, statistics,
-// arithmetic and rounding exactly those of layernorm_vec_kernel -- into an LDS panel [BM][K + 8] that stays resident;
-// the K loop then streams B alone and reads its A fragments from the panel.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int AMODE = 0>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void gemm_pipe_kernel(GemmArgs p) {
-    constexpr bool B_KN = BMODE != 0, CONV = BMODE == 2, LNA = AMODE == 2;
-    static_assert(AMODE == 0 || BMODE != 2, "one gathered operand at a time");
-    constexpr int BK = 64, LD = BK + 8, NT = WAVES_M * WAVES_N * 64;
-    constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, TM = WTM / 32, TN = WTN / 32;
-    constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;     // 16-byte chunks per thread per tile
-    // The [K][N] operand keeps its layout in LDS: BK rows of BN halves, padded by
-    // 32 halves so that the four rows a transposing read touches fall in distinct
-    // bank groups.  Its MFMA fragments come from ds_read_b64_tr_b16 (see fread).
-    constexpr int BLD = BN + 32, CPRB = BN / 8;
-    static_assert(PA >= 1 && PB >= 1, "tile too small for this workgroup");
-    constexpr int BSZ = B_KN ? BK * BLD : BN * LD;      // halves per B buffer
-    extern __shared__ __align__(16) char smem[];
-    half_t *As = reinterpret_cast<half_t *>(smem);   // [2][BM][LD]; AMODE 2: the normalised panel [BM][K + 8]
-    const int KP = p.K + 8;                          // panel row (halves): 16 bytes off a multiple of 128, like LD
-    half_t *Bs = As + (LNA ? BM * KP : 2 * BM * LD); // [2][BN][LD] or [2][BK][BLD]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave % WAVES_M, wn = wave / WAVES_M;
-    int tm_, tn_;
-    tile_of(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, p.group_m, tm_, tn_);
-    const int m0 = tm_ * BM, n0 = tn_ * BN;
-    const long bz = blockIdx.y;
-    const half_t *A = p.A + bz * p.sA;
-    const half_t *B = p.B + bz * p.sB;
-
-    // Per-thread global sources; rows and columns past the edge re-read the last
-    // valid one (their results are never stored).
-    const half_t *ap[PA], *bp[PB];
-#pragma unroll
-    for (int i = 0; i < PA; i++) { const int c = tid + i * NT; ap[i] = A + (long)min(m0 + (c >> 3), p.M - 1) * p.ldA + (c & 7) * 8; }
-#pragma unroll
-    for (int i = 0; i < PB; i++) {
-        const int c = tid + i * NT;
-        if (!B_KN) bp[i] = B + (long)min(n0 + (c >> 3), p.N - 1) * p.ldB + (c & 7) * 8;
-        else       bp[i] = B + (long)(c / CPRB) * p.ldB + min(n0 + (c % CPRB) * 8, p.NB - 8);
-    }
-    // Implicit GEMM: every chunk of this thread lies in the same eight columns (NT is a multiple of
-    // CPRB), i.e. at one pixel offset, in channels NT / CPRB apart; which tap and which 64 channels a tile
-    // covers is the same for the whole workgroup.
-    const half_t *cpix = nullptr;
-    int ctile0 = 0;
-    if constexpr (CONV) {
-        static_assert(NT % CPRB == 0 && PB * (NT / CPRB) == BK, "a thread's chunks share their columns, NT / CPRB rows apart");
-        const int ncol = min(n0 + (tid % CPRB) * 8, p.NB - 8);
-        const int oh = ncol / p.cv.OW, ow = ncol % p.cv.OW;
-        cpix = p.cv.xp + (p.cv.split ? 0 : bz * p.cv.img) + (long)oh * p.cv.sy * p.cv.Wp + ow + (long)(tid / CPRB) * p.cv.HpWp;
-        ctile0 = p.cv.split ? (int)bz * (p.K / BK) : 0;
-    }
-    // Channels-last gather: a thread's rows are fixed output pixels; (iy0, ix0) is where tap (0, 0) of each lands.
-    int aiy0[PA], aix0[PA];
-    int atile0 = 0;
-    if constexpr (AMODE == 1) {
-#pragma unroll
-        for (int i = 0; i < PA; i++) {
-            const int c = tid + i * NT;
-            const int m = min(m0 + (c >> 3), p.M - 1);
-            const int pq = p.ag.OH * p.ag.OW;
-            const int n = m / pq, rem = m - n * pq, oh = rem / p.ag.OW, ow = rem - oh * p.ag.OW;
-            aiy0[i] = oh * p.ag.sy - p.ag.py;
-            aix0[i] = ow * p.ag.sx - p.ag.px;
-            ap[i] = p.ag.x + (long)n * p.ag.H * p.ag.W * p.ag.C + (c & 7) * 8;
-        }
-        atile0 = p.ag.split ? (int)bz * (p.K / BK) : 0;
-    }
-    u32x4 ga[2][PA], gb[2][PB];
-    auto gload = [&](int set, int kt) {
-        const long ko = (long)kt * BK;
-        if constexpr (AMODE == 1) {
-            const int t = atile0 + kt, tap = t / p.ag.cpt, ci0 = (t - tap * p.ag.cpt) * BK;       // the same for every lane
-            const int kh = tap / p.ag.KW, kw = tap - kh * p.ag.KW;
-            const int ddy = kh * p.ag.dy, ddx = kw * p.ag.dx;
-#pragma unroll
-            for (int i = 0; i < PA; i++) {
-                const int iy = aiy0[i] + ddy, ix = aix0[i] + ddx;
-                const bool in = (unsigned)iy < (unsigned)p.ag.H && (unsigned)ix < (unsigned)p.ag.W;
-                const u32x4 z = {0u, 0u, 0u, 0u};
-                ga[set][i] = in ? ldg16(ap[i] + ((long)iy * p.ag.W + ix) * p.ag.C + ci0) : z;
-            }
-        } else if constexpr (!LNA) {
-#pragma unroll
-            for (int i = 0; i < PA; i++) ga[set][i] = ldg16(ap[i] + ko);
-        }
-#pragma unroll
-        for (int i = 0; i < PB; i++) {
-            if constexpr (CONV) {
-                const int t = ctile0 + kt, tap = t / p.cv.cpt, ci0 = (t - tap * p.cv.cpt) * BK;
-                const int kh = tap / p.cv.KW, kw = tap - kh * p.cv.KW;
-                const int toff = ci0 * p.cv.HpWp + kh * p.cv.dyWp + kw * p.cv.dx;       // same for every lane
-                // The eight halves start kw*dx elements into an aligned row, i.e. at a 2-byte boundary, and
-                // vector loads want 4-byte alignment: odd starts are read from the second copy of the padded
-                // input, which is the first shifted by one element (the choice is the same for every lane).
-                const uint32_t *src = reinterpret_cast<const uint32_t *>(cpix + toff + ((toff & 1) ? p.cv.odd : 0L) + (long)i * (NT / CPRB) * p.cv.HpWp);
-                uint32_t w4[4];
-                __builtin_memcpy(w4, src, 16);
-#pragma unroll
-                for (int q = 0; q < 4; q++) gb[set][i][q] = w4[q];
-            } else {
-                gb[set][i] = ldg16(bp[i] + (B_KN ? ko * p.ldB : ko));
-            }
-        }
-    };
-    auto lwrite_a = [&](int set, int buf) {
-        if constexpr (LNA) return;                     // the panel is already there
-#pragma unroll
-        for (int i = 0; i < PA; i++) { const int c = tid + i * NT; *reinterpret_cast<u32x4 *>(As + buf * BM * LD + (c >> 3) * LD + (c & 7) * 8) = ga[set][i]; }
-    };
-    auto lwrite_b = [&](int set, int buf) {
-#pragma unroll
-        for (int i = 0; i < PB; i++) {
-            const int c = tid + i * NT;
-            half_t *dst = !B_KN ? Bs + buf * BSZ + (c >> 3) * LD + (c & 7) * 8 : Bs + buf * BSZ + (c / CPRB) * BLD + (c % CPRB) * 8;
-            *reinterpret_cast<u32x4 *>(dst) = gb[set][i];
-        }
-    };
-
-    float16v acc[TN][TM];
-#pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-        for (int j = 0; j < TM; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    const int frow = lane & 31, fk = (lane >> 5) * 8;
-    const int aoff = (wm * WTM + frow) * (LNA ? KP : LD) + fk, boff = (wn * WTN + frow) * LD + fk;
-    // [K][N] fragments: within each block of 16 lanes, lane i of ds_read_b64_tr_b16
-    // receives, for j = 0..3, element i%4 of the 8 bytes addressed by lane 4j + i/4.
-    // Pointing lane s at row (k0 + s/4), columns (n0 + 4 (s%4) .. +3) therefore hands
-    // lane i the four consecutive k of column n0 + i: the MFMA operand layout.
-    const int tboff = (fk + ((lane & 15) >> 2)) * BLD + wn * WTN + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-    half8v fa[2][TM], fb[2][TN];
-    auto fread = [&](int fs, int buf, int ks, int kt) {
-        const half_t *as = LNA ? As + aoff + kt * BK + ks * 16 : As + buf * BM * LD + aoff + ks * 16;
-        const int jstep = 32 * (LNA ? KP : LD);
-#pragma unroll
-        for (int j = 0; j < TM; j++) fa[fs][j] = *reinterpret_cast<const half8v *>(as + j * jstep);
-        if (!B_KN) {
-            const half_t *bs = Bs + buf * BSZ + boff + ks * 16;
-#pragma unroll
-            for (int i = 0; i < TN; i++) fb[fs][i] = *reinterpret_cast<const half8v *>(bs + i * 32 * LD);
-        } else {
-            const half_t *bs = Bs + buf * BSZ + tboff + ks * 16 * BLD;
-#pragma unroll
-            for (int i = 0; i < TN; i++) {
-                short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(bs + i * 32));
-                short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(bs + i * 32 + 4 * BLD));
-                short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                fb[fs][i] = __builtin_bit_cast(half8v, both);
-            }
-        }
-    };
-    auto mma = [&](int fs) {
-#pragma unroll
-        for (int i = 0; i < TN; i++)
-#pragma unroll
-            for (int j = 0; j < TM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[fs][i], fa[fs][j], acc[i][j], 0, 0, 0);
-    };
-
-    const int nk = p.K / BK;   // the launcher guarantees K % 64 == 0 and nk >= 2
-    gload(0, 0);
-    gload(1, 1);
-    // folded layer norm: (r, r mu) of the tile's rows, worked out while the first tiles are on their way and parked
-    // in LDS behind the operand buffers until the store (the barrier after the first LDS write covers it)
-    float2v *ln_slot = reinterpret_cast<float2v *>(smem + 2 * (BM * LD + BSZ) * 2);
-    if constexpr (!LNA) lnf_stage<BM, BN, NT>(p, ln_slot, m0, n0, bz, tid);
-    if constexpr (LNA) {
-        // One wave per row, all rows of a wave in flight at once (one trip to memory).  Rows past M repeat the last one.
-        constexpr int NW = NT / 64, RB = BM / NW;
-        static_assert(RB >= 1 && RB <= 16 && BM % NW == 0, "a wave's rows fit its registers");
-        const int e0 = lane * 8;
-        const bool mine = e0 < p.K;
-        const u32x4 z = {0u, 0u, 0u, 0u};
-        const half8v gv = as_half8((p.ln_gamma && mine) ? ldg16(p.ln_gamma + e0) : z);
-        const half8v bv = as_half8((p.ln_beta && mine) ? ldg16(p.ln_beta + e0) : z);
-        for (int r0 = wave * (BM / NW); r0 < (wave + 1) * (BM / NW); r0 += RB) {
-            u32x4 raw[RB];
-#pragma unroll
-            for (int q = 0; q < RB; q++) raw[q] = mine ? ldg16(A + (long)min(m0 + r0 + q, p.M - 1) * p.ldA + e0) : z;
-#pragma unroll
-            for (int q = 0; q < RB; q++) {
-                const half8v t = as_half8(raw[q]);
-                float x[8], sum = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; j++) { x[j] = mine ? (float)t[j] : 0.0f; if (mine) sum += x[j]; }
-                sum = wave_sum(sum);
-                const float mu = sum / (float)p.K;
-                float s2 = 0.0f;
-                if (mine) {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) { const float d = x[j] - mu; s2 = fmaf(d, d, s2); }
-                }
-                s2 = wave_sum(s2);
-                const float rs = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps);
-                if (mine) {
-                    half8v o8;
-#pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        o8[j] = ln_norm1(x[j], mu, rs, p.ln_gamma != nullptr, p.ln_gamma ? (float)gv[j] : 0.0f, p.ln_beta != nullptr, p.ln_beta ? (float)bv[j] : 0.0f);
-                    *reinterpret_cast<half8v *>(As + (r0 + q) * KP + e0) = o8;
-                }
-            }
-        }
-    }
-    lwrite_a(0, 0);
-    lwrite_b(0, 0);
-    __syncthreads();
-    fread(0, 0, 0, 0);
-
-    // MODE 0: steady state; 1: second-to-last tile (nothing left to fetch); 2: last tile.
-    // Tile kt is computed from LDS buffer `cur`; register set `gw` holds tile kt+1, set `gl` receives tile kt+2.
-    auto body = [&](auto MODE_, int kt, int cur, int gw, int gl) {
-        constexpr int MODE = decltype(MODE_)::value;
-        constexpr int NM = TM * TN;               // MFMAs per k-step
-        constexpr int NR = TM + (B_KN ? 2 * TN : TN);   // fragment reads per k-step
-        // Each k-step is pinned to: its fragment reads first, then its MFMAs with the step's
-        // memory instructions dealt out between them, so that neither the LDS pipe nor the
-        // vector-memory path sees a burst.
-        if constexpr (MODE == 0) gload(gl, kt + 2);
-        fread(1, cur, 1, kt);
-        mma(0);
-        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-        for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x020, (PA + PB + NM - 1) / NM, 0); }
-        __builtin_amdgcn_sched_barrier(0);
-        fread(0, cur, 2, kt);
-        mma(1);
-        if constexpr (MODE < 2) lwrite_a(gw, cur ^ 1);
-        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-        for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x200, (PA + NM - 1) / NM, 0); }
-        __builtin_amdgcn_sched_barrier(0);
-        fread(1, cur, 3, kt);
-        mma(0);
-        if constexpr (MODE < 2) lwrite_b(gw, cur ^ 1);
-        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-        for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x200, (PB + NM - 1) / NM, 0); }
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        if constexpr (MODE < 2) fread(0, cur ^ 1, 0, kt + 1);
-        mma(1);
-        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    using M0 = std::integral_constant<int, 0>;
-    using M1 = std::integral_constant<int, 1>;
-    using M2 = std::integral_constant<int, 2>;
-    const int npairs = (nk - 2) >> 1;       // steady-state tiles come in (buffer 0, buffer 1) pairs
-    int kt = 0;
-    for (int pr = 0; pr < npairs; pr++, kt += 2) {
-        body(M0{}, kt, 0, 1, 0);
-        body(M0{}, kt + 1, 1, 0, 1);
-    }
-    half4v cb[TN][4];
-    if (nk & 1) {
-        body(M0{}, kt, 0, 1, 0);
-        body(M1{}, kt + 1, 1, 0, 1);
-        load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
-        body(M2{}, kt + 2, 0, 1, 0);
-    } else {
-        body(M1{}, kt, 0, 1, 0);
-        load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
-        body(M2{}, kt + 1, 1, 0, 1);
-    }
-    __syncthreads();
-    LnFold<TM> ln;
-    if (!LNA && p.lnf_stats) {
-        ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN;
-#pragma unroll
-        for (int j = 0; j < TM; j++) { const float2v v = ln_slot[wm * WTM + 32 * j + (lane & 31)]; ln.r[j] = v[0]; ln.rmu[j] = v[1]; }
-    }
-    store_tile<TM, TN, WTM, WTN, WAVES_M * WAVES_N, 2 * (BM * LD + BSZ) * 2>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln);
-}
 
 // ------------------------------------------------------------------------------------------
 // Split-K without fp32 planes and without a second launch: the two workgroups of a tile (gemm_w4_kernel, SK) exchange
@@ -1487,30 +520,6 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
     }
     phase_store();
     if (probe) { p.clk[2] = clock64(); p.clk[3] = wall_clock64(); }
-}
-
-// ------------------------------------------------------------------------------------------
-// Scalar kernel: one thread per output, fp32 accumulation seeded with the bias,
-// any strides.  The arithmetic of the reference's mm2 (matmul.jl:17-27).
-__global__ void gemm_scalar_kernel(GemmArgs p, int b_kn) {
-    long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long total = (long)p.M * p.N;
-    if (idx >= total) return;
-    int n = (int)(idx % p.N), m = (int)(idx / p.N);
-    long bz = blockIdx.y;
-    const half_t *A = p.A + bz * p.sA + (long)m * p.ldA;
-    const half_t *B = p.B + bz * p.sB;
-    const half_t *bias = p.bias ? p.bias + bz * p.sBias : nullptr;
-    float acc = p.bias_mode == MI_BIAS_COL ? (float)bias[n] : p.bias_mode == MI_BIAS_ROW ? (float)bias[m] : 0.0f;
-    if (b_kn) for (int k = 0; k < p.K; k++) acc = fmaf((float)A[k], (float)B[(long)k * p.ldB + n], acc);
-    else      for (int k = 0; k < p.K; k++) acc = fmaf((float)A[k], (float)B[(long)n * p.ldB + k], acc);
-    long off = bz * p.sY + (long)m * p.ldY + n;
-    if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(acc, p.epi);
-    else {
-        half_t o = (half_t)apply_epi((float)(half_t)acc, p.epi);
-        if (p.residual) o = (half_t)((float)o + (float)p.residual[off]);
-        reinterpret_cast<half_t *>(p.Y)[off] = o;
-    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2147,25 +1156,11 @@ void *scratch_of_current_device() {
     return g_scratch_ptr[dev];
 }
 
-template <typename KernelT>
-int raise_lds(KernelT kern, int bytes) {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess ? 0 : 1;
-}
-
 // LDS of the four-wave kernel: three 64-deep stages of both operands (the store's staging reuses them), then a folded
 // layer norm's (r, r mu) per row and colsum and biasp per column
 template <int BM, int BN>
 constexpr int w4_lds_bytes() { return 3 * (BM + BN) * 64 * 2 + BM * 8 + BN * 8; }
 
-template <int BM, int BN, int BK>
-constexpr int gemm_lds_bytes() {
-    constexpr int kc = BN * (BK + 8), kn = BK * (BN + 32);       // B buffer in either layout
-    return 2 * (BM * (BK + 8) + (kc > kn ? kc : kn)) * 2 + BM * 8 + BN * 8;      // + a folded layer norm's (r, r mu) per row, colsum and biasp per column
-}
-
-#define GEMM_BIG 128, 256, 64, 2, 2
-#define GEMM_MID 128, 128, 64, 2, 2
-#define GEMM_SMALL 64, 64, 64, 2, 2
 
 // k-slice depth for the [K][F] skinny kernel: enough workgroups to put ~2 on every CU, slices a
 // multiple of 32 within [64, SKN_KMAX].
@@ -2189,57 +1184,12 @@ bool mfma_addressable(const GemmArgs &a, bool b_kn) {
 }
 
 template <int BM, int BN, int WM, int WN>
-int launch_pipe(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    // the kernel always walks at least two 64-deep tiles (its prologue fetches two ahead): one tile would read past K
-    if (a.K < 128 || a.K % 64) return MI_DECLINE_EXTENT;
-    a.tiles_m = (int)ceil_div(a.M, BM);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    a.vec_store = a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
-                            : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
-    constexpr int lds = gemm_lds_bytes<BM, BN, 64>();
-    if (a.ag.x) {
-        if (a.cv.xp) return MI_DECLINE_UNSUPPORTED;
-        if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1, 1>), grid, dim3(WM * WN * 64), lds, st, a);
-        else      hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0, 1>), grid, dim3(WM * WN * 64), lds, st, a);
-    }
-    else if (a.cv.xp)   hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 2>), grid, dim3(WM * WN * 64), lds, st, a);
-    else if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1>), grid, dim3(WM * WN * 64), lds, st, a);
-    else           hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0>), grid, dim3(WM * WN * 64), lds, st, a);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-}
-
-// The pipelined kernel with the layer norm of A's rows as its prologue (AMODE 2): 64-row tiles, 128 <= K <= 512.
-constexpr int LNA_KMAX = 512;
-template <int BN, int WM, int WN>
-constexpr int lna_lds_bytes(int K) {
-    constexpr int kc = BN * (64 + 8), kn = 64 * (BN + 32);
-    return (64 * (K + 8) + 2 * (kc > kn ? kc : kn)) * 2;
-}
-template <int BN, int WM, int WN>
-int launch_pipe_ln(GemmArgs a, bool b_kn, hipStream_t st) {
-    if (a.K < 128 || a.K % 64 || a.K > LNA_KMAX || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
-    a.tiles_m = (int)ceil_div(a.M, 64);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    a.vec_store = a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
-                            : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1);
-    const int lds = lna_lds_bytes<BN, WM, WN>(a.K);
-    if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<64, BN, WM, WN, 1, 2>), grid, dim3(WM * WN * 64), lds, st, a);
-    else      hipLaunchKernelGGL((gemm_pipe_kernel<64, BN, WM, WN, 0, 2>), grid, dim3(WM * WN * 64), lds, st, a);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-}
-
-template <int BM, int BN, int WM, int WN>
 int launch_w4(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
     if (a.K < 64 || a.K % 64 || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
     a.tiles_m = (int)ceil_div(a.M, BM);
     a.tiles_n = (int)ceil_div(a.N, BN);
     a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    a.vec_store = a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
-                            : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
+    a.vec_store = rows_vec16(a);
     // per-lane load offsets are 32-bit byte offsets from the tile origin
     if ((int64_t)BM * a.ldA * 2 >= (1ll << 31) || (int64_t)(b_kn ? 64 : BN) * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
     a.clk = g_clock_probe;
@@ -2266,8 +1216,7 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
     a.tiles_n = (int)ceil_div(a.N, BN);
     a.group_m = 1;
     while (a.group_m * a.group_m < (int)ceil_div((int64_t)a.tiles_m * a.tiles_n, 8) && a.group_m < a.tiles_m) a.group_m++;
-    a.vec_store = a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
-                            : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
+    a.vec_store = rows_vec16(a);
     if ((int64_t)BM * a.ldA * 2 >= (1ll << 31) || (int64_t)(b_kn ? 64 : BN) * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
     const int tiles = a.tiles_m * a.tiles_n;
     a.sk_S = split;
@@ -2287,32 +1236,16 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
-// tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands only; a gathered operand (implicit-GEMM
-// convolution) planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
+// tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
+// (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
 // output, same bits, and the plan (hence the workspace) stays a function of the extents alone.
 int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    const bool plain = !a.cv.xp && !a.ag.x;
+    const bool plain = !a.cv.xp && !a.ag.x && a.K % 64 == 0;
     switch (tile) {
-        case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : launch_pipe<128, 256, 2, 4>(a, b_kn, nbatch, st);
-        case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : launch_pipe<192, 128, 2, 4>(a, b_kn, nbatch, st);
-        case 2: return launch_pipe<128, 128, 2, 4>(a, b_kn, nbatch, st);
-        case 3: return launch_pipe<64, 128, 2, 4>(a, b_kn, nbatch, st);
-        default: return launch_pipe<64, 64, 2, 2>(a, b_kn, nbatch, st);
+        case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : mi_pipe_launch(0, a, b_kn, nbatch, st);
+        case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : mi_pipe_launch(1, a, b_kn, nbatch, st);
+        default: return mi_pipe_launch(tile, a, b_kn, nbatch, st);
     }
-}
-
-template <int BM, int BN, int BK, int WM, int WN>
-int launch_mfma(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    a.tiles_m = (int)ceil_div(a.M, BM);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    a.vec_store = a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
-                            : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
-    constexpr int lds = gemm_lds_bytes<BM, BN, BK>();
-    if (b_kn) hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WM, WN, true>), grid, dim3(WM * WN * 64), lds, st, a);
-    else      hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WM, WN, false>), grid, dim3(WM * WN * 64), lds, st, a);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
 // Tile and K-split of a pipelined GEMM, chosen by estimated time.  The five tilings of gemm_pipe_kernel were timed
@@ -2342,7 +1275,7 @@ double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, i
     const int64_t rounds = ceil_div(wg, (int64_t)mi_num_cus());
     const double load = wg < mi_num_cus() ? (double)wg / cus : 1.0;
     const double step = wg <= mi_num_cus() ? t.step_lo + (t.step_full - t.step_lo) * load : t.step_full * t.round * (double)rounds;
-    double us = 2.0 + (t.fixed - 2.0) * (1.0 + 0.8 * (double)(rounds - 1)) + (t.fixed - 2.0) * 0.4 * load + (double)(K / (64 * split)) * step;
+    double us = 2.0 + (t.fixed - 2.0) * (1.0 + 0.8 * (double)(rounds - 1)) + (t.fixed - 2.0) * 0.4 * load + (double)((K + 63) / 64 / split) * step;
     if (split > 1) us += 4.0 + 0.25 * (double)split * (double)M * (double)N * 4.0 / 1e6;
     return us;
 }
@@ -2535,8 +1468,8 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // Split K over workgroups when the output alone cannot fill the chip: each K-slice is one plane
         // of a batched launch (plane strides: A advances along k, Y one fp32 M x N plane in ws), and a
         // second small kernel sums the planes and applies bias, activation and residual.
-        const bool pipe = a.K % 64 == 0 && a.K >= 128;
-        if ((a.cv.xp || a.ag.x) && !pipe) return MI_DECLINE_EXTENT;      // only the pipelined kernel gathers
+        const bool pipe = a.K > 64, whole = pipe && a.K % 64 == 0;
+        if ((a.cv.xp || a.ag.x) && !whole) return MI_DECLINE_EXTENT;      // only the pipelined kernel gathers
         TilePlan tp = {4, 1, false};
         // A folded norm on the way in or row statistics on the way out live in the tiled kernels' own store: those calls
         // need the pipelined kernels, 16-byte rows, and K-slices only in the form that ends in that store (the in-launch
@@ -2545,7 +1478,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         if (in_store) {
             const bool rows16 = !a.out_f32 ? (a.N % 8 == 0 && a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)))
                                            : (a.N % 4 == 0 && a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16));
-            if (!pipe || a.cv.xp || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
+            if (!whole || a.cv.xp || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
         }
         if (pipe) {
             tp = plan_tiles(a.M, a.N, a.K, nbatch, !a.lnf_stats);
@@ -2586,16 +1519,9 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
-        // K not a multiple of 64 (or a single tile deep): the unpipelined kernel, big tiles as soon as they cover half the CUs
-        const int64_t big = ceil_div(a.M, 128) * ceil_div(a.N, 256) * nbatch;
-        const int64_t mid = ceil_div(a.M, 128) * ceil_div(a.N, 128) * nbatch;
-        if (big * 2 > mi_num_cus()) return launch_mfma<GEMM_BIG>(a, b_kn, nbatch, st);
-        if (mid >= (mi_num_cus() * 3) / 8) return launch_mfma<GEMM_MID>(a, b_kn, nbatch, st);
-        return launch_mfma<GEMM_SMALL>(a, b_kn, nbatch, st);
+        return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
-    long total = (long)a.M * a.N;
-    hipLaunchKernelGGL(gemm_scalar_kernel, dim3((unsigned)ceil_div(total, 256), (unsigned)nbatch), dim3(256), 0, st, a, b_kn ? 1 : 0);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+    return mi_any_launch(a, b_kn, false, nbatch, st);
 }
 
 }  // namespace
@@ -2658,39 +1584,12 @@ int mi_init(void) {
     if (__builtin_strncmp(prop.gcnArchName, "gfx950", 6) != 0) return MI_ERROR_DEVICE;
     g_cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     int bad = 0;
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_BIG, true>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_BIG, false>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_MID, true>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_MID, false>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_SMALL, true>, gemm_lds_bytes<64, 64, 64>());
-    bad |= raise_lds(gemm_mfma_kernel<GEMM_SMALL, false>, gemm_lds_bytes<64, 64, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 256, 2, 4, true>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 256, 2, 4, false>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 128, 2, 4, true>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 128, 2, 4, false>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<64, 128, 2, 4, 1>, gemm_lds_bytes<64, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<64, 128, 2, 4, 0>, gemm_lds_bytes<64, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<192, 128, 2, 4, 1>, gemm_lds_bytes<192, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<192, 128, 2, 4, 0>, gemm_lds_bytes<192, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<192, 128, 2, 4, 2>, gemm_lds_bytes<192, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<192, 128, 2, 4, 0, 1>, gemm_lds_bytes<192, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<192, 128, 2, 4, 1, 1>, gemm_lds_bytes<192, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 256, 2, 4, 2>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 256, 2, 4, 0, 1>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 256, 2, 4, 1, 1>, gemm_lds_bytes<128, 256, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 128, 2, 4, 0, 1>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 128, 2, 4, 1, 1>, gemm_lds_bytes<128, 128, 64>());
-    bad |= raise_lds(gemm_pipe_kernel<128, 128, 2, 4, 2>, gemm_lds_bytes<128, 128, 64>());
     bad |= raise_lds(gemm_w4_kernel<128, 256, 1, 4, true>, w4_lds_bytes<128, 256>());
     bad |= raise_lds(gemm_w4_kernel<128, 256, 1, 4, false>, w4_lds_bytes<128, 256>());
     bad |= raise_lds(gemm_w4_kernel<192, 128, 2, 2, true>, w4_lds_bytes<192, 128>());
     bad |= raise_lds(gemm_w4_kernel<192, 128, 2, 2, false>, w4_lds_bytes<192, 128>());
     bad |= raise_lds(gemm_w4_kernel<128, 128, 2, 2, true, true>, w4_lds_bytes<128, 128>());
     bad |= raise_lds(gemm_w4_kernel<128, 128, 2, 2, false, true>, w4_lds_bytes<128, 128>());
-    bad |= raise_lds(gemm_pipe_kernel<64, 128, 2, 4, 1, 2>, lna_lds_bytes<128, 2, 4>(LNA_KMAX));
-    bad |= raise_lds(gemm_pipe_kernel<64, 128, 2, 4, 0, 2>, lna_lds_bytes<128, 2, 4>(LNA_KMAX));
-    bad |= raise_lds(gemm_pipe_kernel<64, 64, 2, 2, 1, 2>, lna_lds_bytes<64, 2, 2>(LNA_KMAX));
-    bad |= raise_lds(gemm_pipe_kernel<64, 64, 2, 2, 0, 2>, lna_lds_bytes<64, 2, 2>(LNA_KMAX));
     bad |= raise_lds(skinny_fk_kernel<1, 3>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<2, 3>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 3>, (int)SKINNY_FK_LDS_MAX);
@@ -2699,6 +1598,7 @@ int mi_init(void) {
     bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<8, 12>, (int)SKINNY_FK_LDS_MAX);
+    bad |= mi_pipe_init() | mi_any_init();
     bad |= mi_sdpa_init();
     bad |= scratch_of_current_device() == nullptr;
     sk_probe_current_device();      // a device that fails the probe only loses that path
@@ -2942,14 +1842,14 @@ int mi_ln_gemm_f16(void *Y, const void *X, const void *gamma, const void *beta, 
     const bool b_kn = w_layout == MI_W_KF;
     if (!mfma_addressable(a, b_kn)) return MI_DECLINE_OPERANDS;
     if ((gamma && !aligned_to(gamma, 16)) || (beta && !aligned_to(beta, 16))) return MI_DECLINE_OPERANDS;
-    if (K < 128 || K % 64 || K > LNA_KMAX) return MI_DECLINE_EXTENT;      // the caller runs the two ops
+    if (K < 128 || K % 64 || K > MI_LNA_KMAX) return MI_DECLINE_EXTENT;      // the caller runs the two ops
     // a shape whose plain GEMM would split K sums in another order: keep the promise of identical bits, decline
     if (plan_tiles(T, F, K, 1, true).split != 1) return MI_DECLINE_EXTENT;
     a.ln_on = 1; a.ln_gamma = (const half_t *)gamma; a.ln_beta = (const half_t *)beta; a.ln_eps = eps;
     // 64-row tiles only (the normalised panel of a workgroup stays in LDS); which width, by the same estimate as
     // every other tiled launch
     const bool wide = tile_cost_us(T, F, K, 1, 3, 1) <= tile_cost_us(T, F, K, 1, 4, 1);
-    return wide ? launch_pipe_ln<128, 2, 4>(a, b_kn, (hipStream_t)stream) : launch_pipe_ln<64, 2, 2>(a, b_kn, (hipStream_t)stream);
+    return mi_pipe_launch_ln(wide, a, b_kn, (hipStream_t)stream);
 }
 
 int mi_ln_gemv_f16(void *Y, const void *X, const void *gamma, const void *beta, float eps,

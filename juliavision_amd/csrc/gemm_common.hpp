@@ -1,0 +1,634 @@
+// What the tiled fp16 GEMM kernels share: their arguments, operand staging, the workgroup -> tile map and the store
+// (bias, folded layer norm, activation, residual, clamp, row statistics).
+//
+// Internal problem statement (row-major):  Y[M x N] = A[M x K] . B  (+ bias)
+//   A is K-contiguous.  B is either N-contiguous [K][N] (B_KN) or K-contiguous
+//   [N][K].  For a linear layer M = tokens, N = features, A = X, B = W.
+#pragma once
+#include "common.hpp"
+#include <type_traits>
+
+struct GemmArgs {
+    void *Y;
+    const half_t *A, *B, *bias, *residual;
+    int M, N, K;
+    int NB;                 // columns addressable in B (>= N; a multiple of 8 for the [K][N] layout)
+    long ldY, ldA, ldB;
+    long sY, sA, sB, sBias; // batch strides (elements)
+    int bias_mode, epi, out_f32;
+    int tiles_m, tiles_n, group_m;
+    int vec_store;          // Y (and residual) rows allow 16-byte accesses
+    ConvGather cv;          // cv.xp != nullptr: B is the im2col matrix of a convolution, gathered on the fly
+    NhwcGather ag;          // ag.x != nullptr: A is the patch matrix of a channels-last convolution, gathered on the fly
+    // Decode-sized kernels only: the rows of A are layer-normalised over K on their way into LDS
+    // (ln_on; gamma, beta may be null), exactly as layernorm_vec_kernel would have written them.
+    const half_t *ln_gamma, *ln_beta;
+    float ln_eps;
+    int ln_on;
+    // Output side: when lnout is set, the rows of Y are also layer-normalised over N into lnout (dense rows of N
+    // halves), as mi_layernorm_f16 on Y would write them (the next block's first norm riding in this GEMM's store).
+    half_t *lnout;
+    const half_t *lnout_gamma, *lnout_beta;
+    float lnout_eps;
+    // Tiled kernels and the split-K plane sums: > 0 clamps the fp16 result to [-clamp, clamp] after the residual add,
+    // as a separate aten::clamp on Y would (the overflow guard of exported fp16 encoder layers).
+    float clamp;
+    // Measurement only (mi_set_clock_probe): workgroup 0 of a four-wave launch stores {shader clock, 100 MHz clock}
+    // here when it starts and again after its last store.  Null in ordinary use.
+    unsigned long long *clk;
+    // Measurement only (mi_set_phase_probe): every matrix wave of the first phase_wgs workgroups of a four-wave launch
+    // stores the shader clocks it spent {before its K loop, in it, issuing its store, waiting for the store to drain}.
+    unsigned long long *phase;
+    int phase_wgs;
+    // Split-K with the partial tiles exchanged between the workgroups of a tile instead of written as planes
+    // (gemm_w4_kernel, SK instance): sk_S = 2 workgroups per tile, tiles dealt sk_tpx per XCD; partials in sk_part,
+    // per-wave arrival flags in sk_flags (they carry sk_epoch; the last reader of a flag clears it).
+    int sk_S, sk_tpx;
+    float *sk_part;
+    unsigned *sk_flags;
+    unsigned sk_epoch;
+    // Layer norm folded away (mi_lnfold_gemm_f16): A holds the raw rows, B carries gamma, and the store turns an
+    // accumulator into r (acc - mu colsum[n]) + biasp[n], with the row's (mu, r) combined from lnf_stats.
+    const float *lnf_stats;           // [lnf_nseg][M][2]: (sum, squares about its own mean) of each 32-column segment of a row
+    const float *lnf_colsum, *lnf_biasp;      // fp32[N], plane stride lnf_svec
+    long lnf_svec;
+    int lnf_nseg;
+    float lnf_eps;
+    // Row statistics of the result for a later folded norm: stats_out[n / 32][m] = (sum, squares about the mean) of the
+    // final fp16 values Y[m][32 (n / 32) .. + 32); stats_nseg segments per row.
+    float *stats_out;
+    int stats_nseg;
+    int sk_spin;                      // polls before a wave gives up on its partners
+    unsigned sk_pub_xor, sk_xcc_xor;  // zero in ordinary use: mi_test_exchange_faults makes the waits fail from the host side
+    unsigned *status;                 // the device's sticky status word
+};
+
+namespace {
+
+
+// ------------------------------------------------------------------------------------------
+// Staging of a K-contiguous operand tile ROWS x BK: each thread moves 16-byte
+// chunks global -> registers -> LDS rows of BK+8 halves (the 16-byte pad makes
+// the 32 rows an MFMA operand read touches fall in distinct bank groups).
+template <int ROWS, int BK, int NT>
+struct KcStage {
+    static constexpr int CPR = BK / 8;
+    static constexpr int CHUNKS = ROWS * CPR;
+    static constexpr int PER = (CHUNKS + NT - 1) / NT;
+    static constexpr int LD = BK + 8;
+    u32x4 r[PER];
+
+    __device__ __forceinline__ void load(const half_t *base, long ld, int row0, int nrows, int k0, int K, int tid) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int c = tid + i * NT;
+            int row = c / CPR, kc = c % CPR;
+            int gr = min(row0 + row, nrows - 1);
+            int gk = k0 + kc * 8;
+            u32x4 z = {0u, 0u, 0u, 0u};
+            if (CHUNKS % NT == 0 || c < CHUNKS) r[i] = gk < K ? ldg16(base + (long)gr * ld + gk) : z;
+        }
+    }
+    __device__ __forceinline__ void store(half_t *lds, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int c = tid + i * NT;
+            int row = c / CPR, kc = c % CPR;
+            if (CHUNKS % NT == 0 || c < CHUNKS) *reinterpret_cast<u32x4 *>(lds + row * LD + kc * 8) = r[i];
+        }
+    }
+};
+
+// Staging of an N-contiguous operand tile [BK][COLS] into the same K-contiguous
+// LDS rows: a thread loads an 8(k) x 8(n) block with eight 16-byte row loads,
+// transposes it in registers (v_perm_b32) and writes eight 16-byte LDS rows.
+template <int COLS, int BK, int NT>
+struct KnStage {
+    static constexpr int KB = BK / 8;
+    static constexpr int BLOCKS = KB * (COLS / 8);
+    static constexpr int PER = (BLOCKS + NT - 1) / NT;
+    static constexpr int LD = BK + 8;
+    u32x4 r[PER][8];
+
+    __device__ __forceinline__ void load(const half_t *base, long ld, int col0, int ncols, int k0, int K, int tid) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int blk = tid + i * NT;
+            int kb = blk % KB, nb = blk / KB;
+            int gn = min(col0 + nb * 8, ncols - 8);
+            if (BLOCKS % NT == 0 || blk < BLOCKS) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    int gk = k0 + kb * 8 + j;
+                    u32x4 z = {0u, 0u, 0u, 0u};
+                    r[i][j] = gk < K ? ldg16(base + (long)gk * ld + gn) : z;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void store(half_t *lds, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int blk = tid + i * NT;
+            int kb = blk % KB, nb = blk / KB;
+            if (BLOCKS % NT == 0 || blk < BLOCKS) {
+#pragma unroll
+                for (int w = 0; w < 4; w++) {   // dword w of each row holds columns 2w, 2w+1
+                    u32x4 lo, hi;
+                    lo.x = pack_lo(r[i][0][w], r[i][1][w]); hi.x = pack_hi(r[i][0][w], r[i][1][w]);
+                    lo.y = pack_lo(r[i][2][w], r[i][3][w]); hi.y = pack_hi(r[i][2][w], r[i][3][w]);
+                    lo.z = pack_lo(r[i][4][w], r[i][5][w]); hi.z = pack_hi(r[i][4][w], r[i][5][w]);
+                    lo.w = pack_lo(r[i][6][w], r[i][7][w]); hi.w = pack_hi(r[i][6][w], r[i][7][w]);
+                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w) * LD + kb * 8) = lo;
+                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w + 1) * LD + kb * 8) = hi;
+                }
+            }
+        }
+    }
+};
+
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+// Workgroup id -> output tile.  The hardware deals consecutive workgroups
+// round-robin over the 8 XCDs, each with its own L2; this hands every XCD one
+// contiguous run of the tile order, and the tile order walks GROUP_M row tiles
+// per column tile so a run reuses a small set of A and B panels.
+__device__ __forceinline__ void tile_of(int pid, int nwg, int tiles_m, int tiles_n, int group_m, int &tm, int &tn) {
+    int xcd = pid & 7, idx = pid >> 3;
+    int full = nwg >> 3, rem = nwg & 7;
+    int logical = xcd * full + min(xcd, rem) + idx;
+    int width = group_m * tiles_n;
+    int g = logical / width, in = logical - g * width;
+    int first = g * group_m;
+    int gsz = min(tiles_m - first, group_m);
+    tm = first + in % gsz;
+    tn = in / gsz;
+}
+
+// What the store of a folded norm needs, fetched while the first operand tiles are on their way and parked in `slot`
+// (LDS past everything else the kernel keeps there: BM float2 (r, r mu), then BN column sums, then BN biases).
+//
+// A row's mean and reciprocal standard deviation over its K elements come from the per-segment statistics a producer
+// left (stats[seg][row] = (sum, squares about the segment's own mean)).  LPR lanes share a row, each with every LPR-th
+// segment, many loads in flight at a time (a lane that walked all segments one dependent load after the other held
+// the whole workgroup at its first barrier for 10 us).  One pass: the squares between the segments are taken about the
+// first segment's mean, which lies within a segment mean's spread of the row mean, so the final subtraction cancels
+// nothing that matters -- sum(x^2) - n mean^2 about zero would.  r = 1 / sqrt(var + eps), rmu = r * mean.
+// The caller synchronises the workgroup before anybody reads the slot.
+template <int BM, int BN, int NT, typename Args>
+__device__ __forceinline__ void lnf_stage(const Args &p, float2v *slot, int m0, int n0, long bz, int tid) {
+    if (!p.lnf_stats) return;
+    constexpr int LPR = NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1;
+    static_assert(NT >= BM && (BM * LPR) % 64 == 0, "whole waves work on the rows");
+    if (tid < BM * LPR) {
+        const int row = tid / LPR, q = tid % LPR;
+        const float2v *seg = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + row, p.M - 1);
+        const float ref = seg[0][0] / (float)min(32, p.K);
+        float total = 0.0f, within = 0.0f, between = 0.0f;
+        // U loads in flight per lane: all of a row's segments in one trip to memory for K <= 1536 (2048 with four lanes a
+        // row) -- a trip costs 1 to 2 us here (the statistics were written by another kernel, on other XCDs), and the
+        // first operand tiles, requested before this, take about as long, so one trip is hidden and every further one
+        // is not (two and three batches of eight measured +3.3 and +4.3 us per launch)
+        constexpr int U = LPR == 4 ? 16 : 24;
+        for (int s0 = q; s0 < p.lnf_nseg; s0 += U * LPR) {
+            float2v v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int sg = s0 + u * LPR;
+                const float2v z = {0.0f, 0.0f};
+                v[u] = sg < p.lnf_nseg ? seg[(long)sg * p.M] : z;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int sg = s0 + u * LPR;
+                if (sg < p.lnf_nseg) {
+                    const int left = p.K - 32 * sg;
+                    const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
+                    const float d = fmaf(v[u][0], inv, -ref);
+                    total += v[u][0];
+                    within += v[u][1];
+                    between = fmaf(cnt * d, d, between);
+                }
+            }
+        }
+        if constexpr (LPR >= 2) { total += lane_xor<1>(total); within += lane_xor<1>(within); between += lane_xor<1>(between); }
+        if constexpr (LPR >= 4) { total += lane_xor<2>(total); within += lane_xor<2>(within); between += lane_xor<2>(between); }
+        if (q == 0) {
+            const float mu = total / (float)p.K, dm = mu - ref;
+            const float m2 = within + fmaxf(between - (float)p.K * dm * dm, 0.0f);
+            const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
+            const float2v o = {r, r * mu};
+            slot[row] = o;
+        }
+    }
+    // the tile's columns of colsum and biasp
+    for (int t = tid; t < BN / 2; t += NT) {
+        const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
+        const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
+        float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
+        else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
+        *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = v;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
+// ------------------------------------------------------------------------------------------
+// Accumulator tile -> memory, shared by the tiled kernels.
+// acc[i][j][r]: n = n0 + wn*WTN + 32 i + 8 (r/4) + 4 (lane/32) + r%4,  m = m0 + wm*WTM + 32 j + lane%32.
+// Each wave stages one 32 x WTN sub-tile at a time in its own LDS region (bias
+// joined in fp32, one rounding), then reads it back row-wise so that the
+// activation, the residual add and the global stores run on 16-byte vectors
+// that are contiguous along the output row.  The caller has synchronised the
+// workgroup after its last read of the operand tiles.
+// The column bias of a wave's sub-tile, in the accumulator's order: cb[i][g] covers
+// n = n0 + wn*WTN + 32 i + 8 g + 4 (lane/32) .. +3.  Fetched by the kernels ahead of their last
+// k-step so that the epilogue does not start with a trip to memory.
+template <int TN, int WTN>
+__device__ __forceinline__ void load_col_bias(const GemmArgs &p, half4v (&cb)[TN][4], int n0, int wn, int lane, long bz) {
+    const half4v z = {(half_t)0.0f, (half_t)0.0f, (half_t)0.0f, (half_t)0.0f};
+    const bool on = p.bias_mode == MI_BIAS_COL;
+    const half_t *bias = on ? p.bias + bz * p.sBias : nullptr;
+    const bool vec = (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int n = n0 + wn * WTN + 32 * i + 8 * g + 4 * (lane >> 5);
+            cb[i][g] = z;
+            if (on) {
+                if (n + 3 < p.N && vec) cb[i][g] = *reinterpret_cast<const half4v *>(bias + n);
+                else for (int e = 0; e < 4; e++) if (n + e < p.N) cb[i][g][e] = bias[n + e];
+            }
+        }
+}
+
+// What the store of a folded layer norm carries (by value, so that it stays in registers): (r, r mu) of the lane's rows
+// m0 + wm WTM + 32 j + lane % 32, and the LDS copy of the tile's colsum (bn floats) followed by its biasp.
+template <int TM>
+struct LnFold {
+    bool on = false;
+    float r[TM] = {}, rmu[TM] = {};
+    const float *col = nullptr;
+    int bn = 0;
+};
+template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+__device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
+                                               int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
+    const int frow = lane & 31;
+    const half_t *bias = p.bias ? p.bias + bz * p.sBias : nullptr;
+    constexpr int SLD_H = WTN + 8;                 // halves per staged row (fp16 output)
+    constexpr int SLD_F = WTN + 4;                 // floats per staged row (fp32 output)
+    constexpr int STAGE_BYTES = 32 * SLD_F * 4;
+    static_assert(STAGE_BYTES * NWAVES <= LDS_BYTES, "epilogue staging exceeds the operand LDS");
+    char *stage = smem + wave * STAGE_BYTES;
+    const int hl = lane >> 5;
+    // Row biases for all of the wave's rows before the first store (store_tile_simple says why).
+    float brow_j[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) {
+        const int m = m0 + wm * WTM + 32 * j + frow;
+        brow_j[j] = (p.bias_mode == MI_BIAS_ROW && m < p.M) ? (float)bias[m] : 0.0f;
+    }
+    static_for<TM>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        const int mrow = m0 + wm * WTM + 32 * j;
+        const float brow = brow_j[j];
+#pragma unroll
+        for (int i = 0; i < TN; i++) {
+            // folded layer norm: this lane's columns of colsum and biasp from their LDS copy, a 32-column group at a time
+            float4v lc4[4], lb4[4];
+            if (ln.on) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int nl = 32 * i + 8 * g + 4 * hl;
+                    lc4[g] = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl);
+                    lb4[g] = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int nl = 32 * i + 8 * g + 4 * hl;
+                const int n = n0 + wn * WTN + nl;
+                float v[4];
+                if (ln.on) {      // uniform: r (acc - mu colsum) + biasp
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = fmaf(acc[i][j][4 * g + e], ln.r[j], fmaf(-ln.rmu[j], lc4[g][e], lb4[g][e]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e] + brow + (float)cb[i][g][e];
+                }
+                if (p.out_f32) {
+                    float4v o = {v[0], v[1], v[2], v[3]};
+                    *reinterpret_cast<float4v *>(reinterpret_cast<float *>(stage) + frow * SLD_F + nl) = o;
+                } else {
+                    half4v o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+                    *reinterpret_cast<half4v *>(reinterpret_cast<half_t *>(stage) + frow * SLD_H + nl) = o;
+                }
+            }
+        }
+        // A wave reads back only what it staged itself, and its LDS operations complete in order:
+        // no workgroup barrier, only a stop for the compiler.
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (p.out_f32) {
+            constexpr int CPR = WTN / 4;
+            for (int c = lane; c < 32 * CPR; c += 64) {
+                const int row = c / CPR, ch = c % CPR;
+                const int m = mrow + row, n = n0 + wn * WTN + ch * 4;
+                if (m < p.M && n < p.N) {
+                    float4v x = *reinterpret_cast<const float4v *>(reinterpret_cast<const float *>(stage) + row * SLD_F + ch * 4);
+                    float *yp = reinterpret_cast<float *>(p.Y) + bz * p.sY + (long)m * p.ldY + n;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[e] = apply_epi_c<EPI>(x[e]);
+                    if (n + 3 < p.N) __builtin_memcpy(yp, &x, 16);      // one 16-byte store at any address
+                    else for (int e = 0; e < 4; e++) if (n + e < p.N) yp[e] = x[e];
+                }
+            }
+        } else {
+            constexpr int CPR = WTN / 8;
+            static_assert((32 * CPR) % 64 == 0 && CPR % 4 == 0, "whole waves walk the staged tile; four lanes hold a 32-column segment");
+            for (int c = lane; c < 32 * CPR; c += 64) {
+                const int row = c / CPR, ch = c % CPR;
+                const int m = mrow + row, n = n0 + wn * WTN + ch * 8;
+                half8v x = {};
+                if (m < p.M && n < p.N) {
+                    x = *reinterpret_cast<const half8v *>(reinterpret_cast<const half_t *>(stage) + row * SLD_H + ch * 8);
+                    const long off = bz * p.sY + (long)m * p.ldY + n;
+                    half_t *yp = reinterpret_cast<half_t *>(p.Y) + off;
+                    if constexpr (EPI != MI_EPI_NONE) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) x[e] = (half_t)apply_epi_c<EPI>((float)x[e]);
+                    }
+                    if (n + 7 < p.N) {
+                        if (p.residual) {
+                            half8v rv;
+                            __builtin_memcpy(&rv, p.residual + off, 16);
+#pragma unroll
+                            for (int e = 0; e < 8; e++) x[e] = (half_t)((float)x[e] + (float)rv[e]);
+                        }
+                        if (p.clamp > 0.0f) {
+#pragma unroll
+                            for (int e = 0; e < 8; e++) x[e] = (half_t)fminf(fmaxf((float)x[e], -p.clamp), p.clamp);
+                        }
+                        __builtin_memcpy(yp, &x, 16);
+                    } else {
+                        for (int e = 0; e < 8; e++) {
+                            if (n + e < p.N) {
+                                half_t o = x[e];
+                                if (p.residual) o = (half_t)((float)o + (float)p.residual[off + e]);
+                                if (p.clamp > 0.0f) o = (half_t)fminf(fmaxf((float)o, -p.clamp), p.clamp);
+                                yp[e] = o;
+                            }
+                        }
+                    }
+                }
+                if (p.stats_out) {      // uniform; the launcher admits it with 16-byte stores and N % 8 == 0 only
+                    // the four lanes of a quad hold the 32 columns of one segment of one row (chunks that lie past N
+                    // or below M count nothing): sum, then squares about the segment's own mean, both over the quad
+                    const bool have = m < p.M && n < p.N;
+                    float cnt = have ? 8.0f : 0.0f, sum = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sum += have ? (float)x[e] : 0.0f;
+                    sum += lane_xor<1>(sum); sum += lane_xor<2>(sum);
+                    cnt += lane_xor<1>(cnt); cnt += lane_xor<2>(cnt);
+                    const float mean = sum / fmaxf(cnt, 1.0f);
+                    float sq = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) { const float d = (float)x[e] - mean; sq = have ? fmaf(d, d, sq) : sq; }
+                    sq += lane_xor<1>(sq); sq += lane_xor<2>(sq);
+                    if (have && (ch & 3) == 0) {
+                        const float2v o = {sum, sq};
+                        *reinterpret_cast<float2v *>(p.stats_out + ((long)(n / 32) * p.M + m) * 2) = o;
+                    }
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    });
+}
+
+// Block j (32 rows) of a wave's accumulators -> its staging area `dst` (32 rows of WTN + 8 halves), rounded to fp16 once
+// with the column bias -- or the folded layer norm's r (acc - mu colsum) + biasp -- joined in fp32.
+template <int j, int TM, int TN, int WTN>
+__device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], const LnFold<TM> &ln, int wn, char *dst, int lane) {
+    constexpr int SLD_H = WTN + 8;
+    const int frow = lane & 31, hl = lane >> 5;
+    half_t *st = reinterpret_cast<half_t *>(dst) + frow * SLD_H + 4 * hl;
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int nl = 32 * i + 8 * g;
+            float v[4];
+            if (ln.on) {      // uniform; the tile's colsum and biasp from their LDS copy
+                const float4v lc = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl + 4 * hl);
+                const float4v lb = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl + 4 * hl);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = fmaf(acc[i][j][4 * g + e], ln.r[j], fmaf(-ln.rmu[j], lc[e], lb[e]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e] + (float)cb[i][g][e];
+            }
+            const half4v o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+            *reinterpret_cast<half4v *>(st + nl) = o;
+        }
+}
+
+// The common store: fp16 output in whole 16-byte chunks, column bias (or a folded layer norm), optional activation,
+// residual, clamp and row statistics; no row bias, no fp32 output, no ragged N.
+//
+// Loads and stores of a wave share one counter and complete in order, so a wait for a load -- wherever the compiler
+// places it -- is also a wait for every store issued before that load to be acknowledged: a trip of two microseconds
+// under the burst of all workgroups' stores.  The general store above pays it once per 32-row block of a wave's tile
+// and once per residual chunk (8 000 clocks of a 44 000-clock launch at 1500 x 1280 -> 5120).  Here nothing is fetched
+// behind a store that anybody then waits for: the caller's column bias is pinned in registers ahead of the first store,
+// and the residual chunks of block j + 1 are requested before block j's stores go out.
+// Same arithmetic as the general store (bias joined in fp32, one rounding, activation on the rounded value, residual,
+// clamp), so the two give the same bits.  Two staging areas a wave: block j + 1 is staged while block j's chunks are on
+// their way back from the LDS (a wave's LDS operations complete in order: no wait between staging a block and reading it).
+template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+__device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
+                                                  int wave, int lane, long bz, const LnFold<TM> ln) {
+    constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;      // halves per staged row; one staging area
+    constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI;     // 16-byte chunks per row; rows a wave covers at a time; chunks per lane and block
+    static_assert(2 * BUF_BYTES * NWAVES <= LDS_BYTES && 64 % CPR == 0 && CPR % 4 == 0, "two staging areas a wave; four lanes hold a 32-column segment");
+    char *const buf = smem + wave * 2 * BUF_BYTES;
+    const int frow = lane & 31, hl = lane >> 5;
+    const int ch = lane % CPR, r0 = lane / CPR;                      // this lane's chunks of a block: rows r0 + RPI t, columns 8 ch ..
+    const int mw = m0 + wm * WTM, n = n0 + wn * WTN + ch * 8;
+    const bool col_ok = n < p.N;                                     // N % 8 == 0: a chunk that starts below N ends below it
+    const long off0 = bz * p.sY + (long)(mw + r0) * p.ldY + n;
+    half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + off0;
+    const half_t *const rbase = p.residual ? p.residual + off0 : nullptr;
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) asm volatile("" ::"v"(cb[i][g]));
+    auto stage = [&](auto J) {
+        constexpr int j = decltype(J)::value;
+        stage_block<j, TM, TN, WTN>(acc, cb, ln, wn, buf + (j & 1) * BUF_BYTES, lane);
+    };
+    half8v res[2][NIT];
+    auto fetch_residual = [&](auto J) {
+        constexpr int j = decltype(J)::value;
+#pragma unroll
+        for (int t = 0; t < NIT; t++) {
+            res[j & 1][t] = half8v{};
+            if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) res[j & 1][t] = as_half8(ldg16(rbase + (long)(32 * j + t * RPI) * p.ldY));
+        }
+    };
+    if (rbase) fetch_residual(std::integral_constant<int, 0>{});
+    stage(std::integral_constant<int, 0>{});
+    static_for<TM>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        const half_t *rd = reinterpret_cast<const half_t *>(buf + (j & 1) * BUF_BYTES) + r0 * SLD_H + ch * 8;
+        half8v x[NIT];
+#pragma unroll
+        for (int t = 0; t < NIT; t++) x[t] = *reinterpret_cast<const half8v *>(rd + t * RPI * SLD_H);
+        if constexpr (j + 1 < TM) {
+            stage(std::integral_constant<int, j + 1>{});
+            if (rbase) fetch_residual(std::integral_constant<int, j + 1>{});
+        }
+#pragma unroll
+        for (int t = 0; t < NIT; t++) {
+            const int m = mw + 32 * j + r0 + t * RPI;
+            const bool have = col_ok && m < p.M;
+            if constexpr (EPI != MI_EPI_NONE) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[t][e] = (half_t)apply_epi_c<EPI>((float)x[t][e]);
+            }
+            if (rbase) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[t][e] = (half_t)((float)x[t][e] + (float)res[j & 1][t][e]);
+            }
+            if (p.clamp > 0.0f) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[t][e] = (half_t)fminf(fmaxf((float)x[t][e], -p.clamp), p.clamp);
+            }
+            if (have) *reinterpret_cast<half8v *>(ybase + (long)(32 * j + t * RPI) * p.ldY) = x[t];
+            if (p.stats_out) {      // uniform
+                // the four lanes of a quad hold the 32 columns of one segment of one row (chunks that lie past N or
+                // below M count nothing): sum, then squares about the segment's own mean, both over the quad
+                float cnt = have ? 8.0f : 0.0f, sum = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += have ? (float)x[t][e] : 0.0f;
+                sum += lane_xor<1>(sum); sum += lane_xor<2>(sum);
+                cnt += lane_xor<1>(cnt); cnt += lane_xor<2>(cnt);
+                const float mean = sum / fmaxf(cnt, 1.0f);
+                float sq = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) { const float d = (float)x[t][e] - mean; sq = have ? fmaf(d, d, sq) : sq; }
+                sq += lane_xor<1>(sq); sq += lane_xor<2>(sq);
+                if (have && (ch & 3) == 0) {
+                    const float2v o = {sum, sq};
+                    *reinterpret_cast<float2v *>(p.stats_out + ((long)(n / 32) * p.M + m) * 2) = o;
+                }
+            }
+        }
+    });
+}
+
+// The four-wave kernel's store, shared between a matrix wave and the helper wave on its SIMD.  One wave issues a vector
+// instruction every eight clocks, a SIMD takes one every four: the erf-GELU of a 128 x 256 tile (a reciprocal, an
+// exponential and thirteen other vector instructions on each of 128 values a lane) cost a lone matrix wave 14 600
+// clocks, 8 100 with a helper, and the plain store gains too (1500 x 1280 -> 5120 + bias: 21.8 us against 22.8).  The
+// matrix wave stages its 32-row blocks as in store_tile_simple and takes the first half of each block's chunks, the
+// helper the second half; a workgroup barrier per block says "block j is staged" (a wave passes barrier j + 1 only
+// when it has block j's chunks in registers, so staging block j + 2 over block j's area after that barrier is safe).
+// Launches without residual, clamp or statistics only: the others keep store_tile_simple on the matrix waves alone.
+__host__ __device__ __forceinline__ bool coop_store_applies(const GemmArgs &p) {
+    return !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW && !p.residual &&
+           !(p.clamp > 0.0f) && !p.stats_out;
+}
+template <int EPI, int TM, int WTN, bool HELPER, typename StageF, typename BarrierF>
+__device__ __forceinline__ void store_coop_epi(const GemmArgs &p, char *buf, int mw, int nw, int lane, long bz, StageF stage, BarrierF barrier) {
+    constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;
+    constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI, T0 = HELPER ? NIT / 2 : 0, T1 = HELPER ? NIT : NIT / 2;
+    static_assert(NIT % 2 == 0, "the chunks of a block split in two");
+    const int ch = lane % CPR, r0 = lane / CPR;
+    const int n = nw + ch * 8;
+    const bool col_ok = n < p.N;
+    half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + bz * p.sY + (long)(mw + r0) * p.ldY + n;
+    if constexpr (!HELPER) stage(std::integral_constant<int, 0>{});
+    static_for<TM>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        barrier();                                             // block j is staged
+        const half_t *rd = reinterpret_cast<const half_t *>(buf + (j & 1) * BUF_BYTES) + r0 * SLD_H + ch * 8;
+        half8v x[T1 - T0];
+#pragma unroll
+        for (int t = T0; t < T1; t++) x[t - T0] = *reinterpret_cast<const half8v *>(rd + t * RPI * SLD_H);
+        if constexpr (!HELPER && j + 1 < TM) stage(std::integral_constant<int, j + 1>{});
+#pragma unroll
+        for (int t = T0; t < T1; t++) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[t - T0][e] = (half_t)apply_epi_c<EPI>((float)x[t - T0][e]);
+            if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) *reinterpret_cast<half8v *>(ybase + (long)(32 * j + t * RPI) * p.ldY) = x[t - T0];
+        }
+    });
+}
+template <int TM, int WTN, bool HELPER, typename StageF, typename BarrierF>
+__device__ __forceinline__ void store_coop(const GemmArgs &p, char *buf, int mw, int nw, int lane, long bz, StageF stage, BarrierF barrier) {
+    switch (p.epi) {
+    case MI_EPI_GELU_ERF: store_coop_epi<MI_EPI_GELU_ERF, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
+    case MI_EPI_GELU_TANH: store_coop_epi<MI_EPI_GELU_TANH, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
+    case MI_EPI_RELU: store_coop_epi<MI_EPI_RELU, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
+    default: store_coop_epi<MI_EPI_NONE, TM, WTN, HELPER>(p, buf, mw, nw, lane, bz, stage, barrier); break;
+    }
+}
+
+// The activation is a compile-time choice inside the store loops: one uniform branch per tile
+// instead of one per element.
+template <int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+__device__ __forceinline__ void store_tile(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
+                                           int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
+    const bool simple = !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW;
+    if (simple) {
+        switch (p.epi) {
+        case MI_EPI_GELU_ERF: store_tile_simple<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+        case MI_EPI_GELU_TANH: store_tile_simple<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+        case MI_EPI_RELU: store_tile_simple<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+        default: store_tile_simple<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+        }
+        return;
+    }
+    switch (p.epi) {
+    case MI_EPI_GELU_ERF: store_tile_epi<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+    case MI_EPI_GELU_TANH: store_tile_epi<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+    case MI_EPI_RELU: store_tile_epi<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+    default: store_tile_epi<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+    }
+}
+
+template <typename KernelT>
+int raise_lds(KernelT kern, int bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess ? 0 : 1;
+}
+
+template <int BM, int BN, int BK>
+constexpr int gemm_lds_bytes() {
+    constexpr int kc = BN * (BK + 8), kn = BK * (BN + 32);       // B buffer in either layout
+    return 2 * (BM * (BK + 8) + (kc > kn ? kc : kn)) * 2 + BM * 8 + BN * 8;      // + a folded layer norm's (r, r mu) per row, colsum and biasp per column
+}
+
+// Y (and residual) rows allow 16-byte accesses
+bool rows_vec16(const GemmArgs &a) {
+    return a.out_f32 ? (a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16))
+                     : (a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)));
+}
+
+}  // namespace
+
+// gemm_pipe.hip: the register-staged pipelined kernel.  `tile` indexes TILE_MODELS (gemm.hip).
+int mi_pipe_launch(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
+int mi_pipe_launch_ln(bool wide, const GemmArgs &a, bool b_kn, hipStream_t st);
+constexpr int MI_LNA_KMAX = 512;         // deepest K of the layer-norm prologue
+int mi_pipe_init();
+// gemm_any.hip: the kernels for operands and extents that the others do not take.
+int mi_any_launch(const GemmArgs &a, bool b_kn, bool addressable, int64_t nbatch, hipStream_t st);
+int mi_any_init();
