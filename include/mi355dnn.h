@@ -421,9 +421,9 @@ int64_t mi_convsize(int64_t n, int64_t k, int64_t s, int64_t p, int64_t d);
  * [Cin][Cout/groups][KH][KW] (torch's conv_transpose2d weight); out (OW,OH,Cout,N) with
  * OW = mi_convtransposesize(...); bias[Cout] or NULL.  fp32 accumulation seeded with the
  * bias, one rounding.  kernel == stride with no padding / dilation / output padding and one
- * group is one MFMA GEMM (Cout*KH*KW x Cin x H*W per image) followed by a pixel shuffle,
- * workspace from mi_convtranspose2d_f16_workspace; every other case is the gather kernel
- * and needs no workspace.
+ * group is one MFMA GEMM (Cout*KH*KW x Cin x H*W per image) whose store shuffles the pixels;
+ * every other case is the gather kernel.  Neither writes to ws, which may be NULL
+ * (mi_convtranspose2d_f16_workspace keeps the sizes of a form that staged its operands).
  * Replaces convolutiontranspose!(ctx, out, x, w, bias, stride, padding, dilation, outpad,
  * groups) -- conv.jl:226-294 -- with shufflecase / shuffleout (conv.jl:204-222) and the
  * gather kernel convtranspose2d (conv.jl:149-191). */

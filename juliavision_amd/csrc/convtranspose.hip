@@ -4,10 +4,8 @@
 // Two routes, as the reference has them (conv.jl:204-294):
 //   kernel == stride, no padding / dilation / output padding, one group:
 //       every output pixel has exactly one source pixel and one tap, so per image
-//           y[(co,ky,kx)][H*W] = w2[(co,ky,kx)][Cin] . x[Cin][H*W]        (one GEMM, MFMA)
-//           out[co][iy*KH+ky][ix*KW+kx] = y[(co,ky,kx)][iy*W+ix]          (pixel shuffle)
-//       The bias is expanded to one value per GEMM row, so y is already the rounded result and
-//       the shuffle only moves bits.
+//           out[co][iy*KH+ky][ix*KW+kx] = w[Cin][(co,ky,kx)]^T . x[Cin][H*W] + bias[co]
+//       one GEMM on MFMA whose store does the pixel shuffle.
 //   anything else: one thread per output gathers the inputs that reach it (conv.jl:149-191).
 #include "common.hpp"
 
@@ -20,60 +18,115 @@ struct CtArgs {
     int sx, sy, px, py, dx, dy, groups;
 };
 
-// w2[(co,ky,kx)][ci] = w[ci][(co,ky,kx)] (a 2-D transpose through LDS, 32x32 tiles) and, from the
-// blocks past the transpose, bias2[(co,ky,kx)] = bias[co].
-__global__ void ct_prepare_kernel(half_t *w2, half_t *bias2, const half_t *w, const half_t *bias, int Cin, int M, int taps,
-                                  int tiles_m, int tile_blocks) {
-    if ((int)blockIdx.x >= tile_blocks) {
-        const int r = ((int)blockIdx.x - tile_blocks) * 256 + threadIdx.x;
-        if (r < M) bias2[r] = bias ? bias[r / taps] : (half_t)0.0f;
-        return;
-    }
-    __shared__ half_t tile[32][33];
-    const int tm = ((int)blockIdx.x % tiles_m) * 32, tk = ((int)blockIdx.x / tiles_m) * 32;
-    const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;       // 256 threads: 8 rows a pass
+// Eight halves of row k at column n0, zero outside [0, K) x [0, N): one 16-byte load at any address, by element at the
+// row's end (nothing past the row is read).
+__device__ __forceinline__ u32x4 ct_row8(const half_t *base, int k, int K, long N, long n0) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (k < K) {
+        const half_t *p = base + (long)k * N + n0;
+        if (n0 + 8 <= N) __builtin_memcpy(&v, p, 16);
+        else if (n0 < N) {
+            half8v h = as_half8(v);
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-        const int k = tk + ly + 8 * p, m = tm + lx;
-        tile[ly + 8 * p][lx] = (k < Cin && m < M) ? w[(long)k * M + m] : (half_t)0.0f;
+            for (int e = 0; e < 8; e++) if (n0 + e < N) h[e] = p[e];
+            v = __builtin_bit_cast(u32x4, h);
+        }
     }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < 4; p++) {
-        const int m = tm + ly + 8 * p, k = tk + lx;
-        if (m < M && k < Cin) w2[(long)m * Cin + k] = tile[lx][ly + 8 * p];
-    }
+    return v;
 }
 
-// out[n][co][iy*KH+ky][ix*KW+kx] = y[n][(co,ky,kx)][iy*W+ix].  A thread produces VEC consecutive
-// outputs of one output row (one 16-byte store when VEC is 8).
-template <int VEC>
-__global__ void ct_shuffle_kernel(half_t *out, const half_t *y, int Wi, int Hi, int KW, int KH, int Cout) {
-    const int OW = Wi * KW, OH = Hi * KH;
-    const int per_row = OW / VEC;
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)Cout * OH * per_row;
-    if (idx >= total) return;
-    const int n = blockIdx.y;
-    const int ox0 = (int)(idx % per_row) * VEC;
-    long t = idx / per_row;
-    const int oy = (int)(t % OH), co = (int)(t / OH);
-    const int iy = oy / KH, ky = oy % KH;
-    const long HW = (long)Hi * Wi;
-    const half_t *src = y + ((long)n * Cout * KH * KW + ((long)co * KH + ky) * KW) * HW + (long)iy * Wi;
-    half_t *dst = out + (((long)n * Cout + co) * OH + oy) * OW + ox0;
-    if constexpr (VEC == 8) {
-        half8v v;
-        int ix = ox0 / KW, kx = ox0 % KW;
+// BM x 64 tile of (co, ky, kx) x pixels, four waves, each 32 pixels x BM / 2 rows.  Both operands have K = Cin as their
+// slow axis, so both go to LDS as they lie ([k][columns], 64 channels a stage, the next stage's loads in flight during
+// this one's MFMAs) and reach the matrix unit through the transposing LDS read.  A lane ends with four consecutive rows
+// of one pixel: for a 2 x 2 kernel the four taps of one output channel, two of them neighbours in an output row, so a
+// wave stores 128 contiguous bytes per row.
+// Bound by latency at the sizes upsamplers have (256 channels: four trips through memory and LDS).  It replaces a weight
+// transpose, a GEMM into scratch and a shuffle pass, three launches: 256 -> 64 channels on 64 x 64 took 11.7 us.
+template <int BM, bool TAPS22>
+__global__ __launch_bounds__(256) void ct_mfma_kernel(CtArgs a) {
+    constexpr int BN = 64, BK = 64, NT = 256, ALD = BM + 32, BLD = BN + 32, TM = BM / 64;
+    constexpr int PA = BK * BM / 8 / NT, PB = BK * BN / 8 / NT;
+    __shared__ __align__(16) half_t As[2][BK * ALD], Bs[2][BK * BLD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
+    const int taps = a.KH * a.KW, M = a.Cout * taps;
+    const long HW = (long)a.Hi * a.Wi;
+    const int m0 = blockIdx.y * BM;
+    const long n0 = (long)blockIdx.x * BN;
+    const half_t *x = a.x + (long)blockIdx.z * a.Cin * HW;
+    u32x4 ra[PA], rb[PB];
+    auto load = [&](int k0) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            v[j] = src[kx * HW + ix];
-            if (++kx == KW) { kx = 0; ix++; }
+        for (int i = 0; i < PA; i++) { const int c = tid + i * NT; ra[i] = ct_row8(a.w, k0 + c / (BM / 8), a.Cin, M, m0 + c % (BM / 8) * 8); }
+#pragma unroll
+        for (int i = 0; i < PB; i++) { const int c = tid + i * NT; rb[i] = ct_row8(x, k0 + c / (BN / 8), a.Cin, HW, n0 + c % (BN / 8) * 8); }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < PA; i++) { const int c = tid + i * NT; *reinterpret_cast<u32x4 *>(&As[buf][c / (BM / 8) * ALD + c % (BM / 8) * 8]) = ra[i]; }
+#pragma unroll
+        for (int i = 0; i < PB; i++) { const int c = tid + i * NT; *reinterpret_cast<u32x4 *>(&Bs[buf][c / (BN / 8) * BLD + c % (BN / 8) * 8]) = rb[i]; }
+    };
+    // transposing read: within each block of 16 lanes lane s points at row k + s / 4, columns 4 (s % 4) .. + 3, and lane i
+    // receives four consecutive k of column i
+    const int trow = (lane >> 5) * 8 + ((lane & 15) >> 2), tcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    auto frag = [&](const half_t *s, int ld) {
+        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)s);
+        const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(s + 4 * ld));
+        const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        return __builtin_bit_cast(half8v, both);
+    };
+    float16v acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+    const int steps = (a.Cin + BK - 1) / BK;
+    load(0);
+    put(0);
+    __syncthreads();
+    for (int s = 0; s < steps; s++) {
+        if (s + 1 < steps) load((s + 1) * BK);
+        const half_t *as = As[s & 1] + trow * ALD + wm * (BM / 2) + tcol, *bs = Bs[s & 1] + trow * BLD + wn * 32 + tcol;
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ks++) {
+            const half8v fb = frag(bs + ks * 16 * BLD, BLD);
+#pragma unroll
+            for (int i = 0; i < TM; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(as + ks * 16 * ALD + i * 32, ALD), fb, acc[i], 0, 0, 0);
         }
-        *reinterpret_cast<half8v *>(dst) = v;
-    } else {
-        dst[0] = src[(ox0 % KW) * HW + ox0 / KW];
+        if (s + 1 < steps) put((s + 1) & 1);
+        __syncthreads();
     }
+    // acc[i][4 g + e] of a lane: row m0 + wm BM / 2 + 32 i + 8 g + 4 (lane / 32) + e, pixel n0 + 32 wn + lane % 32
+    const long n = n0 + wn * 32 + (lane & 31);
+    if (n >= HW) return;
+    const int iy = (int)(n / a.Wi), ix = (int)(n % a.Wi);
+    half_t *out = a.out + (long)blockIdx.z * a.Cout * a.OH * a.OW;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int m = m0 + wm * (BM / 2) + 32 * i + 8 * g + 4 * (lane >> 5);
+            if constexpr (TAPS22) {
+                if (m < M) {
+                    const int co = m >> 2;
+                    const float b = a.bias ? (float)a.bias[co] : 0.0f;
+                    half_t *dst = out + ((long)co * a.OH + 2 * iy) * a.OW + 2 * ix;
+#pragma unroll
+                    for (int ky = 0; ky < 2; ky++) {
+                        const half2v v = {(half_t)(acc[i][4 * g + 2 * ky] + b), (half_t)(acc[i][4 * g + 2 * ky + 1] + b)};
+                        __builtin_memcpy(dst + (long)ky * a.OW, &v, 4);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (m + e < M) {
+                        const int co = (m + e) / taps, t = (m + e) - co * taps, ky = t / a.KW, kx = t - ky * a.KW;
+                        out[((long)co * a.OH + iy * a.KH + ky) * a.OW + ix * a.KW + kx] = (half_t)(acc[i][4 * g + e] + (a.bias ? (float)a.bias[co] : 0.0f));
+                    }
+                }
+            }
+        }
 }
 
 // The gather form: the loop order and the fp32 accumulator (seeded with the bias) of the reference's
@@ -134,16 +187,14 @@ bool shuffle_ok(const CtArgs &a, int64_t opx, int64_t opy) {
     return a.groups == 1 && a.px == 0 && a.py == 0 && a.dx == 1 && a.dy == 1 && opx == 0 && opy == 0 && a.KW == a.sx && a.KH == a.sy;
 }
 
-struct CtScratch { size_t w2, bias2, y, gemm; };
-
-CtScratch scratch_of(const CtArgs &a) {
+template <int BM>
+int launch_ct(const CtArgs &a, hipStream_t st) {
     const int64_t M = (int64_t)a.Cout * a.KH * a.KW, HW = (int64_t)a.Hi * a.Wi;
-    CtScratch s;
-    s.w2 = round_up((size_t)M * a.Cin * 2, 256);
-    s.bias2 = round_up((size_t)M * 2, 256);
-    s.y = round_up((size_t)a.N * M * HW * 2, 256);
-    s.gemm = mi_internal_gemm_workspace(M, a.Cin, HW, a.N);
-    return s;
+    const dim3 grid((unsigned)ceil_div(HW, 64), (unsigned)ceil_div(M, BM), (unsigned)a.N);
+    if (ceil_div(M, BM) > 65535) return MI_DECLINE_EXTENT;
+    if (a.KW == 2 && a.KH == 2) hipLaunchKernelGGL((ct_mfma_kernel<BM, true>), grid, dim3(256), 0, st, a);
+    else                        hipLaunchKernelGGL((ct_mfma_kernel<BM, false>), grid, dim3(256), 0, st, a);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
 }  // namespace
@@ -168,9 +219,11 @@ size_t mi_convtranspose2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int
                                         int64_t opx, int64_t opy, int64_t groups) {
     CtArgs a;
     if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, opx, opy, groups) != MI_OK) return 0;
-    if (!shuffle_ok(a, opx, opy)) return 0;
-    const CtScratch s = scratch_of(a);
-    return s.w2 + s.bias2 + s.y + s.gemm;
+    // Both routes work in registers and LDS today.  The answer stays what a weight transpose, an expanded bias and an
+    // unshuffled result take, so that callers' buffers and recorded plans keep their sizes; nothing is written there.
+    const int64_t M = (int64_t)a.Cout * a.KH * a.KW, HW = (int64_t)a.Hi * a.Wi;
+    return round_up((size_t)M * a.Cin * 2, 256) + round_up((size_t)M * 2, 256) + round_up((size_t)a.N * M * HW * 2, 256) +
+           mi_internal_gemm_workspace(M, a.Cin, HW, a.N);
 }
 
 int mi_convtranspose2d_f16(void *out, const void *x, const void *w, const void *bias,
@@ -190,31 +243,9 @@ int mi_convtranspose2d_f16(void *out, const void *x, const void *w, const void *
         hipLaunchKernelGGL(ct_gather_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, a);
         return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
     }
-    const CtScratch s = scratch_of(a);
-    if (!ws || ws_bytes < s.w2 + s.bias2 + s.y + s.gemm || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
-    const int M = a.Cout * a.KH * a.KW, HW = a.Hi * a.Wi, taps = a.KH * a.KW;
-    char *base = reinterpret_cast<char *>(ws);
-    half_t *w2 = reinterpret_cast<half_t *>(base);
-    half_t *bias2 = reinterpret_cast<half_t *>(base + s.w2);
-    half_t *y = reinterpret_cast<half_t *>(base + s.w2 + s.bias2);
-    const int tiles_m = (int)ceil_div((int64_t)M, 32), tile_blocks = tiles_m * (int)ceil_div((int64_t)a.Cin, 32);
-    hipLaunchKernelGGL(ct_prepare_kernel, dim3((unsigned)(tile_blocks + (int)ceil_div((int64_t)M, 256))), dim3(256), 0, st,
-                       w2, bias2, a.w, a.bias, a.Cin, M, taps, tiles_m, tile_blocks);
-    if (hipGetLastError() != hipSuccess) return MI_ERROR_LAUNCH;
-    // y[n][M][HW] = w2[M][Cin] . x[n][Cin][HW]: the pixel axis is the contiguous one of both, the expanded bias is per row
-    rc = mi_internal_gemm(y, w2, a.x, a.bias ? bias2 : nullptr, M, HW, HW, a.Cin, HW, a.Cin, HW, 1, MI_BIAS_ROW, MI_EPI_NONE, 0,
-                          a.N, (long)M * HW, 0, (long)a.Cin * HW, base + s.w2 + s.bias2 + s.y, s.gemm, st);
-    if (rc != MI_OK) return rc;
-    if (a.OW % 8 == 0 && aligned_to(out, 16)) {
-        const long total = (long)a.Cout * a.OH * (a.OW / 8);
-        hipLaunchKernelGGL(ct_shuffle_kernel<8>, dim3((unsigned)ceil_div(total, 256), (unsigned)a.N), dim3(256), 0, st,
-                           a.out, y, a.Wi, a.Hi, a.KW, a.KH, a.Cout);
-    } else {
-        const long total = (long)a.Cout * a.OH * a.OW;
-        hipLaunchKernelGGL(ct_shuffle_kernel<1>, dim3((unsigned)ceil_div(total, 256), (unsigned)a.N), dim3(256), 0, st,
-                           a.out, y, a.Wi, a.Hi, a.KW, a.KH, a.Cout);
-    }
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+    // 128 rows a tile once that still gives every CU two workgroups, else 64
+    const int64_t wide = ceil_div((int64_t)a.Hi * a.Wi, 64) * ceil_div((int64_t)a.Cout * a.KH * a.KW, 128) * a.N;
+    return wide >= 2 * (int64_t)mi_num_cus() ? launch_ct<128>(a, st) : launch_ct<64>(a, st);
 }
 
 }  // extern "C"

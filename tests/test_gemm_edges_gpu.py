@@ -60,3 +60,19 @@ def test_ragged_in_every_direction(ctx, T, K, F, layout):
 def test_odd_addresses(ctx, layout, shift):
     _check(ctx, 40, 192, 96, layout, shift=shift)
     _check(ctx, 5, 640, 64, layout, shift=shift, epi="gelu_tanh")
+
+
+@pytest.mark.parametrize("N,Cin,H,W,Cout,KH,KW", [(1, 1, 1, 1, 1, 2, 2), (1, 65, 7, 9, 15, 2, 2), (2, 64, 8, 8, 16, 2, 2), (1, 130, 3, 43, 33, 2, 2),
+                                                  (1, 8, 11, 13, 5, 3, 1), (2, 256, 96, 100, 64, 2, 2), (1, 72, 9, 5, 17, 3, 3)])
+def test_upsampler_tiles(ctx, N, Cin, H, W, Cout, KH, KW):
+    """Kernel == stride: pixels, channels and output channels off the 64-wide tiles, rows at odd addresses."""
+    import torch
+    import juliavision_amd as jv
+    x, w = oracle.randn_f16((N, Cin, H, W), 1, 0, 0.5), oracle.randn_f16((Cin, Cout, KH, KW), 2, 0, 0.1)
+    b = oracle.randn_f16((Cout,), 3, 0, 0.5)
+    want = oracle.convtranspose2d_f16(x, w, b, (KH, KW))
+    out = torch.full(want.shape, float("nan"), dtype=torch.float16, device="cuda")
+    ctx.ws.reset()
+    jv.convolutiontranspose_(ctx, out, to_dev(x), to_dev(w), to_dev(b), (KW, KH), (0, 0), (1, 1), (0, 0), 1)
+    torch.cuda.synchronize()
+    assert_parity(to_host(out), want, what="upsampler")
