@@ -204,7 +204,7 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
         tm_ = first + in % gsz;
         tn_ = in / gsz;
     } else {
-        tile_of(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, p.group_m, tm_, tn_);
+        tile_of(p, tm_, tn_);
     }
     // (the divisions above run on the vector unit: hand the results back to scalar registers, which the direct loads'
     // base addresses have to be in)
@@ -1186,9 +1186,7 @@ bool mfma_addressable(const GemmArgs &a, bool b_kn) {
 template <int BM, int BN, int WM, int WN>
 int launch_w4(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
     if (a.K < 64 || a.K % 64 || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
-    a.tiles_m = (int)ceil_div(a.M, BM);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
+    set_tiles(a, BM, BN);
     a.vec_store = rows_vec16(a);
     // per-lane load offsets are 32-bit byte offsets from the tile origin
     if ((int64_t)BM * a.ldA * 2 >= (1ll << 31) || (int64_t)(b_kn ? 64 : BN) * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
@@ -1236,6 +1234,7 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
+constexpr int RING_TILE = 5;             // index into TILE_MODELS: gemm_ring_kernel
 // tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
 // output, same bits, and the plan (hence the workspace) stays a function of the extents alone.
@@ -1244,6 +1243,12 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
     switch (tile) {
         case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : mi_pipe_launch(0, a, b_kn, nbatch, st);
         case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : mi_pipe_launch(1, a, b_kn, nbatch, st);
+        case RING_TILE:
+            if (!a.cv.xp && !a.ag.x) {
+                const int rc = mi_ring_launch(a, b_kn, nbatch, st);
+                if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
+            }
+            return mi_pipe_launch(4, a, b_kn, nbatch, st);
         default: return mi_pipe_launch(tile, a, b_kn, nbatch, st);
     }
 }
@@ -1256,7 +1261,7 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
 // the second launch (about 4 us) and the fp32 planes (0.25 us per MB).  Picking the cheapest estimate lands within
 // 1 % of the best measured choice on average over those shapes and within 6 % on 95 % of them.
 struct TileModel { int bm, bn; double step_lo, step_full, round, fixed; };
-constexpr int NTILES = 5;
+constexpr int NTILES = 6;
 constexpr TileModel TILE_MODELS[NTILES] = {
     // (the two tiles of the four-wave kernel, re-timed with it: 1500 x 5120 in 25.3 / 70.5 us at K = 1280 / 5120,
     // 512 x 1280 in 16.3 / 47.2; 1500 x 3840 on 192 x 128 in 20.2 / 55.4, 512 x 1280 in 13.5 / 39.9)
@@ -1265,8 +1270,14 @@ constexpr TileModel TILE_MODELS[NTILES] = {
     {128, 128, 0.428, 0.600, 1.00, 4.0},
     {64, 128, 0.318, 0.430, 0.90, 3.1},
     {64, 64, 0.235, 0.315, 0.73, 3.0},
+    // gemm_ring_kernel: timed over 2 to 256 workgroups and K 384 to 5120 (20 x 1280 -> 1280 tiles in 7.6 us, 128 workgroups
+    // over K = 4096 in 17.4).  Its sum of four partial tiles and deep ring cost a microsecond at the ends, so it starts past
+    // K = 512 -- where the layer-norm prologue's promise of identical bits ends too -- and above one workgroup per CU its
+    // LDS allows no second one: L2 bandwidth (19 to 24 TB/s) is what bounds it there in any case.
+    {64, 64, 0.125, 0.215, 1.00, 4.2},
 };
-struct TilePlan { int tile, split; bool peer; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
+constexpr int RING_KMIN = 513;
+struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split) {
     const TileModel &t = TILE_MODELS[tile];
@@ -1312,20 +1323,21 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split) {
-    TilePlan best = {4, 1, false};
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring) {
+    TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
     for (int split = 1; split <= max_split; split++) {
         if (K % (64 * split) != 0 || (split > 1 && K / split < 128)) continue;
         for (int tile = 0; tile < NTILES; tile++) {
+            if (tile == RING_TILE && (!ring || K / split < RING_KMIN || ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > mi_num_cus())) continue;
             const double us = tile_cost_us(M, N, K, nbatch, tile, split);
-            if (us < best_us) { best_us = us; best = {tile, split, false}; }
+            if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
         if (max_split > 1 && sk_planned()) {
             if (sk_fits(M, N, K, TILE_MODELS[SK_TILE].bm, TILE_MODELS[SK_TILE].bn, split)) {
                 const double us = sk_cost_us(M, N, K, SK_TILE, split);
-                if (us < best_us) { best_us = us; best = {SK_TILE, split, true}; }
+                if (us < best_us) { best_us = us; best = {SK_TILE, split, true, us}; }
             }
         }
     }
@@ -1334,14 +1346,14 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
 
 // The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
 // thread keeps the last answers.  The key holds everything the estimate reads.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split) {
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring = true) {
     struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
     static thread_local Entry table[256] = {};
-    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0);
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (ring ? 8 : 0);
     const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 40;
     Entry &e = table[(h >> 32) & 255];
     if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
-        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split)};
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, ring)};
     return e.plan;
 }
 
@@ -1470,7 +1482,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // second small kernel sums the planes and applies bias, activation and residual.
         const bool pipe = a.K > 64, whole = pipe && a.K % 64 == 0;
         if ((a.cv.xp || a.ag.x) && !whole) return MI_DECLINE_EXTENT;      // only the pipelined kernel gathers
-        TilePlan tp = {4, 1, false};
+        TilePlan tp = {4, 1, false, 0.0};
         // A folded norm on the way in or row statistics on the way out live in the tiled kernels' own store: those calls
         // need the pipelined kernels, 16-byte rows, and K-slices only in the form that ends in that store (the in-launch
         // exchange), never planes.
@@ -1598,7 +1610,7 @@ int mi_init(void) {
     bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<8, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= mi_pipe_init() | mi_any_init();
+    bad |= mi_pipe_init() | mi_ring_init() | mi_any_init();
     bad |= mi_sdpa_init();
     bad |= scratch_of_current_device() == nullptr;
     sk_probe_current_device();      // a device that fails the probe only loses that path
@@ -1665,7 +1677,9 @@ size_t mi_gemm_f16_workspace(int64_t T, int64_t K, int64_t F, int w_layout, int6
     if (T < 1 || nbatch > 1) return 0;
     if (T > 8) {
         if (K % 64 || K < 128) return 0;
-        return plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
+        // never less than the split that the plan takes without the ring kernel: buffers and recorded plans keep their sizes
+        const size_t need = plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F), other = plan_workspace_bytes(plan_tiles(T, F, K, 1, true, false), T, F);
+        return need > other ? need : other;
     }
     if (w_layout != MI_W_KF) return 0;      // the [F][K] skinny kernel finishes its outputs itself
     return round_up((size_t)skinny_splits(K, F) * T * F * sizeof(float), 256);

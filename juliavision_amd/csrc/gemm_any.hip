@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
     half_t *As = reinterpret_cast<half_t *>(smem) + group * GROUP, *Bs = As + 2 * BM * LD;
     const int wm = wave & 1, wn = wave >> 1;
     int tm_, tn_;
-    tile_of(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, p.group_m, tm_, tn_);
+    tile_of(p, tm_, tn_);
     const int m0 = tm_ * BM, n0 = tn_ * BN;
     const long bz = blockIdx.y;
     const half_t *A = p.A + bz * p.sA, *B = p.B + bz * p.sB;
@@ -152,9 +152,7 @@ constexpr int any_lds_bytes() { return KG * 2 * (BM + BN) * 72 * 2; }
 
 template <int BM, int BN, int KG, bool ALIGNED>
 int launch_any(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    a.tiles_m = (int)ceil_div(a.M, BM);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
+    set_tiles(a, BM, BN);
     a.vec_store = rows_vec16(a);
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
     constexpr int lds = any_lds_bytes<BM, BN, KG>();

@@ -17,6 +17,7 @@ struct GemmArgs {
     long sY, sA, sB, sBias; // batch strides (elements)
     int bias_mode, epi, out_f32;
     int tiles_m, tiles_n, group_m;
+    unsigned div_width, div_group, div_last;      // tile_of's divisions as multiplications (set_tiles)
     int vec_store;          // Y (and residual) rows allow 16-byte accesses
     ConvGather cv;          // cv.xp != nullptr: B is the im2col matrix of a convolution, gathered on the fly
     NhwcGather ag;          // ag.x != nullptr: A is the patch matrix of a channels-last convolution, gathered on the fly
@@ -159,16 +160,44 @@ __device__ __forceinline__ void static_for(F &&f) {
 // round-robin over the 8 XCDs, each with its own L2; this hands every XCD one
 // contiguous run of the tile order, and the tile order walks GROUP_M row tiles
 // per column tile so a run reuses a small set of A and B panels.
-__device__ __forceinline__ void tile_of(int pid, int nwg, int tiles_m, int tiles_n, int group_m, int &tm, int &tn) {
-    int xcd = pid & 7, idx = pid >> 3;
-    int full = nwg >> 3, rem = nwg & 7;
-    int logical = xcd * full + min(xcd, rem) + idx;
-    int width = group_m * tiles_n;
-    int g = logical / width, in = logical - g * width;
-    int first = g * group_m;
-    int gsz = min(tiles_m - first, group_m);
-    tm = first + in % gsz;
-    tn = in / gsz;
+// Its divisions are multiplications by reciprocals the host worked out (set_tiles): a division is some thirty vector
+// instructions at eight clocks each, and three of them in a row stood between a launch and its first load.
+__device__ __forceinline__ void tile_of(const GemmArgs &p, int &tm, int &tn) {
+    const int pid = blockIdx.x, nwg = gridDim.x;
+    const int xcd = pid & 7, idx = pid >> 3;
+    const int full = nwg >> 3, rem = nwg & 7;
+    const int logical = xcd * full + min(xcd, rem) + idx;
+    const int width = p.group_m * p.tiles_n;
+    const auto over = [](int x, unsigned recip) { return recip ? (int)__umulhi((unsigned)x, recip) : x; };
+    int g, in, first, gsz;
+    if (p.div_width != 1) {
+        g = over(logical, p.div_width);
+        in = logical - g * width;
+        first = g * p.group_m;
+        gsz = min(p.tiles_m - first, p.group_m);
+        tn = over(in, gsz == p.group_m ? p.div_group : p.div_last);
+    } else {                                              // a grid too large for 32-bit reciprocals
+        g = logical / width;
+        in = logical - g * width;
+        first = g * p.group_m;
+        gsz = min(p.tiles_m - first, p.group_m);
+        tn = in / gsz;
+    }
+    tm = first + in - tn * gsz;
+}
+
+// The tile grid of a launch.  ceil(2^32 / d) divides x exactly while x d < 2^32; 0 stands for d = 1, and 1 as div_width for
+// a grid beyond that.
+inline void set_tiles(GemmArgs &a, int bm, int bn) {
+    a.tiles_m = (int)ceil_div(a.M, bm);
+    a.tiles_n = (int)ceil_div(a.N, bn);
+    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
+    const auto recip = [](int d) { return d <= 1 ? 0u : (unsigned)(((1ull << 32) + (unsigned)d - 1) / (unsigned)d); };
+    const int last = a.tiles_m % a.group_m;
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n, width = (int64_t)a.group_m * a.tiles_n;
+    a.div_width = tiles * width < (1ll << 32) ? recip((int)width) : 1u;
+    a.div_group = recip(a.group_m);
+    a.div_last = recip(last ? last : a.group_m);
 }
 
 // What the store of a folded norm needs, fetched while the first operand tiles are on their way and parked in `slot`
@@ -629,6 +658,9 @@ int mi_pipe_launch(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipSt
 int mi_pipe_launch_ln(bool wide, const GemmArgs &a, bool b_kn, hipStream_t st);
 constexpr int MI_LNA_KMAX = 512;         // deepest K of the layer-norm prologue
 int mi_pipe_init();
+// gemm_ring.hip: small grids of ordinary operands.
+int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
+int mi_ring_init();
 // gemm_any.hip: the kernels for operands and extents that the others do not take.
 int mi_any_launch(const GemmArgs &a, bool b_kn, bool addressable, int64_t nbatch, hipStream_t st);
 int mi_any_init();

@@ -43,13 +43,13 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void gemm_pipe_kernel(Gem
     static_assert(PA >= 1 && PB >= 1, "tile too small for this workgroup");
     constexpr int BSZ = B_KN ? BK * BLD : BN * LD;      // halves per B buffer
     extern __shared__ __align__(16) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     half_t *As = reinterpret_cast<half_t *>(smem);   // [2][BM][LD]; AMODE 2: the normalised panel [BM][K + 8]
     const int KP = p.K + 8;                          // panel row (halves): 16 bytes off a multiple of 128, like LD
     half_t *Bs = As + (LNA ? BM * KP : 2 * BM * LD); // [2][BN][LD] or [2][BK][BLD]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WAVES_M, wn = wave / WAVES_M;
     int tm_, tn_;
-    tile_of(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, p.group_m, tm_, tn_);
+    tile_of(p, tm_, tn_);
     const int m0 = tm_ * BM, n0 = tn_ * BN;
     const long bz = blockIdx.y;
     const half_t *A = p.A + bz * p.sA;
@@ -323,9 +323,7 @@ template <int BM, int BN, int WM, int WN>
 int launch_pipe(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
     // the kernel always walks at least two 64-deep tiles (its prologue fetches two ahead): one tile would read past K
     if (a.K <= 64 || a.K % 8) return MI_DECLINE_EXTENT;
-    a.tiles_m = (int)ceil_div(a.M, BM);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
+    set_tiles(a, BM, BN);
     a.vec_store = rows_vec16(a);
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
     constexpr int lds = gemm_lds_bytes<BM, BN, 64>();
@@ -363,9 +361,7 @@ constexpr int lna_lds_bytes(int K) {
 template <int BN, int WM, int WN>
 int launch_pipe_ln(GemmArgs a, bool b_kn, hipStream_t st) {
     if (a.K < 128 || a.K % 64 || a.K > MI_LNA_KMAX || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
-    a.tiles_m = (int)ceil_div(a.M, 64);
-    a.tiles_n = (int)ceil_div(a.N, BN);
-    a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
+    set_tiles(a, 64, BN);
     a.vec_store = rows_vec16(a);
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1);
     const int lds = lna_lds_bytes<BN, WM, WN>(a.K);

@@ -1,0 +1,310 @@
+// fp16 GEMM for gfx950, 64 x 64 wave tiles over a ring of direct-to-LDS stages: grids too small for the four-wave kernel.
+#include "gemm_common.hpp"
+
+// Sixteen zero bytes for loads of chunks past the end of K.
+static __device__ __align__(16) unsigned ring_zero_words[4];
+
+namespace {
+
+// A workgroup owns a 64 WM x 64 WN tile; its WM x WN x WK waves each hold a 64 x 64 sub-tile of accumulators, WK of them the
+// same one: wave wk takes 4 / WK of the four 16-deep steps of every 64-deep tile of K, and the WK partial tiles are summed
+// through LDS before the store.
+//
+// What bounds such a tile is the CU's LDS and vector-memory path, not the matrix cores.  Per 64-deep tile a 64 x 64 tile
+// takes 256 clocks of 64 B/clock loads and 128 clocks of MFMAs; four 32 x 32 waves (gemm_pipe_kernel) move 16 KB into LDS
+// through registers and read 32 KB of fragments, 384 LDS clocks, and were measured at 480 to 600.  Waves that split K
+// instead of the tile read each fragment once: 16 KB in, 16 KB out, and the loads bypass the registers
+// (global_load_lds_dwordx4), S stages deep, so that a trip to memory is S - 2 tiles long.
+//
+// LDS layout of a stage: A rows of 128 bytes, then B ([N][K]: rows of 128 bytes; [K][N]: 64 rows of BN halves).  Direct loads
+// cannot pad, so 16-byte chunks are permuted inside their row: K-contiguous row r holds chunk c at c ^ (r % 8 ^ r / 8 % 2),
+// [K][N] row k holds chunk c at c ^ (k % 4 * BN / 32) -- the four rows of a transposing read in four bank groups.
+// Chunks past K are read from a page of zeros, so K needs only to be a multiple of 8.
+template <int WM, int WN, int WK, int S, bool B_KN>
+__global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
+    constexpr int BM = 64 * WM, BN = 64 * WN, BK = 64, NW = WM * WN * WK, NT = NW * 64, KS = 4 / WK;
+    constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
+    constexpr int STAGE_BYTES = SLOTS * 1024, A_BYTES = SLOTS_A * 1024;
+    static_assert(S >= 3, "a stage being read, one landed, one on its way");
+    extern __shared__ __align__(16) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wmn = wave / WK, wm = wmn % WM, wn = wmn / WM;
+    int tm_, tn_;
+    tile_of(p, tm_, tn_);
+    const int m0 = __builtin_amdgcn_readfirstlane(tm_ * BM), n0 = __builtin_amdgcn_readfirstlane(tn_ * BN);
+    const long bz = blockIdx.y;
+    const int nk = (p.K + BK - 1) / BK;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
+
+    auto barrier = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    if (wave >= NW) {
+        // The loaders, one for each operand.  A matrix wave that issued its share of the requests stood at those instructions
+        // with its products behind them (800 clocks a 64 x 64 tile), and a loader is quick only if a request costs it next
+        // to nothing: a wave issues an instruction every four to eight clocks, so the lane's byte offset from the tile's
+        // origin is fixed, the origin and the LDS address move in scalar registers, and the steady state has no branch.
+        auto load_all = [&](auto ROLE) {
+            constexpr bool IS_A = decltype(ROLE)::value;
+            constexpr int LPW = IS_A ? SLOTS_A : SLOTS - SLOTS_A;      // 1 KB requests of a tile
+            static_assert((S - 2) * LPW <= 63, "vmcnt is a 6-bit counter");
+            uint32_t off[LPW];
+            int kpos[LPW];                                // first k of the lane's chunk
+            // Request i covers rows 8 i .. 8 i + 7 (K-contiguous) or 512 / BN k-rows; the permutation has period two in i, so
+            // inside the operand an offset is one of two plus i times a constant.
+            constexpr bool ROWS = IS_A || !B_KN;
+            const int pos = lane & 7, sub = lane >> 3;
+            const long ld2 = (IS_A ? p.ldA : p.ldB) * 2;
+            if (ROWS) {
+                const int r0 = IS_A ? m0 : n0, rows = IS_A ? p.M : p.N, c = pos ^ sub;
+                const uint32_t even = (uint32_t)(sub * ld2) + c * 16, odd = even + ((c ^ 1) - c) * 16, step8 = (uint32_t)(8 * ld2);
+                const bool inside = r0 + (IS_A ? BM : BN) <= rows;                    // uniform
+#pragma unroll
+                for (int i = 0; i < LPW; i++) {
+                    off[i] = ((i & 1) ? odd : even) + i * step8;
+                    if (!inside) off[i] = (uint32_t)((min(r0 + 8 * i + sub, rows - 1) - r0) * ld2) + (c ^ (i & 1)) * 16;
+                    kpos[i] = (c ^ (i & 1)) * 8;
+                }
+            } else {
+                constexpr int CPR = BN / 8, PER = 64 / CPR;                           // chunks of a k-row, k-rows of a request
+                const int k = lane / CPR, c = (lane % CPR) ^ ((k & 3) * (BN / 32));
+                // columns past the edge re-read the last chunk
+                const uint32_t first = (uint32_t)(k * ld2) + max(0, min(c * 8, p.NB - 8 - n0)) * 2, stepk = (uint32_t)(PER * ld2);
+                static_assert(PER % 4 == 0, "a request's k-rows start on a multiple of four");
+#pragma unroll
+                for (int i = 0; i < LPW; i++) {
+                    off[i] = first + i * stepk;
+                    kpos[i] = k + i * PER;
+                }
+            }
+            const char *org = IS_A ? reinterpret_cast<const char *>(p.A + bz * p.sA + (long)m0 * p.ldA)
+                                   : reinterpret_cast<const char *>(p.B + bz * p.sB + (B_KN ? (long)n0 : (long)n0 * p.ldB));
+            const long step = IS_A || !B_KN ? BK * 2 : (long)BK * p.ldB * 2;
+            const uint32_t lds1 = lds0 + (IS_A ? 0 : A_BYTES);
+            int next = 0;                                 // the tile requested next, and its stage
+            uint32_t stage = 0;
+            auto request = [&]() {
+                if ((next + 1) * BK <= p.K) {             // uniform
+                    asm volatile("s_mov_b32 m0, %0" ::"s"(lds1 + stage) : "memory");
+#pragma unroll
+                    for (int i = 0; i < LPW; i++)
+                        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_add_u32 m0, m0, 0x400" ::"v"(off[i]), "s"(org) : "memory", "scc");
+                } else {                                  // the tile that K ends in: chunks past it come from the zeros
+#pragma unroll
+                    for (int i = 0; i < LPW; i++) {
+                        const char *from = next * BK + kpos[i] < p.K ? org + off[i] : reinterpret_cast<const char *>(ring_zero_words);
+                        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds1 + stage + i * 1024) : "memory");
+                    }
+                }
+                org += step;
+                next++;
+                stage = stage == (S - 1) * STAGE_BYTES ? 0u : stage + STAGE_BYTES;
+            };
+            // all but the newest `newer` tiles' requests have landed
+            auto landed = [&](int newer) {
+                switch (newer) {
+                case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+                case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory"); break;
+                case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S > 3 ? 2 * LPW : 0) : "memory"); break;
+                case 3: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S > 4 ? 3 * LPW : 0) : "memory"); break;
+                case 4: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S > 5 ? 4 * LPW : 0) : "memory"); break;
+                case 5: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S > 6 ? 5 * LPW : 0) : "memory"); break;
+                default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S > 7 ? 6 * LPW : 0) : "memory"); break;
+                }
+            };
+            static_assert(S <= 8, "landed() counts to six");
+            const int ahead = min(S - 1, nk);
+            for (int kt = 0; kt < ahead; kt++) request();
+            landed(ahead - 1);
+            barrier();                                    // tile 0 has landed
+            int kt = 0;
+            for (; next < nk; kt++) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 3) * LPW) : "memory");      // tile kt + 1 has landed
+                barrier();
+                request();
+            }
+            for (; kt + 1 < nk; kt++) {
+                landed(nk - (kt + 2));
+                barrier();
+            }
+        };
+        if (wave == NW) load_all(std::true_type{});
+        else load_all(std::false_type{});
+        return;
+    }
+
+    // fragment addresses: step ks of a tile is step ks of this wave's KS (all four when WK == 1)
+    const int frow = lane & 31, h = lane >> 5, aswz = (frow & 7) ^ ((frow >> 3) & 1);
+    uint32_t aoff[KS], boff[KS], noff[2];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        const int ks = wk * KS + s;
+        aoff[s] = (uint32_t)((wm * 64 + frow) * 128 + (((2 * ks + h) ^ aswz) * 16));
+        if constexpr (!B_KN) boff[s] = (uint32_t)(A_BYTES + (wn * 64 + frow) * 128 + (((2 * ks + h) ^ aswz) * 16));
+        else boff[s] = (uint32_t)(A_BYTES + (ks * 16 + h * 8 + ((lane & 15) >> 2)) * BN * 2);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int n = wn * 64 + i * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4, k3 = (lane & 15) >> 2;
+        noff[i] = (uint32_t)((((n >> 3) ^ (k3 * (BN / 32))) * 16) + (n & 7) * 2);
+    }
+    half8v fa[2][KS][2], fb[2][KS][2];
+    auto fetch = [&](auto SET, int kt) {
+        constexpr int set = decltype(SET)::value;
+        const char *st = smem + (kt % S) * STAGE_BYTES;
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) fa[set][s][j] = *reinterpret_cast<const half8v *>(st + aoff[s] + j * 32 * 128);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if constexpr (!B_KN) fb[set][s][i] = *reinterpret_cast<const half8v *>(st + boff[s] + i * 32 * 128);
+                else {
+                    const char *b = st + boff[s] + noff[i];
+                    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)b);
+                    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(b + 4 * BN * 2));
+                    const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    fb[set][s][i] = __builtin_bit_cast(half8v, both);
+                }
+            }
+        }
+    };
+    float16v acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    auto products = [&](auto SET) {
+        constexpr int set = decltype(SET)::value;
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][s][i], fa[set][s][j], acc[i][j], 0, 0, 0);
+    };
+
+    // what the store needs of memory, while the first tiles are on their way
+    constexpr int KEEP = WK > 1 ? 4 / WK : 2, STN = WK == 4 ? 32 : 64;       // 32-column blocks a wave stores, columns of its sub-tile
+    const int sm = WK == 1 ? wm : wm * 2 + (WK == 4 ? wk & 1 : wk), sn = WK == 4 ? wn * 2 + (wk >> 1) : wn;
+    half4v cb[KEEP][4];
+    load_col_bias<KEEP, STN>(p, cb, n0, sn, lane, bz);
+    float2v *ln_slot = reinterpret_cast<float2v *>(smem + S * STAGE_BYTES);
+    lnf_stage<BM, BN, NT>(p, ln_slot, m0, n0, bz, tid);
+    barrier();
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    fetch(I0{}, 0);
+    // Tile kt's fragments are in registers (or on their way) when its turn comes: past the barrier its successor has landed and
+    // its predecessor's stage is free for the loaders; the successor's fragments are requested, then its products issued.
+    auto turn = [&](auto SET, auto NEXT, int kt) {
+        if (kt + 1 < nk) {
+            barrier();
+            fetch(NEXT, kt + 1);
+        }
+        products(SET);
+    };
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+        turn(I0{}, I1{}, kt);
+        turn(I1{}, I0{}, kt + 1);
+    }
+    if (kt < nk) turn(I0{}, I1{}, kt);
+
+    barrier();                                            // every wave has read its last fragments
+    LnFold<2> ln2;
+    if constexpr (WK > 1) {
+        // wave wk keeps blocks: WK == 4: (i, j) = (wk / 2, wk % 2); WK == 2: j == wk, both i.  Partial tiles go to LDS by
+        // owner and are added in wave order.
+        float *part = reinterpret_cast<float *>(smem) + wmn * WK * (WK - 1) * KEEP * 1024;
+#pragma unroll
+        for (int o = 0; o < WK; o++) {
+            if (o != wk) {
+                const int from = wk < o ? wk : wk - 1;
+#pragma unroll
+                for (int b = 0; b < KEEP; b++) {
+                    const float16v v = WK == 4 ? acc[o >> 1][o & 1] : acc[b][o];
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; r4++) {
+                        const float4v q = {v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]};
+                        *reinterpret_cast<float4v *>(part + ((o * (WK - 1) + from) * KEEP + b) * 1024 + r4 * 256 + lane * 4) = q;
+                    }
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier();
+        float16v own[KEEP][1];
+#pragma unroll
+        for (int b = 0; b < KEEP; b++) {
+            float16v mine = acc[0][0];
+#pragma unroll
+            for (int o = 0; o < WK; o++) if (o == wk) mine = WK == 4 ? acc[o >> 1][o & 1] : acc[b][o];
+#pragma unroll
+            for (int r = 0; r < 16; r++) own[b][0][r] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < WK; s++) {
+                if (s == wk) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) own[b][0][r] += mine[r];
+                } else {
+                    const int from = s < wk ? s : s - 1;
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; r4++) {
+                        const float4v q = *reinterpret_cast<const float4v *>(part + ((wk * (WK - 1) + from) * KEEP + b) * 1024 + r4 * 256 + lane * 4);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) own[b][0][4 * r4 + e] += q[e];
+                    }
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier();                                        // the store's staging reuses the partial tiles' memory
+        LnFold<1> ln;
+        if (p.lnf_stats) {
+            const float2v v = ln_slot[sm * 32 + frow];
+            ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
+        }
+        store_tile<1, KEEP, 32, STN, NW, S * STAGE_BYTES>(p, own, cb, smem, m0, n0, sm, sn, wave, lane, bz, ln);
+    } else {
+        if (p.lnf_stats) {
+            ln2.on = true; ln2.col = reinterpret_cast<const float *>(ln_slot + BM); ln2.bn = BN;
+#pragma unroll
+            for (int j = 0; j < 2; j++) { const float2v v = ln_slot[wm * 64 + 32 * j + frow]; ln2.r[j] = v[0]; ln2.rmu[j] = v[1]; }
+        }
+        store_tile<2, 2, 64, 64, NW, S * STAGE_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln2);
+    }
+}
+
+template <int WM, int WN, int S>
+constexpr int ring_lds_bytes() { return S * (WM + WN) * 8192 + (WM + WN) * 64 * 8; }
+
+template <int WM, int WN, int WK, int S>
+int launch_ring(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
+    set_tiles(a, 64 * WM, 64 * WN);
+    a.vec_store = rows_vec16(a);
+    // per-lane load offsets are 32-bit byte offsets from the tile's origin
+    if ((int64_t)64 * WM * a.ldA * 2 >= (1ll << 31) || (int64_t)64 * (b_kn ? 1 : WN) * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
+    constexpr int lds = ring_lds_bytes<WM, WN, S>();
+    if (b_kn) hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, WK, S, true>), grid, dim3(WM * WN * WK * 64 + 128), lds, st, a);
+    else      hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, WK, S, false>), grid, dim3(WM * WN * WK * 64 + 128), lds, st, a);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
+template <int WM, int WN, int WK, int S>
+int raise_ring() {
+    return raise_lds(gemm_ring_kernel<WM, WN, WK, S, true>, ring_lds_bytes<WM, WN, S>()) | raise_lds(gemm_ring_kernel<WM, WN, WK, S, false>, ring_lds_bytes<WM, WN, S>());
+}
+
+}  // namespace
+
+int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) { return launch_ring<1, 1, 4, 8>(a, b_kn, nbatch, st); }
+
+int mi_ring_init() {
+    return raise_ring<1, 1, 4, 8>();
+}
