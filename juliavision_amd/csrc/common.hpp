@@ -178,3 +178,5 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
                      const ConvGather *gather = nullptr, const NhwcGather *agather = nullptr, const void *residual = nullptr);
 // Workspace bytes such a call needs (fp32 planes when it splits K); T > 8 rows.
 size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatch);
+// What such a call is estimated to take, in microseconds.
+double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);

@@ -8,16 +8,9 @@
 //   otherwise                   : im2col into scratch, then the same GEMM
 //                                 (conv_coopmat.jl:246-392)
 //   groups != 1                 : the direct kernel (conv.jl:26-51,298-302)
-#include "common.hpp"
+#include "conv_common.hpp"
 
 namespace {
-
-struct ConvArgs {
-    const half_t *x, *w, *bias;
-    void *out;
-    int Wi, Hi, Cin, N, KW, KH, Cout, OW, OH;
-    int sx, sy, px, py, dx, dy, groups, relu;
-};
 
 // wp[co][CRSP] = w[co][CRS] zero-padded: the blocks of an im2col launch past its own work do this (image 0 only), so
 // that padding the weights to the matrix's depth is not a launch of its own.
@@ -276,6 +269,17 @@ int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
         // PQ % 8 == 0 for 16-byte loads, otherwise the scalar GEMM takes it.
         return mi_internal_gemm(out, w, x, bias, a.Cout, PQ, PQ, a.Cin, PQ, a.Cin, PQ, 1, MI_BIAS_ROW, epi, 0,
                                 a.N, (long)a.Cout * PQ, 0, (long)a.Cin * PQ, nullptr, 0, st);
+    }
+    // In one launch where that is estimated to be faster than staging the operand and multiplying it: im2col writes at 0.8 to
+    // 1.1 MB/us, slower where it gathers with a stride (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: 43 us staged,
+    // 25 us in one launch; 144 -> 96 on 45 x 392: 45 and 26), the padded copies of the implicit form take a launch of 4 us.
+    {
+        int64_t PQP, CRSP;
+        im2col_extents(a, PQP, CRSP);
+        const double gemm = mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N);
+        const double staged = path == MI_CONV_IMPLICIT_GEMM ? 5.0 + 1.2 * gemm : 3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + gemm;
+        rc = mi_conv_tile(a, staged, st);
+        if (rc != MI_DECLINE_EXTENT) return rc;
     }
     if (path == MI_CONV_IMPLICIT_GEMM) {
         int Hp, Wp;

@@ -7,6 +7,7 @@
 //   A is K-contiguous.  B is either N-contiguous [K][N] (B_KN) or K-contiguous
 //   [N][K].  For a linear layer M = tokens, N = features, A = X, B = W.
 #include "gemm_common.hpp"
+#include "conv_common.hpp"
 #include "sk_exchange.hpp"
 #include <atomic>
 
@@ -1556,6 +1557,8 @@ size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatc
     return plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
 }
 
+double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return plan_tiles(T, F, K, nbatch, nbatch == 1).us; }
+
 // Internal entry used by the convolution path (conv.hip): Y[M x N] = A . B with
 // every GemmArgs field meaningful.
 int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, int M, int N, int NB, int K,
@@ -1610,7 +1613,7 @@ int mi_init(void) {
     bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<8, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= mi_pipe_init() | mi_ring_init() | mi_any_init();
+    bad |= mi_pipe_init() | mi_ring_init() | mi_any_init() | mi_conv_tile_init();
     bad |= mi_sdpa_init();
     bad |= scratch_of_current_device() == nullptr;
     sk_probe_current_device();      // a device that fails the probe only loses that path

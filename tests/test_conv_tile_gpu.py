@@ -1,0 +1,38 @@
+"""The one-launch convolution at the edges of its tiles: pixel rectangles, channel chunks, output-channel tiles, borders."""
+import numpy as np
+import pytest
+
+import oracle
+from util import assert_parity, poison, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,Cin,H,W,Cout,KH,KW,s,p,d,act", [
+    (1, 1, 1, 1, 1, 3, 3, 1, 1, 1, "none"),                # one output, all border
+    (1, 3, 30, 29, 33, 7, 7, 4, 3, 1, "relu"),             # few channels in one chunk, channels off the 32-wide tile
+    (2, 17, 13, 9, 65, 3, 3, 1, 1, 1, "none"),             # a last chunk of one channel
+    (1, 64, 31, 33, 96, 3, 3, 2, 1, 1, "relu"),
+    (1, 70, 8, 8, 32, 5, 5, 1, 2, 1, "none"),
+    (1, 96, 40, 200, 64, 5, 5, 1, 2, 1, "none"),           # whole rounds of large tiles
+    (1, 32, 12, 50, 160, 3, 1, (1, 2), (0, 1), (3, 1), "none"),
+    (1, 16, 9, 300, 24, 1, 9, (2, 1), (4, 0), (1, 2), "none"),
+    (4, 256, 15, 8, 256, 3, 3, 1, 1, 1, "relu"),           # long K, few pixels
+    (1, 128, 64, 64, 256, 3, 3, 1, 1, 1, "none"),
+    (1, 3, 260, 261, 144, 7, 7, 4, 3, 1, "none"),
+    (1, 384, 5, 5, 384, 3, 3, 1, 0, 1, "none"),
+])
+def test_conv_tiles(ctx, N, Cin, H, W, Cout, KH, KW, s, p, d, act):
+    import torch
+    import juliavision_amd as jv
+    pair = lambda v: v if isinstance(v, tuple) else (v, v)
+    s, p, d = pair(s), pair(p), pair(d)                    # (x, y)
+    x = oracle.randn_f16((N, Cin, H, W), 1)
+    w = oracle.randn_f16((Cout, Cin, KH, KW), 2, 0, 1.0 / np.sqrt(Cin * KH * KW))
+    b = oracle.randn_f16((Cout,), 3, 0, 0.5)
+    want = oracle.conv2d_f16(x, w, b, s[::-1], p[::-1], d[::-1], 1, act == "relu")
+    out = poison(torch.empty(want.shape, dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.convolution_(ctx, out, to_dev(x), to_dev(w), to_dev(b), s, p, d, 1, act=act)
+    torch.cuda.synchronize()
+    assert_parity(to_host(out), want, what=f"conv {Cin},{H},{W}->{Cout} k{KH}x{KW}")
