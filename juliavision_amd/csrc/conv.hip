@@ -372,16 +372,8 @@ int mi_conv2d_tokens_f16(void *out, int64_t ld_out, int64_t out_image_stride,
     if (hipGetLastError() != hipSuccess) return MI_ERROR_LAUNCH;
     const int epi = a.relu ? MI_EPI_RELU : MI_EPI_NONE;
     void *gws = reinterpret_cast<char *>(ws) + col_bytes + wp_bytes;
-    // the residual is addressed like the output; images whose residuals lie at another distance go one launch each
-    const bool together = !residual || N == 1 || res_image_stride == out_image_stride;
-    for (int64_t n = 0; n < (together ? 1 : N); n++) {
-        half_t *yo = reinterpret_cast<half_t *>(out) + n * out_image_stride;
-        const half_t *ro = residual ? reinterpret_cast<const half_t *>(residual) + n * res_image_stride : nullptr;
-        rc = mi_internal_gemm(yo, col + n * PQ * CRSP, wuse, bias, (int)PQ, a.Cout, a.Cout, (int)CRSP, ld_out, CRSP, CRSP, 0, MI_BIAS_COL, epi, 0,
-                              together ? N : 1, out_image_stride, PQ * CRSP, 0, gws, gemm_bytes, st, nullptr, nullptr, ro);
-        if (rc != MI_OK) return rc;
-    }
-    return MI_OK;
+    return mi_internal_gemm(out, col, wuse, bias, (int)PQ, a.Cout, a.Cout, (int)CRSP, ld_out, CRSP, CRSP, 0, MI_BIAS_COL, epi, 0,
+                            N, out_image_stride, PQ * CRSP, 0, gws, gemm_bytes, st, nullptr, nullptr, residual, res_image_stride - out_image_stride);
 }
 
 // Channels-last convolution as an implicit GEMM with nothing staged: out[(n,oh,ow)][Cout] = patch[(n,oh,ow)][(kh,kw,ci)] .

@@ -291,7 +291,7 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
         // beside the K loop instead: tile kt covers segments 2 kt and 2 kt + 1 (K % 64 == 0), so between two barriers
         // it takes in the two segments of each of its BM / 64 rows that it requested four tiles earlier, and the
         // result is in the LDS slot when it arrives at the last barrier, which the matrix waves pass before they
-        // store.  Same arithmetic, in the same order per row, as lnf_stage with one lane a row.
+        // store.  Same arithmetic, in the same order per row, as LnfLoader with one lane a row.
         constexpr int NR = BM / 64, AHEAD = 4;
         static_assert(BM % 64 == 0 && NR * 2 * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
         for (int t = lane; t < BN / 2; t += 64) {
@@ -360,7 +360,12 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
         return;
     }
     // (a launch without the statistics wave and with a folded norm: combine in the prologue, as the other kernels do)
-    if (blockDim.x < 384) lnf_stage<BM, BN, 256>(p, ln_slot, m0, n0, bz, tid);
+    if (blockDim.x < 384 && p.lnf_stats) {                          // no statistics wave: in front of the K loop
+        LnfLoader<BM, BN, 256, 16> lnf;
+        lnf.request(p, m0, n0, bz, tid);
+        lnf.combine(p, ln_slot, m0, tid);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
 
     // fragment read offsets inside a stage (bytes): rows of A, and this wave's columns of B in either layout
     const int frow = lane & 31, fhi = lane >> 5;
@@ -1447,7 +1452,7 @@ int fill_args(GemmArgs &a, void *Y, const void *X, const void *W, const void *bi
     a.bias = bias_mode == MI_BIAS_NONE ? nullptr : (const half_t *)bias;
     a.residual = (const half_t *)residual;
     a.M = (int)T; a.N = (int)F; a.K = (int)K; a.NB = (int)F;
-    a.ldY = ldY; a.ldA = ldX; a.ldB = ldW; a.sY = sY; a.sA = sX; a.sB = sW; a.sBias = sBias;
+    a.ldY = ldY; a.ldA = ldX; a.ldB = ldW; a.sY = sY; a.sA = sX; a.sB = sW; a.sBias = sBias; a.dRes = 0;
     a.bias_mode = bias_mode; a.epi = epi; a.out_f32 = out_dtype == MI_F32;
     a.tiles_m = a.tiles_n = a.group_m = 1; a.vec_store = 0;
     a.cv = ConvGather{};
@@ -1531,6 +1536,11 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)ceil_div(quads, 256)), dim3(256), 0, st, s2, planes, split);
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
+        // A GELU store is some fifteen vector instructions a value: where 128 x 128 tiles leave half the chip without one, 64 x 128
+        // tiles spread it (1370 x 384 -> 1536 inside a ViT block: 2 us of 11; at 204 of 256 workgroups the wide tile is the
+        // faster again).  Every pipelined tile sums K in the same order, so the bits do not change.
+        if (tp.tile == 2 && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH) && ceil_div(a.M, 128) * ceil_div(a.N, 128) * nbatch * 8 <= (int64_t)mi_num_cus() * 5)
+            tp.tile = 3;
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
@@ -1564,7 +1574,7 @@ double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { re
 int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, int M, int N, int NB, int K,
                      long ldY, long ldA, long ldB, int b_kn, int bias_mode, int epi, int out_f32,
                      long nbatch, long sY, long sA, long sB, void *ws, size_t ws_bytes, hipStream_t st,
-                     const ConvGather *gather, const NhwcGather *agather, const void *residual) {
+                     const ConvGather *gather, const NhwcGather *agather, const void *residual, long dres) {
     GemmArgs a;
     a.cv = ConvGather{};
     a.ag = NhwcGather{};
@@ -1575,7 +1585,7 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     a.sk_spin = 0; a.sk_pub_xor = a.sk_xcc_xor = 0; a.status = nullptr;
     a.lnf_stats = a.lnf_colsum = a.lnf_biasp = nullptr; a.lnf_svec = 0; a.lnf_nseg = 0; a.lnf_eps = 0.0f; a.stats_out = nullptr; a.stats_nseg = 0;
     a.Y = Y; a.A = (const half_t *)A; a.B = (const half_t *)B; a.bias = (const half_t *)bias; a.residual = out_f32 ? nullptr : (const half_t *)residual;
-    a.M = M; a.N = N; a.NB = NB; a.K = K; a.ldY = ldY; a.ldA = ldA; a.ldB = ldB; a.sY = sY; a.sA = sA; a.sB = sB; a.sBias = 0;
+    a.M = M; a.N = N; a.NB = NB; a.K = K; a.ldY = ldY; a.ldA = ldA; a.ldB = ldB; a.sY = sY; a.sA = sA; a.sB = sB; a.sBias = 0; a.dRes = dres;
     a.bias_mode = bias ? bias_mode : MI_BIAS_NONE; a.epi = epi; a.out_f32 = out_f32;
     a.tiles_m = a.tiles_n = a.group_m = 1; a.vec_store = 0;
     if (gather) a.cv = *gather;

@@ -15,6 +15,7 @@ struct GemmArgs {
     int NB;                 // columns addressable in B (>= N; a multiple of 8 for the [K][N] layout)
     long ldY, ldA, ldB;
     long sY, sA, sB, sBias; // batch strides (elements)
+    long dRes;              // the residual's batch stride is sY + dRes (one position embedding for every image: -sY)
     int bias_mode, epi, out_f32;
     int tiles_m, tiles_n, group_m;
     unsigned div_width, div_group, div_last;      // tile_of's divisions as multiplications (set_tiles)
@@ -209,64 +210,95 @@ inline void set_tiles(GemmArgs &a, int bm, int bn) {
 // the whole workgroup at its first barrier for 10 us).  One pass: the squares between the segments are taken about the
 // first segment's mean, which lies within a segment mean's spread of the row mean, so the final subtraction cancels
 // nothing that matters -- sum(x^2) - n mean^2 about zero would.  r = 1 / sqrt(var + eps), rmu = r * mean.
-// The caller synchronises the workgroup before anybody reads the slot.
-template <int BM, int BN, int NT, typename Args>
-__device__ __forceinline__ void lnf_stage(const Args &p, float2v *slot, int m0, int n0, long bz, int tid) {
-    if (!p.lnf_stats) return;
-    constexpr int LPR = NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1;
+//
+// The loads and the arithmetic are apart: a kernel requests its share of the statistics behind its first operand tiles,
+// carries it in registers and combines it late in its K loop, between products.  Combined in the prologue, the trip and
+// some sixty dependent instructions per row stood between the launch and its first MFMA: 1.3 to 1.5 us a launch at
+// K = 384, 1.6 to 2.8 at K = 1024 to 1280.  NV loads a lane cover LPR NV segments (K <= 32 LPR NV); beyond that
+// `combine` fetches the rest itself.
+template <int BM, int BN, int NT, int NV>
+struct LnfLoader {
+    static constexpr int LPR = NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1;
     static_assert(NT >= BM && (BM * LPR) % 64 == 0, "whole waves work on the rows");
-    if (tid < BM * LPR) {
-        const int row = tid / LPR, q = tid % LPR;
-        const float2v *seg = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + row, p.M - 1);
-        const float ref = seg[0][0] / (float)min(32, p.K);
-        float total = 0.0f, within = 0.0f, between = 0.0f;
-        // U loads in flight per lane: all of a row's segments in one trip to memory for K <= 1536 (2048 with four lanes a
-        // row) -- a trip costs 1 to 2 us here (the statistics were written by another kernel, on other XCDs), and the
-        // first operand tiles, requested before this, take about as long, so one trip is hidden and every further one
-        // is not (two and three batches of eight measured +3.3 and +4.3 us per launch)
-        constexpr int U = LPR == 4 ? 16 : 24;
-        for (int s0 = q; s0 < p.lnf_nseg; s0 += U * LPR) {
-            float2v v[U];
+    static constexpr int NC = (BN / 2 + NT - 1) / NT;
+    float2v v[NV];
+    float4v col[NC];
+
+    __device__ __forceinline__ static const float2v *row_of(const GemmArgs &p, int m0, int row) {
+        return reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + row, p.M - 1);
+    }
+    __device__ __forceinline__ void request(const GemmArgs &p, int m0, int n0, long bz, int tid) {
+        if (!p.lnf_stats) return;
+        if (tid < BM * LPR) {
+            const float2v *seg = row_of(p, m0, tid / LPR);
+            const int q = tid % LPR;
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int sg = s0 + u * LPR;
+            for (int u = 0; u < NV; u++) {
                 const float2v z = {0.0f, 0.0f};
-                v[u] = sg < p.lnf_nseg ? seg[(long)sg * p.M] : z;
+                v[u] = q + u * LPR < p.lnf_nseg ? seg[(long)(q + u * LPR) * p.M] : z;
             }
+        }
+        // the tile's columns of colsum and biasp
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int sg = s0 + u * LPR;
-                if (sg < p.lnf_nseg) {
-                    const int left = p.K - 32 * sg;
-                    const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
-                    const float d = fmaf(v[u][0], inv, -ref);
-                    total += v[u][0];
-                    within += v[u][1];
-                    between = fmaf(cnt * d, d, between);
+        for (int i = 0; i < NC; i++) {
+            const int t = tid + i * NT, which = t / (BN / 4), n = n0 + (t % (BN / 4)) * 4;
+            const float4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+            col[i] = z;
+            if (t < BN / 2) {
+                const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
+                if (n + 3 < p.N) col[i] = *reinterpret_cast<const float4v *>(src + n);
+                else for (int e = 0; e < 4; e++) if (n + e < p.N) col[i][e] = src[n + e];
+            }
+        }
+    }
+    // (r, r mu) per row, colsum, biasp -> slot.  The caller synchronises the workgroup before anybody reads it.
+    __device__ __forceinline__ void combine(const GemmArgs &p, float2v *slot, int m0, int tid) {
+        if (!p.lnf_stats) return;
+        if (tid < BM * LPR) {
+            const int row = tid / LPR, q = tid % LPR;
+            float total = 0.0f, within = 0.0f, between = 0.0f;
+            // the row's first segment mean: lane q = 0 of its quad (or pair) holds it
+            float first = v[0][0];
+            if constexpr (LPR == 4) first = dpp_mov<0x00>(first);          // quad_perm [0,0,0,0]
+            if constexpr (LPR == 2) first = dpp_mov<0xA0>(first);          // quad_perm [0,0,2,2]
+            const float ref = first / (float)min(32, p.K);
+            auto take = [&](const float2v s, int sg) {
+                const int left = p.K - 32 * sg;
+                const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
+                const float d = fmaf(s[0], inv, -ref);
+                total += s[0];
+                within += s[1];
+                between = fmaf(cnt * d, d, between);
+            };
+#pragma unroll
+            for (int u = 0; u < NV; u++) if (q + u * LPR < p.lnf_nseg) take(v[u], q + u * LPR);
+            if (p.lnf_nseg > NV * LPR) {
+                const float2v *seg = row_of(p, m0, row);
+                for (int s0 = q + NV * LPR; s0 < p.lnf_nseg; s0 += 8 * LPR) {
+                    float2v w[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) w[u] = seg[(long)min(s0 + u * LPR, p.lnf_nseg - 1) * p.M];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) if (s0 + u * LPR < p.lnf_nseg) take(w[u], s0 + u * LPR);
                 }
             }
+            if constexpr (LPR >= 2) { total += lane_xor<1>(total); within += lane_xor<1>(within); between += lane_xor<1>(between); }
+            if constexpr (LPR >= 4) { total += lane_xor<2>(total); within += lane_xor<2>(within); between += lane_xor<2>(between); }
+            if (q == 0) {
+                const float mu = total / (float)p.K, dm = mu - ref;
+                const float m2 = within + fmaxf(between - (float)p.K * dm * dm, 0.0f);
+                const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
+                const float2v o = {r, r * mu};
+                slot[row] = o;
+            }
         }
-        if constexpr (LPR >= 2) { total += lane_xor<1>(total); within += lane_xor<1>(within); between += lane_xor<1>(between); }
-        if constexpr (LPR >= 4) { total += lane_xor<2>(total); within += lane_xor<2>(within); between += lane_xor<2>(between); }
-        if (q == 0) {
-            const float mu = total / (float)p.K, dm = mu - ref;
-            const float m2 = within + fmaxf(between - (float)p.K * dm * dm, 0.0f);
-            const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
-            const float2v o = {r, r * mu};
-            slot[row] = o;
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const int t = tid + i * NT, which = t / (BN / 4), c = (t % (BN / 4)) * 4;
+            if (t < BN / 2) *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = col[i];
         }
     }
-    // the tile's columns of colsum and biasp
-    for (int t = tid; t < BN / 2; t += NT) {
-        const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
-        const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
-        float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
-        else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
-        *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = v;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
+};
 
 // ------------------------------------------------------------------------------------------
 // Accumulator tile -> memory, shared by the tiled kernels.
@@ -397,7 +429,7 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
                     if (n + 7 < p.N) {
                         if (p.residual) {
                             half8v rv;
-                            __builtin_memcpy(&rv, p.residual + off, 16);
+                            __builtin_memcpy(&rv, p.residual + off + bz * p.dRes, 16);
 #pragma unroll
                             for (int e = 0; e < 8; e++) x[e] = (half_t)((float)x[e] + (float)rv[e]);
                         }
@@ -410,7 +442,7 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
                         for (int e = 0; e < 8; e++) {
                             if (n + e < p.N) {
                                 half_t o = x[e];
-                                if (p.residual) o = (half_t)((float)o + (float)p.residual[off + e]);
+                                if (p.residual) o = (half_t)((float)o + (float)p.residual[off + bz * p.dRes + e]);
                                 if (p.clamp > 0.0f) o = (half_t)fminf(fmaxf((float)o, -p.clamp), p.clamp);
                                 yp[e] = o;
                             }
@@ -494,7 +526,7 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
     const bool col_ok = n < p.N;                                     // N % 8 == 0: a chunk that starts below N ends below it
     const long off0 = bz * p.sY + (long)(mw + r0) * p.ldY + n;
     half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + off0;
-    const half_t *const rbase = p.residual ? p.residual + off0 : nullptr;
+    const half_t *const rbase = p.residual ? p.residual + off0 + bz * p.dRes : nullptr;
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll

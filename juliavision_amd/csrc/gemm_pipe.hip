@@ -28,8 +28,9 @@ namespace {
 // KTAIL: K is a multiple of 8 but not of 64.  The last tile's chunks past K re-read the row's last valid chunk (nothing past
 // the row is touched) and are zeroed, in both operands, on their way into LDS: two instructions a chunk and load, which is why
 // whole tiles keep their own instance.  1544 x 1288 -> 1288 with a residual: 25.7 us through the unpipelined kernel before.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int AMODE = 0, bool KTAIL = false>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void gemm_pipe_kernel(GemmArgs p) {
+// LNF: the launch has a layer norm folded away (lnf_stats); the statistics' registers would cost the others a workgroup per CU.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int AMODE = 0, bool KTAIL = false, bool LNF = false>
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ? 4 : 2) void gemm_pipe_kernel(GemmArgs p) {
     constexpr bool B_KN = BMODE != 0, CONV = BMODE == 2, LNA = AMODE == 2;
     static_assert(AMODE == 0 || BMODE != 2, "one gathered operand at a time");
     static_assert(!KTAIL || (AMODE == 0 && BMODE != 2), "gathered operands come in whole tiles");
@@ -206,10 +207,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void gemm_pipe_kernel(Gem
     const int nk = KTAIL ? (p.K + BK - 1) / BK : p.K / BK;   // the launcher guarantees nk >= 2, and K % 64 == 0 without KTAIL
     gload(0, 0);
     gload(1, 1);
-    // folded layer norm: (r, r mu) of the tile's rows, worked out while the first tiles are on their way and parked
-    // in LDS behind the operand buffers until the store (the barrier after the first LDS write covers it)
+    // folded layer norm: the row statistics and column constants of the tile, combined ahead of the last tile into a slot
+    // behind the operand buffers (the last tile's barrier covers it)
     float2v *ln_slot = reinterpret_cast<float2v *>(smem + 2 * (BM * LD + BSZ) * 2);
-    if constexpr (!LNA) lnf_stage<BM, BN, NT>(p, ln_slot, m0, n0, bz, tid);
+    LnfLoader<BM, BN, NT, 40 / (NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1)> lnf;
+    if constexpr (LNF) lnf.request(p, m0, n0, bz, tid);
     if constexpr (LNA) {
         // One wave per row, all rows of a wave in flight at once (one trip to memory).  Rows past M repeat the last one.
         constexpr int NW = NT / 64, RB = BM / NW;
@@ -303,15 +305,17 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void gemm_pipe_kernel(Gem
         body(M0{}, kt, 0, 1, 0);
         body(M1{}, kt + 1, 1, 0, 1);
         load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
+        if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
         body(M2{}, kt + 2, 0, 1, 0);
     } else {
         body(M1{}, kt, 0, 1, 0);
         load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
+        if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
         body(M2{}, kt + 1, 1, 0, 1);
     }
     __syncthreads();
     LnFold<TM> ln;
-    if (!LNA && p.lnf_stats) {
+    if constexpr (LNF) {
         ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN;
 #pragma unroll
         for (int j = 0; j < TM; j++) { const float2v v = ln_slot[wm * WTM + 32 * j + (lane & 31)]; ln.r[j] = v[0]; ln.rmu[j] = v[1]; }
@@ -338,6 +342,12 @@ int launch_pipe(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
         if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, true>), grid, dim3(WM * WN * 64), lds, st, a);
         else      hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, true>), grid, dim3(WM * WN * 64), lds, st, a);
     }
+    else if (a.lnf_stats) {
+        if constexpr (BM * BN <= 128 * 128) {
+            if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, false, true>), grid, dim3(WM * WN * 64), lds, st, a);
+            else      hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, false, true>), grid, dim3(WM * WN * 64), lds, st, a);
+        } else return MI_DECLINE_EXTENT;      // the four-wave kernel's tiles
+    }
     else if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1>), grid, dim3(WM * WN * 64), lds, st, a);
     else           hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0>), grid, dim3(WM * WN * 64), lds, st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
@@ -346,7 +356,10 @@ int launch_pipe(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
 template <int BM, int BN, int WM, int WN>
 int raise_pipe() {
     constexpr int lds = gemm_lds_bytes<BM, BN, 64>();
-    return raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1>, lds) |
+    int bad = 0;
+    if constexpr (BM * BN <= 128 * 128)
+        bad = raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, false, true>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, false, true>, lds);
+    return bad | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1>, lds) |
            raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 2>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 1>, lds) |
            raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 1>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, true>, lds) |
            raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, true>, lds);

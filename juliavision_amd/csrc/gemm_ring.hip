@@ -195,7 +195,8 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
     half4v cb[KEEP][4];
     load_col_bias<KEEP, STN>(p, cb, n0, sn, lane, bz);
     float2v *ln_slot = reinterpret_cast<float2v *>(smem + S * STAGE_BYTES);
-    lnf_stage<BM, BN, NT>(p, ln_slot, m0, n0, bz, tid);
+    LnfLoader<BM, BN, NT, 10> lnf;                       // four lanes a row: K <= 1280 in one request
+    lnf.request(p, m0, n0, bz, tid);
     barrier();
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
@@ -216,6 +217,8 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
     }
     if (kt < nk) turn(I0{}, I1{}, kt);
 
+    lnf.combine(p, ln_slot, m0, tid);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     barrier();                                            // every wave has read its last fragments
     LnFold<2> ln2;
     if constexpr (WK > 1) {
