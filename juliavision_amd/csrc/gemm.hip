@@ -1259,41 +1259,42 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
     }
 }
 
-// Tile and K-split of a pipelined GEMM, chosen by estimated time.  The five tilings of gemm_pipe_kernel were timed
-// on an MI355X over 400 shapes (M 64..8192, N 64..5120, K 128..5120), each unsplit and in 2, 4 and 8 K-slices; per
-// tiling the time is launch + prologue/store + (K / 64) steps, and a step costs step_lo when few workgroups run, rises
-// linearly to step_full when every CU holds one (clock and memory give way under load), and beyond that grows with
-// the number of rounds of CUs-many workgroups (by `round`, below 1 where co-resident workgroups overlap).  A split adds
-// the second launch (about 4 us) and the fp32 planes (0.25 us per MB).  Picking the cheapest estimate lands within
-// 1 % of the best measured choice on average over those shapes and within 6 % on 95 % of them.
-struct TileModel { int bm, bn; double step_lo, step_full, round, fixed; };
+// Tile and K-split of a pipelined GEMM, chosen by estimated time: launch + prologue/store + (K / 64) steps, where a step costs
+// step_lo when few workgroups run, rises linearly to step_full when every CU holds one (clock and memory give way under
+// load), and beyond that grows with the number of rounds of CUs-many workgroups (by `round`, below 1 where co-resident
+// workgroups overlap).  A K that ends inside a tile makes every step `tail` times as long: its rows are no multiple of
+// a cache line, so most 128-byte pieces of them touch two.  A GELU store adds `gelu` a round.  A split adds the second
+// launch (4.4 us) and the fp32 planes (0.38 us per MB).
+// Fitted to every tile timed on 200 shapes in a replayed graph (M 9..8192, N 64..8192, K 72..5120, both layouts, a third of
+// them with K % 64, a third with GELU): the cheapest estimate lands within 0.3 % of the best measured tile on average.
+// What it replaced sent every K % 64 to 64 x 64 tiles: 1544 x 1288 -> 1288 with residual 19.8 -> 15.4 us on 128 x 128,
+// 636 x 4392 -> 104 23.2 -> 13.8 on the ring, 2237 x 5096 -> 2440 with GELU 143 -> 80 on 192 x 128.
+struct TileModel { int bm, bn; double step_lo, step_full, round, fixed, gelu, tail; };
 constexpr int NTILES = 6;
 constexpr TileModel TILE_MODELS[NTILES] = {
-    // (the two tiles of the four-wave kernel, re-timed with it: 1500 x 5120 in 25.3 / 70.5 us at K = 1280 / 5120,
-    // 512 x 1280 in 16.3 / 47.2; 1500 x 3840 on 192 x 128 in 20.2 / 55.4, 512 x 1280 in 13.5 / 39.9)
-    {128, 256, 0.520, 0.760, 1.06, 7.0},
-    {192, 128, 0.420, 0.585, 1.00, 6.0},
-    {128, 128, 0.428, 0.600, 1.00, 4.0},
-    {64, 128, 0.318, 0.430, 0.90, 3.1},
-    {64, 64, 0.235, 0.315, 0.73, 3.0},
-    // gemm_ring_kernel: timed over 2 to 256 workgroups and K 384 to 5120 (20 x 1280 -> 1280 tiles in 7.6 us, 128 workgroups
-    // over K = 4096 in 17.4).  Its sum of four partial tiles and deep ring cost a microsecond at the ends, so it starts past
+    {128, 256, 0.444, 0.720, 1.13, 6.2, 2.9, 1.43},
+    {192, 128, 0.360, 0.556, 1.11, 5.2, 2.4, 1.46},
+    {128, 128, 0.386, 0.534, 1.06, 3.9, 2.0, 1.13},
+    {64, 128, 0.287, 0.356, 0.856, 3.26, 1.0, 1.28},
+    {64, 64, 0.209, 0.252, 0.70, 2.93, 0.46, 1.35},
+    // gemm_ring_kernel: its sum of four partial tiles and deep ring cost a microsecond at the ends, so it starts past
     // K = 512 -- where the layer-norm prologue's promise of identical bits ends too -- and above one workgroup per CU its
     // LDS allows no second one: L2 bandwidth (19 to 24 TB/s) is what bounds it there in any case.
-    {64, 64, 0.125, 0.215, 1.00, 4.2},
+    {64, 64, 0.127, 0.141, 1.00, 4.31, 0.56, 1.10},
 };
 constexpr int RING_KMIN = 513;
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
-double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split) {
+double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
     const TileModel &t = TILE_MODELS[tile];
     const double cus = (double)mi_num_cus();
     const int64_t wg = ceil_div(M, t.bm) * ceil_div(N, t.bn) * nbatch * split;
     const int64_t rounds = ceil_div(wg, (int64_t)mi_num_cus());
     const double load = wg < mi_num_cus() ? (double)wg / cus : 1.0;
-    const double step = wg <= mi_num_cus() ? t.step_lo + (t.step_full - t.step_lo) * load : t.step_full * t.round * (double)rounds;
+    const double step = (wg <= mi_num_cus() ? t.step_lo + (t.step_full - t.step_lo) * load : t.step_full * t.round * (double)rounds) * (K % 64 ? t.tail : 1.0);
     double us = 2.0 + (t.fixed - 2.0) * (1.0 + 0.8 * (double)(rounds - 1)) + (t.fixed - 2.0) * 0.4 * load + (double)((K + 63) / 64 / split) * step;
-    if (split > 1) us += 4.0 + 0.25 * (double)split * (double)M * (double)N * 4.0 / 1e6;
+    if (split > 1) us += 4.4 + 0.38 * (double)split * (double)M * (double)N * 4.0 / 1e6;
+    if (gelu) us += t.gelu * (wg > mi_num_cus() ? (double)wg / cus : 1.0);
     return us;
 }
 
@@ -1320,24 +1321,25 @@ bool sk_planned() {
     return g_sk_state[dev] != -1;
 }
 double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
+    constexpr double step_lo = 0.428, step_full = 0.600, fixed = 4.0;        // of the four-wave kernel's 128 x 128 tile
     const TileModel &t = TILE_MODELS[tile];
     const int64_t wg = ceil_div(M, t.bm) * ceil_div(N, t.bn) * split;
     const double load = (double)wg / (double)mi_num_cus();
-    const double step = t.step_lo + (t.step_full - t.step_lo) * load;
-    return 2.0 + (t.fixed - 2.0) * (0.4 + 0.6 / (double)split) + (t.fixed - 2.0) * 0.4 * load + (double)(K / (64 * split)) * step +
-           sk_exchange_us(wg, t.bm, t.bn);
+    const double step = step_lo + (step_full - step_lo) * load;
+    return 0.9 * (2.0 + (fixed - 2.0) * (0.4 + 0.6 / (double)split) + (fixed - 2.0) * 0.4 * load + (double)(K / (64 * split)) * step +
+           sk_exchange_us(wg, t.bm, t.bn));        // 0.9: 17.1 us at 1500 x 3072 -> 768, 27.9 at 1370 x 5120 -> 1280
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring) {
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring, bool gelu) {
     TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
     for (int split = 1; split <= max_split; split++) {
-        if (K % (64 * split) != 0 || (split > 1 && K / split < 128)) continue;
+        if (split > 1 && (K % (64 * split) != 0 || K / split < 128)) continue;
         for (int tile = 0; tile < NTILES; tile++) {
             if (tile == RING_TILE && (!ring || K / split < RING_KMIN || ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > mi_num_cus())) continue;
-            const double us = tile_cost_us(M, N, K, nbatch, tile, split);
+            const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
         if (max_split > 1 && sk_planned()) {
@@ -1352,14 +1354,14 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
 
 // The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
 // thread keeps the last answers.  The key holds everything the estimate reads.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring = true) {
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring = true, bool gelu = false) {
     struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
     static thread_local Entry table[256] = {};
-    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (ring ? 8 : 0);
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (ring ? 8 : 0) | (gelu ? 16 : 0);
     const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 40;
     Entry &e = table[(h >> 32) & 255];
     if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
-        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, ring)};
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, ring, gelu)};
     return e.plan;
 }
 
@@ -1536,11 +1538,10 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)ceil_div(quads, 256)), dim3(256), 0, st, s2, planes, split);
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
-        // A GELU store is some fifteen vector instructions a value: where 128 x 128 tiles leave half the chip without one, 64 x 128
-        // tiles spread it (1370 x 384 -> 1536 inside a ViT block: 2 us of 11; at 204 of 256 workgroups the wide tile is the
-        // faster again).  Every pipelined tile sums K in the same order, so the bits do not change.
-        if (tp.tile == 2 && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH) && ceil_div(a.M, 128) * ceil_div(a.N, 128) * nbatch * 8 <= (int64_t)mi_num_cus() * 5)
-            tp.tile = 3;
+        // A GELU store is some fifteen vector instructions a value, so narrower tiles can be the faster ones for it (1500 x 384 ->
+        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every pipelined tile sums K in the same order: the bits stay.
+        if (pipe && split == 1 && tp.tile != RING_TILE && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, true);
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
@@ -1690,9 +1691,12 @@ size_t mi_gemm_f16_workspace(int64_t T, int64_t K, int64_t F, int w_layout, int6
     if (T < 1 || nbatch > 1) return 0;
     if (T > 8) {
         if (K % 64 || K < 128) return 0;
-        // never less than the split that the plan takes without the ring kernel: buffers and recorded plans keep their sizes
-        const size_t need = plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F), other = plan_workspace_bytes(plan_tiles(T, F, K, 1, true, false), T, F);
-        return need > other ? need : other;
+        // Room for the exchange wherever it can run on a K of some length, whichever tile the estimate prefers: buffers and
+        // recorded plans keep their sizes when its constants move.
+        const size_t need = plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
+        const TileModel &t = TILE_MODELS[SK_TILE];
+        const size_t peer = K >= 2048 && sk_fits(T, F, K, t.bm, t.bn, 2) ? round_up(sk_workspace_bytes(T, F, t.bm, t.bn, 2), 256) : 0;
+        return need > peer ? need : peer;
     }
     if (w_layout != MI_W_KF) return 0;      // the [F][K] skinny kernel finishes its outputs itself
     return round_up((size_t)skinny_splits(K, F) * T * F * sizeof(float), 256);

@@ -48,6 +48,13 @@ def test_k_ends_inside_a_tile(ctx, T, K, F, layout):
 
 
 @pytest.mark.parametrize("layout", ["kf", "fk"])
+@pytest.mark.parametrize("T,K,F", [(130, 1224, 104), (300, 1096, 264), (300, 136, 264), (2379, 72, 400), (454, 136, 4208), (839, 136, 4752), (1224, 200, 4888)])
+def test_k_ends_inside_a_tile_of_every_size(ctx, T, K, F, layout):
+    """The ring and every pipelined tile (64 x 64 to 128 x 256) with a K that is no multiple of 64."""
+    _check(ctx, T, K, F, layout, residual=True)
+
+
+@pytest.mark.parametrize("layout", ["kf", "fk"])
 @pytest.mark.parametrize("T,K,F", [(1, 1, 1), (3, 7, 9), (2, 464, 73), (8, 9, 8), (17, 65, 33), (64, 63, 65), (70, 257, 129), (3, 2311, 106), (200, 311, 77),
                                    (1100, 130, 1999), (2049, 65, 2051), (33, 8, 24), (100, 64, 40)])
 def test_ragged_in_every_direction(ctx, T, K, F, layout):
