@@ -5,6 +5,8 @@
 //                     product in exactly the register layout the second product
 //                     consumes -- scores and probabilities never touch LDS or
 //                     HBM.  Online softmax in fp32, one query per lane pair.
+//  flash_tile_kernel  (sdpa_tile.hip) the same on 32-query workgroups of independent
+//                     waves: all grids but the largest, head sizes 16 to 128.
 //  sdpa_rows_kernel   one workgroup per (query row, key split): the
 //                     bandwidth-bound form for decode-sized Lq, and the
 //                     always-available path for additive masks, odd head
@@ -13,40 +15,11 @@
 //
 // Operands are (E, L, H, B) with element strides (the reference's layout,
 // DNNKernels/src/kernels/extern/attention.jl:1-22); out is dense (E, Lq, H, B).
-#include "common.hpp"
+#include "sdpa_common.hpp"
 #include <atomic>
 #include <cstdlib>
-#include <type_traits>
 
 namespace {
-
-struct SdpaArgs {
-    void *out;
-    const half_t *q, *k, *v;
-    long qs[4], ks[4], vs[4], os[4];   // (E, L, H, B) element strides
-    const void *bias;
-    long bs[4];                    // (Lk, Lq, H, B) element strides, 0 = broadcast
-    const int *kv_len;
-    float *part_o, *part_ml;       // split partials: [split][row][E], [split][row][2] (sdpa_decode_kernel: [row][split])
-    unsigned *tickets;             // sdpa_decode_kernel with nsplit > 1: one arrival counter per (head, batch), zero between launches
-    // sdpa_decode_kernel only: the newest key/value row (1 x E per head and batch); when set, key kv_len - 1 is
-    // taken from here instead of the cache and written into the cache on the way (k, v are then written to)
-    const half_t *k_new, *v_new;
-    long ns[4];
-    int E, Lq, Lk, H, B;
-    int out_f32, bias_f32, nsplit;
-    float scale;
-};
-
-constexpr float LOG2E = 1.4426950408889634f;
-
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<int, N - 1>{});
-    }
-}
 
 // ------------------------------------------------------------------------------------------
 // Fused kernel.  Workgroup = 4 waves = 128 queries (32 per wave); keys walked in
@@ -664,461 +637,6 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
 }
 
 // ------------------------------------------------------------------------------------------
-// Fused attention for grids that leave most of the chip idle (head size 64, no mask): a workgroup owns 32 queries,
-// and its NW waves (8, or 4 so that two workgroups share a CU) each walk their own run of whole 64-key blocks, so the
-// chain a wave walks is Lk / NW keys long instead of Lk / 2.  Nothing is shared between the waves until the end, so
-// nothing is staged for anyone else and the loop has no workgroup barrier: a wave takes its K fragments straight from
-// memory in the layout the first product wants (lane = key, 16 bytes of one row per k-step: every row is read whole over
-// the four k-steps), and passes its V block through a private stretch of LDS only for the transposing read of the second
-// product (the wave's LDS operations complete in order: the write of block j + 1 follows the reads of block j without a
-// wait).  Both are requested a block ahead.  The softmax is flash_fwd_kernel's (lazy reference point).  The waves'
-// (O, M, l) meet in LDS and are merged with the rescaling identity of flash.jl:1385-1391, each thread finishing four
-// consecutive head-dim values of one query.
-template <int NW>
-__global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void flash_short_kernel(SdpaArgs p) {
-    constexpr int EP = 64, KS = 4, ET = 2, BC = 64, VLD = flash_vld(64);
-    constexpr int WREG = BC * VLD * 2;                        // bytes of a wave's V stretch; holds its (O, m, l) afterwards
-    static_assert((ET * 16 + 2) * 64 * 4 <= WREG, "a wave's partial fits its own stretch");
-    extern __shared__ __align__(16) char smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int hl = lane >> 5, l32 = lane & 31;
-    half_t *Vw = reinterpret_cast<half_t *>(smem + wave * WREG);
-    int qblk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    {
-        // all query blocks of a head on one XCD (workgroups are dealt to the XCDs round robin)
-        const int nqb = gridDim.x, total = nqb * gridDim.y * gridDim.z;
-        if ((total & 7) == 0) {
-            int id = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-            id = (id & 7) * (total >> 3) + (id >> 3);
-            qblk = id % nqb;
-            h = (id / nqb) % gridDim.y;
-            b = id / (nqb * gridDim.y);
-        }
-    }
-    const int q0 = qblk * 32;
-    const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];
-    const half_t *kb = p.k + h * p.ks[2] + b * p.ks[3];
-    const half_t *vb = p.v + h * p.vs[2] + b * p.vs[3];
-    int Lk = p.Lk;
-    if (p.kv_len) Lk = max(0, min(Lk, p.kv_len[b]));
-    // this wave's keys: whole 64-key blocks, [kbeg, kend)
-    const int per = (((Lk + BC - 1) / BC + NW - 1) / NW) * BC;
-    const int kbeg = wave * per, kend = min(Lk, kbeg + per);
-    const int nblk = kend > kbeg ? (kend - kbeg + BC - 1) / BC : 0;
-    const int last = p.Lk - 1;                                // rows past the end re-read the last key that exists
-    const float c = p.scale * LOG2E;
-
-    u32x4 qraw[KS];
-    {
-        const int qr = min(q0 + l32, p.Lq - 1);
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) qraw[ks] = ldg16(qb + (long)qr * p.qs[1] + 16 * ks + 8 * hl);
-    }
-    // K fragments of a block: tile kt (32 keys), k-step ks: key = key0 + 32 kt + l32, head dim 16 ks + 8 hl .. +7
-    auto load_k = [&](u32x4 (&kf)[2][KS], int key0) {
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-            const half_t *row = kb + (long)min(key0 + 32 * kt + l32, last) * p.ks[1] + 8 * hl;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) kf[kt][ks] = ldg16(row + 16 * ks);
-        }
-    };
-    // the wave's V block, 8 chunks of 16 bytes per lane: chunk lane + 64 i = (key, 8 head-dim values)
-    u32x4 vr[8];
-    auto load_v = [&](int key0) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int cidx = lane + 64 * i;
-            vr[i] = ldg16(vb + (long)min(key0 + (cidx >> 3), last) * p.vs[1] + (cidx & 7) * 8);
-        }
-    };
-    auto store_v = [&]() {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int cidx = lane + 64 * i;
-            *reinterpret_cast<u32x4 *>(Vw + (cidx >> 3) * VLD + (cidx & 7) * 8) = vr[i];
-        }
-    };
-    u32x4 ka[2][KS], kc[2][KS];
-    if (nblk > 0) { load_k(ka, kbeg); load_v(kbeg); }
-    half8v qf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const half8v t = as_half8(qraw[ks]);
-#pragma unroll
-        for (int j = 0; j < 8; j++) qf[ks][j] = (half_t)((float)t[j] * c);
-    }
-    float16v o_acc[ET];
-#pragma unroll
-    for (int t = 0; t < ET; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) o_acc[t][r] = 0.0f;
-    float m_run = 0.0f, l_run = 0.0f;                        // m_run: the reference point, always exactly representable in fp16
-    const int vtoff = (4 * hl + ((lane & 15) >> 2)) * VLD + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-    const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-
-    // The reference point of the running softmax is subtracted by the first product itself -- one more k-step with the
-    // operand pair 1.0 and -M[query] -- and moves lazily, as in flash_fwd_kernel: on a wave's first block, and when a
-    // probability would leave fp16 range (seen in the fp32 row sum growing by 2^16 within a block).
-    constexpr float TH = 8.0f;
-    half8v kext, qext;
-#pragma unroll
-    for (int jj = 0; jj < 8; jj++) { kext[jj] = (half_t)0.0f; qext[jj] = (half_t)0.0f; }
-    if (hl == 0) kext[0] = (half_t)1.0f;
-    bool first = true;
-    auto probs = [&](const float16v (&sx)[2], half8v (&pf)[2][2], float &l) {
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(sx[kt][r]), p1 = __builtin_amdgcn_exp2f(sx[kt][r + 1]);
-                pf[kt][r >> 3][r & 7] = (half_t)p0;
-                pf[kt][r >> 3][(r & 7) + 1] = (half_t)p1;
-                l += p0 + p1;
-            }
-    };
-    auto iter = [&](u32x4 (&kcur)[2][KS], u32x4 (&knext)[2][KS], int j) {
-        const int key0 = kbeg + j * BC;
-        store_v();                                           // block j's V (requested one block ago) into the stretch
-        if (j + 1 < nblk) { load_k(knext, key0 + BC); load_v(key0 + BC); }
-        float16v sc[2];
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-            sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(kcur[kt][0]), qf[0], zero16, 0, 0, 0);
-#pragma unroll
-            for (int ks = 1; ks < KS; ks++) sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(kcur[kt][ks]), qf[ks], sc[kt], 0, 0, 0);
-            sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kext, qext, sc[kt], 0, 0, 0);
-        }
-        if (key0 + BC > kend) {                              // the ragged last block: excluded keys get -inf
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    if (key0 + 32 * kt + 8 * (r >> 2) + 4 * hl + (r & 3) >= kend) sc[kt][r] = -INFINITY;
-        }
-        half8v pf[2][2];
-        float l_new = l_run;
-        probs(sc, pf, l_new);
-        if (__any(first || !(l_new - l_run < 65504.0f))) {
-            float tmax = fmaxf(sc[0][0], sc[1][0]);
-#pragma unroll
-            for (int r = 1; r < 16; r++) tmax = fmaxf(fmaxf(tmax, sc[0][r]), sc[1][r]);
-            const float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const bool grow = (mx > TH || first) && mx != -INFINITY;
-            const half_t m16 = (half_t)(m_run + (grow ? mx : 0.0f));
-            const float d = (float)m16 - m_run;
-            const float alpha = __builtin_amdgcn_exp2f(-d);
-            m_run += d;
-            l_run *= alpha;
-            if (hl == 0) qext[0] = -m16;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) sc[kt][r] -= d;
-#pragma unroll
-            for (int t = 0; t < ET; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o_acc[t][r] *= alpha;
-            l_new = l_run;
-            probs(sc, pf, l_new);
-        }
-        l_run = l_new;
-        first = false;
-        // O^T += V^T . P^T
-#pragma unroll
-        for (int t = 0; t < ET; t++) {
-            const half_t *vp = Vw + vtoff + 32 * t;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int bb = 0; bb < 2; bb++) {
-                    const half_t *vq = vp + (32 * kt + 16 * bb) * VLD;
-                    short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq));
-                    short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq + 8 * VLD));
-                    short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, both), pf[kt][bb], o_acc[t], 0, 0, 0);
-                }
-        }
-    };
-    int j = 0;
-    for (; j + 2 <= nblk; j += 2) {
-        iter(ka, kc, j);
-        iter(kc, ka, j + 1);
-    }
-    if (j < nblk) iter(ka, kc, j);
-
-    // both lanes of a query hold half of its row sum
-    l_run += __shfl_xor(l_run, 32, 64);
-    // the wave's partial, lane-major, into its own stretch (its reads of V are behind it)
-    float *xo = reinterpret_cast<float *>(smem + wave * WREG);
-#pragma unroll
-    for (int t = 0; t < ET; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) xo[(t * 16 + r) * 64 + lane] = o_acc[t][r];
-    xo[(ET * 16) * 64 + lane] = m_run;
-    xo[(ET * 16 + 1) * 64 + lane] = l_run;
-    __syncthreads();
-    // Thread (src lane, group) finishes query q0 + l32 at head dims 32 t + 8 g + 4 hl .. +3 for its (t, g).
-    float aw[NW], mm = -INFINITY, den = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        // a wave that saw no valid key has l = 0 and a meaningless reference point
-        const float *xw = reinterpret_cast<const float *>(smem + w * WREG);
-        aw[w] = xw[(ET * 16 + 1) * 64 + lane] > 0.0f ? xw[(ET * 16) * 64 + lane] : -INFINITY;
-        mm = fmaxf(mm, aw[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        const float *xw = reinterpret_cast<const float *>(smem + w * WREG);
-        aw[w] = aw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(aw[w] - mm);
-        den += aw[w] * xw[(ET * 16 + 1) * 64 + lane];
-    }
-    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    const int qi = q0 + l32;
-    constexpr int COMBOS = 8 / NW;                            // (t, g) pairs per thread: 8 pairs over NW waves
-#pragma unroll
-    for (int cidx = 0; cidx < COMBOS; cidx++) {
-        const int tg = wave * COMBOS + cidx, t = tg >> 2, g = tg & 3;
-        float o4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const float *xw = reinterpret_cast<const float *>(smem + w * WREG);
-#pragma unroll
-            for (int i = 0; i < 4; i++) o4[i] += aw[w] * xw[(t * 16 + 4 * g + i) * 64 + lane];
-        }
-        if (qi < p.Lq) {
-            const long off = (long)b * p.os[3] + (long)h * p.os[2] + (long)qi * p.os[1] + 32 * t + 8 * g + 4 * hl;
-            if (p.out_f32) {
-                const float4v o = {o4[0] * inv, o4[1] * inv, o4[2] * inv, o4[3] * inv};
-                *reinterpret_cast<float4v *>(reinterpret_cast<float *>(p.out) + off) = o;
-            } else {
-                const half4v o = {(half_t)(o4[0] * inv), (half_t)(o4[1] * inv), (half_t)(o4[2] * inv), (half_t)(o4[3] * inv)};
-                *reinterpret_cast<half4v *>(reinterpret_cast<half_t *>(p.out) + off) = o;
-            }
-        }
-    }
-}
-
-// The short-chain form on 64-query tiles, for grids whose 32-query tiles would be a few more than the CUs (6 heads x
-// 1370: 258) and for the traffic: in flash_short_kernel every 32-query tile reads all of its head's K and V from the L2,
-// and with 43 tiles a head that read is what the loop waits for.  Here eight waves share a tile: wave w takes key
-// quarter w % 4 for query half w / 4, and the two waves of a quarter share its K and V through LDS -- one of them fetches
-// the K block, the other the V block, a block ahead, 8 chunks of 16 bytes a lane -- so a tile of twice the queries reads
-// the same bytes.  K lies in LDS row-major with 16 bytes of padding (conflict-free 16-byte fragment reads), V as in
-// flash_short_kernel.  One buffer per quarter: a workgroup barrier after the writes of block j, another before the
-// writes of block j + 1; every wave takes part in every barrier (quarters with fewer blocks idle through the rest).
-__global__ __launch_bounds__(512, 1) void flash_pair_kernel(SdpaArgs p) {
-    constexpr int EP = 64, KS = 4, ET = 2, BC = 64, NQ = 4, VLD = flash_vld(64), KLD = EP + 8;
-    constexpr int KBYTES = BC * KLD * 2, VBYTES = BC * VLD * 2, QREG = KBYTES + VBYTES;      // a quarter's K and V
-    constexpr int WPART = (ET * 16 + 2) * 64 * 4;                                            // a wave's (O, m, l)
-    static_assert(8 * WPART <= NQ * QREG, "the partials fit where the stages were");
-    extern __shared__ __align__(16) char smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kq = wave & 3, qh = wave >> 2;
-    const int hl = lane >> 5, l32 = lane & 31;
-    half_t *Kw = reinterpret_cast<half_t *>(smem + kq * QREG);
-    half_t *Vw = reinterpret_cast<half_t *>(smem + kq * QREG + KBYTES);
-    int qblk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    {
-        const int nqb = gridDim.x, total = nqb * gridDim.y * gridDim.z;
-        if ((total & 7) == 0) {
-            int id = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-            id = (id & 7) * (total >> 3) + (id >> 3);
-            qblk = id % nqb;
-            h = (id / nqb) % gridDim.y;
-            b = id / (nqb * gridDim.y);
-        }
-    }
-    const int q0 = qblk * 64 + 32 * qh;
-    const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];
-    const half_t *kb = p.k + h * p.ks[2] + b * p.ks[3];
-    const half_t *vb = p.v + h * p.vs[2] + b * p.vs[3];
-    int Lk = p.Lk;
-    if (p.kv_len) Lk = max(0, min(Lk, p.kv_len[b]));
-    const int per = (((Lk + BC - 1) / BC + NQ - 1) / NQ) * BC;
-    const int nmax = per / BC;                                // barriers are counted over this, by every wave
-    const int kbeg = kq * per, kend = min(Lk, kbeg + per);
-    const int nblk = kend > kbeg ? (kend - kbeg + BC - 1) / BC : 0;
-    const int last = p.Lk - 1;
-    const float c = p.scale * LOG2E;
-
-    u32x4 qraw[KS];
-    {
-        const int qr = min(q0 + l32, p.Lq - 1);
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) qraw[ks] = ldg16(qb + (long)qr * p.qs[1] + 16 * ks + 8 * hl);
-    }
-    // this wave's share of a block: the K rows (query half 0) or the V rows (query half 1), chunk lane + 64 i = (key, 8 head dims)
-    const half_t *src = qh == 0 ? kb : vb;
-    const long srow = qh == 0 ? p.ks[1] : p.vs[1];
-    half_t *dst = qh == 0 ? Kw : Vw;
-    const int dld = qh == 0 ? KLD : VLD;
-    u32x4 pre[8];
-    auto fetch = [&](int key0) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int cidx = lane + 64 * i;
-            pre[i] = ldg16(src + (long)min(key0 + (cidx >> 3), last) * srow + (cidx & 7) * 8);
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int cidx = lane + 64 * i;
-            *reinterpret_cast<u32x4 *>(dst + (cidx >> 3) * dld + (cidx & 7) * 8) = pre[i];
-        }
-    };
-    if (nblk > 0) fetch(kbeg);
-    half8v qf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const half8v t = as_half8(qraw[ks]);
-#pragma unroll
-        for (int j = 0; j < 8; j++) qf[ks][j] = (half_t)((float)t[j] * c);
-    }
-    float16v o_acc[ET];
-#pragma unroll
-    for (int t = 0; t < ET; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) o_acc[t][r] = 0.0f;
-    float m_run = 0.0f, l_run = 0.0f;
-    const int ktoff = l32 * KLD + 8 * hl;
-    const int vtoff = (4 * hl + ((lane & 15) >> 2)) * VLD + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-    const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    constexpr float TH = 8.0f;
-    // the reference point is the first product's accumulator input: every score of a lane belongs to its one query
-    float16v negm = zero16;
-    bool first = true;
-    auto probs = [&](const float16v (&sx)[2], half8v (&pf)[2][2], float &l) {
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(sx[kt][r]), p1 = __builtin_amdgcn_exp2f(sx[kt][r + 1]);
-                pf[kt][r >> 3][r & 7] = (half_t)p0;
-                pf[kt][r >> 3][(r & 7) + 1] = (half_t)p1;
-                l += p0 + p1;
-            }
-    };
-    for (int j = 0; j < nmax; j++) {
-        const bool live = j < nblk;                          // uniform over the wave, and the same for both waves of a quarter
-        const int key0 = kbeg + j * BC;
-        if (j > 0) __syncthreads();                          // block j - 1 has been read by everyone
-        if (live) stage();
-        if (j + 1 < nblk) fetch(key0 + BC);
-        __syncthreads();                                     // block j is in place
-        if (!live) continue;
-        float16v sc[2];
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-            const half_t *kp_ = Kw + ktoff + 32 * kt * KLD;
-            sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8v *>(kp_), qf[0], negm, 0, 0, 0);
-#pragma unroll
-            for (int ks = 1; ks < KS; ks++)
-                sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8v *>(kp_ + 16 * ks), qf[ks], sc[kt], 0, 0, 0);
-        }
-        if (key0 + BC > kend) {
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    if (key0 + 32 * kt + 8 * (r >> 2) + 4 * hl + (r & 3) >= kend) sc[kt][r] = -INFINITY;
-        }
-        half8v pf[2][2];
-        float l_new = l_run;
-        probs(sc, pf, l_new);
-        if (__any(first || !(l_new - l_run < 65504.0f))) {
-            float tmax = fmaxf(sc[0][0], sc[1][0]);
-#pragma unroll
-            for (int r = 1; r < 16; r++) tmax = fmaxf(fmaxf(tmax, sc[0][r]), sc[1][r]);
-            const float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const bool grow = (mx > TH || first) && mx != -INFINITY;
-            const half_t m16 = (half_t)(m_run + (grow ? mx : 0.0f));
-            const float d = (float)m16 - m_run;
-            const float alpha = __builtin_amdgcn_exp2f(-d);
-            m_run += d;
-            l_run *= alpha;
-#pragma unroll
-            for (int r = 0; r < 16; r++) negm[r] = -(float)m16;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) sc[kt][r] -= d;
-#pragma unroll
-            for (int t = 0; t < ET; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o_acc[t][r] *= alpha;
-            l_new = l_run;
-            probs(sc, pf, l_new);
-        }
-        l_run = l_new;
-        first = false;
-#pragma unroll
-        for (int t = 0; t < ET; t++) {
-            const half_t *vp = Vw + vtoff + 32 * t;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int bb = 0; bb < 2; bb++) {
-                    const half_t *vq = vp + (32 * kt + 16 * bb) * VLD;
-                    short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq));
-                    short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq + 8 * VLD));
-                    short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, both), pf[kt][bb], o_acc[t], 0, 0, 0);
-                }
-        }
-    }
-    l_run += __shfl_xor(l_run, 32, 64);
-    __syncthreads();                                         // the last blocks have been read: the stages become the partials
-    float *xo = reinterpret_cast<float *>(smem + wave * WPART);
-#pragma unroll
-    for (int t = 0; t < ET; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) xo[(t * 16 + r) * 64 + lane] = o_acc[t][r];
-    xo[(ET * 16) * 64 + lane] = m_run;
-    xo[(ET * 16 + 1) * 64 + lane] = l_run;
-    __syncthreads();
-    // the four quarters of this wave's query half meet; wave kq finishes (t, g) pairs 2 kq and 2 kq + 1 of its 32 queries
-    float aw[NQ], mm = -INFINITY, den = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NQ; w++) {
-        const float *xw = reinterpret_cast<const float *>(smem + (qh * NQ + w) * WPART);
-        aw[w] = xw[(ET * 16 + 1) * 64 + lane] > 0.0f ? xw[(ET * 16) * 64 + lane] : -INFINITY;
-        mm = fmaxf(mm, aw[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < NQ; w++) {
-        const float *xw = reinterpret_cast<const float *>(smem + (qh * NQ + w) * WPART);
-        aw[w] = aw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(aw[w] - mm);
-        den += aw[w] * xw[(ET * 16 + 1) * 64 + lane];
-    }
-    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    const int qi = q0 + l32;
-#pragma unroll
-    for (int cidx = 0; cidx < 2; cidx++) {
-        const int tg = kq * 2 + cidx, t = tg >> 2, g = tg & 3;
-        float o4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int w = 0; w < NQ; w++) {
-            const float *xw = reinterpret_cast<const float *>(smem + (qh * NQ + w) * WPART);
-#pragma unroll
-            for (int i = 0; i < 4; i++) o4[i] += aw[w] * xw[(t * 16 + 4 * g + i) * 64 + lane];
-        }
-        if (qi < p.Lq) {
-            const long off = (long)b * p.os[3] + (long)h * p.os[2] + (long)qi * p.os[1] + 32 * t + 8 * g + 4 * hl;
-            if (p.out_f32) {
-                const float4v o = {o4[0] * inv, o4[1] * inv, o4[2] * inv, o4[3] * inv};
-                *reinterpret_cast<float4v *>(reinterpret_cast<float *>(p.out) + off) = o;
-            } else {
-                const half4v o = {(half_t)(o4[0] * inv), (half_t)(o4[1] * inv), (half_t)(o4[2] * inv), (half_t)(o4[3] * inv)};
-                *reinterpret_cast<half4v *>(reinterpret_cast<half_t *>(p.out) + off) = o;
-            }
-        }
-    }
-}
-
-
-// ------------------------------------------------------------------------------------------
 // One workgroup (4 waves) per (query row, key split).  A wave walks keys 8 at a
 // time: 8 lanes share a key, each owning 8-element head-dim chunks c, c+8, ...
 // (NCH chunks, E <= 64 NCH).  Every 8-lane group keeps its own running
@@ -1529,8 +1047,6 @@ constexpr int flash_lds_bytes(int EP) { return 3 * 64 * (EP + 8) * 2 + 3 * 64 * 
 // A mask that depends on the key only rides in LDS behind the stages: whole key blocks (of `bcs` keys) and one zero
 constexpr int FLASH_KEYMASK_MAX = 4096;
 constexpr int flash_keymask_bytes(int64_t Lk, int bcs) { return (int)(((Lk + bcs - 1) / bcs * bcs + 1) * 2 + 15) / 16 * 16; }
-constexpr int flash_short_lds_bytes(int NW) { return NW * 64 * flash_vld(64) * 2; }
-constexpr int flash_pair_lds_bytes() { return 4 * (64 * (64 + 8) * 2 + 64 * flash_vld(64) * 2); }
 
 bool vec_addressable(const half_t *ptr, const long st[4], int E) {
     return st[0] == 1 && E % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0 && st[3] % 8 == 0 && aligned_to(ptr, 16);
@@ -1606,33 +1122,28 @@ int flash_splits_over_workgroups(int64_t E, int64_t Lq, int64_t Lk, int64_t H, i
     return (int)want;
 }
 
-// Head size 64, no mask, and at most about one 32-query workgroup per compute unit: flash_short_kernel, unless key
-// splits over workgroups are estimated faster still (a handful of tiles over thousands of keys).  A SIMD finishes a 32 x 64 block of it in
-// about 1.3 us whether it holds one of its waves or two, so what counts is that every SIMD gets one wave: 6 heads x 1344
-// (252 workgroups) 18.5 -> 11.8 us, 12 heads x 577 12.3 -> 7.6 us, 4 heads x 640 over 300 keys 10.6 -> 6.3 us; at 6
-// heads x 1370 two CUs of 256 hold two workgroups, which then take twice as long (17.6 us against 18.5 us), and
-// beyond that the 128-query forms are as fast or faster.
-bool flash_short(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B) {
-    const int64_t tiles = ceil_div(Lq, 32) * H * B, cus = mi_num_cus();
-    if (E != 64 || Lk < 128 || tiles > cus + cus / 16) return false;
-    // against key splits over workgroups (few tiles, many keys): 4.5 us + 1.3 us per block of a wave's quarter here,
-    // 3 us + 1 us per block of a split + the 6 us merge launch there
-    const int64_t blocks = ceil_div(Lk, 64), ns = flash_splits(E, Lq, Lk, H, B);
-    return ns == 1 || 4.5 + 1.3 * (double)ceil_div(blocks, 4) <= 9.0 + 1.0 * (double)ceil_div(blocks, ns);
-}
-
-// The same on 64-query tiles (flash_pair_kernel) where the 32-query tiles would not all find a CU of their own but the
-// 64-query tiles do.  Replayed, against what ran there before (key halves on 128-query tiles, or 32-query tiles two to a
-// CU): 6 heads x 1370 17.8 -> 14.3 us, 16 x 1024 15.8 -> 11.3, 10 x 1500 26.5 -> 14.8, 8 x 2048 31.1 -> 19.6, 6 x 2500
-// 34.5 -> 21.1, 4 x 4096 44.1 -> 30.0; where the 32-query tiles fit they are faster (6 x 1344 11.7 against 13.4 us), and
-// at 12 x 1370 (264 tiles of 64) the key-halves form is (19.4 against 26.5 us).
-bool flash_pair(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B) {
-    const int64_t tiles32 = ceil_div(Lq, 32) * H * B, tiles64 = ceil_div(Lq, 64) * H * B, cus = mi_num_cus();
-    return E == 64 && Lk >= 128 && tiles32 > cus && tiles64 <= cus;
-}
-// either of the two: one launch, keys not split over workgroups
-bool flash_unsplit(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B) {
-    return !flash_few_queries(E, Lq, Lk, H, B) && (flash_pair(E, Lq, Lk, H, B) || flash_short(E, Lq, Lk, H, B));
+// Waves of flash_tile_kernel for a call without a dense mask, or 0 where another form is the better one.  Timed on 190 shapes in
+// a replayed graph (head sizes 16 to 128, 2 to 4096 queries and keys, with and without a key mask), the choice is within
+// 1.2 % of the best on average.  Head sizes 16, 32, 72 and 128 were padded to 64, 96 and 128-query tiles: 1.3 to 1.5
+// times as long on average.  At 64 (12 us instead of 14.3 at 6 heads x 1370, 24.9 instead of 35 at 320 x 300) only a chip
+// full of long rows stays with the 256-query and key-halves forms, whose tiles read K and V an eighth as often: from some
+// 820 workgroups over 43 key tiles on (20 x 1500: 23.3 us there, 24.2 here; 16 x 4096: 79 against 103).
+// Eight waves where every workgroup has a CU of its own and a wave still gets two tiles (6 x 1344: 9.3 us, 10.6 on four);
+// two where the grid fills the chip without more: the merge at the end is what a wave costs (16 x 8 windows of 256 x 72:
+// 12.1 us, 15.7 on four, 23.7 on eight).
+int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B) {
+    const int64_t wgs = ceil_div(Lq, 32) * H * B, nt = ceil_div(Lk, 32), cus = mi_num_cus();
+    if (!mi_sdpa_tile_takes(E) || Lq < 2 || Lk < 1) return 0;
+    if (E == 64 && wgs * 10 >= cus * 32 && nt >= 43) return 0;
+    const int waves = wgs <= cus && nt >= 16 ? 8 : wgs * 4 >= cus * 11 ? 2 : 4;
+    // A handful of tiles over thousands of keys: against keys split over workgroups and a merge launch.  A wave takes 0.55
+    // to 1.2 us a tile here; there it is 1 us a 64-key block of a split and 9 us of two launches.
+    // Few queries over 4096 keys or more stay split (level there: 23 x 4096 x 8 heads in 12.7 us, 11.3 here).
+    if (flash_few_queries(E, Lq, Lk, H, B) && nt >= 128) return 0;
+    const int64_t ns = Lq < 64 && !flash_few_queries(E, Lq, Lk, H, B) ? rows_splits(Lq, Lk, H, B) : flash_splits(E, Lq, Lk, H, B);
+    const double tile_us = E <= 64 ? 0.55 : E == 72 ? 0.8 : 1.2;
+    if (ns > 1 && 4.0 + tile_us * (double)ceil_div(nt, waves) > 9.0 + 1.0 * (double)ceil_div(ceil_div(Lk, 64), ns)) return 0;
+    return waves;
 }
 
 // A single query row (a decode step) runs in one launch of sdpa_decode_kernel: the work follows the device-side kv_len
@@ -1699,13 +1210,18 @@ bool flash_bias_ok(const SdpaArgs &a) {
     return aligned_to(a.bias, 4) && a.bs[1] % 2 == 0 && a.bs[2] % 2 == 0 && a.bs[3] % 2 == 0;
 }
 
+// What the fused kernels need of the operands, whatever the extents.
+bool flash_operands_ok(const SdpaArgs &a) {
+    const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
+    const bool out_ok = (aligned_to(a.out, 16) || a.out == nullptr) && a.os[0] == 1 && a.os[1] % 8 == 0 && a.os[2] % 8 == 0 && a.os[3] % 8 == 0;
+    return mi_plan_mfma() && vec && out_ok && a.scale > 0.0f && a.E <= 128 && a.Lk >= 1;
+}
+
 int sdpa_path(const SdpaArgs &a) {
     if (a.E < 1 || a.E > 256 || a.Lq < 0 || a.Lk < 0 || a.H < 1 || a.B < 1) return MI_SDPA_DECLINE;
     if (a.H > 65535 || a.B > 65535 || (int64_t)a.Lq * a.H * 64 > INT32_MAX) return MI_SDPA_DECLINE;
-    bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
-    bool out_ok = (aligned_to(a.out, 16) || a.out == nullptr) && a.os[0] == 1 && a.os[1] % 8 == 0 && a.os[2] % 8 == 0 && a.os[3] % 8 == 0;
     const bool enough_queries = a.Lq >= 64 || (!a.bias && flash_few_queries(a.E, a.Lq, a.Lk, a.H, a.B));
-    if (mi_plan_mfma() && vec && out_ok && (!a.bias || flash_bias_ok(a)) && a.scale > 0.0f && a.E <= 128 && enough_queries && a.Lk >= 1) return MI_SDPA_FLASH;
+    if (flash_operands_ok(a) && (!a.bias || flash_bias_ok(a)) && enough_queries) return MI_SDPA_FLASH;
     return MI_SDPA_ROWS;
 }
 
@@ -1756,8 +1272,7 @@ int mi_sdpa_init() {
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * flash_lds_bytes(64)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, true, 2, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * flash_lds_bytes(64)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<96, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * flash_lds_bytes(96)) != hipSuccess;
-    bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_short_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_short_lds_bytes(4)) != hipSuccess;
-    bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_pair_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, flash_pair_lds_bytes()) != hipSuccess;
+    bad |= mi_sdpa_tile_init();
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<96, false>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_lds_bytes(96)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<128, false>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_lds_bytes(128)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, false, 1, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_lds_bytes(64)) != hipSuccess;
@@ -1779,7 +1294,7 @@ extern "C" {
 size_t mi_sdpa_f16_workspace(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, int has_bias) {
     // sized for the path the call will most likely take: the fused kernel's key splits for Lq >= 64 without
     // an additive mask (unused if the operands turn out not to be 16-byte addressable), the rows kernel's below
-    int ns = Lq >= 64 ? ((has_bias || flash_unsplit(E, Lq, Lk, H, B)) ? 1 : flash_splits(E, Lq, Lk, H, B)) : rows_splits(Lq, Lk, H, B);
+    int ns = Lq >= 64 ? ((has_bias || flash_tile_waves(E, Lq, Lk, H, B)) ? 1 : flash_splits(E, Lq, Lk, H, B)) : rows_splits(Lq, Lk, H, B);
     // few queries over many keys: whichever of the two routes the operands allow must find its partials' room
     if (!has_bias && flash_few_queries(E, Lq, Lk, H, B) && few_query_splits(Lk, H, B) > ns) ns = few_query_splits(Lk, H, B);
     if (ns <= 1) return 0;
@@ -1801,7 +1316,7 @@ int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4], const void *k, c
     int path = sdpa_path(a);
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
     if (nsplit_out) *nsplit_out = (path == MI_SDPA_ROWS && Lq < 64) ? (one_pass_decode(a, vec) ? decode_splits(E, Lk, H, B) : rows_splits(Lq, Lk, H, B))
-                                  : (path == MI_SDPA_FLASH && !has_bias && !flash_unsplit(E, Lq, Lk, H, B)) ? flash_splits(E, Lq, Lk, H, B) : 1;
+                                  : (path == MI_SDPA_FLASH && !has_bias && !flash_tile_waves(E, Lq, Lk, H, B)) ? flash_splits(E, Lq, Lk, H, B) : 1;
     return path;
 }
 
@@ -1829,6 +1344,12 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
     hipStream_t st = (hipStream_t)stream;
     int path = sdpa_path(a);
     if (path == MI_SDPA_DECLINE) return MI_DECLINE_EXTENT;
+    // (also few queries, which the plan reports with the rows kernel: it reads K and V once per query)
+    if ((!bias || (!a.bias_f32 && (a.bs[1] == 0 || Lq == 1) && Lk <= MI_SDPA_TILE_KEYMASK_MAX)) && (path == MI_SDPA_FLASH || flash_operands_ok(a))) {
+        const int waves = flash_tile_waves(E, Lq, Lk, H, B);
+        rc = waves ? mi_sdpa_tile_launch(a, waves, bias != nullptr, st) : MI_DECLINE_EXTENT;
+        if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
+    }
     if (path == MI_SDPA_FLASH) {
         // The 8-wave ping-pong kernel when 256-query workgroups still cover most of the chip.
         const bool pp = !a.bias && E <= 64 && ceil_div(Lq, 256) * H * B * 4 >= (int64_t)mi_num_cus() * 3;
@@ -1865,14 +1386,6 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
         } else if (pp) {
             dim3 grid((unsigned)ceil_div(Lq, 256), (unsigned)H, (unsigned)B);
             hipLaunchKernelGGL((flash_fwd_kernel<64, true>), grid, dim3(512), flash_lds_bytes(64), st, a);
-        } else if (!flash_few_queries(E, Lq, Lk, H, B) && flash_pair(E, Lq, Lk, H, B)) {
-            a.nsplit = 1;
-            dim3 grid((unsigned)ceil_div(Lq, 64), (unsigned)H, (unsigned)B);
-            hipLaunchKernelGGL(flash_pair_kernel, grid, dim3(512), flash_pair_lds_bytes(), st, a);
-        } else if (!flash_few_queries(E, Lq, Lk, H, B) && flash_short(E, Lq, Lk, H, B)) {
-            a.nsplit = 1;
-            dim3 grid((unsigned)ceil_div(Lq, 32), (unsigned)H, (unsigned)B);
-            hipLaunchKernelGGL(flash_short_kernel<4>, grid, dim3(256), flash_short_lds_bytes(4), st, a);
         } else {
             // few query blocks: split the keys over workgroups too, if the caller brought the workspace for it
             a.nsplit = flash_splits(E, Lq, Lk, H, B);

@@ -1,0 +1,306 @@
+// Fused attention for gfx950 on 32-query workgroups: grids that the 128- and 256-query forms of sdpa.hip leave the chip
+// idle on, and head sizes that those pad to 64 or 96.
+#include "sdpa_common.hpp"
+
+namespace {
+
+// A workgroup owns 32 queries of one (head, batch); its NW waves take the 32-key tiles w, w + NW, ... of the keys, each with its
+// own softmax state and its own stretch of LDS, and share nothing until the (O, M, l) of all waves meet in LDS at the end
+// (the rescaling identity of flash.jl:1385-1391).  No barrier in the loop, nothing staged for anyone else.
+//
+// What bounds it is the vector ALU and the latency of a tile's serial chain (first product, exponentials, second product),
+// so what counts is waves: everything a wave holds fits 128 registers at head size 64 and 8.5 KB of LDS, four waves a SIMD.
+// To that end K and V travel global -> LDS without passing through registers (global_load_lds_dwordx4), into one buffer
+// each: the next tile's K is requested when this tile's fragments have been read, the next V likewise, so a request has
+// the other product and the exponentials to arrive under.  (Fragments straight from memory -- a lane per key row -- cost
+// the CU's vector-memory path a cache line per 32 bytes.)  A second buffer a wave, query tiles that start at different
+// keys, and 64 queries a wave measured the same or slower (6 heads x 1370: 12.3 us; 13.8, 13.4 and 14.7).
+//
+// A direct load cannot pad, so the EC 16-byte chunks of a row (EC = E / 8) are permuted instead: K row r holds chunk c at
+// c ^ kswz(r) such that any eight rows' reads of one chunk fall into eight bank groups, V row r at c ^ vswz(r) such that the
+// four rows of a transposing read do.  Rows of nine chunks (72) need none for K.
+//
+// Products, register layouts and the lazily moved reference point M are flash_fwd_kernel's: S^T = K Q^T, O^T = V^T P^T, -M in
+// the first product's accumulators.  MASK: an fp16 mask of the key alone, copied to LDS once; it joins in one more k-step
+// as (mask, mask) x (log2(e) split into two positive fp16 parts), so that -inf stays -inf.
+// Waves a SIMD that the registers of an instance are budgeted for.
+constexpr int tile_waves(int EC) { return EC == 16 ? 2 : EC == 9 ? 3 : 4; }
+
+template <int EC, int NW, bool MASK>
+__global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(SdpaArgs p) {
+    constexpr int E = EC * 8, KS = (E + 15) / 16, ET = (E + 31) / 32;
+    constexpr int TILE_BYTES = 32 * EC * 16, NI = (32 * EC + 63) / 64;      // one operand's tile; 1 KB requests for it
+    constexpr int WPART = (ET * 16 + 2) * 256, WSTRIDE = WPART > 2 * TILE_BYTES ? WPART : 2 * TILE_BYTES;
+    constexpr float TH = 8.0f;
+    extern __shared__ __align__(16) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hl = lane >> 5, l32 = lane & 31;
+    char *const wave_lds = smem + wave * WSTRIDE;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem + wave * WSTRIDE;
+    half_t *const Ms = reinterpret_cast<half_t *>(smem + NW * WSTRIDE);
+
+    // workgroups are dealt to the 8 XCDs round robin: each gets a contiguous run, so a head's query tiles share an L2
+    int qblk, h, b;
+    {
+        const int nqb = gridDim.x, total = nqb * gridDim.y * gridDim.z;
+        int id = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
+        const int xcd = id & 7, full = total >> 3, rem = total & 7;
+        id = xcd * full + min(xcd, rem) + (id >> 3);
+        qblk = id % nqb;
+        h = (id / nqb) % gridDim.y;
+        b = id / (nqb * gridDim.y);
+    }
+    const int q0 = qblk * 32;
+    const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];
+    int Lk = p.Lk;
+    if (p.kv_len) Lk = max(0, min(Lk, p.kv_len[b]));
+    const int nt = (Lk + 31) / 32, last = p.Lk - 1;           // rows past the end re-read the last key that exists
+    const float c = p.scale * LOG2E;
+
+    u32x4 qraw[KS];
+    {
+        const int qr = min(q0 + l32, p.Lq - 1);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            const int e = 16 * ks + 8 * hl;
+            qraw[ks] = e < E ? ldg16(qb + (long)qr * p.qs[1] + e) : z;
+        }
+    }
+    auto kswz = [](int r) { return EC == 9 ? 0 : EC == 2 ? (r >> 2) & 1 : EC == 4 ? (r >> 1) & 3 : r & 7; };
+    auto vswz = [](int r) { return EC == 8 || EC == 16 ? (r & 3) * 2 : 0; };
+    // Requests: lane and request i stand for 16-byte slot s = 64 i + lane of the tile, row s / EC, position s % EC.
+    const char *const kbase = reinterpret_cast<const char *>(p.k + h * p.ks[2] + b * p.ks[3]);
+    const char *const vbase = reinterpret_cast<const char *>(p.v + h * p.vs[2] + b * p.vs[3]);
+    const uint32_t kpitch = (uint32_t)p.ks[1] * 2, vpitch = (uint32_t)p.vs[1] * 2;
+    uint32_t koff[NI], voff[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int s = 64 * i + lane, row = s / EC, pos = s % EC;
+        koff[i] = row * kpitch + (pos ^ kswz(row)) * 16;
+        voff[i] = row * vpitch + (pos ^ vswz(row)) * 16;
+    }
+    auto request = [&](bool is_k, int tile) {
+        const char *org = (is_k ? kbase : vbase) + (long)tile * 32 * (is_k ? kpitch : vpitch);
+        const int over = tile * 32 + 31 - last;                   // rows of the tile past the last key
+        const uint32_t dst = lds0 + (is_k ? 0 : TILE_BYTES);
+        if (over <= 0) {                                          // uniform
+            if constexpr ((32 * EC) % 64 == 0) {
+                asm volatile("s_mov_b32 m0, %0" ::"s"(dst) : "memory");
+#pragma unroll
+                for (int i = 0; i < NI; i++)
+                    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_add_u32 m0, m0, 0x400" ::"v"(is_k ? koff[i] : voff[i]), "s"(org) : "memory", "scc");
+                return;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int s = 64 * i + lane;
+            uint32_t off = is_k ? koff[i] : voff[i];
+            if (over > 0) off -= max(0, s / EC - (31 - over)) * (is_k ? kpitch : vpitch);
+            if ((32 * EC) % 64 == 0 || s < 32 * EC)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(org), "s"(dst + i * 1024) : "memory");
+        }
+    };
+    if (wave < nt) { request(true, wave); request(false, wave); }
+    if constexpr (MASK) {
+        const unsigned short *mrow = reinterpret_cast<const unsigned short *>(p.bias) + (long)h * p.bs[2] + (long)b * p.bs[3];
+        for (int i = threadIdx.x; i < nt * 32; i += NW * 64)
+            reinterpret_cast<unsigned short *>(Ms)[i] = i < p.Lk ? mrow[(long)i * p.bs[0]] : (unsigned short)0;
+    }
+    half8v qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+        const half8v t = as_half8(qraw[ks]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) qf[ks][j] = (half_t)((float)t[j] * c);
+    }
+    float16v o_acc[ET], negm;
+#pragma unroll
+    for (int r = 0; r < 16; r++) negm[r] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < ET; t++) o_acc[t] = negm;
+    float m_run = 0.0f, l_run = 0.0f;
+    half8v qext;
+    if constexpr (MASK) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) qext[j] = (half_t)0.0f;
+        if (hl == 0) { qext[0] = (half_t)1.4423828125f; qext[1] = (half_t)(1.44269504088896340736f - 1.4423828125f); }
+        __syncthreads();                                          // the mask row is in place
+    }
+    const int vk = (lane & 15) >> 2;                              // key of a transposing read's four
+    auto vchunk = [&](int t) { return min(4 * t + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), EC - 1) ^ vswz(vk); };
+    auto probs = [&](const float16v &sx, half8v (&pf)[2], float &l) {
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            const float p0 = __builtin_amdgcn_exp2f(sx[r]), p1 = __builtin_amdgcn_exp2f(sx[r + 1]);
+            pf[r >> 3][r & 7] = (half_t)p0;
+            pf[r >> 3][(r & 7) + 1] = (half_t)p1;
+            l += p0 + p1;
+        }
+    };
+    bool first = true;
+    const char *const kt_lds = wave_lds, *const vt_lds = wave_lds + TILE_BYTES;
+    for (int tile = wave; tile < nt; tile += NW) {
+        const bool more = tile + NW < nt;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");          // K has landed; V may be on its way
+        half8v kf[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+            kf[ks] = *reinterpret_cast<const half8v *>(kt_lds + (l32 * EC + (min(2 * ks + hl, EC - 1) ^ kswz(l32))) * 16);
+        half8v kx = {};
+        if constexpr (MASK) {
+            const half_t m = Ms[tile * 32 + l32];
+            kx[0] = hl == 0 ? m : (half_t)0.0f;
+            kx[1] = kx[0];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (more) request(true, tile + NW);
+        float16v sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[0], qf[0], negm, 0, 0, 0);
+#pragma unroll
+        for (int ks = 1; ks < KS; ks++) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
+        if constexpr (MASK) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
+        if (tile * 32 + 32 > Lk) {                                // the ragged last tile: excluded keys get -inf
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (tile * 32 + 8 * (r >> 2) + 4 * hl + (r & 3) >= Lk) sc[r] = -INFINITY;
+        }
+        half8v pf[2];
+        float l_new = l_run;
+        probs(sc, pf, l_new);
+        if (__any(first || !(l_new - l_run < 65504.0f))) {        // flash_fwd_kernel says why
+            float tmax = fmaxf(sc[0], sc[1]);
+#pragma unroll
+            for (int r = 2; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, sc[r]), sc[r + 1]);
+            const float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+            const bool grow = (mx > TH || first) && mx != -INFINITY;
+            // (M is fp32 here and may lie far below zero after a first tile of masked keys: nothing to rescale yet)
+            const float d = grow ? mx : 0.0f, alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-d);
+            m_run += d;
+            l_run *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; r++) { negm[r] = -m_run; sc[r] -= d; }
+#pragma unroll
+            for (int t = 0; t < ET; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o_acc[t][r] *= alpha;
+            l_new = l_run;
+            probs(sc, pf, l_new);
+            first = first && mx == -INFINITY;                     // the reference point is found with the first key that counts
+        }
+        l_run = l_new;
+        if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");        // V has landed; the next K may be on its way
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        half8v vf[ET][2];
+#pragma unroll
+        for (int t = 0; t < ET; t++)
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) {
+                const char *vq = vt_lds + ((16 * bb + 4 * hl + vk) * EC + vchunk(t)) * 16 + (lane & 1) * 8;
+                const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)vq);
+                const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq + 8 * EC * 16));
+                const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                vf[t][bb] = __builtin_bit_cast(half8v, both);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (more) request(false, tile + NW);
+#pragma unroll
+        for (int t = 0; t < ET; t++)
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][bb], pf[bb], o_acc[t], 0, 0, 0);
+    }
+    // The waves' partials, lane-major, each into its own stretch, then every wave finishes (t, g) pairs: head dims
+    // 32 t + 8 g + 4 hl .. +3 of its lane's query.
+    float *xo = reinterpret_cast<float *>(wave_lds);
+#pragma unroll
+    for (int t = 0; t < ET; t++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+            const float4v v = {o_acc[t][4 * r4], o_acc[t][4 * r4 + 1], o_acc[t][4 * r4 + 2], o_acc[t][4 * r4 + 3]};
+            *reinterpret_cast<float4v *>(xo + (t * 4 + r4) * 256 + lane * 4) = v;
+        }
+    xo[ET * 1024 + lane] = m_run;
+    xo[ET * 1024 + 64 + lane] = l_run + __shfl_xor(l_run, 32, 64);      // both lanes of a query hold half of its row sum
+    __syncthreads();
+    float aw[NW], mm = -INFINITY, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float *xw = reinterpret_cast<const float *>(smem + w * WSTRIDE) + ET * 1024;
+        aw[w] = xw[64 + lane] > 0.0f ? xw[lane] : -INFINITY;  // a wave that saw no valid key has a meaningless reference point
+        mm = fmaxf(mm, aw[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float *xw = reinterpret_cast<const float *>(smem + w * WSTRIDE) + ET * 1024;
+        aw[w] = aw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(aw[w] - mm);
+        den += aw[w] * xw[64 + lane];
+    }
+    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+    const int qi = q0 + l32;
+    for (int tg = wave; tg < EC; tg += NW) {
+        float4v o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float4v x = *reinterpret_cast<const float4v *>(reinterpret_cast<const float *>(smem + w * WSTRIDE) + tg * 256 + lane * 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[i] += aw[w] * x[i];
+        }
+        if (qi < p.Lq) {
+            const long off = (long)b * p.os[3] + (long)h * p.os[2] + (long)qi * p.os[1] + 8 * tg + 4 * hl;
+            if (p.out_f32) {
+                const float4v r = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+                *reinterpret_cast<float4v *>(reinterpret_cast<float *>(p.out) + off) = r;
+            } else {
+                const half4v r = {(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
+                *reinterpret_cast<half4v *>(reinterpret_cast<half_t *>(p.out) + off) = r;
+            }
+        }
+    }
+}
+
+template <int EC, int NW>
+constexpr int tile_lds_bytes() {
+    constexpr int part = ((EC * 8 + 31) / 32 * 16 + 2) * 256, tiles = 2 * 32 * EC * 16;
+    return NW * (part > tiles ? part : tiles);
+}
+template <int EC, int NW>
+int launch_tiles(const SdpaArgs &p, bool mask, hipStream_t st) {
+    const dim3 grid((unsigned)ceil_div(p.Lq, 32), (unsigned)p.H, (unsigned)p.B);
+    const int lds = tile_lds_bytes<EC, NW>();
+    if (mask) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, true>), grid, dim3(NW * 64), lds + (int)round_up((size_t)ceil_div(p.Lk, 32) * 64, 16), st, p);
+    else      hipLaunchKernelGGL((flash_tile_kernel<EC, NW, false>), grid, dim3(NW * 64), lds, st, p);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
+template <int EC>
+int launch_waves(const SdpaArgs &p, int waves, bool mask, hipStream_t st) {
+    return waves == 2 ? launch_tiles<EC, 2>(p, mask, st) : waves == 4 ? launch_tiles<EC, 4>(p, mask, st) : launch_tiles<EC, 8>(p, mask, st);
+}
+template <int EC, int NW>
+int raise() {
+    const int lds = tile_lds_bytes<EC, NW>();
+    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + 2 * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
+           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
+}
+template <int EC>
+int raise_all() { return raise<EC, 2>() | raise<EC, 4>() | raise<EC, 8>(); }
+
+}  // namespace
+
+bool mi_sdpa_tile_takes(int64_t E) { return E == 16 || E == 32 || E == 64 || E == 72 || E == 128; }
+
+int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool mask, hipStream_t st) {
+    if (!mi_sdpa_tile_takes(p.E) || (mask && p.Lk > MI_SDPA_TILE_KEYMASK_MAX)) return MI_DECLINE_EXTENT;
+    // per-lane load offsets are 32-bit byte offsets from a tile's first row
+    if (p.ks[1] < 0 || p.vs[1] < 0 || p.ks[1] * 64 >= (1l << 31) || p.vs[1] * 64 >= (1l << 31)) return MI_DECLINE_EXTENT;
+    switch (p.E) {
+    case 16: return launch_waves<2>(p, waves, mask, st);
+    case 32: return launch_waves<4>(p, waves, mask, st);
+    case 64: return launch_waves<8>(p, waves, mask, st);
+    case 72: return launch_waves<9>(p, waves, mask, st);
+    default: return launch_waves<16>(p, waves, mask, st);
+    }
+}
+
+int mi_sdpa_tile_init() {
+    return raise_all<2>() | raise_all<4>() | raise_all<8>() | raise_all<9>() | raise_all<16>();
+}
