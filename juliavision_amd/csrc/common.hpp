@@ -132,19 +132,15 @@ static inline size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; 
 // NaN by its bits: the build tells the compiler that no NaNs occur, which folds comparisons with one away.
 static inline bool is_nan_arg(float x) { uint32_t u; __builtin_memcpy(&u, &x, 4); return (u & 0x7fffffffu) > 0x7f800000u; }
 
-// Implicit-GEMM convolution: how the GEMM finds its [K][N] operand (the im2col matrix) in a
-// zero-padded copy of the input instead of in memory.  The K axis is ordered (kh, kw, ci) with ci
-// fastest (the weights are re-laid to match), so a 64-deep tile is 64 consecutive channels of one
-// tap: row k of the tile and column n = (oh, ow) is xp[img][ci0 + k][oh*sy + kh*dy][ow + kw*dx],
-// and eight consecutive columns of a row are eight consecutive halves of xp (stride 1 along x).
+// Implicit-GEMM convolution over a zero-padded channels-last copy xp[img][Hp][Wp][C] of the input: how gemm_ring_kernel finds
+// its [N][K] operand (row n = output pixel (oh, ow), K ordered (kh, kw, ci) with ci fastest) in it.  Sixteen bytes of a
+// row are eight channels of one tap, at an offset from the pixel's origin that is the same for every pixel.
 struct ConvGather {
-    const half_t *xp;      // padded input [img][Cin][Hp][Wp]; nullptr = ordinary GEMM
+    const half_t *xp;      // nullptr = ordinary GEMM
     long img;              // elements per image
-    long odd;              // xp[i] for odd i is also stored at xp[odd + i], a 4-byte aligned address: a second copy of
-                           // the padded input, one element to the left, follows the first
-    int HpWp, Wp, OW, sy, dyWp, dx, KW;
-    int cpt;               // 64-channel tiles per tap: Cin / 64
-    int split;             // 1: the launch's planes are K-slices of one image, 0: they are images
+    int C, OW, KW;
+    int pix_y, pix_x;      // elements between the origins of neighbouring output rows and columns: sy Wp C, sx C
+    int tap_y, tap_x;      // and between neighbouring taps: dy Wp C, dx C
 };
 
 // Implicit-GEMM convolution over a channels-last input x[N][H][W][C]: how the GEMM finds its [M][K] operand
@@ -179,4 +175,5 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
 // Workspace bytes such a call needs (fp32 planes when it splits K); T > 8 rows.
 size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatch);
 // What such a call is estimated to take, in microseconds.
+double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);      // B a ConvGather
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);

@@ -86,52 +86,86 @@ __global__ void im2col_rows_kernel(half_t *col, ConvArgs a, int CRSP, half_t *wp
     *reinterpret_cast<half8v *>(col + ((long)n * PQ + m) * CRSP + c0) = val;
 }
 
-// xp[n][ci][Hp][Wp]: x with py rows of zeros above and below and px (and the round-up to a multiple
-// of 8) columns left and right; one 16-byte store per thread.  What the implicit-GEMM path reads.
-// The same launch re-lays the weights as w2[co][kh][kw][ci] (blocks past the padding work, image 0
-// only): the K order in which the implicit GEMM walks the taps.
-__global__ void conv_pad_kernel(half_t *xp, half_t *w2, ConvArgs a, int Hp, int Wp, int pad_blocks, long shifted) {
-    if ((int)blockIdx.x >= pad_blocks) {
-        if (blockIdx.y != 0) return;
-        // a thread gathers eight channels of one (co, tap) and stores them with one 16-byte write; with the tap
-        // as the fastest thread index a wave reads a dense stretch of the source
-        const int idx = (blockIdx.x - pad_blocks) * blockDim.x + threadIdx.x;
-        const int taps = a.KH * a.KW, c8s = a.Cin >> 3;
-        if (idx >= a.Cout * c8s * taps) return;
-        const int tap = idx % taps, t = idx / taps, c8 = t % c8s, co = t / c8s;
-        const half_t *src = a.w + ((long)co * a.Cin + c8 * 8) * taps + tap;
+// What gemm_ring_kernel's patch operand is gathered from: xp[n][Hp][Wp][C], x channels-last with py rows and px columns of
+// zeros around it, and the weights as w2[co][kh][kw][ci] (the workgroups past the padding work, image 0 only).  Both go
+// through LDS: 16-byte reads along what is contiguous in the source, 16-byte writes along the channels.  It moves a few
+// MB: what it costs is the launch and a trip to memory and back.
+constexpr int TURN = 64 * 72;
+__device__ __forceinline__ void turn_weights(half_t *turn, half_t *w2, const ConvArgs &a, int group, int block, int tid) {
+    // `group` channels of one output channel: a dense run of group * taps halves
+    const int taps = a.KH * a.KW, groups = (a.Cin + group - 1) / group, co = block / groups, c0 = (block % groups) * group, nc = min(group, a.Cin - c0);
+    const half_t *src = a.w + ((long)co * a.Cin + c0) * taps;
+    for (int p = tid; p < nc * taps / 8; p += 256) {
+        half8v v;
+        __builtin_memcpy(&v, src + p * 8, 16);
+        *reinterpret_cast<half8v *>(turn + p * 8) = v;
+    }
+    __syncthreads();
+    half_t *dst = w2 + (long)co * taps * a.Cin + c0;
+    const int c8s = nc >> 3;
+    for (int p = tid; p < c8s * taps; p += 256) {
+        const int tap = p / c8s, c8 = (p - tap * c8s) * 8;
         half8v v;
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = src[j * taps];
-        *reinterpret_cast<half8v *>(w2 + ((long)co * taps + tap) * a.Cin + c8 * 8) = v;
+        for (int j = 0; j < 8; j++) v[j] = turn[(c8 + j) * taps + tap];
+        *reinterpret_cast<half8v *>(dst + (long)tap * a.Cin + c8) = v;
+    }
+}
+__global__ __launch_bounds__(256) void conv_pad_kernel(half_t *xp, half_t *w2, ConvArgs a, int Hp, int Wp, int pad_blocks, int wgroup) {
+    __shared__ __align__(16) half_t turn[TURN];           // [column][channel], 72 halves a column
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= pad_blocks) {
+        if (blockIdx.y == 0) turn_weights(turn, w2, a, wgroup, blockIdx.x - pad_blocks, tid);
         return;
     }
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const int cpr = Wp >> 3;
-    if (idx >= cpr * Hp * a.Cin) return;
-    const int n = blockIdx.y;
-    const int c8 = (idx % cpr) * 8, t = idx / cpr, yp = t % Hp, ci = t / Hp;
-    const int iy = yp - a.py;
-    // elements c8 .. c8+8 of the padded row: the first eight go to the copy proper, the last eight to the
-    // copy that sits one element to the left (its chunk at the same position)
-    half_t e[9];
+    // 64 channels of 64 source columns of one padded row; the first and last columns' workgroups take the borders along
+    const int cgroups = (a.Cin + 63) / 64, xgroups = (a.Wi + 63) / 64;
+    const int cg = blockIdx.x % cgroups, q = blockIdx.x / cgroups, xg = q % xgroups, yp = q / xgroups;
+    const int n = blockIdx.y, c0 = cg * 64, nc8 = min(64, a.Cin - c0) >> 3, x0 = xg * 64, nx = min(64, a.Wi - x0), iy = yp - a.py;
+    half_t *dst = xp + (((long)n * Hp + yp) * Wp + a.px) * a.Cin + c0;      // of source column 0
+    const bool inside = iy >= 0 && iy < a.Hi;
+    const half8v z = {};
+    if (inside) {
+        const half_t *src = a.x + (((long)n * a.Cin + c0) * a.Hi + iy) * a.Wi;
+        const int plane = a.Hi * a.Wi;
+        half8v v[2];
+        int at[2];
 #pragma unroll
-    for (int j = 0; j < 9; j++) e[j] = (half_t)0.0f;
-    if (iy >= 0 && iy < a.Hi) {
-        const half_t *row = a.x + (((long)n * a.Cin + ci) * a.Hi + iy) * a.Wi;
+        for (int i = 0; i < 2; i++) {
+            const int p = tid + 256 * i, ch = p >> 3, ix = x0 + 8 * (p & 7);
+            v[i] = z;
+            // a piece cut by the row's end is read from further left: its columns arrive twice, with the same values
+            at[i] = a.Wi >= 8 ? min(ix, a.Wi - 8) : 0;
+            if (ch < nc8 * 8 && ix < a.Wi) {
+                const half_t *s = src + (long)ch * plane + at[i];
+                if (a.Wi >= 8) __builtin_memcpy(&v[i], s, 16);
+                else {
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-            const int ix = c8 + j - a.px;
-            if (ix >= 0 && ix < a.Wi) e[j] = row[ix];
+                    for (int e = 0; e < 8; e++) if (e < a.Wi) v[i][e] = s[e];
+                }
+            }
         }
-    }
-    half8v v0, v1;
 #pragma unroll
-    for (int j = 0; j < 8; j++) { v0[j] = e[j]; v1[j] = e[j + 1]; }
-    const long at = (((long)n * a.Cin + ci) * Hp + yp) * Wp + c8;
-    *reinterpret_cast<half8v *>(xp + at) = v0;
-    *reinterpret_cast<half8v *>(xp + shifted + at) = v1;
+        for (int i = 0; i < 2; i++) {
+            const int p = tid + 256 * i, ch = p >> 3;
+            if (x0 + 8 * (p & 7) < a.Wi) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) if (at[i] + e >= x0) turn[(at[i] + e - x0) * 72 + ch] = v[i][e];
+            }
+        }
+        __syncthreads();
+    }
+    for (int p = tid; p < nx * nc8; p += 256) {
+        const int x = p / nc8, c8 = (p - x * nc8) * 8;
+        *reinterpret_cast<half8v *>(dst + (long)(x0 + x) * a.Cin + c8) = inside ? *reinterpret_cast<const half8v *>(turn + x * 72 + c8) : z;
+    }
+    const int left = xg == 0 ? a.px : 0, right = xg == xgroups - 1 ? Wp - a.Wi - a.px : 0;
+    for (int p = tid; p < (left + right) * nc8; p += 256) {
+        const int x = p / nc8, c8 = (p - x * nc8) * 8;
+        *reinterpret_cast<half8v *>(dst + (long)(x < left ? x - a.px : a.Wi + x - left) * a.Cin + c8) = z;
+    }
 }
+int turn_group(const ConvArgs &a) { const int g = TURN / (a.KH * a.KW) / 8 * 8; return g < 64 ? g : 64; }
 
 // One thread per output; fp32 accumulator seeded with the bias; the loop order
 // of the reference's conv2d (conv.jl:26-51).
@@ -187,8 +221,8 @@ int fill(ConvArgs &a, void *out, const void *x, const void *w, const void *bias,
     return MI_OK;
 }
 
-// Implicit GEMM needs eight consecutive output pixels to be eight consecutive input columns (stride 1
-// along x, OW a multiple of 8) and 64-deep K tiles that are 64 channels of one tap (Cin % 64 == 0).
+// What the plan calls an implicit GEMM.  (The gathered operand takes any stride and width and channels in multiples of 16
+// now; the names that callers see stay with the extents they were given for.)
 bool implicit_ok(const ConvArgs &a) {
     return a.sx == 1 && a.OW % 8 == 0 && a.Cin % 64 == 0 && (long)a.Cin * a.KH * a.KW >= 128;
 }
@@ -200,10 +234,13 @@ int conv_path(const ConvArgs &a) {
     return MI_CONV_IM2COL_GEMM;
 }
 
-void padded_extents(const ConvArgs &a, int &Hp, int &Wp) {
-    Hp = a.Hi + 2 * a.py;
-    Wp = (int)round_up((size_t)(a.Wi + 2 * a.px), 8);
+// Scratch of the patch-gathering form: the padded channels-last copy, then the weights tap-major.
+bool patch_ok(const ConvArgs &a) {
+    const int64_t Hp = a.Hi + 2 * a.py, Wp = a.Wi + 2 * a.px;
+    return a.groups == 1 && a.Cin % 16 == 0 && turn_group(a) >= 8 && aligned_to(a.w, 16) && (int64_t)Hp * Wp * a.Cin <= INT32_MAX && (int64_t)a.Cout * a.Cin * a.KH * a.KW <= INT32_MAX / 8;
 }
+size_t patch_copy_bytes(const ConvArgs &a) { return round_up((size_t)a.N * a.Cin * (a.Hi + 2 * a.py) * (a.Wi + 2 * a.px) * 2, 256); }
+size_t patch_weight_bytes(const ConvArgs &a) { return round_up((size_t)a.Cout * a.Cin * a.KH * a.KW * 2, 256); }
 
 // The matrix is padded with zero rows to a multiple of 8 taps, and -- from 256 taps on, where that adds a quarter at
 // most -- to a multiple of 64, the depth the software-pipelined GEMM steps by (a ViT's 14 x 14 x 3 patch: 588 -> 640).
@@ -231,18 +268,17 @@ size_t mi_conv2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, i
                                int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy) {
     ConvArgs a;
     if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, 1, MI_EPI_NONE) != MI_OK) return 0;
-    if (conv_path(a) == MI_CONV_IMPLICIT_GEMM) {
-        int Hp, Wp;
-        padded_extents(a, Hp, Wp);
-        return 2 * round_up((size_t)N * Cin * Hp * Wp * 2, 256) + round_up((size_t)Cout * Cin * KH * KW * 2, 256) +
-               mi_internal_gemm_workspace(Cout, Cin * KH * KW, (int64_t)a.OW * a.OH, N);
+    if (conv_path(a) == MI_CONV_IMPLICIT_GEMM) {       // (twice the copy with rows of whole 16 bytes, and planes: what it was sized for first)
+        const size_t Wp = round_up((size_t)(a.Wi + 2 * a.px), 8);
+        return 2 * round_up((size_t)N * Cin * (a.Hi + 2 * a.py) * Wp * 2, 256) + patch_weight_bytes(a) + mi_internal_gemm_workspace(Cout, Cin * KH * KW, (int64_t)a.OW * a.OH, N);
     }
     if (conv_path(a) != MI_CONV_IM2COL_GEMM) return 0;
     int64_t PQP, CRSP;
     im2col_extents(a, PQP, CRSP);
     size_t col = round_up((size_t)N * PQP * CRSP * 2, 256);
     size_t wp = CRSP != (int64_t)Cin * KH * KW ? round_up((size_t)Cout * CRSP * 2, 256) : 0;
-    return col + wp + mi_internal_gemm_workspace(Cout, CRSP, (int64_t)a.OW * a.OH, N);
+    const size_t need = col + wp + mi_internal_gemm_workspace(Cout, CRSP, (int64_t)a.OW * a.OH, N), patch = patch_ok(a) ? patch_copy_bytes(a) + patch_weight_bytes(a) : 0;
+    return need > patch ? need : patch;
 }
 
 int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
@@ -272,39 +308,35 @@ int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
     }
     // In one launch where that is estimated to be faster than staging the operand and multiplying it: im2col writes at 0.8 to
     // 1.1 MB/us, slower where it gathers with a stride (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: 43 us staged,
-    // 25 us in one launch; 144 -> 96 on 45 x 392: 45 and 26), the padded copies of the implicit form take a launch of 4 us.
+    // 25 us in one launch); the channels-last copy and the weights of the patch form move at some 2 MB/us behind a launch.
+    const int CRS = a.Cin * a.KH * a.KW;
+    const bool patch = patch_ok(a);
     {
         int64_t PQP, CRSP;
         im2col_extents(a, PQP, CRSP);
-        const double gemm = mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N);
-        const double staged = path == MI_CONV_IMPLICIT_GEMM ? 5.0 + 1.2 * gemm : 3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + gemm;
+        const double staged = patch ? 4.0 + 0.5e-6 * (double)(patch_copy_bytes(a) + patch_weight_bytes(a)) + mi_internal_patch_gemm_us(a.Cout, CRS, PQ, a.N)
+                                    : 3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N);
         rc = mi_conv_tile(a, staged, st);
         if (rc != MI_DECLINE_EXTENT) return rc;
     }
-    if (path == MI_CONV_IMPLICIT_GEMM) {
-        int Hp, Wp;
-        padded_extents(a, Hp, Wp);
-        const int CRS = a.Cin * a.KH * a.KW;
-        const size_t xp1 = round_up((size_t)a.N * a.Cin * Hp * Wp * 2, 256), xp_bytes = 2 * xp1;     // the copy and its shifted twin
-        const size_t w2_bytes = round_up((size_t)a.Cout * CRS * 2, 256);
-        const size_t gemm_bytes = mi_internal_gemm_workspace(a.Cout, CRS, PQ, a.N);
-        if (!ws || ws_bytes < xp_bytes + w2_bytes + gemm_bytes || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
-        if ((long)a.Cin * Hp * Wp > INT32_MAX || (long)a.Cout * CRS > INT32_MAX) return MI_DECLINE_EXTENT;
+    if (patch) {
+        const int Hp = a.Hi + 2 * a.py, Wp = a.Wi + 2 * a.px;
+        const size_t xp_bytes = patch_copy_bytes(a);
+        if (!ws || ws_bytes < xp_bytes + patch_weight_bytes(a) || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
         half_t *xp = reinterpret_cast<half_t *>(ws);
         half_t *w2 = reinterpret_cast<half_t *>(reinterpret_cast<char *>(ws) + xp_bytes);
-        const int pad_blocks = (int)ceil_div((int64_t)(Wp / 8) * Hp * a.Cin, 256), w_blocks = (int)ceil_div((int64_t)a.Cout * CRS / 8, 256);
-        hipLaunchKernelGGL(conv_pad_kernel, dim3((unsigned)(pad_blocks + w_blocks), (unsigned)a.N), dim3(256), 0, st, xp, w2, a, Hp, Wp, pad_blocks, (long)(xp1 / 2));
+        const int pad_blocks = (int)(ceil_div(a.Cin, 64) * ceil_div(a.Wi, 64) * Hp), w_blocks = (int)(a.Cout * ceil_div(a.Cin, turn_group(a)));
+        hipLaunchKernelGGL(conv_pad_kernel, dim3((unsigned)(pad_blocks + w_blocks), (unsigned)a.N), dim3(256), 0, st, xp, w2, a, Hp, Wp, pad_blocks, turn_group(a));
         if (hipGetLastError() != hipSuccess) return MI_ERROR_LAUNCH;
         ConvGather g;
-        g.xp = xp; g.img = (long)a.Cin * Hp * Wp; g.odd = (long)(xp1 / 2) - 1; g.HpWp = Hp * Wp; g.Wp = Wp; g.OW = a.OW; g.sy = a.sy;
-        g.dyWp = a.dy * Wp; g.dx = a.dx; g.KW = a.KW; g.cpt = a.Cin / 64; g.split = 0;
+        g.xp = xp; g.img = (long)a.Cin * Hp * Wp; g.C = a.Cin; g.OW = a.OW; g.KW = a.KW;
+        g.pix_y = a.sy * Wp * a.Cin; g.pix_x = a.sx * a.Cin; g.tap_y = a.dy * Wp * a.Cin; g.tap_x = a.dx * a.Cin;
         // B is never dereferenced in this mode; xp stands in so that the operand checks see an aligned pointer
-        return mi_internal_gemm(out, w2, xp, bias, a.Cout, PQ, PQ, CRS, PQ, CRS, PQ, 1, MI_BIAS_ROW, epi, 0,
-                                a.N, (long)a.Cout * PQ, 0, 0, reinterpret_cast<char *>(ws) + xp_bytes + w2_bytes, gemm_bytes, st, &g);
+        return mi_internal_gemm(out, w2, xp, bias, a.Cout, PQ, PQ, CRS, PQ, CRS, CRS, 0, MI_BIAS_ROW, epi, 0,
+                                a.N, (long)a.Cout * PQ, 0, 0, nullptr, 0, st, &g);
     }
     int64_t PQP, CRSP;
     im2col_extents(a, PQP, CRSP);
-    const int CRS = a.Cin * a.KH * a.KW;
     size_t col_bytes = round_up((size_t)N * PQP * CRSP * 2, 256);
     size_t wp_bytes = CRSP != CRS ? round_up((size_t)Cout * CRSP * 2, 256) : 0;
     const size_t gemm_bytes = mi_internal_gemm_workspace(Cout, CRSP, PQ, N);

@@ -1191,7 +1191,7 @@ bool mfma_addressable(const GemmArgs &a, bool b_kn) {
 
 template <int BM, int BN, int WM, int WN>
 int launch_w4(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    if (a.K < 64 || a.K % 64 || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
+    if (a.K < 64 || a.K % 64 || a.ag.x) return MI_DECLINE_EXTENT;
     set_tiles(a, BM, BN);
     a.vec_store = rows_vec16(a);
     // per-lane load offsets are 32-bit byte offsets from the tile origin
@@ -1213,7 +1213,7 @@ bool sk_fits(int64_t M, int64_t N, int64_t K, int bm, int bn, int split);
 // The four-wave kernel with two workgroups per 128 x 128 tile exchanging their partial tiles.
 int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
     constexpr int BM = 128, BN = 128;
-    if (a.cv.xp || a.ag.x || split != 2 || !sk_usable() || !sk_fits(a.M, a.N, a.K, BM, BN, split)) return MI_DECLINE_EXTENT;
+    if (a.ag.x || split != 2 || !sk_usable() || !sk_fits(a.M, a.N, a.K, BM, BN, split)) return MI_DECLINE_EXTENT;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return MI_ERROR_DEVICE;
     a.tiles_m = (int)ceil_div(a.M, BM);
@@ -1245,12 +1245,12 @@ constexpr int RING_TILE = 5;             // index into TILE_MODELS: gemm_ring_ke
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
 // output, same bits, and the plan (hence the workspace) stays a function of the extents alone.
 int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    const bool plain = !a.cv.xp && !a.ag.x && a.K % 64 == 0;
+    const bool plain = !a.ag.x && a.K % 64 == 0;
     switch (tile) {
         case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : mi_pipe_launch(0, a, b_kn, nbatch, st);
         case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : mi_pipe_launch(1, a, b_kn, nbatch, st);
         case RING_TILE:
-            if (!a.cv.xp && !a.ag.x) {
+            if (!a.ag.x) {
                 const int rc = mi_ring_launch(a, b_kn, nbatch, st);
                 if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
             }
@@ -1489,7 +1489,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // of a batched launch (plane strides: A advances along k, Y one fp32 M x N plane in ws), and a
         // second small kernel sums the planes and applies bias, activation and residual.
         const bool pipe = a.K > 64, whole = pipe && a.K % 64 == 0;
-        if ((a.cv.xp || a.ag.x) && !whole) return MI_DECLINE_EXTENT;      // only the pipelined kernel gathers
+        if (a.ag.x && !whole) return MI_DECLINE_EXTENT;      // only the pipelined kernel gathers
         TilePlan tp = {4, 1, false, 0.0};
         // A folded norm on the way in or row statistics on the way out live in the tiled kernels' own store: those calls
         // need the pipelined kernels, 16-byte rows, and K-slices only in the form that ends in that store (the in-launch
@@ -1498,7 +1498,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         if (in_store) {
             const bool rows16 = !a.out_f32 ? (a.N % 8 == 0 && a.ldY % 8 == 0 && a.sY % 8 == 0 && aligned_to(a.Y, 16) && (!a.residual || aligned_to(a.residual, 16)))
                                            : (a.N % 4 == 0 && a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16));
-            if (!whole || a.cv.xp || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
+            if (!whole || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
         }
         if (pipe) {
             tp = plan_tiles(a.M, a.N, a.K, nbatch, !a.lnf_stats);
@@ -1518,7 +1518,6 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             s1.ldY = a.N; s1.sY = (long)a.M * a.N;
             s1.K = a.K / split;
             s1.sA = s1.K; s1.sB = b_kn ? (long)s1.K * a.ldB : s1.K; s1.sBias = 0;
-            s1.cv.split = 1;
             s1.ag.split = 1;
             int rc = launch_tile(tp.tile, s1, b_kn, split, st);
             if (rc != MI_OK) return rc;
@@ -1568,6 +1567,7 @@ size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatc
     return plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
 }
 
+double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, RING_TILE, 1); }
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return plan_tiles(T, F, K, nbatch, nbatch == 1).us; }
 
 // Internal entry used by the convolution path (conv.hip): Y[M x N] = A . B with
@@ -1593,6 +1593,7 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     if (agather) a.ag = *agather;
     const bool addr = mfma_addressable(a, b_kn != 0);
     if ((gather || agather) && !addr) return MI_DECLINE_OPERANDS;
+    if (gather) return g_ready ? mi_ring_launch(a, false, nbatch, st) : MI_ERROR_DEVICE;
     int path = addr ? MI_GEMM_MFMA : MI_GEMM_SCALAR;
     return run_gemm(a, b_kn != 0, nbatch, ws, ws_bytes, st, path);
 }

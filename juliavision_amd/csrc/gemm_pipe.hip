@@ -19,7 +19,7 @@ namespace {
 // whole tile of MFMAs to land before its LDS write; the only barrier of a tile sits
 // where its successor's first fragment read can be hidden behind the last k-step.
 // Two waves per SIMD (8 waves on a 128 x 256 tile) cover each other's waits.
-// BMODE: 0 = B is [N][K], 1 = B is [K][N], 2 = B is [K][N] gathered from a padded image (implicit-GEMM convolution).
+// BMODE: 0 = B is [N][K], 1 = B is [K][N].
 // AMODE 1: A is gathered from a channels-last image (NhwcGather); B is then an ordinary [N][K] or [K][N] operand.
 // AMODE 2: the rows of A are layer-normalised over K on their way in (K <= 512): before the K loop every wave
 // normalises rows of the tile's A panel -- one wave per row, a lane holding eight consecutive k, statistics,
@@ -31,9 +31,8 @@ namespace {
 // LNF: the launch has a layer norm folded away (lnf_stats); the statistics' registers would cost the others a workgroup per CU.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int AMODE = 0, bool KTAIL = false, bool LNF = false>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ? 4 : 2) void gemm_pipe_kernel(GemmArgs p) {
-    constexpr bool B_KN = BMODE != 0, CONV = BMODE == 2, LNA = AMODE == 2;
-    static_assert(AMODE == 0 || BMODE != 2, "one gathered operand at a time");
-    static_assert(!KTAIL || (AMODE == 0 && BMODE != 2), "gathered operands come in whole tiles");
+    constexpr bool B_KN = BMODE != 0, LNA = AMODE == 2;
+    static_assert(!KTAIL || AMODE == 0, "gathered operands come in whole tiles");
     constexpr int BK = 64, LD = BK + 8, NT = WAVES_M * WAVES_N * 64;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, TM = WTM / 32, TN = WTN / 32;
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;     // 16-byte chunks per thread per tile
@@ -66,18 +65,6 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         const int c = tid + i * NT;
         if (!B_KN) bp[i] = B + (long)min(n0 + (c >> 3), p.N - 1) * p.ldB + (c & 7) * 8;
         else       bp[i] = B + (long)(c / CPRB) * p.ldB + min(n0 + (c % CPRB) * 8, p.NB - 8);
-    }
-    // Implicit GEMM: every chunk of this thread lies in the same eight columns (NT is a multiple of
-    // CPRB), i.e. at one pixel offset, in channels NT / CPRB apart; which tap and which 64 channels a tile
-    // covers is the same for the whole workgroup.
-    const half_t *cpix = nullptr;
-    int ctile0 = 0;
-    if constexpr (CONV) {
-        static_assert(NT % CPRB == 0 && PB * (NT / CPRB) == BK, "a thread's chunks share their columns, NT / CPRB rows apart");
-        const int ncol = min(n0 + (tid % CPRB) * 8, p.NB - 8);
-        const int oh = ncol / p.cv.OW, ow = ncol % p.cv.OW;
-        cpix = p.cv.xp + (p.cv.split ? 0 : bz * p.cv.img) + (long)oh * p.cv.sy * p.cv.Wp + ow + (long)(tid / CPRB) * p.cv.HpWp;
-        ctile0 = p.cv.split ? (int)bz * (p.K / BK) : 0;
     }
     // Channels-last gather: a thread's rows are fixed output pixels; (iy0, ix0) is where tap (0, 0) of each lands.
     int aiy0[PA], aix0[PA];
@@ -115,23 +102,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         }
 #pragma unroll
         for (int i = 0; i < PB; i++) {
-            if constexpr (CONV) {
-                const int t = ctile0 + kt, tap = t / p.cv.cpt, ci0 = (t - tap * p.cv.cpt) * BK;
-                const int kh = tap / p.cv.KW, kw = tap - kh * p.cv.KW;
-                const int toff = ci0 * p.cv.HpWp + kh * p.cv.dyWp + kw * p.cv.dx;       // same for every lane
-                // The eight halves start kw*dx elements into an aligned row, i.e. at a 2-byte boundary, and
-                // vector loads want 4-byte alignment: odd starts are read from the second copy of the padded
-                // input, which is the first shifted by one element (the choice is the same for every lane).
-                const uint32_t *src = reinterpret_cast<const uint32_t *>(cpix + toff + ((toff & 1) ? p.cv.odd : 0L) + (long)i * (NT / CPRB) * p.cv.HpWp);
-                uint32_t w4[4];
-                __builtin_memcpy(w4, src, 16);
-#pragma unroll
-                for (int q = 0; q < 4; q++) gb[set][i][q] = w4[q];
-            } else {
-                const int c = tid + i * NT;
-                const long kc = KTAIL ? min(ko, (long)(B_KN ? p.K - 1 - c / CPRB : p.K - 8 - (c & 7) * 8)) : ko;
-                gb[set][i] = ldg16(bp[i] + (B_KN ? kc * p.ldB : kc));
-            }
+            const int c = tid + i * NT;
+            const long kc = KTAIL ? min(ko, (long)(B_KN ? p.K - 1 - c / CPRB : p.K - 8 - (c & 7) * 8)) : ko;
+            gb[set][i] = ldg16(bp[i] + (B_KN ? kc * p.ldB : kc));
         }
     };
     // last: the tile that K ends in (KTAIL)
@@ -331,13 +304,11 @@ int launch_pipe(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
     a.vec_store = rows_vec16(a);
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
     constexpr int lds = gemm_lds_bytes<BM, BN, 64>();
-    if ((a.ag.x || a.cv.xp) && a.K % 64) return MI_DECLINE_EXTENT;
+    if (a.ag.x && a.K % 64) return MI_DECLINE_EXTENT;
     if (a.ag.x) {
-        if (a.cv.xp) return MI_DECLINE_UNSUPPORTED;
         if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1, 1>), grid, dim3(WM * WN * 64), lds, st, a);
         else      hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0, 1>), grid, dim3(WM * WN * 64), lds, st, a);
     }
-    else if (a.cv.xp)  hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 2>), grid, dim3(WM * WN * 64), lds, st, a);
     else if (a.K % 64) {
         if (b_kn) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, true>), grid, dim3(WM * WN * 64), lds, st, a);
         else      hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, true>), grid, dim3(WM * WN * 64), lds, st, a);
@@ -373,7 +344,7 @@ constexpr int lna_lds_bytes(int K) {
 }
 template <int BN, int WM, int WN>
 int launch_pipe_ln(GemmArgs a, bool b_kn, hipStream_t st) {
-    if (a.K < 128 || a.K % 64 || a.K > MI_LNA_KMAX || a.cv.xp || a.ag.x) return MI_DECLINE_EXTENT;
+    if (a.K < 128 || a.K % 64 || a.K > MI_LNA_KMAX || a.ag.x) return MI_DECLINE_EXTENT;
     set_tiles(a, 64, BN);
     a.vec_store = rows_vec16(a);
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1);

@@ -20,11 +20,15 @@ namespace {
 // cannot pad, so 16-byte chunks are permuted inside their row: K-contiguous row r holds chunk c at c ^ (r % 8 ^ r / 8 % 2),
 // [K][N] row k holds chunk c at c ^ (k % 4 * BN / 32) -- the four rows of a transposing read in four bank groups.
 // Chunks past K are read from a page of zeros, so K needs only to be a multiple of 8.
-template <int WM, int WN, int WK, int S, bool B_KN>
+//
+// CONV: B is the patch matrix of a convolution (ConvGather).  Its rows' offsets are as fixed as an ordinary operand's; what moves
+// from tile to tile is the tap, for all lanes alike where C is a multiple of 64, by the lane's pair of chunks otherwise.
+template <int WM, int WN, int WK, int S, bool B_KN, bool CONV = false>
 __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
     constexpr int BM = 64 * WM, BN = 64 * WN, BK = 64, NW = WM * WN * WK, NT = NW * 64, KS = 4 / WK;
     constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
     constexpr int STAGE_BYTES = SLOTS * 1024, A_BYTES = SLOTS_A * 1024;
+    static_assert(!(CONV && B_KN), "a patch row is K-contiguous");
     static_assert(S >= 3, "a stage being read, one landed, one on its way");
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -47,8 +51,9 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
         // with its products behind them (800 clocks a 64 x 64 tile), and a loader is quick only if a request costs it next
         // to nothing: a wave issues an instruction every four to eight clocks, so the lane's byte offset from the tile's
         // origin is fixed, the origin and the LDS address move in scalar registers, and the steady state has no branch.
+        // ROLE: 0 A, 1 B, 2 B a patch matrix whose tiles lie in one tap each, 3 any other patch matrix
         auto load_all = [&](auto ROLE) {
-            constexpr bool IS_A = decltype(ROLE)::value;
+            constexpr bool IS_A = decltype(ROLE)::value == 0, PATCH = decltype(ROLE)::value >= 2, ONE_TAP = decltype(ROLE)::value == 2;
             constexpr int LPW = IS_A ? SLOTS_A : SLOTS - SLOTS_A;      // 1 KB requests of a tile
             static_assert((S - 2) * LPW <= 63, "vmcnt is a 6-bit counter");
             uint32_t off[LPW];
@@ -62,6 +67,19 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
                 const int r0 = IS_A ? m0 : n0, rows = IS_A ? p.M : p.N, c = pos ^ sub;
                 const uint32_t even = (uint32_t)(sub * ld2) + c * 16, odd = even + ((c ^ 1) - c) * 16, step8 = (uint32_t)(8 * ld2);
                 const bool inside = r0 + (IS_A ? BM : BN) <= rows;                    // uniform
+                if constexpr (PATCH) {
+                    // rows are pixels, eight apart from request to request: one division, then steps
+                    const int last = rows - 1, last_y = last / p.cv.OW, last_off = last_y * p.cv.pix_y + (last - last_y * p.cv.OW) * p.cv.pix_x;
+                    int n = r0 + sub, oh = n / p.cv.OW, ow = n - oh * p.cv.OW;
+#pragma unroll
+                    for (int i = 0; i < LPW; i++) {
+                        const int ci = c ^ (i & 1);
+                        off[i] = (uint32_t)(n < rows ? oh * p.cv.pix_y + ow * p.cv.pix_x : last_off) * 2u + (ONE_TAP ? ci : ci & 1) * 16;
+                        kpos[i] = ci * 8;
+                        n += 8; ow += 8;
+                        while (ow >= p.cv.OW) { ow -= p.cv.OW; oh++; }
+                    }
+                } else
 #pragma unroll
                 for (int i = 0; i < LPW; i++) {
                     off[i] = ((i & 1) ? odd : even) + i * step8;
@@ -81,25 +99,47 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
                 }
             }
             const char *org = IS_A ? reinterpret_cast<const char *>(p.A + bz * p.sA + (long)m0 * p.ldA)
-                                   : reinterpret_cast<const char *>(p.B + bz * p.sB + (B_KN ? (long)n0 : (long)n0 * p.ldB));
+                              : PATCH ? reinterpret_cast<const char *>(p.cv.xp + bz * p.cv.img)
+                                      : reinterpret_cast<const char *>(p.B + bz * p.sB + (B_KN ? (long)n0 : (long)n0 * p.ldB));
+            // PATCH: where the next tile's first channel lies (ONE_TAP: the same for every lane, kept in `org`), or this lane's
+            // pair of chunks of it (C % 16 == 0: a pair never straddles two taps)
+            const int tap_step = (p.cv.tap_x - p.cv.C) * 2, row_step = (p.cv.tap_y - p.cv.KW * p.cv.tap_x) * 2;
+            int ch = 0, kw = 0, at = 0;
+            const int wraps = PATCH && !ONE_TAP ? (BK + p.cv.C - 1) / p.cv.C : 1;
+            auto advance = [&](int by) {
+                ch += by;
+                at += by * 2;
+                for (int w = 0; w < wraps; w++) {         // past the tap's channels: on to the next tap
+                    const bool over = ch >= p.cv.C;
+                    kw += over ? 1 : 0;
+                    const bool row = kw == p.cv.KW;
+                    at += (over ? tap_step : 0) + (row ? row_step : 0);
+                    ch -= over ? p.cv.C : 0;
+                    kw = row ? 0 : kw;
+                }
+            };
+            if (PATCH && !ONE_TAP) advance(((pos ^ sub) & 6) * 8);
             const long step = IS_A || !B_KN ? BK * 2 : (long)BK * p.ldB * 2;
             const uint32_t lds1 = lds0 + (IS_A ? 0 : A_BYTES);
             int next = 0;                                 // the tile requested next, and its stage
             uint32_t stage = 0;
             auto request = [&]() {
+                const uint32_t add = PATCH && !ONE_TAP ? (uint32_t)at : 0u;
+                const char *from_org = ONE_TAP ? org + at : org;
                 if ((next + 1) * BK <= p.K) {             // uniform
                     asm volatile("s_mov_b32 m0, %0" ::"s"(lds1 + stage) : "memory");
 #pragma unroll
                     for (int i = 0; i < LPW; i++)
-                        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_add_u32 m0, m0, 0x400" ::"v"(off[i]), "s"(org) : "memory", "scc");
+                        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_add_u32 m0, m0, 0x400" ::"v"(off[i] + add), "s"(from_org) : "memory", "scc");
                 } else {                                  // the tile that K ends in: chunks past it come from the zeros
 #pragma unroll
                     for (int i = 0; i < LPW; i++) {
-                        const char *from = next * BK + kpos[i] < p.K ? org + off[i] : reinterpret_cast<const char *>(ring_zero_words);
+                        const char *from = next * BK + kpos[i] < p.K ? from_org + (off[i] + add) : reinterpret_cast<const char *>(ring_zero_words);
                         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds1 + stage + i * 1024) : "memory");
                     }
                 }
-                org += step;
+                if constexpr (PATCH) advance(BK);
+                else org += step;
                 next++;
                 stage = stage == (S - 1) * STAGE_BYTES ? 0u : stage + STAGE_BYTES;
             };
@@ -131,8 +171,10 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
                 barrier();
             }
         };
-        if (wave == NW) load_all(std::true_type{});
-        else load_all(std::false_type{});
+        if (wave == NW) load_all(std::integral_constant<int, 0>{});
+        else if constexpr (!CONV) load_all(std::integral_constant<int, 1>{});
+        else if (p.cv.C % 64 == 0) load_all(std::integral_constant<int, 2>{});
+        else load_all(std::integral_constant<int, 3>{});
         return;
     }
 
@@ -306,8 +348,21 @@ int raise_ring() {
 
 }  // namespace
 
-int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) { return launch_ring<1, 1, 4, 8>(a, b_kn, nbatch, st); }
+int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
+    if (!a.cv.xp) return launch_ring<1, 1, 4, 8>(a, b_kn, nbatch, st);
+    GemmArgs c = a;
+    set_tiles(c, 64, 64);
+    c.vec_store = rows_vec16(c);
+    if (b_kn || (int64_t)64 * c.ldA * 2 >= (1ll << 31) || c.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
+    // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
+    const dim3 grid((unsigned)(c.tiles_m * c.tiles_n), (unsigned)nbatch);
+    constexpr int lds8 = ring_lds_bytes<1, 1, 8>(), lds4 = ring_lds_bytes<1, 1, 4>();
+    if ((int64_t)grid.x * nbatch <= mi_num_cus()) hipLaunchKernelGGL((gemm_ring_kernel<1, 1, 4, 8, false, true>), grid, dim3(4 * 64 + 128), lds8, st, c);
+    else hipLaunchKernelGGL((gemm_ring_kernel<1, 1, 4, 4, false, true>), grid, dim3(4 * 64 + 128), lds4, st, c);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
 
 int mi_ring_init() {
-    return raise_ring<1, 1, 4, 8>();
+    return raise_ring<1, 1, 4, 8>() | raise_lds(gemm_ring_kernel<1, 1, 4, 8, false, true>, ring_lds_bytes<1, 1, 8>()) |
+           raise_lds(gemm_ring_kernel<1, 1, 4, 4, false, true>, ring_lds_bytes<1, 1, 4>());
 }

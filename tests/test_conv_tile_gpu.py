@@ -21,6 +21,14 @@ pytestmark = pytest.mark.gpu
     (1, 128, 64, 64, 256, 3, 3, 1, 1, 1, "none"),
     (1, 3, 260, 261, 144, 7, 7, 4, 3, 1, "none"),
     (1, 384, 5, 5, 384, 3, 3, 1, 0, 1, "none"),
+    # the patch-gathering form: chunk pairs of several taps in a 64-deep tile, maps narrower than a piece, images past the CUs
+    (1, 16, 70, 70, 64, 7, 7, 1, 3, 1, "none"),
+    (1, 48, 65, 66, 72, 5, 5, (2, 1), (2, 0), (1, 2), "relu"),
+    (1, 80, 37, 41, 130, 7, 7, 4, 3, 1, "none"),
+    (2, 144, 30, 5, 256, 5, 3, 1, (1, 2), 1, "none"),      # seven columns with their borders
+    (1, 192, 64, 3, 256, 3, 3, 1, (0, 1), 1, "relu"),      # one output column
+    (2, 96, 120, 131, 96, 7, 7, 1, 3, 1, "none"),          # two workgroups a CU
+    (3, 256, 33, 65, 64, 3, 3, 1, 1, (2, 1), "none"),
 ])
 def test_conv_tiles(ctx, N, Cin, H, W, Cout, KH, KW, s, p, d, act):
     import torch
