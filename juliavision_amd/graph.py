@@ -1682,7 +1682,8 @@ class Executor:
         """Run the graph.  The first run on inputs of given strides and alignment goes op by op through the handlers (it
         prepares folded constants and sizes the workspace), the second notes the library calls it makes, and later ones
         issue those calls again from native code with the new inputs' addresses: 62 launches of a 12-layer ViT took
-        1.66 ms of host time through the handlers and 0.7 ms on the GPU."""
+        1.66 ms of host time through the handlers and 0.7 ms on the GPU.  A run whose inputs share memory with each other or
+        with this executor (a result handed back) is not the one that is noted."""
         if len(inputs) != len(self.g.inputs):
             raise ValueError(f"{self.g.name} takes {len(self.g.inputs)} inputs")
         for bid, x in zip(self.g.inputs, inputs):
@@ -1698,7 +1699,7 @@ class Executor:
                 return self._results()
             if status is not False:
                 raise K.DeclineError(f"{self.g.name}: a recorded call was refused", status)
-        record = self._seen == like and isinstance(ctx, K.Ctx)
+        record = self._seen == like and isinstance(ctx, K.Ctx) and K.apart([K.span(x) for x in inputs], self._owned())
         if record:
             self.ctx = K.CallRecorder(ctx)
         try:
@@ -1710,6 +1711,20 @@ class Executor:
             self.ctx = ctx
         self._seen = (ctx, ctx.ws.buf.data_ptr(), ctx.ws.buf.numel(), like[3])
         return self._results()
+
+    def _owned(self):
+        """The memory that this executor's calls name and that is no input's: weights, buffers, folded constants, workspace."""
+        inputs, spans, todo = set(self.g.inputs), [K.span(self.ctx.ws.buf)], list(self.scaled.values())
+        todo += [t for bid, t in self.t.items() if bid not in inputs]
+        while todo:
+            v = todo.pop()
+            if isinstance(v, torch.Tensor):
+                spans.append(K.span(v))
+            elif isinstance(v, (tuple, list)):
+                todo += v
+            elif isinstance(v, K.LnFoldedLinear):
+                todo += [v.wp, v.colsum, v.biasp]
+        return spans
 
     def _results(self):
         outs = [self.get(bid) for bid in self.g.outputs]

@@ -187,7 +187,8 @@ class CallRecorder:
     """Stands in for a context while a fixed sequence of calls runs once more: every call that enqueues work is carried out
     and noted.  ``calls(inputs)`` then gives the sequence as one native object that issues it again on other inputs of the
     same shapes, strides and alignment -- each address inside an input's memory is taken relative to the new input -- or
-    None where a call is not one that can be repeated (``_host.calls_new``)."""
+    None where a call is not one that can be repeated (``_host.calls_new``).  The inputs have to be ``apart`` from each other
+    and from everything else the calls name."""
 
     _QUERIES = ("_plan", "_plan_caps", "_workspace", "mi_convsize", "mi_convtransposesize", "mi_version", "mi_device_caps")
 
@@ -210,14 +211,22 @@ class CallRecorder:
         return call
 
     def calls(self, inputs):
-        spans = []
-        for x in inputs:
-            n = x.element_size() * (1 + sum((s - 1) * st for s, st in zip(x.shape, x.stride()))) if x.numel() else 0
-            spans.append((x.data_ptr(), n))
-        order = sorted(s for s in spans if s[1])
-        if any(a[0] + a[1] > b[0] for a, b in zip(order, order[1:])):
-            return None                                   # inputs that share memory: an address would not say whose it is
-        return _fast.calls_new(self.noted, spans)
+        return _fast.calls_new(self.noted, [span(x) for x in inputs])
+
+
+def span(t: torch.Tensor):
+    """The memory a strided tensor covers: first address, bytes."""
+    return t.data_ptr(), t.element_size() * (1 + sum((s - 1) * st for s, st in zip(t.shape, t.stride()))) if t.numel() else 0
+
+
+def apart(inputs, owned) -> bool:
+    """Whether every input's memory is its own: no two spans of ``inputs`` overlap, and none overlaps one of ``owned``.  A recorded
+    address that lies in an input moves with it, so an address must say whose it is: a result buffer handed back as an
+    input would have the calls write their result into whatever tensor comes next."""
+    ins = sorted(s for s in inputs if s[1])
+    if any(a + n > b for (a, n), (b, _) in zip(ins, ins[1:])):
+        return False
+    return not any(a < b + m and b < a + n for a, n in ins for b, m in owned if m)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

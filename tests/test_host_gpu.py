@@ -13,12 +13,22 @@ class _Net(nn.Module):
         self.heads, self.norm = heads, nn.LayerNorm(d)
         self.q, self.k, self.v, self.o, self.fc = (nn.Linear(d, d) for _ in range(5))
 
-    def forward(self, x):
+    def attended(self, x):
         B, T, D = x.shape
         split = lambda t: t.view(B, T, self.heads, D // self.heads).transpose(1, 2)
         y = self.norm(x)
         a = F.scaled_dot_product_attention(split(self.q(y)), split(self.k(y)), split(self.v(y)))
-        return x + self.o(a.transpose(1, 2).reshape(B, T, D)), F.gelu(self.fc(x))
+        return x + self.o(a.transpose(1, 2).reshape(B, T, D))
+
+    def forward(self, x):
+        return self.attended(x), F.gelu(self.fc(x))
+
+
+class _State(_Net):
+    """One result, of the input's shape; its last op reads the input elementwise, so it may be handed back."""
+
+    def forward(self, x):
+        return self.attended(x)
 
 
 @pytest.mark.parametrize("T", [5, 130])
@@ -38,6 +48,31 @@ def test_recorded_calls_follow_their_inputs(T):
         fresh = G.Executor(g, m.state_dict(), jv.Ctx("cuda"))(x)
         for a, b in zip(got, fresh):
             assert torch.equal(a, b.float()), f"run {i}"
+    assert run._calls is not None
+
+
+@pytest.mark.parametrize("T", [5, 130])
+def test_a_result_handed_back_is_not_taken_for_an_input(T):
+    """``x = run(x)``: the run that is noted must not take the result buffer for an input's memory, or the next call on a tensor
+    of the user's writes its result there."""
+    import juliavision_amd as jv
+    from juliavision_amd import graph as G
+    torch.manual_seed(T)
+    m = _State(128, 2).eval().half()
+    g = G.optimize(G.Graph.load(G.convert(torch.export.export(m, (torch.randn(1, T, 128).half(),)), "state")))
+    run, ref = (G.Executor(g, m.state_dict(), jv.Ctx("cuda")) for _ in range(2))
+    x = torch.randn(1, T, 128, device="cuda").half()
+    want = x
+    for i in range(4):
+        want = ref(want.clone()).clone()
+        x = run(x)
+        assert torch.equal(x, want), f"pass {i}"
+    for i in range(4):
+        z = torch.randn(1, T, 128, device="cuda").half()
+        kept = z.clone()
+        got = run(z)
+        assert torch.equal(z, kept), f"the input of call {i} was written to"
+        assert torch.equal(got, G.Executor(g, m.state_dict(), jv.Ctx("cuda"))(kept)), f"call {i}"
     assert run._calls is not None
 
 
