@@ -1254,7 +1254,7 @@ class Executor:
         self.device = torch.device(device)
         self.t: Dict[str, torch.Tensor] = {}
         self.scaled: Dict[str, Any] = {}                  # op id -> (weight, bias) with a folded per-feature scale
-        self._calls, self._calls_for, self._seen = None, None, None      # the recorded calls of a run (``__call__``)
+        self._calls, self._calls_for, self._seen, self._refused = None, None, None, None      # the recorded calls of a run (``__call__``)
         for b in graph.buffers.values():
             if b["kind"] == "weight":
                 w = weights[b["key"]]
@@ -1699,14 +1699,18 @@ class Executor:
                 return self._results()
             if status is not False:
                 raise K.DeclineError(f"{self.g.name}: a recorded call was refused", status)
-        record = self._seen == like and isinstance(ctx, K.Ctx) and K.apart([K.span(x) for x in inputs], self._owned())
+        record = self._seen == like and like not in (self._refused, self._calls_for) and isinstance(ctx, K.Ctx) and K.apart([K.span(x) for x in inputs], self._owned())
         if record:
             self.ctx = K.CallRecorder(ctx)
         try:
             for o in self.g.ops:
                 self.HANDLERS[o["aten"]](self, o)
             if record and (ctx.ws.buf.data_ptr(), ctx.ws.buf.numel()) == like[1:3]:
-                self._calls, self._calls_for = self.ctx.calls(inputs), like
+                calls = self.ctx.calls(inputs)
+                if calls is None:                         # a call that cannot be repeated: noting it again would only cost time
+                    self._refused = like
+                else:
+                    self._calls, self._calls_for = calls, like
         finally:
             self.ctx = ctx
         self._seen = (ctx, ctx.ws.buf.data_ptr(), ctx.ws.buf.numel(), like[3])

@@ -76,6 +76,46 @@ def test_a_result_handed_back_is_not_taken_for_an_input(T):
     assert run._calls is not None
 
 
+class _Two(nn.Module):
+    def __init__(self, d):
+        super().__init__()
+        self.a, self.b = nn.Linear(d, d), nn.Linear(d, d)
+
+    def forward(self, x, y):
+        return self.a(x) + self.b(y)
+
+
+@pytest.mark.parametrize("why", ["shared", "refused", "described"])
+def test_calls_that_are_not_noted_are_not_noted_again(why, monkeypatch):
+    """Inputs that share memory, a call that cannot be repeated, a context that the native side does not take: the runs that
+    follow go through the handlers and their native calls, not through the recorder's slow ones."""
+    import juliavision_amd as jv
+    from juliavision_amd import graph as G, kernels as K
+    torch.manual_seed(0)
+    m, T = _Two(64).eval().half(), 20
+    g = G.optimize(G.Graph.load(G.convert(torch.export.export(m, (torch.randn(T, 64).half(),) * 2), "two")))
+    run, made = G.Executor(g, m.state_dict(), jv.Ctx("cuda", dev=jv.MI355X if why == "described" else None)), []
+
+    class Recorder(K.CallRecorder):
+        def __init__(self, ctx):
+            made.append(self)
+            super().__init__(ctx)
+
+        def calls(self, inputs):
+            return None if why == "refused" else super().calls(inputs)
+    monkeypatch.setattr(K, "CallRecorder", Recorder)
+    x, y = (torch.randn(T, 64, device="cuda").half() for _ in range(2))
+    for i in range(5):
+        args = (x, x) if why == "shared" else (x, y)
+        got = run(*args)
+        assert torch.equal(got, G.Executor(g, m.state_dict(), jv.Ctx("cuda"))(*args)), f"run {i}"
+    assert len(made) == (why != "shared") and (run._calls is not None) == (why == "described")
+    if why == "shared":                                                               # ... and apart again they are noted
+        for _ in range(2):
+            run(x, y)
+        assert run._calls is not None and len(made) == 1
+
+
 def test_what_the_native_side_leaves_is_still_refused_by_name():
     import juliavision_amd as jv
     ctx = jv.Ctx("cuda")
