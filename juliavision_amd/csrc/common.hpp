@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "extents.hpp"
 #include "../../include/mi355dnn.h"
 
 typedef _Float16 half_t;
@@ -127,8 +128,6 @@ MI_DEVICE half_t ln_norm1(float x, float mu, float r, bool has_g, float g, bool 
 }
 
 static inline bool aligned_to(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
-static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-static inline size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 // NaN by its bits: the build tells the compiler that no NaNs occur, which folds comparisons with one away.
 static inline bool is_nan_arg(float x) { uint32_t u; __builtin_memcpy(&u, &x, 4); return (u & 0x7fffffffu) > 0x7f800000u; }
 

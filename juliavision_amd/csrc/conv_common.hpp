@@ -1,12 +1,11 @@
 // The arguments the convolution kernels share.
 #pragma once
 #include "common.hpp"
+#include "conv_tile_plan.hpp"
 
-struct ConvArgs {
+struct ConvArgs : ConvShape {
     const half_t *x, *w, *bias;
     void *out;
-    int Wi, Hi, Cin, N, KW, KH, Cout, OW, OH;
-    int sx, sy, px, py, dx, dy, groups, relu;
 };
 
 // conv_tile.hip: the one-launch implicit GEMM over channel-first maps, one group.  MI_DECLINE_EXTENT (nothing enqueued)

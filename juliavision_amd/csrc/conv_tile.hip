@@ -11,24 +11,15 @@
 // Bound by the LDS: per 16-deep step a wave reads 8 x 64 two-byte elements, 16 bytes of table and 1 KB per weight
 // fragment.  The im2col matrix (K / CC times the input), its GEMM's two reads of it and the launches between are gone.
 #include "conv_common.hpp"
-#include <algorithm>
 #include <type_traits>
+
+using namespace conv_tile;
 
 namespace {
 
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
-struct TileConv {
-    ConvArgs a;
-    int TH, TW, tiles_x, tiles_y;     // output rectangle, rectangles per image
-    int CC, nchunk, kc;               // channels a chunk, chunks, CC KH KW
-    int ksteps;                       // 16-deep steps of a full chunk
-    int PR, PC8, PCL;                 // patch rows, 16-byte pieces a row, halves a row
-    int WLD, wpieces;                 // weight row pitch in LDS (halves), 16-byte pieces a row
-    int patch_pieces, weight_pieces;  // per chunk
-    int tab_off, patch_off, weight_off, stage_bytes;      // LDS layout in bytes: table, then `nbuf` stages of patch + weights
-    int nbuf;
-};
+struct TileConv : TilePlan { ConvArgs a; };
 
 // PW waves side by side over pixels, KG groups of them over the steps of a chunk, TCO x 32 output channels each.
 // WP, PP: weight and patch pieces a thread carries in registers for the next chunk.
@@ -67,7 +58,7 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         const u32x4 r = {(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
         return r;
     };
-    const bool narrow = a.Wi < 8, short_w = CRS < 8;      // uniform: rows without a whole piece go by element
+    const bool narrow = a.Wi < 8, short_w = weights_by_element(t.kc, CRS);      // uniform: rows without a whole piece go by element
     const u32x4 zero4 = {0u, 0u, 0u, 0u};
     // A 16-byte piece: where it lies in memory (halves from the chunk's start) and in the stage (bytes); k or channel of the
     // chunk it starts at; how many of its halves a load moved back to stay inside the row drops.
@@ -117,8 +108,8 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
             for (int e = 0; e < 8; e++) if (e < left) h[e] = s[e];
             return __builtin_bit_cast(u32x4, h);
         }
-        __builtin_memcpy(&v, s + min(left, 8) - 8, 16);
-        return left < 8 ? shifted(v, 8 - left) : v;
+        __builtin_memcpy(&v, s - weight_back(left), 16);
+        return left < 8 ? shifted(v, weight_back(left)) : v;
     };
     auto patch_lds = [&](int buf, int dst) { return reinterpret_cast<u32x4 *>(smem + t.patch_off + buf * t.stage_bytes + dst); };
     auto weight_lds = [&](int buf, int dst) { return reinterpret_cast<u32x4 *>(smem + t.weight_off + buf * t.stage_bytes + dst); };
@@ -296,50 +287,6 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         }
 }
 
-constexpr int LDS_MAX = 160 * 1024;
-
-// The rectangle of `px` pixels with the fewest tiles, then the smallest patch; widths are powers of two so that a wave's
-// pixels are whole row pieces.
-void choose_rectangle(TileConv &t, int px) {
-    const ConvArgs &a = t.a;
-    int64_t best = INT64_MAX;
-    for (int tw = 4; tw <= px; tw *= 2) {
-        const int th = px / tw;
-        // how far a tile's first column may lie past a multiple of eight: ox0 sx - px is a fixed residue if tw sx is one
-        const int slack = tw * a.sx % 8 == 0 ? (int)(((-a.px) % 8 + 8) % 8) : 7;
-        const int64_t tiles = ceil_div(a.OW, tw) * ceil_div(a.OH, th);
-        const int64_t rows = (int64_t)(th - 1) * a.sy + (a.KH - 1) * a.dy + 1, cols = (int64_t)(tw - 1) * a.sx + (a.KW - 1) * a.dx + 1 + slack;
-        const int64_t cost = tiles * (rows * round_up(cols, 8) + px / 2);
-        if (cost < best) { best = cost; t.TW = tw; t.TH = th; t.PR = (int)rows; t.PC8 = (int)ceil_div(cols, 8); }
-    }
-    t.PCL = t.PC8 * 8;
-    t.tiles_x = (int)ceil_div(a.OW, t.TW);
-    t.tiles_y = (int)ceil_div(a.OH, t.TH);
-}
-
-// Chunk depth and LDS layout for `co` output channels and `nt` threads; false where no chunk fits.
-bool choose_chunk(TileConv &t, int co, int nt, int parts_bytes) {
-    const ConvArgs &a = t.a;
-    const int taps = a.KH * a.KW;
-    auto fits = [&](int cc, bool single) {
-        t.CC = cc; t.kc = cc * taps; t.ksteps = (int)ceil_div(t.kc, 16);
-        t.wpieces = t.ksteps * 2;                        // whole steps: zero past kc
-        t.WLD = t.ksteps * 16 + 8;                       // 16 bytes off a multiple of 32 bytes: rows start in distinct bank groups
-        t.patch_pieces = cc * t.PR * t.PC8; t.weight_pieces = co * t.wpieces;
-        t.nchunk = (int)ceil_div(a.Cin, cc); t.nbuf = t.nchunk > 1 ? 2 : 1;
-        const int64_t patch = round_up(((size_t)cc * t.PR * t.PCL + 8) * 2, 16), weights = (int64_t)co * t.WLD * 2;
-        if ((int64_t)cc * t.PR * t.PCL > 65535 || patch + weights > LDS_MAX) return false;
-        t.tab_off = 0; t.patch_off = (int)round_up((size_t)t.ksteps * 32, 16);
-        t.weight_off = t.patch_off + (int)patch; t.stage_bytes = (int)(patch + weights);
-        if (t.patch_off + (int64_t)t.nbuf * t.stage_bytes > LDS_MAX || parts_bytes > LDS_MAX) return false;
-        return single || (t.patch_pieces <= 3 * nt && t.weight_pieces <= (co > 64 ? 6 : 5) * nt);
-    };
-    if (a.Cin <= 16 && fits(a.Cin, true)) return true;
-    for (int cc : {64, 32, 16, 8, 4, 2, 1})
-        if (cc <= (int)round_up((size_t)a.Cin, 4) && fits(cc, false)) return true;
-    return false;
-}
-
 template <int PW, int KG, int TCO>
 int launch(const TileConv &t, hipStream_t st) {
     constexpr int parts = (KG - 1) * TCO * 16 * PW * 64 * 4;
@@ -349,9 +296,6 @@ int launch(const TileConv &t, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
-struct Shape { int pw, kg, tco; };
-constexpr Shape SHAPES[] = {{8, 1, 1}, {8, 1, 2}, {8, 1, 3}, {8, 1, 4}, {4, 1, 1}, {4, 1, 2}, {4, 1, 3}, {4, 1, 5}, {4, 2, 1}, {4, 2, 2}, {4, 2, 3}, {4, 2, 4}, {2, 4, 1}, {2, 4, 2}, {2, 4, 4}, {2, 2, 1}, {2, 2, 2}};
-
 template <typename F>
 int with_shape(const Shape &s, F f) {
 #define ONE(P, K, T) if (s.pw == P && s.kg == K && s.tco == T) return f(std::integral_constant<int, P>{}, std::integral_constant<int, K>{}, std::integral_constant<int, T>{});
@@ -360,34 +304,11 @@ int with_shape(const Shape &s, F f) {
     return MI_DECLINE_EXTENT;
 }
 
-// The workgroup shape with the lowest estimate (us), or false where no chunk fits.  Fitted to 24 convolutions in 17 shapes each
-// (1 x 1 to 7 x 7, strides 1, 2 and 4, 3 to 384 channels, 300 to 65 536 pixels): half of the estimates lie within 20 %.  A
-// chunk costs its trip to memory and its pieces, a step of a wave its eight gathers and its weight fragments.
-bool choose(TileConv &t, Shape &best, double &best_us) {
-    const ConvArgs &a = t.a;
-    if ((int64_t)a.Cout * a.Cin * a.KH * a.KW > INT32_MAX / 2) return false;      // 32-bit offsets
-    best_us = 1e30;
-    TileConv pick = t;
-    for (const Shape &s : SHAPES) {
-        TileConv c = t;
-        choose_rectangle(c, 32 * s.pw);
-        if (!choose_chunk(c, 32 * s.tco, s.pw * s.kg * 64, (s.kg - 1) * s.tco * 16 * s.pw * 64 * 4)) continue;
-        const int64_t wgs = (int64_t)c.tiles_x * c.tiles_y * ceil_div(a.Cout, 32 * s.tco) * a.N;
-        const double rounds = (double)ceil_div(wgs, mi_num_cus()), steps = (double)c.nchunk * c.ksteps * s.pw / 4.0;
-        const double us = 3.2 + rounds * (2.6 + 0.19 * s.tco * s.pw + c.nchunk * (1.1 + 0.36e-3 * (c.patch_pieces + c.weight_pieces)) +
-                                          steps * (0.0113 + 0.0137 * s.tco));
-        if (us < best_us) { best_us = us; best = s; pick = c; }
-    }
-    if (best_us >= 1e30) return false;
-    t = pick;
-    return true;
-}
-
 }  // namespace
 
 int mi_conv_tile(const ConvArgs &a, double limit_us, hipStream_t st) {
     // the last choices of this thread: an estimate of every shape takes the host a few microseconds
-    struct Entry { int key[12]; double us; Shape s; TileConv t; };
+    struct Entry { int key[12]; double us; Shape s; TilePlan t; };
     static thread_local Entry table[16] = {};
     const int key[12] = {1, a.Wi, a.Hi, a.Cin, a.N, a.KW * 65536 + a.KH, a.Cout, a.sx * 65536 + a.sy, a.px * 65536 + a.py, a.dx * 65536 + a.dy, a.OW, mi_num_cus()};
     unsigned h = 0;
@@ -395,12 +316,10 @@ int mi_conv_tile(const ConvArgs &a, double limit_us, hipStream_t st) {
     Entry &e = table[h >> 28];
     if (__builtin_memcmp(e.key, key, sizeof(key)) != 0) {
         __builtin_memcpy(e.key, key, sizeof(key));
-        e.t.a = a;
-        if (!choose(e.t, e.s, e.us)) e.us = 1e30;
+        if (!choose(a, mi_num_cus(), e.t, e.s, e.us)) e.us = 1e30;
     }
     if (e.us >= limit_us) return MI_DECLINE_EXTENT;
-    TileConv t = e.t;
-    t.a = a;
+    const TileConv t{e.t, a};
     return with_shape(e.s, [&](auto P, auto K, auto T) { return launch<P, K, T>(t, st); });
 }
 

@@ -21,6 +21,10 @@ pytestmark = pytest.mark.gpu
     (1, 128, 64, 64, 256, 3, 3, 1, 1, 1, "none"),
     (1, 3, 260, 261, 144, 7, 7, 4, 3, 1, "none"),
     (1, 384, 5, 5, 384, 3, 3, 1, 0, 1, "none"),
+    # strides that leave room for chunks of fewer than eight weights a channel, and a last chunk of one
+    (1, 32, 512, 512, 84, 1, 1, (2, 8), 0, 1, "none"),
+    (1, 33, 256, 300, 70, 1, 1, (8, 5), 0, 1, "relu"),
+    (1, 35, 128, 100, 70, 3, 1, (8, 8), 0, 1, "none"),
     # the patch-gathering form: chunk pairs of several taps in a 64-deep tile, maps narrower than a piece, images past the CUs
     (1, 16, 70, 70, 64, 7, 7, 1, 3, 1, "none"),
     (1, 48, 65, 66, 72, 5, 5, (2, 1), (2, 0), (1, 2), "relu"),
