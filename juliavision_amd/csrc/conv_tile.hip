@@ -308,15 +308,14 @@ int with_shape(const Shape &s, F f) {
 
 int mi_conv_tile(const ConvArgs &a, double limit_us, hipStream_t st) {
     // the last choices of this thread: an estimate of every shape takes the host a few microseconds
-    struct Entry { int key[12]; double us; Shape s; TilePlan t; };
+    struct Entry { int cus; ConvShape key; double us; Shape s; TilePlan t; };
     static thread_local Entry table[16] = {};
-    const int key[12] = {1, a.Wi, a.Hi, a.Cin, a.N, a.KW * 65536 + a.KH, a.Cout, a.sx * 65536 + a.sy, a.px * 65536 + a.py, a.dx * 65536 + a.dy, a.OW, mi_num_cus()};
-    unsigned h = 0;
-    for (int k : key) h = h * 0x9E3779B1u + (unsigned)k;
-    Entry &e = table[h >> 28];
-    if (__builtin_memcmp(e.key, key, sizeof(key)) != 0) {
-        __builtin_memcpy(e.key, key, sizeof(key));
-        if (!choose(a, mi_num_cus(), e.t, e.s, e.us)) e.us = 1e30;
+    const int cus = mi_num_cus();
+    Entry &e = table[shape_hash(a, cus) >> 28];
+    if (e.cus != cus || !same_shape(e.key, a)) {
+        e.cus = cus;
+        e.key = a;
+        if (!choose(a, cus, e.t, e.s, e.us)) e.us = 1e30;
     }
     if (e.us >= limit_us) return MI_DECLINE_EXTENT;
     const TileConv t{e.t, a};

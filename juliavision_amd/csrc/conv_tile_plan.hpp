@@ -12,6 +12,21 @@ struct ConvShape {
 
 namespace conv_tile {
 
+// Choices are kept by every extent they were made for, each whole: packed two to a word, strides and kernels beyond 65 535 answered
+// for one another, and a plan of another stride sends the kernel past its patch.
+constexpr int ConvShape::*KEY[] = {&ConvShape::Wi, &ConvShape::Hi, &ConvShape::Cin, &ConvShape::N, &ConvShape::KW, &ConvShape::KH, &ConvShape::Cout, &ConvShape::OW,
+                                   &ConvShape::OH, &ConvShape::sx, &ConvShape::sy, &ConvShape::px, &ConvShape::py, &ConvShape::dx, &ConvShape::dy};
+inline bool same_shape(const ConvShape &a, const ConvShape &b) {
+    for (auto f : KEY)
+        if (a.*f != b.*f) return false;
+    return true;
+}
+inline unsigned shape_hash(const ConvShape &a, int cus) {
+    unsigned h = (unsigned)cus;
+    for (auto f : KEY) h = h * 0x9E3779B1u + (unsigned)(a.*f);
+    return h;
+}
+
 struct TilePlan {
     int TH, TW, tiles_x, tiles_y;     // output rectangle, rectangles per image
     int CC, nchunk, kc;               // channels a chunk, chunks, CC KH KW
