@@ -234,10 +234,11 @@ int conv_path(const ConvArgs &a) {
     return MI_CONV_IM2COL_GEMM;
 }
 
-// Scratch of the patch-gathering form: the padded channels-last copy, then the weights tap-major.
+// Scratch of the patch-gathering form: the padded channels-last copy, then the weights tap-major.  Extents alone decide, so that the
+// workspace asked for is the one the call finds: x and w may lie at any address (conv_pad_kernel's reads ask for none).
 bool patch_ok(const ConvArgs &a) {
     const int64_t Hp = a.Hi + 2 * a.py, Wp = a.Wi + 2 * a.px;
-    return a.groups == 1 && a.Cin % 16 == 0 && turn_group(a) >= 8 && aligned_to(a.w, 16) && (int64_t)Hp * Wp * a.Cin <= INT32_MAX && (int64_t)a.Cout * a.Cin * a.KH * a.KW <= INT32_MAX / 8;
+    return a.groups == 1 && a.Cin % 16 == 0 && turn_group(a) >= 8 && (int64_t)Hp * Wp * a.Cin <= INT32_MAX && (int64_t)a.Cout * a.Cin * a.KH * a.KW <= INT32_MAX / 8;
 }
 size_t patch_copy_bytes(const ConvArgs &a) { return round_up((size_t)a.N * a.Cin * (a.Hi + 2 * a.py) * (a.Wi + 2 * a.px) * 2, 256); }
 size_t patch_weight_bytes(const ConvArgs &a) { return round_up((size_t)a.Cout * a.Cin * a.KH * a.KW * 2, 256); }
@@ -268,16 +269,20 @@ size_t mi_conv2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, i
                                int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy) {
     ConvArgs a;
     if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, 1, MI_EPI_NONE) != MI_OK) return 0;
-    if (conv_path(a) == MI_CONV_IMPLICIT_GEMM) {       // (twice the copy with rows of whole 16 bytes, and planes: what it was sized for first)
+    if (a.groups != 1 || onebyone(a)) return 0;
+    // what the route needs, and never less than the answers that callers' buffers are sized by: two padded copies with rows of
+    // whole 16 bytes and planes for an implicit GEMM's extents, the im2col matrix for the others
+    const size_t patch = patch_ok(a) ? patch_copy_bytes(a) + patch_weight_bytes(a) : 0;
+    size_t need;
+    if (patch && implicit_ok(a)) {
         const size_t Wp = round_up((size_t)(a.Wi + 2 * a.px), 8);
-        return 2 * round_up((size_t)N * Cin * (a.Hi + 2 * a.py) * Wp * 2, 256) + patch_weight_bytes(a) + mi_internal_gemm_workspace(Cout, Cin * KH * KW, (int64_t)a.OW * a.OH, N);
+        need = 2 * round_up((size_t)N * Cin * (a.Hi + 2 * a.py) * Wp * 2, 256) + patch_weight_bytes(a) + mi_internal_gemm_workspace(Cout, Cin * KH * KW, (int64_t)a.OW * a.OH, N);
+    } else {
+        int64_t PQP, CRSP;
+        im2col_extents(a, PQP, CRSP);
+        const size_t wp = CRSP != (int64_t)Cin * KH * KW ? round_up((size_t)Cout * CRSP * 2, 256) : 0;
+        need = round_up((size_t)N * PQP * CRSP * 2, 256) + wp + mi_internal_gemm_workspace(Cout, CRSP, (int64_t)a.OW * a.OH, N);
     }
-    if (conv_path(a) != MI_CONV_IM2COL_GEMM) return 0;
-    int64_t PQP, CRSP;
-    im2col_extents(a, PQP, CRSP);
-    size_t col = round_up((size_t)N * PQP * CRSP * 2, 256);
-    size_t wp = CRSP != (int64_t)Cin * KH * KW ? round_up((size_t)Cout * CRSP * 2, 256) : 0;
-    const size_t need = col + wp + mi_internal_gemm_workspace(Cout, CRSP, (int64_t)a.OW * a.OH, N), patch = patch_ok(a) ? patch_copy_bytes(a) + patch_weight_bytes(a) : 0;
     return need > patch ? need : patch;
 }
 

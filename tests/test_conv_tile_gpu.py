@@ -48,3 +48,29 @@ def test_conv_tiles(ctx, N, Cin, H, W, Cout, KH, KW, s, p, d, act):
     jv.convolution_(ctx, out, to_dev(x), to_dev(w), to_dev(b), s, p, d, 1, act=act)
     torch.cuda.synchronize()
     assert_parity(to_host(out), want, what=f"conv {Cin},{H},{W}->{Cout} k{KH}x{KW}")
+
+
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("Cin,H,W,Cout,k,s,p", [
+    (64, 32, 32, 64, 3, 1, 1), (256, 32, 32, 256, 3, 1, 1), (64, 24, 40, 48, 5, 1, 2), (128, 16, 24, 256, 1, 1, 0),      # extents of an implicit GEMM; 1 x 1
+    (48, 30, 33, 64, 3, 2, 1), (96, 60, 57, 96, 5, 1, 2), (3, 70, 70, 40, 7, 4, 3), (70, 20, 20, 33, 3, 1, 1),           # patch copy, one launch, im2col
+])
+def test_operands_off_sixteen_bytes(ctx, Cin, H, W, Cout, k, s, p, off):
+    """Weights sliced out of a flat buffer: every operand `off` elements behind an aligned address, guards around the result."""
+    import torch
+    import juliavision_amd as jv
+    x, w = oracle.randn_f16((1, Cin, H, W), 1), oracle.randn_f16((Cout, Cin, k, k), 2, 0, 1.0 / np.sqrt(Cin * k * k))
+    b = oracle.randn_f16((Cout,), 3, 0, 0.5)
+    want = oracle.conv2d_f16(x, w, b, (s, s), (p, p), (1, 1), 1, False)
+
+    def shifted(a):
+        flat = torch.empty(a.size + off, dtype=torch.float16, device="cuda")
+        flat[off:] = torch.from_numpy(a).cuda().reshape(-1)
+        return flat[off:].view(a.shape)
+    flat = torch.full((want.size + 2 * off,), float("nan"), dtype=torch.float16, device="cuda")
+    out = flat[off:off + want.size].view(want.shape)
+    ctx.ws.reset()
+    jv.convolution_(ctx, out, shifted(x), shifted(w), shifted(b), (s, s), (p, p), (1, 1), 1)
+    torch.cuda.synchronize()
+    assert_parity(to_host(out), want, what=f"conv {Cin},{H},{W}->{Cout} k{k} off {off}")
+    assert bool(torch.isnan(flat[:off]).all()) and bool(torch.isnan(flat[off + want.size:]).all())
