@@ -135,15 +135,16 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
     const half_t *vb = p.v + h * p.vs[2] + b * p.vs[3];
     int Lk = p.Lk;
     if (p.kv_len) Lk = max(0, min(Lk, p.kv_len[b]));
-    int LkLoad = p.Lk;                 // keys that exist in memory (rows past it are re-reads of the last one)
     if (!PP && p.nsplit > 1) {
         const int per = (((p.Lk + BC - 1) / BC + p.nsplit - 1) / p.nsplit) * BC;      // keys per split, whole blocks
         const int kbeg = split * per;
         kb += (long)kbeg * p.ks[1];
         vb += (long)kbeg * p.vs[1];
         Lk = max(0, min(Lk - kbeg, per));
-        LkLoad = max(1, min(p.Lk - kbeg, per));
     }
+    // Rows past the last key that counts are re-reads of it: their weights are zero, which would not hide an infinity or a NaN
+    // in a cache slot that nothing has written yet.
+    const int LkLoad = max(1, Lk);
     const float c = p.scale * LOG2E;
     // barrier between the half-block intervals of the ping-pong: LDS traffic of this wave done, nothing else waited for
     auto pp_barrier = [&]() {
@@ -897,6 +898,7 @@ __global__ __launch_bounds__(512) void sdpa_decode_kernel(SdpaArgs p) {
                         *reinterpret_cast<u32x4 *>(vb + (long)key * p.vs[1] + e0) = vn;
                     }
                 }
+                if (key >= Lk) vr = z;                           // a weight of zero would not hide what an unwritten slot may hold
                 const half8v kt = as_half8(kr), vt = as_half8(vr);
                 float d = 0.0f;
 #pragma unroll

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
     const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];
     int Lk = p.Lk;
     if (p.kv_len) Lk = max(0, min(Lk, p.kv_len[b]));
-    const int nt = (Lk + 31) / 32, last = p.Lk - 1;           // rows past the end re-read the last key that exists
+    const int nt = (Lk + 31) / 32, last = Lk - 1;             // rows past the end re-read the last key that counts: whatever lies behind it, a weight of zero would not hide an infinity
     const float c = p.scale * LOG2E;
 
     u32x4 qraw[KS];

@@ -39,3 +39,25 @@ def test_tiles(ctx, B, H, Lq, Lk, E, mask):
     p = np.exp(s - s.max(-1, keepdims=True))
     want = np.einsum("bhqk,bhke->bhqe", p / p.sum(-1, keepdims=True), np.float32(v[:, :, 2]).transpose(0, 2, 1, 3))
     assert_parity(to_host(out.contiguous()), want, what=f"{B}x{H} {Lq} over {Lk}, head size {E}, mask {mask}")
+
+
+@pytest.mark.parametrize("garbage", [float("inf"), float("nan")])
+@pytest.mark.parametrize("B,H,Lq,Lk,E", [(2, 3, 31, 97, 64), (3, 2, 5, 200, 72), (2, 8, 2, 64, 16), (2, 4, 40, 700, 128),          # few queries
+                                         (3, 2, 70, 130, 32), (3, 4, 130, 300, 64), (2, 20, 400, 1500, 64), (2, 2, 100, 300, 96),     # every fused form
+                                         (2, 16, 800, 1500, 64), (2, 1, 128, 8192, 64), (3, 2, 1, 300, 64), (3, 2, 1, 300, 80)])
+def test_cache_slots_past_the_length_do_not_matter(ctx, B, H, Lq, Lk, E, garbage):
+    """Keys at and past kv_len get weight exactly zero, whatever the unwritten slots of a caller's cache hold."""
+    import torch
+    import juliavision_amd as jv
+    q, k, v = (to_dev(oracle.randn_f16((B, H, L, E), s)) for s, L in ((1, Lq), (2, Lk), (3, Lk)))
+    lens = [Lk // 2 + 1, 1, Lk][:B]
+    kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    outs = []
+    for fill in (0.0, garbage):
+        for b, n in enumerate(lens):
+            k[b, :, n:], v[b, :, n:] = fill, fill
+        out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float16, device="cuda")
+        ctx.ws.reset()
+        jv.sdpa(ctx, q, k, v, kv_len=kv_len, out=out)
+        outs.append(out)
+    assert bool(torch.isfinite(outs[0]).all()) and torch.equal(*outs)
