@@ -237,8 +237,14 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
         // log2(e) = 1.4423828125 (the fp16 value below it) + 0.00031220...: both factors positive
         if (hl == 0) { qext[1] = (half_t)1.4423828125f; qext[2] = (half_t)(1.44269504088896340736f - 1.4423828125f); }
     }
-    float m_ref = 0.0f, l_run = 0.0f;    // m_ref is always exactly representable in fp16
+    float m_ref = BIAS != 0 ? -INFINITY : 0.0f, l_run = 0.0f;    // m_ref, once found, is exactly representable in fp16
     bool first = true;
+    // With a mask, blocks of masked keys may come first: finfo.min times log2(e) is -94 498, and scores formed against a point
+    // down there carry fp32 steps of 2^-7.  M is found with the first block above FLOOR.  Until then the products run against
+    // zero, and what the blocks below would weigh among themselves -- the result of a row that has no other keys -- is kept
+    // against a point of its own (m_ref while `first` holds), which only that branch subtracts; the first key that counts
+    // discards it.
+    constexpr float FLOOR = BIAS != 0 ? -1024.0f : -INFINITY;
 
     // Three LDS stages: while block j is in its softmax and second product, the first
     // product of block j+1 already runs (its MFMAs fill the matrix pipe under the
@@ -442,11 +448,21 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
                 for (int r = 1; r < 16; r++) tmax = fmaxf(fmaxf(tmax, sc[0][r]), sc[1][r]);
             }
             float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const bool grow = (mx > TH || first) && mx != -INFINITY;
-            const half_t m16 = (half_t)(m_ref + (grow ? mx : 0.0f));
-            const float d = (float)m16 - m_ref;
-            const float alpha = __builtin_amdgcn_exp2f(-d);
-            m_ref += d;
+            const bool grow = (mx > TH || first) && mx > FLOOR;
+            const float from = first ? 0.0f : m_ref;
+            const half_t m16 = (half_t)(from + (grow ? mx : 0.0f));
+            const float d = (float)m16 - from;
+            // (on the first block there is nothing to rescale, and 0 x 2^-d is no number from d = -128 on)
+            float to = (float)m16, alpha = first ? 0.0f : __builtin_amdgcn_exp2f(-d), dsc = d;
+            if constexpr (BIAS != 0) {
+                if (first && !grow) {                    // masked keys only, so far
+                    to = fmaxf(m_ref, mx);
+                    dsc = to == -INFINITY ? 0.0f : to;
+                    alpha = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_ref - to);
+                }
+                first = first && !grow;
+            }
+            m_ref = to;
             l_run *= alpha;
             if constexpr (SEED) {
 #pragma unroll
@@ -455,7 +471,7 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) { sc[kt][r] -= d; if constexpr (!PP) sn[kt][r] -= d; }   // sn was formed against the old M
+                for (int r = 0; r < 16; r++) { sc[kt][r] -= dsc; if constexpr (!PP) sn[kt][r] -= d; }   // sn was formed against the old M
 #pragma unroll
             for (int t = 0; t < ET; t++)
 #pragma unroll
@@ -464,7 +480,7 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
             probs(sc, pf, l_new);
         }
         l_run = l_new;
-        first = false;
+        if constexpr (BIAS == 0) first = false;
         if constexpr (PP) {
             // Second half of the block.  Block j+2 goes into the stage whose last readers (the other
             // group's second product of block j-1) finished before the barrier just passed; the barrier

@@ -61,3 +61,49 @@ def test_cache_slots_past_the_length_do_not_matter(ctx, B, H, Lq, Lk, E, garbage
         jv.sdpa(ctx, q, k, v, kv_len=kv_len, out=out)
         outs.append(out)
     assert bool(torch.isfinite(outs[0]).all()) and torch.equal(*outs)
+
+
+@pytest.mark.parametrize("fill", [-65504.0, -1000.0, -np.inf])
+@pytest.mark.parametrize("kind", ["key16", "dense16", "dense32"])
+@pytest.mark.parametrize("B,H,Lq,Lk,E", [(2, 2, 90, 300, 40), (1, 3, 130, 270, 80), (1, 2, 70, 270, 120), (2, 16, 830, 1400, 64)])
+def test_left_padding(ctx, B, H, Lq, Lk, E, kind, fill):
+    """Keys masked from the left, by more than a tile or block of them, in every form that carries a mask: a reference point that
+    followed the masked keys down would cost the first keys that count their last bits (fp32 steps of 2^-7 at -65504 log2(e)) or
+    every number (0 x infinity).  With fp16 probabilities and queries such a result is within 4e-4 of fp64; rows whose keys are
+    all masked by one finite value are the softmax of their scores, to the steps that fp32 leaves of s - 65504."""
+    import torch
+    import juliavision_amd as jv
+    q, k, v = (to_dev(oracle.randn_f16((B, H, L, E), s)) for s, L in ((1, Lq), (2, Lk), (3, Lk)))
+    pad = [Lk // 3 + 77, 40][:B]
+    mask = torch.zeros((B, 1, 1 if kind == "key16" else Lq, Lk), dtype=torch.float32 if kind == "dense32" else torch.float16, device="cuda")
+    for b, n in enumerate(pad):
+        mask[b, ..., :n] = fill
+    whole = kind != "key16" and fill != -np.inf
+    if whole:
+        mask[:, :, ::7] = fill                                                        # rows without a key that counts
+    out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, mask, out=out)
+    s = torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3)) / np.sqrt(E) + mask.double().cpu()
+    want, got = torch.matmul(torch.softmax(s, -1), v.double().cpu()), out.double().cpu()
+    rel = lambda a, b: float((a - b).norm() / b.norm())
+    some = torch.ones(Lq, dtype=torch.bool)
+    if whole:
+        some[::7] = False
+        assert rel(got[:, :, ~some], want[:, :, ~some]) <= 1e-2
+    assert rel(got[:, :, some], want[:, :, some]) <= 6e-4
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,E", [(1, 2, 100, 300, 64), (2, 20, 1500, 1500, 64), (1, 2, 130, 270, 80), (1, 2, 70, 270, 120), (1, 2, 40, 300, 64)])
+def test_scores_far_below_zero(ctx, B, H, Lq, Lk, E):
+    """Every score near -200: the first block settles the reference point there, with nothing to rescale yet."""
+    import torch
+    import juliavision_amd as jv
+    c = 2.0 ** round(np.log2(np.sqrt(200 / np.sqrt(E))))                              # exact in fp16: all queries round alike
+    q = torch.full((B, H, Lq, E), c, dtype=torch.float16, device="cuda")
+    k, v = -q.new_full((B, H, Lk, E), c), to_dev(oracle.randn_f16((B, H, Lk, E), 3))
+    out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float16, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, out=out)
+    want = v.float().mean(2, keepdim=True).expand(out.shape)                          # equal scores: equal weights
+    assert float((out.float() - want).norm() / want.norm()) <= 1e-2
