@@ -120,7 +120,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
     for (int r = 0; r < 16; r++) negm[r] = 0.0f;
 #pragma unroll
     for (int t = 0; t < ET; t++) o_acc[t] = negm;
-    float m_run = 0.0f, l_run = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;                        // no reference point yet: negm is 0
     half8v qext;
     if constexpr (MASK) {
 #pragma unroll
@@ -140,6 +140,9 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
         }
     };
     bool first = true;
+    // Keys that a finite mask excludes (finfo.min: -94 498 here) do not settle M, which scores formed against it would pay with
+    // their last bits: see flash_fwd_kernel's FLOOR.
+    constexpr float FLOOR = MASK ? -1024.0f : -INFINITY;
     const char *const kt_lds = wave_lds, *const vt_lds = wave_lds + TILE_BYTES;
     for (int tile = wave; tile < nt; tile += NW) {
         const bool more = tile + NW < nt;
@@ -173,20 +176,29 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
 #pragma unroll
             for (int r = 2; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, sc[r]), sc[r + 1]);
             const float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const bool grow = (mx > TH || first) && mx != -INFINITY;
-            // (M is fp32 here and may lie far below zero after a first tile of masked keys: nothing to rescale yet)
-            const float d = grow ? mx : 0.0f, alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-d);
-            m_run += d;
+            const bool grow = (mx > TH || first) && mx > FLOOR;
+            float d = grow ? mx : 0.0f, alpha = first ? 0.0f : __builtin_amdgcn_exp2f(-d);
+            float to = first ? d : m_run + d;
+#pragma unroll
+            for (int r = 0; r < 16; r++) negm[r] = -to;
+            if constexpr (MASK) {
+                if (first && !grow) {                             // masked keys only, so far
+                    to = fmaxf(m_run, mx);
+                    d = to == -INFINITY ? 0.0f : to;
+                    alpha = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - to);
+                }
+            }
+            m_run = to;
             l_run *= alpha;
 #pragma unroll
-            for (int r = 0; r < 16; r++) { negm[r] = -m_run; sc[r] -= d; }
+            for (int r = 0; r < 16; r++) sc[r] -= d;
 #pragma unroll
             for (int t = 0; t < ET; t++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) o_acc[t][r] *= alpha;
             l_new = l_run;
             probs(sc, pf, l_new);
-            first = first && mx == -INFINITY;                     // the reference point is found with the first key that counts
+            first = first && !grow;                               // the reference point is found with the first key that counts
         }
         l_run = l_new;
         if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");        // V has landed; the next K may be on its way

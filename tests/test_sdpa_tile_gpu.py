@@ -65,7 +65,8 @@ def test_cache_slots_past_the_length_do_not_matter(ctx, B, H, Lq, Lk, E, garbage
 
 @pytest.mark.parametrize("fill", [-65504.0, -1000.0, -np.inf])
 @pytest.mark.parametrize("kind", ["key16", "dense16", "dense32"])
-@pytest.mark.parametrize("B,H,Lq,Lk,E", [(2, 2, 90, 300, 40), (1, 3, 130, 270, 80), (1, 2, 70, 270, 120), (2, 16, 830, 1400, 64)])
+@pytest.mark.parametrize("B,H,Lq,Lk,E", [(1, 2, 100, 300, 64), (2, 3, 20, 300, 64), (1, 2, 70, 330, 72), (1, 2, 33, 300, 16), (1, 2, 65, 260, 128),
+                                         (2, 2, 90, 300, 40), (1, 3, 130, 270, 80), (1, 2, 70, 270, 120), (2, 16, 830, 1400, 64), (2, 16, 300, 520, 64)])
 def test_left_padding(ctx, B, H, Lq, Lk, E, kind, fill):
     """Keys masked from the left, by more than a tile or block of them, in every form that carries a mask: a reference point that
     followed the masked keys down would cost the first keys that count their last bits (fp32 steps of 2^-7 at -65504 log2(e)) or
