@@ -57,6 +57,15 @@ enum mi_bias_mode { MI_BIAS_NONE = 0, MI_BIAS_COL = 1, MI_BIAS_ROW = 2 };
  * planner (the reference's `mmplan`, matmul.jl:87-95) can be tested without a launch. */
 enum mi_gemm_path { MI_GEMM_DECLINE = 0, MI_GEMM_MFMA = 1, MI_GEMM_SKINNY = 2, MI_GEMM_SCALAR = 3 };
 enum mi_sdpa_path { MI_SDPA_DECLINE = 0, MI_SDPA_FLASH = 1, MI_SDPA_ROWS = 2 };
+/* ... and the kernels of that path. */
+enum mi_sdpa_kernel {
+    MI_SDPA_KERNEL_NONE = 0,       /* declined */
+    MI_SDPA_KERNEL_FUSED = 1,      /* flash: 128 or 256 queries a workgroup, head sizes padded to 64, 96 or 128 */
+    MI_SDPA_KERNEL_TILES = 2,      /* flash: 32 queries a workgroup, keys divided among its waves */
+    MI_SDPA_KERNEL_TILES_F32 = 3,  /* rows: the same with scores and probabilities in fp32 */
+    MI_SDPA_KERNEL_ROWS = 4,       /* rows: a query (and key split) a workgroup, any strides and head size */
+    MI_SDPA_KERNEL_ONE_QUERY = 5   /* rows: one query, one launch, split keys merged inside it */
+};
 enum mi_conv_path { MI_CONV_DECLINE = 0, MI_CONV_GEMM_1X1 = 1, MI_CONV_IM2COL_GEMM = 2, MI_CONV_DIRECT = 3, MI_CONV_IMPLICIT_GEMM = 4 };
 enum mi_convt_path { MI_CONVT_DECLINE = 0, MI_CONVT_GEMM_SHUFFLE = 1, MI_CONVT_GATHER = 2 };
 
@@ -326,7 +335,9 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
                 void *ws, size_t ws_bytes, void *stream);
 size_t mi_sdpa_f16_workspace(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, int has_bias);
 /* Returns an mi_sdpa_path; replaces sdpaplan / flashcm_plan -- attention.jl:735-759,
- * flash.jl:1322-1374.  nsplit_out (optional) receives the key-split count
+ * flash.jl:1322-1374.  The path is the precision: MI_SDPA_FLASH rounds scaled queries and
+ * probabilities to fp16 for the matrix units, MI_SDPA_ROWS keeps scores and probabilities in
+ * fp32.  nsplit_out (optional) receives the key-split count of that path's split form
  * (splitcount, flash.jl:1288-1303). */
 int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4],
                      const void *k, const int64_t k_strides[4],

@@ -1140,27 +1140,42 @@ int flash_splits_over_workgroups(int64_t E, int64_t Lq, int64_t Lk, int64_t H, i
     return (int)want;
 }
 
-// Waves of flash_tile_kernel for a call without a dense mask, or 0 where another form is the better one.  Timed on 190 shapes in
-// a replayed graph (head sizes 16 to 128, 2 to 4096 queries and keys, with and without a key mask), the choice is within
-// 1.2 % of the best on average.  Head sizes 16, 32, 72 and 128 were padded to 64, 96 and 128-query tiles: 1.3 to 1.5
-// times as long on average.  At 64 (12 us instead of 14.3 at 6 heads x 1370, 24.9 instead of 35 at 320 x 300) only a chip
-// full of long rows stays with the 256-query and key-halves forms, whose tiles read K and V an eighth as often: from some
-// 820 workgroups over 43 key tiles on (20 x 1500: 23.3 us there, 24.2 here; 16 x 4096: 79 against 103).
+// Waves of flash_tile_kernel for a call that it takes, or 0 where another form is the better one.  `f32`: a call of the rows
+// kernel, whose scores and probabilities stay in fp32.
+// Timed on 190 shapes in a replayed graph (head sizes 16 to 128, 64 to 4096 queries and keys, with and without a key mask): head
+// sizes 16, 32, 72 and 128 were padded to 64, 96 and 128-query tiles, 1.3 to 1.5 times as long on average.  At 64 (12 us
+// instead of 14.3 at 6 heads x 1370, 24.9 instead of 35 at 320 x 300) only a chip full of long rows stays with the 256-query
+// and key-halves forms, whose tiles read K and V an eighth as often: from some 820 workgroups over 43 key tiles on (20 x 1500:
+// 23.3 us there, 24.2 here; 16 x 4096: 79 against 103).
 // Eight waves where every workgroup has a CU of its own and a wave still gets two tiles (6 x 1344: 9.3 us, 10.6 on four);
 // two where the grid fills the chip without more: the merge at the end is what a wave costs (16 x 8 windows of 256 x 72:
 // 12.1 us, 15.7 on four, 23.7 on eight).
-int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B) {
-    const int64_t wgs = ceil_div(Lq, 32) * H * B, nt = ceil_div(Lk, 32), cus = mi_num_cus();
-    if (!mi_sdpa_tile_takes(E) || Lq < 2 || Lk < 1) return 0;
-    if (E == 64 && wgs * 10 >= cus * 32 && nt >= 43) return 0;
+int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, bool f32) {
+    const int64_t wgs = ceil_div(Lq, 32) * H * B, nt = ceil_div(Lk, 32), cus = mi_num_cus(), blocks = ceil_div(Lk, 64);
+    if (!mi_sdpa_tile_head_size(E) || Lq < 2 || Lk < 1) return 0;
     const int waves = wgs <= cus && nt >= 16 ? 8 : wgs * 4 >= cus * 11 ? 2 : 4;
-    // A handful of tiles over thousands of keys: against keys split over workgroups and a merge launch.  A wave takes 0.55
-    // to 1.2 us a tile here; there it is 1 us a 64-key block of a split and 9 us of two launches.
-    // Few queries over 4096 keys or more stay split (level there: 23 x 4096 x 8 heads in 12.7 us, 11.3 here).
-    if (flash_few_queries(E, Lq, Lk, H, B) && nt >= 128) return 0;
-    const int64_t ns = Lq < 64 && !flash_few_queries(E, Lq, Lk, H, B) ? rows_splits(Lq, Lk, H, B) : flash_splits(E, Lq, Lk, H, B);
-    const double tile_us = E <= 64 ? 0.55 : E == 72 ? 0.8 : 1.2;
-    if (ns > 1 && 4.0 + tile_us * (double)ceil_div(nt, waves) > 9.0 + 1.0 * (double)ceil_div(ceil_div(Lk, 64), ns)) return 0;
+    const double tiles = (double)ceil_div(nt, waves), wide = E <= 64 ? 1.0 : E <= 96 ? 1.5 : 1.9;
+    if (f32) {
+        // Against a workgroup per query row (and key split, with a merge launch).  170 shapes of 2 to 63 queries, 16 to 4096
+        // keys, 1 to 320 (head, batch): 12.5 us there, 8.0 here, 7.8 as chosen, 7.7 with the best of both and of 2, 4 and 8
+        // waves (geometric means).  4 x 20 x 60 over 1500 keys: 134 us there, 13.2 here; 16 x 20 x 63 over 4000: 1213 and 73;
+        // 7 queries x 4 heads over 64 keys: 3.8 and 4.2; 8 heads x 4 queries over 2000 keys: 8.3 and 12.
+        const int64_t ns = rows_splits(Lq, Lk, H, B);
+        const double k = E <= 64 ? 1.0 : 1.2, chain = k * (2.2 + 1.4 * (double)ceil_div(blocks, ns)), all = 3.0 + 1.2e-3 * k * k * (double)(Lq * H * B * blocks);
+        const double rows_us = (chain > all ? chain : all) + (ns > 1 ? 2.4 + 0.07 * (double)ns : 0.0);
+        return 2.7 + 0.013 * (double)E + (0.75 + 0.0065 * (double)E) * tiles <= rows_us ? waves : 0;
+    }
+    if (E == 64 && wgs * 10 >= cus * 32 && nt >= 43) return 0;
+    const int64_t ns = flash_splits(E, Lq, Lk, H, B);
+    if (ns > 1) {
+        // A handful of tiles over thousands of keys, against keys split over workgroups and a merge launch (us there, here on
+        // eight waves; 1 head x 128 queries unless said): 64 x 8192 keys 19.1, 24.0; x 4096 18.4, 14.7; 72 x 8192 27.8, 30.6;
+        // 16 x 8192 20.6, 18.2; 128 x 4096 33.9, 22.3; 8 heads x 23 queries x 16 over 4096 12.7, 11.3.
+        const bool few = flash_few_queries(E, Lq, Lk, H, B);
+        if (few && nt >= 128) return 0;                  // (level there)
+        const double per = (double)ceil_div(blocks, ns), split_us = few ? wide * (10.5 + 0.35 * per) : wide * (8.0 + 0.85 * per);
+        if (3.2 + 0.025 * (double)E + (E <= 32 ? 0.46 : E == 64 ? 0.6 : E == 72 ? 0.8 : 1.02) * tiles > split_us) return 0;
+    }
     return waves;
 }
 
@@ -1243,6 +1258,22 @@ int sdpa_path(const SdpaArgs &a) {
     return MI_SDPA_ROWS;
 }
 
+// What runs.  The path says in which precision; within one, the 32-query tiles take what they are estimated to be faster at.
+struct Route { int kernel, waves, nsplit; };
+Route route_of(const SdpaArgs &a) {
+    const int path = sdpa_path(a);
+    if (path == MI_SDPA_DECLINE) return {MI_SDPA_KERNEL_NONE, 0, 1};
+    // (at head size 72 an fp32 result would be 5 % further from exact on the tiles: flash_tile_kernel)
+    if (flash_operands_ok(a) && mi_sdpa_tile_takes(a) && !(path == MI_SDPA_ROWS && a.E == 72 && a.out_f32)) {
+        const int waves = flash_tile_waves(a.E, a.Lq, a.Lk, a.H, a.B, path == MI_SDPA_ROWS);
+        if (waves) return {path == MI_SDPA_ROWS ? MI_SDPA_KERNEL_TILES_F32 : MI_SDPA_KERNEL_TILES, waves, 1};
+    }
+    if (path == MI_SDPA_FLASH) return {MI_SDPA_KERNEL_FUSED, 0, a.bias ? 1 : flash_splits(a.E, a.Lq, a.Lk, a.H, a.B)};
+    const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
+    if (one_pass_decode(a, vec)) return {MI_SDPA_KERNEL_ONE_QUERY, 0, decode_splits(a.E, a.Lk, a.H, a.B)};
+    return {MI_SDPA_KERNEL_ROWS, 0, a.Lq < 64 ? rows_splits(a.Lq, a.Lk, a.H, a.B) : 1};
+}
+
 int fill(SdpaArgs &a, void *out, int out_dtype, const int64_t *os, const void *q, const int64_t *qs, const void *k, const int64_t *ks,
          const void *v, const int64_t *vs, const void *bias, int bias_dtype, const int64_t *bs, const int32_t *kv_len,
          int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, float scale) {
@@ -1312,7 +1343,7 @@ extern "C" {
 size_t mi_sdpa_f16_workspace(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, int has_bias) {
     // sized for the path the call will most likely take: the fused kernel's key splits for Lq >= 64 without
     // an additive mask (unused if the operands turn out not to be 16-byte addressable), the rows kernel's below
-    int ns = Lq >= 64 ? ((has_bias || flash_tile_waves(E, Lq, Lk, H, B)) ? 1 : flash_splits(E, Lq, Lk, H, B)) : rows_splits(Lq, Lk, H, B);
+    int ns = Lq >= 64 ? ((has_bias || flash_tile_waves(E, Lq, Lk, H, B, false)) ? 1 : flash_splits(E, Lq, Lk, H, B)) : rows_splits(Lq, Lk, H, B);
     // few queries over many keys: whichever of the two routes the operands allow must find its partials' room
     if (!has_bias && flash_few_queries(E, Lq, Lk, H, B) && few_query_splits(Lk, H, B) > ns) ns = few_query_splits(Lk, H, B);
     if (ns <= 1) return 0;
@@ -1334,7 +1365,7 @@ int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4], const void *k, c
     int path = sdpa_path(a);
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
     if (nsplit_out) *nsplit_out = (path == MI_SDPA_ROWS && Lq < 64) ? (one_pass_decode(a, vec) ? decode_splits(E, Lk, H, B) : rows_splits(Lq, Lk, H, B))
-                                  : (path == MI_SDPA_FLASH && !has_bias && !flash_tile_waves(E, Lq, Lk, H, B)) ? flash_splits(E, Lq, Lk, H, B) : 1;
+                                  : (path == MI_SDPA_FLASH && !has_bias && !flash_tile_waves(E, Lq, Lk, H, B, false)) ? flash_splits(E, Lq, Lk, H, B) : 1;
     return path;
 }
 
@@ -1360,15 +1391,10 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
     if (rc != MI_OK) return rc;
     if (Lq == 0 || H == 0 || B == 0 || E == 0) return MI_OK;
     hipStream_t st = (hipStream_t)stream;
-    int path = sdpa_path(a);
-    if (path == MI_SDPA_DECLINE) return MI_DECLINE_EXTENT;
-    // (also few queries, which the plan reports with the rows kernel: it reads K and V once per query)
-    if ((!bias || (!a.bias_f32 && (a.bs[1] == 0 || Lq == 1) && Lk <= MI_SDPA_TILE_KEYMASK_MAX)) && (path == MI_SDPA_FLASH || flash_operands_ok(a))) {
-        const int waves = flash_tile_waves(E, Lq, Lk, H, B);
-        rc = waves ? mi_sdpa_tile_launch(a, waves, bias != nullptr, st) : MI_DECLINE_EXTENT;
-        if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
-    }
-    if (path == MI_SDPA_FLASH) {
+    const Route r = route_of(a);
+    if (r.kernel == MI_SDPA_KERNEL_NONE) return MI_DECLINE_EXTENT;
+    if (r.kernel == MI_SDPA_KERNEL_TILES || r.kernel == MI_SDPA_KERNEL_TILES_F32) return mi_sdpa_tile_launch(a, r.waves, r.kernel == MI_SDPA_KERNEL_TILES_F32, st);
+    if (r.kernel == MI_SDPA_KERNEL_FUSED) {
         // The 8-wave ping-pong kernel when 256-query workgroups still cover most of the chip.
         const bool pp = !a.bias && E <= 64 && ceil_div(Lq, 256) * H * B * 4 >= (int64_t)mi_num_cus() * 3;
         if (a.bias) {
@@ -1406,7 +1432,7 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
             hipLaunchKernelGGL((flash_fwd_kernel<64, true>), grid, dim3(512), flash_lds_bytes(64), st, a);
         } else {
             // few query blocks: split the keys over workgroups too, if the caller brought the workspace for it
-            a.nsplit = flash_splits(E, Lq, Lk, H, B);
+            a.nsplit = r.nsplit;
             const size_t rows = (size_t)Lq * H * B;
             const size_t o_bytes = round_up((size_t)a.nsplit * rows * E * sizeof(float), 256);
             if (a.nsplit > 1 && ws && aligned_to(ws, 256) && ws_bytes >= o_bytes + round_up((size_t)a.nsplit * rows * 2 * sizeof(float), 256)) {
@@ -1436,8 +1462,8 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
     }
     // rows path
     bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
-    if (one_pass_decode(a, vec)) return launch_decode(a, st);
-    a.nsplit = Lq < 64 ? rows_splits(Lq, Lk, H, B) : 1;
+    if (r.kernel == MI_SDPA_KERNEL_ONE_QUERY) return launch_decode(a, st);
+    a.nsplit = r.nsplit;
     if (a.nsplit > 1) {
         size_t rows = (size_t)Lq * H * B;
         size_t o_bytes = round_up((size_t)a.nsplit * rows * E * sizeof(float), 256);

@@ -35,8 +35,10 @@ __device__ __forceinline__ void static_for(F &&f) {
 
 }  // namespace
 
-// sdpa_tile.hip: 32-query workgroups whose waves share nothing but the final merge.  `mask`: p.bias is an fp16 row per (head, batch).
-int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool mask, hipStream_t st);
+// sdpa_tile.hip: 32-query workgroups whose waves share nothing but the final merge, for operands that the fused kernels can address
+// and that mi_sdpa_tile_takes.  `f32`: scores and probabilities keep the fp32 that the rows kernel gives them.
 constexpr int MI_SDPA_TILE_KEYMASK_MAX = 4096;
-bool mi_sdpa_tile_takes(int64_t E);
+bool mi_sdpa_tile_head_size(int64_t E);
+bool mi_sdpa_tile_takes(const SdpaArgs &p);
+int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st);
 int mi_sdpa_tile_init();

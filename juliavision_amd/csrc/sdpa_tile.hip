@@ -23,21 +23,31 @@ namespace {
 // Products, register layouts and the lazily moved reference point M are flash_fwd_kernel's: S^T = K Q^T, O^T = V^T P^T, -M in
 // the first product's accumulators.  MASK: an fp16 mask of the key alone, copied to LDS once; it joins in one more k-step
 // as (mask, mask) x (log2(e) split into two positive fp16 parts), so that -inf stays -inf.
+//
+// F32: calls of few queries, which the rows kernel answers with its scores and probabilities in fp32.  Nothing is rounded to fp16
+// here either: Q goes into the product as it lies and the scale joins the scores in fp32 (with the mask, times log2(e), from
+// an fp32 row), a probability enters the second product as two fp16 values (hi, lo) that hold 22 bits of 2^10 p, and what a
+// product adds up is kept short -- 16 head dims, 32 keys -- and joined with vector adds, whose roundings are smaller than the
+// matrix unit's.  Relative error against 64 bits (2-norm, random operands, fp32 result; rows kernel | here | fp16 operands):
+// 23 x 300 x 64: 1.48e-7 | 1.45e-7 | 2.7e-4; 63 x 4000 x 64: 2.4e-7 | 2.0e-7 | 3.0e-4; 23 x 300 x 128: 1.66e-7 | 1.58e-7.  Only at head size
+// 72 it is larger, 1.57e-7 | 1.65e-7: there fp32 results stay with the rows kernel (fp16 ones are off by their rounding, 2.1e-4,
+// either way).
 // Waves a SIMD that the registers of an instance are budgeted for.
-constexpr int tile_waves(int EC) { return EC == 16 ? 2 : EC == 9 ? 3 : 4; }
+constexpr int tile_waves(int EC, bool F32) { return EC == 16 ? 2 : EC == 9 ? (F32 ? 2 : 3) : EC == 8 && F32 ? 3 : 4; }
 
-template <int EC, int NW, bool MASK>
-__global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(SdpaArgs p) {
+template <int EC, int NW, bool MASK, bool F32>
+__global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kernel(SdpaArgs p) {
+    typedef std::conditional_t<F32, float, half_t> mask_t;
     constexpr int E = EC * 8, KS = (E + 15) / 16, ET = (E + 31) / 32;
     constexpr int TILE_BYTES = 32 * EC * 16, NI = (32 * EC + 63) / 64;      // one operand's tile; 1 KB requests for it
     constexpr int WPART = (ET * 16 + 2) * 256, WSTRIDE = WPART > 2 * TILE_BYTES ? WPART : 2 * TILE_BYTES;
-    constexpr float TH = 8.0f;
+    constexpr float UP = F32 ? 1024.0f : 1.0f, TH = F32 ? 4.0f : 8.0f;      // probabilities times UP stay in fp16 range
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hl = lane >> 5, l32 = lane & 31;
     char *const wave_lds = smem + wave * WSTRIDE;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem + wave * WSTRIDE;
-    half_t *const Ms = reinterpret_cast<half_t *>(smem + NW * WSTRIDE);
+    mask_t *const Ms = reinterpret_cast<mask_t *>(smem + NW * WSTRIDE);
 
     // workgroups are dealt to the 8 XCDs round robin: each gets a contiguous run, so a head's query tiles share an L2
     int qblk, h, b;
@@ -99,28 +109,31 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
             uint32_t off = is_k ? koff[i] : voff[i];
             if (over > 0) off -= max(0, s / EC - (31 - over)) * (is_k ? kpitch : vpitch);
             if ((32 * EC) % 64 == 0 || s < 32 * EC)
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(org), "s"(dst + i * 1024) : "memory");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(org), "s"(__builtin_amdgcn_readfirstlane(dst + i * 1024)) : "memory");
         }
     };
     if (wave < nt) { request(true, wave); request(false, wave); }
     if constexpr (MASK) {
         const unsigned short *mrow = reinterpret_cast<const unsigned short *>(p.bias) + (long)h * p.bs[2] + (long)b * p.bs[3];
-        for (int i = threadIdx.x; i < nt * 32; i += NW * 64)
-            reinterpret_cast<unsigned short *>(Ms)[i] = i < p.Lk ? mrow[(long)i * p.bs[0]] : (unsigned short)0;
+        for (int i = threadIdx.x; i < nt * 32; i += NW * 64) {
+            const half_t m = __builtin_bit_cast(half_t, i < p.Lk ? mrow[(long)i * p.bs[0]] : (unsigned short)0);
+            if constexpr (F32) Ms[i] = (float)m * LOG2E;
+            else Ms[i] = m;
+        }
     }
     half8v qf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
         const half8v t = as_half8(qraw[ks]);
 #pragma unroll
-        for (int j = 0; j < 8; j++) qf[ks][j] = (half_t)((float)t[j] * c);
+        for (int j = 0; j < 8; j++) qf[ks][j] = F32 ? t[j] : (half_t)((float)t[j] * c);
     }
     float16v o_acc[ET], negm;
 #pragma unroll
     for (int r = 0; r < 16; r++) negm[r] = 0.0f;
 #pragma unroll
     for (int t = 0; t < ET; t++) o_acc[t] = negm;
-    float m_run = -INFINITY, l_run = 0.0f;                        // no reference point yet: negm is 0
+    float m_run = F32 ? 0.0f : -INFINITY, l_run = 0.0f;           // no reference point yet: negm is 0
     half8v qext;
     if constexpr (MASK) {
 #pragma unroll
@@ -130,19 +143,23 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
     }
     const int vk = (lane & 15) >> 2;                              // key of a transposing read's four
     auto vchunk = [&](int t) { return min(4 * t + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), EC - 1) ^ vswz(vk); };
-    auto probs = [&](const float16v &sx, half8v (&pf)[2], float &l) {
+    auto probs = [&](const float16v &sx, half8v (&pf)[2], half8v (&lo)[2], float &l) {
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(sx[r]), p1 = __builtin_amdgcn_exp2f(sx[r + 1]);
+            const float p0 = __builtin_amdgcn_exp2f(sx[r]) * UP, p1 = __builtin_amdgcn_exp2f(sx[r + 1]) * UP;
             pf[r >> 3][r & 7] = (half_t)p0;
             pf[r >> 3][(r & 7) + 1] = (half_t)p1;
+            if constexpr (F32) {
+                lo[r >> 3][r & 7] = (half_t)(p0 - (float)(half_t)p0);
+                lo[r >> 3][(r & 7) + 1] = (half_t)(p1 - (float)(half_t)p1);
+            }
             l += p0 + p1;
         }
     };
     bool first = true;
     // Keys that a finite mask excludes (finfo.min: -94 498 here) do not settle M, which scores formed against it would pay with
     // their last bits: see flash_fwd_kernel's FLOOR.
-    constexpr float FLOOR = MASK ? -1024.0f : -INFINITY;
+    constexpr float FLOOR = MASK && !F32 ? -1024.0f : -INFINITY;      // (F32: the scores are kept, and scaled again)
     const char *const kt_lds = wave_lds, *const vt_lds = wave_lds + TILE_BYTES;
     for (int tile = wave; tile < nt; tile += NW) {
         const bool more = tile + NW < nt;
@@ -152,7 +169,15 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
         for (int ks = 0; ks < KS; ks++)
             kf[ks] = *reinterpret_cast<const half8v *>(kt_lds + (l32 * EC + (min(2 * ks + hl, EC - 1) ^ kswz(l32))) * 16);
         half8v kx = {};
-        if constexpr (MASK) {
+        float16v ms;
+        if constexpr (MASK && F32) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const float4v m = *reinterpret_cast<const float4v *>(Ms + tile * 32 + 8 * g + 4 * hl);
+#pragma unroll
+                for (int e = 0; e < 4; e++) ms[4 * g + e] = m[e];
+            }
+        } else if constexpr (MASK) {
             const half_t m = Ms[tile * 32 + l32];
             kx[0] = hl == 0 ? m : (half_t)0.0f;
             kx[1] = kx[0];
@@ -161,16 +186,31 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
         if (more) request(true, tile + NW);
         float16v sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[0], qf[0], negm, 0, 0, 0);
 #pragma unroll
-        for (int ks = 1; ks < KS; ks++) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
-        if constexpr (MASK) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
-        if (tile * 32 + 32 > Lk) {                                // the ragged last tile: excluded keys get -inf
+        for (int ks = 1; ks < KS; ks++) {
+            if constexpr (F32) {
+                const float16v part = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], negm, 0, 0, 0);      // (negm stays 0)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (tile * 32 + 8 * (r >> 2) + 4 * hl + (r & 3) >= Lk) sc[r] = -INFINITY;
+                for (int r = 0; r < 16; r++) sc[r] += part[r];
+            } else sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
         }
-        half8v pf[2];
+        if constexpr (MASK && !F32) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
+        const float16v raw = sc;
+        auto scale = [&]() {
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] = fmaf(raw[r], c, MASK ? ms[r] - m_run : -m_run);
+        };
+        auto cut = [&]() {                                        // the ragged last tile: excluded keys get -inf
+            if (tile * 32 + 32 > Lk) {
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (tile * 32 + 8 * (r >> 2) + 4 * hl + (r & 3) >= Lk) sc[r] = -INFINITY;
+            }
+        };
+        if constexpr (F32) scale();
+        cut();
+        half8v pf[2], lo[2];
         float l_new = l_run;
-        probs(sc, pf, l_new);
+        probs(sc, pf, lo, l_new);
         if (__any(first || !(l_new - l_run < 65504.0f))) {        // flash_fwd_kernel says why
             float tmax = fmaxf(sc[0], sc[1]);
 #pragma unroll
@@ -179,9 +219,11 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
             const bool grow = (mx > TH || first) && mx > FLOOR;
             float d = grow ? mx : 0.0f, alpha = first ? 0.0f : __builtin_amdgcn_exp2f(-d);
             float to = first ? d : m_run + d;
+            if constexpr (!F32) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) negm[r] = -to;
-            if constexpr (MASK) {
+                for (int r = 0; r < 16; r++) negm[r] = -to;
+            }
+            if constexpr (MASK && !F32) {
                 if (first && !grow) {                             // masked keys only, so far
                     to = fmaxf(m_run, mx);
                     d = to == -INFINITY ? 0.0f : to;
@@ -190,14 +232,19 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
             }
             m_run = to;
             l_run *= alpha;
+            if constexpr (F32) {
+                scale();
+                cut();
+            } else {
 #pragma unroll
-            for (int r = 0; r < 16; r++) sc[r] -= d;
+                for (int r = 0; r < 16; r++) sc[r] -= d;
+            }
 #pragma unroll
             for (int t = 0; t < ET; t++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) o_acc[t][r] *= alpha;
             l_new = l_run;
-            probs(sc, pf, l_new);
+            probs(sc, pf, lo, l_new);
             first = first && !grow;                               // the reference point is found with the first key that counts
         }
         l_run = l_new;
@@ -217,9 +264,19 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC)) void flash_tile_kernel(Sdp
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (more) request(false, tile + NW);
 #pragma unroll
-        for (int t = 0; t < ET; t++)
+        for (int t = 0; t < ET; t++) {
+            if constexpr (F32) {                                  // the small parts first
+                float16v part = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][0], lo[0], negm, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][1], lo[1], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][0], pf[0], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][1], pf[1], part, 0, 0, 0);
 #pragma unroll
-            for (int bb = 0; bb < 2; bb++) o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][bb], pf[bb], o_acc[t], 0, 0, 0);
+                for (int r = 0; r < 16; r++) o_acc[t][r] += part[r];
+            } else {
+#pragma unroll
+                for (int bb = 0; bb < 2; bb++) o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][bb], pf[bb], o_acc[t], 0, 0, 0);
+            }
+        }
     }
     // The waves' partials, lane-major, each into its own stretch, then every wave finishes (t, g) pairs: head dims
     // 32 t + 8 g + 4 hl .. +3 of its lane's query.
@@ -275,41 +332,49 @@ constexpr int tile_lds_bytes() {
     constexpr int part = ((EC * 8 + 31) / 32 * 16 + 2) * 256, tiles = 2 * 32 * EC * 16;
     return NW * (part > tiles ? part : tiles);
 }
-template <int EC, int NW>
+template <int EC, int NW, bool F32>
 int launch_tiles(const SdpaArgs &p, bool mask, hipStream_t st) {
     const dim3 grid((unsigned)ceil_div(p.Lq, 32), (unsigned)p.H, (unsigned)p.B);
     const int lds = tile_lds_bytes<EC, NW>();
-    if (mask) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, true>), grid, dim3(NW * 64), lds + (int)round_up((size_t)ceil_div(p.Lk, 32) * 64, 16), st, p);
-    else      hipLaunchKernelGGL((flash_tile_kernel<EC, NW, false>), grid, dim3(NW * 64), lds, st, p);
+    if (mask) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, true, F32>), grid, dim3(NW * 64), lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st, p);
+    else      hipLaunchKernelGGL((flash_tile_kernel<EC, NW, false, F32>), grid, dim3(NW * 64), lds, st, p);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
-template <int EC>
+template <int EC, bool F32>
 int launch_waves(const SdpaArgs &p, int waves, bool mask, hipStream_t st) {
-    return waves == 2 ? launch_tiles<EC, 2>(p, mask, st) : waves == 4 ? launch_tiles<EC, 4>(p, mask, st) : launch_tiles<EC, 8>(p, mask, st);
+    return waves == 2 ? launch_tiles<EC, 2, F32>(p, mask, st) : waves == 4 ? launch_tiles<EC, 4, F32>(p, mask, st) : launch_tiles<EC, 8, F32>(p, mask, st);
 }
-template <int EC, int NW>
+template <int EC, int NW, bool F32>
 int raise() {
     const int lds = tile_lds_bytes<EC, NW>();
-    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + 2 * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
-           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
+    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, true, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + (F32 ? 4 : 2) * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
+           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, false, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
 }
 template <int EC>
-int raise_all() { return raise<EC, 2>() | raise<EC, 4>() | raise<EC, 8>(); }
+int raise_all() { return raise<EC, 2, false>() | raise<EC, 4, false>() | raise<EC, 8, false>() | raise<EC, 2, true>() | raise<EC, 4, true>() | raise<EC, 8, true>(); }
 
 }  // namespace
 
-bool mi_sdpa_tile_takes(int64_t E) { return E == 16 || E == 32 || E == 64 || E == 72 || E == 128; }
-
-int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool mask, hipStream_t st) {
-    if (!mi_sdpa_tile_takes(p.E) || (mask && p.Lk > MI_SDPA_TILE_KEYMASK_MAX)) return MI_DECLINE_EXTENT;
+// Head sizes: those of this package's models and tests.  The chunk permutations hold for rows of 2, 4, 8, 9 and 16 chunks; 40, 48, 80,
+// 96 and the rest run the padded forms of flash_fwd_kernel, which no figure here has been taken against.
+bool mi_sdpa_tile_head_size(int64_t E) { return E == 16 || E == 32 || E == 64 || E == 72 || E == 128; }
+bool mi_sdpa_tile_takes(const SdpaArgs &p) {
+    if (!mi_sdpa_tile_head_size(p.E)) return false;
+    // an fp16 mask of the key alone, whose row fits the LDS
+    if (p.bias && (p.bias_f32 || (p.bs[1] != 0 && p.Lq != 1) || p.Lk > MI_SDPA_TILE_KEYMASK_MAX)) return false;
     // per-lane load offsets are 32-bit byte offsets from a tile's first row
-    if (p.ks[1] < 0 || p.vs[1] < 0 || p.ks[1] * 64 >= (1l << 31) || p.vs[1] * 64 >= (1l << 31)) return MI_DECLINE_EXTENT;
+    return p.ks[1] >= 0 && p.vs[1] >= 0 && p.ks[1] * 64 < (1l << 31) && p.vs[1] * 64 < (1l << 31);
+}
+
+int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st) {
+    if (!mi_sdpa_tile_takes(p)) return MI_DECLINE_EXTENT;
+    const bool mask = p.bias != nullptr;
     switch (p.E) {
-    case 16: return launch_waves<2>(p, waves, mask, st);
-    case 32: return launch_waves<4>(p, waves, mask, st);
-    case 64: return launch_waves<8>(p, waves, mask, st);
-    case 72: return launch_waves<9>(p, waves, mask, st);
-    default: return launch_waves<16>(p, waves, mask, st);
+    case 16: return f32 ? launch_waves<2, true>(p, waves, mask, st) : launch_waves<2, false>(p, waves, mask, st);
+    case 32: return f32 ? launch_waves<4, true>(p, waves, mask, st) : launch_waves<4, false>(p, waves, mask, st);
+    case 64: return f32 ? launch_waves<8, true>(p, waves, mask, st) : launch_waves<8, false>(p, waves, mask, st);
+    case 72: return f32 ? launch_waves<9, true>(p, waves, mask, st) : launch_waves<9, false>(p, waves, mask, st);
+    default: return f32 ? launch_waves<16, true>(p, waves, mask, st) : launch_waves<16, false>(p, waves, mask, st);
     }
 }
 

@@ -108,3 +108,26 @@ def test_scores_far_below_zero(ctx, B, H, Lq, Lk, E):
     jv.sdpa(ctx, q, k, v, out=out)
     want = v.float().mean(2, keepdim=True).expand(out.shape)                          # equal scores: equal weights
     assert float((out.float() - want).norm() / want.norm()) <= 1e-2
+
+
+# Relative errors (2-norm, fp32 result) against fp64 of a workgroup per query row, which keeps everything in fp32 and answered these
+# calls before there were tiles: measured on these operands, the third digit rounded up.
+@pytest.mark.parametrize("B,H,Lq,Lk,E,mask,rows", [
+    (8, 8, 32, 32, 64, False, 1.18e-7), (2, 8, 23, 300, 64, True, 1.44e-7), (4, 20, 60, 1500, 64, True, 1.91e-7), (16, 8, 40, 256, 64, False, 1.46e-7),
+    (8, 16, 2, 1000, 64, False, 1.66e-7), (2, 8, 23, 300, 16, True, 1.44e-7), (4, 20, 60, 1500, 16, True, 1.98e-7), (16, 8, 40, 256, 32, False, 1.62e-7),
+    (2, 8, 23, 300, 128, False, 1.66e-7), (8, 16, 2, 1000, 128, True, 1.79e-7)])
+def test_few_queries_keep_fp32(ctx, B, H, Lq, Lk, E, mask, rows):
+    import torch
+    import juliavision_amd as jv
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(B, H, L, E, generator=gen, device="cuda").half() for L in (Lq, Lk, Lk))
+    bias = None
+    if mask:
+        length = Lk - torch.randint(0, Lk // 3, (B, 1), generator=gen, device="cuda")
+        bias = torch.where(torch.arange(Lk, device="cuda")[None] < length, 0.0, -65504.0).half().view(B, 1, 1, Lk)
+    out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, bias, out=out)
+    s = torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3)) / np.sqrt(E) + (0.0 if bias is None else bias.double().cpu())
+    want = torch.matmul(torch.softmax(s, -1), v.double().cpu())
+    assert float((out.double().cpu() - want).norm() / want.norm()) <= rows
