@@ -57,7 +57,7 @@ enum mi_bias_mode { MI_BIAS_NONE = 0, MI_BIAS_COL = 1, MI_BIAS_ROW = 2 };
  * planner (the reference's `mmplan`, matmul.jl:87-95) can be tested without a launch. */
 enum mi_gemm_path { MI_GEMM_DECLINE = 0, MI_GEMM_MFMA = 1, MI_GEMM_SKINNY = 2, MI_GEMM_SCALAR = 3 };
 enum mi_sdpa_path { MI_SDPA_DECLINE = 0, MI_SDPA_FLASH = 1, MI_SDPA_ROWS = 2 };
-/* ... and the kernels of that path. */
+/* ... and which kernel of that path runs (mi_sdpa_f16_kernel). */
 enum mi_sdpa_kernel {
     MI_SDPA_KERNEL_NONE = 0,       /* declined */
     MI_SDPA_KERNEL_FUSED = 1,      /* flash: 128 or 256 queries a workgroup, head sizes padded to 64, 96 or 128 */
@@ -338,13 +338,23 @@ size_t mi_sdpa_f16_workspace(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64
  * flash.jl:1322-1374.  The path is the precision: MI_SDPA_FLASH rounds scaled queries and
  * probabilities to fp16 for the matrix units, MI_SDPA_ROWS keeps scores and probabilities in
  * fp32.  nsplit_out (optional) receives the key-split count of that path's split form
- * (splitcount, flash.jl:1288-1303). */
+ * (splitcount, flash.jl:1288-1303); mi_sdpa_f16_kernel says which form a call runs. */
 int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4],
                      const void *k, const int64_t k_strides[4],
                      const void *v, const int64_t v_strides[4],
                      int has_bias, int has_kv_len,
                      int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, float scale,
                      int *nsplit_out);
+
+/* Which kernel mi_sdpa_f16 launches for these operands (an mi_sdpa_kernel; out may be NULL for a dense, aligned result,
+ * q, k, v and bias are not read) and, in nsplit_out (optional), over how many workgroups it cuts the keys. */
+int mi_sdpa_f16_kernel(const void *out, int out_dtype, const int64_t out_strides[4],
+                       const void *q, const int64_t q_strides[4],
+                       const void *k, const int64_t k_strides[4],
+                       const void *v, const int64_t v_strides[4],
+                       const void *bias, int bias_dtype, const int64_t bias_strides[4],
+                       int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, float scale,
+                       int *nsplit_out);
 
 /* mi_sdpa_f16_plan for a device the caller describes (see mi_gemm_f16_plan_caps): without a matrix unit the fused
  * kernel is not offered, and the compute-unit count decides the key splits (splitcount(dev, ...), flash.jl:1288-1303). */

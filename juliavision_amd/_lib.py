@@ -22,6 +22,7 @@ W_KF, W_FK = 0, 1
 BIAS_NONE, BIAS_COL, BIAS_ROW = 0, 1, 2
 GEMM_PATHS = {0: "decline", 1: "mfma", 2: "skinny", 3: "scalar"}
 SDPA_PATHS = {0: "decline", 1: "flash", 2: "rows"}
+SDPA_KERNELS = {0: "none", 1: "fused", 2: "tiles", 3: "tiles_f32", 4: "rows", 5: "one_query"}
 CONV_PATHS = {0: "decline", 1: "gemm_1x1", 2: "im2col_gemm", 3: "direct", 4: "implicit_gemm"}
 CONVT_PATHS = {0: "decline", 1: "gemm_shuffle", 2: "gather"}
 
@@ -60,6 +61,7 @@ SIGNATURES = {
     "mi_sdpa_f16": (_int, [_vp, _int, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _int, _i64p, _vp] + [_i64] * 5 + [_f32, _vp, _sz, _vp]),
     "mi_sdpa_f16_workspace": (_sz, [_i64] * 5 + [_int]),
     "mi_sdpa_f16_plan": (_int, [_vp, _i64p, _vp, _i64p, _vp, _i64p, _int, _int] + [_i64] * 5 + [_f32, C.POINTER(C.c_int)]),
+    "mi_sdpa_f16_kernel": (_int, [_vp, _int, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _int, _i64p] + [_i64] * 5 + [_f32, C.POINTER(C.c_int)]),
     "mi_conv2d_f16": (_int, [_vp] * 4 + [_i64] * 14 + [_int, _vp, _sz, _vp]),
     "mi_conv2d_f16_workspace": (_sz, [_i64] * 13),
     "mi_conv2d_f16_plan": (_int, [_i64] * 14),

@@ -1365,7 +1365,7 @@ int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4], const void *k, c
     int path = sdpa_path(a);
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
     if (nsplit_out) *nsplit_out = (path == MI_SDPA_ROWS && Lq < 64) ? (one_pass_decode(a, vec) ? decode_splits(E, Lk, H, B) : rows_splits(Lq, Lk, H, B))
-                                  : (path == MI_SDPA_FLASH && !has_bias && !flash_tile_waves(E, Lq, Lk, H, B, false)) ? flash_splits(E, Lq, Lk, H, B) : 1;
+                                  : (path == MI_SDPA_FLASH && !has_bias && !(E == 64 && Lq >= 64 && flash_tile_waves(E, Lq, Lk, H, B, false))) ? flash_splits(E, Lq, Lk, H, B) : 1;
     return path;
 }
 
@@ -1376,6 +1376,19 @@ int mi_sdpa_f16_plan_caps(const int64_t caps[6], const void *q, const int64_t q_
     const int path = mi_sdpa_f16_plan(q, q_strides, k, k_strides, v, v_strides, has_bias, has_kv_len, E, Lq, Lk, H, B, scale, nsplit_out);
     mi_plan_caps_end();
     return path;
+}
+
+int mi_sdpa_f16_kernel(const void *out, int out_dtype, const int64_t out_strides[4],
+                       const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                       const void *v, const int64_t v_strides[4],
+                       const void *bias, int bias_dtype, const int64_t bias_strides[4],
+                       int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, float scale, int *nsplit_out) {
+    SdpaArgs a;
+    if (fill(a, const_cast<void *>(out), out_dtype, out_strides, q, q_strides, k, k_strides, v, v_strides, bias, bias_dtype, bias_strides, nullptr, E, Lq, Lk, H, B, scale) != MI_OK)
+        return MI_SDPA_KERNEL_NONE;
+    const Route r = route_of(a);
+    if (nsplit_out) *nsplit_out = r.nsplit;
+    return r.kernel;
 }
 
 int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],

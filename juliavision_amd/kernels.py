@@ -30,7 +30,7 @@ import weakref
 
 import ctypes as C
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import NamedTuple, Optional
 
 import torch
@@ -638,15 +638,20 @@ def matmul_heads_(ctx: Ctx, out, A, B, bias=None):
 
 @dataclass(frozen=True)
 class FlashPlan:
-    """Fused MFMA kernel (the counterpart of FlashCMPlan, kernelplans.jl:54-324)."""
+    """Fused MFMA kernel with queries and probabilities in fp16 (the counterpart of FlashCMPlan, kernelplans.jl:54-324).
+    ``nsplit``: key splits of the form that has them.  ``kernel``: what runs on this device (``L.SDPA_KERNELS``), not part of
+    what makes two plans equal."""
     nsplit: int = 1
+    kernel: str = field(default="", compare=False)
 
 
 @dataclass(frozen=True)
 class RowsSDPAPlan:
-    """One workgroup per query row and key split: decode-sized Lq, additive masks,
-    strided or odd-sized heads (takes the place of the three-pass path, attention.jl:790-834)."""
+    """Scores and probabilities in fp32: decode-sized Lq, strided or odd-sized heads, masks the fused kernel does not carry
+    (takes the place of the three-pass path, attention.jl:790-834).  ``nsplit``: key splits of a workgroup per query row;
+    ``kernel``: what runs on this device."""
     nsplit: int = 1
+    kernel: str = field(default="", compare=False)
 
 
 def _strides_elbh(t: torch.Tensor):
@@ -679,6 +684,9 @@ def sdpaplan(ctx: Ctx, q, k, v, bias=None, scale=None, kv_len=None):
     scale = (1.0 / math.sqrt(E)) if scale is None else float(scale)
     ns = C.c_int(1)
     devcaps = _caps_array(ctx.dev)
+    runs = L.SDPA_KERNELS[L.load().mi_sdpa_f16_kernel(
+        None, L.F16, None, q.data_ptr(), _strides_elbh(q), k.data_ptr(), _strides_elbh(k), v.data_ptr(), _strides_elbh(v), _ptr(bias),
+        L.F32 if bias is not None and bias.dtype == torch.float32 else L.F16, None if bias is None else _bias_strides(bias, Lk, Lq, H, Bq), E, Lq, Lk, H, Bq, scale, None)]
     path = L.load().mi_sdpa_f16_plan_caps(devcaps, q.data_ptr(), _strides_elbh(q), k.data_ptr(), _strides_elbh(k), v.data_ptr(), _strides_elbh(v),
                                           0, int(kv_len is not None), E, Lq, Lk, H, Bq, scale, C.byref(ns))
     if bias is not None:
@@ -687,18 +695,18 @@ def sdpaplan(ctx: Ctx, q, k, v, bias=None, scale=None, kv_len=None):
         # dense fp16 one, so the mask's own layout is judged here, as mi_sdpa_f16 judges it at the call.
         bst = list(_bias_strides(bias, Lk, Lq, H, Bq))
         by_key = bias.dtype == torch.float16 and (bst[1] == 0 or Lq == 1) and Lk <= 4096    # the same for every query: no layout conditions
-        fused = path == 1 and (by_key or ((bst[0] == 1 or Lk == 1) and bias.data_ptr() % 4 == 0 and
+        fused = path == 1 and Lq >= 64 and (by_key or ((bst[0] == 1 or Lk == 1) and bias.data_ptr() % 4 == 0 and
                                           (bias.dtype == torch.float32 or all(x % 2 == 0 for x in bst[1:]))))
         if fused:
-            return FlashPlan(1)
+            return FlashPlan(1, runs)
         ns1 = C.c_int(1)
         L.load().mi_sdpa_f16_plan_caps(devcaps, q.data_ptr(), _strides_elbh(q), k.data_ptr(), _strides_elbh(k), v.data_ptr(), _strides_elbh(v),
                                        1, int(kv_len is not None), E, Lq, Lk, H, Bq, scale, C.byref(ns1))
-        return RowsSDPAPlan(ns1.value if Lq < 64 else 1) if path in (1, 2) else Decline("extent")
+        return RowsSDPAPlan(ns1.value if Lq < 64 else 1, runs) if path in (1, 2) else Decline("extent")
     if path == 1:
-        return FlashPlan(ns.value)
+        return FlashPlan(ns.value, runs)
     if path == 2:
-        return RowsSDPAPlan(ns.value)
+        return RowsSDPAPlan(ns.value, runs)
     return Decline("extent")
 
 

@@ -1,0 +1,49 @@
+"""Which kernel runs, asked on the CPU: the answer follows the path (the precision) that the plan names, over the forms a call can take."""
+import ctypes as C
+import itertools
+
+import pytest
+
+from juliavision_amd import _lib as L
+
+PTR = 0x10000
+OF_PATH = {"decline": {"none"}, "flash": {"fused", "tiles"}, "rows": {"tiles_f32", "rows", "one_query"}}
+
+
+def _sdpa(E, Lq, Lk, H, B, *, packed=False, mask=None, q=PTR, out=None, out_strides=None, f32=False):
+    row = 3 * H * E if packed else E
+    st = (lambda n: L.strides4(1, row, E, row * n)) if packed else (lambda n: L.strides4(1, E, E * n, E * n * H))
+    ns, nsplit = C.c_int(0), C.c_int(0)
+    path = L.load().mi_sdpa_f16_plan(q, st(Lq), PTR, st(Lk), PTR, st(Lk), int(mask is not None), 0, E, Lq, Lk, H, B, 0.125, C.byref(ns))
+    bst = {None: None, "key": L.strides4(1, 0, 0, Lk), "dense": L.strides4(1, Lk, Lk * Lq, Lk * Lq * H), "key32": L.strides4(1, 0, 0, Lk)}[mask]
+    kernel = L.load().mi_sdpa_f16_kernel(out, L.F32 if f32 else L.F16, out_strides, q, st(Lq), PTR, st(Lk), PTR, st(Lk), None if mask is None else PTR,
+                                         L.F32 if mask == "key32" else L.F16, bst, E, Lq, Lk, H, B, 0.125, C.byref(nsplit))
+    return L.SDPA_PATHS[path], L.SDPA_KERNELS[kernel], ns.value, nsplit.value
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_the_kernel_is_one_of_the_plans_path(packed):
+    seen = set()
+    for E, Lq, Lk, (H, B), mask in itertools.product([16, 20, 32, 40, 64, 72, 80, 128, 160, 256], [1, 2, 7, 23, 63, 64, 128, 700, 4096],
+                                                     [1, 16, 64, 300, 1500, 4096, 8192], [(1, 1), (8, 1), (20, 4)], [None, "key", "dense"]):
+        path, kernel, plan_splits, splits = _sdpa(E, Lq, Lk, H, B, packed=packed, mask=mask)
+        if mask == "key" and path == "rows" and Lq >= 64:                      # the plan sees a dense mask, whose rows may start off 4 bytes
+            assert kernel in OF_PATH["flash"] | OF_PATH["rows"]
+        else:
+            assert kernel in OF_PATH[path], (E, Lq, Lk, H, B, mask)
+        assert splits <= max(plan_splits, 1), (E, Lq, Lk, H, B, mask)             # the workspace has room for the plan's
+        seen.add(kernel)
+    assert seen == {"none"} | OF_PATH["flash"] | OF_PATH["rows"] or seen == OF_PATH["flash"] | OF_PATH["rows"]
+
+
+def test_what_the_tiles_do_not_take():
+    assert _sdpa(64, 256, 256, 8, 4)[1] == "tiles"
+    assert _sdpa(64, 256, 256, 8, 4, q=PTR + 2)[1] == "rows"                       # off 16 bytes
+    assert _sdpa(64, 256, 256, 8, 4, out=PTR + 2)[1] == "rows"
+    assert _sdpa(64, 256, 256, 8, 4, mask="dense")[1] == "fused" and _sdpa(64, 256, 256, 8, 4, mask="key32")[1] == "fused"
+    assert _sdpa(64, 256, 5000, 8, 4, mask="key")[1] in ("fused", "rows")          # a mask row longer than its LDS
+    assert _sdpa(80, 256, 256, 8, 4)[1] == "fused"                                 # a head size without chunk permutations
+    assert _sdpa(64, 23, 300, 8, 2)[1] == _sdpa(64, 23, 300, 8, 2, f32=True)[1] == "tiles_f32"
+    assert _sdpa(72, 23, 300, 8, 2)[1] == "tiles_f32" and _sdpa(72, 23, 300, 8, 2, f32=True)[1] == "rows"
+    assert _sdpa(64, 23, 300, 8, 2, mask="key")[1] == "tiles_f32" and _sdpa(64, 23, 300, 8, 2, mask="key32")[1] == "rows"
+    assert _sdpa(64, 1, 1500, 20, 1)[1:] == ("one_query", 4, 4)

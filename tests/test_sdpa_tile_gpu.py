@@ -125,9 +125,21 @@ def test_few_queries_keep_fp32(ctx, B, H, Lq, Lk, E, mask, rows):
     if mask:
         length = Lk - torch.randint(0, Lk // 3, (B, 1), generator=gen, device="cuda")
         bias = torch.where(torch.arange(Lk, device="cuda")[None] < length, 0.0, -65504.0).half().view(B, 1, 1, Lk)
+    plan = jv.sdpaplan(ctx, q, k, v, bias)
+    assert type(plan).__name__ == "RowsSDPAPlan" and plan.kernel == "tiles_f32", plan
     out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float32, device="cuda")
     ctx.ws.reset()
     jv.sdpa(ctx, q, k, v, bias, out=out)
     s = torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3)) / np.sqrt(E) + (0.0 if bias is None else bias.double().cpu())
     want = torch.matmul(torch.softmax(s, -1), v.double().cpu())
     assert float((out.double().cpu() - want).norm() / want.norm()) <= rows
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,E,mask,kernel", [(1, 4, 7, 64, 64, False, "rows"), (1, 20, 1, 448, 64, False, "one_query"), (1, 8, 23, 700, 16, False, "tiles"),
+                                                     (1, 8, 23, 4096, 16, False, "fused"), (1, 16, 4096, 4096, 64, False, "fused"), (1, 6, 1370, 1370, 64, True, "tiles"),
+                                                     (2, 8, 23, 300, 72, True, "tiles_f32")])
+def test_the_plan_names_the_kernel(ctx, B, H, Lq, Lk, E, mask, kernel):
+    import torch
+    import juliavision_amd as jv
+    q, k, v = (torch.zeros(B, H, L, E, dtype=torch.float16, device="cuda") for L in (Lq, Lk, Lk))
+    assert jv.sdpaplan(ctx, q, k, v, q.new_zeros(B, 1, 1, Lk) if mask else None).kernel == kernel
