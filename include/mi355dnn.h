@@ -67,6 +67,15 @@ enum mi_sdpa_kernel {
     MI_SDPA_KERNEL_ONE_QUERY = 5   /* rows: one query, one launch, split keys merged inside it */
 };
 enum mi_conv_path { MI_CONV_DECLINE = 0, MI_CONV_GEMM_1X1 = 1, MI_CONV_IM2COL_GEMM = 2, MI_CONV_DIRECT = 3, MI_CONV_IMPLICIT_GEMM = 4 };
+/* ... and which kernel runs (mi_conv2d_f16_kernel). */
+enum mi_conv_kernel {
+    MI_CONV_KERNEL_NONE = 0,         /* declined */
+    MI_CONV_KERNEL_GEMM_1X1 = 1,     /* x is the operand as it lies */
+    MI_CONV_KERNEL_IM2COL_GEMM = 2,  /* the patch matrix written out, then a GEMM */
+    MI_CONV_KERNEL_DIRECT = 3,       /* groups: a thread per output */
+    MI_CONV_KERNEL_PATCH_GEMM = 4,   /* a padded channels-last copy, patches gathered from it by the GEMM */
+    MI_CONV_KERNEL_TILE = 5          /* one launch: patches and weights staged in LDS as they lie */
+};
 enum mi_convt_path { MI_CONVT_DECLINE = 0, MI_CONVT_GEMM_SHUFFLE = 1, MI_CONVT_GATHER = 2 };
 
 /* Library / device. */
@@ -391,12 +400,18 @@ size_t mi_conv2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
                                int64_t KW, int64_t KH, int64_t Cout,
                                int64_t stride_x, int64_t stride_y, int64_t pad_x, int64_t pad_y,
                                int64_t dil_x, int64_t dil_y);
-/* Returns an mi_conv_path; replaces conv_coopmat_plan / onebyone -- conv_coopmat.jl:83-155,
- * conv.jl:63-66. */
+/* Returns an mi_conv_path -- which of the reference's formulations the extents are given to -- and replaces
+ * conv_coopmat_plan / onebyone -- conv_coopmat.jl:83-155, conv.jl:63-66.  What runs is mi_conv2d_f16_kernel's to say. */
 int mi_conv2d_f16_plan(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
                        int64_t KW, int64_t KH, int64_t Cout,
                        int64_t stride_x, int64_t stride_y, int64_t pad_x, int64_t pad_y,
                        int64_t dil_x, int64_t dil_y, int64_t groups);
+/* Which kernel mi_conv2d_f16 runs for these extents on the current device (an mi_conv_kernel), and in scratch_out (optional) the
+ * workspace bytes it uses: mi_conv2d_f16_workspace's answer or less. */
+int mi_conv2d_f16_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
+                         int64_t KW, int64_t KH, int64_t Cout,
+                         int64_t stride_x, int64_t stride_y, int64_t pad_x, int64_t pad_y,
+                         int64_t dil_x, int64_t dil_y, int64_t groups, size_t *scratch_out);
 /* The same convolution over channels-last tensors: x [N][H][W][Cin], w [Cout][KH][KW][Cin], out [N][OH][OW][Cout]
  * (groups = 1).  An implicit GEMM with nothing staged: out[(n,oh,ow)][Cout] = patch . w^T, the patch matrix gathered
  * from x by the GEMM's own operand loads, the weights read as they lie; split-K planes in ws where the output tiles

@@ -24,6 +24,7 @@ GEMM_PATHS = {0: "decline", 1: "mfma", 2: "skinny", 3: "scalar"}
 SDPA_PATHS = {0: "decline", 1: "flash", 2: "rows"}
 SDPA_KERNELS = {0: "none", 1: "fused", 2: "tiles", 3: "tiles_f32", 4: "rows", 5: "one_query"}
 CONV_PATHS = {0: "decline", 1: "gemm_1x1", 2: "im2col_gemm", 3: "direct", 4: "implicit_gemm"}
+CONV_KERNELS = {0: "none", 1: "gemm_1x1", 2: "im2col_gemm", 3: "direct", 4: "patch_gemm", 5: "tile"}
 CONVT_PATHS = {0: "decline", 1: "gemm_shuffle", 2: "gather"}
 
 _i64, _int, _vp, _sz, _f32 = C.c_int64, C.c_int, C.c_void_p, C.c_size_t, C.c_float
@@ -65,6 +66,7 @@ SIGNATURES = {
     "mi_conv2d_f16": (_int, [_vp] * 4 + [_i64] * 14 + [_int, _vp, _sz, _vp]),
     "mi_conv2d_f16_workspace": (_sz, [_i64] * 13),
     "mi_conv2d_f16_plan": (_int, [_i64] * 14),
+    "mi_conv2d_f16_kernel": (_int, [_i64] * 14 + [C.POINTER(_sz)]),
     "mi_conv2d_nhwc_f16": (_int, [_vp] * 4 + [_i64] * 13 + [_int, _vp, _sz, _vp]),
     "mi_conv2d_nhwc_f16_workspace": (_sz, [_i64] * 13),
     "mi_conv2d_tokens_f16": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64] + [_i64] * 13 + [_int, _vp, _sz, _vp]),

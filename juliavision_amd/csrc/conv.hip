@@ -221,8 +221,8 @@ int fill(ConvArgs &a, void *out, const void *x, const void *w, const void *bias,
     return MI_OK;
 }
 
-// What the plan calls an implicit GEMM.  (The gathered operand takes any stride and width and channels in multiples of 16
-// now; the names that callers see stay with the extents they were given for.)
+// What the plan calls an implicit GEMM: the reference's extents.  (The gathered operand takes any stride and width and channels in
+// multiples of 16; mi_conv2d_f16_kernel says what runs.)
 bool implicit_ok(const ConvArgs &a) {
     return a.sx == 1 && a.OW % 8 == 0 && a.Cin % 64 == 0 && (long)a.Cin * a.KH * a.KW >= 128;
 }
@@ -249,6 +249,26 @@ void im2col_extents(const ConvArgs &a, int64_t &PQP, int64_t &CRSP) {
     const size_t CRS = (size_t)a.Cin * a.KH * a.KW;
     PQP = round_up((size_t)a.OW * a.OH, 8);
     CRSP = round_up(CRS, CRS >= 256 ? 64 : 8);
+}
+
+// What runs, and the scratch it takes.  In one launch where that is estimated to be faster than staging the operand and multiplying
+// it: im2col writes at 0.8 to 1.1 MB/us, slower where it gathers with a stride (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: 43 us
+// staged, 25 us in one launch); the channels-last copy and the weights of the patch form move at some 2 MB/us behind a launch.
+struct Route { int kernel; size_t scratch; };
+Route route_of(const ConvArgs &a) {
+    if (a.groups != 1) return {MI_CONV_KERNEL_DIRECT, 0};
+    if (onebyone(a)) return {MI_CONV_KERNEL_GEMM_1X1, 0};
+    const int64_t CRS = (int64_t)a.Cin * a.KH * a.KW, PQ = (int64_t)a.OW * a.OH;
+    int64_t PQP, CRSP;
+    im2col_extents(a, PQP, CRSP);
+    const size_t patch_bytes = patch_copy_bytes(a) + patch_weight_bytes(a);
+    const bool patch = patch_ok(a);
+    const double staged = patch ? 4.0 + 0.5e-6 * (double)patch_bytes + mi_internal_patch_gemm_us(a.Cout, CRS, PQ, a.N)
+                                : 3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N);
+    if (mi_conv_tile_us(a) < staged) return {MI_CONV_KERNEL_TILE, 0};
+    if (patch) return {MI_CONV_KERNEL_PATCH_GEMM, patch_bytes};
+    return {MI_CONV_KERNEL_IM2COL_GEMM, round_up((size_t)a.N * PQP * CRSP * 2, 256) + (CRSP != CRS ? round_up((size_t)a.Cout * CRSP * 2, 256) : 0) +
+                                            mi_internal_gemm_workspace(a.Cout, CRSP, PQ, a.N)};
 }
 
 }  // namespace
@@ -286,6 +306,15 @@ size_t mi_conv2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, i
     return need > patch ? need : patch;
 }
 
+int mi_conv2d_f16_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, int64_t KW, int64_t KH, int64_t Cout,
+                         int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy, int64_t groups, size_t *scratch_out) {
+    ConvArgs a;
+    if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, groups, MI_EPI_NONE) != MI_OK) return MI_CONV_KERNEL_NONE;
+    const Route r = route_of(a);
+    if (scratch_out) *scratch_out = r.scratch;
+    return r.kernel;
+}
+
 int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
                   int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, int64_t KW, int64_t KH, int64_t Cout,
                   int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy, int64_t groups, int act,
@@ -297,37 +326,25 @@ int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
     if (rc != MI_OK) return rc;
     if (N == 0) return MI_OK;
     hipStream_t st = (hipStream_t)stream;
-    const int path = conv_path(a);
-    const int PQ = a.OW * a.OH;
+    const Route r = route_of(a);
+    const int PQ = a.OW * a.OH, CRS = a.Cin * a.KH * a.KW;
     const int epi = a.relu ? MI_EPI_RELU : MI_EPI_NONE;
-    if (path == MI_CONV_DIRECT) {
+    if (r.kernel == MI_CONV_KERNEL_DIRECT) {
         long total = (long)a.N * a.Cout * PQ;
         hipLaunchKernelGGL(conv_direct_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, a);
         return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
     }
-    if (path == MI_CONV_GEMM_1X1) {
+    if (r.kernel == MI_CONV_KERNEL_GEMM_1X1) {
         // out[n][Cout][PQ] = w[Cout][Cin] . x[n][Cin][PQ]; the [K][N] operand needs
         // PQ % 8 == 0 for 16-byte loads, otherwise the scalar GEMM takes it.
         return mi_internal_gemm(out, w, x, bias, a.Cout, PQ, PQ, a.Cin, PQ, a.Cin, PQ, 1, MI_BIAS_ROW, epi, 0,
                                 a.N, (long)a.Cout * PQ, 0, (long)a.Cin * PQ, nullptr, 0, st);
     }
-    // In one launch where that is estimated to be faster than staging the operand and multiplying it: im2col writes at 0.8 to
-    // 1.1 MB/us, slower where it gathers with a stride (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: 43 us staged,
-    // 25 us in one launch); the channels-last copy and the weights of the patch form move at some 2 MB/us behind a launch.
-    const int CRS = a.Cin * a.KH * a.KW;
-    const bool patch = patch_ok(a);
-    {
-        int64_t PQP, CRSP;
-        im2col_extents(a, PQP, CRSP);
-        const double staged = patch ? 4.0 + 0.5e-6 * (double)(patch_copy_bytes(a) + patch_weight_bytes(a)) + mi_internal_patch_gemm_us(a.Cout, CRS, PQ, a.N)
-                                    : 3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N);
-        rc = mi_conv_tile(a, staged, st);
-        if (rc != MI_DECLINE_EXTENT) return rc;
-    }
-    if (patch) {
+    if (r.kernel == MI_CONV_KERNEL_TILE) return mi_conv_tile(a, st);
+    if (!ws || ws_bytes < r.scratch || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
+    if (r.kernel == MI_CONV_KERNEL_PATCH_GEMM) {
         const int Hp = a.Hi + 2 * a.py, Wp = a.Wi + 2 * a.px;
         const size_t xp_bytes = patch_copy_bytes(a);
-        if (!ws || ws_bytes < xp_bytes + patch_weight_bytes(a) || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
         half_t *xp = reinterpret_cast<half_t *>(ws);
         half_t *w2 = reinterpret_cast<half_t *>(reinterpret_cast<char *>(ws) + xp_bytes);
         const int pad_blocks = (int)(ceil_div(a.Cin, 64) * ceil_div(a.Wi, 64) * Hp), w_blocks = (int)(a.Cout * ceil_div(a.Cin, turn_group(a)));
@@ -345,7 +362,6 @@ int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
     size_t col_bytes = round_up((size_t)N * PQP * CRSP * 2, 256);
     size_t wp_bytes = CRSP != CRS ? round_up((size_t)Cout * CRSP * 2, 256) : 0;
     const size_t gemm_bytes = mi_internal_gemm_workspace(Cout, CRSP, PQ, N);
-    if (!ws || ws_bytes < col_bytes + wp_bytes + gemm_bytes || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
     if (PQP * CRSP > INT32_MAX) return MI_DECLINE_EXTENT;
     half_t *col = reinterpret_cast<half_t *>(ws);
     const half_t *wuse = a.w;

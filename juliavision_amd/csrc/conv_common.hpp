@@ -8,7 +8,8 @@ struct ConvArgs : ConvShape {
     void *out;
 };
 
-// conv_tile.hip: the one-launch implicit GEMM over channel-first maps, one group.  MI_DECLINE_EXTENT (nothing enqueued)
-// where its own estimate is not below limit_us, or where a chunk of one channel does not fit the LDS.
-int mi_conv_tile(const ConvArgs &a, double limit_us, hipStream_t st);
+// conv_tile.hip: the one-launch implicit GEMM over channel-first maps, one group.  Its own estimate, 1e30 where a chunk of one
+// channel does not fit the LDS; the launch, MI_DECLINE_EXTENT (nothing enqueued) in that case.
+double mi_conv_tile_us(const ConvArgs &a);
+int mi_conv_tile(const ConvArgs &a, hipStream_t st);
 int mi_conv_tile_init();

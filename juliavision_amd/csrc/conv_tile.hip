@@ -304,20 +304,27 @@ int with_shape(const Shape &s, F f) {
     return MI_DECLINE_EXTENT;
 }
 
-}  // namespace
-
-int mi_conv_tile(const ConvArgs &a, double limit_us, hipStream_t st) {
-    // the last choices of this thread: an estimate of every shape takes the host a few microseconds
-    struct Entry { int cus; ConvShape key; double us; Shape s; TilePlan t; };
-    static thread_local Entry table[16] = {};
+// The last choices of this thread: an estimate of every shape takes the host a few microseconds.
+struct Choice { int cus; ConvShape key; double us; Shape s; TilePlan t; };
+const Choice &choice_of(const ConvArgs &a) {
+    static thread_local Choice table[16] = {};
     const int cus = mi_num_cus();
-    Entry &e = table[shape_hash(a, cus) >> 28];
+    Choice &e = table[shape_hash(a, cus) >> 28];
     if (e.cus != cus || !same_shape(e.key, a)) {
         e.cus = cus;
         e.key = a;
         if (!choose(a, cus, e.t, e.s, e.us)) e.us = 1e30;
     }
-    if (e.us >= limit_us) return MI_DECLINE_EXTENT;
+    return e;
+}
+
+}  // namespace
+
+double mi_conv_tile_us(const ConvArgs &a) { return choice_of(a).us; }
+
+int mi_conv_tile(const ConvArgs &a, hipStream_t st) {
+    const Choice &e = choice_of(a);
+    if (e.us >= 1e30) return MI_DECLINE_EXTENT;
     const TileConv t{e.t, a};
     return with_shape(e.s, [&](auto P, auto K, auto T) { return launch<P, K, T>(t, st); });
 }

@@ -363,7 +363,8 @@ PyObject *convolution(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     const int64_t groups = PyLong_AsLongLong(a[8]), N = x->size(0), Cin = x->size(1), Hi = x->size(2), Wi = x->size(3), Cout = w->size(0), KH = w->size(2), KW = w->size(3);
     if (groups < 1 || w->size(1) * groups != Cin || s[0] < 1 || s[1] < 1 || x->numel() < 1 || out->numel() < 1 || !vec_ok(bias, Cout)) NO;
     if (!shape_is(*out, N, Cout, conv_extent(Hi, KH, s[1], p[1], d[1]), conv_extent(Wi, KW, s[0], p[0], d[0])) || !env_of(a[0], e)) NO;
-    const size_t need = mi_conv2d_f16_workspace(Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1]);
+    size_t need = 0;
+    if (mi_conv2d_f16_kernel(Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], groups, &need) == MI_CONV_KERNEL_NONE) NO;
     if (!scratch(e, need, ws)) return nullptr;
     return answer(mi_conv2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], groups, act, ws, need, e.stream));
 }

@@ -773,9 +773,11 @@ def sdpa_append(ctx: Ctx, q, cache_k, cache_v, k_new, v_new, kv_len, scale=None,
 
 @dataclass(frozen=True)
 class ConvGemmPlan:
-    """1x1 or im2col + MFMA GEMM (the counterpart of ConvCoopMatPlan, kernelplans.jl:405-410)."""
+    """A convolution as a GEMM (the counterpart of ConvCoopMatPlan, kernelplans.jl:405-410).  ``path``: the formulation that the
+    extents are given to; ``kernel``: what runs on this device (``L.CONV_KERNELS``), and ``workspace`` the bytes that takes."""
     path: str
     workspace: int
+    kernel: str = field(default="", compare=False)
 
 
 def convsize(n, k, s, p, d) -> int:
@@ -798,7 +800,9 @@ def conv_plan(dev: DeviceCaps, out, x, w, stride=(1, 1), padding=(0, 0), dilatio
     path = lib.mi_conv2d_f16_plan(*args, groups)
     if path == 0:
         return Decline("extent")
-    return ConvGemmPlan(L.CONV_PATHS[path], int(lib.mi_conv2d_f16_workspace(*args)))
+    need = C.c_size_t(0)
+    runs = lib.mi_conv2d_f16_kernel(*args, groups, C.byref(need))
+    return ConvGemmPlan(L.CONV_PATHS[path], int(need.value), L.CONV_KERNELS[runs])
 
 
 def convolution_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, groups, *, act="none"):

@@ -47,3 +47,20 @@ def test_what_the_tiles_do_not_take():
     assert _sdpa(72, 23, 300, 8, 2)[1] == "tiles_f32" and _sdpa(72, 23, 300, 8, 2, f32=True)[1] == "rows"
     assert _sdpa(64, 23, 300, 8, 2, mask="key")[1] == "tiles_f32" and _sdpa(64, 23, 300, 8, 2, mask="key32")[1] == "rows"
     assert _sdpa(64, 1, 1500, 20, 1)[1:] == ("one_query", 4, 4)
+
+
+def test_the_workspace_covers_whichever_convolution_kernel_runs():
+    import random
+    rng, lib, seen = random.Random(0), L.load(), set()
+    for i in range(4000):
+        k, groups = rng.choice([1, 3, 3, 5, 7, 26]), rng.choice([1, 1, 1, 4])
+        cin, cout = (rng.choice([1, 3, 16, 32, 64, 70, 96, 128, 256]) * groups, rng.choice([1, 6, 32, 64, 96, 256]) * groups)
+        w, h, s, p = rng.randint(1, 200), rng.randint(1, 200), rng.choice([1, 1, 2, 4]), rng.choice([0, k // 2])
+        args = (w, h, cin, rng.choice([1, 2]), k, k, cout, s, s, p, p, 1, 1)
+        need = C.c_size_t(0)
+        kernel = L.CONV_KERNELS[lib.mi_conv2d_f16_kernel(*args, groups, C.byref(need))]
+        path = L.CONV_PATHS[lib.mi_conv2d_f16_plan(*args, groups)]
+        assert (kernel == "none") == (path == "decline") and (kernel == "direct") == (path == "direct") and (kernel == "gemm_1x1") == (path == "gemm_1x1")
+        assert need.value <= lib.mi_conv2d_f16_workspace(*args), args
+        seen.add(kernel)
+    assert seen == set(L.CONV_KERNELS.values())
