@@ -290,13 +290,15 @@ size_t mi_conv2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, i
     ConvArgs a;
     if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, 1, MI_EPI_NONE) != MI_OK) return 0;
     if (a.groups != 1 || onebyone(a)) return 0;
-    // what the route needs, and never less than the answers that callers' buffers are sized by: two padded copies with rows of
-    // whole 16 bytes and planes for an implicit GEMM's extents, the im2col matrix for the others
+    // Whichever kernel runs, on any device, and never less than what callers have sized their buffers by: for an implicit GEMM's
+    // extents two padded copies with rows of whole 16 bytes and, from 4096 deep on, two fp32 planes of the result; the im2col
+    // matrix for the others.  (mi_conv2d_f16_kernel tells what the running device's choice takes.)
     const size_t patch = patch_ok(a) ? patch_copy_bytes(a) + patch_weight_bytes(a) : 0;
     size_t need;
     if (patch && implicit_ok(a)) {
         const size_t Wp = round_up((size_t)(a.Wi + 2 * a.px), 8);
-        need = 2 * round_up((size_t)N * Cin * (a.Hi + 2 * a.py) * Wp * 2, 256) + patch_weight_bytes(a) + mi_internal_gemm_workspace(Cout, Cin * KH * KW, (int64_t)a.OW * a.OH, N);
+        need = 2 * round_up((size_t)N * Cin * (a.Hi + 2 * a.py) * Wp * 2, 256) + patch_weight_bytes(a) +
+               (Cin * KH * KW >= 4096 ? 2 * (size_t)N * Cout * a.OW * a.OH * 4 : 0);
     } else {
         int64_t PQP, CRSP;
         im2col_extents(a, PQP, CRSP);
