@@ -219,8 +219,9 @@ size_t mi_convtranspose2d_f16_workspace(int64_t Wi, int64_t Hi, int64_t Cin, int
                                         int64_t opx, int64_t opy, int64_t groups) {
     CtArgs a;
     if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, opx, opy, groups) != MI_OK) return 0;
-    // Both routes work in registers and LDS today.  The answer stays what a weight transpose, an expanded bias and an
-    // unshuffled result take, so that callers' buffers and recorded plans keep their sizes; nothing is written there.
+    if (!shuffle_ok(a, opx, opy)) return 0;
+    // Nothing is written there: both kernels work in registers and LDS.  The answer stays what a weight transpose, an expanded
+    // bias and an unshuffled result would take, which callers have sized their buffers by.
     const int64_t M = (int64_t)a.Cout * a.KH * a.KW, HW = (int64_t)a.Hi * a.Wi;
     return round_up((size_t)M * a.Cin * 2, 256) + round_up((size_t)M * 2, 256) + round_up((size_t)a.N * M * HW * 2, 256) +
            mi_internal_gemm_workspace(M, a.Cin, HW, a.N);

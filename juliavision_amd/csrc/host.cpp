@@ -373,7 +373,6 @@ PyObject *convolution(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
 PyObject *convolutiontranspose(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     ARITY(10)
     Env e;
-    void *ws;
     const Tensor *out = tensor(a[1]), *x = tensor(a[2]), *w = tensor(a[3]), *bias;
     int64_t s[2], p[2], d[2], o[2];
     if (!plain4(out) || !plain4(x) || !plain4(w) || !optional(a[4], bias) || !pair(a[5], s) || !pair(a[6], p) || !pair(a[7], d) || !pair(a[8], o) ||
@@ -383,10 +382,8 @@ PyObject *convolutiontranspose(PyObject *, PyObject *const *a, Py_ssize_t nargs)
     const auto extent = [](int64_t n, int64_t k, int64_t st, int64_t pd, int64_t dl, int64_t op) { return (n - 1) * st - 2 * pd + dl * (k - 1) + op + 1; };
     if (groups < 1 || w->size(0) != Cin || x->numel() < 1 || out->numel() < 1 || !vec_ok(bias, Cout)) NO;
     if (!shape_is(*out, N, Cout, extent(Hi, KH, s[1], p[1], d[1], o[1]), extent(Wi, KW, s[0], p[0], d[0], o[0])) || !env_of(a[0], e)) NO;
-    const size_t need = mi_convtranspose2d_f16_workspace(Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], o[0], o[1], groups);
-    if (!scratch(e, need, ws)) return nullptr;
     return answer(mi_convtranspose2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], o[0], o[1], groups,
-                                         ws, need, e.stream));
+                                         nullptr, 0, e.stream));
 }
 
 // ------------------------------------------------------------------------------------------ recorded calls

@@ -906,7 +906,7 @@ def convtranspose_plan(dev: DeviceCaps, out, x, w, stride=(1, 1), padding=(0, 0)
     path = lib.mi_convtranspose2d_f16_plan(*args)
     if path == 0:
         return Decline("extent")
-    return ConvGemmPlan(L.CONVT_PATHS[path], int(lib.mi_convtranspose2d_f16_workspace(*args)))
+    return ConvGemmPlan(L.CONVT_PATHS[path], 0, L.CONVT_PATHS[path])      # neither kernel uses scratch
 
 
 def convolutiontranspose_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, outpad, groups):
@@ -926,10 +926,9 @@ def convolutiontranspose_(ctx: Ctx, out, x, w, bias, stride, padding, dilation, 
     OH = convtransposesize(Hi, KH, stride[1], padding[1], dilation[1], outpad[1])
     if tuple(out.shape) != (N, Cout, OH, OW) or not out.is_contiguous() or out.dtype != torch.float16:
         raise DeclineError("convolutiontranspose_: out must be dense fp16 (N,Cout,OH,OW)", L.DECLINE_OPERANDS)
-    ws = ctx.ws.scratch(plan.workspace)
     rc = lib.mi_convtranspose2d_f16(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout,
                                     stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1],
-                                    outpad[0], outpad[1], groups, ws, plan.workspace, ctx.stream)
+                                    outpad[0], outpad[1], groups, None, 0, ctx.stream)
     if rc != L.OK:
         raise DeclineError("mi_convtranspose2d_f16", rc)
     return out
