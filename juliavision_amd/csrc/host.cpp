@@ -523,9 +523,24 @@ PyObject *setup(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     Py_RETURN_NONE;
 }
 
-#define M(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {M(setup), M(matmul), M(matmul_rowstats), M(lnfold_matmul), M(ln_matmul), M(layernorm), M(rowstats), M(add), M(sdpa), M(sdpa_append),
-                         M(convolution), M(convolutiontranspose), M(calls_new), M(calls_run), {nullptr, nullptr, 0, nullptr}};
+// What torch throws -- an operand without storage, a device that is gone -- ends here: nothing has been enqueued by then (a call
+// into the library is the last thing a function does and throws nothing), so the answer is the one that sends the caller to
+// the Python form, which meets the same trouble as a Python exception.
+typedef PyObject *(*Fast)(PyObject *, PyObject *const *, Py_ssize_t);
+template <Fast F, bool TRUTH> PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t nargs) {
+    try {
+        return F(self, a, nargs);
+    } catch (...) {
+        PyErr_Clear();
+        if (TRUTH) Py_RETURN_FALSE;
+        Py_RETURN_NONE;
+    }
+}
+
+#define M(f) {#f, (PyCFunction)(void (*)(void))(Fast)guarded<f, true>, METH_FASTCALL, nullptr}
+#define M_NONE(f) {#f, (PyCFunction)(void (*)(void))(Fast)guarded<f, false>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {M_NONE(setup), M(matmul), M(matmul_rowstats), M(lnfold_matmul), M(ln_matmul), M(layernorm), M(rowstats), M(add), M(sdpa), M(sdpa_append),
+                         M(convolution), M(convolutiontranspose), M_NONE(calls_new), M(calls_run), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
