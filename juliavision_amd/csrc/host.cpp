@@ -149,7 +149,16 @@ bool scratch(const Env &e, size_t need, void *&p) {
     return !PyErr_Occurred();
 }
 
-PyObject *answer(int rc) { return PyBool_FromLong(rc == MI_OK); }
+// A call into the library, with the GIL released as ctypes does: a launch may wait for room in the device's queue.
+struct Released {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+};
+template <typename F> int without_gil(F f) {
+    Released r;
+    return f();
+}
+#define ANSWER(call) return PyBool_FromLong(without_gil([&] { return call; }) == MI_OK)
 #define NO Py_RETURN_FALSE
 #define ARITY(n) if (nargs != (n)) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; }
 
@@ -193,7 +202,7 @@ PyObject *matmul(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     void *ws;
     if (!linear_of(l, a[1], a[2], a[3], a[4], a[5], a[6]) || !env_of(a[0], e)) NO;
     if (!scratch(e, l.need, ws)) return nullptr;
-    return answer(mi_gemm_f16(ptr(l.out), ptr(l.B), ptr(l.A), ptr(l.bias), ptr(l.res), l.T, l.K, l.F, l.lo.ld, l.lb.ld, l.la.ld, l.layout,
+    ANSWER(mi_gemm_f16(ptr(l.out), ptr(l.B), ptr(l.A), ptr(l.bias), ptr(l.res), l.T, l.K, l.F, l.lo.ld, l.lb.ld, l.la.ld, l.layout,
                               l.bias_mode, l.epi, l.out_code, ws, l.need, e.stream));
 }
 
@@ -208,7 +217,7 @@ PyObject *matmul_rowstats(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     if (!linear_of(l, a[1], a[3], a[4], a[5], a[6], a[7]) || l.T <= 8 || !dense(*l.out) || !stats_ok(stats, l.F, l.T) ||
         (a[8] != Py_None && !number(a[8], clamp)) || !env_of(a[0], e)) NO;
     if (!scratch(e, l.need, ws)) return nullptr;
-    return answer(mi_gemm_rowstats_f16(ptr(l.out), (float *)ptr(stats), ptr(l.B), ptr(l.A), ptr(l.bias), ptr(l.res), (float)clamp, l.T, l.K, l.F,
+    ANSWER(mi_gemm_rowstats_f16(ptr(l.out), (float *)ptr(stats), ptr(l.B), ptr(l.A), ptr(l.bias), ptr(l.res), (float)clamp, l.T, l.K, l.F,
                                        l.lb.ld, l.la.ld, l.layout, l.bias_mode, l.epi, ws, l.need, e.stream));
 }
 
@@ -227,7 +236,7 @@ PyObject *lnfold_matmul(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     const int64_t Fp = l.F / P, sW = l.layout == MI_W_KF ? Fp : Fp * l.la.ld;
     const size_t need = P == 1 ? l.need : mi_gemm_f16_workspace(l.T, l.K, Fp, l.layout, P);
     if (!scratch(e, need, ws)) return nullptr;
-    return answer(mi_lnfold_gemm_f16(ptr(l.out), (float *)ptr(stats_out), ptr(l.B), (const float *)ptr(stats), (float)eps, ptr(l.A), (const float *)ptr(colsum),
+    ANSWER(mi_lnfold_gemm_f16(ptr(l.out), (float *)ptr(stats_out), ptr(l.B), (const float *)ptr(stats), (float)eps, ptr(l.A), (const float *)ptr(colsum),
                                      (const float *)ptr(biasp), ptr(l.res), (float)clamp, l.T, l.K, Fp, l.lo.ld, l.lb.ld, l.la.ld, l.layout, l.epi, l.out_code,
                                      P, Fp, sW, Fp, ws, need, e.stream));
 }
@@ -243,7 +252,7 @@ PyObject *ln_matmul(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     if (!linear_of(l, a[1], a[2], a[3], a[7], a[8], a[9]) || l.T > 8 || !optional(a[4], g) || !optional(a[5], b) || !vec_ok(g, l.K) || !vec_ok(b, l.K) ||
         (l.bias && l.bias->numel() != l.F) || !number(a[6], eps) || !env_of(a[0], e)) NO;
     if (!scratch(e, l.need, ws)) return nullptr;
-    return answer(mi_ln_gemm_f16(ptr(l.out), ptr(l.B), ptr(g), ptr(b), (float)eps, ptr(l.A), ptr(l.bias), ptr(l.res), l.T, l.K, l.F, l.lo.ld, l.lb.ld, l.la.ld,
+    ANSWER(mi_ln_gemm_f16(ptr(l.out), ptr(l.B), ptr(g), ptr(b), (float)eps, ptr(l.A), ptr(l.bias), ptr(l.res), l.T, l.K, l.F, l.lo.ld, l.lb.ld, l.la.ld,
                                  l.layout, l.bias ? MI_BIAS_COL : MI_BIAS_NONE, l.epi, l.out_code, ws, l.need, e.stream));
 }
 
@@ -258,7 +267,7 @@ PyObject *layernorm(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     if (!is_f16(out) || !is_f16(x) || !out->is_contiguous() || !x->is_contiguous() || out->sizes() != x->sizes() || !PyLong_CheckExact(a[5])) NO;
     const int64_t C = PyLong_AsLongLong(a[5]), n = x->numel();
     if (C < 1 || n % C || !optional(a[3], g) || !optional(a[4], b) || !vec_ok(g, C) || !vec_ok(b, C) || !number(a[6], eps) || !env_of(a[0], e)) NO;
-    return answer(mi_layernorm_f16(ptr(out), nullptr, nullptr, ptr(x), ptr(g), ptr(b), C, n / C, (float)eps, e.stream));
+    ANSWER(mi_layernorm_f16(ptr(out), nullptr, nullptr, ptr(x), ptr(g), ptr(b), C, n / C, (float)eps, e.stream));
 }
 
 // rowstats(ctx, stats, x)
@@ -267,7 +276,7 @@ PyObject *rowstats(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     Env e;
     const Tensor *s = tensor(a[1]), *x = tensor(a[2]);
     if (!is_f16(x) || x->dim() != 2 || x->stride(1) != 1 || !stats_ok(s, x->size(1), x->size(0)) || !env_of(a[0], e)) NO;
-    return answer(mi_rowstats_f16((float *)ptr(s), ptr(x), x->stride(0), x->size(1), x->size(0), e.stream));
+    ANSWER(mi_rowstats_f16((float *)ptr(s), ptr(x), x->stride(0), x->size(1), x->size(0), e.stream));
 }
 
 // add(ctx, out, a, b)
@@ -277,7 +286,7 @@ PyObject *add(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     const Tensor *out = tensor(a[1]), *x = tensor(a[2]), *y = tensor(a[3]);
     if (!is_f16(out) || !is_f16(x) || !is_f16(y) || !out->is_contiguous() || !x->is_contiguous() || !y->is_contiguous() || out->sizes() != x->sizes() ||
         out->sizes() != y->sizes() || !env_of(a[0], e)) NO;
-    return answer(mi_add_f16(ptr(out), ptr(x), ptr(y), x->numel(), e.stream));
+    ANSWER(mi_add_f16(ptr(out), ptr(x), ptr(y), x->numel(), e.stream));
 }
 
 // ------------------------------------------------------------------------------------------ attention
@@ -317,7 +326,7 @@ PyObject *sdpa(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     strides_elbh(*out, os); strides_elbh(*q, qs); strides_elbh(*k, ks); strides_elbh(*v, vs);
     const size_t need = mi_sdpa_f16_workspace(E, Lq, Lk, H, B, bias ? 1 : 0);
     if (!scratch(e, need, ws)) return nullptr;
-    return answer(mi_sdpa_f16(ptr(out), out_code, out->is_contiguous() ? nullptr : os, ptr(q), qs, ptr(k), ks, ptr(v), vs, ptr(bias), bias_code, bias ? bs : nullptr,
+    ANSWER(mi_sdpa_f16(ptr(out), out_code, out->is_contiguous() ? nullptr : os, ptr(q), qs, ptr(k), ks, ptr(v), vs, ptr(bias), bias_code, bias ? bs : nullptr,
                               (const int32_t *)ptr(kv), E, Lq, Lk, H, B, (float)scale, ws, need, e.stream));
 }
 
@@ -338,7 +347,7 @@ PyObject *sdpa_append(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     if (!env_of(a[0], e)) NO;
     int64_t os[4], qs[4], ks[4], vs[4], ns[4];
     strides_elbh(*out, os); strides_elbh(*q, qs); strides_elbh(*ck, ks); strides_elbh(*cv, vs); strides_elbh(*kn, ns);
-    return answer(mi_sdpa_append_f16(ptr(out), out_code, out->is_contiguous() ? nullptr : os, ptr(q), qs, ptr(ck), ks, ptr(cv), vs, ptr(kn), ptr(vn), ns,
+    ANSWER(mi_sdpa_append_f16(ptr(out), out_code, out->is_contiguous() ? nullptr : os, ptr(q), qs, ptr(ck), ks, ptr(cv), vs, ptr(kn), ptr(vn), ns,
                                      (const int32_t *)ptr(kv), E, Lk, H, B, (float)scale, e.stream));
 }
 
@@ -366,7 +375,7 @@ PyObject *convolution(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     size_t need = 0;
     if (mi_conv2d_f16_kernel(Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], groups, &need) == MI_CONV_KERNEL_NONE) NO;
     if (!scratch(e, need, ws)) return nullptr;
-    return answer(mi_conv2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], groups, act, ws, need, e.stream));
+    ANSWER(mi_conv2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], groups, act, ws, need, e.stream));
 }
 
 // convolutiontranspose(ctx, out, x, w, bias, stride, padding, dilation, outpad, groups)
@@ -382,7 +391,7 @@ PyObject *convolutiontranspose(PyObject *, PyObject *const *a, Py_ssize_t nargs)
     const auto extent = [](int64_t n, int64_t k, int64_t st, int64_t pd, int64_t dl, int64_t op) { return (n - 1) * st - 2 * pd + dl * (k - 1) + op + 1; };
     if (groups < 1 || w->size(0) != Cin || x->numel() < 1 || out->numel() < 1 || !vec_ok(bias, Cout)) NO;
     if (!shape_is(*out, N, Cout, extent(Hi, KH, s[1], p[1], d[1], o[1]), extent(Wi, KW, s[0], p[0], d[0], o[0])) || !env_of(a[0], e)) NO;
-    return answer(mi_convtranspose2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], o[0], o[1], groups,
+    ANSWER(mi_convtranspose2d_f16(ptr(out), ptr(x), ptr(w), ptr(bias), Wi, Hi, Cin, N, KW, KH, Cout, s[0], s[1], p[0], p[1], d[0], d[1], o[0], o[1], groups,
                                          nullptr, 0, e.stream));
 }
 
@@ -391,7 +400,7 @@ PyObject *convolutiontranspose(PyObject *, PyObject *const *a, Py_ssize_t nargs)
 // A C-ABI call with its arguments in 8-byte slots; `fours` keeps the stride arrays that slots point to.
 constexpr int MAX_ARGS = 32;
 struct Call;
-typedef int (*Invoke)(const Call &);
+typedef int (*Invoke)(const uint64_t *);
 struct Call {
     Invoke invoke;
     int nargs;
@@ -431,8 +440,8 @@ template <auto Fn> struct Bound;
 template <typename... A, int (*Fn)(A...)> struct Bound<Fn> {
     static constexpr int N = sizeof...(A);
     static_assert(N <= MAX_ARGS, "more arguments than a recorded call holds");
-    template <size_t... I> static int go(const Call &c, std::index_sequence<I...>) { return Fn(arg_of<A>(c.slot[I])...); }
-    static int invoke(const Call &c) { return go(c, std::index_sequence_for<A...>{}); }
+    template <size_t... I> static int go(const uint64_t *s, std::index_sequence<I...>) { return Fn(arg_of<A>(s[I])...); }
+    static int invoke(const uint64_t *s) { return go(s, std::index_sequence_for<A...>{}); }
     template <size_t... I> static bool fill_(Call &c, PyObject *args, std::index_sequence<I...>) {
         return (slot_of<A>(PyTuple_GET_ITEM(args, I), c.slot[I], c) && ...);
     }
@@ -454,7 +463,7 @@ const std::unordered_map<std::string, Entry> &recordable() {          // every c
 #undef R
     return table;
 }
-struct Patch { int call, slot, input; int64_t offset; };
+struct Patch { int call, slot, input; int64_t offset; };         // sorted by call
 struct CallList {
     std::vector<Call> calls;
     std::vector<Patch> patches;
@@ -497,20 +506,31 @@ PyObject *calls_new(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
 // calls_run(ctx, capsule, inputs tuple) -> True, False (the context is not one this file takes), or the status of the call that was refused
 PyObject *calls_run(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     ARITY(3)
-    CallList *list = static_cast<CallList *>(PyCapsule_GetPointer(a[1], "mi_calls"));
+    const CallList *list = static_cast<CallList *>(PyCapsule_GetPointer(a[1], "mi_calls"));
     if (!list) return nullptr;
     Env e;
     if (!env_of(a[0], e)) NO;
-    for (const Patch &p : list->patches) {
-        const Tensor *t = tensor(PyTuple_GetItem(a[2], p.input));
+    // the addresses first: the list itself stays as it was recorded, so that threads may run it at once
+    std::vector<uint64_t> base;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[2]); i++) {
+        const Tensor *t = tensor(PyTuple_GET_ITEM(a[2], i));
         if (!t) NO;
-        list->calls[p.call].slot[p.slot] = (uint64_t)((uintptr_t)t->data_ptr() + p.offset);
+        base.push_back((uint64_t)(uintptr_t)t->data_ptr());
     }
-    for (Call &c : list->calls) {
-        c.slot[c.nargs - 1] = (uint64_t)(uintptr_t)e.stream;
-        const int rc = c.invoke(c);
-        if (rc != MI_OK) return PyLong_FromLong(rc);
-    }
+    const int rc = without_gil([&] {
+        auto patch = list->patches.begin();                 // in the order of the calls
+        for (size_t i = 0; i < list->calls.size(); i++) {
+            const Call &c = list->calls[i];
+            uint64_t slot[MAX_ARGS];
+            std::memcpy(slot, c.slot, sizeof(uint64_t) * c.nargs);
+            for (; patch != list->patches.end() && patch->call == (int)i; ++patch) slot[patch->slot] = base[patch->input] + patch->offset;
+            slot[c.nargs - 1] = (uint64_t)(uintptr_t)e.stream;
+            const int r = c.invoke(slot);
+            if (r != MI_OK) return r;
+        }
+        return (int)MI_OK;
+    });
+    if (rc != MI_OK) return PyLong_FromLong(rc);
     Py_RETURN_TRUE;
 }
 

@@ -116,6 +116,30 @@ def test_calls_that_are_not_noted_are_not_noted_again(why, monkeypatch):
         assert run._calls is not None and len(made) == 1
 
 
+def test_threads_issue_calls_at_once():
+    import threading
+    import juliavision_amd as jv
+    torch.manual_seed(0)
+    w, xs = torch.randn(256, 512, device="cuda").half(), [torch.randn(40, 256, device="cuda").half() for _ in range(4)]
+    want = [jv.matmul_(jv.Ctx("cuda"), torch.empty(40, 512, dtype=torch.float16, device="cuda"), w, x).clone() for x in xs]
+    bad = []
+
+    def work(i):
+        ctx, out = jv.Ctx("cuda"), torch.empty(40, 512, dtype=torch.float16, device="cuda")
+        for _ in range(50):
+            ctx.ws.reset()
+            jv.matmul_(ctx, out, w, xs[i])
+        torch.cuda.synchronize()
+        if not torch.equal(out, want[i]):
+            bad.append(i)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
 def test_what_the_native_side_leaves_is_still_refused_by_name():
     import juliavision_amd as jv
     ctx = jv.Ctx("cuda")
