@@ -28,6 +28,7 @@ using at::Tensor;
 
 PyObject *s_dev, *s_own, *s_ws, *s_device, *s_buf, *s_off, *s_scratch;
 PyObject *g_workspace_type = nullptr;              // kernels.Workspace: its scratch() is done in here while it need not grow
+PyObject *g_ctx_type = nullptr;                    // kernels.Ctx: a subclass may have a stream or a library of its own and goes the long way
 
 // ------------------------------------------------------------------------------------------ operands
 
@@ -101,6 +102,7 @@ struct Env {
     ~Env() { Py_XDECREF(ws); }
 };
 bool env_of(PyObject *ctx, Env &e) {
+    if ((PyObject *)Py_TYPE(ctx) != g_ctx_type) return false;
     PyObject *own = PyObject_GetAttr(ctx, s_own), *dev = own ? PyObject_GetAttr(ctx, s_dev) : nullptr;
     const bool mine = own && dev && own == dev && own != Py_None;
     Py_XDECREF(own);
@@ -534,12 +536,15 @@ PyObject *calls_run(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     Py_RETURN_TRUE;
 }
 
-// setup(Workspace type)
+// setup(Workspace type, Ctx type)
 PyObject *setup(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    ARITY(1)
+    ARITY(2)
     Py_INCREF(a[0]);
+    Py_INCREF(a[1]);
     Py_XDECREF(g_workspace_type);
+    Py_XDECREF(g_ctx_type);
     g_workspace_type = a[0];
+    g_ctx_type = a[1];
     Py_RETURN_NONE;
 }
 

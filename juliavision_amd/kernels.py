@@ -157,7 +157,7 @@ class Ctx:
         self.lib = L.init()
         if _fast is None:
             host = L.load_host()
-            host.setup(Workspace)
+            host.setup(Workspace, Ctx)
             _fast = host
         self.device = torch.device(device)
         self.dev = dev if dev is not None else caps()

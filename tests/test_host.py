@@ -25,7 +25,7 @@ import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 from juliavision_amd import _lib as L, kernels as K
 host = L.load_host()
-host.setup(K.Workspace)
+host.setup(K.Workspace, K.Ctx)
 ctx = object.__new__(K.Ctx)
 ctx.dev = ctx._own = K.MI355X
 ctx.device, ctx.ws = torch.device("cuda"), None

@@ -116,6 +116,24 @@ def test_calls_that_are_not_noted_are_not_noted_again(why, monkeypatch):
         assert run._calls is not None and len(made) == 1
 
 
+def test_a_subclass_of_the_context_keeps_its_stream():
+    import juliavision_amd as jv
+    side = torch.cuda.Stream()
+    asked = []
+
+    class Mine(jv.Ctx):
+        @property
+        def stream(self):
+            asked.append(1)
+            return side.cuda_stream
+    ctx = Mine("cuda")
+    x = torch.randn(16, 64, device="cuda").half()
+    side.wait_stream(torch.cuda.current_stream())
+    out = jv.add_(ctx, torch.empty_like(x), x, x)
+    torch.cuda.synchronize()
+    assert asked and torch.equal(out, x + x)
+
+
 def test_threads_issue_calls_at_once():
     import threading
     import juliavision_amd as jv
