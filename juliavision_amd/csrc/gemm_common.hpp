@@ -67,88 +67,6 @@ struct GemmArgs {
 
 namespace {
 
-
-// ------------------------------------------------------------------------------------------
-// Staging of a K-contiguous operand tile ROWS x BK: each thread moves 16-byte
-// chunks global -> registers -> LDS rows of BK+8 halves (the 16-byte pad makes
-// the 32 rows an MFMA operand read touches fall in distinct bank groups).
-template <int ROWS, int BK, int NT>
-struct KcStage {
-    static constexpr int CPR = BK / 8;
-    static constexpr int CHUNKS = ROWS * CPR;
-    static constexpr int PER = (CHUNKS + NT - 1) / NT;
-    static constexpr int LD = BK + 8;
-    u32x4 r[PER];
-
-    __device__ __forceinline__ void load(const half_t *base, long ld, int row0, int nrows, int k0, int K, int tid) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int c = tid + i * NT;
-            int row = c / CPR, kc = c % CPR;
-            int gr = min(row0 + row, nrows - 1);
-            int gk = k0 + kc * 8;
-            u32x4 z = {0u, 0u, 0u, 0u};
-            if (CHUNKS % NT == 0 || c < CHUNKS) r[i] = gk < K ? ldg16(base + (long)gr * ld + gk) : z;
-        }
-    }
-    __device__ __forceinline__ void store(half_t *lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int c = tid + i * NT;
-            int row = c / CPR, kc = c % CPR;
-            if (CHUNKS % NT == 0 || c < CHUNKS) *reinterpret_cast<u32x4 *>(lds + row * LD + kc * 8) = r[i];
-        }
-    }
-};
-
-// Staging of an N-contiguous operand tile [BK][COLS] into the same K-contiguous
-// LDS rows: a thread loads an 8(k) x 8(n) block with eight 16-byte row loads,
-// transposes it in registers (v_perm_b32) and writes eight 16-byte LDS rows.
-template <int COLS, int BK, int NT>
-struct KnStage {
-    static constexpr int KB = BK / 8;
-    static constexpr int BLOCKS = KB * (COLS / 8);
-    static constexpr int PER = (BLOCKS + NT - 1) / NT;
-    static constexpr int LD = BK + 8;
-    u32x4 r[PER][8];
-
-    __device__ __forceinline__ void load(const half_t *base, long ld, int col0, int ncols, int k0, int K, int tid) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int blk = tid + i * NT;
-            int kb = blk % KB, nb = blk / KB;
-            int gn = min(col0 + nb * 8, ncols - 8);
-            if (BLOCKS % NT == 0 || blk < BLOCKS) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    int gk = k0 + kb * 8 + j;
-                    u32x4 z = {0u, 0u, 0u, 0u};
-                    r[i][j] = gk < K ? ldg16(base + (long)gk * ld + gn) : z;
-                }
-            }
-        }
-    }
-    __device__ __forceinline__ void store(half_t *lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            int blk = tid + i * NT;
-            int kb = blk % KB, nb = blk / KB;
-            if (BLOCKS % NT == 0 || blk < BLOCKS) {
-#pragma unroll
-                for (int w = 0; w < 4; w++) {   // dword w of each row holds columns 2w, 2w+1
-                    u32x4 lo, hi;
-                    lo.x = pack_lo(r[i][0][w], r[i][1][w]); hi.x = pack_hi(r[i][0][w], r[i][1][w]);
-                    lo.y = pack_lo(r[i][2][w], r[i][3][w]); hi.y = pack_hi(r[i][2][w], r[i][3][w]);
-                    lo.z = pack_lo(r[i][4][w], r[i][5][w]); hi.z = pack_hi(r[i][4][w], r[i][5][w]);
-                    lo.w = pack_lo(r[i][6][w], r[i][7][w]); hi.w = pack_hi(r[i][6][w], r[i][7][w]);
-                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w) * LD + kb * 8) = lo;
-                    *reinterpret_cast<u32x4 *>(lds + (nb * 8 + 2 * w + 1) * LD + kb * 8) = hi;
-                }
-            }
-        }
-    }
-};
-
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F &&f) {
     if constexpr (N > 0) {

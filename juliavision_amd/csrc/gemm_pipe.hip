@@ -331,9 +331,8 @@ int raise_pipe() {
     if constexpr (BM * BN <= 128 * 128)
         bad = raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, false, true>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, false, true>, lds);
     return bad | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1>, lds) |
-           raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 2>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 1>, lds) |
-           raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 1>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, true>, lds) |
-           raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, true>, lds);
+           raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 1>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 1>, lds) |
+           raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 0, 0, true>, lds) | raise_lds(gemm_pipe_kernel<BM, BN, WM, WN, 1, 0, true>, lds);
 }
 
 // The pipelined kernel with the layer norm of A's rows as its prologue (AMODE 2): 64-row tiles, 128 <= K <= 512.

@@ -6,9 +6,8 @@ static __device__ __align__(16) unsigned ring_zero_words[4];
 
 namespace {
 
-// A workgroup owns a 64 WM x 64 WN tile; its WM x WN x WK waves each hold a 64 x 64 sub-tile of accumulators, WK of them the
-// same one: wave wk takes 4 / WK of the four 16-deep steps of every 64-deep tile of K, and the WK partial tiles are summed
-// through LDS before the store.
+// A workgroup owns a 64 x 64 tile; each of its four matrix waves holds all of it in accumulators and takes one of the four 16-deep
+// steps of every 64-deep tile of K.  The four partial tiles are summed through LDS before the store.
 //
 // What bounds such a tile is the CU's LDS and vector-memory path, not the matrix cores.  Per 64-deep tile a 64 x 64 tile
 // takes 256 clocks of 64 B/clock loads and 128 clocks of MFMAs; four 32 x 32 waves (gemm_pipe_kernel) move 16 KB into LDS
@@ -23,16 +22,15 @@ namespace {
 //
 // CONV: B is the patch matrix of a convolution (ConvGather).  Its rows' offsets are as fixed as an ordinary operand's; what moves
 // from tile to tile is the tap, for all lanes alike where C is a multiple of 64, by the lane's pair of chunks otherwise.
-template <int WM, int WN, int WK, int S, bool B_KN, bool CONV = false>
-__global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
-    constexpr int BM = 64 * WM, BN = 64 * WN, BK = 64, NW = WM * WN * WK, NT = NW * 64, KS = 4 / WK;
+template <int S, bool B_KN, bool CONV = false>
+__global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
+    constexpr int BM = 64, BN = 64, BK = 64, NW = 4, NT = NW * 64;
     constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
     constexpr int STAGE_BYTES = SLOTS * 1024, A_BYTES = SLOTS_A * 1024;
     static_assert(!(CONV && B_KN), "a patch row is K-contiguous");
     static_assert(S >= 3, "a stage being read, one landed, one on its way");
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wk = wave % WK, wmn = wave / WK, wm = wmn % WM, wn = wmn / WM;
     int tm_, tn_;
     tile_of(p, tm_, tn_);
     const int m0 = __builtin_amdgcn_readfirstlane(tm_ * BM), n0 = __builtin_amdgcn_readfirstlane(tn_ * BN);
@@ -178,39 +176,32 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
         return;
     }
 
-    // fragment addresses: step ks of a tile is step ks of this wave's KS (all four when WK == 1)
+    // fragment addresses of this wave's step of a tile
     const int frow = lane & 31, h = lane >> 5, aswz = (frow & 7) ^ ((frow >> 3) & 1);
-    uint32_t aoff[KS], boff[KS], noff[2];
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-        const int ks = wk * KS + s;
-        aoff[s] = (uint32_t)((wm * 64 + frow) * 128 + (((2 * ks + h) ^ aswz) * 16));
-        if constexpr (!B_KN) boff[s] = (uint32_t)(A_BYTES + (wn * 64 + frow) * 128 + (((2 * ks + h) ^ aswz) * 16));
-        else boff[s] = (uint32_t)(A_BYTES + (ks * 16 + h * 8 + ((lane & 15) >> 2)) * BN * 2);
-    }
+    const uint32_t aoff = (uint32_t)(frow * 128 + (((2 * wave + h) ^ aswz) * 16));
+    uint32_t boff, noff[2];
+    if constexpr (!B_KN) boff = (uint32_t)(A_BYTES + frow * 128 + (((2 * wave + h) ^ aswz) * 16));
+    else boff = (uint32_t)(A_BYTES + (wave * 16 + h * 8 + ((lane & 15) >> 2)) * BN * 2);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const int n = wn * 64 + i * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4, k3 = (lane & 15) >> 2;
+        const int n = i * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4, k3 = (lane & 15) >> 2;
         noff[i] = (uint32_t)((((n >> 3) ^ (k3 * (BN / 32))) * 16) + (n & 7) * 2);
     }
-    half8v fa[2][KS][2], fb[2][KS][2];
+    half8v fa[2][2], fb[2][2];
     auto fetch = [&](auto SET, int kt) {
         constexpr int set = decltype(SET)::value;
         const char *st = smem + (kt % S) * STAGE_BYTES;
 #pragma unroll
-        for (int s = 0; s < KS; s++) {
+        for (int j = 0; j < 2; j++) fa[set][j] = *reinterpret_cast<const half8v *>(st + aoff + j * 32 * 128);
 #pragma unroll
-            for (int j = 0; j < 2; j++) fa[set][s][j] = *reinterpret_cast<const half8v *>(st + aoff[s] + j * 32 * 128);
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                if constexpr (!B_KN) fb[set][s][i] = *reinterpret_cast<const half8v *>(st + boff[s] + i * 32 * 128);
-                else {
-                    const char *b = st + boff[s] + noff[i];
-                    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)b);
-                    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(b + 4 * BN * 2));
-                    const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    fb[set][s][i] = __builtin_bit_cast(half8v, both);
-                }
+        for (int i = 0; i < 2; i++) {
+            if constexpr (!B_KN) fb[set][i] = *reinterpret_cast<const half8v *>(st + boff + i * 32 * 128);
+            else {
+                const char *b = st + boff + noff[i];
+                const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)b);
+                const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(b + 4 * BN * 2));
+                const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                fb[set][i] = __builtin_bit_cast(half8v, both);
             }
         }
     };
@@ -224,18 +215,15 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
     auto products = [&](auto SET) {
         constexpr int set = decltype(SET)::value;
 #pragma unroll
-        for (int s = 0; s < KS; s++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][s][i], fa[set][s][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][i], fa[set][j], acc[i][j], 0, 0, 0);
     };
 
-    // what the store needs of memory, while the first tiles are on their way
-    constexpr int KEEP = WK > 1 ? 4 / WK : 2, STN = WK == 4 ? 32 : 64;       // 32-column blocks a wave stores, columns of its sub-tile
-    const int sm = WK == 1 ? wm : wm * 2 + (WK == 4 ? wk & 1 : wk), sn = WK == 4 ? wn * 2 + (wk >> 1) : wn;
-    half4v cb[KEEP][4];
-    load_col_bias<KEEP, STN>(p, cb, n0, sn, lane, bz);
+    // what the store needs of memory, while the first tiles are on their way: wave w stores the 32 x 32 block (w % 2, w / 2)
+    const int sm = wave & 1, sn = wave >> 1;
+    half4v cb[1][4];
+    load_col_bias<1, 32>(p, cb, n0, sn, lane, bz);
     float2v *ln_slot = reinterpret_cast<float2v *>(smem + S * STAGE_BYTES);
     LnfLoader<BM, BN, NT, 10> lnf;                       // four lanes a row: K <= 1280 in one request
     lnf.request(p, m0, n0, bz, tid);
@@ -262,107 +250,78 @@ __global__ __launch_bounds__(WM *WN *WK * 64 + 128) void gemm_ring_kernel(GemmAr
     lnf.combine(p, ln_slot, m0, tid);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     barrier();                                            // every wave has read its last fragments
-    LnFold<2> ln2;
-    if constexpr (WK > 1) {
-        // wave wk keeps blocks: WK == 4: (i, j) = (wk / 2, wk % 2); WK == 2: j == wk, both i.  Partial tiles go to LDS by
-        // owner and are added in wave order.
-        float *part = reinterpret_cast<float *>(smem) + wmn * WK * (WK - 1) * KEEP * 1024;
+    // Partial tiles go to LDS by owner -- wave w keeps block acc[w / 2][w % 2] -- and are added in wave order.
+    float *part = reinterpret_cast<float *>(smem);
 #pragma unroll
-        for (int o = 0; o < WK; o++) {
-            if (o != wk) {
-                const int from = wk < o ? wk : wk - 1;
+    for (int o = 0; o < NW; o++) {
+        if (o != wave) {
+            const int from = wave < o ? wave : wave - 1;
+            const float16v v = acc[o >> 1][o & 1];
 #pragma unroll
-                for (int b = 0; b < KEEP; b++) {
-                    const float16v v = WK == 4 ? acc[o >> 1][o & 1] : acc[b][o];
-#pragma unroll
-                    for (int r4 = 0; r4 < 4; r4++) {
-                        const float4v q = {v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]};
-                        *reinterpret_cast<float4v *>(part + ((o * (WK - 1) + from) * KEEP + b) * 1024 + r4 * 256 + lane * 4) = q;
-                    }
-                }
+            for (int r4 = 0; r4 < 4; r4++) {
+                const float4v q = {v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]};
+                *reinterpret_cast<float4v *>(part + (o * (NW - 1) + from) * 1024 + r4 * 256 + lane * 4) = q;
             }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        barrier();
-        float16v own[KEEP][1];
-#pragma unroll
-        for (int b = 0; b < KEEP; b++) {
-            float16v mine = acc[0][0];
-#pragma unroll
-            for (int o = 0; o < WK; o++) if (o == wk) mine = WK == 4 ? acc[o >> 1][o & 1] : acc[b][o];
-#pragma unroll
-            for (int r = 0; r < 16; r++) own[b][0][r] = 0.0f;
-#pragma unroll
-            for (int s = 0; s < WK; s++) {
-                if (s == wk) {
-#pragma unroll
-                    for (int r = 0; r < 16; r++) own[b][0][r] += mine[r];
-                } else {
-                    const int from = s < wk ? s : s - 1;
-#pragma unroll
-                    for (int r4 = 0; r4 < 4; r4++) {
-                        const float4v q = *reinterpret_cast<const float4v *>(part + ((wk * (WK - 1) + from) * KEEP + b) * 1024 + r4 * 256 + lane * 4);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) own[b][0][4 * r4 + e] += q[e];
-                    }
-                }
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        barrier();                                        // the store's staging reuses the partial tiles' memory
-        LnFold<1> ln;
-        if (p.lnf_stats) {
-            const float2v v = ln_slot[sm * 32 + frow];
-            ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
-        }
-        store_tile<1, KEEP, 32, STN, NW, S * STAGE_BYTES>(p, own, cb, smem, m0, n0, sm, sn, wave, lane, bz, ln);
-    } else {
-        if (p.lnf_stats) {
-            ln2.on = true; ln2.col = reinterpret_cast<const float *>(ln_slot + BM); ln2.bn = BN;
-#pragma unroll
-            for (int j = 0; j < 2; j++) { const float2v v = ln_slot[wm * 64 + 32 * j + frow]; ln2.r[j] = v[0]; ln2.rmu[j] = v[1]; }
-        }
-        store_tile<2, 2, 64, 64, NW, S * STAGE_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln2);
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();
+    float16v own[1][1], mine = acc[0][0];
+#pragma unroll
+    for (int o = 0; o < NW; o++) if (o == wave) mine = acc[o >> 1][o & 1];
+#pragma unroll
+    for (int r = 0; r < 16; r++) own[0][0][r] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NW; s++) {
+        if (s == wave) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) own[0][0][r] += mine[r];
+        } else {
+            const int from = s < wave ? s : s - 1;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+                const float4v q = *reinterpret_cast<const float4v *>(part + (wave * (NW - 1) + from) * 1024 + r4 * 256 + lane * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) own[0][0][4 * r4 + e] += q[e];
+            }
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();                                            // the store's staging reuses the partial tiles' memory
+    LnFold<1> ln;
+    if (p.lnf_stats) {
+        const float2v v = ln_slot[sm * 32 + frow];
+        ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
+    }
+    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, own, cb, smem, m0, n0, sm, sn, wave, lane, bz, ln);
 }
 
-template <int WM, int WN, int S>
-constexpr int ring_lds_bytes() { return S * (WM + WN) * 8192 + (WM + WN) * 64 * 8; }
+constexpr int ring_lds_bytes(int S) { return S * 2 * 8192 + 2 * 64 * 8; }
 
-template <int WM, int WN, int WK, int S>
-int launch_ring(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    set_tiles(a, 64 * WM, 64 * WN);
-    a.vec_store = rows_vec16(a);
-    // per-lane load offsets are 32-bit byte offsets from the tile's origin
-    if ((int64_t)64 * WM * a.ldA * 2 >= (1ll << 31) || (int64_t)64 * (b_kn ? 1 : WN) * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
-    constexpr int lds = ring_lds_bytes<WM, WN, S>();
-    if (b_kn) hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, WK, S, true>), grid, dim3(WM * WN * WK * 64 + 128), lds, st, a);
-    else      hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, WK, S, false>), grid, dim3(WM * WN * WK * 64 + 128), lds, st, a);
+template <int S, bool B_KN, bool CONV>
+int launch_ring(const GemmArgs &a, int64_t nbatch, hipStream_t st) {
+    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(4 * 64 + 128), ring_lds_bytes(S), st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-}
-template <int WM, int WN, int WK, int S>
-int raise_ring() {
-    return raise_lds(gemm_ring_kernel<WM, WN, WK, S, true>, ring_lds_bytes<WM, WN, S>()) | raise_lds(gemm_ring_kernel<WM, WN, WK, S, false>, ring_lds_bytes<WM, WN, S>());
 }
 
 }  // namespace
 
-int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
-    if (!a.cv.xp) return launch_ring<1, 1, 4, 8>(a, b_kn, nbatch, st);
-    GemmArgs c = a;
-    set_tiles(c, 64, 64);
-    c.vec_store = rows_vec16(c);
-    if (b_kn || (int64_t)64 * c.ldA * 2 >= (1ll << 31) || c.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
-    // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
-    const dim3 grid((unsigned)(c.tiles_m * c.tiles_n), (unsigned)nbatch);
-    constexpr int lds8 = ring_lds_bytes<1, 1, 8>(), lds4 = ring_lds_bytes<1, 1, 4>();
-    if ((int64_t)grid.x * nbatch <= mi_num_cus()) hipLaunchKernelGGL((gemm_ring_kernel<1, 1, 4, 8, false, true>), grid, dim3(4 * 64 + 128), lds8, st, c);
-    else hipLaunchKernelGGL((gemm_ring_kernel<1, 1, 4, 4, false, true>), grid, dim3(4 * 64 + 128), lds4, st, c);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t st) {
+    GemmArgs a = args;
+    set_tiles(a, 64, 64);
+    a.vec_store = rows_vec16(a);
+    // per-lane load offsets are 32-bit byte offsets from the tile's origin (patches: from the image's)
+    if ((int64_t)64 * a.ldA * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+    if (a.cv.xp) {
+        if (b_kn || a.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
+        // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
+        return (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus() ? launch_ring<8, false, true>(a, nbatch, st) : launch_ring<4, false, true>(a, nbatch, st);
+    }
+    if ((int64_t)64 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+    return b_kn ? launch_ring<8, true, false>(a, nbatch, st) : launch_ring<8, false, false>(a, nbatch, st);
 }
 
 int mi_ring_init() {
-    return raise_ring<1, 1, 4, 8>() | raise_lds(gemm_ring_kernel<1, 1, 4, 8, false, true>, ring_lds_bytes<1, 1, 8>()) |
-           raise_lds(gemm_ring_kernel<1, 1, 4, 4, false, true>, ring_lds_bytes<1, 1, 4>());
+    return raise_lds(gemm_ring_kernel<8, true>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<8, false>, ring_lds_bytes(8)) |
+           raise_lds(gemm_ring_kernel<8, false, true>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, false, true>, ring_lds_bytes(4));
 }
