@@ -109,7 +109,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
             uint32_t off = is_k ? koff[i] : voff[i];
             if (over > 0) off -= max(0, s / EC - (31 - over)) * (is_k ? kpitch : vpitch);
             if ((32 * EC) % 64 == 0 || s < 32 * EC)
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(org), "s"(__builtin_amdgcn_readfirstlane(dst + i * 1024)) : "memory");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(org), "s"(F32 ? __builtin_amdgcn_readfirstlane(dst + i * 1024) : dst + i * 1024) : "memory");
         }
     };
     if (wave < nt) { request(true, wave); request(false, wave); }
