@@ -378,18 +378,18 @@ int mi_sdpa_f16_plan_caps(const int64_t caps[6], const void *q, const int64_t q_
  * Reference layout: x (W,H,Cin,N) = row-major [N][Cin][H][W]; w (KW,KH,Cin,Cout) =
  * [Cout][Cin][KH][KW]; out (OW,OH,Cout,N); bias[Cout] or NULL; stride / padding /
  * dilation as (x, y) pairs; act MI_EPI_NONE or MI_EPI_RELU (anything else returns
- * MI_DECLINE_UNSUPPORTED).  groups = 1 runs as a GEMM (1x1, implicit, or im2col: see
- * mi_conv2d_f16_plan); groups > 1 -- w then holds Cin / groups input channels per filter --
+ * MI_DECLINE_UNSUPPORTED).  groups = 1 runs on the matrix units (1x1 as a GEMM, in one launch
+ * over patches, a gathered or an im2col GEMM: see mi_conv2d_f16_kernel); groups > 1 -- w then holds Cin / groups input channels per filter --
  * runs a direct kernel, one thread per output element, as the reference routes
  * grouped convolutions to its direct kernel (conv.jl:100-145); Cin or Cout not
  * divisible by groups declines.  fp32 accumulation seeded with the bias, one rounding,
  * relu on the rounded value.
  * Replaces convolution!(ctx, out, x, w, bias, stride, padding, dilation, groups; act)
  * -- conv.jl:100-145 -- and convolution_coopmat! / im2col_kernel! /
- * conv_epilogue_kernel! -- conv_coopmat.jl:246-392; the implicit-GEMM path (stride_x 1,
- * OW % 8 == 0, Cin*KH*KW % 64 == 0) is the MFMA counterpart of conv2d_igemm! --
- * conv_implicit.jl:53-355: the im2col matrix is never written, the GEMM gathers its
- * operand from a zero-padded copy of x in the workspace. */
+ * conv_epilogue_kernel! -- conv_coopmat.jl:246-392; the one-launch form and the gather are
+ * the MFMA counterparts of conv2d_igemm! -- conv_implicit.jl:53-355: the im2col matrix is
+ * never written, its rows are put together from patches in LDS or read from a zero-padded
+ * channels-last copy of x in the workspace. */
 int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
                   int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
                   int64_t KW, int64_t KH, int64_t Cout,

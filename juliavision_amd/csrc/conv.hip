@@ -5,9 +5,10 @@
 // so the weight is the K-contiguous operand as it lies, the pixel axis is the
 // contiguous axis of both col and out, and the bias is per output ROW.
 //   1x1 / stride 1 / no padding : col is x itself, no copy (conv.jl:63-66,117-131)
-//   otherwise                   : im2col into scratch, then the same GEMM
-//                                 (conv_coopmat.jl:246-392)
 //   groups != 1                 : the direct kernel (conv.jl:26-51,298-302)
+//   otherwise, by estimate      : one launch over LDS patches (conv_tile.hip); or, where the channels come in sixteens
+//                                 (patch_ok), a zero-padded channels-last copy whose patches gemm_ring.hip gathers, and
+//                                 im2col into scratch with the same GEMM (conv_coopmat.jl:246-392) for the others.
 #include "conv_common.hpp"
 
 namespace {

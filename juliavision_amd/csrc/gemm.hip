@@ -1,7 +1,8 @@
 // fp16 GEMM for gfx950: MFMA 32x32x16 f16 with fp32 accumulation, LDS
 // double-buffered operand tiles, 128-bit global loads, fused bias / activation /
 // residual store; a split-K bandwidth kernel for decode-sized T.  The four-wave kernel, the decode-sized kernels, the plans and
-// the C ABI are here; gemm_pipe.hip has the small and gathered tiles, gemm_any.hip what neither can address.
+// the C ABI are here; gemm_pipe.hip has the small tiles, gemm_ring.hip those of small deep grids and the gathered ones of a
+// convolution, gemm_any.hip what none of them can address.
 //
 // Internal problem statement (row-major):  Y[M x N] = A[M x K] . B  (+ bias)
 //   A is K-contiguous.  B is either N-contiguous [K][N] (B_KN) or K-contiguous
@@ -1266,7 +1267,8 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
 // a cache line, so most 128-byte pieces of them touch two.  A GELU store adds `gelu` a round.  A split adds the second
 // launch (4.4 us) and the fp32 planes (0.38 us per MB).
 // Fitted to every tile timed on 200 shapes in a replayed graph (M 9..8192, N 64..8192, K 72..5120, both layouts, a third of
-// them with K % 64, a third with GELU): the cheapest estimate lands within 0.3 % of the best measured tile on average.
+// them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.3 % of the best measured tile on average;
+// on 80 further shapes of the same ranges 1.7 %, at most 16 % (3001 x 2304 -> 3136 with GELU: 60.5 us as planned, 52.1 on 192 x 128).
 // What it replaced sent every K % 64 to 64 x 64 tiles: 1544 x 1288 -> 1288 with residual 19.8 -> 15.4 us on 128 x 128,
 // 636 x 4392 -> 104 23.2 -> 13.8 on the ring, 2237 x 5096 -> 2440 with GELU 143 -> 80 on 192 x 128.
 struct TileModel { int bm, bn; double step_lo, step_full, round, fixed, gelu, tail; };

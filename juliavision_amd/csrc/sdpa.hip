@@ -1157,7 +1157,7 @@ int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, bo
     const double tiles = (double)ceil_div(nt, waves), wide = E <= 64 ? 1.0 : E <= 96 ? 1.5 : 1.9;
     if (f32) {
         // Against a workgroup per query row (and key split, with a merge launch).  170 shapes of 2 to 63 queries, 16 to 4096
-        // keys, 1 to 320 (head, batch): 12.5 us there, 8.0 here, 7.8 as chosen, 7.7 with the best of both and of 2, 4 and 8
+        // keys, 1 to 320 (head, batch): 12.5 us there, 8.3 here, 7.8 as chosen, 7.7 with the best of both and of 2, 4 and 8
         // waves (geometric means).  4 x 20 x 60 over 1500 keys: 134 us there, 13.2 here; 16 x 20 x 63 over 4000: 1213 and 73;
         // 7 queries x 4 heads over 64 keys: 3.8 and 4.2; 8 heads x 4 queries over 2000 keys: 8.3 and 12.
         const int64_t ns = rows_splits(Lq, Lk, H, B);

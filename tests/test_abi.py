@@ -169,9 +169,9 @@ def test_conv_planner_and_extents():
     assert plan(64, 64, 255, 1, 3, 3, 256, 1, 1, 1, 1, 1, 1, 4) == "decline"
     assert plan(2, 2, 3, 1, 5, 5, 8, 1, 1, 0, 0, 1, 1, 1) == "decline"              # empty output
     assert lib.mi_convsize(518, 14, 14, 0, 1) == 37 and lib.mi_convsize(256, 7, 4, 3, 1) == 64
-    # implicit GEMM scratch: the zero-padded input [Cin][H+2][W+2 -> 72] fp16 twice (the second copy shifted by one
-    # element, for taps that start at an odd column), the weights re-laid tap-major; K = 2304 is shallow enough for
-    # one pass of 64 x 64 tiles, K = 9216 is split into fp32 planes of the 256 x 4096 output
+    # what callers size an implicit GEMM's scratch by (more than its kernel takes: mi_conv2d_f16_kernel has that): the zero-padded
+    # input [Cin][H+2][W+2 -> 72] fp16 twice, the weights re-laid tap-major, and for K = 9216 fp32 planes of the 256 x 4096
+    # output; K = 2304 is shallow enough for none
     ws = lib.mi_conv2d_f16_workspace(64, 64, 256, 1, 3, 3, 256, 1, 1, 1, 1, 1, 1)
     assert ws == 2 * 256 * 66 * 72 * 2 + 256 * 2304 * 2
     ws = lib.mi_conv2d_f16_workspace(64, 64, 1024, 1, 3, 3, 256, 1, 1, 1, 1, 1, 1)
