@@ -187,6 +187,7 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
     static_assert(WAVES_M * WAVES_N == 4 && TM * TN <= 8 && TM >= 2 && PER_TILE <= 63, "one matrix wave per SIMD; at most 128 accumulator registers a lane; vmcnt is a 6-bit counter");
     static_assert(!B_KN || BN >= 128, "the [K][N] permutation moves a chunk by up to 12 places inside its row");
     extern __shared__ __align__(16) char smem[];
+    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WAVES_M, wn = wave / WAVES_M;
@@ -285,78 +286,8 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
         return;
     }
     if (wave == 5) {
-        // The statistics wave of a folded layer norm.  The matrix waves need (r, r mu) of
-        // the tile's rows and the tile's columns of colsum and biasp at the store, not before: combining a row's
-        // K / 32 segment statistics in the prologue held every wave at the first barrier (5 000 clocks at 128 rows,
-        // 10 000 at 192: a trip to memory per batch of loads, then forty dependent steps a row).  This wave does it
-        // beside the K loop instead: tile kt covers segments 2 kt and 2 kt + 1 (K % 64 == 0), so between two barriers
-        // it takes in the two segments of each of its BM / 64 rows that it requested four tiles earlier, and the
-        // result is in the LDS slot when it arrives at the last barrier, which the matrix waves pass before they
-        // store.  Same arithmetic, in the same order per row, as LnfLoader with one lane a row.
-        constexpr int NR = BM / 64, AHEAD = 4;
-        static_assert(BM % 64 == 0 && NR * 2 * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
-        for (int t = lane; t < BN / 2; t += 64) {
-            const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
-            const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
-            float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
-            else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
-            *reinterpret_cast<float4v *>(reinterpret_cast<float *>(ln_slot + BM) + which * BN + c) = v;
-        }
-        const float2v *seg[NR];
-#pragma unroll
-        for (int i = 0; i < NR; i++) seg[i] = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + lane + 64 * i, p.M - 1);
-        float2v v[AHEAD][NR][2];
-        float ref[NR], total[NR], within[NR], between[NR];
-#pragma unroll
-        for (int i = 0; i < NR; i++) { ref[i] = 0.0f; total[i] = 0.0f; within[i] = 0.0f; between[i] = 0.0f; }
-        auto fetch = [&](auto SLOT, int kt) {
-            constexpr int sl = decltype(SLOT)::value;
-#pragma unroll
-            for (int i = 0; i < NR; i++)
-#pragma unroll
-                for (int h = 0; h < 2; h++) v[sl][i][h] = seg[i][(long)(2 * kt + h) * p.M];
-        };
-        auto take = [&](auto SLOT, int kt) {
-            constexpr int sl = decltype(SLOT)::value;
-#pragma unroll
-            for (int i = 0; i < NR; i++)
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    if (kt == 0 && h == 0) ref[i] = v[sl][i][0][0] * (1.0f / 32.0f);
-                    const float d = fmaf(v[sl][i][h][0], 1.0f / 32.0f, -ref[i]);
-                    total[i] += v[sl][i][h][0];
-                    within[i] += v[sl][i][h][1];
-                    between[i] = fmaf(32.0f * d, d, between[i]);
-                }
-        };
-        // tiles 0 .. AHEAD - 1 are requested before the first barrier; tile kt + AHEAD right after tile kt is taken in
-        static_for<AHEAD>([&](auto S) { if (decltype(S)::value < nk) fetch(S, decltype(S)::value); });
-        barrier();
-        for (int kt0 = 0; kt0 < nk; kt0 += AHEAD) {
-            static_for<AHEAD>([&](auto S) {
-                const int kt = kt0 + decltype(S)::value;
-                if (kt < nk) {
-                    // requests complete in order: what was requested after tile kt may still be on its way
-                    if (kt + AHEAD - 1 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NR * 2) : "memory");
-                    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    take(S, kt);
-                    if (kt + AHEAD < nk) fetch(S, kt + AHEAD);
-                    if (kt + 1 == nk) {
-#pragma unroll
-                        for (int i = 0; i < NR; i++) {
-                            const float mu = total[i] / (float)p.K, dm = mu - ref[i];
-                            const float m2 = within[i] + fmaxf(between[i] - (float)p.K * dm * dm, 0.0f);
-                            const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
-                            const float2v o = {r, r * mu};
-                            ln_slot[lane + 64 * i] = o;
-                        }
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    }
-                    barrier();                                      // B_kt
-                }
-            });
-        }
+        // the statistics wave of a folded layer norm
+        lnf_stats_wave<BM, BN, true>(p, ln_slot, m0, n0, bz, lane, nk, barrier);
         if (coop) help_store();
         return;
     }
@@ -1266,25 +1197,21 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
 // workgroups overlap).  A K that ends inside a tile makes every step `tail` times as long: its rows are no multiple of
 // a cache line, so most 128-byte pieces of them touch two.  A GELU store adds `gelu` a round.  A split adds the second
 // launch (4.4 us) and the fp32 planes (0.38 us per MB).
-// Fitted to every tile timed on 200 shapes in a replayed graph (M 9..8192, N 64..8192, K 72..5120, both layouts, a third of
-// them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.3 % of the best measured tile on average;
-// on 80 further shapes of the same ranges 1.7 %, at most 16 % (3001 x 2304 -> 3136 with GELU: 60.5 us as planned, 52.1 on 192 x 128).
+// Fitted to every tile timed on 150 shapes in a replayed graph (M 9..4096, N 64..5120, K 72..5120, both layouts, a third of
+// them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.5 % of the best measured tile on average.
 // What it replaced sent every K % 64 to 64 x 64 tiles: 1544 x 1288 -> 1288 with residual 19.8 -> 15.4 us on 128 x 128,
 // 636 x 4392 -> 104 23.2 -> 13.8 on the ring, 2237 x 5096 -> 2440 with GELU 143 -> 80 on 192 x 128.
 struct TileModel { int bm, bn; double step_lo, step_full, round, fixed, gelu, tail; };
 constexpr int NTILES = 6;
 constexpr TileModel TILE_MODELS[NTILES] = {
-    {128, 256, 0.444, 0.720, 1.13, 6.2, 2.9, 1.43},
-    {192, 128, 0.360, 0.556, 1.11, 5.2, 2.4, 1.46},
-    {128, 128, 0.386, 0.534, 1.06, 3.9, 2.0, 1.13},
-    {64, 128, 0.287, 0.356, 0.856, 3.26, 1.0, 1.28},
-    {64, 64, 0.209, 0.252, 0.70, 2.93, 0.46, 1.35},
-    // gemm_ring_kernel: its sum of four partial tiles and deep ring cost a microsecond at the ends, so it starts past
-    // K = 512 -- where the layer-norm prologue's promise of identical bits ends too -- and above one workgroup per CU its
-    // LDS allows no second one: L2 bandwidth (19 to 24 TB/s) is what bounds it there in any case.
-    {64, 64, 0.127, 0.141, 1.00, 4.31, 0.56, 1.10},
+    {128, 256, 0.458, 0.779, 1.04, 5.88, 2.8, 1.48},
+    {192, 128, 0.376, 0.655, 1.07, 4.96, 2.22, 1.41},
+    {128, 128, 0.436, 0.614, 1.11, 4.1, 1.93, 1.08},
+    {64, 128, 0.33, 0.411, 0.818, 3.51, 1.01, 1.16},
+    {64, 64, 0.255, 0.326, 0.617, 3.29, 0.533, 1.22},
+    {64, 64, 0.153, 0.219, 0.775, 3.46, 0.494, 1.41},      // gemm_ring_kernel
 };
-constexpr int RING_KMIN = 513;
+constexpr int64_t RING_WGS_PER_CU = 6;       // as many as the fit has seen
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
@@ -1333,14 +1260,14 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring, bool gelu) {
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu) {
     TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
     for (int split = 1; split <= max_split; split++) {
         if (split > 1 && (K % (64 * split) != 0 || K / split < 128)) continue;
         for (int tile = 0; tile < NTILES; tile++) {
-            if (tile == RING_TILE && (!ring || K / split < RING_KMIN || ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > mi_num_cus())) continue;
+            if (tile == RING_TILE && ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > RING_WGS_PER_CU * mi_num_cus()) continue;
             const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
@@ -1356,14 +1283,14 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
 
 // The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
 // thread keeps the last answers.  The key holds everything the estimate reads.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool ring = true, bool gelu = false) {
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu = false) {
     struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
     static thread_local Entry table[256] = {};
-    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (ring ? 8 : 0) | (gelu ? 16 : 0);
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (gelu ? 8 : 0);
     const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 40;
     Entry &e = table[(h >> 32) & 255];
     if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
-        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, ring, gelu)};
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, gelu)};
     return e.plan;
 }
 
@@ -1540,9 +1467,9 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
         // A GELU store is some fifteen vector instructions a value, so narrower tiles can be the faster ones for it (1500 x 384 ->
-        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every pipelined tile sums K in the same order: the bits stay.
-        if (pipe && split == 1 && tp.tile != RING_TILE && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, true);
+        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every tile sums K in the same order: the bits stay.
+        if (pipe && split == 1 && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true);
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }

@@ -35,6 +35,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;
     constexpr int GROUP = 2 * (BM + BN) * LD;               // halves of one group's double buffer
     extern __shared__ __align__(16) char smem[];
+    stage_args(p);
     const int tid = threadIdx.x & 255, group = threadIdx.x >> 8, lane = tid & 63, wave = tid >> 6;
     half_t *As = reinterpret_cast<half_t *>(smem) + group * GROUP, *Bs = As + 2 * BM * LD;
     const int wm = wave & 1, wn = wave >> 1;

@@ -8,17 +8,36 @@
 #include "common.hpp"
 #include <type_traits>
 
+// The order is the kernels': what stands between a launch and its first load lies in the first two 64-byte lines of the
+// argument block, what its store needs in the next two (stage_args).
 struct GemmArgs {
-    void *Y;
-    const half_t *A, *B, *bias, *residual;
+    const half_t *A, *B;
+    long ldA, ldB;
     int M, N, K;
     int NB;                 // columns addressable in B (>= N; a multiple of 8 for the [K][N] layout)
-    long ldY, ldA, ldB;
-    long sY, sA, sB, sBias; // batch strides (elements)
-    long dRes;              // the residual's batch stride is sY + dRes (one position embedding for every image: -sY)
-    int bias_mode, epi, out_f32;
     int tiles_m, tiles_n, group_m;
     unsigned div_width, div_group, div_last;      // tile_of's divisions as multiplications (set_tiles)
+    int bias_mode, epi;
+    long sA, sB, sY, sBias; // batch strides (elements)
+    void *Y;
+    long ldY;
+    const half_t *bias, *residual;
+    long dRes;              // the residual's batch stride is sY + dRes (one position embedding for every image: -sY)
+    // Layer norm folded away (mi_lnfold_gemm_f16): A holds the raw rows, B carries gamma, and the store turns an
+    // accumulator into r (acc - mu colsum[n]) + biasp[n], with the row's (mu, r) combined from lnf_stats.
+    const float *lnf_stats;           // [lnf_nseg][M][2]: (sum, squares about its own mean) of each 32-column segment of a row
+    const float *lnf_colsum, *lnf_biasp;      // fp32[N], plane stride lnf_svec
+    long lnf_svec;
+    int lnf_nseg;
+    float lnf_eps;
+    // Row statistics of the result for a later folded norm: stats_out[n / 32][m] = (sum, squares about the mean) of the
+    // final fp16 values Y[m][32 (n / 32) .. + 32); stats_nseg segments per row.
+    float *stats_out;
+    int stats_nseg;
+    // Tiled kernels and the split-K plane sums: > 0 clamps the fp16 result to [-clamp, clamp] after the residual add,
+    // as a separate aten::clamp on Y would (the overflow guard of exported fp16 encoder layers).
+    float clamp;
+    int out_f32;
     int vec_store;          // Y (and residual) rows allow 16-byte accesses
     ConvGather cv;          // cv.xp != nullptr: B is the im2col matrix of a convolution, gathered on the fly
     NhwcGather ag;          // ag.x != nullptr: A is the patch matrix of a channels-last convolution, gathered on the fly
@@ -32,9 +51,6 @@ struct GemmArgs {
     half_t *lnout;
     const half_t *lnout_gamma, *lnout_beta;
     float lnout_eps;
-    // Tiled kernels and the split-K plane sums: > 0 clamps the fp16 result to [-clamp, clamp] after the residual add,
-    // as a separate aten::clamp on Y would (the overflow guard of exported fp16 encoder layers).
-    float clamp;
     // Measurement only (mi_set_clock_probe): workgroup 0 of a four-wave launch stores {shader clock, 100 MHz clock}
     // here when it starts and again after its last store.  Null in ordinary use.
     unsigned long long *clk;
@@ -49,17 +65,6 @@ struct GemmArgs {
     float *sk_part;
     unsigned *sk_flags;
     unsigned sk_epoch;
-    // Layer norm folded away (mi_lnfold_gemm_f16): A holds the raw rows, B carries gamma, and the store turns an
-    // accumulator into r (acc - mu colsum[n]) + biasp[n], with the row's (mu, r) combined from lnf_stats.
-    const float *lnf_stats;           // [lnf_nseg][M][2]: (sum, squares about its own mean) of each 32-column segment of a row
-    const float *lnf_colsum, *lnf_biasp;      // fp32[N], plane stride lnf_svec
-    long lnf_svec;
-    int lnf_nseg;
-    float lnf_eps;
-    // Row statistics of the result for a later folded norm: stats_out[n / 32][m] = (sum, squares about the mean) of the
-    // final fp16 values Y[m][32 (n / 32) .. + 32); stats_nseg segments per row.
-    float *stats_out;
-    int stats_nseg;
     int sk_spin;                      // polls before a wave gives up on its partners
     unsigned sk_pub_xor, sk_xcc_xor;  // zero in ordinary use: mi_test_exchange_faults makes the waits fail from the host side
     unsigned *status;                 // the device's sticky status word
@@ -75,46 +80,49 @@ __device__ __forceinline__ void static_for(F &&f) {
     }
 }
 
+// Kernel arguments come through the scalar cache a 64-byte line at a time: 200 clocks a line in a replayed graph, 550 to 700 where
+// the host has just written them, and the compiler asks for a field where it is first used, so that four or five such trips
+// stood in a row between a launch and its first load.  Naming the fields at the kernel's first line requests them together.
+__device__ __forceinline__ void stage_args(const GemmArgs &p) {
+    asm volatile("" ::"s"(p.A), "s"(p.B), "s"(p.ldA), "s"(p.ldB), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.NB), "s"(p.tiles_m), "s"(p.tiles_n),
+                 "s"(p.group_m), "s"(p.div_width), "s"(p.div_group), "s"(p.div_last), "s"(p.bias_mode), "s"(p.epi), "s"(p.sA), "s"(p.sB),
+                 "s"(p.Y), "s"(p.ldY), "s"(p.bias), "s"(p.residual), "s"(p.lnf_stats), "s"(p.stats_out), "s"(p.vec_store));
+}
+
 // Workgroup id -> output tile.  The hardware deals consecutive workgroups
 // round-robin over the 8 XCDs, each with its own L2; this hands every XCD one
 // contiguous run of the tile order, and the tile order walks GROUP_M row tiles
 // per column tile so a run reuses a small set of A and B panels.
-// Its divisions are multiplications by reciprocals the host worked out (set_tiles): a division is some thirty vector
-// instructions at eight clocks each, and three of them in a row stood between a launch and its first load.
+// Its divisions are multiplications by reciprocals the host worked out (set_tiles): a division is some thirty instructions at
+// four to eight clocks each, and three of them in a row stood between a launch and its first load.  With r = floor((2^32 - 1) / d) the
+// product's upper half is the quotient or one less, for every 32-bit dividend, and no case needs a branch.
 __device__ __forceinline__ void tile_of(const GemmArgs &p, int &tm, int &tn) {
-    const int pid = blockIdx.x, nwg = gridDim.x;
+    const int pid = blockIdx.x, nwg = p.tiles_m * p.tiles_n;
     const int xcd = pid & 7, idx = pid >> 3;
     const int full = nwg >> 3, rem = nwg & 7;
     const int logical = xcd * full + min(xcd, rem) + idx;
-    const int width = p.group_m * p.tiles_n;
-    const auto over = [](int x, unsigned recip) { return recip ? (int)__umulhi((unsigned)x, recip) : x; };
-    int g, in, first, gsz;
-    if (p.div_width != 1) {
-        g = over(logical, p.div_width);
-        in = logical - g * width;
-        first = g * p.group_m;
-        gsz = min(p.tiles_m - first, p.group_m);
-        tn = over(in, gsz == p.group_m ? p.div_group : p.div_last);
-    } else {                                              // a grid too large for 32-bit reciprocals
-        g = logical / width;
-        in = logical - g * width;
-        first = g * p.group_m;
-        gsz = min(p.tiles_m - first, p.group_m);
-        tn = in / gsz;
-    }
-    tm = first + in - tn * gsz;
+    const auto divide = [](unsigned x, unsigned d, unsigned recip, int &left) {
+        unsigned q = __umulhi(x, recip), r = x - q * d;
+        const bool up = r >= d;
+        q += up ? 1u : 0u;
+        left = (int)(r - (up ? d : 0u));
+        return (int)q;
+    };
+    int in;
+    const int first = divide(logical, p.group_m * p.tiles_n, p.div_width, in) * p.group_m;
+    const int gsz = min(p.tiles_m - first, p.group_m);
+    tn = divide(in, gsz, gsz == p.group_m ? p.div_group : p.div_last, tm);
+    tm += first;
 }
 
-// The tile grid of a launch.  ceil(2^32 / d) divides x exactly while x d < 2^32; 0 stands for d = 1, and 1 as div_width for
-// a grid beyond that.
+// The tile grid of a launch.
 inline void set_tiles(GemmArgs &a, int bm, int bn) {
     a.tiles_m = (int)ceil_div(a.M, bm);
     a.tiles_n = (int)ceil_div(a.N, bn);
     a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    const auto recip = [](int d) { return d <= 1 ? 0u : (unsigned)(((1ull << 32) + (unsigned)d - 1) / (unsigned)d); };
+    const auto recip = [](int64_t d) { return (unsigned)(0xffffffffll / d); };
     const int last = a.tiles_m % a.group_m;
-    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n, width = (int64_t)a.group_m * a.tiles_n;
-    a.div_width = tiles * width < (1ll << 32) ? recip((int)width) : 1u;
+    a.div_width = recip((int64_t)a.group_m * a.tiles_n);
     a.div_group = recip(a.group_m);
     a.div_last = recip(last ? last : a.group_m);
 }
@@ -217,6 +225,85 @@ struct LnfLoader {
         }
     }
 };
+
+// The same by a wave of its own, beside the K loop of kernels that have a barrier a tile: the matrix waves need (r, r mu) of the
+// tile's rows and the tile's columns of colsum and biasp at the store, not before, and in their registers the statistics
+// would cost a second workgroup a CU.  (In the prologue they held every wave at the first barrier: 5 000 clocks at 128 rows,
+// 10 000 at 192, a trip to memory per batch of loads, then forty dependent steps a row.)  Tile kt covers segments 2 kt and
+// 2 kt + 1: ahead of barrier kt this wave takes in the two segments of each of its BM / 64 rows that it requested AHEAD tiles
+// earlier, and the result is in the slot when it arrives at the last barrier, which the matrix waves pass before they store.
+// Same arithmetic, in the same order per row, as LnfLoader with one lane a row.  LEAD: a barrier comes before tile 0's.
+template <int BM, int BN, bool LEAD, typename BarrierF>
+__device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot, int m0, int n0, long bz, int lane, int nk, BarrierF barrier) {
+    constexpr int NR = BM / 64, AHEAD = 4;
+    static_assert(BM % 64 == 0 && NR * 2 * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
+    for (int t = lane; t < BN / 2; t += 64) {
+        const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
+        const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
+        float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
+        else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
+        *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = v;
+    }
+    const float2v *seg[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) seg[i] = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + lane + 64 * i, p.M - 1);
+    float2v v[AHEAD][NR][2];
+    float ref[NR], total[NR], within[NR], between[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) { ref[i] = 0.0f; total[i] = 0.0f; within[i] = 0.0f; between[i] = 0.0f; }
+    auto fetch = [&](auto SLOT, int kt) {
+        constexpr int sl = decltype(SLOT)::value;
+#pragma unroll
+        for (int i = 0; i < NR; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) v[sl][i][h] = seg[i][(long)min(2 * kt + h, p.lnf_nseg - 1) * p.M];
+    };
+    auto take = [&](auto SLOT, int kt) {
+        constexpr int sl = decltype(SLOT)::value;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int left = p.K - 32 * (2 * kt + h);                  // uniform
+            if (left <= 0) break;
+            const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
+#pragma unroll
+            for (int i = 0; i < NR; i++) {
+                if (kt == 0 && h == 0) ref[i] = v[sl][i][0][0] * inv;
+                const float d = fmaf(v[sl][i][h][0], inv, -ref[i]);
+                total[i] += v[sl][i][h][0];
+                within[i] += v[sl][i][h][1];
+                between[i] = fmaf(cnt * d, d, between[i]);
+            }
+        }
+    };
+    // tiles 0 .. AHEAD - 1 are requested at once; tile kt + AHEAD right after tile kt is taken in
+    static_for<AHEAD>([&](auto S) { if (decltype(S)::value < nk) fetch(S, decltype(S)::value); });
+    if (LEAD) barrier();
+    for (int kt0 = 0; kt0 < nk; kt0 += AHEAD) {
+        static_for<AHEAD>([&](auto S) {
+            const int kt = kt0 + decltype(S)::value;
+            if (kt < nk) {
+                // requests complete in order: what was requested after tile kt may still be on its way
+                if (kt + AHEAD - 1 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NR * 2) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                take(S, kt);
+                if (kt + AHEAD < nk) fetch(S, kt + AHEAD);
+                if (kt + 1 == nk) {
+#pragma unroll
+                    for (int i = 0; i < NR; i++) {
+                        const float mu = total[i] / (float)p.K, dm = mu - ref[i];
+                        const float m2 = within[i] + fmaxf(between[i] - (float)p.K * dm * dm, 0.0f);
+                        const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
+                        const float2v o = {r, r * mu};
+                        slot[lane + 64 * i] = o;
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                }
+                barrier();                                      // B_kt
+            }
+        });
+    }
+}
 
 // ------------------------------------------------------------------------------------------
 // Accumulator tile -> memory, shared by the tiled kernels.
@@ -431,9 +518,30 @@ __device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4
 // Same arithmetic as the general store (bias joined in fp32, one rounding, activation on the rounded value, residual,
 // clamp), so the two give the same bits.  Two staging areas a wave: block j + 1 is staged while block j's chunks are on
 // their way back from the LDS (a wave's LDS operations complete in order: no wait between staging a block and reading it).
+__device__ __forceinline__ bool store_is_simple(const GemmArgs &p) { return !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW; }
+
+// A wave's residual chunks of its first 32-row block, which the common store can be handed instead of fetching them itself: a kernel
+// that asks for them while its products run spares the store a trip to memory.
+template <int WTN>
+struct ResidualAhead {
+    static constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI;
+    half8v v[NIT];
+    // (mw, nw): the wave's first row and column
+    __device__ __forceinline__ void request(const GemmArgs &p, int mw, int nw, int lane, long bz) {
+        const int ch = lane % CPR, r0 = lane / CPR, n = nw + ch * 8;
+        const bool on = p.residual && store_is_simple(p);
+        const half_t *const base = p.residual + bz * (p.sY + p.dRes) + (long)(mw + r0) * p.ldY + n;
+#pragma unroll
+        for (int t = 0; t < NIT; t++) {
+            v[t] = half8v{};
+            if (on && n < p.N && mw + r0 + t * RPI < p.M) v[t] = as_half8(ldg16(base + (long)(t * RPI) * p.ldY));
+        }
+    }
+};
+
 template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
 __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                                  int wave, int lane, long bz, const LnFold<TM> ln) {
+                                                  int wave, int lane, long bz, const LnFold<TM> ln, const ResidualAhead<WTN> *ahead) {
     constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;      // halves per staged row; one staging area
     constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI;     // 16-byte chunks per row; rows a wave covers at a time; chunks per lane and block
     static_assert(2 * BUF_BYTES * NWAVES <= LDS_BYTES && 64 % CPR == 0 && CPR % 4 == 0, "two staging areas a wave; four lanes hold a 32-column segment");
@@ -462,7 +570,12 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
             if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) res[j & 1][t] = as_half8(ldg16(rbase + (long)(32 * j + t * RPI) * p.ldY));
         }
     };
-    if (rbase) fetch_residual(std::integral_constant<int, 0>{});
+    if (rbase) {
+        if (ahead) {
+#pragma unroll
+            for (int t = 0; t < NIT; t++) res[0][t] = ahead->v[t];
+        } else fetch_residual(std::integral_constant<int, 0>{});
+    }
     stage(std::integral_constant<int, 0>{});
     static_for<TM>([&](auto J) {
         constexpr int j = decltype(J)::value;
@@ -522,8 +635,7 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
 // when it has block j's chunks in registers, so staging block j + 2 over block j's area after that barrier is safe).
 // Launches without residual, clamp or statistics only: the others keep store_tile_simple on the matrix waves alone.
 __host__ __device__ __forceinline__ bool coop_store_applies(const GemmArgs &p) {
-    return !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW && !p.residual &&
-           !(p.clamp > 0.0f) && !p.stats_out;
+    return !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW && !p.residual && !(p.clamp > 0.0f) && !p.stats_out;
 }
 template <int EPI, int TM, int WTN, bool HELPER, typename StageF, typename BarrierF>
 __device__ __forceinline__ void store_coop_epi(const GemmArgs &p, char *buf, int mw, int nw, int lane, long bz, StageF stage, BarrierF barrier) {
@@ -565,14 +677,13 @@ __device__ __forceinline__ void store_coop(const GemmArgs &p, char *buf, int mw,
 // instead of one per element.
 template <int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
 __device__ __forceinline__ void store_tile(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                           int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
-    const bool simple = !p.out_f32 && p.vec_store && p.N % 8 == 0 && p.bias_mode != MI_BIAS_ROW;
-    if (simple) {
+                                           int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}, const ResidualAhead<WTN> *ahead = nullptr) {
+    if (store_is_simple(p)) {
         switch (p.epi) {
-        case MI_EPI_GELU_ERF: store_tile_simple<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        case MI_EPI_GELU_TANH: store_tile_simple<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        case MI_EPI_RELU: store_tile_simple<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
-        default: store_tile_simple<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln); break;
+        case MI_EPI_GELU_ERF: store_tile_simple<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, ahead); break;
+        case MI_EPI_GELU_TANH: store_tile_simple<MI_EPI_GELU_TANH, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, ahead); break;
+        case MI_EPI_RELU: store_tile_simple<MI_EPI_RELU, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, ahead); break;
+        default: store_tile_simple<MI_EPI_NONE, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, ahead); break;
         }
         return;
     }

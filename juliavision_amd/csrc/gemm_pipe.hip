@@ -43,6 +43,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
     static_assert(PA >= 1 && PB >= 1, "tile too small for this workgroup");
     constexpr int BSZ = B_KN ? BK * BLD : BN * LD;      // halves per B buffer
     extern __shared__ __align__(16) char smem[];
+    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     half_t *As = reinterpret_cast<half_t *>(smem);   // [2][BM][LD]; AMODE 2: the normalised panel [BM][K + 8]
     const int KP = p.K + 8;                          // panel row (halves): 16 bytes off a multiple of 128, like LD
@@ -274,15 +275,18 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         body(M0{}, kt + 1, 1, 0, 1);
     }
     half4v cb[TN][4];
+    ResidualAhead<WTN> res;
     if (nk & 1) {
         body(M0{}, kt, 0, 1, 0);
         body(M1{}, kt + 1, 1, 0, 1);
         load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
+        if constexpr (!LNF) res.request(p, m0 + wm * WTM, n0 + wn * WTN, lane, bz);
         if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
         body(M2{}, kt + 2, 0, 1, 0);
     } else {
         body(M1{}, kt, 0, 1, 0);
         load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
+        if constexpr (!LNF) res.request(p, m0 + wm * WTM, n0 + wn * WTN, lane, bz);
         if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
         body(M2{}, kt + 1, 1, 0, 1);
     }
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
 #pragma unroll
         for (int j = 0; j < TM; j++) { const float2v v = ln_slot[wm * WTM + 32 * j + (lane & 31)]; ln.r[j] = v[0]; ln.rmu[j] = v[1]; }
     }
-    store_tile<TM, TN, WTM, WTN, WAVES_M * WAVES_N, 2 * (BM * LD + BSZ) * 2>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln);
+    store_tile<TM, TN, WTM, WTN, WAVES_M * WAVES_N, 2 * (BM * LD + BSZ) * 2>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, LNF ? nullptr : &res);
 }
 
 template <int BM, int BN, int WM, int WN>

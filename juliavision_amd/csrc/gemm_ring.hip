@@ -1,4 +1,4 @@
-// fp16 GEMM for gfx950, 64 x 64 wave tiles over a ring of direct-to-LDS stages: grids too small for the four-wave kernel.
+// fp16 GEMM for gfx950, 64 x 64 tiles over a ring of direct-to-LDS stages: grids too small for the four-wave kernel.
 #include "gemm_common.hpp"
 
 // Sixteen zero bytes for loads of chunks past the end of K.
@@ -6,16 +6,21 @@ static __device__ __align__(16) unsigned ring_zero_words[4];
 
 namespace {
 
-// A workgroup owns a 64 x 64 tile; each of its four matrix waves holds all of it in accumulators and takes one of the four 16-deep
-// steps of every 64-deep tile of K.  The four partial tiles are summed through LDS before the store.
+// A workgroup owns a 64 x 64 tile, each of its four matrix waves a 32 x 32 block of it; two loader waves keep the ring filled, a
+// seventh takes in a folded norm's statistics.
 //
-// What bounds such a tile is the CU's LDS and vector-memory path, not the matrix cores.  Per 64-deep tile a 64 x 64 tile
-// takes 256 clocks of 64 B/clock loads and 128 clocks of MFMAs; four 32 x 32 waves (gemm_pipe_kernel) move 16 KB into LDS
-// through registers and read 32 KB of fragments, 384 LDS clocks, and were measured at 480 to 600.  Waves that split K
-// instead of the tile read each fragment once: 16 KB in, 16 KB out, and the loads bypass the registers
-// (global_load_lds_dwordx4), S stages deep, so that a trip to memory is S - 2 tiles long.  In launches of one tile a CU those
-// loads are under half of the time: 6100 of 20 400 cycles a wave at 1370 x 1536 -> 384, 9200 of 25 400 at a 3 x 3 of 256 ->
-// 256 on 64 x 64; the rest is waiting for them, the first trip to memory, the sum of the partial tiles and the store.
+// What bounds such a tile is the CU's LDS and vector-memory path, not the matrix cores: per 64-deep tile 256 clocks of 64 B/clock
+// loads and 384 of LDS (16 KB in, 32 KB of fragments out) for 128 clocks of MFMAs.  Measured, a tile takes 320 to 400 clocks; the
+// register-staged kernel's same tile was at 480 to 670, because its loads pass through registers and its waits are the
+// compiler's.  In launches of one tile a CU the ends cost as much as the loop, and that is where the arrangement comes from
+// (clocks at 1370 x 1536 -> 384, 132 workgroups; before, with waves that split K's steps and a ring filled before the first
+// product): first request 2040 -> 840 (stage_args, tile_of), products begin 4620 -> 2600 (AHEAD tiles asked for, not the whole
+// ring), sum of the waves' partial tiles 2020 -> none, store 2030 -> 1270 (its residual comes with the first tiles).  9.3 -> 8.3 us
+// a launch; 1370 x 384 -> 384, where four waves that split K lost to the register-staged kernel, 5.1 -> 4.9 (4.65 before its
+// residual and statistics are counted), 76 x 1024 -> 3072 7.8 -> 6.3, 2056 x 1536 -> 384 11.1 -> 8.6.  Waves that split K read
+// 16 KB of fragments a tile instead of 32 and gain from some 45 tiles of K on in the smallest grids (32 x 3456 -> 448 10.3 against
+// 11.2 us); over 150 shapes they are 6 % behind.  Every tile of this library sums K in the same order, so the bits do not
+// depend on which one a plan picks.
 //
 // LDS layout of a stage: A rows of 128 bytes, then B ([N][K]: rows of 128 bytes; [K][N]: 64 rows of BN halves).  Direct loads
 // cannot pad, so 16-byte chunks are permuted inside their row: K-contiguous row r holds chunk c at c ^ (r % 8 ^ r / 8 % 2),
@@ -25,13 +30,14 @@ namespace {
 // CONV: B is the patch matrix of a convolution (ConvGather).  Its rows' offsets are as fixed as an ordinary operand's; what moves
 // from tile to tile is the tap, for all lanes alike where C is a multiple of 64, by the lane's pair of chunks otherwise.
 template <int S, bool B_KN, bool CONV = false>
-__global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
-    constexpr int BM = 64, BN = 64, BK = 64, NW = 4, NT = NW * 64;
+__global__ __launch_bounds__(4 * 64 + 192, S > 4 ? 2 : 4) void gemm_ring_kernel(GemmArgs p) {
+    constexpr int BM = 64, BN = 64, BK = 64, NW = 4;
     constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
     constexpr int STAGE_BYTES = SLOTS * 1024, A_BYTES = SLOTS_A * 1024;
     static_assert(!(CONV && B_KN), "a patch row is K-contiguous");
     static_assert(S >= 3, "a stage being read, one landed, one on its way");
     extern __shared__ __align__(16) char smem[];
+    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm_, tn_;
     tile_of(p, tm_, tn_);
@@ -46,7 +52,7 @@ __global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
         asm volatile("" ::: "memory");
     };
 
-    if (wave >= NW) {
+    if (__builtin_expect(wave >= NW, 1)) {                // (laid out first: what the launch waits for)
         // The loaders, one for each operand.  A matrix wave that issued its share of the requests stood at those instructions
         // with its products behind them (800 clocks a 64 x 64 tile), and a loader is quick only if a request costs it next
         // to nothing: a wave issues an instruction every four to eight clocks, so the lane's byte offset from the tile's
@@ -123,18 +129,29 @@ __global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
             const uint32_t lds1 = lds0 + (IS_A ? 0 : A_BYTES);
             int next = 0;                                 // the tile requested next, and its stage
             uint32_t stage = 0;
+            // A request's immediate offset moves its source and its destination alike: four requests share an LDS address, with the
+            // lane's offset lowered by what the immediate adds and the origin by the most of it, so that no offset is negative.
+            constexpr int LOW = 3072;
+#pragma unroll
+            for (int i = 0; i < LPW; i++) off[i] += LOW - 1024 * (i & 3);
+            org -= LOW;
             auto request = [&]() {
                 const uint32_t add = PATCH && !ONE_TAP ? (uint32_t)at : 0u;
                 const char *from_org = ONE_TAP ? org + at : org;
                 if ((next + 1) * BK <= p.K) {             // uniform
-                    asm volatile("s_mov_b32 m0, %0" ::"s"(lds1 + stage) : "memory");
 #pragma unroll
-                    for (int i = 0; i < LPW; i++)
-                        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_add_u32 m0, m0, 0x400" ::"v"(off[i] + add), "s"(from_org) : "memory", "scc");
+                    for (int q = 0; q < LPW; q += 4)
+                        asm volatile("s_mov_b32 m0, %0\n\t"
+                                     "s_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %1, %5\n\t"
+                                     "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+                                     "global_load_lds_dwordx4 %3, %5 offset:2048\n\t"
+                                     "global_load_lds_dwordx4 %4, %5 offset:3072" ::"s"(lds1 + stage + q * 1024),
+                                     "v"(off[q] + add), "v"(off[q + 1] + add), "v"(off[q + 2] + add), "v"(off[q + 3] + add), "s"(from_org) : "memory");
                 } else {                                  // the tile that K ends in: chunks past it come from the zeros
 #pragma unroll
                     for (int i = 0; i < LPW; i++) {
-                        const char *from = next * BK + kpos[i] < p.K ? from_org + (off[i] + add) : reinterpret_cast<const char *>(ring_zero_words);
+                        const char *from = next * BK + kpos[i] < p.K ? from_org + (off[i] + add) + 1024 * (i & 3) : reinterpret_cast<const char *>(ring_zero_words);
                         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds1 + stage + i * 1024) : "memory");
                     }
                 }
@@ -156,13 +173,16 @@ __global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
                 }
             };
             static_assert(S <= 8, "landed() counts to six");
-            const int ahead = min(S - 1, nk);
+            // Products start when the first AHEAD tiles have been asked for, at 256 clocks a tile: enough of them to cover a trip to
+            // memory, and no more.
+            constexpr int AHEAD = S > 4 ? 5 : S - 1;
+            const int ahead = min(AHEAD, nk);
             for (int kt = 0; kt < ahead; kt++) request();
             landed(ahead - 1);
             barrier();                                    // tile 0 has landed
             int kt = 0;
             for (; next < nk; kt++) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 3) * LPW) : "memory");      // tile kt + 1 has landed
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 2) * LPW) : "memory");      // tile kt + 1 has landed
                 barrier();
                 request();
             }
@@ -171,140 +191,124 @@ __global__ __launch_bounds__(4 * 64 + 128) void gemm_ring_kernel(GemmArgs p) {
                 barrier();
             }
         };
-        if (wave == NW) load_all(std::integral_constant<int, 0>{});
+        if (wave == NW + 2) lnf_stats_wave<BM, BN, false>(p, reinterpret_cast<float2v *>(smem + S * STAGE_BYTES), m0, n0, bz, lane, nk, barrier);
+        else if (wave == NW) load_all(std::integral_constant<int, 0>{});
         else if constexpr (!CONV) load_all(std::integral_constant<int, 1>{});
         else if (p.cv.C % 64 == 0) load_all(std::integral_constant<int, 2>{});
         else load_all(std::integral_constant<int, 3>{});
         return;
     }
 
-    // fragment addresses of this wave's step of a tile
-    const int frow = lane & 31, h = lane >> 5, aswz = (frow & 7) ^ ((frow >> 3) & 1);
-    const uint32_t aoff = (uint32_t)(frow * 128 + (((2 * wave + h) ^ aswz) * 16));
-    uint32_t boff, noff[2];
-    if constexpr (!B_KN) boff = (uint32_t)(A_BYTES + frow * 128 + (((2 * wave + h) ^ aswz) * 16));
-    else boff = (uint32_t)(A_BYTES + (wave * 16 + h * 8 + ((lane & 15) >> 2)) * BN * 2);
+    // fragment addresses of this wave's 32 x 32 block, a 16-deep step of a tile each
+    constexpr int NKS = BK / 16;
+    const int sm = wave & 1, sn = wave >> 1;
+    const int frow = lane & 31, h = lane >> 5, aswz = (frow & 7) ^ ((frow >> 3) & 1), k3 = (lane & 15) >> 2;
+    const int n = sn * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    const uint32_t noff = (uint32_t)((((n >> 3) ^ (k3 * (BN / 32))) * 16) + (n & 7) * 2);
+    uint32_t aoff[NKS], boff[NKS];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int n = i * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4, k3 = (lane & 15) >> 2;
-        noff[i] = (uint32_t)((((n >> 3) ^ (k3 * (BN / 32))) * 16) + (n & 7) * 2);
+    for (int ks = 0; ks < NKS; ks++) {
+        const uint32_t chunk = (uint32_t)(((2 * ks + h) ^ aswz) * 16);
+        aoff[ks] = (sm * 32 + frow) * 128 + chunk;
+        if constexpr (!B_KN) boff[ks] = A_BYTES + (sn * 32 + frow) * 128 + chunk;
+        else boff[ks] = (uint32_t)(A_BYTES + (ks * 16 + h * 8 + k3) * BN * 2) + noff;
     }
-    half8v fa[2][2], fb[2][2];
+    half8v fa[2][NKS], fb[2][NKS];
     auto fetch = [&](auto SET, int kt) {
         constexpr int set = decltype(SET)::value;
         const char *st = smem + (kt % S) * STAGE_BYTES;
 #pragma unroll
-        for (int j = 0; j < 2; j++) fa[set][j] = *reinterpret_cast<const half8v *>(st + aoff + j * 32 * 128);
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            if constexpr (!B_KN) fb[set][i] = *reinterpret_cast<const half8v *>(st + boff + i * 32 * 128);
+        for (int ks = 0; ks < NKS; ks++) {
+            fa[set][ks] = *reinterpret_cast<const half8v *>(st + aoff[ks]);
+            if constexpr (!B_KN) fb[set][ks] = *reinterpret_cast<const half8v *>(st + boff[ks]);
             else {
-                const char *b = st + boff + noff[i];
+                const char *b = st + boff[ks];
                 const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)b);
                 const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(b + 4 * BN * 2));
                 const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                fb[set][i] = __builtin_bit_cast(half8v, both);
+                fb[set][ks] = __builtin_bit_cast(half8v, both);
             }
         }
     };
-    float16v acc[2][2];
+    float16v acc[1][1];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    for (int r = 0; r < 16; r++) acc[0][0][r] = 0.0f;
     auto products = [&](auto SET) {
         constexpr int set = decltype(SET)::value;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][i], fa[set][j], acc[i][j], 0, 0, 0);
+        for (int ks = 0; ks < NKS; ks++) acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][ks], fa[set][ks], acc[0][0], 0, 0, 0);
     };
 
-    // what the store needs of memory, while the first tiles are on their way: wave w stores the 32 x 32 block (w % 2, w / 2)
-    const int sm = wave & 1, sn = wave >> 1;
+    // what the store needs of memory, while the first tiles are on their way
     half4v cb[1][4];
     load_col_bias<1, 32>(p, cb, n0, sn, lane, bz);
-    float2v *ln_slot = reinterpret_cast<float2v *>(smem + S * STAGE_BYTES);
-    LnfLoader<BM, BN, NT, 10> lnf;                       // four lanes a row: K <= 1280 in one request
-    lnf.request(p, m0, n0, bz, tid);
+    // (two workgroups a CU have no registers to spare for the residual, and each other to hide behind)
+    ResidualAhead<32> res;
+    if constexpr (S > 4) res.request(p, m0 + sm * 32, n0 + sn * 32, lane, bz);
+    const float2v *ln_slot = reinterpret_cast<const float2v *>(smem + S * STAGE_BYTES);
     barrier();
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
-    fetch(I0{}, 0);
     // Tile kt's fragments are in registers (or on their way) when its turn comes: past the barrier its successor has landed and
     // its predecessor's stage is free for the loaders; the successor's fragments are requested, then its products issued.
+    // (The steady state has no branch: where a tile may or may not have a successor, the compiler's wait for its fragments is also
+    // one for the successor's, and a turn is longer by an LDS latency.)
     auto turn = [&](auto SET, auto NEXT, int kt) {
-        if (kt + 1 < nk) {
-            barrier();
-            fetch(NEXT, kt + 1);
-        }
+        barrier();
+        fetch(NEXT, kt + 1);
+        __builtin_amdgcn_sched_barrier(0);                // the reads go out ahead of the products,
         products(SET);
+        __builtin_amdgcn_sched_barrier(0);                // which stay ahead of the next barrier: by then this tile has been read
     };
-    int kt = 0;
-    for (; kt + 1 < nk; kt += 2) {
+    // (an odd tile comes first: one way into the loop and one out of it, or the accumulators are copied between registers)
+    if (nk & 1) {
+        fetch(I1{}, 0);
+        if (nk > 1) turn(I1{}, I0{}, 0);
+    } else fetch(I0{}, 0);
+    int kt = nk & 1;
+    for (; kt + 2 < nk; kt += 2) {
         turn(I0{}, I1{}, kt);
         turn(I1{}, I0{}, kt + 1);
     }
-    if (kt < nk) turn(I0{}, I1{}, kt);
+    if (nk > 1) turn(I0{}, I1{}, kt);
+    products(I1{});
 
-    lnf.combine(p, ln_slot, m0, tid);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    barrier();                                            // every wave has read its last fragments
-    // Partial tiles go to LDS by owner -- wave w keeps block acc[w / 2][w % 2] -- and are added in wave order.
-    float *part = reinterpret_cast<float *>(smem);
-#pragma unroll
-    for (int o = 0; o < NW; o++) {
-        if (o != wave) {
-            const int from = wave < o ? wave : wave - 1;
-            const float16v v = acc[o >> 1][o & 1];
-#pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) {
-                const float4v q = {v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]};
-                *reinterpret_cast<float4v *>(part + (o * (NW - 1) + from) * 1024 + r4 * 256 + lane * 4) = q;
-            }
-        }
+    // Past its last barrier of the loop a wave knows that every wave has read all tiles but the last two.  The store's staging keeps
+    // clear of their stages where the ring has room for it elsewhere.
+    constexpr int STAGING = NW * 2 * 32 * 40 * 2;
+    char *staging = smem;
+    if constexpr (S > 4) {
+        static_assert((S - 1) * STAGE_BYTES - STAGING >= STAGING + STAGE_BYTES, "above the last tile's stage, or below the one before it");
+        const int l = (nk - 1) % S;
+        if ((l + 1) * STAGE_BYTES + STAGING <= S * STAGE_BYTES) staging = smem + (l + 1) * STAGE_BYTES;
+    } else {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier();                                        // every wave has read its last fragments
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    barrier();
-    float16v own[1][1], mine = acc[0][0];
-#pragma unroll
-    for (int o = 0; o < NW; o++) if (o == wave) mine = acc[o >> 1][o & 1];
-#pragma unroll
-    for (int r = 0; r < 16; r++) own[0][0][r] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < NW; s++) {
-        if (s == wave) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) own[0][0][r] += mine[r];
-        } else {
-            const int from = s < wave ? s : s - 1;
-#pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) {
-                const float4v q = *reinterpret_cast<const float4v *>(part + (wave * (NW - 1) + from) * 1024 + r4 * 256 + lane * 4);
-#pragma unroll
-                for (int e = 0; e < 4; e++) own[0][0][4 * r4 + e] += q[e];
-            }
-        }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    barrier();                                            // the store's staging reuses the partial tiles' memory
     LnFold<1> ln;
     if (p.lnf_stats) {
         const float2v v = ln_slot[sm * 32 + frow];
         ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
     }
-    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, own, cb, smem, m0, n0, sm, sn, wave, lane, bz, ln);
+    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, acc, cb, staging, m0, n0, sm, sn, wave, lane, bz, ln, S > 4 ? &res : nullptr);
 }
 
 constexpr int ring_lds_bytes(int S) { return S * 2 * 8192 + 2 * 64 * 8; }
 
 template <int S, bool B_KN, bool CONV>
 int launch_ring(const GemmArgs &a, int64_t nbatch, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(4 * 64 + 128), ring_lds_bytes(S), st, a);
+    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(a.lnf_stats ? 448 : 384), ring_lds_bytes(S), st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
+template <bool CONV>
+int launch_stages(const GemmArgs &a, bool b_kn, bool deep, int64_t nbatch, hipStream_t st) {
+    if constexpr (!CONV) {
+        if (b_kn) return deep ? launch_ring<8, true, false>(a, nbatch, st) : launch_ring<4, true, false>(a, nbatch, st);
+    }
+    return deep ? launch_ring<8, false, CONV>(a, nbatch, st) : launch_ring<4, false, CONV>(a, nbatch, st);
+}
+template <bool B_KN, bool CONV>
+int raise_ring() { return raise_lds(gemm_ring_kernel<8, B_KN, CONV>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, B_KN, CONV>, ring_lds_bytes(4)); }
 
 }  // namespace
 
@@ -314,16 +318,16 @@ int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t 
     a.vec_store = rows_vec16(a);
     // per-lane load offsets are 32-bit byte offsets from the tile's origin (patches: from the image's)
     if ((int64_t)64 * a.ldA * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+    // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
+    const bool deep = (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus();
     if (a.cv.xp) {
         if (b_kn || a.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
-        // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
-        return (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus() ? launch_ring<8, false, true>(a, nbatch, st) : launch_ring<4, false, true>(a, nbatch, st);
+        return launch_stages<true>(a, false, deep, nbatch, st);
     }
     if ((int64_t)64 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
-    return b_kn ? launch_ring<8, true, false>(a, nbatch, st) : launch_ring<8, false, false>(a, nbatch, st);
+    return launch_stages<false>(a, b_kn, deep, nbatch, st);
 }
 
 int mi_ring_init() {
-    return raise_lds(gemm_ring_kernel<8, true>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<8, false>, ring_lds_bytes(8)) |
-           raise_lds(gemm_ring_kernel<8, false, true>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, false, true>, ring_lds_bytes(4));
+    return raise_ring<false, true>() | raise_ring<true, false>() | raise_ring<false, false>();
 }
