@@ -1264,7 +1264,9 @@ Route route_of(const SdpaArgs &a) {
     const int path = sdpa_path(a);
     if (path == MI_SDPA_DECLINE) return {MI_SDPA_KERNEL_NONE, 0, 1};
     // (at head size 72 an fp32 result would be 5 % further from exact on the tiles: flash_tile_kernel)
-    if (flash_operands_ok(a) && mi_sdpa_tile_takes(a) && !(path == MI_SDPA_ROWS && a.E == 72 && a.out_f32)) {
+    // (a mask that differs from query to query, of a form the fused kernel carries, stays with it)
+    const bool fused_mask = path == MI_SDPA_FLASH && a.bias && !mi_sdpa_tile_keymask(a);
+    if (flash_operands_ok(a) && mi_sdpa_tile_takes(a) && !fused_mask && !(path == MI_SDPA_ROWS && a.E == 72 && a.out_f32)) {
         const int waves = flash_tile_waves(a.E, a.Lq, a.Lk, a.H, a.B, path == MI_SDPA_ROWS);
         if (waves) return {path == MI_SDPA_ROWS ? MI_SDPA_KERNEL_TILES_F32 : MI_SDPA_KERNEL_TILES, waves, 1};
     }

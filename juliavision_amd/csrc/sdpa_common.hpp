@@ -40,5 +40,6 @@ __device__ __forceinline__ void static_for(F &&f) {
 constexpr int MI_SDPA_TILE_KEYMASK_MAX = 4096;
 bool mi_sdpa_tile_head_size(int64_t E);
 bool mi_sdpa_tile_takes(const SdpaArgs &p);
+bool mi_sdpa_tile_keymask(const SdpaArgs &p);
 int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st);
 int mi_sdpa_tile_init();

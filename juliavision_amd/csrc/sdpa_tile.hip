@@ -21,8 +21,14 @@ namespace {
 // four rows of a transposing read do.  Rows of nine chunks (72) need none for K.
 //
 // Products, register layouts and the lazily moved reference point M are flash_fwd_kernel's: S^T = K Q^T, O^T = V^T P^T, -M in
-// the first product's accumulators.  MASK: an fp16 mask of the key alone, copied to LDS once; it joins in one more k-step
-// as (mask, mask) x (log2(e) split into two positive fp16 parts), so that -inf stays -inf.
+// the first product's accumulators. 
+//
+// KEYS, DENSE: what a mask is.  KEYS: fp16 and of the key alone, copied to LDS once; it joins in one more k-step as (mask, mask) x
+// (log2(e) split into two positive fp16 parts), so that -inf stays -inf.  DENSE (with F32): anything else -- any strides, addresses
+// and either type -- read a tile ahead, a lane the sixteen values of its query, and added to the scores in fp32.  The loads are the
+// compiler's, whose waits know nothing of the requests: they are waited for where K has had a tile's time to land, before V is
+// asked for.  Such calls went to a workgroup per query row: 5 x 12 x 3559 x 3559 x 16 11 170 us, 6 x 20 x 189 x 189 x 16 88 -> 8.6,
+// 14 x 12 x 53 x 53 x 64 22 -> 6.9, 4 x 4 x 77 x 3238 57 -> 22, 4 x 6 x 257 x 257 35 -> 9.7.
 //
 // F32: calls of few queries, which the rows kernel answers with its scores and probabilities in fp32.  Nothing is rounded to fp16
 // here either: Q goes into the product as it lies and the scale joins the scores in fp32 (with the mask, times log2(e), from
@@ -33,11 +39,13 @@ namespace {
 // 72 it is larger, 1.57e-7 | 1.65e-7: there fp32 results stay with the rows kernel (fp16 ones are off by their rounding, 2.1e-4,
 // either way).
 // Waves a SIMD that the registers of an instance are budgeted for.
-constexpr int tile_waves(int EC, bool F32) { return EC == 16 ? 2 : EC == 9 ? (F32 ? 2 : 3) : EC == 8 && F32 ? 3 : 4; }
+enum TileMask { NO_MASK, KEYS, DENSE };
+constexpr int tile_waves(int EC, bool F32, int MASK) { return EC == 16 ? 2 : EC == 9 ? (F32 ? 2 : 3) : EC == 8 && F32 ? (MASK == DENSE ? 2 : 3) : MASK == DENSE ? 3 : 4; }
 
-template <int EC, int NW, bool MASK, bool F32>
-__global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kernel(SdpaArgs p) {
+template <int EC, int NW, int MASK, bool F32>
+__global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile_kernel(SdpaArgs p) {
     typedef std::conditional_t<F32, float, half_t> mask_t;
+    static_assert(MASK != DENSE || F32, "calls with fp16 probabilities and such a mask run flash_fwd_kernel");
     constexpr int E = EC * 8, KS = (E + 15) / 16, ET = (E + 31) / 32;
     constexpr int TILE_BYTES = 32 * EC * 16, NI = (32 * EC + 63) / 64;      // one operand's tile; 1 KB requests for it
     constexpr int WPART = (ET * 16 + 2) * 256, WSTRIDE = WPART > 2 * TILE_BYTES ? WPART : 2 * TILE_BYTES;
@@ -113,7 +121,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
         }
     };
     if (wave < nt) { request(true, wave); request(false, wave); }
-    if constexpr (MASK) {
+    if constexpr (MASK == KEYS) {
         const unsigned short *mrow = reinterpret_cast<const unsigned short *>(p.bias) + (long)h * p.bs[2] + (long)b * p.bs[3];
         for (int i = threadIdx.x; i < nt * 32; i += NW * 64) {
             const half_t m = __builtin_bit_cast(half_t, i < p.Lk ? mrow[(long)i * p.bs[0]] : (unsigned short)0);
@@ -135,7 +143,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
     for (int t = 0; t < ET; t++) o_acc[t] = negm;
     float m_run = F32 ? 0.0f : -INFINITY, l_run = 0.0f;           // no reference point yet: negm is 0
     half8v qext;
-    if constexpr (MASK) {
+    if constexpr (MASK == KEYS) {
 #pragma unroll
         for (int j = 0; j < 8; j++) qext[j] = (half_t)0.0f;
         if (hl == 0) { qext[0] = (half_t)1.4423828125f; qext[1] = (half_t)(1.44269504088896340736f - 1.4423828125f); }
@@ -156,6 +164,58 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
             l += p0 + p1;
         }
     };
+    // DENSE: the lane's sixteen values of a tile, keys 32 tile + 8 g + 4 hl .. +3, raw as they lie in memory (g holds four values:
+    // four words of fp32, two of fp16).  A tile that the keys end in, and keys apart in memory, are read by element, past the end
+    // the last one again: such keys' scores are cut.
+    u32x4 mraw[MASK == DENSE ? 4 : 1];
+    const char *drow = nullptr;
+    if constexpr (MASK == DENSE) drow = reinterpret_cast<const char *>(p.bias) + ((long)min(q0 + l32, p.Lq - 1) * p.bs[1] + (long)h * p.bs[2] + (long)b * p.bs[3]) * (p.bias_f32 ? 4 : 2);
+    auto mask_load = [&](int tile) {
+        const bool run = p.bs[0] == 1 && tile * 32 + 32 <= p.Lk;          // uniform
+        if (p.bias_f32) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int key = tile * 32 + 8 * g + 4 * hl;
+                if (run) __builtin_memcpy(&mraw[g], drow + (long)key * 4, 16);
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) mraw[g][e] = reinterpret_cast<const uint32_t *>(drow)[(long)min(key + e, p.Lk - 1) * p.bs[0]];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int key = tile * 32 + 8 * g + 4 * hl;
+                if (run) {
+                    u32x2 t;
+                    __builtin_memcpy(&t, drow + (long)key * 2, 8);      // at any address
+                    mraw[g][0] = t[0]; mraw[g][1] = t[1];
+                } else {
+                    unsigned short t[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t[e] = reinterpret_cast<const unsigned short *>(drow)[(long)min(key + e, p.Lk - 1) * p.bs[0]];
+                    mraw[g][0] = t[0] | (uint32_t)t[1] << 16; mraw[g][1] = t[2] | (uint32_t)t[3] << 16;
+                }
+            }
+        }
+    };
+    float16v ms;                                                  // times log2(e)
+    auto mask_take = [&]() {
+        if (p.bias_f32) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) { const uint32_t w = mraw[r >> 2][r & 3]; ms[r] = __builtin_bit_cast(float, w) * LOG2E; }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const uint32_t w = mraw[r >> 2][(r & 3) >> 1];
+                const half2v t = __builtin_bit_cast(half2v, w);
+                ms[r] = (float)t[0] * LOG2E; ms[r + 1] = (float)t[1] * LOG2E;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) asm volatile("" : "+v"(ms[r]));      // here, not where they are used
+    };
+    if constexpr (MASK == DENSE) { if (wave < nt) { mask_load(wave); mask_take(); } }
     bool first = true;
     // Keys that a finite mask excludes (finfo.min: -94 498 here) do not settle M, which scores formed against it would pay with
     // their last bits: see flash_fwd_kernel's FLOOR.
@@ -169,21 +229,23 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
         for (int ks = 0; ks < KS; ks++)
             kf[ks] = *reinterpret_cast<const half8v *>(kt_lds + (l32 * EC + (min(2 * ks + hl, EC - 1) ^ kswz(l32))) * 16);
         half8v kx = {};
-        float16v ms;
-        if constexpr (MASK && F32) {
+        if constexpr (MASK == KEYS && F32) {
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const float4v m = *reinterpret_cast<const float4v *>(Ms + tile * 32 + 8 * g + 4 * hl);
 #pragma unroll
                 for (int e = 0; e < 4; e++) ms[4 * g + e] = m[e];
             }
-        } else if constexpr (MASK) {
+        } else if constexpr (MASK == KEYS) {
             const half_t m = Ms[tile * 32 + l32];
             kx[0] = hl == 0 ? m : (half_t)0.0f;
             kx[1] = kx[0];
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (more) request(true, tile + NW);
+        if (more) {
+            request(true, tile + NW);
+            if constexpr (MASK == DENSE) mask_load(tile + NW);
+        }
         float16v sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[0], qf[0], negm, 0, 0, 0);
 #pragma unroll
         for (int ks = 1; ks < KS; ks++) {
@@ -193,7 +255,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
                 for (int r = 0; r < 16; r++) sc[r] += part[r];
             } else sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
         }
-        if constexpr (MASK && !F32) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
+        if constexpr (MASK == KEYS && !F32) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
         const float16v raw = sc;
         auto scale = [&]() {
 #pragma unroll
@@ -248,6 +310,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32)) void flash_tile_kerne
             first = first && !grow;                               // the reference point is found with the first key that counts
         }
         l_run = l_new;
+        if constexpr (MASK == DENSE) { if (more) mask_take(); }
         if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");        // V has landed; the next K may be on its way
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         half8v vf[ET][2];
@@ -333,22 +396,27 @@ constexpr int tile_lds_bytes() {
     return NW * (part > tiles ? part : tiles);
 }
 template <int EC, int NW, bool F32>
-int launch_tiles(const SdpaArgs &p, bool mask, hipStream_t st) {
+int launch_tiles(const SdpaArgs &p, TileMask mask, hipStream_t st) {
     const dim3 grid((unsigned)ceil_div(p.Lq, 32), (unsigned)p.H, (unsigned)p.B);
     const int lds = tile_lds_bytes<EC, NW>();
-    if (mask) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, true, F32>), grid, dim3(NW * 64), lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st, p);
-    else      hipLaunchKernelGGL((flash_tile_kernel<EC, NW, false, F32>), grid, dim3(NW * 64), lds, st, p);
+    if (mask == KEYS)       hipLaunchKernelGGL((flash_tile_kernel<EC, NW, KEYS, F32>), grid, dim3(NW * 64), lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st, p);
+    else if (mask == DENSE) {
+        if constexpr (F32) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, DENSE, true>), grid, dim3(NW * 64), lds, st, p);
+        else return MI_DECLINE_BIAS;
+    }
+    else                    hipLaunchKernelGGL((flash_tile_kernel<EC, NW, NO_MASK, F32>), grid, dim3(NW * 64), lds, st, p);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 template <int EC, bool F32>
-int launch_waves(const SdpaArgs &p, int waves, bool mask, hipStream_t st) {
+int launch_waves(const SdpaArgs &p, int waves, TileMask mask, hipStream_t st) {
     return waves == 2 ? launch_tiles<EC, 2, F32>(p, mask, st) : waves == 4 ? launch_tiles<EC, 4, F32>(p, mask, st) : launch_tiles<EC, 8, F32>(p, mask, st);
 }
 template <int EC, int NW, bool F32>
 int raise() {
     const int lds = tile_lds_bytes<EC, NW>();
-    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, true, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + (F32 ? 4 : 2) * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
-           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, false, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
+    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, KEYS, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + (F32 ? 4 : 2) * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
+           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, DENSE, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) |
+           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, NO_MASK, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
 }
 template <int EC>
 int raise_all() { return raise<EC, 2, false>() | raise<EC, 4, false>() | raise<EC, 8, false>() | raise<EC, 2, true>() | raise<EC, 4, true>() | raise<EC, 8, true>(); }
@@ -358,17 +426,19 @@ int raise_all() { return raise<EC, 2, false>() | raise<EC, 4, false>() | raise<E
 // Head sizes: those of this package's models and tests.  The chunk permutations hold for rows of 2, 4, 8, 9 and 16 chunks; 40, 48, 80,
 // 96 and the rest run the padded forms of flash_fwd_kernel, which no figure here has been taken against.
 bool mi_sdpa_tile_head_size(int64_t E) { return E == 16 || E == 32 || E == 64 || E == 72 || E == 128; }
+// An fp16 mask of the key alone whose row fits the LDS is copied there; one that differs from query to query is read where it lies.  (An
+// fp32 one of the key alone keeps the rows kernel, the fused one its own blocks.)
+bool mi_sdpa_tile_keymask(const SdpaArgs &p) { return p.bias && !p.bias_f32 && (p.bs[1] == 0 || p.Lq == 1) && p.Lk <= MI_SDPA_TILE_KEYMASK_MAX; }
 bool mi_sdpa_tile_takes(const SdpaArgs &p) {
     if (!mi_sdpa_tile_head_size(p.E)) return false;
-    // an fp16 mask of the key alone, whose row fits the LDS
-    if (p.bias && (p.bias_f32 || (p.bs[1] != 0 && p.Lq != 1) || p.Lk > MI_SDPA_TILE_KEYMASK_MAX)) return false;
+    if (p.bias && !mi_sdpa_tile_keymask(p) && p.bs[1] == 0) return false;
     // per-lane load offsets are 32-bit byte offsets from a tile's first row
     return p.ks[1] >= 0 && p.vs[1] >= 0 && p.ks[1] * 64 < (1l << 31) && p.vs[1] * 64 < (1l << 31);
 }
 
 int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st) {
     if (!mi_sdpa_tile_takes(p)) return MI_DECLINE_EXTENT;
-    const bool mask = p.bias != nullptr;
+    const TileMask mask = !p.bias ? NO_MASK : mi_sdpa_tile_keymask(p) ? KEYS : DENSE;
     switch (p.E) {
     case 16: return f32 ? launch_waves<2, true>(p, waves, mask, st) : launch_waves<2, false>(p, waves, mask, st);
     case 32: return f32 ? launch_waves<4, true>(p, waves, mask, st) : launch_waves<4, false>(p, waves, mask, st);
