@@ -1197,21 +1197,22 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
 // workgroups overlap).  A K that ends inside a tile makes every step `tail` times as long: its rows are no multiple of
 // a cache line, so most 128-byte pieces of them touch two.  A GELU store adds `gelu` a round.  A split adds the second
 // launch (4.4 us) and the fp32 planes (0.38 us per MB).
-// Fitted to every tile timed on 150 shapes in a replayed graph (M 9..4096, N 64..5120, K 72..5120, both layouts, a third of
-// them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.5 % of the best measured tile on average.
+// Fitted to every tile timed on 260 shapes in a replayed graph (M 9..8192, N 64..8192, K 72..5120, both layouts, a third of
+// them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.4 % of the best measured tile on average,
+// 15 % at worst (259 x 1728 -> 3584 with GELU).
 // What it replaced sent every K % 64 to 64 x 64 tiles: 1544 x 1288 -> 1288 with residual 19.8 -> 15.4 us on 128 x 128,
 // 636 x 4392 -> 104 23.2 -> 13.8 on the ring, 2237 x 5096 -> 2440 with GELU 143 -> 80 on 192 x 128.
 struct TileModel { int bm, bn; double step_lo, step_full, round, fixed, gelu, tail; };
 constexpr int NTILES = 6;
 constexpr TileModel TILE_MODELS[NTILES] = {
-    {128, 256, 0.458, 0.779, 1.04, 5.88, 2.8, 1.48},
-    {192, 128, 0.376, 0.655, 1.07, 4.96, 2.22, 1.41},
-    {128, 128, 0.436, 0.614, 1.11, 4.1, 1.93, 1.08},
-    {64, 128, 0.33, 0.411, 0.818, 3.51, 1.01, 1.16},
-    {64, 64, 0.255, 0.326, 0.617, 3.29, 0.533, 1.22},
-    {64, 64, 0.153, 0.219, 0.775, 3.46, 0.494, 1.41},      // gemm_ring_kernel
+    {128, 256, 0.453, 0.746, 1.02, 6.1, 2.89, 1.41},
+    {192, 128, 0.369, 0.613, 1.03, 5.19, 2.17, 1.38},
+    {128, 128, 0.457, 0.568, 1.09, 4.27, 1.86, 1.13},
+    {64, 128, 0.315, 0.394, 0.841, 3.47, 0.946, 1.17},
+    {64, 64, 0.267, 0.302, 0.632, 3.04, 0.423, 1.2},
+    {64, 64, 0.135, 0.22, 0.818, 3.28, 0.362, 1.3},      // gemm_ring_kernel
 };
-constexpr int64_t RING_WGS_PER_CU = 6;       // as many as the fit has seen
+constexpr int64_t RING_WGS_PER_CU = 11;      // as many as the fit has seen
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
