@@ -26,6 +26,17 @@ MI_DEVICE u32x2 ldg8(const half_t *p) { return *reinterpret_cast<const u32x2 *>(
 MI_DEVICE uint32_t pack_lo(uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x05040100u); }
 MI_DEVICE uint32_t pack_hi(uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x07060302u); }
 
+// x / d and what is left, with recip = recip_of(d) from the host: the product's upper half is the quotient or one less, for every 32-bit
+// dividend, and no case needs a branch.  A division by a value that arrives with the launch is some thirty instructions.
+MI_DEVICE unsigned divide(unsigned x, unsigned d, unsigned recip, unsigned &left) {
+    unsigned q = __umulhi(x, recip), r = x - q * d;
+    const bool up = r >= d;
+    q += up ? 1u : 0u;
+    left = r - (up ? d : 0u);
+    return q;
+}
+static inline unsigned recip_of(int64_t d) { return (unsigned)(0xffffffffll / d); }
+
 MI_DEVICE half8v as_half8(u32x4 v) { return __builtin_bit_cast(half8v, v); }
 
 // Lane exchanges without the LDS crossbar.  lane_xor<O>(v) is v of lane (lane ^ O) for O = 1, 2, 4, 8: data-parallel

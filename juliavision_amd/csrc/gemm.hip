@@ -537,12 +537,19 @@ __device__ __forceinline__ u32x4 ln_apply8(const GemmArgs &p, u32x4 raw, float m
     return __builtin_bit_cast(u32x4, o);
 }
 
+// stage_args for the decode-sized kernels
+__device__ __forceinline__ void stage_skinny(const GemmArgs &p) {
+    asm volatile("" ::"s"(p.A), "s"(p.B), "s"(p.ldA), "s"(p.ldB), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.bias_mode), "s"(p.epi), "s"(p.Y), "s"(p.ldY), "s"(p.bias),
+                 "s"(p.residual), "s"(p.out_f32), "s"(p.ln_gamma), "s"(p.ln_beta), "s"(p.ln_eps), "s"(p.ln_on), "s"(p.div_k8));
+}
+
 constexpr int SKN_COLS = 128;      // columns per workgroup
 constexpr int SKN_KMAX = 256;      // deepest k-slice: 16 loads of 16 bytes per thread, all in flight at once
 constexpr int SKN_LOADS = SKN_KMAX / 32;
 
 template <int MT>
 __global__ __launch_bounds__(256) void skinny_kn_kernel(GemmArgs p, float *part, int kper) {
+    stage_skinny(p);
     __shared__ __align__(16) half_t xs[MT][SKN_KMAX];
     __shared__ float red[4][MT][SKN_COLS];
     __shared__ float lnst[MT][2];
@@ -661,6 +668,7 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     constexpr int FK_XCAP = MT == 8 ? 1 : 4;              // eight rows of accumulators and operands leave room for one
     constexpr int FK_XPF = (MT * FK_PF * 64 + 255) / 256 < FK_XCAP ? (MT * FK_PF * 64 + 255) / 256 : FK_XCAP;
     extern __shared__ __align__(16) char smem[];
+    stage_skinny(p);
     half_t *xs = reinterpret_cast<half_t *>(smem);       // [MT][K]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ float lnst[MT][2];
@@ -681,7 +689,8 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     u32x4 xr[FK_XPF], gr[FK_XPF], br[FK_XPF];
 #pragma unroll
     for (int i = 0; i < FK_XPF; i++) {
-        const int c = tid + 256 * i, m = c / kch, ch = c % kch;
+        unsigned ch;
+        const int c = tid + 256 * i, m = (int)divide(c, kch, p.div_k8, ch);
         xr[i] = gr[i] = br[i] = z;
         if (c < MT * kch && m < p.M) {
             xr[i] = ldg16(p.A + (long)m * p.ldA + ch * 8);
@@ -695,7 +704,8 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < FK_XPF; i++) {
-        const int c = tid + 256 * i, m = c / kch, ch = c % kch;
+        unsigned ch;
+        const int c = tid + 256 * i, m = (int)divide(c, kch, p.div_k8, ch);
         if (c < MT * kch) {
             u32x4 v = xr[i];
             if (p.ln_on && m < p.M) {
@@ -710,7 +720,8 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
         }
     }
     for (int c = tid + 256 * FK_XPF; c < MT * kch; c += 256) {
-        const int m = c / kch, ch = c % kch;
+        unsigned ch;
+        const int m = (int)divide(c, kch, p.div_k8, ch);
         u32x4 v = z;
         if (m < p.M) {
             v = ldg16(p.A + (long)m * p.ldA + ch * 8);
@@ -801,6 +812,7 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
 // two waves and stay with the staged kernel.
 template <int MT, int PF, int R>
 __global__ __launch_bounds__(256) void skinny_fk_reg_kernel(GemmArgs p) {
+    stage_skinny(p);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const u32x4 z = {0u, 0u, 0u, 0u};
     const int n0 = (blockIdx.x * 4 + wave) * R;
@@ -1389,7 +1401,7 @@ int fill_args(GemmArgs &a, void *Y, const void *X, const void *W, const void *bi
     a.tiles_m = a.tiles_n = a.group_m = 1; a.vec_store = 0;
     a.cv = ConvGather{};
     a.ag = NhwcGather{};
-    a.ln_gamma = a.ln_beta = nullptr; a.ln_eps = 0.0f; a.ln_on = 0;
+    a.ln_gamma = a.ln_beta = nullptr; a.ln_eps = 0.0f; a.ln_on = 0; a.div_k8 = K >= 8 ? recip_of(K / 8) : 0;
     a.lnout = nullptr; a.lnout_gamma = a.lnout_beta = nullptr; a.lnout_eps = 0.0f; a.clamp = 0.0f;
     a.clk = nullptr; a.phase = nullptr; a.phase_wgs = 0;
     a.sk_S = 0; a.sk_tpx = 0; a.sk_part = nullptr; a.sk_flags = nullptr; a.sk_epoch = 0;
@@ -1509,7 +1521,7 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     GemmArgs a;
     a.cv = ConvGather{};
     a.ag = NhwcGather{};
-    a.ln_gamma = a.ln_beta = nullptr; a.ln_eps = 0.0f; a.ln_on = 0;
+    a.ln_gamma = a.ln_beta = nullptr; a.ln_eps = 0.0f; a.ln_on = 0; a.div_k8 = K >= 8 ? recip_of(K / 8) : 0;
     a.lnout = nullptr; a.lnout_gamma = a.lnout_beta = nullptr; a.lnout_eps = 0.0f; a.clamp = 0.0f;
     a.clk = nullptr; a.phase = nullptr; a.phase_wgs = 0;
     a.sk_S = 0; a.sk_tpx = 0; a.sk_part = nullptr; a.sk_flags = nullptr; a.sk_epoch = 0;

@@ -46,6 +46,7 @@ struct GemmArgs {
     const half_t *ln_gamma, *ln_beta;
     float ln_eps;
     int ln_on;
+    unsigned div_k8;        // recip_of(K / 8)
     // Output side: when lnout is set, the rows of Y are also layer-normalised over N into lnout (dense rows of N
     // halves), as mi_layernorm_f16 on Y would write them (the next block's first norm riding in this GEMM's store).
     half_t *lnout;
@@ -93,26 +94,18 @@ __device__ __forceinline__ void stage_args(const GemmArgs &p) {
 // round-robin over the 8 XCDs, each with its own L2; this hands every XCD one
 // contiguous run of the tile order, and the tile order walks GROUP_M row tiles
 // per column tile so a run reuses a small set of A and B panels.
-// Its divisions are multiplications by reciprocals the host worked out (set_tiles): a division is some thirty instructions at
-// four to eight clocks each, and three of them in a row stood between a launch and its first load.  With r = floor((2^32 - 1) / d) the
-// product's upper half is the quotient or one less, for every 32-bit dividend, and no case needs a branch.
+// Its divisions are multiplications by reciprocals the host worked out (set_tiles, divide): three in a row stood between a launch and
+// its first load.
 __device__ __forceinline__ void tile_of(const GemmArgs &p, int &tm, int &tn) {
     const int pid = blockIdx.x, nwg = p.tiles_m * p.tiles_n;
     const int xcd = pid & 7, idx = pid >> 3;
     const int full = nwg >> 3, rem = nwg & 7;
     const int logical = xcd * full + min(xcd, rem) + idx;
-    const auto divide = [](unsigned x, unsigned d, unsigned recip, int &left) {
-        unsigned q = __umulhi(x, recip), r = x - q * d;
-        const bool up = r >= d;
-        q += up ? 1u : 0u;
-        left = (int)(r - (up ? d : 0u));
-        return (int)q;
-    };
-    int in;
-    const int first = divide(logical, p.group_m * p.tiles_n, p.div_width, in) * p.group_m;
+    unsigned in, row;
+    const int first = (int)divide(logical, p.group_m * p.tiles_n, p.div_width, in) * p.group_m;
     const int gsz = min(p.tiles_m - first, p.group_m);
-    tn = divide(in, gsz, gsz == p.group_m ? p.div_group : p.div_last, tm);
-    tm += first;
+    tn = (int)divide(in, gsz, gsz == p.group_m ? p.div_group : p.div_last, row);
+    tm = first + (int)row;
 }
 
 // The tile grid of a launch.
@@ -120,11 +113,10 @@ inline void set_tiles(GemmArgs &a, int bm, int bn) {
     a.tiles_m = (int)ceil_div(a.M, bm);
     a.tiles_n = (int)ceil_div(a.N, bn);
     a.group_m = a.tiles_m < 6 ? a.tiles_m : 6;
-    const auto recip = [](int64_t d) { return (unsigned)(0xffffffffll / d); };
     const int last = a.tiles_m % a.group_m;
-    a.div_width = recip((int64_t)a.group_m * a.tiles_n);
-    a.div_group = recip(a.group_m);
-    a.div_last = recip(last ? last : a.group_m);
+    a.div_width = recip_of((int64_t)a.group_m * a.tiles_n);
+    a.div_group = recip_of(a.group_m);
+    a.div_last = recip_of(last ? last : a.group_m);
 }
 
 // What the store of a folded norm needs, fetched while the first operand tiles are on their way and parked in `slot`

@@ -103,6 +103,7 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
     half_t (*Ks)[BCS * KLD] = reinterpret_cast<half_t (*)[BCS * KLD]>(smem);
     half_t (*Vs)[BCS * VLD] = reinterpret_cast<half_t (*)[BCS * VLD]>(smem + 3 * BCS * KLD * 2);
     half_t *Ms = reinterpret_cast<half_t *>(smem + 3 * BCS * (KLD + VLD) * 2);       // BIAS 3: the mask row, then zeros
+    stage_args(p);
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int tid = threadIdx.x & (NT - 1);                  // index among the staging threads
@@ -663,6 +664,7 @@ template <int NCH, bool VEC>
 __global__ __launch_bounds__(256) void sdpa_rows_kernel(SdpaArgs p) {
     __shared__ float red_ml[4][2];
     __shared__ float red_o[4][64 * NCH];
+    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 3, cl = lane & 7;
     const int split = blockIdx.x % p.nsplit;
@@ -854,15 +856,17 @@ __global__ __launch_bounds__(512) void sdpa_decode_kernel(SdpaArgs p) {
     __shared__ float red_ml[8][2];
     __shared__ float red_o[8][64];
     __shared__ int is_last;
+    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 3, cl = lane & 7;
     const int S = p.nsplit;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int split = slot % S, unit = (slot / S) * 8 + xcd;
+    unsigned split_, h_;
+    const int unit = (int)divide(slot, S, p.div_split, split_) * 8 + xcd, split = (int)split_;
     if (unit >= p.H * p.B) return;                       // the grid is padded to whole groups of 8 rows
-    const int h = unit % p.H, b = unit / p.H;
+    const int b = (int)divide(unit, p.H, p.div_h, h_), h = (int)h_;
     const int cap = p.Lk;
-    const int npass = (cap + 63) / 64, per = (npass + S - 1) / S;
+    const int npass = (cap + 63) >> 6, per = p.per;
     const int t_lo = split * per, t_hi = min(npass, t_lo + per);
     const half_t *qp = p.q + h * p.qs[2] + b * p.qs[3];
     half_t *kb = const_cast<half_t *>(p.k) + h * p.ks[2] + b * p.ks[3];
@@ -1228,6 +1232,8 @@ int launch_decode(SdpaArgs &a, hipStream_t st) {
             a.part_ml = a.part_o + (size_t)a.H * a.B * a.nsplit * a.E;
         }
     }
+    a.per = (int)ceil_div(ceil_div(a.Lk, 64), a.nsplit);
+    a.div_split = recip_of(a.nsplit);
     const unsigned units8 = (unsigned)ceil_div((int64_t)a.H * a.B, 8);
     hipLaunchKernelGGL(sdpa_decode_kernel, dim3(units8 * 8 * a.nsplit), dim3(512), 0, st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
@@ -1294,6 +1300,8 @@ int fill(SdpaArgs &a, void *out, int out_dtype, const int64_t *os, const void *q
     for (int i = 0; i < 4; i++) a.ns[i] = 0;
     a.E = (int)E; a.Lq = (int)Lq; a.Lk = (int)Lk; a.H = (int)H; a.B = (int)B;
     a.out_f32 = out_dtype == MI_F32; a.nsplit = 1; a.scale = scale;
+    a.nqb = 1; a.per = 0;
+    a.div_x = a.div_split = recip_of(1); a.div_h = recip_of(H < 1 ? 1 : H);
     return MI_OK;
 }
 

@@ -3,27 +3,39 @@
 #include "common.hpp"
 #include <type_traits>
 
+// The order is the kernels': see stage_args.
 struct SdpaArgs {
-    void *out;
     const half_t *q, *k, *v;
+    void *out;
+    int Lq, Lk, H, B;
+    unsigned div_h, div_x, div_split;      // recip_of(H), of the grid's query blocks (flash_tile_kernel: nqb), of nsplit
+    int nqb;                       // flash_tile_kernel: query blocks
     long qs[4], ks[4], vs[4], os[4];   // (E, L, H, B) element strides
+    int E, out_f32, bias_f32, nsplit;
+    float scale;
+    int per;                       // sdpa_decode_kernel: 64-key passes of a split
     const void *bias;
-    long bs[4];                    // (Lk, Lq, H, B) element strides, 0 = broadcast
     const int *kv_len;
-    float *part_o, *part_ml;       // split partials: [split][row][E], [split][row][2] (sdpa_decode_kernel: [row][split])
-    unsigned *tickets;             // sdpa_decode_kernel with nsplit > 1: one arrival counter per (head, batch), zero between launches
     // sdpa_decode_kernel only: the newest key/value row (1 x E per head and batch); when set, key kv_len - 1 is
     // taken from here instead of the cache and written into the cache on the way (k, v are then written to)
     const half_t *k_new, *v_new;
     long ns[4];
-    int E, Lq, Lk, H, B;
-    int out_f32, bias_f32, nsplit;
-    float scale;
+    unsigned *tickets;             // sdpa_decode_kernel with nsplit > 1: one arrival counter per (head, batch), zero between launches
+    float *part_o, *part_ml;       // split partials: [split][row][E], [split][row][2] (sdpa_decode_kernel: [row][split])
+    long bs[4];                    // (Lk, Lq, H, B) element strides, 0 = broadcast
 };
 
 namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
+
+// Asks for the argument block at once.  The compiler asks for a field where it is first used, a line of the block at a time and each a trip
+// of 200 (replayed graphs) to 700 clocks behind the other; four to six of them stood between these launches and their first load.
+__device__ __forceinline__ void stage_args(const SdpaArgs &p) {
+    asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.out), "s"(p.Lq), "s"(p.Lk), "s"(p.H), "s"(p.B), "s"(p.div_h), "s"(p.qs[2]), "s"(p.qs[3]),
+                 "s"(p.ks[1]), "s"(p.ks[2]), "s"(p.ks[3]), "s"(p.vs[1]), "s"(p.vs[2]), "s"(p.vs[3]), "s"(p.os[2]), "s"(p.os[3]), "s"(p.E),
+                 "s"(p.nsplit), "s"(p.scale), "s"(p.bias), "s"(p.kv_len), "s"(p.k_new), "s"(p.ns[3]), "s"(p.part_ml));
+}
 
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F &&f) {

@@ -51,6 +51,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
     constexpr int WPART = (ET * 16 + 2) * 256, WSTRIDE = WPART > 2 * TILE_BYTES ? WPART : 2 * TILE_BYTES;
     constexpr float UP = F32 ? 1024.0f : 1.0f, TH = F32 ? 4.0f : 8.0f;      // probabilities times UP stay in fp16 range
     extern __shared__ __align__(16) char smem[];
+    stage_args(p);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hl = lane >> 5, l32 = lane & 31;
     char *const wave_lds = smem + wave * WSTRIDE;
@@ -60,13 +61,12 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
     // workgroups are dealt to the 8 XCDs round robin: each gets a contiguous run, so a head's query tiles share an L2
     int qblk, h, b;
     {
-        const int nqb = gridDim.x, total = nqb * gridDim.y * gridDim.z;
-        int id = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-        const int xcd = id & 7, full = total >> 3, rem = total & 7;
-        id = xcd * full + min(xcd, rem) + (id >> 3);
-        qblk = id % nqb;
-        h = (id / nqb) % gridDim.y;
-        b = id / (nqb * gridDim.y);
+        const int total = p.nqb * p.H * p.B, xcd = blockIdx.x & 7, full = total >> 3, rem = total & 7;
+        unsigned x, y;
+        const unsigned hb = divide(xcd * full + min(xcd, rem) + (blockIdx.x >> 3), p.nqb, p.div_x, x);
+        b = divide(hb, p.H, p.div_h, y);
+        qblk = x;
+        h = y;
     }
     const int q0 = qblk * 32;
     const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];
@@ -397,7 +397,7 @@ constexpr int tile_lds_bytes() {
 }
 template <int EC, int NW, bool F32>
 int launch_tiles(const SdpaArgs &p, TileMask mask, hipStream_t st) {
-    const dim3 grid((unsigned)ceil_div(p.Lq, 32), (unsigned)p.H, (unsigned)p.B);
+    const dim3 grid((unsigned)(p.nqb * p.H * p.B));
     const int lds = tile_lds_bytes<EC, NW>();
     if (mask == KEYS)       hipLaunchKernelGGL((flash_tile_kernel<EC, NW, KEYS, F32>), grid, dim3(NW * 64), lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st, p);
     else if (mask == DENSE) {
@@ -432,12 +432,16 @@ bool mi_sdpa_tile_keymask(const SdpaArgs &p) { return p.bias && !p.bias_f32 && (
 bool mi_sdpa_tile_takes(const SdpaArgs &p) {
     if (!mi_sdpa_tile_head_size(p.E)) return false;
     if (p.bias && !mi_sdpa_tile_keymask(p) && p.bs[1] == 0) return false;
+    if (ceil_div(p.Lq, 32) * p.H * p.B > INT32_MAX) return false;
     // per-lane load offsets are 32-bit byte offsets from a tile's first row
     return p.ks[1] >= 0 && p.vs[1] >= 0 && p.ks[1] * 64 < (1l << 31) && p.vs[1] * 64 < (1l << 31);
 }
 
-int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st) {
-    if (!mi_sdpa_tile_takes(p)) return MI_DECLINE_EXTENT;
+int mi_sdpa_tile_launch(const SdpaArgs &args, int waves, bool f32, hipStream_t st) {
+    if (!mi_sdpa_tile_takes(args)) return MI_DECLINE_EXTENT;
+    SdpaArgs p = args;
+    p.nqb = (int)ceil_div(p.Lq, 32);
+    p.div_x = recip_of(p.nqb);
     const TileMask mask = !p.bias ? NO_MASK : mi_sdpa_tile_keymask(p) ? KEYS : DENSE;
     switch (p.E) {
     case 16: return f32 ? launch_waves<2, true>(p, waves, mask, st) : launch_waves<2, false>(p, waves, mask, st);
