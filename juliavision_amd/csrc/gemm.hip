@@ -472,10 +472,10 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
 // Layer-norm statistics of up to MT rows of A, one wave per row, in the summation order of
 // layernorm_vec_kernel (a lane takes the 16-byte chunks lane, lane + 64, ...; butterfly over the wave):
 // the fused result is bit-identical to running that kernel first.  stats[m] = (mean, rstd).
-template <int MT, int NCH = 8>                              // rows up to NCH * 512 halves stay in registers between the passes
+template <int MT, int NCH = 8, int NWAVES = 4>              // rows up to NCH * 512 halves stay in registers between the passes
 __device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2], int tid) {
     const int lane = tid & 63, wave = tid >> 6;
-    for (int m = wave; m < MT && m < p.M; m += 4) {
+    for (int m = wave; m < MT && m < p.M; m += NWAVES) {
         const half_t *row = p.A + (long)m * p.ldA;
         float s = 0.0f, s2 = 0.0f;
         if (p.K <= NCH * 512) {
@@ -665,8 +665,7 @@ __global__ void skinny_epilogue_kernel(GemmArgs p, const float *part, int nsplit
 template <int MT, int FK_PF>
 __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     // activation chunks per thread requested up front: the whole MT x K panel up to four per thread
-    constexpr int FK_XCAP = MT == 8 ? 1 : 4;              // eight rows of accumulators and operands leave room for one
-    constexpr int FK_XPF = (MT * FK_PF * 64 + 255) / 256 < FK_XCAP ? (MT * FK_PF * 64 + 255) / 256 : FK_XCAP;
+    constexpr int FK_XPF = (MT * FK_PF * 64 + 255) / 256 < 4 ? (MT * FK_PF * 64 + 255) / 256 : 4;
     extern __shared__ __align__(16) char smem[];
     stage_skinny(p);
     half_t *xs = reinterpret_cast<half_t *>(smem);       // [MT][K]
@@ -798,6 +797,110 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
 #pragma unroll
             for (int i = 0; i < FK_PF; i++) w[i] = wn[i];
             bv = bvn; rv = rvn;
+        }
+    }
+}
+
+// Five to eight rows: on the matrix cores.  A workgroup owns sixteen output columns (`cols`; eight where that gives more CUs work), its
+// eight waves an eighth of K each: the weight rows by 32 k are one operand of v_mfma_f32_16x16x32_f16, the activation rows the
+// other (zeros past either), both straight from memory in the layout the instruction wants -- a lane's sixteen bytes -- and all of a wave's share asked for at its first
+// lines (PF steps at a time).  The eight partial sums meet in LDS, in pairs.  With a norm in front a wave finds one row's statistics,
+// in layernorm_vec_kernel's order, and the fragments are normalised and rounded on their way into the product.
+// What bounds it is the trip to memory.  The kernel above staged M x K activations in every workgroup of four columns and read them back
+// once a column: 80 KB of LDS traffic a wave at 8 x 5120.
+template <int PF, bool LN>
+__global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
+    constexpr int NW = 8;
+    __shared__ float4v red[NW][64];
+    __shared__ float lnst[8][2];
+    stage_skinny(p);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = lane & 15, kq = lane >> 4, n0 = blockIdx.x * cols;
+    const int steps = (p.K + 31) >> 5, per = (steps + NW - 1) / NW, s0 = wave * per, s1 = min(steps, s0 + per);
+    const half_t *const wrow = p.B + (long)min(n0 + row, p.N - 1) * p.ldB, *const xrow = p.A + (long)min(row, p.M - 1) * p.ldA;
+    u32x4 w[PF], x[PF], g[LN ? PF : 1], b[LN ? PF : 1];
+    auto fetch = [&](int base) {
+#pragma unroll
+        for (int i = 0; i < PF; i++) {
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            const int k = (base + i) * 32 + kq * 8;
+            const bool on = base + i < s1 && k < p.K;
+            w[i] = on && row < cols ? ldg16(wrow + k) : z;
+            x[i] = on && row < p.M ? ldg16(xrow + k) : z;
+            if constexpr (LN) {
+                g[i] = on && p.ln_gamma ? ldg16(p.ln_gamma + k) : z;
+                b[i] = on && p.ln_beta ? ldg16(p.ln_beta + k) : z;
+            }
+        }
+    };
+    fetch(s0);
+    // what the store needs, by the wave that stores: lane (row, kq) holds columns n0 + 4 kq .. +3 of row `row`
+    const int n = n0 + 4 * kq;
+    const bool stores = wave == 0 && row < p.M && 4 * kq < cols;
+    float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, rv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (stores) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (n + e < p.N) {
+                if (p.bias_mode == MI_BIAS_COL) bv[e] = (float)p.bias[n + e];
+                else if (p.bias_mode == MI_BIAS_ROW) bv[e] = (float)p.bias[row];
+                if (p.residual && !p.out_f32) rv[e] = (float)p.residual[(long)row * p.ldY + n + e];
+            }
+        }
+    }
+    float mu = 0.0f, rs = 0.0f;
+    if constexpr (LN) {
+        ln_row_stats<8, 8, NW>(p, lnst, tid);
+        __syncthreads();
+        mu = lnst[min(row, p.M - 1)][0];
+        rs = lnst[min(row, p.M - 1)][1];
+    }
+    // five chains, step i of the share in chain i % 5 whatever PF is: short ones keep the error at that of the dot products below five rows
+    constexpr int NA = 5;
+    static_assert(PF % NA == 0, "one order of the sum, with a norm in front and without");
+    float4v acc[NA];
+#pragma unroll
+    for (int i = 0; i < NA; i++) acc[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int base = s0;;) {
+#pragma unroll
+        for (int i = 0; i < PF; i++) {
+            half8v xv = as_half8(x[i]);
+            if constexpr (LN) {
+                const half8v gv = as_half8(g[i]), be = as_half8(b[i]);
+#pragma unroll
+                for (int j = 0; j < 8; j++) xv[j] = ln_norm1((float)xv[j], mu, rs, p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)be[j]);
+            }
+            acc[i % NA] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(w[i]), xv, acc[i % NA], 0, 0, 0);      // (steps past the share multiply zeros)
+        }
+        if ((base += PF) >= s1) break;
+        fetch(base);
+    }
+#pragma unroll
+    for (int d = 1; d < NA; d *= 2)
+#pragma unroll
+        for (int i = 0; i + d < NA; i += 2 * d) acc[i] += acc[i + d];
+    red[wave][lane] = acc[0];
+    __syncthreads();
+    if (!stores) return;
+    float4v sum[NW];
+#pragma unroll
+    for (int q = 0; q < NW; q++) sum[q] = red[q][lane];
+#pragma unroll
+    for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+        for (int q = 0; q < NW; q += 2 * d) sum[q] += sum[q + d];
+    const float4v v = sum[0];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        if (n + e < p.N) {
+            const float t = v[e] + bv[e];
+            const long off = (long)row * p.ldY + n + e;
+            if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(t, p.epi);
+            else {
+                half_t o = (half_t)apply_epi((float)(half_t)t, p.epi);
+                if (p.residual) o = (half_t)((float)o + rv[e]);
+                reinterpret_cast<half_t *>(p.Y)[off] = o;
+            }
         }
     }
 }
@@ -1322,6 +1425,9 @@ int gemm_path(const GemmArgs &a, bool b_kn, int64_t nbatch) {
     return MI_GEMM_SCALAR;
 }
 
+// few_rows_kernel from five rows on (us at 4 and 8 rows, staged kernel | matrix cores; 1280 -> 5120 6.8 | 7.15 and 8.6 | 7.4; 4096 -> 1024
+// 6.4 | 7.1 and 10.3 | 7.9; 5120 -> 1280 8.9 | 8.2 and 20.4 | 9.0; 1280 -> 51866 35.8 | 35.0 and 48 | 38; 1536 -> 384 3.8 | 4.4 and 4.9 | 4.65).
+constexpr int FEW_ROWS_MIN = 5;
 int run_skinny(GemmArgs a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st) {
     if (b_kn) {
         const int kper = skinny_kper(a.K, a.N), nsplit = (int)ceil_div(a.K, kper);
@@ -1337,9 +1443,22 @@ int run_skinny(GemmArgs a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st)
         long total = (long)a.M * a.N;
         hipLaunchKernelGGL(skinny_epilogue_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, a, part, nsplit);
     } else {
-        const int mt = a.M <= 1 ? 1 : a.M <= 2 ? 2 : a.M <= 4 ? 4 : 8;
+        const int mt = a.M <= 1 ? 1 : a.M <= 2 ? 2 : 4;
         const size_t lds = (size_t)mt * a.K * sizeof(half_t);
         if (a.M > 8 || lds > SKINNY_FK_LDS_MAX) return MI_DECLINE_EXTENT;
+        if (a.M >= FEW_ROWS_MIN) {
+            const int cols = ceil_div(a.N, 16) * 2 <= mi_num_cus() ? 8 : 16, per = (int)ceil_div(ceil_div(a.K, 32), 8);
+            const dim3 grid((unsigned)ceil_div(a.N, cols));
+            if (a.ln_on) {
+                if (per <= 5) hipLaunchKernelGGL((few_rows_kernel<5, true>), grid, dim3(512), 0, st, a, cols);
+                else          hipLaunchKernelGGL((few_rows_kernel<10, true>), grid, dim3(512), 0, st, a, cols);
+            } else {
+                if (per <= 5)       hipLaunchKernelGGL((few_rows_kernel<5, false>), grid, dim3(512), 0, st, a, cols);
+                else if (per <= 10) hipLaunchKernelGGL((few_rows_kernel<10, false>), grid, dim3(512), 0, st, a, cols);
+                else                hipLaunchKernelGGL((few_rows_kernel<20, false>), grid, dim3(512), 0, st, a, cols);
+            }
+            return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+        }
         // rows per wave: as many as still leave every CU a workgroup, at most eight (a workgroup stages
         // all M activation rows once, whatever the number of weight rows it then streams)
         // One weight row per wave.  More rows per wave would amortise the staging of the activations, but the
@@ -1368,13 +1487,11 @@ int run_skinny(GemmArgs a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st)
         if (a.K <= 1536) {
             if (mt == 1)      hipLaunchKernelGGL((skinny_fk_kernel<1, 3>), grid, dim3(256), lds, st, a);
             else if (mt == 2) hipLaunchKernelGGL((skinny_fk_kernel<2, 3>), grid, dim3(256), lds, st, a);
-            else if (mt == 4) hipLaunchKernelGGL((skinny_fk_kernel<4, 3>), grid, dim3(256), lds, st, a);
-            else              hipLaunchKernelGGL((skinny_fk_kernel<8, 3>), grid, dim3(256), lds, st, a);
+            else              hipLaunchKernelGGL((skinny_fk_kernel<4, 3>), grid, dim3(256), lds, st, a);
         } else {
             if (mt == 1)      hipLaunchKernelGGL((skinny_fk_kernel<1, 12>), grid, dim3(256), lds, st, a);
             else if (mt == 2) hipLaunchKernelGGL((skinny_fk_kernel<2, 12>), grid, dim3(256), lds, st, a);
-            else if (mt == 4) hipLaunchKernelGGL((skinny_fk_kernel<4, 12>), grid, dim3(256), lds, st, a);
-            else              hipLaunchKernelGGL((skinny_fk_kernel<8, 12>), grid, dim3(256), lds, st, a);
+            else              hipLaunchKernelGGL((skinny_fk_kernel<4, 12>), grid, dim3(256), lds, st, a);
         }
     }
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
@@ -1562,11 +1679,9 @@ int mi_init(void) {
     bad |= raise_lds(skinny_fk_kernel<1, 3>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<2, 3>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 3>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<8, 3>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<1, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<8, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= mi_pipe_init() | mi_ring_init() | mi_any_init() | mi_conv_tile_init();
     bad |= mi_sdpa_init();
     bad |= scratch_of_current_device() == nullptr;

@@ -140,7 +140,7 @@ def decoder_layer_step(ctx: Ctx, W: DecoderLayerWeights, cache: KVCache, layer: 
     """One token through one decoder layer: self-attention over the cache (the new
     row appended in place first), cross-attention over the window's encoder K/V,
     GELU MLP; the three layer norms ride in the prologues of the GEMVs that read
-    them (batch <= 4; separate launches above), the residuals in the epilogues.  ``cache.advance`` must have
+    them (batch <= 8 with ``[F][K]`` weights, 4 with others; separate launches above), the residuals in the epilogues.  ``cache.advance`` must have
     run once for this step.  ``x``, ``out``: ``(B, d_model)`` fp16."""
     B, d = x.shape
     H, E = cache.heads, cache.headdim
@@ -148,10 +148,10 @@ def decoder_layer_step(ctx: Ctx, W: DecoderLayerWeights, cache: KVCache, layer: 
     self_k, self_v, cross_k, cross_v = cache.layer(layer)
 
     def normed_linear(dst, w, src, g, b_, bias, epi="none"):
-        # every workgroup of the folded form recomputes the row statistics: worth it for a few rows
-        # (one launch less per norm), not for eight
+        # every workgroup of the folded form recomputes the row statistics: one launch less per norm, worth it up to the
+        # eight rows that the decode-sized kernels take, where they are one launch ([F][K] weights)
         ctx.ws.reset()
-        if B <= 4:
+        if B <= (8 if w.stride(0) == 1 else 4):
             ln_matmul_(ctx, dst, w, src, g, b_, eps, bias, epi=epi)
         else:
             layernorm_(ctx, buf.h, None, None, src, g, b_, d, eps)

@@ -1,0 +1,39 @@
+"""Five to eight rows against [F][K] weights, on the matrix cores: K that ends inside a 32-deep step and a wave's share, one step and
+many, columns off the tiles of eight and sixteen, the norm in front bit for bit as its own launch."""
+import numpy as np
+import pytest
+
+import oracle
+from util import assert_parity, poison, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T", [5, 8])
+@pytest.mark.parametrize("K,F", [(8, 16), (24, 3), (40, 7), (256, 130), (264, 17), (1280, 33), (1288, 2100), (2568, 24), (5128, 40), (8192, 9)])
+def test_rows(ctx, T, K, F):
+    import torch
+    import juliavision_amd as jv
+    X, W, b = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K, F), 2), oracle.randn_f16((F,), 3, 0, 0.02)
+    R, g, beta = oracle.randn_f16((T, F), 4), oracle.randn_f16((K,), 5, 1.0, 0.1), oracle.randn_f16((K,), 6, 0, 0.1)
+    w, dx, db = to_dev(np.ascontiguousarray(W.T)).t(), to_dev(X), to_dev(b)
+    new = lambda dt=torch.float16: poison(torch.empty((T, F), dtype=dt, device="cuda"))
+    for epi, res, dt in (("gelu", None, torch.float16), ("none", R, torch.float16), ("relu", None, torch.float32)):
+        out = new(dt)
+        ctx.ws.reset()
+        jv.matmul_(ctx, out, w, dx, db, epi=epi, residual=None if res is None else to_dev(res))
+        assert_parity(to_host(out), oracle.gemm_f16(X, W, b, epi=epi, residual=res), what=f"T{T} K{K} F{F} {epi}")
+    # fp32 results: sums of K products in fp32, each half exact (2^-24 sqrt(K) of a result that is a sum of as many, with room)
+    exact = X.astype(np.float64) @ W.astype(np.float64) + b.astype(np.float64)
+    out = new(torch.float32)
+    ctx.ws.reset()
+    jv.matmul_(ctx, out, w, dx, db)
+    assert np.linalg.norm(to_host(out) - exact) <= 2.0 ** -24 * max(8.0, np.sqrt(K)) * np.linalg.norm(exact)
+    h, folded, apart = torch.empty((T, K), dtype=torch.float16, device="cuda"), new(), new()
+    ctx.ws.reset()
+    jv.ln_matmul_(ctx, folded, w, dx, to_dev(g), to_dev(beta), 1e-5, db)
+    jv.layernorm_(ctx, h, None, None, dx, to_dev(g), to_dev(beta), K, 1e-5)
+    ctx.ws.reset()
+    jv.matmul_(ctx, apart, w, h, db)
+    if K <= 4096:                                         # the norm kernel walks longer rows in another order
+        assert torch.equal(folded, apart)
