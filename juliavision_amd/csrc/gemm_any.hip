@@ -7,8 +7,8 @@ namespace {
 // Eight halves of a row of `len` around column c, in one 16-byte load (the target takes any address): where they would run past
 // the row, the row's last eight.  place_row8 puts them where they belong when they are needed, not when they are asked for: a
 // load by element there cost its column of tiles eight trips to memory a row (35 x 4743 -> 723 121 us).
-// Rows shorter than eight are read by element, by an instance of their own (SHORT): a branch around the load would end in a copy
-// of its result, which waits for it.
+// Rows shorter than eight are read by element, by instances of their own (SHORT): a branch around the load would end in a copy
+// of its result, which waits for it.  For the same reason an element past the row is the row's last one, and cleared in its place.
 enum RowLoad { ALIGNED, ANY, SHORT };
 template <RowLoad ROW>
 __device__ __forceinline__ u32x4 load_row8(const half_t *row, int c, int len) {
@@ -16,9 +16,9 @@ __device__ __forceinline__ u32x4 load_row8(const half_t *row, int c, int len) {
     if constexpr (ROW == ALIGNED) v = ldg16(row + min(c, len - 8));
     else if constexpr (ROW == ANY) __builtin_memcpy(&v, row + min(c, len - 8), 16);
     else {
-        half8v h = as_half8(v);
+        half8v h;
 #pragma unroll
-        for (int e = 0; e < 8; e++) if (c + e < len) h[e] = row[c + e];
+        for (int e = 0; e < 8; e++) h[e] = row[min(c + e, len - 1)];
         v = __builtin_bit_cast(u32x4, h);
     }
     return v;
@@ -26,7 +26,12 @@ __device__ __forceinline__ u32x4 load_row8(const half_t *row, int c, int len) {
 // Columns c .. c + 7 of what load_row8 brought, zeros from column len on.
 template <RowLoad ROW>
 __device__ __forceinline__ u32x4 place_row8(u32x4 v, int c, int len) {
-    if constexpr (ROW == SHORT) return v;                 // already in place
+    if constexpr (ROW == SHORT) {                         // in place already
+        half8v h = as_half8(v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) h[e] = c + e < len ? h[e] : (half_t)0.0f;
+        return __builtin_bit_cast(u32x4, h);
+    }
     const uint32_t by = (uint32_t)min(max(c + 8 - len, 0), 8);                      // halves to drop
     const uint32_t two = by & 2 ? ~0u : 0u, four = by & 4 ? ~0u : 0u, keep = by & 8 ? 0u : ~0u;
     const auto pick = [](uint32_t m, uint32_t a, uint32_t b) { return (a & m) | (b & ~m); };
@@ -46,9 +51,10 @@ __device__ __forceinline__ u32x4 place_row8(u32x4 v, int c, int len) {
 // transposed in registers by a quarter of the threads.  us, before -> now: 45 x 3553 -> 1292 81 -> 21, 3593 x 376 -> 197 31 -> 8.4,
 // 10 x 252 -> 132 19 -> 5.2, 1500 x 1283 -> 1281 66 -> 21, 2237 x 1000 -> 2437 108 -> 33 ([K][N] weights); 35 x 4743 -> 723 39 -> 26,
 // 164 x 190 -> 287 7.4 -> 4.8, 1500 x 1283 -> 1281 22.5 -> 19.8, 2237 x 1001 -> 2437 32.7 -> 33.3 ([N][K]).
-template <int BM, int BN, int KG, bool B_KN, RowLoad ROW>
+template <int BM, int BN, int KG, bool B_KN, RowLoad ROW_A, RowLoad ROW_B>
 __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
     constexpr int NT = 256, BK = 64, LD = BK + 8;
+    constexpr bool ONE = ROW_A == SHORT;                    // K < 8: a single tile
     constexpr int WTM = BM / 2, WTN = BN / 2, TM = WTM / 32, TN = WTN / 32;
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;
     constexpr int BLD = BN + 8, CPRB = BN / 8;              // [K][N]: halves and chunks of a k-row
@@ -71,13 +77,13 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
 #pragma unroll
         for (int i = 0; i < PA; i++) {
             const int c = tid + i * NT;
-            ra[set][i] = load_row8<ROW>(A + (long)min(m0 + (c >> 3), p.M - 1) * p.ldA, k0 + (c & 7) * 8, p.K);
+            ra[set][i] = load_row8<ROW_A>(A + (long)min(m0 + (c >> 3), p.M - 1) * p.ldA, k0 + (c & 7) * 8, p.K);
         }
 #pragma unroll
         for (int i = 0; i < PB; i++) {
             const int c = tid + i * NT;
-            if constexpr (B_KN) rb[set][i] = load_row8<ROW>(B + (long)min(k0 + c / CPRB, p.K - 1) * p.ldB, n0 + (c % CPRB) * 8, p.NB);
-            else rb[set][i] = load_row8<ROW>(B + (long)min(n0 + (c >> 3), p.N - 1) * p.ldB, k0 + (c & 7) * 8, p.K);
+            if constexpr (B_KN) rb[set][i] = load_row8<ROW_B>(B + (long)min(k0 + c / CPRB, p.K - 1) * p.ldB, n0 + (c % CPRB) * 8, p.NB);
+            else rb[set][i] = load_row8<ROW_B>(B + (long)min(n0 + (c >> 3), p.N - 1) * p.ldB, k0 + (c & 7) * 8, p.K);
         }
     };
     auto put = [&](auto SET, int kt) {
@@ -85,16 +91,16 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
         const int k0 = kt * BK;
         if (k0 + BK > p.K) {                                // uniform: the tile that K ends in, or one past it
 #pragma unroll
-            for (int i = 0; i < PA; i++) ra[set][i] = place_row8<ROW>(ra[set][i], k0 + ((tid + i * NT) & 7) * 8, p.K);
+            for (int i = 0; i < PA; i++) ra[set][i] = place_row8<ROW_A>(ra[set][i], k0 + ((tid + i * NT) & 7) * 8, p.K);
 #pragma unroll
             for (int i = 0; i < PB; i++) {
                 if constexpr (B_KN) rb[set][i] &= k0 + (tid + i * NT) / CPRB < p.K ? 0xffffffffu : 0u;
-                else rb[set][i] = place_row8<ROW>(rb[set][i], k0 + ((tid + i * NT) & 7) * 8, p.K);
+                else rb[set][i] = place_row8<ROW_B>(rb[set][i], k0 + ((tid + i * NT) & 7) * 8, p.K);
             }
         }
         if (B_KN && n0 + BN > p.NB) {                       // uniform: the column tile that the rows end in
 #pragma unroll
-            for (int i = 0; i < PB; i++) rb[set][i] = place_row8<ROW>(rb[set][i], n0 + ((tid + i * NT) % CPRB) * 8, p.NB);
+            for (int i = 0; i < PB; i++) rb[set][i] = place_row8<ROW_B>(rb[set][i], n0 + ((tid + i * NT) % CPRB) * 8, p.NB);
         }
 #pragma unroll
         for (int i = 0; i < PA; i++) { const int c = tid + i * NT; *reinterpret_cast<u32x4 *>(As + set * BM * LD + (c >> 3) * LD + (c & 7) * 8) = ra[set][i]; }
@@ -119,14 +125,14 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     load(I0{}, group);
-    load(I1{}, KG + group);
+    if constexpr (!ONE) load(I1{}, KG + group);
     put(I0{}, group);
     __syncthreads();
     // step s: tile s KG + group lies in buffer CUR, its successor is on its way in the other set.  What is asked for past the last tile
     // lies inside the rows: behind a condition the compiler would wait for all loads at every step.
     auto step = [&](auto CUR, int s) {
         constexpr int cur = decltype(CUR)::value;
-        load(CUR, (s + 2) * KG + group);
+        if constexpr (!ONE) load(CUR, (s + 2) * KG + group);
         const half_t *as = As + cur * BM * LD + (wm * WTM + frow) * LD + fk;
 #pragma unroll
         for (int ks = 0; ks < BK / 16; ks++) {
@@ -149,15 +155,18 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_kernel(GemmArgs p) {
                 for (int j = 0; j < TM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[i], fa[j], acc[i][j], 0, 0, 0);
         }
     };
-    for (int s = 0;; s += 2) {
-        step(I0{}, s);
-        if (s + 1 >= steps) break;
-        put(I1{}, (s + 1) * KG + group);
-        __syncthreads();
-        step(I1{}, s + 1);
-        if (s + 2 >= steps) break;
-        put(I0{}, (s + 2) * KG + group);
-        __syncthreads();
+    if constexpr (ONE) step(I0{}, 0);
+    else {
+        for (int s = 0;; s += 2) {
+            step(I0{}, s);
+            if (s + 1 >= steps) break;
+            put(I1{}, (s + 1) * KG + group);
+            __syncthreads();
+            step(I1{}, s + 1);
+            if (s + 2 >= steps) break;
+            put(I0{}, (s + 2) * KG + group);
+            __syncthreads();
+        }
     }
     __syncthreads();
     if constexpr (KG > 1) {
@@ -189,15 +198,17 @@ constexpr int any_lds_bytes() {                             // either layout of 
     return KG * 2 * (BM * 72 + (nk > kn ? nk : kn)) * 2;
 }
 
-template <int BM, int BN, int KG, RowLoad ROW>
-int launch_any(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
+template <int BM, int BN, int KG, bool B_KN, RowLoad ROW_A, RowLoad ROW_B = ROW_A>
+int launch_any(GemmArgs a, int64_t nbatch, hipStream_t st) {
     set_tiles(a, BM, BN);
     a.vec_store = rows_vec16(a);
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
-    constexpr int lds = any_lds_bytes<BM, BN, KG>();
-    if (b_kn) hipLaunchKernelGGL((gemm_any_kernel<BM, BN, KG, true, ROW>), grid, dim3(256 * KG), lds, st, a);
-    else      hipLaunchKernelGGL((gemm_any_kernel<BM, BN, KG, false, ROW>), grid, dim3(256 * KG), lds, st, a);
+    const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch);
+    hipLaunchKernelGGL((gemm_any_kernel<BM, BN, KG, B_KN, ROW_A, ROW_B>), grid, dim3(256 * KG), (any_lds_bytes<BM, BN, KG>()), st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
+template <int BM, int BN, int KG, RowLoad ROW>
+int launch_any(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
+    return b_kn ? launch_any<BM, BN, KG, true, ROW>(a, nbatch, st) : launch_any<BM, BN, KG, false, ROW>(a, nbatch, st);
 }
 
 }  // namespace
@@ -206,7 +217,13 @@ int launch_any(GemmArgs a, bool b_kn, int64_t nbatch, hipStream_t st) {
 // one; with 64 x 64 tiles below half a chip and more than four tiles of K, the K-groups.
 int mi_any_launch(const GemmArgs &a, bool b_kn, bool addressable, int64_t nbatch, hipStream_t st) {
     if (addressable) return launch_any<64, 64, 1, ALIGNED>(a, b_kn, nbatch, st);
-    if (a.K < 8 || (b_kn && a.NB < 8)) return launch_any<64, 64, 1, SHORT>(a, b_kn, nbatch, st);
+    // rows shorter than a load: of A (and of a K-contiguous B) where K < 8 -- a 1 x 1 convolution of an image's three channels, 6.6 us
+    // by element as the whole of B was, 4.2 with B in wide loads --, of a [K][N] operand where N < 8
+    if (a.K < 8) {
+        if (!b_kn) return launch_any<64, 64, 1, false, SHORT>(a, nbatch, st);
+        return a.NB < 8 ? launch_any<64, 64, 1, true, SHORT>(a, nbatch, st) : launch_any<64, 64, 1, true, SHORT, ANY>(a, nbatch, st);
+    }
+    if (b_kn && a.NB < 8) return launch_any<64, 64, 1, true, ANY, SHORT>(a, nbatch, st);
     const int64_t big = ceil_div(a.M, 128) * ceil_div(a.N, 128) * nbatch, small = ceil_div(a.M, 64) * ceil_div(a.N, 64) * nbatch;
     if (big >= mi_num_cus()) return launch_any<128, 128, 1, ANY>(a, b_kn, nbatch, st);
     if (small <= mi_num_cus() / 2 && a.K > 256) return launch_any<64, 64, 4, ANY>(a, b_kn, nbatch, st);
@@ -215,9 +232,9 @@ int mi_any_launch(const GemmArgs &a, bool b_kn, bool addressable, int64_t nbatch
 
 int mi_any_init() {
     int bad = 0;
-    bad |= raise_lds(gemm_any_kernel<64, 64, 4, true, ANY>, any_lds_bytes<64, 64, 4>());
-    bad |= raise_lds(gemm_any_kernel<64, 64, 4, false, ANY>, any_lds_bytes<64, 64, 4>());
-    bad |= raise_lds(gemm_any_kernel<128, 128, 1, true, ANY>, any_lds_bytes<128, 128, 1>());
-    bad |= raise_lds(gemm_any_kernel<128, 128, 1, false, ANY>, any_lds_bytes<128, 128, 1>());
+    bad |= raise_lds(gemm_any_kernel<64, 64, 4, true, ANY, ANY>, any_lds_bytes<64, 64, 4>());
+    bad |= raise_lds(gemm_any_kernel<64, 64, 4, false, ANY, ANY>, any_lds_bytes<64, 64, 4>());
+    bad |= raise_lds(gemm_any_kernel<128, 128, 1, true, ANY, ANY>, any_lds_bytes<128, 128, 1>());
+    bad |= raise_lds(gemm_any_kernel<128, 128, 1, false, ANY, ANY>, any_lds_bytes<128, 128, 1>());
     return bad;
 }

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("layout", ["kf", "fk"])
-@pytest.mark.parametrize("T,K,F", [(70, 121 + r, 65 + r) for r in range(8)] + [(9, 3, 70), (9, 70, 3), (5, 7, 7), (130, 63, 9), (33, 65, 129), (40, 193, 17),
+@pytest.mark.parametrize("T,K,F", [(70, 121 + r, 65 + r) for r in range(8)] + [(9, 3, 70), (9, 70, 3), (5, 7, 7), (130, 63, 9), (33, 65, 129), (40, 193, 17), (100, 5, 200), (100, 200, 5), (100, 5, 5),
                                                                                 (70, 257, 71), (70, 321, 71), (17, 515, 614), (30, 1025, 77), (2200, 131, 2057)])
 def test_every_remainder(ctx, T, K, F, layout):
     import torch
