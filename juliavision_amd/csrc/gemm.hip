@@ -10,6 +10,7 @@
 #include "gemm_common.hpp"
 #include "conv_common.hpp"
 #include "sk_exchange.hpp"
+#include <algorithm>
 #include <atomic>
 
 // Arrival flags of the split-K peer reduction (gemm_w4_kernel, SK): SK_BANKS banks of SK_FLAGS words, and as many
@@ -1287,10 +1288,10 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
-constexpr int RING_TILE = 5;             // index into TILE_MODELS: gemm_ring_kernel
+constexpr int RING_TILE = 5, DEEP_TILE = 6, DEEP_SERIAL_TILE = 7;      // indices into TILE_MODELS: gemm_ring_kernel, gemm_deep_kernel with four matrix waves and one
 // tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
-// output, same bits, and the plan (hence the workspace) stays a function of the extents alone.
+// output, same bits (the deep tile is not planned for a gathered operand: its K order is its own), and the plan (hence the workspace) stays a function of the extents alone.
 int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
     const bool plain = !a.ag.x && a.K % 64 == 0;
     switch (tile) {
@@ -1300,6 +1301,13 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
             if (!a.ag.x) {
                 const int rc = mi_ring_launch(a, b_kn, nbatch, st);
                 if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
+            }
+            return mi_pipe_launch(4, a, b_kn, nbatch, st);
+        case DEEP_TILE:
+        case DEEP_SERIAL_TILE:
+            if (!a.ag.x) {
+                const int rc = mi_deep_launch(a, tile == DEEP_TILE, b_kn, nbatch, st);
+                if (rc != MI_DECLINE_EXTENT) return rc;
             }
             return mi_pipe_launch(4, a, b_kn, nbatch, st);
         default: return mi_pipe_launch(tile, a, b_kn, nbatch, st);
@@ -1314,11 +1322,13 @@ int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStrea
 // launch (4.4 us) and the fp32 planes (0.38 us per MB).
 // Fitted to every tile timed on 260 shapes in a replayed graph (M 9..8192, N 64..8192, K 72..5120, both layouts, a third of
 // them with K % 64, a third with GELU).  On these the cheapest estimate lands within 0.4 % of the best measured tile on average,
-// 15 % at worst (259 x 1728 -> 3584 with GELU).
+// 15 % at worst (259 x 1728 -> 3584 with GELU).  The 32 x 32 tiles, at most one workgroup a CU, were fitted to 300 more (M 9..2048,
+// N 64..5120, K 72..8192): 18 % above the best tile on average without them, 1.2 % with them.  A K that mi_ln_gemm_f16 takes, up to
+// MI_LNA_KMAX, keeps one chain of sums an element: that call gives the bits of a norm followed by this GEMM, on whichever tile.
 // What it replaced sent every K % 64 to 64 x 64 tiles: 1544 x 1288 -> 1288 with residual 19.8 -> 15.4 us on 128 x 128,
 // 636 x 4392 -> 104 23.2 -> 13.8 on the ring, 2237 x 5096 -> 2440 with GELU 143 -> 80 on 192 x 128.
 struct TileModel { int bm, bn; double step_lo, step_full, round, fixed, gelu, tail; };
-constexpr int NTILES = 6;
+constexpr int NTILES = 8;
 constexpr TileModel TILE_MODELS[NTILES] = {
     {128, 256, 0.453, 0.746, 1.02, 6.1, 2.89, 1.41},
     {192, 128, 0.369, 0.613, 1.03, 5.19, 2.17, 1.38},
@@ -1326,8 +1336,10 @@ constexpr TileModel TILE_MODELS[NTILES] = {
     {64, 128, 0.315, 0.394, 0.841, 3.47, 0.946, 1.17},
     {64, 64, 0.267, 0.302, 0.632, 3.04, 0.423, 1.2},
     {64, 64, 0.135, 0.22, 0.818, 3.28, 0.362, 1.3},      // gemm_ring_kernel
+    {32, 32, 0.0857, 0.132, 0.624, 3.15, 0.508, 1.21},   // gemm_deep_kernel, K split over its waves
+    {32, 32, 0.142, 0.112, 0.8, 3.14, 0.409, 1.15},      // gemm_deep_kernel, one chain of sums
 };
-constexpr int64_t RING_WGS_PER_CU = 11;      // as many as the fit has seen
+constexpr int64_t RING_WGS_PER_CU = 11, DEEP_WGS = 256;      // as many as the fits have seen
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
@@ -1376,7 +1388,7 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu) {
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu, bool deep) {
     TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
@@ -1384,6 +1396,10 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
         if (split > 1 && (K % (64 * split) != 0 || K / split < 128)) continue;
         for (int tile = 0; tile < NTILES; tile++) {
             if (tile == RING_TILE && ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > RING_WGS_PER_CU * mi_num_cus()) continue;
+            if (tile == DEEP_TILE || tile == DEEP_SERIAL_TILE) {
+                if (!deep || (K > MI_LNA_KMAX) != (tile == DEEP_TILE)) continue;
+                if (ceil_div(M, 32) * ceil_div(N, 32) * nbatch * split > std::min(DEEP_WGS, (int64_t)mi_num_cus())) continue;
+            }
             const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
@@ -1398,15 +1414,15 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
 }
 
 // The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
-// thread keeps the last answers.  The key holds everything the estimate reads.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu = false) {
+// thread keeps the last answers.  The key holds everything the estimate reads; flags tell places apart, as one call asks under several.
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu = false, bool deep = true) {
     struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
     static thread_local Entry table[256] = {};
-    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (gelu ? 8 : 0);
-    const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 40;
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (gelu ? 8 : 0) | (deep ? 16 : 0);
+    const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 32;
     Entry &e = table[(h >> 32) & 255];
     if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
-        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, gelu)};
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, gelu, deep)};
     return e.plan;
 }
 
@@ -1415,6 +1431,12 @@ TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_sp
 size_t plan_workspace_bytes(const TilePlan &tp, int64_t M, int64_t N) {
     if (tp.split <= 1) return 0;
     return round_up(tp.peer ? sk_workspace_bytes(M, N, TILE_MODELS[tp.tile].bm, TILE_MODELS[tp.tile].bn, tp.split) : (size_t)tp.split * M * N * sizeof(float), 256);
+}
+
+// Workspace to ask for: of the plan, and of the plan without the 32 x 32 tiles -- a gathered operand's, and the size that recorded
+// plans and callers' buffers had before those tiles.
+size_t planned_workspace(int64_t M, int64_t N, int64_t K) {
+    return std::max(plan_workspace_bytes(plan_tiles(M, N, K, 1, true), M, N), plan_workspace_bytes(plan_tiles(M, N, K, 1, true, false, false), M, N));
 }
 
 int gemm_path(const GemmArgs &a, bool b_kn, int64_t nbatch) {
@@ -1559,17 +1581,18 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
                                            : (a.N % 4 == 0 && a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16));
             if (!whole || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
         }
+        const bool deep = !a.ag.x;
         if (pipe) {
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, !a.lnf_stats);
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, !a.lnf_stats, false, deep);
             if (tp.split > 1 && !(ws && aligned_to(ws, 256) && ws_bytes >= plan_workspace_bytes(tp, a.M, a.N)))
-                tp = plan_tiles(a.M, a.N, a.K, nbatch, false);
-            if (in_store && tp.split > 1 && !(tp.peer && sk_usable())) tp = plan_tiles(a.M, a.N, a.K, nbatch, false);
+                tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep);
+            if (in_store && tp.split > 1 && !(tp.peer && sk_usable())) tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep);
         }
         int split = tp.split;
         if (split > 1 && tp.peer && ws && aligned_to(ws, 256) && ws_bytes >= plan_workspace_bytes(tp, a.M, a.N)) {
             const int rc = launch_w4_peer(a, b_kn, split, ws, st);
             if (rc != MI_DECLINE_EXTENT) return rc;     // declined (a gathered operand, a device that failed the probe): planes
-            if (in_store) { tp = plan_tiles(a.M, a.N, a.K, nbatch, false); split = 1; }
+            if (in_store) { tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep); split = 1; }
         }
         if (split > 1 && ws && aligned_to(ws, 256) && ws_bytes >= (size_t)split * a.M * a.N * sizeof(float)) {
             GemmArgs s1 = a;
@@ -1597,9 +1620,10 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
         // A GELU store is some fifteen vector instructions a value, so narrower tiles can be the faster ones for it (1500 x 384 ->
-        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every tile sums K in the same order: the bits stay.
-        if (pipe && split == 1 && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true);
+        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every tile but the one that splits K over its waves sums K in the same order, so the
+        // choice is among those (or stays with it): the bits are the ones without a GELU.
+        if (pipe && split == 1 && tp.tile != DEEP_TILE && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep && a.K <= MI_LNA_KMAX);
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
@@ -1623,7 +1647,7 @@ bool mi_xcd_round_robin() { return sk_usable(); }
 size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatch) {
     if (T <= 8) return mi_gemm_f16_workspace(T, K, F, MI_W_KF, nbatch);      // decode-sized: the [K][F] kernel's planes
     if (nbatch > 1 || K % 64 || K < 128) return 0;
-    return plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
+    return planned_workspace(T, F, K);
 }
 
 double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, RING_TILE, 1); }
@@ -1682,7 +1706,7 @@ int mi_init(void) {
     bad |= raise_lds(skinny_fk_kernel<1, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
     bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= mi_pipe_init() | mi_ring_init() | mi_any_init() | mi_conv_tile_init();
+    bad |= mi_pipe_init() | mi_ring_init() | mi_deep_init() | mi_any_init() | mi_conv_tile_init();
     bad |= mi_sdpa_init();
     bad |= scratch_of_current_device() == nullptr;
     sk_probe_current_device();      // a device that fails the probe only loses that path
@@ -1751,7 +1775,7 @@ size_t mi_gemm_f16_workspace(int64_t T, int64_t K, int64_t F, int w_layout, int6
         if (K % 64 || K < 128) return 0;
         // Room for the exchange wherever it can run on a K of some length, whichever tile the estimate prefers: buffers and
         // recorded plans keep their sizes when its constants move.
-        const size_t need = plan_workspace_bytes(plan_tiles(T, F, K, 1, true), T, F);
+        const size_t need = planned_workspace(T, F, K);
         const TileModel &t = TILE_MODELS[SK_TILE];
         const size_t peer = K >= 2048 && sk_fits(T, F, K, t.bm, t.bn, 2) ? round_up(sk_workspace_bytes(T, F, t.bm, t.bn, 2), 256) : 0;
         return need > peer ? need : peer;

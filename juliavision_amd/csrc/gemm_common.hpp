@@ -222,13 +222,14 @@ struct LnfLoader {
 // tile's rows and the tile's columns of colsum and biasp at the store, not before, and in their registers the statistics
 // would cost a second workgroup a CU.  (In the prologue they held every wave at the first barrier: 5 000 clocks at 128 rows,
 // 10 000 at 192, a trip to memory per batch of loads, then forty dependent steps a row.)  Tile kt covers segments 2 kt and
-// 2 kt + 1: ahead of barrier kt this wave takes in the two segments of each of its BM / 64 rows that it requested AHEAD tiles
-// earlier, and the result is in the slot when it arrives at the last barrier, which the matrix waves pass before they store.
-// Same arithmetic, in the same order per row, as LnfLoader with one lane a row.  LEAD: a barrier comes before tile 0's.
-template <int BM, int BN, bool LEAD, typename BarrierF>
+// 2 kt + 1 (SEGS = 2; a 128-deep tile four): ahead of barrier kt this wave takes in the segments of each of its rows that it
+// requested AHEAD tiles earlier, and the result is in the slot when it arrives at the last barrier, which the matrix waves pass
+// before they store.  Same arithmetic, in the same order per row, as LnfLoader with one lane a row.  LEAD: a barrier comes before
+// tile 0's.
+template <int BM, int BN, bool LEAD, int SEGS = 2, typename BarrierF>
 __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot, int m0, int n0, long bz, int lane, int nk, BarrierF barrier) {
-    constexpr int NR = BM / 64, AHEAD = 4;
-    static_assert(BM % 64 == 0 && NR * 2 * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
+    constexpr int NR = (BM + 63) / 64, AHEAD = 4;
+    static_assert((BM % 64 == 0 || BM == 32) && NR * SEGS * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
     for (int t = lane; t < BN / 2; t += 64) {
         const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
         const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
@@ -240,7 +241,7 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
     const float2v *seg[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) seg[i] = reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + lane + 64 * i, p.M - 1);
-    float2v v[AHEAD][NR][2];
+    float2v v[AHEAD][NR][SEGS];
     float ref[NR], total[NR], within[NR], between[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) { ref[i] = 0.0f; total[i] = 0.0f; within[i] = 0.0f; between[i] = 0.0f; }
@@ -249,13 +250,13 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
 #pragma unroll
         for (int i = 0; i < NR; i++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) v[sl][i][h] = seg[i][(long)min(2 * kt + h, p.lnf_nseg - 1) * p.M];
+            for (int h = 0; h < SEGS; h++) v[sl][i][h] = seg[i][(long)min(SEGS * kt + h, p.lnf_nseg - 1) * p.M];
     };
     auto take = [&](auto SLOT, int kt) {
         constexpr int sl = decltype(SLOT)::value;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int left = p.K - 32 * (2 * kt + h);                  // uniform
+        for (int h = 0; h < SEGS; h++) {
+            const int left = p.K - 32 * (SEGS * kt + h);                  // uniform
             if (left <= 0) break;
             const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
 #pragma unroll
@@ -276,7 +277,7 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
             const int kt = kt0 + decltype(S)::value;
             if (kt < nk) {
                 // requests complete in order: what was requested after tile kt may still be on its way
-                if (kt + AHEAD - 1 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NR * 2) : "memory");
+                if (kt + AHEAD - 1 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NR * SEGS) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 take(S, kt);
                 if (kt + AHEAD < nk) fetch(S, kt + AHEAD);
@@ -287,7 +288,7 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
                         const float m2 = within[i] + fmaxf(between[i] - (float)p.K * dm * dm, 0.0f);
                         const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
                         const float2v o = {r, r * mu};
-                        slot[lane + 64 * i] = o;
+                        if (BM % 64 == 0 || lane < BM) slot[lane + 64 * i] = o;
                     }
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 }
@@ -714,6 +715,9 @@ int mi_pipe_init();
 // gemm_ring.hip: small grids of ordinary operands.
 int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_ring_init();
+// gemm_deep.hip: few output tiles, of ordinary operands.
+int mi_deep_launch(const GemmArgs &a, bool split_k, bool b_kn, int64_t nbatch, hipStream_t st);
+int mi_deep_init();
 // gemm_any.hip: the kernels for operands and extents that the others do not take.
 int mi_any_launch(const GemmArgs &a, bool b_kn, bool addressable, int64_t nbatch, hipStream_t st);
 int mi_any_init();

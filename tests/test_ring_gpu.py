@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("layout", ["kf", "fk"])
 @pytest.mark.parametrize("K", [72, 128, 136, 192, 256, 320, 384, 448, 512, 520, 576, 640, 1096])
-@pytest.mark.parametrize("T,F", [(65, 72), (1100, 1096)])      # 4 workgroups, and 324: more than one on a CU
+@pytest.mark.parametrize("T,F", [(1000, 1000), (1100, 1096)])      # 256 workgroups, and 324: more than one on a CU
 def test_tiles_of_k(ctx, T, F, K, layout):
     import torch
     import juliavision_amd as jv
@@ -26,7 +26,7 @@ def test_tiles_of_k(ctx, T, F, K, layout):
 
 
 @pytest.mark.parametrize("K", [128, 192, 320, 512, 576, 1280])
-@pytest.mark.parametrize("T,F", [(70, 72), (1100, 1096)])
+@pytest.mark.parametrize("T,F", [(1000, 1000), (1100, 1096)])
 def test_folded_norm(ctx, T, F, K):
     """The statistics wave keeps the loop's barriers, whatever the count of tiles."""
     import torch
