@@ -1340,6 +1340,10 @@ constexpr TileModel TILE_MODELS[NTILES] = {
     {32, 32, 0.142, 0.112, 0.8, 3.14, 0.409, 1.15},      // gemm_deep_kernel, one chain of sums
 };
 constexpr int64_t RING_WGS_PER_CU = 11, DEEP_WGS = 256;      // as many as the fits have seen
+// A folded norm costs the four-wave kernel and the ring more than the pipelined kernel, whose threads take the statistics in before the K
+// loop: the same kernels behind each other in a model, whole blocks, 1280 wide: 572 tokens 227 -> 216 us for three blocks with these, 700
+// 231 -> 224, 1500 352 -> 351; 900 x 1024 209 -> 202; 1370 x 384 132 either way.  (Alone, on weights that L2 holds, 192 x 128 tiles win.)
+constexpr double LNF_W4_US = 3.0, LNF_RING_US = 1.0;
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
@@ -1388,7 +1392,7 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
 }
 
 // The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
-TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu, bool deep) {
+TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu, bool deep, bool lnf) {
     TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
@@ -1400,7 +1404,7 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
                 if (!deep || (K > MI_LNA_KMAX) != (tile == DEEP_TILE)) continue;
                 if (ceil_div(M, 32) * ceil_div(N, 32) * nbatch * split > std::min(DEEP_WGS, (int64_t)mi_num_cus())) continue;
             }
-            const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu);
+            const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu) + (!lnf ? 0.0 : tile <= 1 ? LNF_W4_US : tile == RING_TILE ? LNF_RING_US : 0.0);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
         if (max_split > 1 && sk_planned()) {
@@ -1415,14 +1419,14 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
 
 // The estimate of every tile and split takes the host about 2 us, twice a call (workspace, launch): a small table per
 // thread keeps the last answers.  The key holds everything the estimate reads; flags tell places apart, as one call asks under several.
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu = false, bool deep = true) {
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu = false, bool deep = true, bool lnf = false) {
     struct Entry { int64_t M, N, K, nbatch; int cus, flags; TilePlan plan; };
     static thread_local Entry table[256] = {};
-    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (gelu ? 8 : 0) | (deep ? 16 : 0);
+    const int cus = mi_num_cus(), flags = 1 | (may_split ? 2 : 0) | (may_split && sk_planned() ? 4 : 0) | (gelu ? 8 : 0) | (deep ? 16 : 0) | (lnf ? 32 : 0);
     const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)K * 0x165667B19E3779F9ull) ^ ((uint64_t)nbatch << 17) ^ (uint64_t)flags << 32;
     Entry &e = table[(h >> 32) & 255];
     if (e.flags != flags || e.M != M || e.N != N || e.K != K || e.nbatch != nbatch || e.cus != cus)
-        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, gelu, deep)};
+        e = {M, N, K, nbatch, cus, flags, estimate_tiles(M, N, K, nbatch, may_split, gelu, deep, lnf)};
     return e.plan;
 }
 
@@ -1581,18 +1585,18 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
                                            : (a.N % 4 == 0 && a.ldY % 4 == 0 && a.sY % 4 == 0 && aligned_to(a.Y, 16));
             if (!whole || a.ag.x || !rows16 || (a.stats_out && a.out_f32)) return MI_DECLINE_EXTENT;
         }
-        const bool deep = !a.ag.x;
+        const bool deep = !a.ag.x, lnf = a.lnf_stats;
         if (pipe) {
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, !a.lnf_stats, false, deep);
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, !lnf, false, deep, lnf);
             if (tp.split > 1 && !(ws && aligned_to(ws, 256) && ws_bytes >= plan_workspace_bytes(tp, a.M, a.N)))
-                tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep);
-            if (in_store && tp.split > 1 && !(tp.peer && sk_usable())) tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep);
+                tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep, lnf);
+            if (in_store && tp.split > 1 && !(tp.peer && sk_usable())) tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep, lnf);
         }
         int split = tp.split;
         if (split > 1 && tp.peer && ws && aligned_to(ws, 256) && ws_bytes >= plan_workspace_bytes(tp, a.M, a.N)) {
             const int rc = launch_w4_peer(a, b_kn, split, ws, st);
             if (rc != MI_DECLINE_EXTENT) return rc;     // declined (a gathered operand, a device that failed the probe): planes
-            if (in_store) { tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep); split = 1; }
+            if (in_store) { tp = plan_tiles(a.M, a.N, a.K, nbatch, false, false, deep, lnf); split = 1; }
         }
         if (split > 1 && ws && aligned_to(ws, 256) && ws_bytes >= (size_t)split * a.M * a.N * sizeof(float)) {
             GemmArgs s1 = a;
@@ -1623,7 +1627,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every tile but the one that splits K over its waves sums K in the same order, so the
         // choice is among those (or stays with it): the bits are the ones without a GELU.
         if (pipe && split == 1 && tp.tile != DEEP_TILE && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep && a.K <= MI_LNA_KMAX);
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep && a.K <= MI_LNA_KMAX, lnf);
         if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
