@@ -199,17 +199,17 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
             }
         }
     };
-    float16v ms;                                                  // times log2(e)
+    float16v ms;                                                  // KEYS: times log2(e); DENSE: as it came
     auto mask_take = [&]() {
         if (p.bias_f32) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) { const uint32_t w = mraw[r >> 2][r & 3]; ms[r] = __builtin_bit_cast(float, w) * LOG2E; }
+            for (int r = 0; r < 16; r++) { const uint32_t w = mraw[r >> 2][r & 3]; ms[r] = __builtin_bit_cast(float, w); }
         } else {
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 const uint32_t w = mraw[r >> 2][(r & 3) >> 1];
                 const half2v t = __builtin_bit_cast(half2v, w);
-                ms[r] = (float)t[0] * LOG2E; ms[r + 1] = (float)t[1] * LOG2E;
+                ms[r] = (float)t[0]; ms[r + 1] = (float)t[1];
             }
         }
 #pragma unroll
@@ -256,11 +256,6 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
             } else sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
         }
         if constexpr (MASK == KEYS && !F32) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kx, qext, sc, 0, 0, 0);
-        const float16v raw = sc;
-        auto scale = [&]() {
-#pragma unroll
-            for (int r = 0; r < 16; r++) sc[r] = fmaf(raw[r], c, MASK ? ms[r] - m_run : -m_run);
-        };
         auto cut = [&]() {                                        // the ragged last tile: excluded keys get -inf
             if (tile * 32 + 32 > Lk) {
 #pragma unroll
@@ -268,19 +263,39 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
                     if (tile * 32 + 8 * (r >> 2) + 4 * hl + (r & 3) >= Lk) sc[r] = -INFINITY;
             }
         };
+        // DENSE: score and mask are rounded into one number, once, and M is the largest such number itself.  However large a mask
+        // (1e9 swallows its score, finfo.min times log2(e) would be infinite), no score of M's tile is above M, and a row of
+        // equal numbers is a row of equal weights.
+        if constexpr (MASK == DENSE) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] = fmaf(sc[r], p.scale, ms[r]);
+            cut();
+        }
+        const float16v raw = sc;
+        auto scale = [&]() {
+            if constexpr (MASK == DENSE) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) sc[r] = (raw[r] - m_run) * LOG2E;
+                return;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] = fmaf(raw[r], c, MASK ? ms[r] - m_run : -m_run);
+            cut();
+        };
         if constexpr (F32) scale();
-        cut();
+        else cut();
         half8v pf[2], lo[2];
         float l_new = l_run;
         probs(sc, pf, lo, l_new);
         if (__any(first || !(l_new - l_run < 65504.0f))) {        // flash_fwd_kernel says why
-            float tmax = fmaxf(sc[0], sc[1]);
+            const float16v &from = MASK == DENSE ? raw : sc;
+            float tmax = fmaxf(from[0], from[1]);
 #pragma unroll
-            for (int r = 2; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, sc[r]), sc[r + 1]);
-            const float mx = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const bool grow = (mx > TH || first) && mx > FLOOR;
+            for (int r = 2; r < 16; r += 2) tmax = fmaxf(fmaxf(tmax, from[r]), from[r + 1]);
+            const float top = fmaxf(tmax, __shfl_xor(tmax, 32, 64)), mx = MASK == DENSE ? (top - m_run) * LOG2E : top;
+            const bool grow = (mx > TH || first) && top > FLOOR;
             float d = grow ? mx : 0.0f, alpha = first ? 0.0f : __builtin_amdgcn_exp2f(-d);
-            float to = first ? d : m_run + d;
+            float to = MASK == DENSE ? (grow ? top : m_run) : first ? d : m_run + d;
             if constexpr (!F32) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) negm[r] = -to;
@@ -294,10 +309,8 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
             }
             m_run = to;
             l_run *= alpha;
-            if constexpr (F32) {
-                scale();
-                cut();
-            } else {
+            if constexpr (F32) scale();
+            else {
 #pragma unroll
                 for (int r = 0; r < 16; r++) sc[r] -= d;
             }
@@ -364,7 +377,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
 #pragma unroll
     for (int w = 0; w < NW; w++) {
         const float *xw = reinterpret_cast<const float *>(smem + w * WSTRIDE) + ET * 1024;
-        aw[w] = aw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(aw[w] - mm);
+        aw[w] = aw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(MASK == DENSE ? (aw[w] - mm) * LOG2E : aw[w] - mm);
         den += aw[w] * xw[64 + lane];
     }
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;

@@ -51,3 +51,37 @@ def test_dense_masks(ctx, B, H, Lq, Lk, E, f32, kind):
     exact = type(jv.sdpaplan(ctx, q, k, v, mask)).__name__ == "RowsSDPAPlan" or (kind == "odd" and not f32) or (kind == "keys_apart" and Lk > 1)
     err = float((out.double().cpu() - want).norm() / want.norm())
     assert err <= (4e-7 if exact else 6e-4), (err, exact)
+
+
+@pytest.mark.parametrize("fill", [-1e4, -1e7, -1e9, -1e30, "min"])
+@pytest.mark.parametrize("apart", [False, True])
+@pytest.mark.parametrize("E,half", [(16, False), (32, False), (64, False), (72, True), (128, False)])
+def test_large_finite_masks(ctx, E, half, apart, fill):
+    """fp32 masks that exclude keys by a large finite number: padding in front, behind, on both sides, none, and rows masked
+    throughout.  Scores have a standard deviation of 3.  A key that counts outweighs the others without trace; a row without
+    one is its scores rounded to the mask's spacing, which from 1e9 on is one value: the mean of V (below, such rows are left out)."""
+    import torch
+    import juliavision_amd as jv
+    B, H, Lq, Lk = 1, 2, 63 if not apart else 130, 545
+    lowest = float(np.finfo(np.float32).min) if fill == "min" else fill
+    q, k, v = (to_dev(oracle.randn_f16((B, H, L, E), s)) for s, L in ((11, Lq), (12, Lk), (13, Lk)))
+    q = (q.float() * 3).half()
+    m = torch.zeros((B, H, Lq, Lk), dtype=torch.float32)
+    for i in range(Lq):
+        front, behind = ((300, 0), (0, 412), (100, 130), (0, 0), (544, 0), (0, 544))[i % 6]
+        m[:, :, i, :front] = lowest
+        m[:, :, i, Lk - behind:] = lowest
+    if lowest <= -1e9:
+        m[:, :, 7::9] = lowest
+    mask = m.cuda()
+    if apart:
+        mask = mask.transpose(2, 3).contiguous().transpose(2, 3)
+    out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float16 if half else torch.float32, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, mask, out=out)
+    s = (torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3)) / np.sqrt(E) + m.double()).float().double()
+    want = torch.matmul(torch.softmax(s, -1), v.double().cpu())
+    assert bool(torch.isfinite(out).all())
+    err = (out.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    # per row: eight roundings of scores of up to 20 (2^-21 each) with fp32 results, half a unit of fp16 with fp16 ones
+    assert float(err.max()) <= (2.0 ** -10 if half else 4e-6), float(err.max())
