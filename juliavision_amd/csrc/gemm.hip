@@ -1291,15 +1291,15 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
 constexpr int RING_TILE = 5, DEEP_TILE = 6, DEEP_SERIAL_TILE = 7;      // indices into TILE_MODELS: gemm_ring_kernel, gemm_deep_kernel with four matrix waves and one
 // tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
-// output, same bits (the deep tile is not planned for a gathered operand: its K order is its own), and the plan (hence the workspace) stays a function of the extents alone.
-int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
+// output, same bits (the 32 x 32 tiles are not planned for a gathered operand: their order of a long K is their own).
+int launch_tile(int tile, const GemmArgs &a, bool one_chain, bool b_kn, int64_t nbatch, hipStream_t st) {
     const bool plain = !a.ag.x && a.K % 64 == 0;
     switch (tile) {
         case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : mi_pipe_launch(0, a, b_kn, nbatch, st);
         case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : mi_pipe_launch(1, a, b_kn, nbatch, st);
         case RING_TILE:
             if (!a.ag.x) {
-                const int rc = mi_ring_launch(a, b_kn, nbatch, st);
+                const int rc = mi_ring_launch(a, one_chain, b_kn, nbatch, st);
                 if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
             }
             return mi_pipe_launch(4, a, b_kn, nbatch, st);
@@ -1391,7 +1391,11 @@ double sk_cost_us(int64_t M, int64_t N, int64_t K, int tile, int split) {
            sk_exchange_us(wg, t.bm, t.bn));        // 0.9: 17.1 us at 1500 x 3072 -> 768, 27.9 at 1370 x 5120 -> 1280
 }
 
-// The plan depends on the extents alone, so a GEMM gives the same bits whichever entry point issues it.
+// Tiles that sum a long K in an order of their own: several chains an element (gemm_ring_kernel, gemm_deep_kernel).
+bool own_order(int tile, int64_t K) { return K > MI_LNA_KMAX && (tile == RING_TILE || tile == DEEP_TILE); }
+
+// The plan depends on the extents, and on whether the operand is gathered (no 32 x 32 tiles there) and a norm folded: calls alike in
+// these give the same bits whichever entry point issues them.  Up to K = MI_LNA_KMAX all unsplit calls do.
 TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_split, bool gelu, bool deep, bool lnf) {
     TilePlan best = {4, 1, false, 0.0};
     double best_us = 1e30;
@@ -1404,6 +1408,7 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
                 if (!deep || (K > MI_LNA_KMAX) != (tile == DEEP_TILE)) continue;
                 if (ceil_div(M, 32) * ceil_div(N, 32) * nbatch * split > std::min(DEEP_WGS, (int64_t)mi_num_cus())) continue;
             }
+            if (gelu && own_order(tile, K)) continue;
             const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu) + (!lnf ? 0.0 : tile <= 1 ? LNF_W4_US : tile == RING_TILE ? LNF_RING_US : 0.0);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
@@ -1605,7 +1610,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             s1.K = a.K / split;
             s1.sA = s1.K; s1.sB = b_kn ? (long)s1.K * a.ldB : s1.K; s1.sBias = 0;
             s1.ag.split = 1;
-            int rc = launch_tile(tp.tile, s1, b_kn, split, st);
+            int rc = launch_tile(tp.tile, s1, false, b_kn, split, st);
             if (rc != MI_OK) return rc;
             GemmArgs s2 = a;
             s2.vec_store = !a.out_f32 && a.ldY % 4 == 0 && aligned_to(a.Y, 8);
@@ -1624,11 +1629,11 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
         }
         // A GELU store is some fifteen vector instructions a value, so narrower tiles can be the faster ones for it (1500 x 384 ->
-        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  Every tile but the one that splits K over its waves sums K in the same order, so the
-        // choice is among those (or stays with it): the bits are the ones without a GELU.
-        if (pipe && split == 1 && tp.tile != DEEP_TILE && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
-            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep && a.K <= MI_LNA_KMAX, lnf);
-        if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
+        // 1536: 9.1 us on 128 x 128, 8.0 on 64 x 64).  The choice is among the tiles that sum K in the same order, or stays with one that
+        // has its own: the bits are the ones without a GELU.
+        if (pipe && split == 1 && !own_order(tp.tile, a.K) && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
+            tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep, lnf);
+        if (pipe) return launch_tile(tp.tile, a, a.K <= MI_LNA_KMAX, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
     return mi_any_launch(a, b_kn, false, nbatch, st);
@@ -1680,7 +1685,7 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     if (agather) a.ag = *agather;
     const bool addr = mfma_addressable(a, b_kn != 0);
     if ((gather || agather) && !addr) return MI_DECLINE_OPERANDS;
-    if (gather) return g_ready ? mi_ring_launch(a, false, nbatch, st) : MI_ERROR_DEVICE;
+    if (gather) return g_ready ? mi_ring_launch(a, false, false, nbatch, st) : MI_ERROR_DEVICE;
     int path = addr ? MI_GEMM_MFMA : MI_GEMM_SCALAR;
     return run_gemm(a, b_kn != 0, nbatch, ws, ws_bytes, st, path);
 }

@@ -8,7 +8,7 @@ namespace {
 
 // A workgroup owns a 32 x 32 tile.  Two loader waves keep a ring of 128-deep stages filled (gemm_ring_kernel says how).  NW = 4: each of
 // four matrix waves holds all of the tile in accumulators and takes two of the eight 16-deep steps of every stage; the partial tiles
-// meet in LDS and wave 0 stores the sum, eight chains of fp32 sums an element, added pairwise.  NW = 1, for a short K: one wave
+// meet in LDS and wave 0 stores the sum, eight chains of fp32 sums an element (sixteen past K = 4096), added pairwise.  NW = 1, for a short K: one wave
 // takes all steps in one chain, the other tiles' order and bits.
 //
 // What bounds a small grid is its CUs' vector-memory paths: a 64 x 64 tile takes 256 clocks of loads per 64 k, and 24 of them (70 x
@@ -24,10 +24,10 @@ namespace {
 // inside their row: K-contiguous row r holds chunk c at c ^ (r % 16), [K][N] row k at c ^ (k % 4).
 constexpr int S = 8;                      // stages of the ring: 128 KB
 
-template <int NW, bool B_KN>
+template <int NW, int CHAINS, bool B_KN>
 __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p) {
     constexpr int BM = 32, BN = 32, BK = 128, LPW = 8, AHEAD = 5;
-    constexpr int STEPS = 8 / NW, CHAINS = NW > 1 ? 2 : 1;           // a matrix wave's steps of a stage; its accumulators
+    constexpr int STEPS = 8 / NW;                         // a matrix wave's steps of a stage
     constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = 2 * A_BYTES;
     extern __shared__ __align__(16) char smem[];
     stage_args(p);
@@ -161,7 +161,10 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
     auto products = [&](auto SET) {
         constexpr int set = decltype(SET)::value;
 #pragma unroll
-        for (int s = 0; s < STEPS; s++) acc[s % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][s], fa[set][s], acc[s % CHAINS], 0, 0, 0);
+        for (int s = 0; s < STEPS; s++) {
+            constexpr int first = set * STEPS;            // (four chains: odd and even stages' steps apart)
+            acc[(first + s) % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][s], fa[set][s], acc[(first + s) % CHAINS], 0, 0, 0);
+        }
     };
 
     // what the store needs of memory, while the first stages are on their way
@@ -202,7 +205,7 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
     if ((l + 1) * STAGE_BYTES + ROOM <= S * STAGE_BYTES) room = smem + (l + 1) * STAGE_BYTES;
     float16v own[1][1];
 #pragma unroll
-    for (int r = 0; r < 16; r++) own[0][0][r] = NW > 1 ? acc[0][r] + acc[CHAINS - 1][r] : acc[0][r];
+    for (int r = 0; r < 16; r++) own[0][0][r] = CHAINS == 4 ? (acc[0][r] + acc[1 % CHAINS][r]) + (acc[2 % CHAINS][r] + acc[3 % CHAINS][r]) : CHAINS == 2 ? acc[0][r] + acc[1 % CHAINS][r] : acc[0][r];
     if constexpr (NW > 1) {
         float *part = reinterpret_cast<float *>(room);
         if (wave > 0) {
@@ -234,15 +237,15 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
 
 constexpr int DEEP_LDS_BYTES = S * 2 * 32 * 128 * 2 + 2 * 32 * 8;       // the stages; rows' and columns' parts of a folded norm
 
-template <int NW>
+template <int NW, int CHAINS>
 int launch_deep(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
     const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), block((NW + (a.lnf_stats ? 3 : 2)) * 64);
-    if (b_kn) hipLaunchKernelGGL((gemm_deep_kernel<NW, true>), grid, block, DEEP_LDS_BYTES, st, a);
-    else      hipLaunchKernelGGL((gemm_deep_kernel<NW, false>), grid, block, DEEP_LDS_BYTES, st, a);
+    if (b_kn) hipLaunchKernelGGL((gemm_deep_kernel<NW, CHAINS, true>), grid, block, DEEP_LDS_BYTES, st, a);
+    else      hipLaunchKernelGGL((gemm_deep_kernel<NW, CHAINS, false>), grid, block, DEEP_LDS_BYTES, st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
-template <int NW>
-int raise_deep() { return raise_lds(gemm_deep_kernel<NW, true>, DEEP_LDS_BYTES) | raise_lds(gemm_deep_kernel<NW, false>, DEEP_LDS_BYTES); }
+template <int NW, int CHAINS>
+int raise_deep() { return raise_lds(gemm_deep_kernel<NW, CHAINS, true>, DEEP_LDS_BYTES) | raise_lds(gemm_deep_kernel<NW, CHAINS, false>, DEEP_LDS_BYTES); }
 
 }  // namespace
 
@@ -252,7 +255,10 @@ int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch
     a.vec_store = rows_vec16(a);
     // per-lane load offsets are 32-bit byte offsets from the tile's origin
     if ((int64_t)32 * a.ldA * 2 >= (1ll << 31) || (int64_t)128 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
-    return split_k ? launch_deep<4>(a, b_kn, nbatch, st) : launch_deep<1>(a, b_kn, nbatch, st);
+    // Past K = 4096 such calls had twelve to twenty chains, as slices of K on the ring; short of it eight are as good as what they had, and
+    // the second pair of accumulators costs 0.05 to 0.1 us (50 x 3224 -> 992 6.67 | 6.75).
+    if (!split_k) return launch_deep<1, 1>(a, b_kn, nbatch, st);
+    return a.K > 4096 ? launch_deep<4, 4>(a, b_kn, nbatch, st) : launch_deep<4, 2>(a, b_kn, nbatch, st);
 }
 
-int mi_deep_init() { return raise_deep<4>() | raise_deep<1>(); }
+int mi_deep_init() { return raise_deep<4, 4>() | raise_deep<4, 2>() | raise_deep<1, 1>(); }

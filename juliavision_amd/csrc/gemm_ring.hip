@@ -19,8 +19,7 @@ namespace {
 // a launch; 1370 x 384 -> 384, where four waves that split K lost to the register-staged kernel, 5.1 -> 4.9 (4.65 before its
 // residual and statistics are counted), 76 x 1024 -> 3072 7.8 -> 6.3, 2056 x 1536 -> 384 11.1 -> 8.6.  Waves that split K read
 // 16 KB of fragments a tile instead of 32 and gain from some 45 tiles of K on in the smallest grids (32 x 3456 -> 448 10.3 against
-// 11.2 us); over 150 shapes they are 6 % behind.  Every tile of this library sums K in the same order, so the bits do not
-// depend on which one a plan picks.
+// 11.2 us); over 150 shapes they are 6 % behind.
 //
 // LDS layout of a stage: A rows of 128 bytes, then B ([N][K]: rows of 128 bytes; [K][N]: 64 rows of BN halves).  Direct loads
 // cannot pad, so 16-byte chunks are permuted inside their row: K-contiguous row r holds chunk c at c ^ (r % 8 ^ r / 8 % 2),
@@ -29,8 +28,14 @@ namespace {
 //
 // CONV: B is the patch matrix of a convolution (ConvGather).  Its rows' offsets are as fixed as an ordinary operand's; what moves
 // from tile to tile is the tap, for all lanes alike where C is a multiple of 64, by the lane's pair of chunks otherwise.
-template <int S, bool B_KN, bool CONV = false>
-__global__ __launch_bounds__(4 * 64 + 192, S > 4 ? 2 : 4) void gemm_ring_kernel(GemmArgs p) {
+//
+// CHAINS: accumulators an element, the 16-deep step ks of every tile in chain ks % CHAINS.  Four from K = 513 on and for patches: one
+// chain has 1.8 times the error of four (fp32 results against 64 bits: K = 768 1.78e-7 | 1.00e-7, 1536 2.49e-7 | 1.33e-7, 5120 4.55e-7 |
+// 2.32e-7) at the same time (1000 x 1536 -> 1000 8.13 | 8.17 us, 1000 x 5120 -> 1000 22.3 | 20.8).  One up to there, in the order of
+// every other tile: a call that folds a layer norm promises the bits of the norm and this GEMM apart.  One too for ordinary operands
+// past one workgroup a CU, whose registers are short.
+template <int S, bool B_KN, bool CONV, int CHAINS>
+__global__ __launch_bounds__(4 * 64 + (CONV ? 128 : 192), S > 4 ? 2 : CONV ? 3 : 4) void gemm_ring_kernel(GemmArgs p) {
     constexpr int BM = 64, BN = 64, BK = 64, NW = 4;
     constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
     constexpr int STAGE_BYTES = SLOTS * 1024, A_BYTES = SLOTS_A * 1024;
@@ -230,13 +235,15 @@ __global__ __launch_bounds__(4 * 64 + 192, S > 4 ? 2 : 4) void gemm_ring_kernel(
             }
         }
     };
-    float16v acc[1][1];
+    float16v acc[CHAINS];
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[0][0][r] = 0.0f;
+    for (int s = 0; s < CHAINS; s++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[s][r] = 0.0f;
     auto products = [&](auto SET) {
         constexpr int set = decltype(SET)::value;
 #pragma unroll
-        for (int ks = 0; ks < NKS; ks++) acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][ks], fa[set][ks], acc[0][0], 0, 0, 0);
+        for (int ks = 0; ks < NKS; ks++) acc[ks % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][ks], fa[set][ks], acc[ks % CHAINS], 0, 0, 0);
     };
 
     // what the store needs of memory, while the first tiles are on their way
@@ -285,34 +292,40 @@ __global__ __launch_bounds__(4 * 64 + 192, S > 4 ? 2 : 4) void gemm_ring_kernel(
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         barrier();                                        // every wave has read its last fragments
     }
+    float16v own[1][1] = {{acc[0]}};
+#pragma unroll
+    for (int s = 1; s < CHAINS; s++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) own[0][0][r] += acc[s][r];
     LnFold<1> ln;
     if (p.lnf_stats) {
         const float2v v = ln_slot[sm * 32 + frow];
         ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
     }
-    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, acc, cb, staging, m0, n0, sm, sn, wave, lane, bz, ln, S > 4 ? &res : nullptr);
+    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, own, cb, staging, m0, n0, sm, sn, wave, lane, bz, ln, S > 4 ? &res : nullptr);
 }
 
 constexpr int ring_lds_bytes(int S) { return S * 2 * 8192 + 2 * 64 * 8; }
 
-template <int S, bool B_KN, bool CONV>
+template <int S, bool B_KN, bool CONV, int CHAINS>
 int launch_ring(const GemmArgs &a, int64_t nbatch, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(a.lnf_stats ? 448 : 384), ring_lds_bytes(S), st, a);
+    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV, CHAINS>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(a.lnf_stats ? 448 : 384), ring_lds_bytes(S), st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
-template <bool CONV>
-int launch_stages(const GemmArgs &a, bool b_kn, bool deep, int64_t nbatch, hipStream_t st) {
-    if constexpr (!CONV) {
-        if (b_kn) return deep ? launch_ring<8, true, false>(a, nbatch, st) : launch_ring<4, true, false>(a, nbatch, st);
-    }
-    return deep ? launch_ring<8, false, CONV>(a, nbatch, st) : launch_ring<4, false, CONV>(a, nbatch, st);
+template <bool B_KN>
+int launch_plain(const GemmArgs &a, bool deep, bool one_chain, int64_t nbatch, hipStream_t st) {
+    if (!deep) return launch_ring<4, B_KN, false, 1>(a, nbatch, st);
+    return one_chain ? launch_ring<8, B_KN, false, 1>(a, nbatch, st) : launch_ring<8, B_KN, false, 4>(a, nbatch, st);
 }
-template <bool B_KN, bool CONV>
-int raise_ring() { return raise_lds(gemm_ring_kernel<8, B_KN, CONV>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, B_KN, CONV>, ring_lds_bytes(4)); }
+template <bool B_KN>
+int raise_plain() {
+    return raise_lds(gemm_ring_kernel<8, B_KN, false, 1>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<8, B_KN, false, 4>, ring_lds_bytes(8)) |
+           raise_lds(gemm_ring_kernel<4, B_KN, false, 1>, ring_lds_bytes(4));
+}
 
 }  // namespace
 
-int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t st) {
+int mi_ring_launch(const GemmArgs &args, bool one_chain, bool b_kn, int64_t nbatch, hipStream_t st) {
     GemmArgs a = args;
     set_tiles(a, 64, 64);
     a.vec_store = rows_vec16(a);
@@ -322,12 +335,12 @@ int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t 
     const bool deep = (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus();
     if (a.cv.xp) {
         if (b_kn || a.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
-        return launch_stages<true>(a, false, deep, nbatch, st);
+        return deep ? launch_ring<8, false, true, 4>(a, nbatch, st) : launch_ring<4, false, true, 4>(a, nbatch, st);
     }
     if ((int64_t)64 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
-    return launch_stages<false>(a, b_kn, deep, nbatch, st);
+    return b_kn ? launch_plain<true>(a, deep, one_chain, nbatch, st) : launch_plain<false>(a, deep, one_chain, nbatch, st);
 }
 
 int mi_ring_init() {
-    return raise_ring<false, true>() | raise_ring<true, false>() | raise_ring<false, false>();
+    return raise_plain<true>() | raise_plain<false>() | raise_lds(gemm_ring_kernel<8, false, true, 4>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, false, true, 4>, ring_lds_bytes(4));
 }

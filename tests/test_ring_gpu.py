@@ -42,3 +42,26 @@ def test_folded_norm(ctx, T, F, K):
     torch.cuda.synchronize()
     want = oracle.gemm_f16(oracle.layernorm_f16(x, g, beta, 1e-5)[0], W, b)
     assert_parity(to_host(out), want, what=f"T{T} K{K} F{F}")
+
+
+@pytest.mark.parametrize("T,K,F,chains", [(1000, 768, 1000, 4), (1000, 1536, 1000, 4), (300, 2304, 1000, 4), (1000, 5120, 1000, 4), (70, 3072, 768, 8), (12, 4832, 64, 16)])
+def test_error_against_64_bits(ctx, T, K, F, chains):
+    """fp32 results are as near as this many chains of fp32 sums leave them: 16-deep step j in chain j % chains, rounded after each half
+    of it, the chains then added pairwise.  (One chain is off by 1.8 to 2 times the figure of four; a twentieth is four times the
+    spread between this sum and the measured one.)  The last two are gemm_deep_kernel's."""
+    import torch
+    import juliavision_amd as jv
+    X, W = oracle.randn_f16((T, K), 1), oracle.randn_f16((K, F), 2, 0, 1.0 / np.sqrt(K))
+    out = poison(torch.empty((T, F), dtype=torch.float32, device="cuda"))
+    ctx.ws.reset()
+    jv.matmul_(ctx, out, to_dev(np.ascontiguousarray(W.T)).t(), to_dev(X))
+    n = min(T, 96)
+    x, w = X[:n].astype(np.float64), W.astype(np.float64)
+    want = x @ w
+    acc = np.zeros((chains, n, F), np.float32)
+    for k in range(0, K, 8):
+        acc[k // 16 % chains] = (acc[k // 16 % chains] + x[:, k:k + 8] @ w[k:k + 8]).astype(np.float32)
+    while len(acc) > 1:
+        acc = acc[::2] + acc[1::2]
+    err = lambda a: np.linalg.norm(a - want) / np.linalg.norm(want)
+    assert err(to_host(out)[:n].astype(np.float64)) <= 1.05 * err(acc[0].astype(np.float64))
