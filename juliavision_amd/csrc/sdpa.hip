@@ -103,7 +103,6 @@ __global__ __launch_bounds__((PP || KH == 2) ? 512 : 256, (EP <= 96 && !PP && KH
     half_t (*Ks)[BCS * KLD] = reinterpret_cast<half_t (*)[BCS * KLD]>(smem);
     half_t (*Vs)[BCS * VLD] = reinterpret_cast<half_t (*)[BCS * VLD]>(smem + 3 * BCS * KLD * 2);
     half_t *Ms = reinterpret_cast<half_t *>(smem + 3 * BCS * (KLD + VLD) * 2);       // BIAS 3: the mask row, then zeros
-    stage_args(p);
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int tid = threadIdx.x & (NT - 1);                  // index among the staging threads
@@ -664,7 +663,6 @@ template <int NCH, bool VEC>
 __global__ __launch_bounds__(256) void sdpa_rows_kernel(SdpaArgs p) {
     __shared__ float red_ml[4][2];
     __shared__ float red_o[4][64 * NCH];
-    stage_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 3, cl = lane & 7;
     const int split = blockIdx.x % p.nsplit;
@@ -856,7 +854,7 @@ __global__ __launch_bounds__(512) void sdpa_decode_kernel(SdpaArgs p) {
     __shared__ float red_ml[8][2];
     __shared__ float red_o[8][64];
     __shared__ int is_last;
-    stage_args(p);
+    stage_decode_args(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 3, cl = lane & 7;
     const int S = p.nsplit;
@@ -1157,7 +1155,11 @@ int flash_splits_over_workgroups(int64_t E, int64_t Lq, int64_t Lk, int64_t H, i
 int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, bool f32) {
     const int64_t wgs = ceil_div(Lq, 32) * H * B, nt = ceil_div(Lk, 32), cus = mi_num_cus(), blocks = ceil_div(Lk, 64);
     if (!mi_sdpa_tile_head_size(E) || Lq < 2 || Lk < 1) return 0;
-    const int waves = wgs <= cus && nt >= 16 ? 8 : wgs * 4 >= cus * 11 ? 2 : 4;
+    // Two waves from 2.75 workgroups a CU on; wide heads over few keys from 2.25 (600 workgroups, us on four waves | two: 64 wide
+    // over 159 keys 7.93 | 7.11, 300 8.83 | 8.30, 500 10.05 | 10.13; 72 8.32 | 7.85, 9.48 | 9.40, 11.1 | 11.8; 128 13.9 | 10.1, 15.9 | 11.9,
+    // 17.7 | 14.5; 32 5.73 | 5.68, 6.40 | 6.50, 7.23 | 8.05).
+    const bool wide_few = E >= 64 && wgs * 4 >= cus * 9 && (E == 128 || nt <= 12);
+    const int waves = wgs <= cus && nt >= 16 ? 8 : wgs * 4 >= cus * 11 || wide_few ? 2 : 4;
     const double tiles = (double)ceil_div(nt, waves), wide = E <= 64 ? 1.0 : E <= 96 ? 1.5 : 1.9;
     if (f32) {
         // Against a workgroup per query row (and key split, with a merge launch).  170 shapes of 2 to 63 queries, 16 to 4096

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
     constexpr int WPART = (ET * 16 + 2) * 256, WSTRIDE = WPART > 2 * TILE_BYTES ? WPART : 2 * TILE_BYTES;
     constexpr float UP = F32 ? 1024.0f : 1.0f, TH = F32 ? 4.0f : 8.0f;      // probabilities times UP stay in fp16 range
     extern __shared__ __align__(16) char smem[];
-    stage_args(p);
+    stage_tile_args(p);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hl = lane >> 5, l32 = lane & 31;
     char *const wave_lds = smem + wave * WSTRIDE;
@@ -64,9 +64,10 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
         const int total = p.nqb * p.H * p.B, xcd = blockIdx.x & 7, full = total >> 3, rem = total & 7;
         unsigned x, y;
         const unsigned hb = divide(xcd * full + min(xcd, rem) + (blockIdx.x >> 3), p.nqb, p.div_x, x);
-        b = divide(hb, p.H, p.div_h, y);
-        qblk = x;
-        h = y;
+        // (said to be scalar: the carry of a quotient was kept in a vector register as far as the mask copy, which spilled)
+        b = __builtin_amdgcn_readfirstlane(divide(hb, p.H, p.div_h, y));
+        qblk = __builtin_amdgcn_readfirstlane(x);
+        h = __builtin_amdgcn_readfirstlane(y);
     }
     const int q0 = qblk * 32;
     const half_t *qb = p.q + h * p.qs[2] + b * p.qs[3];

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("mask", ["none", "right", "left", "len"])
 @pytest.mark.parametrize("E", [16, 32, 64, 72, 128])
-@pytest.mark.parametrize("B,H,Lq,Lk", [(1, 1, 2, 1), (2, 3, 31, 33), (2, 2, 65, 97), (1, 2, 33, 545), (3, 16, 520, 64), (12, 20, 90, 130)])
+@pytest.mark.parametrize("B,H,Lq,Lk", [(1, 1, 2, 1), (2, 3, 31, 33), (2, 2, 65, 97), (1, 2, 33, 545), (3, 16, 520, 64), (12, 20, 90, 130), (6, 20, 159, 159)])
 def test_tiles(ctx, B, H, Lq, Lk, E, mask):
     import torch
     import juliavision_amd as jv
