@@ -1292,14 +1292,14 @@ constexpr int RING_TILE = 5, DEEP_TILE = 6, DEEP_SERIAL_TILE = 7;      // indice
 // tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
 // output, same bits (the 32 x 32 tiles are not planned for a gathered operand: their order of a long K is their own).
-int launch_tile(int tile, const GemmArgs &a, bool one_chain, bool b_kn, int64_t nbatch, hipStream_t st) {
+int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
     const bool plain = !a.ag.x && a.K % 64 == 0;
     switch (tile) {
         case 0: return plain ? launch_w4<128, 256, 1, 4>(a, b_kn, nbatch, st) : mi_pipe_launch(0, a, b_kn, nbatch, st);
         case 1: return plain ? launch_w4<192, 128, 2, 2>(a, b_kn, nbatch, st) : mi_pipe_launch(1, a, b_kn, nbatch, st);
         case RING_TILE:
             if (!a.ag.x) {
-                const int rc = mi_ring_launch(a, one_chain, b_kn, nbatch, st);
+                const int rc = mi_ring_launch(a, b_kn, nbatch, st);
                 if (rc != MI_DECLINE_EXTENT) return rc;     // declined: a row pitch beyond its 32-bit offsets
             }
             return mi_pipe_launch(4, a, b_kn, nbatch, st);
@@ -1403,6 +1403,7 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
     for (int split = 1; split <= max_split; split++) {
         if (split > 1 && (K % (64 * split) != 0 || K / split < 128)) continue;
         for (int tile = 0; tile < NTILES; tile++) {
+            if (tile == RING_TILE && split > 1 && K / split <= MI_LNA_KMAX) continue;      // (a slice would be one chain)
             if (tile == RING_TILE && ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > RING_WGS_PER_CU * mi_num_cus()) continue;
             if (tile == DEEP_TILE || tile == DEEP_SERIAL_TILE) {
                 if (!deep || (K > MI_LNA_KMAX) != (tile == DEEP_TILE)) continue;
@@ -1610,7 +1611,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
             s1.K = a.K / split;
             s1.sA = s1.K; s1.sB = b_kn ? (long)s1.K * a.ldB : s1.K; s1.sBias = 0;
             s1.ag.split = 1;
-            int rc = launch_tile(tp.tile, s1, false, b_kn, split, st);
+            int rc = launch_tile(tp.tile, s1, b_kn, split, st);
             if (rc != MI_OK) return rc;
             GemmArgs s2 = a;
             s2.vec_store = !a.out_f32 && a.ldY % 4 == 0 && aligned_to(a.Y, 8);
@@ -1633,7 +1634,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // has its own: the bits are the ones without a GELU.
         if (pipe && split == 1 && !own_order(tp.tile, a.K) && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
             tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep, lnf);
-        if (pipe) return launch_tile(tp.tile, a, a.K <= MI_LNA_KMAX, b_kn, nbatch, st);
+        if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
     return mi_any_launch(a, b_kn, false, nbatch, st);
@@ -1685,7 +1686,7 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     if (agather) a.ag = *agather;
     const bool addr = mfma_addressable(a, b_kn != 0);
     if ((gather || agather) && !addr) return MI_DECLINE_OPERANDS;
-    if (gather) return g_ready ? mi_ring_launch(a, false, false, nbatch, st) : MI_ERROR_DEVICE;
+    if (gather) return g_ready ? mi_ring_launch(a, false, nbatch, st) : MI_ERROR_DEVICE;
     int path = addr ? MI_GEMM_MFMA : MI_GEMM_SCALAR;
     return run_gemm(a, b_kn != 0, nbatch, ws, ws_bytes, st, path);
 }

@@ -712,8 +712,8 @@ int mi_pipe_launch(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipSt
 int mi_pipe_launch_ln(bool wide, const GemmArgs &a, bool b_kn, hipStream_t st);
 constexpr int MI_LNA_KMAX = 512;         // deepest K of the layer-norm prologue
 int mi_pipe_init();
-// gemm_ring.hip: small grids of ordinary operands, and patch matrices of a convolution.  one_chain: K in the order of the larger tiles.
-int mi_ring_launch(const GemmArgs &a, bool one_chain, bool b_kn, int64_t nbatch, hipStream_t st);
+// gemm_ring.hip: small grids of ordinary operands, and patch matrices of a convolution.
+int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_ring_init();
 // gemm_deep.hip: few output tiles, of ordinary operands.
 int mi_deep_launch(const GemmArgs &a, bool split_k, bool b_kn, int64_t nbatch, hipStream_t st);

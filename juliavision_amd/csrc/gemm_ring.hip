@@ -29,12 +29,13 @@ namespace {
 // CONV: B is the patch matrix of a convolution (ConvGather).  Its rows' offsets are as fixed as an ordinary operand's; what moves
 // from tile to tile is the tap, for all lanes alike where C is a multiple of 64, by the lane's pair of chunks otherwise.
 //
-// CHAINS: accumulators an element, the 16-deep step ks of every tile in chain ks % CHAINS.  Four from K = 513 on and for patches: one
+// Chains of fp32 sums an element, the 16-deep step ks of every tile in chain ks % chains: four from K = 513 on and for patches.  One
 // chain has 1.8 times the error of four (fp32 results against 64 bits: K = 768 1.78e-7 | 1.00e-7, 1536 2.49e-7 | 1.33e-7, 5120 4.55e-7 |
 // 2.32e-7) at the same time (1000 x 1536 -> 1000 8.13 | 8.17 us, 1000 x 5120 -> 1000 22.3 | 20.8).  One up to there, in the order of
 // every other tile: a call that folds a layer norm promises the bits of the norm and this GEMM apart.  One too for ordinary operands
-// past one workgroup a CU, whose registers are short.
-template <int S, bool B_KN, bool CONV, int CHAINS>
+// past one workgroup a CU, whose registers are short.  Both loops are in one kernel: as two, a model that alternates between them paid
+// for each one's cold instructions (ViT-S of 1370 tokens, 24 such launches: 529 us as two, 521 so, 514 with one chain throughout).
+template <int S, bool B_KN, bool CONV = false>
 __global__ __launch_bounds__(4 * 64 + (CONV ? 128 : 192), S > 4 ? 2 : CONV ? 3 : 4) void gemm_ring_kernel(GemmArgs p) {
     constexpr int BM = 64, BN = 64, BK = 64, NW = 4;
     constexpr int SLOTS_A = BM / 8, SLOTS = (BM + BN) / 8;        // 1 KB requests of a stage
@@ -235,15 +236,11 @@ __global__ __launch_bounds__(4 * 64 + (CONV ? 128 : 192), S > 4 ? 2 : CONV ? 3 :
             }
         }
     };
-    float16v acc[CHAINS];
+    float16v acc[1][1];
+    auto products = [&](auto &chain, auto SET) __attribute__((always_inline)) {
+        constexpr int ch = sizeof(chain) / sizeof(float16v), set = decltype(SET)::value;
 #pragma unroll
-    for (int s = 0; s < CHAINS; s++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[s][r] = 0.0f;
-    auto products = [&](auto SET) {
-        constexpr int set = decltype(SET)::value;
-#pragma unroll
-        for (int ks = 0; ks < NKS; ks++) acc[ks % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][ks], fa[set][ks], acc[ks % CHAINS], 0, 0, 0);
+        for (int ks = 0; ks < NKS; ks++) chain[ks % ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[set][ks], fa[set][ks], chain[ks % ch], 0, 0, 0);
     };
 
     // what the store needs of memory, while the first tiles are on their way
@@ -260,25 +257,41 @@ __global__ __launch_bounds__(4 * 64 + (CONV ? 128 : 192), S > 4 ? 2 : CONV ? 3 :
     // its predecessor's stage is free for the loaders; the successor's fragments are requested, then its products issued.
     // (The steady state has no branch: where a tile may or may not have a successor, the compiler's wait for its fragments is also
     // one for the successor's, and a turn is longer by an LDS latency.)
-    auto turn = [&](auto SET, auto NEXT, int kt) {
+    auto turn = [&](auto &chain, auto SET, auto NEXT, int kt) __attribute__((always_inline)) {
         barrier();
         fetch(NEXT, kt + 1);
         __builtin_amdgcn_sched_barrier(0);                // the reads go out ahead of the products,
-        products(SET);
+        products(chain, SET);
         __builtin_amdgcn_sched_barrier(0);                // which stay ahead of the next barrier: by then this tile has been read
     };
-    // (an odd tile comes first: one way into the loop and one out of it, or the accumulators are copied between registers)
-    if (nk & 1) {
-        fetch(I1{}, 0);
-        if (nk > 1) turn(I1{}, I0{}, 0);
-    } else fetch(I0{}, 0);
-    int kt = nk & 1;
-    for (; kt + 2 < nk; kt += 2) {
-        turn(I0{}, I1{}, kt);
-        turn(I1{}, I0{}, kt + 1);
-    }
-    if (nk > 1) turn(I0{}, I1{}, kt);
-    products(I1{});
+    auto tiles = [&](auto CH) __attribute__((always_inline)) {
+        constexpr int ch = decltype(CH)::value;
+        float16v chain[ch];
+#pragma unroll
+        for (int s = 0; s < ch; s++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) chain[s][r] = 0.0f;
+        // (an odd tile comes first: one way into the loop and one out of it, or the accumulators are copied between registers)
+        if (nk & 1) {
+            fetch(I1{}, 0);
+            if (nk > 1) turn(chain, I1{}, I0{}, 0);
+        } else fetch(I0{}, 0);
+        int kt = nk & 1;
+        for (; kt + 2 < nk; kt += 2) {
+            turn(chain, I0{}, I1{}, kt);
+            turn(chain, I1{}, I0{}, kt + 1);
+        }
+        if (nk > 1) turn(chain, I0{}, I1{}, kt);
+        products(chain, I1{});
+        acc[0][0] = chain[0];
+#pragma unroll
+        for (int s = 1; s < ch; s++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[0][0][r] += chain[s][r];
+    };
+    if constexpr (CONV) tiles(std::integral_constant<int, 4>{});
+    else if (S > 4 && p.K > MI_LNA_KMAX) tiles(std::integral_constant<int, 4>{});
+    else tiles(I1{});
 
     // Past its last barrier of the loop a wave knows that every wave has read all tiles but the last two.  The store's staging keeps
     // clear of their stages where the ring has room for it elsewhere.
@@ -292,40 +305,34 @@ __global__ __launch_bounds__(4 * 64 + (CONV ? 128 : 192), S > 4 ? 2 : CONV ? 3 :
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         barrier();                                        // every wave has read its last fragments
     }
-    float16v own[1][1] = {{acc[0]}};
-#pragma unroll
-    for (int s = 1; s < CHAINS; s++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) own[0][0][r] += acc[s][r];
     LnFold<1> ln;
     if (p.lnf_stats) {
         const float2v v = ln_slot[sm * 32 + frow];
         ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN; ln.r[0] = v[0]; ln.rmu[0] = v[1];
     }
-    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, own, cb, staging, m0, n0, sm, sn, wave, lane, bz, ln, S > 4 ? &res : nullptr);
+    store_tile<1, 1, 32, 32, NW, S * STAGE_BYTES>(p, acc, cb, staging, m0, n0, sm, sn, wave, lane, bz, ln, S > 4 ? &res : nullptr);
 }
 
 constexpr int ring_lds_bytes(int S) { return S * 2 * 8192 + 2 * 64 * 8; }
 
-template <int S, bool B_KN, bool CONV, int CHAINS>
+template <int S, bool B_KN, bool CONV>
 int launch_ring(const GemmArgs &a, int64_t nbatch, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV, CHAINS>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(a.lnf_stats ? 448 : 384), ring_lds_bytes(S), st, a);
+    hipLaunchKernelGGL((gemm_ring_kernel<S, B_KN, CONV>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(a.lnf_stats ? 448 : 384), ring_lds_bytes(S), st, a);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
-template <bool B_KN>
-int launch_plain(const GemmArgs &a, bool deep, bool one_chain, int64_t nbatch, hipStream_t st) {
-    if (!deep) return launch_ring<4, B_KN, false, 1>(a, nbatch, st);
-    return one_chain ? launch_ring<8, B_KN, false, 1>(a, nbatch, st) : launch_ring<8, B_KN, false, 4>(a, nbatch, st);
+template <bool CONV>
+int launch_stages(const GemmArgs &a, bool b_kn, bool deep, int64_t nbatch, hipStream_t st) {
+    if constexpr (!CONV) {
+        if (b_kn) return deep ? launch_ring<8, true, false>(a, nbatch, st) : launch_ring<4, true, false>(a, nbatch, st);
+    }
+    return deep ? launch_ring<8, false, CONV>(a, nbatch, st) : launch_ring<4, false, CONV>(a, nbatch, st);
 }
-template <bool B_KN>
-int raise_plain() {
-    return raise_lds(gemm_ring_kernel<8, B_KN, false, 1>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<8, B_KN, false, 4>, ring_lds_bytes(8)) |
-           raise_lds(gemm_ring_kernel<4, B_KN, false, 1>, ring_lds_bytes(4));
-}
+template <bool B_KN, bool CONV>
+int raise_ring() { return raise_lds(gemm_ring_kernel<8, B_KN, CONV>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, B_KN, CONV>, ring_lds_bytes(4)); }
 
 }  // namespace
 
-int mi_ring_launch(const GemmArgs &args, bool one_chain, bool b_kn, int64_t nbatch, hipStream_t st) {
+int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t st) {
     GemmArgs a = args;
     set_tiles(a, 64, 64);
     a.vec_store = rows_vec16(a);
@@ -335,12 +342,12 @@ int mi_ring_launch(const GemmArgs &args, bool one_chain, bool b_kn, int64_t nbat
     const bool deep = (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus();
     if (a.cv.xp) {
         if (b_kn || a.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
-        return deep ? launch_ring<8, false, true, 4>(a, nbatch, st) : launch_ring<4, false, true, 4>(a, nbatch, st);
+        return launch_stages<true>(a, false, deep, nbatch, st);
     }
     if ((int64_t)64 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
-    return b_kn ? launch_plain<true>(a, deep, one_chain, nbatch, st) : launch_plain<false>(a, deep, one_chain, nbatch, st);
+    return launch_stages<false>(a, b_kn, deep, nbatch, st);
 }
 
 int mi_ring_init() {
-    return raise_plain<true>() | raise_plain<false>() | raise_lds(gemm_ring_kernel<8, false, true, 4>, ring_lds_bytes(8)) | raise_lds(gemm_ring_kernel<4, false, true, 4>, ring_lds_bytes(4));
+    return raise_ring<false, true>() | raise_ring<true, false>() | raise_ring<false, false>();
 }
