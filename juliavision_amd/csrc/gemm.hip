@@ -830,7 +830,9 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
             w[i] = on && row < cols ? ldg16(wrow + k) : z;
             x[i] = on && row < p.M ? ldg16(xrow + k) : z;
             if constexpr (LN) {
-                g[i] = on && p.ln_gamma ? ldg16(p.ln_gamma + k) : z;
+                // (columns that are not there have gamma zero, whatever the row's mean: as a half it may be an infinity)
+                const u32x4 ones = {0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u};
+                g[i] = !on ? z : p.ln_gamma ? ldg16(p.ln_gamma + k) : ones;
                 b[i] = on && p.ln_beta ? ldg16(p.ln_beta + k) : z;
             }
         }
@@ -870,7 +872,7 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
             if constexpr (LN) {
                 const half8v gv = as_half8(g[i]), be = as_half8(b[i]);
 #pragma unroll
-                for (int j = 0; j < 8; j++) xv[j] = ln_norm1((float)xv[j], mu, rs, p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)be[j]);
+                for (int j = 0; j < 8; j++) xv[j] = ln_norm1((float)xv[j], mu, rs, true, (float)gv[j], p.ln_beta != nullptr, (float)be[j]);
             }
             acc[i % NA] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(w[i]), xv, acc[i % NA], 0, 0, 0);      // (steps past the share multiply zeros)
         }

@@ -37,3 +37,21 @@ def test_rows(ctx, T, K, F):
     jv.matmul_(ctx, apart, w, h, db)
     if K <= 4096:                                         # the norm kernel walks longer rows in another order
         assert torch.equal(folded, apart)
+
+
+@pytest.mark.parametrize("beta", [False, True])
+@pytest.mark.parametrize("K", [8, 40, 1280, 1288])
+def test_norm_without_gamma_of_rows_far_from_zero(ctx, K, beta):
+    """The columns that pad a wave's share have no value to normalise: minus the mean times 1 / sigma is beyond fp16 here."""
+    import torch
+    import juliavision_amd as jv
+    T, F = 6, 40
+    X = np.full((T, K), 900.0, np.float16)
+    X[1::2, ::3] = 901.0
+    W, be = oracle.randn_f16((K, F), 2, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K,), 6, 0, 0.1)
+    out = poison(torch.empty((T, F), dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.ln_matmul_(ctx, out, to_dev(np.ascontiguousarray(W.T)).t(), to_dev(X), None, to_dev(be) if beta else None, 1e-5, None)
+    h = poison(torch.empty((T, K), dtype=torch.float16, device="cuda"))
+    jv.layernorm_(ctx, h, None, None, to_dev(X), None, to_dev(be) if beta else None, K, 1e-5)
+    assert_parity(to_host(out), oracle.gemm_f16(to_host(h), W), what=f"K{K} beta {beta}")
