@@ -152,10 +152,14 @@ def decoder_layer_step(ctx: Ctx, W: DecoderLayerWeights, cache: KVCache, layer: 
         # eight rows that the decode-sized kernels take, where they are one launch ([F][K] weights)
         ctx.ws.reset()
         if B <= (8 if w.stride(0) == 1 else 4):
-            ln_matmul_(ctx, dst, w, src, g, b_, eps, bias, epi=epi)
-        else:
-            layernorm_(ctx, buf.h, None, None, src, g, b_, d, eps)
-            matmul_(ctx, dst, w, buf.h, bias, epi=epi)
+            try:
+                ln_matmul_(ctx, dst, w, src, g, b_, eps, bias, epi=epi)
+                return
+            except DeclineError:                           # before anything is launched: operands off 16 bytes, d_model past 8192
+                if B <= 4:
+                    raise
+        layernorm_(ctx, buf.h, None, None, src, g, b_, d, eps)
+        matmul_(ctx, dst, w, buf.h, bias, epi=epi)
 
     normed_linear(buf.qkv, W.wqkv, x, W.ln1_g, W.ln1_b, W.bqkv)
     q, k_new, v_new = memo_view(buf, "qkv", (d, H, E), lambda t: tuple(t[:, i * d:(i + 1) * d].unflatten(1, (H, 1, E)) for i in range(3)))

@@ -131,6 +131,37 @@ def test_decoder_layer_steps_match_oracle(ctx, B, layout):
         assert_parity(to_host(cache.self_k[0]), hk, what=f"self_k after step {step}")
 
 
+@pytest.mark.parametrize("off", ["gamma", "beta", "weight address", "weight pitch"])
+def test_decoder_layer_step_of_operands_off_sixteen_bytes(ctx, off):
+    """Six rows: the norms fold into the linears behind them where their operands allow it, and run as launches of their own elsewhere."""
+    import torch
+    from dataclasses import replace
+    from juliavision_amd.decode import DecodeBuffers, KVCache, decoder_layer_step
+    B, d, H, E, ffn, Ls = 6, 256, 4, 64, 512, 40
+    Wh, Wd = _weights(d, ffn, 100, "fk")
+
+    def moved(t):                                          # the same values at an odd address
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape)
+        return buf.copy_(t)
+
+    def pitched(w):                                        # ... or with an odd row pitch
+        buf = torch.empty((w.shape[1], w.shape[0] + 1), dtype=w.dtype, device="cuda")[:, :w.shape[0]]
+        return buf.copy_(w.t()).t()
+
+    Wd = replace(Wd, **{"gamma": {"ln1_g": moved(Wd.ln1_g), "ln3_g": moved(Wd.ln3_g)}, "beta": {"ln2_b": moved(Wd.ln2_b)},
+                        "weight address": {"wqkv": moved(Wd.wqkv.t()).t(), "w1": moved(Wd.w1.t()).t()}, "weight pitch": {"wq_c": pitched(Wd.wq_c)}}[off])
+    cache = KVCache(1, B, H, E, max_target=8, src_len=Ls)
+    ck, cv = oracle.randn_f16((1, B, H, Ls, E), 31), oracle.randn_f16((1, B, H, Ls, E), 32)
+    cache.cross_k.copy_(to_dev(ck))
+    cache.cross_v.copy_(to_dev(cv))
+    hk, hv = (np.zeros((B, H, 8, E), dtype=np.float16) for _ in range(2))
+    x, out = oracle.randn_f16((B, d), 60), poison(torch.empty((B, d), dtype=torch.float16, device="cuda"))
+    cache.advance(ctx)
+    decoder_layer_step(ctx, Wd, cache, 0, to_dev(x), out, DecodeBuffers(B, d, ffn))
+    want = _oracle_layer_step(Wh, x, hk, hv, ck[0], cv[0], np.ones(B, np.int32), H, E)
+    assert_parity(to_host(out), want, what=off)
+
+
 def test_weights_relaid_at_load_run_the_one_launch_linears(ctx):
     """DecoderLayerWeights.k_contiguous: [K][F] weights re-laid once to [F][K] hold the same values, and a layer step
     over them gives the bits of a step over weights that were [F][K] from the start."""
