@@ -446,7 +446,8 @@ bool mi_sdpa_tile_keymask(const SdpaArgs &p) { return p.bias && !p.bias_f32 && (
 bool mi_sdpa_tile_takes(const SdpaArgs &p) {
     if (!mi_sdpa_tile_head_size(p.E)) return false;
     if (p.bias && !mi_sdpa_tile_keymask(p) && p.bs[1] == 0) return false;
-    if (ceil_div(p.Lq, 32) * p.H * p.B > INT32_MAX) return false;
+    // a launch has fewer than 2^32 threads along its one dimension (grids of this size run two waves a workgroup)
+    if ((int64_t)ceil_div(p.Lq, 32) * p.H * p.B * 128 > UINT32_MAX) return false;
     // per-lane load offsets are 32-bit byte offsets from a tile's first row
     return p.ks[1] >= 0 && p.vs[1] >= 0 && p.ks[1] * 64 < (1l << 31) && p.vs[1] * 64 < (1l << 31);
 }

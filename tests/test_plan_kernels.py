@@ -47,6 +47,9 @@ def test_what_the_tiles_do_not_take():
     assert _sdpa(72, 23, 300, 8, 2)[1] == "tiles_f32" and _sdpa(72, 23, 300, 8, 2, f32=True)[1] == "rows"
     assert _sdpa(64, 23, 300, 8, 2, mask="key")[1] == "tiles_f32" and _sdpa(64, 23, 300, 8, 2, mask="key32")[1] == "rows"
     assert _sdpa(64, 1, 1500, 20, 1)[1:] == ("one_query", 4, 4)
+    # 2^25 workgroups of 128 threads are more than one launch dimension holds
+    assert _sdpa(16, 2, 64, 512, 65535)[1] == "tiles_f32" and _sdpa(16, 2, 64, 520, 65535)[1] == "rows"
+    assert _sdpa(16, 128, 64, 128, 65535)[1] == "tiles" and _sdpa(16, 128, 64, 130, 65535)[1] == "fused"
 
 
 def test_the_workspace_covers_whichever_convolution_kernel_runs():
