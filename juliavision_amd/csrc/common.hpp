@@ -142,6 +142,8 @@ static inline bool aligned_to(const void *p, size_t a) { return (reinterpret_cas
 // NaN by its bits: the build tells the compiler that no NaNs occur, which folds comparisons with one away.
 static inline bool is_nan_arg(float x) { uint32_t u; __builtin_memcpy(&u, &x, 4); return (u & 0x7fffffffu) > 0x7f800000u; }
 
+// Largest image, in halves, of the gather below: gemm_ring_kernel's offsets into it are 32-bit byte offsets, raised by up to 3072.
+constexpr int64_t MI_PATCH_IMAGE_MAX = INT32_MAX - 1536;
 // Implicit-GEMM convolution over a zero-padded channels-last copy xp[img][Hp][Wp][C] of the input: how gemm_ring_kernel finds
 // its [N][K] operand (row n = output pixel (oh, ow), K ordered (kh, kw, ci) with ci fastest) in it.  Sixteen bytes of a
 // row are eight channels of one tap, at an offset from the pixel's origin that is the same for every pixel.

@@ -239,7 +239,7 @@ int conv_path(const ConvArgs &a) {
 // workspace asked for is the one the call finds: x and w may lie at any address (conv_pad_kernel's reads ask for none).
 bool patch_ok(const ConvArgs &a) {
     const int64_t Hp = a.Hi + 2 * a.py, Wp = a.Wi + 2 * a.px;
-    return a.groups == 1 && a.Cin % 16 == 0 && turn_group(a) >= 8 && (int64_t)Hp * Wp * a.Cin <= INT32_MAX && (int64_t)a.Cout * a.Cin * a.KH * a.KW <= INT32_MAX / 8;
+    return a.groups == 1 && a.Cin % 16 == 0 && turn_group(a) >= 8 && (int64_t)Hp * Wp * a.Cin <= MI_PATCH_IMAGE_MAX && (int64_t)a.Cout * a.Cin * a.KH * a.KW <= INT32_MAX / 8;
 }
 size_t patch_copy_bytes(const ConvArgs &a) { return round_up((size_t)a.N * a.Cin * (a.Hi + 2 * a.py) * (a.Wi + 2 * a.px) * 2, 256); }
 size_t patch_weight_bytes(const ConvArgs &a) { return round_up((size_t)a.Cout * a.Cin * a.KH * a.KW * 2, 256); }

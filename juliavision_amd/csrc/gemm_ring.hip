@@ -341,7 +341,7 @@ int mi_ring_launch(const GemmArgs &args, bool b_kn, int64_t nbatch, hipStream_t 
     // past one workgroup a CU, half the stages: two of them on a CU (96 -> 384 channels, 3 x 3 stride 2, 27 x 445: 21.1 -> 19.1 us)
     const bool deep = (int64_t)a.tiles_m * a.tiles_n * nbatch <= mi_num_cus();
     if (a.cv.xp) {
-        if (b_kn || a.cv.img > INT32_MAX) return MI_DECLINE_EXTENT;
+        if (b_kn || a.cv.img > MI_PATCH_IMAGE_MAX) return MI_DECLINE_EXTENT;
         return launch_stages<true>(a, false, deep, nbatch, st);
     }
     if ((int64_t)64 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;

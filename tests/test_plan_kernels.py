@@ -52,6 +52,13 @@ def test_what_the_tiles_do_not_take():
     assert _sdpa(16, 128, 64, 128, 65535)[1] == "tiles" and _sdpa(16, 128, 64, 130, 65535)[1] == "fused"
 
 
+def test_the_largest_image_of_the_patch_gather():
+    """Its byte offsets are 32 bits and are raised by up to 3072 on their way into the loads."""
+    kernel = lambda h: L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(47, h, 256, 1, 3, 3, 512, 4, 4, 0, 0, 1, 1, 1, C.byref(C.c_size_t(0)))]
+    assert 47 * 178481 * 256 > 2 ** 31 - 1536 > 47 * 178480 * 256
+    assert kernel(178480) == "patch_gemm" and kernel(178481) == "im2col_gemm"
+
+
 def test_the_workspace_covers_whichever_convolution_kernel_runs():
     import random
     rng, lib, seen = random.Random(0), L.load(), set()
