@@ -1405,7 +1405,9 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
     const int max_split = (may_split && nbatch == 1 && M > 8 && N % 4 == 0 && K % 64 == 0) ? 8 : 1;
     for (int split = 1; split <= max_split; split++) {
         if (split > 1 && (K % (64 * split) != 0 || K / split < 128)) continue;
-        for (int tile = 0; tile < NTILES; tile++) {
+        // planes that mi_gemm_f16_noalloc has room for: a call is not refused there because its estimate moved
+        const bool planes = split == 1 || (double)split * (double)M * (double)N * 4.0 <= (double)MI_NOALLOC_SCRATCH_BYTES;
+        for (int tile = 0; planes && tile < NTILES; tile++) {
             if (tile == RING_TILE && split > 1 && K / split <= MI_LNA_KMAX) continue;      // (a slice would be one chain)
             if (tile == RING_TILE && ceil_div(M, 64) * ceil_div(N, 64) * nbatch * split > RING_WGS_PER_CU * mi_num_cus()) continue;
             if (tile == DEEP_TILE || tile == DEEP_SERIAL_TILE) {

@@ -41,6 +41,12 @@ def test_compute_calls_refuse_without_a_device():
         L.init()
 
 
+@pytest.mark.parametrize("T,K,F", [(8416, 7936, 832), (6740, 7872, 1128), (1670, 6656, 5048), (4617, 6656, 1680), (1188, 7424, 6504), (5736, 7424, 1536)])
+def test_tiled_calls_fit_the_static_scratch(T, K, F):
+    """K-slices are planned within what ``mi_gemm_f16_noalloc`` holds, so that no tiled GEMM is refused there for its planes."""
+    assert L.load().mi_gemm_f16_workspace(T, K, F, L.W_KF, 1) <= L.NOALLOC_SCRATCH_BYTES
+
+
 def _gemm_plan(T, K, F, *, ldY=None, ldX=None, ldW=None, layout=L.W_KF, y=0x10000, x=0x20000, w=0x30000, dt=L.F16, nb=1):
     ldY = F if ldY is None else ldY
     ldX = K if ldX is None else ldX
