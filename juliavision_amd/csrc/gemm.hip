@@ -1343,10 +1343,10 @@ constexpr TileModel TILE_MODELS[NTILES] = {
     {32, 32, 0.142, 0.112, 0.8, 3.14, 0.409, 1.15},      // gemm_deep_kernel, one chain of sums
 };
 constexpr int64_t RING_WGS_PER_CU = 11, DEEP_WGS = 256;      // as many as the fits have seen
-// A folded norm costs the four-wave kernel and the ring more than the pipelined kernel, whose threads take the statistics in before the K
-// loop: the same kernels behind each other in a model, whole blocks, 1280 wide: 572 tokens 227 -> 216 us for three blocks with these, 700
-// 231 -> 224, 1500 352 -> 351; 900 x 1024 209 -> 202; 1370 x 384 132 either way.  (Alone, on weights that L2 holds, 192 x 128 tiles win.)
-constexpr double LNF_W4_US = 3.0, LNF_RING_US = 1.0;
+// A folded norm costs the four-wave kernel, which gives it a wave beside the K loop, more than the pipelined kernel, whose threads take the
+// statistics in before it, where other kernels' weights come between.  Three blocks of 64 to 1500 tokens, 384 to 1280 wide (35 stacks,
+// replayed): 572 x 1280 235 -> 223 us with this, 1100 x 1024 259 -> 252, the others within 1 %.
+constexpr double LNF_W4_US = 3.0;
 struct TilePlan { int tile, split; bool peer; double us; };      // peer: the K-slices exchange partial tiles in the kernel (no planes)
 
 double tile_cost_us(int64_t M, int64_t N, int64_t K, int64_t nbatch, int tile, int split, bool gelu = false) {
@@ -1415,7 +1415,7 @@ TilePlan estimate_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool ma
                 if (ceil_div(M, 32) * ceil_div(N, 32) * nbatch * split > std::min(DEEP_WGS, (int64_t)mi_num_cus())) continue;
             }
             if (gelu && own_order(tile, K)) continue;
-            const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu) + (!lnf ? 0.0 : tile <= 1 ? LNF_W4_US : tile == RING_TILE ? LNF_RING_US : 0.0);
+            const double us = tile_cost_us(M, N, K, nbatch, tile, split, gelu) + (lnf && tile <= 1 ? LNF_W4_US : 0.0);
             if (us < best_us) { best_us = us; best = {tile, split, false, us}; }
         }
         if (max_split > 1 && sk_planned()) {
