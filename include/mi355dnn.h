@@ -56,6 +56,18 @@ enum mi_bias_mode { MI_BIAS_NONE = 0, MI_BIAS_COL = 1, MI_BIAS_ROW = 2 };
 /* Which kernel a GEMM call takes; returned by mi_gemm_f16_plan so a host-side
  * planner (the reference's `mmplan`, matmul.jl:87-95) can be tested without a launch. */
 enum mi_gemm_path { MI_GEMM_DECLINE = 0, MI_GEMM_MFMA = 1, MI_GEMM_SKINNY = 2, MI_GEMM_SCALAR = 3 };
+/* ... and which kernel of the matrix path runs (mi_gemm_f16_kernel). */
+enum mi_gemm_kernel {
+    MI_GEMM_KERNEL_NONE = 0,        /* not that path, or rows that are no multiple of 16 bytes */
+    MI_GEMM_KERNEL_ONE_TILE = 1,    /* K up to 64 */
+    MI_GEMM_KERNEL_WIDE = 2,        /* 128 x 256 and 192 x 128 tiles */
+    MI_GEMM_KERNEL_STAGED = 3,      /* 128 x 128 to 64 x 64 tiles staged through registers */
+    MI_GEMM_KERNEL_RING = 4,        /* 64 x 64 tiles over a ring of direct-to-LDS stages, at most one workgroup a CU */
+    MI_GEMM_KERNEL_RING_SHALLOW = 5,/* the same with half the stages, two workgroups a CU */
+    MI_GEMM_KERNEL_DEEP = 6,        /* 32 x 32 tiles, K split over the waves */
+    MI_GEMM_KERNEL_DEEP_SERIAL = 7, /* 32 x 32 tiles, K in one chain */
+    MI_GEMM_KERNEL_EXCHANGE = 8     /* 128 x 128 tiles, two slices of K that exchange partial tiles */
+};
 enum mi_sdpa_path { MI_SDPA_DECLINE = 0, MI_SDPA_FLASH = 1, MI_SDPA_ROWS = 2 };
 /* ... and which kernel of that path runs (mi_sdpa_f16_kernel). */
 enum mi_sdpa_kernel {
@@ -311,6 +323,11 @@ int mi_gemm_f16_plan(const void *Y, const void *X, const void *W,
 int mi_gemm_f16_plan_caps(const int64_t caps[6], const void *Y, const void *X, const void *W,
                           int64_t T, int64_t K, int64_t F, int64_t ldY, int64_t ldX, int64_t ldW,
                           int w_layout, int out_dtype, int64_t nbatch, int64_t sY, int64_t sX, int64_t sW, int *ksplit_out);
+
+/* Which kernel mi_gemm_f16 runs for these extents on the current device (an mi_gemm_kernel), operands and results on 16 bytes with a
+ * workspace of the size asked for; folded_norm: mi_lnfold_gemm_f16.  ksplit_out (optional): the slices of K, each on that
+ * kernel.  Never launches, needs no GPU.  (The reference's plans name their kernels: matmul.jl:87-95.) */
+int mi_gemm_f16_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch, int epi, int folded_norm, int *ksplit_out);
 
 /* ---------------------------------------------------------------- attention
  * out(E,Lq,H,B) = softmax_over_keys(scale * q.k + bias) . v

@@ -22,6 +22,7 @@ W_KF, W_FK = 0, 1
 BIAS_NONE, BIAS_COL, BIAS_ROW = 0, 1, 2
 GEMM_PATHS = {0: "decline", 1: "mfma", 2: "skinny", 3: "scalar"}
 SDPA_PATHS = {0: "decline", 1: "flash", 2: "rows"}
+GEMM_KERNELS = {0: "none", 1: "one_tile", 2: "wide", 3: "staged", 4: "ring", 5: "ring_shallow", 6: "deep", 7: "deep_serial", 8: "exchange"}
 SDPA_KERNELS = {0: "none", 1: "fused", 2: "tiles", 3: "tiles_f32", 4: "rows", 5: "one_query"}
 CONV_PATHS = {0: "decline", 1: "gemm_1x1", 2: "im2col_gemm", 3: "direct", 4: "implicit_gemm"}
 CONV_KERNELS = {0: "none", 1: "gemm_1x1", 2: "im2col_gemm", 3: "direct", 4: "patch_gemm", 5: "tile"}
@@ -58,6 +59,7 @@ SIGNATURES = {
     "mi_gemm_f16_noalloc": (_int, [_vp] * 5 + [_i64] * 6 + [_int] * 4 + [_vp]),
     "mi_gemm_f16_plan": (_int, [_vp] * 3 + [_i64] * 6 + [_int] * 2 + [_i64] * 4),
     "mi_gemm_f16_plan_caps": (_int, [_i64p] + [_vp] * 3 + [_i64] * 6 + [_int] * 2 + [_i64] * 4 + [C.POINTER(C.c_int)]),
+    "mi_gemm_f16_kernel": (_int, [_i64] * 4 + [_int] * 2 + [C.POINTER(C.c_int)]),
     "mi_sdpa_f16_plan_caps": (_int, [_i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _int, _int] + [_i64] * 5 + [_f32, C.POINTER(C.c_int)]),
     "mi_sdpa_f16": (_int, [_vp, _int, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _int, _i64p, _vp] + [_i64] * 5 + [_f32, _vp, _sz, _vp]),
     "mi_sdpa_f16_workspace": (_sz, [_i64] * 5 + [_int]),

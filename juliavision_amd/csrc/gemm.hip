@@ -1823,6 +1823,24 @@ int mi_gemm_f16_plan_caps(const int64_t caps[6], const void *Y, const void *X, c
     return path;
 }
 
+int mi_gemm_f16_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch, int epi, int folded_norm, int *ksplit_out) {
+    if (ksplit_out) *ksplit_out = 1;
+    if (T <= 8 || K < 8 || K % 8 || F < 8 || F % 8 || nbatch < 1 || T > INT32_MAX || K > INT32_MAX || F > INT32_MAX) return MI_GEMM_KERNEL_NONE;
+    if (K <= 64) return MI_GEMM_KERNEL_ONE_TILE;
+    const bool lnf = folded_norm != 0;
+    TilePlan tp = plan_tiles(T, F, K, nbatch, !lnf, false, true, lnf);
+    if (tp.split == 1 && !own_order(tp.tile, K) && (epi == MI_EPI_GELU_ERF || epi == MI_EPI_GELU_TANH)) tp = plan_tiles(T, F, K, nbatch, false, true, true, lnf);
+    if (ksplit_out) *ksplit_out = tp.split;
+    if (tp.peer) return MI_GEMM_KERNEL_EXCHANGE;
+    switch (tp.tile) {
+        case 0: case 1: return MI_GEMM_KERNEL_WIDE;
+        case RING_TILE: return ceil_div(T, 64) * ceil_div(F, 64) * nbatch * tp.split <= mi_num_cus() ? MI_GEMM_KERNEL_RING : MI_GEMM_KERNEL_RING_SHALLOW;
+        case DEEP_TILE: return MI_GEMM_KERNEL_DEEP;
+        case DEEP_SERIAL_TILE: return MI_GEMM_KERNEL_DEEP_SERIAL;
+        default: return MI_GEMM_KERNEL_STAGED;
+    }
+}
+
 int mi_gemm_f16_batched(void *Y, const void *X, const void *W, const void *bias, const void *residual,
                         int64_t T, int64_t K, int64_t F, int64_t ldY, int64_t ldX, int64_t ldW,
                         int w_layout, int bias_mode, int epi, int out_dtype,

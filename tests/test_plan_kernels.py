@@ -36,6 +36,22 @@ def test_the_kernel_is_one_of_the_plans_path(packed):
     assert seen == {"none"} | OF_PATH["flash"] | OF_PATH["rows"] or seen == OF_PATH["flash"] | OF_PATH["rows"]
 
 
+def test_which_kernel_a_gemm_runs():
+    kernel = lambda T, K, F, epi="none", folded=0: L.GEMM_KERNELS[L.load().mi_gemm_f16_kernel(T, K, F, 1, L.EPI[epi], folded, None)]
+    for K in (72, 128, 256, 512, 520, 1024, 2304):           # few tiles: 32 x 32 ones, K in one chain up to 512
+        assert kernel(9, K, 64) == kernel(70, K, 72) == ("deep" if K > 512 else "deep_serial")
+    for K in (520, 640, 768, 1152, 2304):
+        assert kernel(500, K, 504) == "deep" and kernel(500, K, 520) == "ring"      # 256 tiles of 32 x 32, and more
+    assert kernel(1500, 1280, 5120, "gelu") == "wide" and kernel(1544, 1288, 1288) == "staged" and kernel(1500, 5120, 1280) == "exchange"
+    assert kernel(8, 1280, 1280) == kernel(100, 1284, 64) == "none" and kernel(100, 64, 64) == "one_tile"
+    # a GELU moves a call only between tiles that sum K in one order
+    for T, K, F in itertools.product((70, 300, 500, 1000, 1370, 3000), (384, 520, 1024, 1536, 2304), (64, 384, 520, 1536, 4096)):
+        plain, gelu = kernel(T, K, F), kernel(T, K, F, "gelu")
+        own = {"ring", "ring_shallow", "deep", "exchange"}
+        if K > 512:
+            assert (plain in own) == (gelu in own) and (plain not in own or plain == gelu), (T, K, F)
+
+
 def test_what_the_tiles_do_not_take():
     assert _sdpa(64, 256, 256, 8, 4)[1] == "tiles"
     assert _sdpa(64, 256, 256, 8, 4, q=PTR + 2)[1] == "rows"                       # off 16 bytes

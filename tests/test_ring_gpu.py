@@ -65,3 +65,35 @@ def test_error_against_64_bits(ctx, T, K, F, chains):
         acc = acc[::2] + acc[1::2]
     err = lambda a: np.linalg.norm(a - want) / np.linalg.norm(want)
     assert err(to_host(out)[:n].astype(np.float64)) <= 1.05 * err(acc[0].astype(np.float64))
+
+
+def _kernel(T, K, F, folded=0):
+    from juliavision_amd import _lib as L
+    return L.GEMM_KERNELS[L.load().mi_gemm_f16_kernel(T, K, F, 1, 0, folded, None)]
+
+
+RUNS = [(500, K, 520, "ring") for K in (136, 192, 256, 320, 384, 448, 512, 520, 576, 640, 1096)] + \
+       [(T, K, F, "ring_shallow") for T, K, F in ((1097, 1600, 1672), (1753, 1600, 1040), (3956, 1920, 392))]
+
+
+@pytest.mark.parametrize("layout", ["kf", "fk"])
+@pytest.mark.parametrize("T,K,F,kernel", RUNS)
+def test_the_kernel_that_is_meant(ctx, T, K, F, kernel, layout):
+    """Three tiles of K (the fewest it is planned for) to eighteen, and the half ring with odd and even counts, on the kernel named."""
+    import torch
+    import juliavision_amd as jv
+    assert _kernel(T, K, F) == kernel
+    X, W = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K, F), 2)
+    b, R = oracle.randn_f16((F,), 3, 0, 0.02), oracle.randn_f16((T, F), 4)
+    w = to_dev(W) if layout == "kf" else to_dev(np.ascontiguousarray(W.T)).t()
+    for res, dt in ((R, torch.float16), (None, torch.float32)):
+        out = poison(torch.empty((T, F), dtype=dt, device="cuda"))
+        ctx.ws.reset()
+        jv.matmul_(ctx, out, w, to_dev(X), to_dev(b), residual=None if res is None else to_dev(res))
+        assert_parity(to_host(out), oracle.gemm_f16(X, W, b, residual=res), what=f"T{T} K{K} F{F} {layout}")
+
+
+@pytest.mark.parametrize("T,K,F,kernel", [(500, K, 520, "ring") for K in (192, 320, 512, 576, 1280)] + [r for r in RUNS if r[3] == "ring_shallow"])
+def test_folded_norm_on_the_kernel_that_is_meant(ctx, T, K, F, kernel):
+    assert _kernel(T, K, F, 1) == kernel
+    test_folded_norm(ctx, T, F, K)

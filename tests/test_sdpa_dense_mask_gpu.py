@@ -53,6 +53,32 @@ def test_dense_masks(ctx, B, H, Lq, Lk, E, f32, kind):
     assert err <= (4e-7 if exact else 6e-4), (err, exact)
 
 
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("E,half", [(16, False), (32, False), (64, False), (72, True), (128, False)])
+@pytest.mark.parametrize("Lq,apart", [(63, False), (130, True)])
+def test_rows_without_a_key(ctx, Lq, apart, E, half, f32):
+    """Rows of -inf give zeros, beside rows of the same 32-query tile that have keys.  fp16 results bring head size 72 here too."""
+    import torch
+    import juliavision_amd as jv
+    B, H, Lk = 2, 3, 189
+    q, k, v = (to_dev(oracle.randn_f16((B, H, L, E), s)) for s, L in ((1, Lq), (2, Lk), (3, Lk)))
+    mask = to_dev(oracle.randn_f16((B, H, Lq, Lk), 7)).to(torch.float32 if f32 else torch.float16)
+    mask[:, :, 1::3] = float("-inf")
+    mask[0, 1] = float("-inf")                            # whole tiles of them
+    mask[:, :, ::3, 40:] = float("-inf")                  # and rows whose keys are the first wave's
+    if apart:
+        mask = mask.transpose(2, 3).contiguous().transpose(2, 3)
+    out = torch.full((B, H, Lq, E), float("nan"), dtype=torch.float16 if half else torch.float32, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, mask, out=out)
+    s = torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3)) / np.sqrt(E) + mask.double().cpu()
+    want = torch.matmul(torch.softmax(s, -1), v.double().cpu()).nan_to_num(0.0)
+    got, dead = out.double().cpu(), torch.isneginf(mask.cpu()).all(-1)
+    assert dead.any() and bool((got[dead] == 0).all())
+    # fp32 sums and products of an fp16 pair each: as test_dense_masks
+    assert float((got - want).norm() / want.norm()) <= (2.0 ** -11 if half else 4e-7)
+
+
 @pytest.mark.parametrize("fill", [-1e4, -1e7, -1e9, -1e30, "min"])
 @pytest.mark.parametrize("apart", [False, True])
 @pytest.mark.parametrize("E,half", [(16, False), (32, False), (64, False), (72, True), (128, False)])
