@@ -21,7 +21,7 @@ namespace {
 // four rows of a transposing read do.  Rows of nine chunks (72) need none for K.
 //
 // Products, register layouts and the lazily moved reference point M are flash_fwd_kernel's: S^T = K Q^T, O^T = V^T P^T, -M in
-// the first product's accumulators. 
+// the first product's accumulators.
 //
 // KEYS, DENSE: what a mask is.  KEYS: fp16 and of the key alone, copied to LDS once; it joins in one more k-step as (mask, mask) x
 // (log2(e) split into two positive fp16 parts), so that -inf stays -inf.  DENSE (with F32): anything else -- any strides, addresses
@@ -266,7 +266,9 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
         };
         // DENSE: score and mask are rounded into one number, once, and M is the largest such number itself.  However large a mask
         // (1e9 swallows its score, finfo.min times log2(e) would be infinite), no score of M's tile is above M, and a row of
-        // equal numbers is a row of equal weights.
+        // equal numbers is a row of equal weights.  (Error with fp32 results against the row kernel's, over 80 calls of 16 to 128 wide
+        // heads, 60 to 1500 keys and scores of standard deviation 1 and 3: 3.5 % less on average, at 64 2 % more.  One log2(e) inside the
+        // fma instead of behind the difference, where M is small enough for it, took off 0.3 % more and cost 3 % of the time.)
         if constexpr (MASK == DENSE) {
 #pragma unroll
             for (int r = 0; r < 16; r++) sc[r] = fmaf(sc[r], p.scale, ms[r]);
