@@ -471,7 +471,7 @@ def decoder_layer_case(bsz, layout="kf", steps=200):
     replay = timed(graph.replay)
     weights = 2.0 * (3 * d * d + 3 * d * d + 2 * d * ffn)
     kv = 2.0 * 2 * bsz * H * E * (448 + 1500)
-    return {"eager_us": round(eager * 1e6, 1), "graph_us": round(replay * 1e6, 1), "launches": (14 if layout == "kf" else 8) + (3 if bsz > 4 else 0),
+    return {"eager_us": round(eager * 1e6, 1), "graph_us": round(replay * 1e6, 1), "launches": (14 if layout == "kf" else 8) + (3 if bsz > (8 if layout == "fk" else 4) else 0),
             "GB/s_graph": round((weights + kv) / replay / 1e9, 1), "frac_hbm_peak_graph": round((weights + kv) / replay / 1e9 / PEAK_HBM_GBS, 4)}
 
 
