@@ -15,9 +15,9 @@ namespace {
 // compiler's.  In launches of one tile a CU the ends cost as much as the loop, and that is where the arrangement comes from
 // (clocks at 1370 x 1536 -> 384, 132 workgroups; before, with waves that split K's steps and a ring filled before the first
 // product): first request 2040 -> 840 (stage_args, tile_of), products begin 4620 -> 2600 (AHEAD tiles asked for, not the whole
-// ring), sum of the waves' partial tiles 2020 -> none, store 2030 -> 1270 (its residual comes with the first tiles).  9.3 -> 8.3 us
-// a launch; 1370 x 384 -> 384, where four waves that split K lost to the register-staged kernel, 5.1 -> 4.9 (4.65 before its
-// residual and statistics are counted), 76 x 1024 -> 3072 7.8 -> 6.3, 2056 x 1536 -> 384 11.1 -> 8.6.  Waves that split K read
+// ring), sum of the waves' partial tiles 2020 -> none, store 2030 -> 1270 (its residual comes with the first tiles).  8.3 -> 7.3 us
+// a launch; 1370 x 384 -> 384, where four waves that split K lost to the register-staged kernel, 4.8 -> 4.6, 76 x 1024 -> 3072
+// 6.7 -> 5.9, 2056 x 1536 -> 384 8.7 -> 7.8.  Waves that split K read
 // 16 KB of fragments a tile instead of 32 and gain from some 45 tiles of K on in the smallest grids (32 x 3456 -> 448 10.3 against
 // 11.2 us); over 150 shapes they are 6 % behind.
 //
