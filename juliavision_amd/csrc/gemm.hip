@@ -1294,7 +1294,8 @@ int launch_w4_peer(GemmArgs a, bool b_kn, int split, void *ws, hipStream_t st) {
 constexpr int RING_TILE = 5, DEEP_TILE = 6, DEEP_SERIAL_TILE = 7;      // indices into TILE_MODELS: gemm_ring_kernel, gemm_deep_kernel with four matrix waves and one
 // tile: index into TILE_MODELS.  The four-wave kernel takes ordinary operands in whole 64-deep tiles only; a gathered operand
 // (implicit-GEMM convolution) or a K % 64 planned onto one of its tiles runs the pipelined kernel's same tile instead: same K order per
-// output, same bits (the 32 x 32 tiles are not planned for a gathered operand: their order of a long K is their own).
+// output, same bits.  On the ring a gathered operand runs the pipelined 64 x 64 tile, whose order of a long K is not the ring's; the 32 x 32
+// tiles are not planned for one.
 int launch_tile(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
     const bool plain = !a.ag.x && a.K % 64 == 0;
     switch (tile) {
