@@ -15,20 +15,20 @@ namespace {
 // Layer-norm statistics of up to MT rows of A, one wave per row, in the summation order of
 // layernorm_vec_kernel (a lane takes the 16-byte chunks lane, lane + 64, ...; butterfly over the wave):
 // the fused result is bit-identical to running that kernel first.  stats[m] = (mean, rstd).
-template <int MT, int NCH = 8, int NWAVES = 4>              // rows up to NCH * 512 halves stay in registers between the passes
-__device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2], int tid) {
-    const int lane = tid & 63, wave = tid >> 6;
-    for (int m = wave; m < MT && m < p.M; m += NWAVES) {
+// In two halves, so that a caller can ask for more in between.  Rows up to NCH * 512 halves stay in registers between the passes; a
+// longer one is read twice.
+template <int NCH>
+struct LnRow {
+    u32x4 raw[NCH];
+    __device__ __forceinline__ void request(const GemmArgs &p, int m, int lane) {
+        if (p.K > NCH * 512) return;                        // uniform
         const half_t *row = p.A + (long)m * p.ldA;
-        float s = 0.0f, s2 = 0.0f;
-        if (p.K <= NCH * 512) {
-            u32x4 raw[NCH];
 #pragma unroll
-            for (int i = 0; i < NCH; i++) {
-                const int e0 = (lane + 64 * i) * 8;
-                const u32x4 z = {0u, 0u, 0u, 0u};
-                raw[i] = e0 < p.K ? ldg16(row + e0) : z;
-            }
+        for (int i = 0; i < NCH; i++) raw[i] = ldg16(row + min((lane + 64 * i) * 8, p.K - 8));
+    }
+    __device__ __forceinline__ void finish(const GemmArgs &p, float (*stats)[2], int m, int lane) {
+        float s = 0.0f, s2 = 0.0f, mu;
+        if (p.K <= NCH * 512) {
 #pragma unroll
             for (int i = 0; i < NCH; i++) {
                 if ((lane + 64 * i) * 8 < p.K) {
@@ -38,7 +38,7 @@ __device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2
                 }
             }
             s = wave_sum(s);
-            const float mu = s / (float)p.K;
+            mu = s / (float)p.K;
 #pragma unroll
             for (int i = 0; i < NCH; i++) {
                 if ((lane + 64 * i) * 8 < p.K) {
@@ -47,24 +47,32 @@ __device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2
                     for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
                 }
             }
-            s2 = wave_sum(s2);
-            if (lane == 0) { stats[m][0] = mu; stats[m][1] = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps); }
         } else {
+            const half_t *row = p.A + (long)m * p.ldA;
             for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
                 const half8v t = as_half8(ldg16(row + e0));
 #pragma unroll
                 for (int j = 0; j < 8; j++) s += (float)t[j];
             }
             s = wave_sum(s);
-            const float mu = s / (float)p.K;
+            mu = s / (float)p.K;
             for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
                 const half8v t = as_half8(ldg16(row + e0));
 #pragma unroll
                 for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
             }
-            s2 = wave_sum(s2);
-            if (lane == 0) { stats[m][0] = mu; stats[m][1] = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps); }
         }
+        s2 = wave_sum(s2);
+        if (lane == 0) { stats[m][0] = mu; stats[m][1] = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps); }
+    }
+};
+template <int MT, int NCH = 8, int NWAVES = 4>
+__device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2], int tid) {
+    const int lane = tid & 63, wave = tid >> 6;
+    for (int m = wave; m < MT && m < p.M; m += NWAVES) {
+        LnRow<NCH> row;
+        row.request(p, m, lane);
+        row.finish(p, stats, m, lane);
     }
 }
 
@@ -195,375 +203,362 @@ __global__ void skinny_epilogue_kernel(GemmArgs p, const float *part, int nsplit
     }
 }
 
-// [F][K] weights (K-contiguous): one wave per output column, lanes stride K in 16-byte chunks,
-// wave reduction, and the epilogue in the same launch: no workspace, no second kernel.  The
-// activations are staged in LDS once per workgroup (dynamic: MT rows of K halves).
+// [F][K] weights (K-contiguous): one wave per R output columns, lanes stride K in 16-byte chunks,
+// wave reduction, and the epilogue in the same launch: no workspace, no second kernel.
 //
-// A decode-sized call moves a few MB, so its duration is a chain of trips to memory, not bandwidth.  Everything whose
-// address does not depend on loaded data is therefore requested at the top, before anything is waited for: the wave's
-// weight row (FK_PF chunks of 16 bytes per lane: K <= 6144 whole), its bias and residual elements, the thread's
-// share of the activations and of gamma / beta.  The statistics of the layer-norm prologue, the staging and the dot
-// products then run on data that arrives together: one trip instead of three or four in a row.
-// FK_PF = 3 (K <= 1536) or 12: the registers of the up-front requests decide how many waves a SIMD holds, and a
-// wide output (1280 -> 5120 is five waves per SIMD, a vocabulary projection many more) needs them all resident.
-template <int MT, int FK_PF>
+// A decode-sized call moves a few MB, so its duration is a chain of trips to memory, not bandwidth: everything whose
+// address does not depend on loaded data is requested at the top, before anything is waited for.  For that no load may stand
+// behind a condition -- where the registers of the two sides meet the compiler waits for the load, and with it, as loads come back
+// in the order they were asked for, for every load before it (the bias, behind `if (lane < M)`, cost a trip of its own, the
+// residual another, the activations a third: 1280 -> 1280 behind a norm 3.57 us, hot in a replayed graph).  So every address is made
+// valid instead -- chunks past K re-read the row's last one, columns past N the last row, an operand that is not there the
+// weights -- and what was read in vain is left out where it would be used.
+// Bias and residual of the output of lane r * MT + m: row m of a wave's column r.
+template <int MT, int R>
+struct FkOut {
+    half_t bias, residual;
+    __device__ __forceinline__ void request(const GemmArgs &p, int n0, int lane) {
+        const int m = min(lane % MT, p.M - 1), n = min(n0 + min(lane / MT, R - 1), p.N - 1);
+        const half_t *b = p.bias_mode == MI_BIAS_NONE ? p.B : p.bias + (p.bias_mode == MI_BIAS_COL ? n : m);
+        const half_t *r = p.residual && !p.out_f32 ? p.residual + (long)m * p.ldY + n : p.B;
+        bias = *b;
+        residual = *r;
+    }
+    __device__ __forceinline__ void store(const GemmArgs &p, float sum, int n0, int lane) const {
+        const int m = lane % MT, n = n0 + lane / MT;
+        if (lane >= MT * R || m >= p.M || n >= p.N) return;
+        const float v = sum + (p.bias_mode == MI_BIAS_NONE ? 0.0f : (float)bias);
+        const long off = (long)m * p.ldY + n;
+        if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(v, p.epi);
+        else {
+            half_t o = (half_t)apply_epi((float)(half_t)v, p.epi);
+            if (p.residual) o = (half_t)((float)o + (float)residual);
+            reinterpret_cast<half_t *>(p.Y)[off] = o;
+        }
+    }
+};
+template <int R, int PF>
+__device__ __forceinline__ void fk_request(const GemmArgs &p, u32x4 (&w)[R][PF], int n0, int lane) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const half_t *bp = p.B + (long)min(n0 + r, p.N - 1) * p.ldB;
+#pragma unroll
+        for (int i = 0; i < PF; i++) w[r][i] = ldg16(bp + min(lane * 8 + 512 * i, p.K - 8));
+    }
+}
+__device__ __forceinline__ float fk_dot(u32x4 w, u32x4 x, float acc) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t wq = w[q], xq = x[q];              // bit_cast wants an addressable scalar, not a vector element
+        acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, wq), __builtin_bit_cast(half2v, xq), acc, false);
+    }
+    return acc;
+}
+
+// The activations staged in LDS once per workgroup (dynamic: MT rows of K halves), behind the layer norm of their rows (LN).
+// PF: 512-column chunks of a row asked for at the top, all of K up to 6144.  R columns a wave: the norm, the staging and their two
+// barriers are paid once a workgroup, so behind a norm a wave takes as many as leave one workgroup a CU (us, weights from memory, with 1
+// and with R columns: 1280 -> 1280 3.9 and 3.5, -> 3840 5.2 and 4.2, -> 5120 5.6 and 4.7); without one the launch gains nothing by it.
+template <int MT, int PF, int R, bool LN>
 __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
-    // activation chunks per thread requested up front: the whole MT x K panel up to four per thread
-    constexpr int FK_XPF = (MT * FK_PF * 64 + 255) / 256 < 4 ? (MT * FK_PF * 64 + 255) / 256 : 4;
+    // activation chunks per thread requested up front: the whole MT x K panel, up to twelve per thread (four behind a norm: gamma and beta come with them)
+    constexpr int XPF_MAX = LN ? 4 : 12, XPF = (MT * PF * 64 + 255) / 256 < XPF_MAX ? (MT * PF * 64 + 255) / 256 : XPF_MAX;
     extern __shared__ __align__(16) char smem[];
     stage_skinny(p);
     half_t *xs = reinterpret_cast<half_t *>(smem);       // [MT][K]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ float lnst[MT][2];
     const int kch = p.K >> 3;
     const u32x4 z = {0u, 0u, 0u, 0u};
-    const int n = blockIdx.x * 4 + wave;
-    const bool live = n < p.N;                            // uniform over the wave
-    const half_t *bp = p.B + (long)(live ? n : 0) * p.ldB;
-    u32x4 w[FK_PF];
+    // what the norm and the staging wait for goes first
+    LnRow<PF <= 10 ? PF : 8> lnrow;
+    if constexpr (LN) lnrow.request(p, min(wave, p.M - 1), lane);      // (MT is at most the workgroup's four waves)
+    u32x4 xr[XPF], gr[LN ? XPF : 1], br[LN ? XPF : 1];
 #pragma unroll
-    for (int i = 0; i < FK_PF; i++) w[i] = live && lane * 8 + 512 * i < p.K ? ldg16(bp + lane * 8 + 512 * i) : z;
-    float bv = 0.0f, rv = 0.0f;
-    if (live && lane < p.M) {
-        if (p.bias_mode == MI_BIAS_COL) bv = (float)p.bias[n];
-        else if (p.bias_mode == MI_BIAS_ROW) bv = (float)p.bias[lane];
-        if (p.residual && !p.out_f32) rv = (float)p.residual[(long)lane * p.ldY + n];
-    }
-    u32x4 xr[FK_XPF], gr[FK_XPF], br[FK_XPF];
-#pragma unroll
-    for (int i = 0; i < FK_XPF; i++) {
+    for (int i = 0; i < XPF; i++) {
         unsigned ch;
         const int c = tid + 256 * i, m = (int)divide(c, kch, p.div_k8, ch);
-        xr[i] = gr[i] = br[i] = z;
-        if (c < MT * kch && m < p.M) {
-            xr[i] = ldg16(p.A + (long)m * p.ldA + ch * 8);
-            if (p.ln_on && p.ln_gamma) gr[i] = ldg16(p.ln_gamma + ch * 8);
-            if (p.ln_on && p.ln_beta) br[i] = ldg16(p.ln_beta + ch * 8);
+        xr[i] = ldg16(p.A + (long)min(m, p.M - 1) * p.ldA + ch * 8);
+        if constexpr (LN) {
+            gr[i] = ldg16((p.ln_gamma ? p.ln_gamma : p.A) + ch * 8);
+            br[i] = ldg16((p.ln_beta ? p.ln_beta : p.A) + ch * 8);
         }
     }
-    if (p.ln_on) {                                      // uniform
-        ln_row_stats<MT, (FK_PF < 8 ? FK_PF : 8)>(p, lnst, tid);
+    const int n = (blockIdx.x * 4 + wave) * R;
+    u32x4 w[R][PF];
+    FkOut<MT, R> out;
+    fk_request(p, w, n, lane);
+    out.request(p, n, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (LN) {
+        if (wave < p.M) lnrow.finish(p, lnst, wave, lane);
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < FK_XPF; i++) {
+    for (int i = 0; i < XPF; i++) {
         unsigned ch;
         const int c = tid + 256 * i, m = (int)divide(c, kch, p.div_k8, ch);
         if (c < MT * kch) {
             u32x4 v = xr[i];
-            if (p.ln_on && m < p.M) {
+            if constexpr (LN) {
+                const int ms = min(m, p.M - 1);
                 const half8v x = as_half8(v), gv = as_half8(gr[i]), bb = as_half8(br[i]);
                 half8v o;
 #pragma unroll
                 for (int j = 0; j < 8; j++)
-                    o[j] = ln_norm1((float)x[j], lnst[m][0], lnst[m][1], p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bb[j]);
+                    o[j] = ln_norm1((float)x[j], lnst[ms][0], lnst[ms][1], p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bb[j]);
                 v = __builtin_bit_cast(u32x4, o);
             }
-            *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;
+            *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;      // (rows past M repeat the last one; their sums go nowhere)
         }
     }
-    for (int c = tid + 256 * FK_XPF; c < MT * kch; c += 256) {
+    for (int c = tid + 256 * XPF; c < MT * kch; c += 256) {
         unsigned ch;
-        const int m = (int)divide(c, kch, p.div_k8, ch);
-        u32x4 v = z;
-        if (m < p.M) {
-            v = ldg16(p.A + (long)m * p.ldA + ch * 8);
-            if (p.ln_on) v = ln_apply8(p, v, lnst[m][0], lnst[m][1], ch * 8);
-        }
-        *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;
+        const int m = min((int)divide(c, kch, p.div_k8, ch), p.M - 1);
+        u32x4 v = ldg16(p.A + (long)m * p.ldA + ch * 8);
+        if constexpr (LN) v = ln_apply8(p, v, lnst[m][0], lnst[m][1], ch * 8);
+        *reinterpret_cast<u32x4 *>(xs + (long)(c / kch) * p.K + ch * 8) = v;
     }
     __syncthreads();
-    if (!live) return;
-    // A wave walks columns n, n + 4 gridDim.x, ...: one for the widths of a decoder layer (the launcher gives every
-    // column its wave), several for a vocabulary-sized output, where the staged activations and their norm are then
-    // paid once per workgroup instead of once per four columns and the next column's row is requested under the
-    // current one's dot products.
-    const int stride = (int)gridDim.x * 4;
-    for (int nc = n; nc < p.N; nc += stride) {
-        const int nn = nc + stride;
-        const bool more = nn < p.N;                       // uniform over the wave
-        const half_t *bn = p.B + (long)(more ? nn : nc) * p.ldB;
-        u32x4 wn[FK_PF];
-        float bvn = 0.0f, rvn = 0.0f;
-        if (more) {
+    // A wave walks its columns n .. n + R - 1, then those 4 R gridDim.x further on: once for the widths of a decoder layer
+    // (the launcher gives every group its wave), several times for a vocabulary-sized output, where the staged activations
+    // and their norm are then paid once per workgroup and the next rows are requested under the current ones' dot products.
+    if (n >= p.N) return;                                 // uniform over the wave
+    const int stride = (int)gridDim.x * 4 * R;
+    for (int nc = n;; nc += stride) {
+        u32x4 wn[R][PF];
+        FkOut<MT, R> outn;
+        const bool more = p.N - nc > stride;              // (past the end: the last row once more)
+        const int nn = more ? nc + stride : p.N - 1;
+        fk_request(p, wn, nn, lane);
+        outn.request(p, nn, lane);
+        float acc[R][MT];
 #pragma unroll
-            for (int i = 0; i < FK_PF; i++) wn[i] = lane * 8 + 512 * i < p.K ? ldg16(bn + lane * 8 + 512 * i) : z;
-            if (lane < p.M) {
-                if (p.bias_mode == MI_BIAS_COL) bvn = (float)p.bias[nn];
-                else if (p.bias_mode == MI_BIAS_ROW) bvn = (float)p.bias[lane];
-                if (p.residual && !p.out_f32) rvn = (float)p.residual[(long)lane * p.ldY + nn];
-            }
-        }
-        float acc[MT];
+        for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int m = 0; m < MT; m++) acc[m] = 0.0f;
-        auto dot = [&](const u32x4 &wv, int k) {
+            for (int m = 0; m < MT; m++) acc[r][m] = 0.0f;
 #pragma unroll
-            for (int m = 0; m < MT; m++) {
-                const u32x4 x = *reinterpret_cast<const u32x4 *>(xs + (long)m * p.K + k);
+        for (int i = 0; i < PF; i++)
+            if (lane * 8 + 512 * i < p.K) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const uint32_t wq = wv[q], xq = x[q];     // bit_cast wants an addressable scalar, not a vector element
-                    acc[m] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, wq), __builtin_bit_cast(half2v, xq), acc[m], false);
+                for (int m = 0; m < MT; m++) {
+                    const u32x4 x = *reinterpret_cast<const u32x4 *>(xs + (long)m * p.K + lane * 8 + 512 * i);
+#pragma unroll
+                    for (int r = 0; r < R; r++) acc[r][m] = fk_dot(w[r][i], x, acc[r][m]);
                 }
             }
-        };
+        if (p.K > 512 * PF)                               // uniform
 #pragma unroll
-        for (int i = 0; i < FK_PF; i++)
-            if (lane * 8 + 512 * i < p.K) dot(w[i], lane * 8 + 512 * i);
-        const half_t *bc = p.B + (long)nc * p.ldB;
-        for (int kb = lane * 8 + 512 * FK_PF; kb < p.K; kb += 4 * 512) {
-            u32x4 t[4];
+            for (int r = 0; r < R; r++) {
+                const half_t *bc = p.B + (long)min(nc + r, p.N - 1) * p.ldB;
+                for (int kb = lane * 8 + 512 * PF; kb < p.K; kb += 4 * 512) {
+                    u32x4 t[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) t[i] = kb + 512 * i < p.K ? ldg16(bc + kb + 512 * i) : z;
+                    for (int i = 0; i < 4; i++) t[i] = ldg16(bc + min(kb + 512 * i, p.K - 8));
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (kb + 512 * i < p.K) dot(t[i], kb + 512 * i);
-        }
-        float mine = 0.0f;                                    // lane m keeps row m's sum
+                    for (int i = 0; i < 4; i++)
+                        if (kb + 512 * i < p.K)
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-            float sres = acc[m];
-            sres = wave_sum(sres);
-            if (lane == m) mine = sres;
-        }
-        if (lane < p.M) {
-            const float v = mine + bv;
-            const long off = (long)lane * p.ldY + nc;
-            if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(v, p.epi);
-            else {
-                half_t o = (half_t)apply_epi((float)(half_t)v, p.epi);
-                if (p.residual) o = (half_t)((float)o + rv);
-                reinterpret_cast<half_t *>(p.Y)[off] = o;
+                            for (int m = 0; m < MT; m++) acc[r][m] = fk_dot(t[i], *reinterpret_cast<const u32x4 *>(xs + (long)m * p.K + kb + 512 * i), acc[r][m]);
+                }
             }
-        }
-        if (more) {
+        float mine = 0.0f;                                // lane r * MT + m keeps its sum
 #pragma unroll
-            for (int i = 0; i < FK_PF; i++) w[i] = wn[i];
-            bv = bvn; rv = rvn;
-        }
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const float sres = wave_sum(acc[r][m]);
+                if (lane == r * MT + m) mine = sres;
+            }
+        out.store(p, mine, nc, lane);
+        if (!more) break;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < PF; i++) w[r][i] = wn[r][i];
+        out = outn;
     }
 }
 
 // Five to eight rows: on the matrix cores.  A workgroup owns sixteen output columns (`cols`; eight where that gives more CUs work), its
 // eight waves an eighth of K each: the weight rows by 32 k are one operand of v_mfma_f32_16x16x32_f16, the activation rows the
-// other (zeros past either), both straight from memory in the layout the instruction wants -- a lane's sixteen bytes -- and all of a wave's share asked for at its first
-// lines (PF steps at a time).  The eight partial sums meet in LDS, in pairs.  With a norm in front a wave finds one row's statistics,
+// other, both straight from memory in the layout the instruction wants -- a lane's sixteen bytes -- and all of a wave's share asked for at its first
+// lines (PF steps; a longer share in TURNS of them).  The eight partial sums meet in LDS, in pairs.  With a norm in front a wave finds one row's statistics,
 // in layernorm_vec_kernel's order, and the fragments are normalised and rounded on their way into the product.
-// What bounds it is the trip to memory.  The kernel above staged M x K activations in every workgroup of four columns and read them back
-// once a column: 80 KB of LDS traffic a wave at 8 x 5120.
-template <int PF, bool LN>
+// What bounds it is the trip to memory, as above; no load stands behind a condition here either (rows past either operand's
+// re-read its last one: they reach sums that nobody stores).
+// WALK: past one workgroup a CU it goes on to the columns of gridDim.x workgroups further, whose weights it asks for under the current
+// ones' products; the activations stay in registers, normalised once.
+template <int PF, int TURNS, bool LN, bool WALK>
 __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
-    constexpr int NW = 8;
-    __shared__ float4v red[NW][64];
+    static_assert(TURNS == 1 || !WALK, "activations in registers");
+    constexpr int NW = 8, NA = 5;
+    __shared__ float4v red[WALK ? 2 : 1][NW][64];
     __shared__ float lnst[8][2];
     stage_skinny(p);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row = lane & 15, kq = lane >> 4, n0 = blockIdx.x * cols;
+    const int row = lane & 15, kq = lane >> 4, nfirst = blockIdx.x * cols, stride = (int)gridDim.x * cols;
     const int steps = (p.K + 31) >> 5, per = (steps + NW - 1) / NW, s0 = wave * per, s1 = min(steps, s0 + per);
-    const half_t *const wrow = p.B + (long)min(n0 + row, p.N - 1) * p.ldB, *const xrow = p.A + (long)min(row, p.M - 1) * p.ldA;
-    u32x4 w[PF], x[PF], g[LN ? PF : 1], b[LN ? PF : 1];
-    auto fetch = [&](int base) {
+    const int mrow = min(row, p.M - 1), wrow = min(row, cols - 1);
+    const half_t *const xrow = p.A + (long)mrow * p.ldA;
+    struct Cols { u32x4 w[PF]; half_t bias, residual; };
+    const int om = (tid >> 4) & 7, oc = tid & 15, omc = min(om, p.M - 1);      // outputs: one of each of the first 128 threads
+    auto at = [&](int base, int i) { return min((base + i) * 32 + kq * 8, p.K - 8); };
+    auto fetch_w = [&](Cols &c, int n0, int base) {
+        const half_t *from = p.B + (long)min(n0 + wrow, p.N - 1) * p.ldB;
+#pragma unroll
+        for (int i = 0; i < PF; i++) c.w[i] = ldg16(from + at(base, i));
+    };
+    auto fetch_out = [&](Cols &c, int n0) {
+        const int n = min(n0 + min(oc, cols - 1), p.N - 1);
+        const half_t *b = p.bias_mode == MI_BIAS_NONE ? p.B : p.bias + (p.bias_mode == MI_BIAS_COL ? n : omc);
+        const half_t *r = p.residual && !p.out_f32 ? p.residual + (long)omc * p.ldY + n : p.B;
+        c.bias = *b;
+        c.residual = *r;
+    };
+    u32x4 x[PF], gm[LN ? PF : 1], be[LN ? PF : 1];
+    auto fetch_x = [&](int base) {
 #pragma unroll
         for (int i = 0; i < PF; i++) {
-            const u32x4 z = {0u, 0u, 0u, 0u};
-            const int k = (base + i) * 32 + kq * 8;
-            const bool on = base + i < s1 && k < p.K;
-            w[i] = on && row < cols ? ldg16(wrow + k) : z;
-            x[i] = on && row < p.M ? ldg16(xrow + k) : z;
+            x[i] = ldg16(xrow + at(base, i));
             if constexpr (LN) {
-                // (columns that are not there have gamma zero, whatever the row's mean: as a half it may be an infinity)
-                const u32x4 ones = {0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u};
-                g[i] = !on ? z : p.ln_gamma ? ldg16(p.ln_gamma + k) : ones;
-                b[i] = on && p.ln_beta ? ldg16(p.ln_beta + k) : z;
+                gm[i] = ldg16((p.ln_gamma ? p.ln_gamma : p.A) + at(base, i));
+                be[i] = ldg16((p.ln_beta ? p.ln_beta : p.A) + at(base, i));
             }
         }
     };
-    fetch(s0);
-    // what the store needs, by the wave that stores: lane (row, kq) holds columns n0 + 4 kq .. +3 of row `row`
-    const int n = n0 + 4 * kq;
-    const bool stores = wave == 0 && row < p.M && 4 * kq < cols;
-    float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, rv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (stores) {
+    float mu = 0.0f, rs = 0.0f;
+    auto normalise = [&]() {
+        if constexpr (LN) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            if (n + e < p.N) {
-                if (p.bias_mode == MI_BIAS_COL) bv[e] = (float)p.bias[n + e];
-                else if (p.bias_mode == MI_BIAS_ROW) bv[e] = (float)p.bias[row];
-                if (p.residual && !p.out_f32) rv[e] = (float)p.residual[(long)row * p.ldY + n + e];
+            for (int i = 0; i < PF; i++) {
+                const half8v xv = as_half8(x[i]), gv = as_half8(gm[i]), bv = as_half8(be[i]);
+                half8v o;
+#pragma unroll
+                for (int j = 0; j < 8; j++) o[j] = ln_norm1((float)xv[j], mu, rs, p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bv[j]);
+                x[i] = __builtin_bit_cast(u32x4, o);
             }
         }
-    }
-    float mu = 0.0f, rs = 0.0f;
+    };
+    LnRow<(PF * TURNS + 1) / 2 < 8 ? (PF * TURNS + 1) / 2 : 8> lnrow;      // 512 columns are two steps of eight waves
+    if constexpr (LN) lnrow.request(p, min(wave, p.M - 1), lane);
+    fetch_x(s0);
+    Cols cur;
+    fetch_w(cur, nfirst, s0);
+    fetch_out(cur, nfirst);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (LN) {
-        ln_row_stats<8, 8, NW>(p, lnst, tid);
+        if (wave < p.M) lnrow.finish(p, lnst, wave, lane);
         __syncthreads();
-        mu = lnst[min(row, p.M - 1)][0];
-        rs = lnst[min(row, p.M - 1)][1];
+        mu = lnst[mrow][0];
+        rs = lnst[mrow][1];
+        normalise();
     }
-    // five chains, step i of the share in chain i % 5 whatever PF is: short ones keep the error at that of the dot products below five rows
-    constexpr int NA = 5;
-    static_assert(PF % NA == 0, "one order of the sum, with a norm in front and without");
     float4v acc[NA];
-#pragma unroll
-    for (int i = 0; i < NA; i++) acc[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int base = s0;;) {
+    // five chains, step i of the share in chain i % 5 whatever PF is: short ones keep the error at that of the dot products below five rows
+    auto products = [&](const Cols &c, auto TURN) {
+        constexpr int turn = decltype(TURN)::value;
+        const int base = s0 + turn * PF;
 #pragma unroll
         for (int i = 0; i < PF; i++) {
-            half8v xv = as_half8(x[i]);
-            if constexpr (LN) {
-                const half8v gv = as_half8(g[i]), be = as_half8(b[i]);
-#pragma unroll
-                for (int j = 0; j < 8; j++) xv[j] = ln_norm1((float)xv[j], mu, rs, true, (float)gv[j], p.ln_beta != nullptr, (float)be[j]);
+            if (base + i < s1) {                          // uniform
+                u32x4 xv = x[i], wv = c.w[i];
+                const bool past = (base + i) * 32 + kq * 8 >= p.K;      // in the step that K ends in: neither operand counts there
+                const u32x4 z = {0u, 0u, 0u, 0u};
+                if ((base + i) * 32 + 32 > p.K) { xv = past ? z : xv; wv = past ? z : wv; }
+                float4v &a = acc[(turn * PF + i) % NA];
+                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wv), as_half8(xv), a, 0, 0, 0);
             }
-            acc[i % NA] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(w[i]), xv, acc[i % NA], 0, 0, 0);      // (steps past the share multiply zeros)
         }
-        if ((base += PF) >= s1) break;
-        fetch(base);
-    }
+    };
+    int set = 0;
+    for (int nc = nfirst;; nc += stride) {
+        Cols nxt;
+        const bool more = WALK && p.N - nc > stride;
+        if constexpr (WALK) {
+            const int nn = more ? nc + stride : p.N - 1;  // (past the end: the last row once more)
+            fetch_w(nxt, nn, s0);
+            fetch_out(nxt, nn);
+        }
 #pragma unroll
-    for (int d = 1; d < NA; d *= 2)
+        for (int i = 0; i < NA; i++) acc[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        products(cur, std::integral_constant<int, 0>{});
+        auto turn = [&](auto TURN) {
+            if constexpr (decltype(TURN)::value < TURNS) {
+                fetch_x(s0 + decltype(TURN)::value * PF);
+                fetch_w(cur, nc, s0 + decltype(TURN)::value * PF);
+                normalise();
+                products(cur, TURN);
+            }
+        };
+        turn(std::integral_constant<int, 1>{});
+        turn(std::integral_constant<int, 2>{});
+        turn(std::integral_constant<int, 3>{});
+        static_assert(TURNS <= 4, "turns above");
 #pragma unroll
-        for (int i = 0; i + d < NA; i += 2 * d) acc[i] += acc[i + d];
-    red[wave][lane] = acc[0];
-    __syncthreads();
-    if (!stores) return;
-    float4v sum[NW];
+        for (int d = 1; d < NA; d *= 2)
 #pragma unroll
-    for (int q = 0; q < NW; q++) sum[q] = red[q][lane];
+            for (int i = 0; i + d < NA; i += 2 * d) acc[i] += acc[i + d];
+        red[set][wave][lane] = acc[0];
+        __syncthreads();
+        if (tid < 128 && om < p.M && oc < cols && nc + oc < p.N) {
+            const int n = nc + oc;
+            float sum[NW];
 #pragma unroll
-    for (int d = 1; d < NW; d *= 2)
+            for (int q = 0; q < NW; q++) sum[q] = reinterpret_cast<const float *>(&red[set][q][(oc >> 2) * 16 + om])[oc & 3];
 #pragma unroll
-        for (int q = 0; q < NW; q += 2 * d) sum[q] += sum[q + d];
-    const float4v v = sum[0];
+            for (int d = 1; d < NW; d *= 2)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        if (n + e < p.N) {
-            const float t = v[e] + bv[e];
-            const long off = (long)row * p.ldY + n + e;
+                for (int q = 0; q < NW; q += 2 * d) sum[q] += sum[q + d];
+            const float t = sum[0] + (p.bias_mode == MI_BIAS_NONE ? 0.0f : (float)cur.bias);
+            const long off = (long)om * p.ldY + n;
             if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(t, p.epi);
             else {
                 half_t o = (half_t)apply_epi((float)(half_t)t, p.epi);
-                if (p.residual) o = (half_t)((float)o + rv[e]);
+                if (p.residual) o = (half_t)((float)o + (float)cur.residual);
                 reinterpret_cast<half_t *>(p.Y)[off] = o;
             }
+        }
+        if constexpr (!WALK) break;
+        else {
+            if (!more) break;
+            cur = nxt;
+            set ^= 1;                                     // (a wave two turns ahead of a reader has passed that reader's barrier)
         }
     }
 }
 
-// The same product with the activations in registers instead of LDS, for the few rows of a decode step: a lane's
+// The same product with the activations in registers instead of LDS, for one or two rows of K <= 1536 without a norm: a lane's
 // weight chunks sit at k = 8 lane + 512 i, so it needs exactly those chunks of every activation row and asks for
-// them itself (the rows come from the L2: every wave of the launch reads the same few KB).  No staging, no barrier:
-// a wave is a chain of one trip to memory, the norm statistics (its own copy, same summation order as
-// ln_row_stats, so the same bits), the dot products, one wave reduction and a store.  R output columns per wave,
-// all their weight rows requested up front.  (MT + R + 2) * PF chunks of registers: built for one and two rows of
-// K <= 1536 (78 to 119 registers, four to six waves per SIMD); four rows, or K = 5120, would leave a SIMD one or
-// two waves and stay with the staged kernel.
-template <int MT, int PF, int R>
+// them itself (the rows come from the L2: every wave of the launch reads the same few KB).  No staging, no barrier: one trip to
+// memory, the dot products, one wave reduction and a store.
+template <int MT, int PF>
 __global__ __launch_bounds__(256) void skinny_fk_reg_kernel(GemmArgs p) {
     stage_skinny(p);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    const int n0 = (blockIdx.x * 4 + wave) * R;
-    if (n0 >= p.N) return;                                // uniform over the wave; no barrier below
-    u32x4 w[R][PF];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = blockIdx.x * 4 + wave;
+    u32x4 x[MT][PF], w[1][PF];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const half_t *bp = p.B + (long)min(n0 + r, p.N - 1) * p.ldB;
+    for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int i = 0; i < PF; i++) w[r][i] = lane * 8 + 512 * i < p.K ? ldg16(bp + lane * 8 + 512 * i) : z;
-    }
-    u32x4 x[MT][PF], gr[PF], br[PF];
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-        const int k = lane * 8 + 512 * i;
-        gr[i] = br[i] = z;
-#pragma unroll
-        for (int m = 0; m < MT; m++) x[m][i] = m < p.M && k < p.K ? ldg16(p.A + (long)m * p.ldA + k) : z;
-        if (p.ln_on && k < p.K) {
-            if (p.ln_gamma) gr[i] = ldg16(p.ln_gamma + k);
-            if (p.ln_beta) br[i] = ldg16(p.ln_beta + k);
-        }
-    }
-    float bv[R], rv[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        bv[r] = rv[r] = 0.0f;
-        if (lane < p.M && n0 + r < p.N) {
-            if (p.bias_mode == MI_BIAS_COL) bv[r] = (float)p.bias[n0 + r];
-            else if (p.bias_mode == MI_BIAS_ROW) bv[r] = (float)p.bias[lane];
-            if (p.residual && !p.out_f32) rv[r] = (float)p.residual[(long)lane * p.ldY + n0 + r];
-        }
-    }
-    if (p.ln_on) {                                        // uniform
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            float s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-            for (int i = 0; i < PF; i++) {
-                if (lane * 8 + 512 * i < p.K) {
-                    const half8v t = as_half8(x[m][i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) s1 += (float)t[j];
-                }
-            }
-            s1 = wave_sum(s1);
-            const float mu = s1 / (float)p.K;
-#pragma unroll
-            for (int i = 0; i < PF; i++) {
-                if (lane * 8 + 512 * i < p.K) {
-                    const half8v t = as_half8(x[m][i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
-                }
-            }
-            s2 = wave_sum(s2);
-            const float rs = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps);
-#pragma unroll
-            for (int i = 0; i < PF; i++) {
-                const half8v t = as_half8(x[m][i]), gv = as_half8(gr[i]), bb = as_half8(br[i]);
-                half8v o;
-#pragma unroll
-                for (int j = 0; j < 8; j++) o[j] = ln_norm1((float)t[j], mu, rs, p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bb[j]);
-                x[m][i] = lane * 8 + 512 * i < p.K ? __builtin_bit_cast(u32x4, o) : z;
-            }
-        }
-    }
-    float acc[R][MT];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int m = 0; m < MT; m++) acc[r][m] = 0.0f;
+        for (int i = 0; i < PF; i++) x[m][i] = ldg16(p.A + (long)min(m, p.M - 1) * p.ldA + min(lane * 8 + 512 * i, p.K - 8));
+    fk_request(p, w, n, lane);
+    FkOut<MT, 1> out;
+    out.request(p, n, lane);
+    float acc[MT] = {};
 #pragma unroll
     for (int i = 0; i < PF; i++)
+        if (lane * 8 + 512 * i < p.K) {
 #pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int m = 0; m < MT; m++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const uint32_t wq = w[r][i][q], xq = x[m][i][q];
-                    acc[r][m] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, wq), __builtin_bit_cast(half2v, xq), acc[r][m], false);
-                }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        float mine = 0.0f;                                // lane m keeps row m's sum
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            const float sres = wave_sum(acc[r][m]);
-            if (lane == m) mine = sres;
+            for (int m = 0; m < MT; m++) acc[m] = fk_dot(w[0][i], x[m][i], acc[m]);
         }
-        if (lane < p.M && n0 + r < p.N) {
-            const float v = mine + bv[r];
-            const long off = (long)lane * p.ldY + n0 + r;
-            if (p.out_f32) reinterpret_cast<float *>(p.Y)[off] = apply_epi(v, p.epi);
-            else {
-                half_t o = (half_t)apply_epi((float)(half_t)v, p.epi);
-                if (p.residual) o = (half_t)((float)o + rv[r]);
-                reinterpret_cast<half_t *>(p.Y)[off] = o;
-            }
-        }
+    float mine = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+        const float sres = wave_sum(acc[m]);
+        if (lane == m) mine = sres;
     }
+    out.store(p, mine, n, lane);
 }
 
 // k-slice depth for the [K][F] skinny kernel: enough workgroups to put ~2 on every CU, slices a
@@ -577,9 +572,109 @@ int skinny_kper(int64_t K, int64_t F) {
     return (int)kper;
 }
 
-// few_rows_kernel from five rows on (us at 4 and 8 rows, staged kernel | matrix cores; 1280 -> 5120 6.8 | 7.15 and 8.6 | 7.4; 4096 -> 1024
-// 6.4 | 7.1 and 10.3 | 7.9; 5120 -> 1280 8.9 | 8.2 and 20.4 | 9.0; 1280 -> 51866 35.8 | 35.0 and 48 | 38; 1536 -> 384 3.8 | 4.4 and 4.9 | 4.65).
+// few_rows_kernel from five rows on.  us at four rows on the kernels above, at eight on the matrix cores: 1280 -> 5120 5.2 and 6.6, 4096 -> 1024
+// 5.7 and 7.2, 5120 -> 1280 7.6 and 8.4, 1280 -> 51866 27.3 and 26.2, 1536 -> 384 3.2 and 3.8 (the kernels above hold four rows at most).
 constexpr int FEW_ROWS_MIN = 5;
+
+template <int PF, int TURNS, bool LN>
+void launch_few(const GemmArgs &a, hipStream_t st) {
+    const int cols = ceil_div(a.N, 16) * 2 <= mi_num_cus() ? 8 : 16;
+    const int64_t wgs = ceil_div(a.N, cols);
+    // Past one workgroup a CU the registers of a norm (160 and up) let no second one in, and without a norm the activations are read once a
+    // workgroup: eight rows of 1280 -> 51866 30.5 us with a workgroup for every sixteen columns, 26.2 walking (behind a norm 70.5 and 28.4).
+    // Two workgroups a CU where the registers allow it and there are turns enough (384 -> 51866 13.6 | 10.0, -> 9000 3.9 | 4.0); from
+    // K = 1281 on none walks (2048 -> 8192 9.5 | 10.2).
+    if constexpr (TURNS == 1 && PF <= 5) {
+        const int64_t cus = mi_num_cus(), two = PF <= (LN ? 2 : 3) && wgs > 4 * cus ? 2 : 1;
+        if (wgs > cus) {
+            hipLaunchKernelGGL((few_rows_kernel<PF, 1, LN, true>), dim3((unsigned)(cus * two)), dim3(512), 0, st, a, cols);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((few_rows_kernel<PF, TURNS, LN, false>), dim3((unsigned)wgs), dim3(512), 0, st, a, cols);
+}
+
+// by the 32-deep steps that each of the eight waves takes of K <= 8192
+int launch_few_k(const GemmArgs &a, hipStream_t st) {
+    const int64_t per = ceil_div(ceil_div(a.K, 32), 8);
+    if (per > 32) return MI_DECLINE_EXTENT;
+    if (a.ln_on) {
+        if (per <= 2)       launch_few<2, 1, true>(a, st);
+        else if (per <= 3)  launch_few<3, 1, true>(a, st);
+        else if (per <= 4)  launch_few<4, 1, true>(a, st);
+        else if (per <= 5)  launch_few<5, 1, true>(a, st);
+        else if (per <= 6)  launch_few<6, 1, true>(a, st);
+        else if (per <= 8)  launch_few<8, 1, true>(a, st);
+        else if (per <= 10) launch_few<10, 1, true>(a, st);
+        else if (per <= 12) launch_few<6, 2, true>(a, st);
+        else if (per <= 16) launch_few<8, 2, true>(a, st);
+        else if (per <= 20) launch_few<10, 2, true>(a, st);
+        else if (per <= 24) launch_few<8, 3, true>(a, st);
+        else                launch_few<8, 4, true>(a, st);
+    } else {
+        if (per <= 2)       launch_few<2, 1, false>(a, st);
+        else if (per <= 3)  launch_few<3, 1, false>(a, st);
+        else if (per <= 4)  launch_few<4, 1, false>(a, st);
+        else if (per <= 5)  launch_few<5, 1, false>(a, st);
+        else if (per <= 6)  launch_few<6, 1, false>(a, st);
+        else if (per <= 8)  launch_few<8, 1, false>(a, st);
+        else if (per <= 10) launch_few<10, 1, false>(a, st);
+        else if (per <= 12) launch_few<12, 1, false>(a, st);
+        else if (per <= 16) launch_few<16, 1, false>(a, st);
+        else if (per <= 20) launch_few<20, 1, false>(a, st);
+        else if (per <= 24) launch_few<12, 2, false>(a, st);
+        else                launch_few<16, 2, false>(a, st);
+    }
+    return MI_OK;
+}
+
+template <int MT, int PF>
+void launch_fk(const GemmArgs &a, hipStream_t st) {
+    const size_t lds = (size_t)MT * a.K * sizeof(half_t);
+    const int64_t cus = mi_num_cus();
+    auto go = [&](auto R_, auto LN_, int64_t cap) {
+        constexpr int R = decltype(R_)::value;
+        const int64_t wgs = ceil_div(a.N, 4 * R);
+        hipLaunchKernelGGL((skinny_fk_kernel<MT, PF, R, decltype(LN_)::value>), dim3((unsigned)(wgs < cap ? wgs : cap)), dim3(256), lds, st, a);
+    };
+    using std::integral_constant;
+    if constexpr (PF > 3) {                               // (a long row fills the registers by itself)
+        if (a.ln_on) go(integral_constant<int, 1>{}, std::true_type{}, 8 * cus);
+        else go(integral_constant<int, 1>{}, std::false_type{}, 8 * cus);
+    } else {
+        // Up to 8192 columns every group has its wave.  A wider output -- a vocabulary -- is walked by two or three workgroups a CU, three columns a
+        // wave and turn: 1280 -> 51866 at one, two and four rows 24.3, 25.1, 27.3 us (30.5, 32.1, 35.0 with a column a wave, eight
+        // workgroups a CU and the next column asked for behind a branch), behind a norm 24.0, 24.6, 27.6 (31.9, 34.4, 38.4).
+        if (!a.ln_on && a.N <= 8192) {
+            if constexpr (MT <= 2) hipLaunchKernelGGL((skinny_fk_reg_kernel<MT, PF>), dim3((unsigned)ceil_div(a.N, 4)), dim3(256), 0, st, a);
+            else go(integral_constant<int, 1>{}, std::false_type{}, 8 * cus);
+        } else if (!a.ln_on) {
+            go(integral_constant<int, 3>{}, std::false_type{}, 3 * cus);
+        } else switch (a.N <= 8192 ? ceil_div(a.N, 4 * cus) : 3) {
+            case 0: case 1: case 2: go(integral_constant<int, 2>{}, std::true_type{}, 2 * cus); break;
+            case 3: go(integral_constant<int, 3>{}, std::true_type{}, 2 * cus); break;
+            case 4: go(integral_constant<int, 4>{}, std::true_type{}, 2 * cus); break;
+            default: go(integral_constant<int, 5>{}, std::true_type{}, 2 * cus); break;
+        }
+    }
+}
+
+template <int MT, int PF>
+int raise_fk() {
+    auto up = [](auto kern) { return raise_lds(kern, (int)SKINNY_FK_LDS_MAX); };
+    return up(skinny_fk_kernel<MT, PF, 1, false>) | up(skinny_fk_kernel<MT, PF, 1, true>);
+}
+
+template <int MT>
+void launch_fk_k(const GemmArgs &a, hipStream_t st) {
+    if (a.K <= 512) launch_fk<MT, 1>(a, st);
+    else if (a.K <= 1024) launch_fk<MT, 2>(a, st);
+    else if (a.K <= 1536) launch_fk<MT, 3>(a, st);
+    else if (a.K <= 3072) launch_fk<MT, 6>(a, st);
+    else if (a.K <= 4096) launch_fk<MT, 8>(a, st);
+    else if (a.K <= 5120) launch_fk<MT, 10>(a, st);
+    else launch_fk<MT, 12>(a, st);
+}
 
 }  // namespace
 
@@ -604,63 +699,19 @@ int mi_skinny_launch(const GemmArgs &a, bool b_kn, void *ws, size_t ws_bytes, hi
         const size_t lds = (size_t)mt * a.K * sizeof(half_t);
         if (a.M > 8 || lds > SKINNY_FK_LDS_MAX) return MI_DECLINE_EXTENT;
         if (a.M >= FEW_ROWS_MIN) {
-            const int cols = ceil_div(a.N, 16) * 2 <= mi_num_cus() ? 8 : 16, per = (int)ceil_div(ceil_div(a.K, 32), 8);
-            const dim3 grid((unsigned)ceil_div(a.N, cols));
-            if (a.ln_on) {
-                if (per <= 5) hipLaunchKernelGGL((few_rows_kernel<5, true>), grid, dim3(512), 0, st, a, cols);
-                else          hipLaunchKernelGGL((few_rows_kernel<10, true>), grid, dim3(512), 0, st, a, cols);
-            } else {
-                if (per <= 5)       hipLaunchKernelGGL((few_rows_kernel<5, false>), grid, dim3(512), 0, st, a, cols);
-                else if (per <= 10) hipLaunchKernelGGL((few_rows_kernel<10, false>), grid, dim3(512), 0, st, a, cols);
-                else                hipLaunchKernelGGL((few_rows_kernel<20, false>), grid, dim3(512), 0, st, a, cols);
-            }
-            return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-        }
-        // rows per wave: as many as still leave every CU a workgroup, at most eight (a workgroup stages
-        // all M activation rows once, whatever the number of weight rows it then streams)
-        // One weight row per wave.  More rows per wave would amortise the staging of the activations, but the
-        // rows of a wave run one after the other, each a chain of dependent memory trips: measured slower at
-        // every batch size (1280 -> 5120, batch 8: 9.1 us with one row, 13.7 us with four).
-        // One or two rows without a norm in front: activations in registers, no staging (hot in a replayed graph at
-        // batch 1: 2.88 / 3.13 / 3.34 us for 1280 -> 1280 / 3840 / 5120 against 3.01 / 3.33 / 3.57 us staged).  With
-        // the layer-norm prologue every wave would normalise its own copy of the row -- 4.5 / 6.1 / 6.9 us against
-        // 3.9 / 4.3 / 4.7 us -- so that stays staged, and so does a very wide output (51866 columns: 24.5 against 23.0 us).
-        int R = 1;
-        if (!a.ln_on && a.N <= 8192 && a.K <= 1536 && mt <= 2) {
-            dim3 rg((unsigned)ceil_div(a.N, 4 * R));
-            if (R == 2) {
-                if (mt == 1)      hipLaunchKernelGGL((skinny_fk_reg_kernel<1, 3, 2>), rg, dim3(256), 0, st, a);
-                else              hipLaunchKernelGGL((skinny_fk_reg_kernel<2, 3, 2>), rg, dim3(256), 0, st, a);
-            } else {
-                if (mt == 1)      hipLaunchKernelGGL((skinny_fk_reg_kernel<1, 3, 1>), rg, dim3(256), 0, st, a);
-                else              hipLaunchKernelGGL((skinny_fk_reg_kernel<2, 3, 1>), rg, dim3(256), 0, st, a);
-            }
-            return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-        }
-        // every column its own wave up to eight workgroups per CU; beyond that (a vocabulary projection) a wave walks
-        // several columns behind one staging of the activations
-        const int64_t wgs = ceil_div(a.N, 4), cap = (int64_t)mi_num_cus() * 8;
-        dim3 grid((unsigned)(wgs < cap ? wgs : cap));
-        if (a.K <= 1536) {
-            if (mt == 1)      hipLaunchKernelGGL((skinny_fk_kernel<1, 3>), grid, dim3(256), lds, st, a);
-            else if (mt == 2) hipLaunchKernelGGL((skinny_fk_kernel<2, 3>), grid, dim3(256), lds, st, a);
-            else              hipLaunchKernelGGL((skinny_fk_kernel<4, 3>), grid, dim3(256), lds, st, a);
-        } else {
-            if (mt == 1)      hipLaunchKernelGGL((skinny_fk_kernel<1, 12>), grid, dim3(256), lds, st, a);
-            else if (mt == 2) hipLaunchKernelGGL((skinny_fk_kernel<2, 12>), grid, dim3(256), lds, st, a);
-            else              hipLaunchKernelGGL((skinny_fk_kernel<4, 12>), grid, dim3(256), lds, st, a);
-        }
+            const int rc = launch_few_k(a, st);
+            if (rc != MI_OK) return rc;
+        } else if (mt == 1) launch_fk_k<1>(a, st);
+        else if (mt == 2) launch_fk_k<2>(a, st);
+        else launch_fk_k<4>(a, st);
     }
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
 int mi_skinny_init() {
     int bad = 0;
-    bad |= raise_lds(skinny_fk_kernel<1, 3>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<2, 3>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<4, 3>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<1, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<2, 12>, (int)SKINNY_FK_LDS_MAX);
-    bad |= raise_lds(skinny_fk_kernel<4, 12>, (int)SKINNY_FK_LDS_MAX);
+    bad |= raise_fk<1, 6>() | raise_fk<1, 8>() | raise_fk<1, 10>() | raise_fk<1, 12>();
+    bad |= raise_fk<2, 6>() | raise_fk<2, 8>() | raise_fk<2, 10>() | raise_fk<2, 12>();
+    bad |= raise_fk<4, 6>() | raise_fk<4, 8>() | raise_fk<4, 10>() | raise_fk<4, 12>();
     return bad;
 }

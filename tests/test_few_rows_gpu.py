@@ -55,3 +55,32 @@ def test_norm_without_gamma_of_rows_far_from_zero(ctx, K, beta):
     h = poison(torch.empty((T, K), dtype=torch.float16, device="cuda"))
     jv.layernorm_(ctx, h, None, None, to_dev(X), None, to_dev(be) if beta else None, K, 1e-5)
     assert_parity(to_host(out), oracle.gemm_f16(to_host(h), W), what=f"K{K} beta {beta}")
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 6, 8])
+@pytest.mark.parametrize("K,F", [(8, 12353), (512, 2053), (520, 8197), (1024, 3071), (1032, 4099), (1288, 5117), (1536, 16397), (3072, 37), (4104, 21), (6152, 19)])
+def test_rows_of_every_depth_and_width(ctx, T, K, F):
+    """The kernels are picked by K (chunks asked for at the top) and F (columns a wave, workgroups that walk): either side of each edge,
+    columns off every group, with a bias and without, with the norm in front and without."""
+    import torch
+    import juliavision_amd as jv
+    X, W, b = oracle.randn_f16((T, K), 1, 0, 1.0), oracle.randn_f16((K, F), 2, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((F,), 3, 0, 0.1)
+    R, g, beta = oracle.randn_f16((T, F), 4), oracle.randn_f16((K,), 5, 1.0, 0.1), oracle.randn_f16((K,), 6, 0, 0.1)
+    w, dx, db, dr = to_dev(np.ascontiguousarray(W.T)).t(), to_dev(X), to_dev(b), to_dev(R)
+    new = lambda: poison(torch.empty((T, F), dtype=torch.float16, device="cuda"))
+    h = torch.empty((T, K), dtype=torch.float16, device="cuda")
+    jv.layernorm_(ctx, h, None, None, dx, to_dev(g), to_dev(beta), K, 1e-5)
+    for bias, res in ((db, dr), (None, None)):
+        plain, folded, apart = new(), new(), new()
+        kw = {"residual": res, "epi": "gelu"}
+        ctx.ws.reset()
+        jv.matmul_(ctx, plain, w, dx, bias, **kw)
+        assert_parity(to_host(plain), oracle.gemm_f16(X, W, None if bias is None else b, epi="gelu", residual=None if res is None else R), what=f"T{T} K{K} F{F}")
+        ctx.ws.reset()
+        jv.ln_matmul_(ctx, folded, w, dx, to_dev(g), to_dev(beta), 1e-5, bias, **kw)
+        ctx.ws.reset()
+        jv.matmul_(ctx, apart, w, h, bias, **kw)
+        if K <= 4096:                                     # the norm kernel walks longer rows in another order
+            assert torch.equal(folded, apart)
+        else:
+            assert_parity(to_host(folded), to_host(apart), what=f"norm T{T} K{K} F{F}")
