@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmi355dnn.so")
 HOST = os.path.join(HERE, "_host.so")
-SOURCES = ["gemm.hip", "gemm_skinny.hip", "gemm_pipe.hip", "gemm_ring.hip", "gemm_deep.hip", "gemm_any.hip", "sdpa.hip", "sdpa_tile.hip", "conv.hip", "conv_tile.hip", "convtranspose.hip", "layernorm.hip", "kvcache.hip", "layout.hip", "probe.hip"]
+SOURCES = ["gemm.hip", "gemm_skinny.hip", "gemm_pipe.hip", "gemm_ring.hip", "gemm_deep.hip", "gemm_any.hip", "sdpa.hip", "sdpa_tile.hip", "sdpa_decode.hip", "conv.hip", "conv_tile.hip", "convtranspose.hip", "layernorm.hip", "kvcache.hip", "layout.hip", "probe.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.
 # -Xarch_device -fno-honor-nans: no kernel relies on NaN propagation (infinities stay honoured: they are the masks);

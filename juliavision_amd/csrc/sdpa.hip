@@ -16,7 +16,6 @@
 // Operands are (E, L, H, B) with element strides (the reference's layout,
 // DNNKernels/src/kernels/extern/attention.jl:1-22); out is dense (E, Lq, H, B).
 #include "sdpa_common.hpp"
-#include <atomic>
 #include <cstdlib>
 
 namespace {
@@ -830,197 +829,6 @@ __global__ __launch_bounds__(256) void sdpa_rows_kernel(SdpaArgs p) {
     }
 }
 
-// Single query row per (head, batch): 8-wave workgroups, `nsplit` of them per row, each over its share of the key
-// range.  A wave takes keys 8 at a time (8 lanes per key, one 16-byte chunk of the head dim each) with a stride of
-// 64 keys, in rounds of SD_U passes whose K and V loads are all issued before the first is used, the next round's
-// before the current round is consumed: about 190 KB in flight per workgroup.
-//
-// Such a launch moves a few MB, so its duration is a chain of trips to memory.  Every address is therefore made
-// independent of loaded data: the key range is cut by the cache's capacity (p.Lk), not by kv_len, and keys are
-// requested up to the capacity -- valid memory whatever the length -- together with the length itself, the query
-// and the new row; the length only masks scores afterwards.  One trip, then arithmetic.
-//
-// nsplit > 1: the workgroups of one row run on one XCD (workgroup ids are dealt to XCDs round robin, so ids that
-// differ by multiples of 8 share an L2), write their partial (max, sum, o[E]) to part_o / part_ml, and take a ticket;
-// whoever draws the last ticket merges the partials in split order -- so the result does not depend on who that
-// is -- writes the row and puts the ticket counter back to zero.  Nobody waits for anybody: every workgroup exits
-// after its own work.  The exchange stays inside that one L2: a partial is written with plain stores, waited for
-// (vmcnt) and followed by the ticket, an atomic the L2 performs; the merging workgroup reads with loads that go to
-// the L2.  A device-scope release per workgroup instead (__threadfence) writes the whole L2 back each time: measured
-// 63 us for 320 workgroups against 6 us unsplit.  The host only splits on a device whose probe showed the round-robin
-// placement this relies on.
-constexpr int SD_U = 6;
-__global__ __launch_bounds__(512) void sdpa_decode_kernel(SdpaArgs p) {
-    __shared__ float red_ml[8][2];
-    __shared__ float red_o[8][64];
-    __shared__ int is_last;
-    stage_decode_args(p);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int grp = lane >> 3, cl = lane & 7;
-    const int S = p.nsplit;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    unsigned split_, h_;
-    const int unit = (int)divide(slot, S, p.div_split, split_) * 8 + xcd, split = (int)split_;
-    if (unit >= p.H * p.B) return;                       // the grid is padded to whole groups of 8 rows
-    const int b = (int)divide(unit, p.H, p.div_h, h_), h = (int)h_;
-    const int cap = p.Lk;
-    const int npass = (cap + 63) >> 6, per = p.per;
-    const int t_lo = split * per, t_hi = min(npass, t_lo + per);
-    const half_t *qp = p.q + h * p.qs[2] + b * p.qs[3];
-    half_t *kb = const_cast<half_t *>(p.k) + h * p.ks[2] + b * p.ks[3];
-    half_t *vb = const_cast<half_t *>(p.v) + h * p.vs[2] + b * p.vs[3];
-    const int e0 = cl * 8;
-    const bool eok = e0 < p.E;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    const int n_raw = p.kv_len ? p.kv_len[b] : cap;
-    u32x4 kc[2][SD_U], vc[2][SD_U];
-    // pass t of this wave covers keys 64 t + 8 wave + grp
-    auto fetch = [&](int set, int t0) {
-#pragma unroll
-        for (int u = 0; u < SD_U; u++) {
-            const int kk = min(64 * (t0 + u) + 8 * wave + grp, cap - 1);
-            const bool on = eok && t0 + u < t_hi;
-            kc[set][u] = on ? ldg16(kb + (long)kk * p.ks[1] + e0) : z;
-            vc[set][u] = on ? ldg16(vb + (long)kk * p.vs[1] + e0) : z;
-        }
-    };
-    if (t_lo < t_hi) fetch(0, t_lo);
-    if (t_lo + SD_U < t_hi) fetch(1, t_lo + SD_U);
-    u32x4 kn = z, vn = z;                                // the row that this step appends
-    if (p.k_new && eok) {
-        kn = ldg16(p.k_new + h * p.ns[2] + b * p.ns[3] + e0);
-        vn = ldg16(p.v_new + h * p.ns[2] + b * p.ns[3] + e0);
-    }
-    float qv[8];
-    {
-        const half8v t = as_half8(eok ? ldg16(qp + e0) : z);
-#pragma unroll
-        for (int j = 0; j < 8; j++) qv[j] = (float)t[j] * p.scale;
-    }
-    // a length past the capacity: the cache is full, the new row is neither stored nor attended
-    const int Lk = max(0, min(cap, n_raw));
-    const int fresh = p.k_new && n_raw <= cap ? Lk - 1 : -1;
-    float m = -INFINITY, l = 0.0f, acc[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) acc[j] = 0.0f;
-    auto consume = [&](int set, int t0) {
-#pragma unroll
-        for (int u = 0; u < SD_U; u++) {
-            if (t0 + u < t_hi && 64 * (t0 + u) < Lk) {           // uniform: the shuffles below need the whole wave
-                const int key = 64 * (t0 + u) + 8 * wave + grp;
-                u32x4 kr = kc[set][u], vr = vc[set][u];
-                if (key == fresh) {                              // exactly eight lanes of one workgroup own it
-                    kr = kn; vr = vn;
-                    if (eok) {
-                        *reinterpret_cast<u32x4 *>(kb + (long)key * p.ks[1] + e0) = kn;
-                        *reinterpret_cast<u32x4 *>(vb + (long)key * p.vs[1] + e0) = vn;
-                    }
-                }
-                if (key >= Lk) vr = z;                           // a weight of zero would not hide what an unwritten slot may hold
-                const half8v kt = as_half8(kr), vt = as_half8(vr);
-                float d = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; j++) d = fmaf(qv[j], (float)kt[j], d);
-                d += lane_xor<1>(d);
-                d += lane_xor<2>(d);
-                d += lane_xor<4>(d);
-                const float sc = key < Lk ? d : -INFINITY;
-                const float mn = fmaxf(m, sc);
-                const float mu = mn == -INFINITY ? 0.0f : mn;
-                const float al = __expf(m - mu), pw = __expf(sc - mu);
-                l = l * al + pw;
-                m = mn;
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[j] = fmaf(pw, (float)vt[j], acc[j] * al);
-            }
-        }
-    };
-    for (int t0 = t_lo; t0 < t_hi; t0 += 2 * SD_U) {
-        consume(0, t0);
-        if (t0 + 2 * SD_U < t_hi) fetch(0, t0 + 2 * SD_U);
-        if (t0 + SD_U < t_hi) consume(1, t0 + SD_U);
-        if (t0 + 3 * SD_U < t_hi) fetch(1, t0 + 3 * SD_U);
-    }
-    // merge the 8 groups of the wave, then the 8 waves through LDS (flash.jl:1385-1391)
-#pragma unroll
-    for (int o = 8; o < 64; o <<= 1) {
-        const float mo = __shfl_xor(m, o, 64), lo = __shfl_xor(l, o, 64);
-        const float mn = fmaxf(m, mo);
-        const float mu = mn == -INFINITY ? 0.0f : mn;
-        const float a0 = __expf(m - mu), a1 = __expf(mo - mu);
-        l = l * a0 + lo * a1;
-#pragma unroll
-        for (int j = 0; j < 8; j++) acc[j] = acc[j] * a0 + __shfl_xor(acc[j], o, 64) * a1;
-        m = mn;
-    }
-    if (lane < 8) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) red_o[wave][cl * 8 + j] = acc[j];
-        if (lane == 0) { red_ml[wave][0] = m; red_ml[wave][1] = l; }
-    }
-    __syncthreads();
-    float mm = -INFINITY, L = 0.0f, O = 0.0f;
-    if (tid < 64) {
-#pragma unroll
-        for (int w = 0; w < 8; w++) mm = fmaxf(mm, red_ml[w][0]);
-        const float mu = mm == -INFINITY ? 0.0f : mm;
-#pragma unroll
-        for (int w = 0; w < 8; w++) {
-            const float a = __expf(red_ml[w][0] - mu);
-            L += a * red_ml[w][1];
-            O += a * red_o[w][tid];
-        }
-    }
-    if (S > 1) {                                         // uniform
-        const long row = (long)unit * S + split;
-        if (tid < p.E) p.part_o[row * p.E + tid] = O;
-        if (tid == 0) { p.part_ml[row * 2] = mm; p.part_ml[row * 2 + 1] = L; }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's part of the partial has reached the L2 ...
-        __syncthreads();                                  // ... and so has everybody's, before the ticket is drawn
-        if (tid == 0) {
-            const unsigned t = __hip_atomic_fetch_add(p.tickets + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            is_last = t == (unsigned)(S - 1);
-            if (is_last) __hip_atomic_store(p.tickets + unit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
-        }
-        __syncthreads();
-        if (!is_last) return;
-        mm = -INFINITY; L = 0.0f; O = 0.0f;
-        if (tid < p.E) {
-            const long r0 = (long)unit * S;
-            for (int s0 = 0; s0 < S; s0 += 8) {
-                float ms[8], ls[8], os_[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const long r = r0 + min(s0 + j, S - 1);
-                    // read at the L2, past this compute unit's own cache
-                    ms[j] = s0 + j < S ? __hip_atomic_load(p.part_ml + r * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
-                    ls[j] = __hip_atomic_load(p.part_ml + r * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    os_[j] = __hip_atomic_load(p.part_o + r * p.E + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                float mb = mm;
-#pragma unroll
-                for (int j = 0; j < 8; j++) mb = fmaxf(mb, ms[j]);
-                const float mu = mb == -INFINITY ? 0.0f : mb;
-                const float a0 = __expf(mm - mu);
-                L *= a0; O *= a0;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float a = __expf(ms[j] - mu);  // a split past the end has m = -inf: weight 0
-                    L += a * ls[j];
-                    O += a * os_[j];
-                }
-                mm = mb;
-            }
-        }
-    }
-    if (tid < p.E) {
-        const float r = L > 0.0f ? O / L : 0.0f;
-        const long oo = (long)b * p.os[3] + (long)h * p.os[2] + (long)tid * p.os[0];
-        if (p.out_f32) reinterpret_cast<float *>(p.out)[oo] = r;
-        else reinterpret_cast<half_t *>(p.out)[oo] = (half_t)r;
-    }
-}
-
 // One thread per (row, e): merges the key splits (attn_flash_cm_merge!, flash.jl:1398-1421).
 __global__ void sdpa_merge_kernel(SdpaArgs p) {
     const long rows = (long)p.B * p.H * p.Lq;
@@ -1185,61 +993,7 @@ int flash_tile_waves(int64_t E, int64_t Lq, int64_t Lk, int64_t H, int64_t B, bo
     return waves;
 }
 
-// A single query row (a decode step) runs in one launch of sdpa_decode_kernel: the work follows the device-side kv_len
-// and the cache write can ride along (mi_sdpa_append_f16).  Twenty heads alone leave most of the chip idle and give each
-// workgroup a long chain of keys, so a long key range is cut over several workgroups per row -- at most one workgroup
-// per compute unit, a round of six 64-key passes each -- which merge inside the launch.  Head dim <= 64, 16-byte addressable
-// operands, no additive mask; the rest goes to sdpa_rows_kernel (+ sdpa_merge_kernel).
-constexpr int SD_BANKS = 16, SD_TICKETS = 4096, SD_PART_FLOATS = 1 << 16;
-// Arrival counters and partials of the split form: a launch takes the next of SD_BANKS banks, so launches in flight
-// together on one GPU (up to SD_BANKS of them) do not touch each other's.  Zero when the module loads; every launch
-// leaves its counters at zero.
-static __device__ unsigned sd_ticket_words[SD_BANKS * SD_TICKETS];
-static __device__ __align__(256) float sd_part_words[SD_BANKS * SD_PART_FLOATS];
-constexpr int SD_MAX_DEVICES = 64;
-unsigned *g_sd_tickets[SD_MAX_DEVICES] = {};
-float *g_sd_parts[SD_MAX_DEVICES] = {};
-std::atomic<unsigned> g_sd_launch{0};
-
-bool one_pass_decode(const SdpaArgs &a, bool vec) {
-    return a.Lq == 1 && vec && !a.bias && a.E <= 64 && a.Lk >= 1 && (int64_t)a.H * a.B <= SD_TICKETS;
-}
-
-int decode_splits(int64_t E, int64_t Lk, int64_t H, int64_t B) {
-    const int64_t units = H * B, passes = ceil_div(Lk, 64);
-    // The exchange adds about 3 us of its own (partial out, ticket, partials in: three trips in a row), a workgroup
-    // walks six passes in about one trip: 448 keys stay whole (5.9 us either way at batch 1), 1500 keys are cut
-    // four ways at batch 1 (11.1 us whole, 7.2 us cut in 4, 10.2 us cut in 12) and three ways at batch 4.
-    int64_t want = mi_num_cus() / units;                 // at most one workgroup per compute unit
-    if (want > ceil_div(passes, SD_U)) want = ceil_div(passes, SD_U);      // one round of passes each
-    if (passes <= 8) want = 1;
-    if (want > 32) want = 32;
-    while (want > 1 && units * want * (E + 2) > SD_PART_FLOATS) want--;
-    if (want < 1) want = 1;
-    // no empty split: with `per` passes each, the last one must still start inside the range
-    while (want > 1 && ceil_div(passes, want) * (want - 1) >= passes) want--;
-    return (int)want;
-}
-
-// Fills in the split count and, for a split launch, this launch's bank of counters and partials, and launches.
-int launch_decode(SdpaArgs &a, hipStream_t st) {
-    a.nsplit = decode_splits(a.E, a.Lk, a.H, a.B);
-    if (a.nsplit > 1) {
-        int dev = -1;
-        if (!mi_xcd_round_robin() || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= SD_MAX_DEVICES || !g_sd_tickets[dev]) a.nsplit = 1;
-        else {
-            const unsigned bank = g_sd_launch++ % SD_BANKS;
-            a.tickets = g_sd_tickets[dev] + (size_t)bank * SD_TICKETS;
-            a.part_o = g_sd_parts[dev] + (size_t)bank * SD_PART_FLOATS;
-            a.part_ml = a.part_o + (size_t)a.H * a.B * a.nsplit * a.E;
-        }
-    }
-    a.per = (int)ceil_div(ceil_div(a.Lk, 64), a.nsplit);
-    a.div_split = recip_of(a.nsplit);
-    const unsigned units8 = (unsigned)ceil_div((int64_t)a.H * a.B, 8);
-    hipLaunchKernelGGL(sdpa_decode_kernel, dim3(units8 * 8 * a.nsplit), dim3(512), 0, st, a);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
-}
+bool one_pass_decode(const SdpaArgs &a, bool vec) { return vec && mi_sdpa_decode_takes(a); }
 
 // A mask the fused kernel can carry: keys contiguous (a lane reads runs of four), the other axes any stride including
 // broadcast; fp16 runs are read as two dwords, so every row must start on a 4-byte boundary.  An fp16 mask with the
@@ -1280,7 +1034,7 @@ Route route_of(const SdpaArgs &a) {
     }
     if (path == MI_SDPA_FLASH) return {MI_SDPA_KERNEL_FUSED, 0, a.bias ? 1 : flash_splits(a.E, a.Lq, a.Lk, a.H, a.B)};
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
-    if (one_pass_decode(a, vec)) return {MI_SDPA_KERNEL_ONE_QUERY, 0, decode_splits(a.E, a.Lk, a.H, a.B)};
+    if (one_pass_decode(a, vec)) return {MI_SDPA_KERNEL_ONE_QUERY, 0, mi_sdpa_decode_splits(a.E, a.Lk, a.H, a.B)};
     return {MI_SDPA_KERNEL_ROWS, 0, a.Lq < 64 ? rows_splits(a.Lq, a.Lk, a.H, a.B) : 1};
 }
 
@@ -1319,15 +1073,7 @@ void launch_rows(const SdpaArgs &a, bool vec, dim3 grid, hipStream_t st) {
 // default 64 KiB of dynamic LDS.
 int mi_sdpa_init() {
     int bad = 0;
-    {   // this device's copies of the decode kernel's counters and partials (zeroed at load; never named in host code again)
-        int dev = -1;
-        void *t = nullptr, *pw = nullptr;
-        if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < SD_MAX_DEVICES &&
-            hipGetSymbolAddress(&t, HIP_SYMBOL(sd_ticket_words)) == hipSuccess && hipGetSymbolAddress(&pw, HIP_SYMBOL(sd_part_words)) == hipSuccess) {
-            g_sd_tickets[dev] = reinterpret_cast<unsigned *>(t);
-            g_sd_parts[dev] = reinterpret_cast<float *>(pw);
-        }
-    }
+    mi_sdpa_decode_init();
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, false>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_lds_bytes(64)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, true>), hipFuncAttributeMaxDynamicSharedMemorySize, flash_lds_bytes(64)) != hipSuccess;
     bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_fwd_kernel<64, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * flash_lds_bytes(64)) != hipSuccess;
@@ -1376,7 +1122,7 @@ int mi_sdpa_f16_plan(const void *q, const int64_t q_strides[4], const void *k, c
     if (rc != MI_OK) return MI_SDPA_DECLINE;
     int path = sdpa_path(a);
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
-    if (nsplit_out) *nsplit_out = (path == MI_SDPA_ROWS && Lq < 64) ? (one_pass_decode(a, vec) ? decode_splits(E, Lk, H, B) : rows_splits(Lq, Lk, H, B))
+    if (nsplit_out) *nsplit_out = (path == MI_SDPA_ROWS && Lq < 64) ? (one_pass_decode(a, vec) ? mi_sdpa_decode_splits(E, Lk, H, B) : rows_splits(Lq, Lk, H, B))
                                   : (path == MI_SDPA_FLASH && !has_bias && !(E == 64 && Lq >= 64 && flash_tile_waves(E, Lq, Lk, H, B, false))) ? flash_splits(E, Lq, Lk, H, B) : 1;
     return path;
 }
@@ -1487,7 +1233,7 @@ int mi_sdpa_f16(void *out, int out_dtype, const int64_t out_strides[4],
     }
     // rows path
     bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E);
-    if (r.kernel == MI_SDPA_KERNEL_ONE_QUERY) return launch_decode(a, st);
+    if (r.kernel == MI_SDPA_KERNEL_ONE_QUERY) return mi_sdpa_decode_launch(a, st);
     a.nsplit = r.nsplit;
     if (a.nsplit > 1) {
         size_t rows = (size_t)Lq * H * B;
@@ -1527,7 +1273,7 @@ int mi_sdpa_append_f16(void *out, int out_dtype, const int64_t out_strides[4],
     const bool vec = vec_addressable(a.q, a.qs, a.E) && vec_addressable(a.k, a.ks, a.E) && vec_addressable(a.v, a.vs, a.E) &&
                      vec_addressable(a.k_new, a.ns, a.E) && vec_addressable(a.v_new, a.ns, a.E);
     if (!one_pass_decode(a, vec)) return MI_DECLINE_UNSUPPORTED;      // the caller appends and attends in two calls
-    return launch_decode(a, (hipStream_t)stream);
+    return mi_sdpa_decode_launch(a, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -42,7 +42,7 @@ __device__ __forceinline__ void stage_tile_args(const SdpaArgs &p) {
 __device__ __forceinline__ void stage_decode_args(const SdpaArgs &p) {
     asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.out), "s"(p.Lq), "s"(p.Lk), "s"(p.H), "s"(p.B), "s"(p.div_h), "s"(p.qs[2]), "s"(p.qs[3]),
                  "s"(p.ks[1]), "s"(p.ks[2]), "s"(p.ks[3]), "s"(p.vs[1]), "s"(p.vs[2]), "s"(p.vs[3]), "s"(p.os[2]), "s"(p.os[3]), "s"(p.E),
-                 "s"(p.nsplit), "s"(p.scale), "s"(p.kv_len), "s"(p.part_ml), "s"(p.k_new), "s"(p.ns[3]));
+                 "s"(p.nsplit), "s"(p.scale), "s"(p.kv_len), "s"(p.part_ml), "s"(p.k_new), "s"(p.ns[3]), "s"(p.per));
 }
 
 template <int N, typename F>
@@ -63,3 +63,9 @@ bool mi_sdpa_tile_takes(const SdpaArgs &p);
 bool mi_sdpa_tile_keymask(const SdpaArgs &p);
 int mi_sdpa_tile_launch(const SdpaArgs &p, int waves, bool f32, hipStream_t st);
 int mi_sdpa_tile_init();
+
+// sdpa_decode.hip: one query per (head, batch) in one launch, for operands that 16-byte loads can address.
+bool mi_sdpa_decode_takes(const SdpaArgs &p);
+int mi_sdpa_decode_splits(int64_t E, int64_t Lk, int64_t H, int64_t B);
+int mi_sdpa_decode_launch(const SdpaArgs &p, hipStream_t st);
+void mi_sdpa_decode_init();

@@ -297,3 +297,33 @@ def test_fill_cross_writes_the_projections_head_major(ctx, B, S, H, E, layout):
         for b in range(B):
             want = oracle.gemm_f16(enc[b], w, bias).reshape(S, H, E).transpose(1, 0, 2)
             assert_parity(got[1, b], want, what=f"fill_cross batch {b}")
+
+
+@pytest.mark.parametrize("Lk", [70, 700])
+def test_keys_too_far_apart_for_32_bit_offsets(ctx, Lk):
+    """A cache whose keys lie beyond 32-bit byte offsets: the same output and cache bits as the same cache laid out densely."""
+    import torch
+    import juliavision_amd as jv
+    B, H, E = 1, 2, 16
+    step = 2 ** 32 // (2 * (Lk + 64)) // 8 * 8 + 8                      # halves between keys: just past the limit
+    hk, hv = to_dev(oracle.randn_f16((B, H, Lk, E), 21)), to_dev(oracle.randn_f16((B, H, Lk, E), 22))
+    far = [torch.empty(step * Lk, dtype=torch.float16, device="cuda").as_strided((B, H, Lk, E), (step * Lk, E, step, 1)) for _ in range(2)]
+    far[0].copy_(hk)
+    far[1].copy_(hv)
+    q, kn, vn = (to_dev(oracle.randn_f16((B, H, 1, E), 23 + i)) for i in range(3))
+    length = torch.tensor([Lk - 3], dtype=torch.int32, device="cuda")
+    outs = []
+    for ck, cv in ((hk, hv), far):
+        for append in (False, True):
+            out = torch.full((B, H, 1, E), float("nan"), dtype=torch.float16, device="cuda")
+            ctx.ws.reset()
+            if append:
+                jv.sdpa_append(ctx, q, ck, cv, kn, vn, length, out=out)
+            else:
+                jv.sdpa(ctx, q, ck, cv, out=out, kv_len=length)
+            outs.append(to_host(out))
+    assert np.array_equal(to_host(far[0]), to_host(hk)) and np.array_equal(to_host(far[1]), to_host(hv))
+    want = oracle.sdpa_threepass_f16(to_host(q), to_host(hk), to_host(hv), kv_len=np.array([Lk - 3], dtype=np.int32))
+    assert_parity(outs[1], want, what=f"keys far apart Lk{Lk}")
+    for a, b in zip(outs[:2], outs[2:]):
+        assert_parity(a, b, what=f"far against dense Lk{Lk}")
