@@ -9,10 +9,9 @@
 // The next chunk's pieces are in flight in registers during this chunk's MFMAs.
 //
 // The im2col matrix (K / CC times the input), its GEMM's two reads of it and the launches between are gone: 1024 x 1024 x 3 ->
-// 144, 7 x 7 stride 4, 50.9 -> 24.2 us (floor 4.8).  Bound by its own serial chain: there (one chunk, all of it staged before the
-// first product) two waves a SIMD issue vector instructions in half of the cycles -- addresses, border shifts, the pixel operand
-// put together from two-byte reads, two-byte stores: 3200 a wave around 50 products -- and wait in the other half.  The LDS is
-// 11 % busy, the matrix units 6 %.
+// 144, 7 x 7 stride 4, 50.9 -> 15.1 us (floor 4.8).  Bound by its own serial chain, there one chunk, all of it staged before the
+// first product: of 25 000 clocks in the kernel 12 000 are the staging (two batches of loads, each a trip to memory, and at two-byte
+// addresses four times the vector-memory time of aligned ones), 6400 the products and the pixel operand's two-byte reads, 6500 the store.
 #include "conv_common.hpp"
 #include <type_traits>
 
@@ -22,19 +21,28 @@ namespace {
 
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
-struct TileConv : TilePlan { ConvArgs a; };
+// The plan, the problem, and the kernel's divisions as multiplications (divide): some thirty instructions each otherwise, four a piece.
+struct TileConv : TilePlan {
+    ConvArgs a;
+    unsigned div_x, div_taps, div_kw, div_tw, div_pc, div_pr, div_wp;
+};
 
 // PW waves side by side over pixels, KG groups of them over the steps of a chunk, TCO x 32 output channels each.
 // WP, PP: weight and patch pieces a thread carries in registers for the next chunk.
-template <int PW, int KG, int TCO>
+// CHUNKS: 1 a single chunk, 2 several, each a kernel of its own: together their conditions did not fit the scalar registers.  0 either,
+// for rows of the image or of the weights too short for a 16-byte piece, read by element.
+template <int PW, int KG, int TCO, int CHUNKS>
 __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
+    constexpr bool ELEM = CHUNKS == 0;
     constexpr int NT = PW * KG * 64, CO = 32 * TCO, WP = TCO > 2 ? 6 : 5, PP = 3;
     extern __shared__ __align__(16) char smem[];
     const ConvArgs &a = t.a;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pw = wave % PW, kg = wave / PW;
     const int taps = a.KH * a.KW, CRS = a.Cin * taps;
     const int HiWi = a.Hi * a.Wi;
-    const int tx = blockIdx.x % t.tiles_x, ty = blockIdx.x / t.tiles_x;
+    auto over = [](int v, int d, unsigned recip, int &left) { unsigned l; const int q = (int)divide((unsigned)v, (unsigned)d, recip, l); left = (int)l; return q; };
+    int tx;
+    const int ty = over(blockIdx.x, t.tiles_x, t.div_x, tx);
     const int oy0 = ty * t.TH, ox0 = tx * t.TW, co0 = blockIdx.y * CO;
     const half_t *x = a.x + (long)blockIdx.z * a.Cin * HiWi;
     const int iy0 = oy0 * a.sy - a.py, ix0 = ox0 * a.sx - a.px;
@@ -46,14 +54,15 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
     for (int k = tid; k < t.ksteps * 16; k += NT) {
         int off = zero_at;
         if (k < t.kc) {
-            const int ci = k / taps, r = k - ci * taps, kh = r / a.KW, kw = r - kh * a.KW;
+            int r, kw;
+            const int ci = over(k, taps, t.div_taps, r), kh = over(r, a.KW, t.div_kw, kw);
             off = (ci * t.PR + kh * a.dy) * t.PCL + kw * a.dx;
         }
         tab[k] = (unsigned short)off;
     }
 
     // Eight halves of which the first `gone` are dropped and zeros follow: what a load that was moved back to stay inside its
-    // row turns into.  Branches around such loads instead made every border tile wait for eight loads one after the other.
+    // row turns into.
     auto shifted = [](u32x4 v, int gone) {
         const uint64_t lo = (uint64_t)v[0] | (uint64_t)v[1] << 32, hi = (uint64_t)v[2] | (uint64_t)v[3] << 32;
         const int b = 16 * gone;                         // 0 .. 112
@@ -61,14 +70,15 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         const u32x4 r = {(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
         return r;
     };
-    const bool narrow = a.Wi < 8, short_w = weights_by_element(t.kc, CRS);      // uniform: rows without a whole piece go by element
+    const bool narrow = ELEM && a.Wi < 8, short_w = ELEM && weights_by_element(t.kc, CRS);      // uniform
     const u32x4 zero4 = {0u, 0u, 0u, 0u};
     // A 16-byte piece: where it lies in memory (halves from the chunk's start) and in the stage (bytes); k or channel of the
     // chunk it starts at; how many of its halves a load moved back to stay inside the row drops.
     struct Piece { int src, dst, lim, gone; bool have; };
     // Patch: row `row` of channel `ci`, image columns ix .. ix + 7 (ix a multiple of 8: never cut at the left).
     auto patch_of = [&](int c) {
-        const int j = c % t.PC8, q = c / t.PC8, row = q % t.PR, ci = q / t.PR, iy = iy0 + row, ix = xa + 8 * j;
+        int j, row;
+        const int q = over(c, t.PC8, t.div_pc, j), ci = over(q, t.PR, t.div_pr, row), iy = iy0 + row, ix = xa + 8 * j;
         Piece p;
         p.have = c < t.patch_pieces && (unsigned)iy < (unsigned)a.Hi && (unsigned)ix < (unsigned)a.Wi;
         p.gone = p.have && !narrow ? max(0, ix + 8 - a.Wi) : 0;
@@ -78,7 +88,8 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         return p;
     };
     auto weight_of = [&](int c) {
-        const int j = c % t.wpieces, co = c / t.wpieces;
+        int j;
+        const int co = over(c, t.wpieces, t.div_wp, j);
         Piece p;
         p.have = c < t.weight_pieces && 8 * j < t.kc;
         p.src = p.have ? min(co0 + co, a.Cout - 1) * CRS + 8 * j : 0;      // rows past Cout repeat the last one: their results are never stored
@@ -87,41 +98,79 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         p.gone = 0;
         return p;
     };
-    auto patch_load = [&](const Piece &p, int c0) {       // zeros where the piece or its channel does not exist
+    // A load and what it turns into (`patch_fixed`, `weight_fixed`, once it is used) are apart, and no load stands behind a condition: where
+    // the two sides of one meet the compiler waits for it, and the pieces of a chunk came one trip to memory after the other.
+    // What does not exist -- outside the image, past the chunk or past Cin -- reads the tensor's first piece.
+    auto patch_in = [&](const Piece &p, int c0) { return p.have && c0 + p.lim < a.Cin; };
+    auto weight_left = [&](const Piece &p, int c0) { return p.have ? min(t.kc, CRS - c0 * taps) - p.lim : 0; };
+    auto patch_load = [&](const Piece &p, int c0) {
         u32x4 v = zero4;
-        if (!p.have || c0 + p.lim >= a.Cin) return v;
-        const half_t *s = x + (long)c0 * HiWi + p.src;
         if (narrow) {
             half8v h = as_half8(v);
+            if (patch_in(p, c0)) {
+                const half_t *s = x + (long)c0 * HiWi + p.src;
 #pragma unroll
-            for (int e = 0; e < 8; e++) if (e < a.Wi) h[e] = s[e];      // ix is 0
+                for (int e = 0; e < 8; e++) if (e < a.Wi) h[e] = s[e];      // ix is 0
+            }
             return __builtin_bit_cast(u32x4, h);
         }
+        const half_t *s = patch_in(p, c0) ? x + (long)c0 * HiWi + p.src : x;
         __builtin_memcpy(&v, s, 16);
-        return p.gone ? shifted(v, p.gone) : v;
+        return v;
     };
-    auto weight_load = [&](const Piece &p, int c0) {      // zeros past the chunk and past Cin
-        const int left = min(t.kc, CRS - c0 * taps) - p.lim;
+    auto patch_fixed = [&](u32x4 v, const Piece &p, int c0) {
+        if (narrow) return v;
+        if (__any(p.gone)) v = shifted(v, p.gone);
+        return patch_in(p, c0) ? v : zero4;
+    };
+    auto weight_load = [&](const Piece &p, int c0) {
+        const int left = weight_left(p, c0);
         u32x4 v = zero4;
-        if (!p.have || left <= 0) return v;
-        const half_t *s = a.w + c0 * taps + p.src;
         if (short_w) {
             half8v h = as_half8(v);
+            if (left > 0) {
+                const half_t *s = a.w + c0 * taps + p.src;
 #pragma unroll
-            for (int e = 0; e < 8; e++) if (e < left) h[e] = s[e];
+                for (int e = 0; e < 8; e++) if (e < left) h[e] = s[e];
+            }
             return __builtin_bit_cast(u32x4, h);
         }
-        __builtin_memcpy(&v, s - weight_back(left), 16);
-        return left < 8 ? shifted(v, weight_back(left)) : v;
+        const half_t *s = left > 0 ? a.w + c0 * taps + p.src - weight_back(left) : a.w;
+        __builtin_memcpy(&v, s, 16);
+        return v;
+    };
+    auto weight_fixed = [&](u32x4 v, const Piece &p, int c0) {
+        if (short_w) return v;
+        const int left = weight_left(p, c0);
+        if (__any(left < 8)) v = left <= 0 ? zero4 : shifted(v, weight_back(left));
+        return v;
     };
     auto patch_lds = [&](int buf, int dst) { return reinterpret_cast<u32x4 *>(smem + t.patch_off + buf * t.stage_bytes + dst); };
     auto weight_lds = [&](int buf, int dst) { return reinterpret_cast<u32x4 *>(smem + t.weight_off + buf * t.stage_bytes + dst); };
 
+    // The bias is asked for at once, of a single chunk here, of several behind their loop: a load behind a store is waited for
+    // together with the store's acknowledgement (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: a store of 20 300 clocks, 5200 so).
+    const int cl = 4 * (lane >> 5);                       // acc[i][4 g + e] of a lane is channel co0 + 32 i + 8 g + cl + e
+    const bool all = co0 + CO <= a.Cout;                  // uniform
+    half4v bias[TCO][4];
+    auto load_bias = [&]() {
+        const half_t *from = a.bias ? a.bias : a.w;       // (Cout halves there too)
+        if (all) {
+#pragma unroll
+            for (int i = 0; i < TCO; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) __builtin_memcpy(&bias[i][g], from + co0 + cl + 32 * i + 8 * g, 8);
+        } else {
+#pragma unroll
+            for (int i = 0; i < TCO; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) bias[i][g][e] = from[min(co0 + 32 * i + 8 * g + cl + e, a.Cout - 1)];
+        }
+    };
+    if (CHUNKS == 1) load_bias();
     float16v acc[TCO];
-#pragma unroll
-    for (int i = 0; i < TCO; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
 
     // A single chunk of any size goes to LDS in batches; of several, every thread carries the same few pieces of each.
     Piece pp[PP], wp[WP];
@@ -144,28 +193,58 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
 #pragma unroll
         for (int i = 0; i < PP; i++) __builtin_memcpy(&v.p[i], xbase + (uint32_t)pp[i].src * 2u, 16);
     };
-    // Pieces outside the image or past kc were zeroed in both stages at the start and stay so.
-    auto put = [&](Set &v, int buf, bool raw) {
+    // Chunk ch goes to LDS.  Pieces outside the image or past kc were zeroed in both stages at the start and stay so.
+    auto put = [&](Set &v, int ch) {
+        const int buf = ch & 1, c0 = ch * t.CC;
+        const bool whole = ch < nwhole;                  // uniform
 #pragma unroll
-        for (int i = 0; i < WP; i++) if (wp[i].have) *weight_lds(buf, wp[i].dst) = v.w[i];
+        for (int i = 0; i < WP; i++)
+            if (wp[i].have) *weight_lds(buf, wp[i].dst) = whole ? v.w[i] : weight_fixed(v.w[i], wp[i], c0);
 #pragma unroll
         for (int i = 0; i < PP; i++)
             if (pp[i].have) {
-                if (raw && __any(pp[i].gone)) v.p[i] = shifted(v.p[i], pp[i].gone);
+                if (whole) {
+                    if (__any(pp[i].gone)) v.p[i] = shifted(v.p[i], pp[i].gone);
+                } else v.p[i] = patch_fixed(v.p[i], pp[i], c0);
                 *patch_lds(buf, pp[i].dst) = v.p[i];
             }
     };
-    if (t.nchunk == 1) {
-        for (int c = tid, d = tid; c < t.weight_pieces || d < t.patch_pieces; c += NT * WP, d += NT * PP) {
+    const bool one = CHUNKS == 1 || (CHUNKS == 0 && t.nchunk == 1);
+    if (one) {
+        // In batches of a few pieces a thread, each one trip to memory.  The pieces that the weight rows' ends cut are cut alike.
+        const int wgone = weight_back(t.kc % 8 ? t.kc % 8 : 8);
+        auto stage = [&](auto P_, auto W_) __attribute__((always_inline)) {
+            constexpr int P1 = decltype(P_)::value, W1 = decltype(W_)::value;
+            for (int d0 = 0, c0 = 0; d0 < t.patch_pieces || c0 < t.weight_pieces; d0 += NT * P1, c0 += NT * W1) {
+                Piece pq[P1], wq[W1];
+                u32x4 pv[P1], wv[W1];
+                if (d0 < t.patch_pieces)                  // uniform, as all four
 #pragma unroll
-            for (int i = 0; i < PP; i++) { pp[i] = patch_of(d + i * NT); set0.p[i] = patch_load(pp[i], 0); }
+                    for (int i = 0; i < P1; i++) { pq[i] = patch_of(d0 + tid + i * NT); pv[i] = patch_load(pq[i], 0); }
+                if (c0 < t.weight_pieces)
 #pragma unroll
-            for (int i = 0; i < WP; i++) { wp[i] = weight_of(c + i * NT); set0.w[i] = weight_load(wp[i], 0); }
+                    for (int i = 0; i < W1; i++) { wq[i] = weight_of(c0 + tid + i * NT); wv[i] = weight_load(wq[i], 0); }
+                if (d0 < t.patch_pieces)
 #pragma unroll
-            for (int i = 0; i < PP; i++) if (d + i * NT < t.patch_pieces) *patch_lds(0, pp[i].dst) = set0.p[i];
+                    for (int i = 0; i < P1; i++) {
+                        pv[i] = patch_fixed(pv[i], pq[i], 0);
+                        if (d0 + tid + i * NT < t.patch_pieces) *patch_lds(0, pq[i].dst) = pv[i];
+                    }
+                if (c0 < t.weight_pieces)
 #pragma unroll
-            for (int i = 0; i < WP; i++) if (c + i * NT < t.weight_pieces) *weight_lds(0, wp[i].dst) = set0.w[i];
-        }
+                    for (int i = 0; i < W1; i++) {
+                        if (!short_w) {
+                            const u32x4 cut = shifted(wv[i], wgone);
+                            wv[i] = wq[i].lim + 8 > t.kc ? cut : wv[i];
+                            wv[i] = wq[i].have ? wv[i] : zero4;
+                        }
+                        if (c0 + tid + i * NT < t.weight_pieces) *weight_lds(0, wq[i].dst) = wv[i];
+                    }
+            }
+        };
+        using std::integral_constant;
+        if (t.patch_pieces <= NT && t.weight_pieces <= 2 * NT) stage(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+        else stage(integral_constant<int, 4>{}, integral_constant<int, (TCO > 2 ? 7 : 5)>{});
     } else {
 #pragma unroll
         for (int i = 0; i < WP; i++) wp[i] = weight_of(tid + i * NT);
@@ -173,7 +252,7 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         for (int i = 0; i < PP; i++) pp[i] = patch_of(tid + i * NT);
         load(set0, 0);
         if (TWO) load(set1, 1);
-        put(set0, 0, false);
+        put(set0, 0);
 #pragma unroll
         for (int i = 0; i < WP; i++)
             if (!wp[i].have && tid + i * NT < t.weight_pieces) { *weight_lds(0, wp[i].dst) = zero4; *weight_lds(1, wp[i].dst) = zero4; }
@@ -184,8 +263,14 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
     if (tid < t.nbuf) *patch_lds(tid, zero_at * 2) = zero4;
     __syncthreads();
 
+#pragma unroll
+    for (int i = 0; i < TCO; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+
     // this lane's pixel: its origin in the patch
-    const int px = pw * 32 + (lane & 31), ly = px / t.TW, lx = px - ly * t.TW, h8 = (lane >> 5) * 8;
+    int lx;
+    const int px = pw * 32 + (lane & 31), ly = over(px, t.TW, t.div_tw, lx), h8 = (lane >> 5) * 8;
     const int origin = ly * a.sy * t.PCL + lx * a.sx + (ix0 - xa);
     const int whole = t.kc / 16;                         // steps with sixteen k of the chunk
     auto compute = [&](int buf) {
@@ -226,11 +311,14 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         if (fast) load_whole(now, ch + AHEAD);
         else if (ch + AHEAD < t.nchunk) load(now, ch + AHEAD);
         compute(ch & 1);
-        if (ch + 1 < t.nchunk) put(TWO ? next : now, (ch + 1) & 1, ch + 1 >= AHEAD && ch + 1 < nwhole);
+        if (ch + 1 < t.nchunk) put(TWO ? next : now, ch + 1);
         __syncthreads();
     };
     int ch = 0;
-    if constexpr (TWO) {
+    if (one) {
+        compute(0);
+        if constexpr (KG > 1) __syncthreads();            // (below, the groups' sums lie over the operands)
+    } else if constexpr (TWO) {
         for (; ch + 3 < nwhole; ch += 2) {
             turn(set0, set1, ch, true);
             turn(set1, set0, ch + 1, true);
@@ -261,32 +349,44 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][r] += part[((g * TCO + i) * 16 + r) * (PW * 64) + pw * 64 + lane];
     }
-    // acc[i][4 g + e] of a lane: channel co0 + 32 i + 8 g + 4 (lane / 32) + e of pixel `px`: 32 lanes store neighbours of a row
+    if (CHUNKS != 1) load_bias();
     const int oy = oy0 + ly, ox = ox0 + lx;
-    if (oy >= a.OH || ox >= a.OW || ly >= t.TH) return;
     const int plane = a.OH * a.OW;                        // Cout planes of an image fit 31 bits
     char *out = reinterpret_cast<char *>(reinterpret_cast<half_t *>(a.out) + (long)blockIdx.z * a.Cout * plane);
-    const int cl = 4 * (lane >> 5);
-    uint32_t at = (uint32_t)((co0 + cl) * plane + oy * a.OW + ox) * 2u;
     const uint32_t step = (uint32_t)plane * 2u;
-    const bool all = co0 + CO <= a.Cout;                  // uniform
+    auto rounded = [&](float v0, float v1) {
+        half2v v = {(half_t)v0, (half_t)v1};
+        if (a.relu) v = __builtin_elementwise_max(v, half2v{(half_t)0.0f, (half_t)0.0f});
+        return __builtin_bit_cast(uint32_t, v);
+    };
 #pragma unroll
     for (int i = 0; i < TCO; i++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int co = co0 + 32 * i + 8 * g + cl;
-            float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (a.bias) {
+        for (int r = 0; r < 16; r++) acc[i][r] += a.bias ? (float)bias[i][r / 4][r % 4] : 0.0f;
+    // Four lanes, four neighbouring pixels of a row, hold four channels each: they exchange, so that a lane stores four pixels of one
+    // channel, eight bytes at any address (by pixel where the row ends between them).
+    const int q = lane & 3, left = a.OW - (ox - q);       // pixels of the row from the four's first on
+    const bool odd = lane & 1, upper = lane & 2, row_in = oy < a.OH && ly < t.TH && left > 0;
+    uint32_t at = (uint32_t)((co0 + cl + q) * plane + oy * a.OW + ox - q) * 2u;
+    const bool cut = __any(row_in && left < 4);
 #pragma unroll
-                for (int e = 0; e < 4; e++) b[e] = (float)a.bias[min(co + e, a.Cout - 1)];
-            }
+    for (int i = 0; i < TCO; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                half_t v = (half_t)(acc[i][4 * g + e] + b[e]);
-                if (a.relu) v = (half_t)fmaxf((float)v, 0.0f);
-                if (all || co + e < a.Cout) *reinterpret_cast<half_t *>(out + at + e * step) = v;
+        for (int g = 0; g < 4; g++, at += 8 * step) {
+            // even lanes keep channels 0 and 2 of their own and the next pixel, odd ones 1 and 3 of the one before and their own
+            const uint32_t p01 = rounded(acc[i][4 * g], acc[i][4 * g + 1]), p23 = rounded(acc[i][4 * g + 2], acc[i][4 * g + 3]);
+            const uint32_t n01 = __builtin_amdgcn_update_dpp(0, p01, 0xB1, 0xF, 0xF, true), n23 = __builtin_amdgcn_update_dpp(0, p23, 0xB1, 0xF, 0xF, true);
+            const uint32_t a01 = odd ? pack_hi(n01, p01) : pack_lo(p01, n01), a23 = odd ? pack_hi(n23, p23) : pack_lo(p23, n23);
+            const uint32_t give = upper ? a01 : a23, keep = upper ? a23 : a01, got = __builtin_amdgcn_update_dpp(0, give, 0x4E, 0xF, 0xF, true);
+            const u32x2 v = {upper ? got : keep, upper ? keep : got};
+            if (row_in && (all || co0 + 32 * i + 8 * g + cl + q < a.Cout)) {
+                if (left >= 4) __builtin_memcpy(out + at, &v, 8);
+                else if (cut) {
+                    const half4v h = __builtin_bit_cast(half4v, v);
+#pragma unroll
+                    for (int e = 0; e < 3; e++) if (e < left) *reinterpret_cast<half_t *>(out + at + 2 * e) = h[e];
+                }
             }
-            at += 8 * step;
         }
 }
 
@@ -295,14 +395,16 @@ int launch(const TileConv &t, hipStream_t st) {
     constexpr int parts = (KG - 1) * TCO * 16 * PW * 64 * 4;
     const int lds = (int)std::max<int64_t>(t.patch_off + (int64_t)t.nbuf * t.stage_bytes, parts);
     const dim3 grid((unsigned)(t.tiles_x * t.tiles_y), (unsigned)ceil_div(t.a.Cout, 32 * TCO), (unsigned)t.a.N);
-    hipLaunchKernelGGL((conv_tile_kernel<PW, KG, TCO>), grid, dim3(PW * KG * 64), lds, st, t);
+    if (t.a.Wi < 8 || weights_by_element(t.kc, t.a.Cin * t.a.KH * t.a.KW)) hipLaunchKernelGGL((conv_tile_kernel<PW, KG, TCO, 0>), grid, dim3(PW * KG * 64), lds, st, t);
+    else if (t.nchunk == 1) hipLaunchKernelGGL((conv_tile_kernel<PW, KG, TCO, 1>), grid, dim3(PW * KG * 64), lds, st, t);
+    else hipLaunchKernelGGL((conv_tile_kernel<PW, KG, TCO, 2>), grid, dim3(PW * KG * 64), lds, st, t);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
 
 template <typename F>
 int with_shape(const Shape &s, F f) {
 #define ONE(P, K, T) if (s.pw == P && s.kg == K && s.tco == T) return f(std::integral_constant<int, P>{}, std::integral_constant<int, K>{}, std::integral_constant<int, T>{});
-    ONE(8, 1, 1) ONE(8, 1, 2) ONE(8, 1, 3) ONE(8, 1, 4) ONE(4, 1, 1) ONE(4, 1, 2) ONE(4, 1, 3) ONE(4, 1, 5) ONE(4, 2, 1) ONE(4, 2, 2) ONE(4, 2, 3) ONE(4, 2, 4) ONE(2, 4, 1) ONE(2, 4, 2) ONE(2, 4, 4) ONE(2, 2, 1) ONE(2, 2, 2)
+    ONE(8, 1, 1) ONE(8, 1, 2) ONE(8, 1, 3) ONE(8, 1, 4) ONE(8, 1, 5) ONE(4, 1, 1) ONE(4, 1, 2) ONE(4, 1, 3) ONE(4, 1, 5) ONE(4, 2, 1) ONE(4, 2, 2) ONE(4, 2, 3) ONE(4, 2, 4) ONE(2, 4, 1) ONE(2, 4, 2) ONE(2, 4, 4) ONE(2, 2, 1) ONE(2, 2, 2)
 #undef ONE
     return MI_DECLINE_EXTENT;
 }
@@ -328,7 +430,7 @@ double mi_conv_tile_us(const ConvArgs &a) { return choice_of(a).us; }
 int mi_conv_tile(const ConvArgs &a, hipStream_t st) {
     const Choice &e = choice_of(a);
     if (e.us >= 1e30) return MI_DECLINE_EXTENT;
-    const TileConv t{e.t, a};
+    const TileConv t{e.t, a, recip_of(e.t.tiles_x), recip_of(a.KH * a.KW), recip_of(a.KW), recip_of(e.t.TW), recip_of(e.t.PC8), recip_of(e.t.PR), recip_of(e.t.wpieces)};
     return with_shape(e.s, [&](auto P, auto K, auto T) { return launch<P, K, T>(t, st); });
 }
 
@@ -336,7 +438,8 @@ int mi_conv_tile_init() {
     int bad = 0;
     for (const Shape &s : SHAPES)
         bad |= with_shape(s, [&](auto P, auto K, auto T) {
-            return hipFuncSetAttribute(reinterpret_cast<const void *>(conv_tile_kernel<P, K, T>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX) == hipSuccess ? 0 : 1;
+            auto up = [](auto kern) { return hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX) == hipSuccess ? 0 : 1; };
+            return up(conv_tile_kernel<P, K, T, 0>) | up(conv_tile_kernel<P, K, T, 1>) | up(conv_tile_kernel<P, K, T, 2>);
         });
     return bad;
 }

@@ -86,14 +86,14 @@ inline bool choose_chunk(TilePlan &t, const ConvShape &a, int co, int nt, int pa
 }
 
 struct Shape { int pw, kg, tco; };
-constexpr Shape SHAPES[] = {{8, 1, 1}, {8, 1, 2}, {8, 1, 3}, {8, 1, 4}, {4, 1, 1}, {4, 1, 2}, {4, 1, 3}, {4, 1, 5}, {4, 2, 1}, {4, 2, 2}, {4, 2, 3}, {4, 2, 4}, {2, 4, 1}, {2, 4, 2}, {2, 4, 4}, {2, 2, 1}, {2, 2, 2}};
+constexpr Shape SHAPES[] = {{8, 1, 1}, {8, 1, 2}, {8, 1, 3}, {8, 1, 4}, {8, 1, 5}, {4, 1, 1}, {4, 1, 2}, {4, 1, 3}, {4, 1, 5}, {4, 2, 1}, {4, 2, 2}, {4, 2, 3}, {4, 2, 4}, {2, 4, 1}, {2, 4, 2}, {2, 4, 4}, {2, 2, 1}, {2, 2, 2}};
 
 
-// The workgroup shape with the lowest estimate (us), or false where no chunk fits.  Fitted to 24 convolutions in 17 shapes each
-// (1 x 1 to 7 x 7, strides 1, 2 and 4, 3 to 384 channels, 300 to 65 536 pixels): half of the estimates lie within 20 %.  On 60 further
-// convolutions the choice between one launch and staging that this estimate decides is 1.8 % above the faster of the two on average
-// (one launch everywhere 22 %, staging everywhere 3.2 %), at most 19 % (2 x 96 x 73 x 204 -> 96, 3 x 3: 30.8 us staged, 25.8 in
-// one launch).  A chunk costs its trip to memory and its pieces, a step of a wave its eight gathers and its weight fragments.
+// The workgroup shape with the lowest estimate (us), or false where no chunk fits.  Fitted to 130 convolutions in all 18 shapes
+// (2 x 2 to 7 x 7, strides 1, 2 and 4, 3 to 384 channels, 16 to 200 000 pixels): the choice is 3 % above the best shape on average.
+// With the staged routes' estimate (route_of) the choice between one launch and staging is 3.4 % above the best of all of them,
+// 32 % at worst (972 x 23 x 3 -> 96, 2 x 2: 7.4 us, 5.6 in another shape); one launch is the faster in 94 of the 130.
+// A chunk costs its trip to memory and its pieces, a step of a wave its eight gathers and its weight fragments; large outputs 0.1 us a megabyte.
 inline bool choose(const ConvShape &a, int cus, TilePlan &t, Shape &best, double &best_us) {
     if ((int64_t)a.Cout * a.Cin * a.KH * a.KW > INT32_MAX / 2) return false;      // 32-bit offsets
     best_us = 1e30;
@@ -102,10 +102,11 @@ inline bool choose(const ConvShape &a, int cus, TilePlan &t, Shape &best, double
         TilePlan c = {};
         choose_rectangle(c, a, 32 * s.pw);
         if (!choose_chunk(c, a, 32 * s.tco, s.pw * s.kg * 64, (s.kg - 1) * s.tco * 16 * s.pw * 64 * 4)) continue;
+        if (s.kg > 1 && c.nchunk * c.ksteps < 2 * s.kg) continue;      // (too few steps to split: one chain of sums, as the GEMMs have)
         const int64_t wgs = (int64_t)c.tiles_x * c.tiles_y * ceil_div(a.Cout, 32 * s.tco) * a.N;
         const double rounds = (double)ceil_div(wgs, cus), steps = (double)c.nchunk * c.ksteps * s.pw / 4.0;
-        const double us = 3.2 + rounds * (2.6 + 0.19 * s.tco * s.pw + c.nchunk * (1.1 + 0.36e-3 * (c.patch_pieces + c.weight_pieces)) +
-                                          steps * (0.0113 + 0.0137 * s.tco));
+        const double us = 4.9 + 0.1e-6 * 2.0 * (double)a.N * a.Cout * a.OH * a.OW + rounds * (0.3 + 0.147 * s.tco * s.pw + c.nchunk * (0.836 + 0.417e-3 * (c.patch_pieces + c.weight_pieces)) +
+                                          steps * (0.027 + 0.0096 * s.tco));
         if (us < best_us) { best_us = us; best = s; pick = c; }
     }
     if (best_us >= 1e30) return false;

@@ -74,3 +74,23 @@ def test_operands_off_sixteen_bytes(ctx, Cin, H, W, Cout, k, s, p, off):
     torch.cuda.synchronize()
     assert_parity(to_host(out), want, what=f"conv {Cin},{H},{W}->{Cout} k{k} off {off}")
     assert bool(torch.isnan(flat[:off]).all()) and bool(torch.isnan(flat[off + want.size:]).all())
+
+
+@pytest.mark.parametrize("Cin", [3, 24])
+@pytest.mark.parametrize("OW", [1, 2, 3, 5, 6, 7, 18, 37])
+@pytest.mark.parametrize("Cout", [30, 33, 64])
+def test_rows_that_end_between_four_pixels(ctx, Cin, OW, Cout):
+    """Lanes exchange four pixels by four channels and store eight bytes: rows that end inside, channels that end inside, with a bias at an
+    odd address and without, one chunk and several, nothing written past a row (the next one's first pixels follow it)."""
+    import torch
+    import juliavision_amd as jv
+    H = 9
+    x, w, b = oracle.randn_f16((2, Cin, H, OW), 1), oracle.randn_f16((Cout, Cin, 3, 3), 2, 0, 0.1), oracle.randn_f16((Cout + 1,), 3)
+    held = torch.from_numpy(b).cuda()
+    for bias in (held[1:], None):
+        for act in ("none", "relu"):
+            out = torch.full((2, Cout, H, OW), float("nan"), dtype=torch.float16, device="cuda")
+            ctx.ws.reset()
+            jv.convolution_(ctx, out, torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), bias, (1, 1), (1, 1), (1, 1), 1, act=act)
+            want = oracle.conv2d_f16(x, w, None if bias is None else b[1:], (1, 1), (1, 1), (1, 1), 1, act == "relu")
+            assert_parity(to_host(out), want, what=f"Cin{Cin} OW{OW} Cout{Cout} {act}")
