@@ -291,13 +291,6 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
         if (coop) help_store();
         return;
     }
-    // (a launch without the statistics wave and with a folded norm: combine in the prologue, as the other kernels do)
-    if (blockDim.x < 384 && p.lnf_stats) {                          // no statistics wave: in front of the K loop
-        LnfLoader<BM, BN, 256, 16> lnf;
-        lnf.request(p, m0, n0, bz, tid);
-        lnf.combine(p, ln_slot, m0, tid);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
 
     // fragment read offsets inside a stage (bytes): rows of A, and this wave's columns of B in either layout
     const int frow = lane & 31, fhi = lane >> 5;

@@ -119,124 +119,93 @@ inline void set_tiles(GemmArgs &a, int bm, int bn) {
     a.div_last = recip_of(last ? last : a.group_m);
 }
 
-// What the store of a folded norm needs, fetched while the first operand tiles are on their way and parked in `slot`
-// (LDS past everything else the kernel keeps there: BM float2 (r, r mu), then BN column sums, then BN biases).
-//
-// A row's mean and reciprocal standard deviation over its K elements come from the per-segment statistics a producer
-// left (stats[seg][row] = (sum, squares about the segment's own mean)).  LPR lanes share a row, each with every LPR-th
-// segment, many loads in flight at a time (a lane that walked all segments one dependent load after the other held
-// the whole workgroup at its first barrier for 10 us).  One pass: the squares between the segments are taken about the
-// first segment's mean, which lies within a segment mean's spread of the row mean, so the final subtraction cancels
-// nothing that matters -- sum(x^2) - n mean^2 about zero would.  r = 1 / sqrt(var + eps), rmu = r * mean.
-//
-// The loads and the arithmetic are apart: a kernel requests its share of the statistics behind its first operand tiles,
-// carries it in registers and combines it late in its K loop, between products.  Combined in the prologue, the trip and
-// some sixty dependent instructions per row stood between the launch and its first MFMA: 1.3 to 1.5 us a launch at
-// K = 384, 1.6 to 2.8 at K = 1024 to 1280.  NV loads a lane cover LPR NV segments (K <= 32 LPR NV); beyond that
-// `combine` fetches the rest itself.
-template <int BM, int BN, int NT, int NV>
-struct LnfLoader {
-    static constexpr int LPR = NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1;
-    static_assert(NT >= BM && (BM * LPR) % 64 == 0, "whole waves work on the rows");
-    static constexpr int NC = (BN / 2 + NT - 1) / NT;
-    float2v v[NV];
-    float4v col[NC];
+// A folded norm's row statistics, r (acc - mu colsum) + biasp: a row's mean and reciprocal standard deviation over its K elements
+// come from the per-segment statistics a producer left (stats[seg][row] = (sum, squares about the segment's own mean)).  One
+// pass: the squares between the segments are taken about the first segment's mean, which lies within a segment mean's
+// spread of the row mean, so the final subtraction cancels nothing that matters -- sum(x^2) - n mean^2 about zero would.
+// r = 1 / sqrt(var + eps), rmu = r * mean.
 
-    __device__ __forceinline__ static const float2v *row_of(const GemmArgs &p, int m0, int row) {
-        return reinterpret_cast<const float2v *>(p.lnf_stats) + min(m0 + row, p.M - 1);
+// Four of colsum's or biasp's floats from n on; past the edge the last ones again (such launches have whole quads of columns and
+// whole 64-deep tiles of K).
+__device__ __forceinline__ float4v lnf_columns(const GemmArgs &p, const float *vec, int n, long bz) {
+    return *reinterpret_cast<const float4v *>(vec + bz * p.lnf_svec + min(n, p.N - 4));
+}
+
+// In the matrix waves of a kernel whose K tiles are two segments deep and pass through registers: a lane's rows are those of its
+// accumulators, its half of the wave takes every other segment, a load and some eight vector instructions a tile and row, all
+// beside the products; what the store needs is in registers under the last tile.  (Requested in the prologue, ten conditional
+// loads a lane with a wait where each condition ended, combined in one go ahead of the last tile by four lanes a row and handed
+// over through LDS, the norm spilled registers and cost 1370 x 384 -> 1152 2 400 clocks, 11 080 against 8 700 without it;
+// now 1 900, of which 1 000 are instructions beside the loop's.  Launch to first product 2 220 -> 2 080, store 2 200 -> 1 790.
+// ViT-S of 1370 tokens, 24 such launches: 521 -> 506 us.)
+template <int TM>
+struct LnfRows {
+    const float2v *seg[TM];
+    float ref[TM], total[TM], within[TM], between[TM];
+    float2v v[2][TM];
+    // mw: the wave's first row
+    __device__ __forceinline__ LnfRows(const GemmArgs &p, int mw, int lane) {
+#pragma unroll
+        for (int j = 0; j < TM; j++) {
+            seg[j] = reinterpret_cast<const float2v *>(p.lnf_stats) + (long)(lane >> 5) * p.M + min(mw + 32 * j + (lane & 31), p.M - 1);
+            total[j] = within[j] = between[j] = 0.0f;
+        }
     }
-    __device__ __forceinline__ void request(const GemmArgs &p, int m0, int n0, long bz, int tid) {
-        if (!p.lnf_stats) return;
-        if (tid < BM * LPR) {
-            const float2v *seg = row_of(p, m0, tid / LPR);
-            const int q = tid % LPR;
+    __device__ __forceinline__ void request(const GemmArgs &p, int set, int kt) {
 #pragma unroll
-            for (int u = 0; u < NV; u++) {
-                const float2v z = {0.0f, 0.0f};
-                v[u] = q + u * LPR < p.lnf_nseg ? seg[(long)(q + u * LPR) * p.M] : z;
-            }
-        }
-        // the tile's columns of colsum and biasp
+        for (int j = 0; j < TM; j++) v[set][j] = seg[j][(long)(2 * kt) * p.M];
+    }
+    template <bool FIRST = false>
+    __device__ __forceinline__ void take(int set) {
 #pragma unroll
-        for (int i = 0; i < NC; i++) {
-            const int t = tid + i * NT, which = t / (BN / 4), n = n0 + (t % (BN / 4)) * 4;
-            const float4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-            col[i] = z;
-            if (t < BN / 2) {
-                const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
-                if (n + 3 < p.N) col[i] = *reinterpret_cast<const float4v *>(src + n);
-                else for (int e = 0; e < 4; e++) if (n + e < p.N) col[i][e] = src[n + e];
+        for (int j = 0; j < TM; j++) {
+            const float2v s = v[set][j];
+            if constexpr (FIRST) {
+                float other = s[0];
+                ref[j] = s[0];
+                swap_rows32(ref[j], other);                       // the first segment's sum, in both halves of the wave
+                ref[j] *= 1.0f / 32.0f;
             }
+            const float d = fmaf(s[0], 1.0f / 32.0f, -ref[j]);
+            total[j] += s[0];
+            within[j] += s[1];
+            between[j] = fmaf(32.0f * d, d, between[j]);
         }
     }
-    // (r, r mu) per row, colsum, biasp -> slot.  The caller synchronises the workgroup before anybody reads it.
-    __device__ __forceinline__ void combine(const GemmArgs &p, float2v *slot, int m0, int tid) {
-        if (!p.lnf_stats) return;
-        if (tid < BM * LPR) {
-            const int row = tid / LPR, q = tid % LPR;
-            float total = 0.0f, within = 0.0f, between = 0.0f;
-            // the row's first segment mean: lane q = 0 of its quad (or pair) holds it
-            float first = v[0][0];
-            if constexpr (LPR == 4) first = dpp_mov<0x00>(first);          // quad_perm [0,0,0,0]
-            if constexpr (LPR == 2) first = dpp_mov<0xA0>(first);          // quad_perm [0,0,2,2]
-            const float ref = first / (float)min(32, p.K);
-            auto take = [&](const float2v s, int sg) {
-                const int left = p.K - 32 * sg;
-                const float cnt = left >= 32 ? 32.0f : (float)left, inv = left >= 32 ? 1.0f / 32.0f : 1.0f / (float)left;
-                const float d = fmaf(s[0], inv, -ref);
-                total += s[0];
-                within += s[1];
-                between = fmaf(cnt * d, d, between);
-            };
+    __device__ __forceinline__ void finish(const GemmArgs &p, float (&r)[TM], float (&rmu)[TM]) {
+        // (a division by K is one by a reciprocal and its remainder, the root of the variance an estimate and a Newton step: as
+        // exact to within a last bit, and a third of the instructions between the last statistics and the last product)
+        const float k = (float)p.K, ik = __builtin_amdgcn_rcpf(k), inv = fmaf(fmaf(-k, ik, 1.0f), ik, ik);
+        auto both = [](float x) { float y = x; swap_rows32(x, y); return x + y; };
+        auto over_k = [&](float x) { const float t = x * inv; return fmaf(fmaf(-k, t, x), inv, t); };
 #pragma unroll
-            for (int u = 0; u < NV; u++) if (q + u * LPR < p.lnf_nseg) take(v[u], q + u * LPR);
-            if (p.lnf_nseg > NV * LPR) {
-                const float2v *seg = row_of(p, m0, row);
-                for (int s0 = q + NV * LPR; s0 < p.lnf_nseg; s0 += 8 * LPR) {
-                    float2v w[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) w[u] = seg[(long)min(s0 + u * LPR, p.lnf_nseg - 1) * p.M];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) if (s0 + u * LPR < p.lnf_nseg) take(w[u], s0 + u * LPR);
-                }
-            }
-            if constexpr (LPR >= 2) { total += lane_xor<1>(total); within += lane_xor<1>(within); between += lane_xor<1>(between); }
-            if constexpr (LPR >= 4) { total += lane_xor<2>(total); within += lane_xor<2>(within); between += lane_xor<2>(between); }
-            if (q == 0) {
-                const float mu = total / (float)p.K, dm = mu - ref;
-                const float m2 = within + fmaxf(between - (float)p.K * dm * dm, 0.0f);
-                const float r = 1.0f / sqrtf(m2 / (float)p.K + p.lnf_eps);
-                const float2v o = {r, r * mu};
-                slot[row] = o;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NC; i++) {
-            const int t = tid + i * NT, which = t / (BN / 4), c = (t % (BN / 4)) * 4;
-            if (t < BN / 2) *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = col[i];
+        for (int j = 0; j < TM; j++) {
+            const float mu = over_k(both(total[j])), dm = mu - ref[j];
+            const float var = over_k(both(within[j]) + fmaxf(both(between[j]) - k * dm * dm, 0.0f)) + p.lnf_eps;
+            const float e = __builtin_amdgcn_rsqf(var);
+            r[j] = var > 0.0f ? fmaf(0.5f * e, fmaf(-var * e, e, 1.0f), e) : e;      // (fp16 rows: a variance is 0 or far from the smallest floats)
+            rmu[j] = r[j] * mu;
         }
     }
 };
 
-// The same by a wave of its own, beside the K loop of kernels that have a barrier a tile: the matrix waves need (r, r mu) of the
+// By a wave of its own, beside the K loop of kernels whose tiles go straight to LDS: the matrix waves need (r, r mu) of the
 // tile's rows and the tile's columns of colsum and biasp at the store, not before, and in their registers the statistics
 // would cost a second workgroup a CU.  (In the prologue they held every wave at the first barrier: 5 000 clocks at 128 rows,
 // 10 000 at 192, a trip to memory per batch of loads, then forty dependent steps a row.)  Tile kt covers segments 2 kt and
 // 2 kt + 1 (SEGS = 2; a 128-deep tile four): ahead of barrier kt this wave takes in the segments of each of its rows that it
 // requested AHEAD tiles earlier, and the result is in the slot when it arrives at the last barrier, which the matrix waves pass
-// before they store.  Same arithmetic, in the same order per row, as LnfLoader with one lane a row.  LEAD: a barrier comes before
-// tile 0's.
+// before they store.  The slot: (r, r mu) of BM rows, BN column sums, BN biases.  LEAD: a barrier comes before tile 0's.
 template <int BM, int BN, bool LEAD, int SEGS = 2, typename BarrierF>
 __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot, int m0, int n0, long bz, int lane, int nk, BarrierF barrier) {
     constexpr int NR = (BM + 63) / 64, AHEAD = 4;
     static_assert((BM % 64 == 0 || BM == 32) && NR * SEGS * AHEAD <= 63, "whole rows per lane; vmcnt is a 6-bit counter");
-    for (int t = lane; t < BN / 2; t += 64) {
-        const int which = t / (BN / 4), c = (t % (BN / 4)) * 4, n = n0 + c;
-        const float *src = (which == 0 ? p.lnf_colsum : p.lnf_biasp) + bz * p.lnf_svec;
-        float4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (n + 3 < p.N) v = *reinterpret_cast<const float4v *>(src + n);
-        else for (int e = 0; e < 4; e++) if (n + e < p.N) v[e] = src[n + e];
-        *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + which * BN + c) = v;
+    constexpr int NC = (BN / 2 + 63) / 64;
+    float4v col[NC];
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+        const int t = min(lane + 64 * i, BN / 2 - 1);
+        col[i] = lnf_columns(p, t < BN / 4 ? p.lnf_colsum : p.lnf_biasp, n0 + (t % (BN / 4)) * 4, bz);
     }
     const float2v *seg[NR];
 #pragma unroll
@@ -272,6 +241,11 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
     // tiles 0 .. AHEAD - 1 are requested at once; tile kt + AHEAD right after tile kt is taken in
     static_for<AHEAD>([&](auto S) { if (decltype(S)::value < nk) fetch(S, decltype(S)::value); });
     if (LEAD) barrier();
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+        const int t = lane + 64 * i;
+        if (t < BN / 2) *reinterpret_cast<float4v *>(reinterpret_cast<float *>(slot + BM) + t / (BN / 4) * BN + (t % (BN / 4)) * 4) = col[i];
+    }
     for (int kt0 = 0; kt0 < nk; kt0 += AHEAD) {
         static_for<AHEAD>([&](auto S) {
             const int kt = kt0 + decltype(S)::value;
@@ -312,20 +286,29 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
 template <int TN, int WTN>
 __device__ __forceinline__ void load_col_bias(const GemmArgs &p, half4v (&cb)[TN][4], int n0, int wn, int lane, long bz) {
     const half4v z = {(half_t)0.0f, (half_t)0.0f, (half_t)0.0f, (half_t)0.0f};
-    const bool on = p.bias_mode == MI_BIAS_COL;
-    const half_t *bias = on ? p.bias + bz * p.sBias : nullptr;
-    const bool vec = (reinterpret_cast<uintptr_t>(bias) & 7) == 0;
+    const int nl = n0 + wn * WTN + 4 * (lane >> 5), last = p.N - 1;
+    // (uniform choices, and columns past the edge re-read the last ones: no load behind a condition of its lane)
+    if (p.bias_mode != MI_BIAS_COL) {
 #pragma unroll
-    for (int i = 0; i < TN; i++)
+        for (int i = 0; i < TN; i++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int n = n0 + wn * WTN + 32 * i + 8 * g + 4 * (lane >> 5);
-            cb[i][g] = z;
-            if (on) {
-                if (n + 3 < p.N && vec) cb[i][g] = *reinterpret_cast<const half4v *>(bias + n);
-                else for (int e = 0; e < 4; e++) if (n + e < p.N) cb[i][g][e] = bias[n + e];
-            }
-        }
+            for (int g = 0; g < 4; g++) cb[i][g] = z;
+        return;
+    }
+    const half_t *bias = p.bias + bz * p.sBias;
+    if ((reinterpret_cast<uintptr_t>(bias) & 7) == 0 && p.N % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) cb[i][g] = *reinterpret_cast<const half4v *>(bias + min(nl + 32 * i + 8 * g, p.N - 4));
+    } else {
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) cb[i][g][e] = bias[min(nl + 32 * i + 8 * g + e, last)];
+    }
 }
 
 // What the store of a folded layer norm carries (by value, so that it stays in registers): (r, r mu) of the lane's rows
@@ -336,10 +319,33 @@ struct LnFold {
     float r[TM] = {}, rmu[TM] = {};
     const float *col = nullptr;
     int bn = 0;
+    // columns 32 i + 8 g + 4 (lane / 32) .. +3 of the wave's sub-tile, which starts at column `wcol` of the tile
+    __device__ __forceinline__ float4v colsum(int i, int g, int wcol, int hl) const { return *reinterpret_cast<const float4v *>(col + wcol + 32 * i + 8 * g + 4 * hl); }
+    __device__ __forceinline__ float4v biasp(int i, int g, int wcol, int hl) const { return *reinterpret_cast<const float4v *>(col + bn + wcol + 32 * i + 8 * g + 4 * hl); }
 };
-template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+// The same with the columns in registers, fetched ahead of the last tile like the column bias.
+template <int TM, int TN>
+struct LnFoldRegs {
+    static constexpr bool on = true;
+    float r[TM], rmu[TM];
+    float4v c[TN][4], b[TN][4];
+    // nw: the wave's first column
+    __device__ __forceinline__ void load(const GemmArgs &p, int nw, int lane, long bz) {
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int n = nw + 32 * i + 8 * g + 4 * (lane >> 5);
+                c[i][g] = lnf_columns(p, p.lnf_colsum, n, bz);
+                b[i][g] = lnf_columns(p, p.lnf_biasp, n, bz);
+            }
+    }
+    __device__ __forceinline__ float4v colsum(int i, int g, int, int) const { return c[i][g]; }
+    __device__ __forceinline__ float4v biasp(int i, int g, int, int) const { return b[i][g]; }
+};
+template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES, typename LN>
 __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                               int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}) {
+                                               int wave, int lane, long bz, const LN &ln) {
     const int frow = lane & 31;
     const half_t *bias = p.bias ? p.bias + bz * p.sBias : nullptr;
     constexpr int SLD_H = WTN + 8;                 // halves per staged row (fp16 output)
@@ -365,11 +371,7 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
             float4v lc4[4], lb4[4];
             if (ln.on) {
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int nl = 32 * i + 8 * g + 4 * hl;
-                    lc4[g] = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl);
-                    lb4[g] = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl);
-                }
+                for (int g = 0; g < 4; g++) { lc4[g] = ln.colsum(i, g, wn * WTN, hl); lb4[g] = ln.biasp(i, g, wn * WTN, hl); }
             }
 #pragma unroll
             for (int g = 0; g < 4; g++) {
@@ -474,8 +476,8 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
 
 // Block j (32 rows) of a wave's accumulators -> its staging area `dst` (32 rows of WTN + 8 halves), rounded to fp16 once
 // with the column bias -- or the folded layer norm's r (acc - mu colsum) + biasp -- joined in fp32.
-template <int j, int TM, int TN, int WTN>
-__device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], const LnFold<TM> &ln, int wn, char *dst, int lane) {
+template <int j, int TM, int TN, int WTN, typename LN>
+__device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], const LN &ln, int wn, char *dst, int lane) {
     constexpr int SLD_H = WTN + 8;
     const int frow = lane & 31, hl = lane >> 5;
     half_t *st = reinterpret_cast<half_t *>(dst) + frow * SLD_H + 4 * hl;
@@ -485,9 +487,8 @@ __device__ __forceinline__ void stage_block(float16v (&acc)[TN][TM], const half4
         for (int g = 0; g < 4; g++) {
             const int nl = 32 * i + 8 * g;
             float v[4];
-            if (ln.on) {      // uniform; the tile's colsum and biasp from their LDS copy
-                const float4v lc = *reinterpret_cast<const float4v *>(ln.col + wn * WTN + nl + 4 * hl);
-                const float4v lb = *reinterpret_cast<const float4v *>(ln.col + ln.bn + wn * WTN + nl + 4 * hl);
+            if (ln.on) {      // uniform
+                const float4v lc = ln.colsum(i, g, wn * WTN, hl), lb = ln.biasp(i, g, wn * WTN, hl);
 #pragma unroll
                 for (int e = 0; e < 4; e++) v[e] = fmaf(acc[i][j][4 * g + e], ln.r[j], fmaf(-ln.rmu[j], lc[e], lb[e]));
             } else {
@@ -522,19 +523,20 @@ struct ResidualAhead {
     // (mw, nw): the wave's first row and column
     __device__ __forceinline__ void request(const GemmArgs &p, int mw, int nw, int lane, long bz) {
         const int ch = lane % CPR, r0 = lane / CPR, n = nw + ch * 8;
-        const bool on = p.residual && store_is_simple(p);
-        const half_t *const base = p.residual + bz * (p.sY + p.dRes) + (long)(mw + r0) * p.ldY + n;
+        if (!p.residual || !store_is_simple(p)) {                 // uniform
 #pragma unroll
-        for (int t = 0; t < NIT; t++) {
-            v[t] = half8v{};
-            if (on && n < p.N && mw + r0 + t * RPI < p.M) v[t] = as_half8(ldg16(base + (long)(t * RPI) * p.ldY));
+            for (int t = 0; t < NIT; t++) v[t] = half8v{};
+            return;
         }
+        const half_t *const base = p.residual + bz * (p.sY + p.dRes) + min(n, p.N - 8);      // rows and columns past the edge: the last ones
+#pragma unroll
+        for (int t = 0; t < NIT; t++) v[t] = as_half8(ldg16(base + (long)min(mw + r0 + t * RPI, p.M - 1) * p.ldY));
     }
 };
 
-template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES, typename LN>
 __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                                  int wave, int lane, long bz, const LnFold<TM> ln, const ResidualAhead<WTN> *ahead) {
+                                                  int wave, int lane, long bz, const LN &ln, const ResidualAhead<WTN> *ahead) {
     constexpr int SLD_H = WTN + 8, BUF_BYTES = 32 * SLD_H * 2;      // halves per staged row; one staging area
     constexpr int CPR = WTN / 8, RPI = 64 / CPR, NIT = 32 / RPI;     // 16-byte chunks per row; rows a wave covers at a time; chunks per lane and block
     static_assert(2 * BUF_BYTES * NWAVES <= LDS_BYTES && 64 % CPR == 0 && CPR % 4 == 0, "two staging areas a wave; four lanes hold a 32-column segment");
@@ -545,7 +547,7 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
     const bool col_ok = n < p.N;                                     // N % 8 == 0: a chunk that starts below N ends below it
     const long off0 = bz * p.sY + (long)(mw + r0) * p.ldY + n;
     half_t *const ybase = reinterpret_cast<half_t *>(p.Y) + off0;
-    const half_t *const rbase = p.residual ? p.residual + off0 + bz * p.dRes : nullptr;
+    const half_t *const rbase = p.residual ? p.residual + bz * (p.sY + p.dRes) + min(n, p.N - 8) : nullptr;
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll
@@ -558,10 +560,7 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
     auto fetch_residual = [&](auto J) {
         constexpr int j = decltype(J)::value;
 #pragma unroll
-        for (int t = 0; t < NIT; t++) {
-            res[j & 1][t] = half8v{};
-            if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) res[j & 1][t] = as_half8(ldg16(rbase + (long)(32 * j + t * RPI) * p.ldY));
-        }
+        for (int t = 0; t < NIT; t++) res[j & 1][t] = as_half8(ldg16(rbase + (long)min(mw + 32 * j + r0 + t * RPI, p.M - 1) * p.ldY));
     };
     if (rbase) {
         if (ahead) {
@@ -668,9 +667,9 @@ __device__ __forceinline__ void store_coop(const GemmArgs &p, char *buf, int mw,
 
 // The activation is a compile-time choice inside the store loops: one uniform branch per tile
 // instead of one per element.
-template <int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES>
+template <int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES, typename LN = LnFold<TM>>
 __device__ __forceinline__ void store_tile(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
-                                           int wave, int lane, long bz, const LnFold<TM> ln = LnFold<TM>{}, const ResidualAhead<WTN> *ahead = nullptr) {
+                                           int wave, int lane, long bz, const LN &ln = LN{}, const ResidualAhead<WTN> *ahead = nullptr) {
     if (store_is_simple(p)) {
         switch (p.epi) {
         case MI_EPI_GELU_ERF: store_tile_simple<MI_EPI_GELU_ERF, TM, TN, WTM, WTN, NWAVES, LDS_BYTES>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, ahead); break;
@@ -696,7 +695,7 @@ int raise_lds(KernelT kern, int bytes) {
 template <int BM, int BN, int BK>
 constexpr int gemm_lds_bytes() {
     constexpr int kc = BN * (BK + 8), kn = BK * (BN + 32);       // B buffer in either layout
-    return 2 * (BM * (BK + 8) + (kc > kn ? kc : kn)) * 2 + BM * 8 + BN * 8;      // + a folded layer norm's (r, r mu) per row, colsum and biasp per column
+    return 2 * (BM * (BK + 8) + (kc > kn ? kc : kn)) * 2;
 }
 
 // Y (and residual) rows allow 16-byte accesses

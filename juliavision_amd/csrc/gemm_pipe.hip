@@ -28,7 +28,7 @@ namespace {
 // KTAIL: K is a multiple of 8 but not of 64.  The last tile's chunks past K re-read the row's last valid chunk (nothing past
 // the row is touched) and are zeroed, in both operands, on their way into LDS: two instructions a chunk and load, which is why
 // whole tiles keep their own instance.  1544 x 1288 -> 1288 with a residual: 25.7 us through the unpipelined kernel before.
-// LNF: the launch has a layer norm folded away (lnf_stats); the statistics' registers would cost the others a workgroup per CU.
+// LNF: the launch has a layer norm folded away (lnf_stats, LnfRows).
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int AMODE = 0, bool KTAIL = false, bool LNF = false>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ? 4 : 2) void gemm_pipe_kernel(GemmArgs p) {
     constexpr bool B_KN = BMODE != 0, LNA = AMODE == 2;
@@ -84,7 +84,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         atile0 = p.ag.split ? (int)bz * (p.K / BK) : 0;
     }
     u32x4 ga[2][PA], gb[2][PB];
+    LnfRows<TM> lnf(p, m0 + wm * WTM, lane);
     auto gload = [&](int set, int kt) {
+        if constexpr (LNF) lnf.request(p, set, kt);       // (ahead of the tile's own: where those have landed, these have)
         const long ko = (long)kt * BK;
         if constexpr (AMODE == 1) {
             const int t = atile0 + kt, tap = t / p.ag.cpt, ci0 = (t - tap * p.ag.cpt) * BK;       // the same for every lane
@@ -181,11 +183,6 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
     const int nk = KTAIL ? (p.K + BK - 1) / BK : p.K / BK;   // the launcher guarantees nk >= 2, and K % 64 == 0 without KTAIL
     gload(0, 0);
     gload(1, 1);
-    // folded layer norm: the row statistics and column constants of the tile, combined ahead of the last tile into a slot
-    // behind the operand buffers (the last tile's barrier covers it)
-    float2v *ln_slot = reinterpret_cast<float2v *>(smem + 2 * (BM * LD + BSZ) * 2);
-    LnfLoader<BM, BN, NT, 40 / (NT >= 4 * BM ? 4 : NT >= 2 * BM ? 2 : 1)> lnf;
-    if constexpr (LNF) lnf.request(p, m0, n0, bz, tid);
     if constexpr (LNA) {
         // One wave per row, all rows of a wave in flight at once (one trip to memory).  Rows past M repeat the last one.
         constexpr int NW = NT / 64, RB = BM / NW;
@@ -226,6 +223,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
     }
     lwrite_a(0, 0, false);
     lwrite_b(0, 0, false);
+    if constexpr (LNF) lnf.template take<true>(0);
     __syncthreads();
     fread(0, 0, 0, 0);
 
@@ -243,7 +241,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         mma(0);
         __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
 #pragma unroll
-        for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x020, (PA + PB + NM - 1) / NM, 0); }
+        for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x020, (PA + PB + (LNF ? TM : 0) + NM - 1) / NM, 0); }
         __builtin_amdgcn_sched_barrier(0);
         fread(0, cur, 2, kt);
         mma(1);
@@ -255,6 +253,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         fread(1, cur, 3, kt);
         mma(0);
         if constexpr (MODE < 2) lwrite_b(gw, cur ^ 1, MODE == 1);
+        if constexpr (LNF && MODE < 2) lnf.take(gw);
         __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
 #pragma unroll
         for (int g = 0; g < NM; g++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x200, (PB + NM - 1) / NM, 0); }
@@ -274,29 +273,26 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, LNF && BM * BN == 64 * 128 ?
         body(M0{}, kt, 0, 1, 0);
         body(M0{}, kt + 1, 1, 0, 1);
     }
-    half4v cb[TN][4];
+    half4v cb[TN][4] = {};                    // (a folded norm has its bias in biasp)
     ResidualAhead<WTN> res;
+    std::conditional_t<LNF, LnFoldRegs<TM, TN>, LnFold<TM>> ln;
+    // what the store needs of memory, under the last tile
+    auto ends = [&](int kt, int cur, int gw, int gl) __attribute__((always_inline)) {
+        body(M1{}, kt, cur, gw, gl);
+        if constexpr (LNF) {
+            ln.load(p, n0 + wn * WTN, lane, bz);
+            lnf.finish(p, ln.r, ln.rmu);
+        } else {
+            load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
+            res.request(p, m0 + wm * WTM, n0 + wn * WTN, lane, bz);
+        }
+        body(M2{}, kt + 1, cur ^ 1, gl, gw);
+    };
     if (nk & 1) {
         body(M0{}, kt, 0, 1, 0);
-        body(M1{}, kt + 1, 1, 0, 1);
-        load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
-        if constexpr (!LNF) res.request(p, m0 + wm * WTM, n0 + wn * WTN, lane, bz);
-        if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
-        body(M2{}, kt + 2, 0, 1, 0);
-    } else {
-        body(M1{}, kt, 0, 1, 0);
-        load_col_bias<TN, WTN>(p, cb, n0, wn, lane, bz);
-        if constexpr (!LNF) res.request(p, m0 + wm * WTM, n0 + wn * WTN, lane, bz);
-        if constexpr (LNF) lnf.combine(p, ln_slot, m0, tid);
-        body(M2{}, kt + 1, 1, 0, 1);
-    }
+        ends(kt + 1, 1, 0, 1);
+    } else ends(kt, 0, 1, 0);
     __syncthreads();
-    LnFold<TM> ln;
-    if constexpr (LNF) {
-        ln.on = true; ln.col = reinterpret_cast<const float *>(ln_slot + BM); ln.bn = BN;
-#pragma unroll
-        for (int j = 0; j < TM; j++) { const float2v v = ln_slot[wm * WTM + 32 * j + (lane & 31)]; ln.r[j] = v[0]; ln.rmu[j] = v[1]; }
-    }
     store_tile<TM, TN, WTM, WTN, WAVES_M * WAVES_N, 2 * (BM * LD + BSZ) * 2>(p, acc, cb, smem, m0, n0, wm, wn, wave, lane, bz, ln, LNF ? nullptr : &res);
 }
 

@@ -166,3 +166,14 @@ def test_folded_norm_declines_what_it_does_not_cover(ctx):
         out = torch.empty((T, F), dtype=torch.float16, device="cuda")
         with pytest.raises(jv.DeclineError):
             jv.lnfold_matmul_(ctx, out, fw, x, stats, 1e-5)
+
+
+# Statistics taken in by the matrix waves, a K tile's two segments at a time: two, three, an even and an odd number of tiles, rows
+# and columns that end inside a tile, fp32 results, and rows far from zero.
+@pytest.mark.parametrize("T,K,F,layout,more", [
+    (1370, 128, 1152, "kf", {}), (1370, 192, 1160, "fk", {}), (1001, 448, 1536, "fk", dict(epi="gelu")), (1370, 576, 1144, "fk", {}),
+    (1370, 384, 1156, "fk", dict(out_f32=True)), (999, 512, 2056, "kf", dict(residual=True)), (2056, 384, 1152, "kf", dict(mean=-30.0, planes=3)),
+    (65, 128, 72, "fk", dict(epi="relu")),
+])
+def test_statistics_by_the_matrix_waves(ctx, T, K, F, layout, more):
+    _folded(ctx, T, K, F, layout=layout, seed=60 + K, **more)
