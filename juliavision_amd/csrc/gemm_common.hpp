@@ -422,10 +422,7 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
                     x = *reinterpret_cast<const half8v *>(reinterpret_cast<const half_t *>(stage) + row * SLD_H + ch * 8);
                     const long off = bz * p.sY + (long)m * p.ldY + n;
                     half_t *yp = reinterpret_cast<half_t *>(p.Y) + off;
-                    if constexpr (EPI != MI_EPI_NONE) {
-#pragma unroll
-                        for (int e = 0; e < 8; e++) x[e] = (half_t)apply_epi_c<EPI>((float)x[e]);
-                    }
+                    x = apply_epi8<EPI>(x);
                     if (n + 7 < p.N) {
                         if (p.residual) {
                             half8v rv;
@@ -583,10 +580,7 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
         for (int t = 0; t < NIT; t++) {
             const int m = mw + 32 * j + r0 + t * RPI;
             const bool have = col_ok && m < p.M;
-            if constexpr (EPI != MI_EPI_NONE) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[t][e] = (half_t)apply_epi_c<EPI>((float)x[t][e]);
-            }
+            x[t] = apply_epi8<EPI>(x[t]);
             if (rbase) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) x[t][e] = (half_t)((float)x[t][e] + (float)res[j & 1][t][e]);
@@ -620,8 +614,8 @@ __device__ __forceinline__ void store_tile_simple(const GemmArgs &p, float16v (&
 
 // The four-wave kernel's store, shared between a matrix wave and the helper wave on its SIMD.  One wave issues a vector
 // instruction every eight clocks, a SIMD takes one every four: the erf-GELU of a 128 x 256 tile (a reciprocal, an
-// exponential and thirteen other vector instructions on each of 128 values a lane) cost a lone matrix wave 14 600
-// clocks, 8 100 with a helper, and the plain store gains too (1500 x 1280 -> 5120 + bias: 21.8 us against 22.8).  The
+// exponential and then thirteen other vector instructions on each of 128 values a lane) cost a lone matrix wave 14 600
+// clocks, 8 100 with a helper (apply_epi8 has fewer now), and the plain store gains too (1500 x 1280 -> 5120 + bias: 21.8 us against 22.8).  The
 // matrix wave stages its 32-row blocks as in store_tile_simple and takes the first half of each block's chunks, the
 // helper the second half; a workgroup barrier per block says "block j is staged" (a wave passes barrier j + 1 only
 // when it has block j's chunks in registers, so staging block j + 2 over block j's area after that barrier is safe).
@@ -649,8 +643,7 @@ __device__ __forceinline__ void store_coop_epi(const GemmArgs &p, char *buf, int
         if constexpr (!HELPER && j + 1 < TM) stage(std::integral_constant<int, j + 1>{});
 #pragma unroll
         for (int t = T0; t < T1; t++) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[t - T0][e] = (half_t)apply_epi_c<EPI>((float)x[t - T0][e]);
+            x[t - T0] = apply_epi8<EPI>(x[t - T0]);
             if (col_ok && mw + 32 * j + r0 + t * RPI < p.M) *reinterpret_cast<half8v *>(ybase + (long)(32 * j + t * RPI) * p.ldY) = x[t - T0];
         }
     });

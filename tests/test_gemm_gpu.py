@@ -505,3 +505,44 @@ def test_clamped_gemm_declines_a_clamp_that_is_not_positive(ctx):
         rc = lib.mi_gemm_clamp_ln_f16(y.data_ptr(), None, x.data_ptr(), w.data_ptr(), None, None, None, None, 1e-5, bad,
                                       16, 64, 64, 64, 64, L.W_KF, L.BIAS_NONE, L.EPI["none"], None, 0, ctx.stream)
         assert rc == L.DECLINE_OPERANDS
+
+
+@pytest.mark.parametrize("T,K", [(256, 256), (1500, 1280), (64, 1024), (8, 1024)])
+def test_gelu_of_every_fp16(ctx, T, K):
+    """Through an identity product, every fp16 value meets the store's GELU (tiles of both kinds, the split store, decode rows): the
+    formula in 64 bits, rounded once, to within one fp16 step where the fp32 evaluation lies next to a tie -- some 1e-7 of
+    |v|, more than a hundredth of a step from a tie in 1 % of the cases."""
+    import torch
+    import juliavision_amd as jv
+    bits = np.arange(65536, dtype=np.uint16).view(np.float16)
+    fin = np.where(np.isfinite(bits), bits, np.float16(0))
+    X = np.resize(fin, T * K).reshape(T, K)
+    out = poison(torch.empty((T, K), dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.matmul_(ctx, out, torch.eye(K, dtype=torch.float16, device="cuda").t(), to_dev(X), epi="gelu")
+    torch.cuda.synchronize()
+    v = X.astype(np.float64)
+    t = 1.0 / (1.0 + 0.3275911 * np.abs(v) / np.sqrt(2.0))
+    q = 0.5 * ((((1.061405429 * t - 1.453152027) * t + 1.421413741) * t - 0.284496736) * t + 0.254829592) * t * np.exp(-v * v / 2)
+    want = (np.maximum(v, 0.0) - np.abs(v) * q).astype(np.float16)
+    got = to_host(out)
+    step = np.spacing(np.abs(want).clip(max=np.float16(60000))).astype(np.float64)
+    diff = np.abs(got.astype(np.float64) - want.astype(np.float64))
+    assert (diff <= step).all() and (diff > 0).mean() < 0.01
+
+
+def test_gelu_of_infinities_and_nan(ctx):
+    import torch
+    import juliavision_amd as jv
+    X = np.full((70, 128), np.nan, dtype=np.float16)
+    X[0, :] = 65504
+    X[1, :] = -65504
+    X[2:, :] = 0
+    X[3, 0] = np.nan
+    W = np.ones((128, 64), dtype=np.float16)               # rows 0 and 1 sum to +-inf in fp16
+    out = poison(torch.empty((70, 64), dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.matmul_(ctx, out, to_dev(W), to_dev(X), epi="gelu")
+    torch.cuda.synchronize()
+    got = to_host(out)
+    assert np.isposinf(got[0]).all() and (got[1] == 0).all() and np.isnan(got[3]).all() and (got[4:] == 0).all()
