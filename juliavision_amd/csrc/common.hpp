@@ -160,8 +160,8 @@ static inline bool is_nan_arg(float x) { uint32_t u; __builtin_memcpy(&u, &x, 4)
 
 // Largest image, in halves, of the gather below: gemm_ring_kernel's offsets into it are 32-bit byte offsets, raised by up to 3072.
 constexpr int64_t MI_PATCH_IMAGE_MAX = INT32_MAX - 1536;
-// Implicit-GEMM convolution over a zero-padded channels-last copy xp[img][Hp][Wp][C] of the input: how gemm_ring_kernel finds
-// its [N][K] operand (row n = output pixel (oh, ow), K ordered (kh, kw, ci) with ci fastest) in it.  Sixteen bytes of a
+// Implicit-GEMM convolution over a zero-padded channels-last copy xp[img][Hp][Wp][C] of the input: how gemm_ring_kernel and
+// gemm_deep_kernel find their [N][K] operand (row n = output pixel (oh, ow), K ordered (kh, kw, ci) with ci fastest) in it.  Sixteen bytes of a
 // row are eight channels of one tap, at an offset from the pixel's origin that is the same for every pixel.
 struct ConvGather {
     const half_t *xp;      // nullptr = ordinary GEMM
@@ -169,6 +169,7 @@ struct ConvGather {
     int C, OW, KW;
     int pix_y, pix_x;      // elements between the origins of neighbouring output rows and columns: sy Wp C, sx C
     int tap_y, tap_x;      // and between neighbouring taps: dy Wp C, dx C
+    unsigned div_C, div_OW, div_KW;      // recip_of
 };
 
 // Implicit-GEMM convolution over a channels-last input x[N][H][W][C]: how the GEMM finds its [M][K] operand
@@ -203,5 +204,5 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
 // Workspace bytes such a call needs (fp32 planes when it splits K); T > 8 rows.
 size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatch);
 // What such a call is estimated to take, in microseconds.
-double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);      // B a ConvGather
+double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);      // B a ConvGather: on the kernel that is estimated to be faster
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);

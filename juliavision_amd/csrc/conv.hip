@@ -361,6 +361,7 @@ int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
         ConvGather g;
         g.xp = xp; g.img = (long)a.Cin * Hp * Wp; g.C = a.Cin; g.OW = a.OW; g.KW = a.KW;
         g.pix_y = a.sy * Wp * a.Cin; g.pix_x = a.sx * a.Cin; g.tap_y = a.dy * Wp * a.Cin; g.tap_x = a.dx * a.Cin;
+        g.div_C = recip_of(g.C); g.div_OW = recip_of(g.OW); g.div_KW = recip_of(g.KW);
         // B is never dereferenced in this mode; xp stands in so that the operand checks see an aligned pointer
         return mi_internal_gemm(out, w2, xp, bias, a.Cout, PQ, PQ, CRS, PQ, CRS, CRS, 0, MI_BIAS_ROW, epi, 0,
                                 a.N, (long)a.Cout * PQ, 0, 0, nullptr, 0, st, &g);

@@ -1010,7 +1010,13 @@ size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatc
     return planned_workspace(T, F, K);
 }
 
-double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, RING_TILE, 1); }
+// A patch matrix is gathered by two kernels: 64 x 64 tiles, and 32 x 32 ones with K split over their waves where they are at most one
+// workgroup a CU (as many as their estimate was fitted to): 43 such convolutions 0.62 to 0.96 of the ring's time.
+static bool patches_deep(int64_t T, int64_t K, int64_t F, int64_t nbatch) {
+    return ceil_div(T, 32) * ceil_div(F, 32) * nbatch <= std::min(DEEP_WGS, (int64_t)mi_num_cus()) &&
+           tile_cost_us(T, F, K, nbatch, DEEP_TILE, 1) < tile_cost_us(T, F, K, nbatch, RING_TILE, 1);
+}
+double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, patches_deep(T, K, F, nbatch) ? DEEP_TILE : RING_TILE, 1); }
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return plan_tiles(T, F, K, nbatch, nbatch == 1).us; }
 
 // Internal entry used by the convolution path (conv.hip): Y[M x N] = A . B with
@@ -1036,7 +1042,10 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
     if (agather) a.ag = *agather;
     const bool addr = mfma_addressable(a, b_kn != 0);
     if ((gather || agather) && !addr) return MI_DECLINE_OPERANDS;
-    if (gather) return g_ready ? mi_ring_launch(a, false, nbatch, st) : MI_ERROR_DEVICE;
+    if (gather) {
+        if (!g_ready) return MI_ERROR_DEVICE;
+        return patches_deep(M, K, N, nbatch) ? mi_deep_launch(a, true, false, nbatch, st) : mi_ring_launch(a, false, nbatch, st);
+    }
     int path = addr ? MI_GEMM_MFMA : MI_GEMM_SCALAR;
     return run_gemm(a, b_kn != 0, nbatch, ws, ws_bytes, st, path);
 }

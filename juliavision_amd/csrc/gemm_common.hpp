@@ -713,7 +713,7 @@ int mi_pipe_init();
 // gemm_ring.hip: small grids of ordinary operands, and patch matrices of a convolution.
 int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_ring_init();
-// gemm_deep.hip: few output tiles, of ordinary operands.
+// gemm_deep.hip: few output tiles, of ordinary operands (split_k: K over its waves) and of patch matrices (always).
 int mi_deep_launch(const GemmArgs &a, bool split_k, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_deep_init();
 // gemm_any.hip: the kernels for operands and extents that the others do not take.

@@ -1,4 +1,5 @@
-// fp16 GEMM for gfx950, 32 x 32 tiles, the waves of a long K splitting it: grids of few output tiles.
+// fp16 GEMM for gfx950, 32 x 32 tiles, the waves of a long K splitting it: grids of few output tiles, of ordinary operands and of
+// convolutions' patch matrices.
 #include "gemm_common.hpp"
 
 // Sixteen zero bytes for loads of chunks past the end of K.
@@ -22,11 +23,21 @@ namespace {
 //
 // LDS layout of a stage: A rows of 256 bytes, then B ([N][K]: the same; [K][N]: 128 rows of 64 bytes).  Sixteen-byte chunks are permuted
 // inside their row: K-contiguous row r holds chunk c at c ^ (r % 16), [K][N] row k at c ^ (k % 4).
+//
+// CONV: B is the patch matrix of a convolution (ConvGather), its rows' offsets fixed and the tap moving.  A 128-deep stage may hold
+// eight taps (sixteen channels each), and the permutation gives a lane another chunk in each of four requests in a row.  Two loader
+// waves take two of the four each, request by request, so a lane keeps two (tap, channel) states, advanced by whole taps and what is
+// left of a stage: some twelve instructions each for the 400 clocks of a stage.  K is split whatever its depth: nothing promises one
+// chain of sums of a convolution.
+// Against the 64 x 64 ring, both behind conv_pad_kernel, in us (workgroups): 144 x 34 x 60 -> 32, 7 x 7 stride 4 (5) 29.5 -> 20.3;
+// 96 x 22 x 23 -> 96, 5 x 5 (48) 15.5 -> 11.6; 256 x 29 x 11 -> 384, 5 x 5 (120) 29.1 -> 23.6; 256 x 30 x 112 -> 64, 3 x 3 (210) 13.9 -> 12.4.
+// 43 convolutions of at most 256 workgroups, 2304 deep in the middle: 0.81 of the time, geometric mean, none slower.
 constexpr int S = 8;                      // stages of the ring: 128 KB
 
-template <int NW, int CHAINS, bool B_KN>
+template <int NW, int CHAINS, bool B_KN, bool CONV = false>
 __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p) {
-    constexpr int BM = 32, BN = 32, BK = 128, LPW = 8, AHEAD = 5;
+    static_assert(!(CONV && B_KN), "a patch row is K-contiguous");
+    constexpr int BM = 32, BN = 32, BK = 128, AHEAD = 5;
     constexpr int STEPS = 8 / NW;                         // a matrix wave's steps of a stage
     constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = 2 * A_BYTES;
     extern __shared__ __align__(16) char smem[];
@@ -46,14 +57,23 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
 
     if (__builtin_expect(wave >= NW, 1)) {
         auto load_all = [&](auto IS_A_) __attribute__((always_inline)) {
-            constexpr bool IS_A = decltype(IS_A_)::value, ROWS = IS_A || !B_KN;
+            constexpr bool IS_A = decltype(IS_A_)::value, ROWS = IS_A || !B_KN, PATCH = CONV && !IS_A;
+            // 1 KB requests of a stage, a run of RUN in a row sharing an LDS address.  PATCH: 2 half + {0, 1, 4, 5}
+            constexpr int LPW = PATCH ? 4 : 8, RUN = PATCH ? 2 : 4;
+            const int half = PATCH ? wave - (NW + 1) : 0;
             uint32_t off[LPW];
             int kpos[LPW];                                // first k of the lane's chunk
             const long ld2 = (IS_A ? p.ldA : p.ldB) * 2;
             const int r0 = IS_A ? m0 : n0, rows = IS_A ? p.M : p.N;
 #pragma unroll
             for (int i = 0; i < LPW; i++) {
-                if constexpr (ROWS) {                     // request i: rows 4 i .. 4 i + 3; past the edge the last one again
+                if constexpr (PATCH) {
+                    const int slot = 2 * half + (i & 1) + 4 * (i >> 1), r = 4 * slot + (lane >> 4), c = (lane & 15) ^ (r & 15);
+                    unsigned ow;
+                    const unsigned oh = divide(min(r0 + r, rows - 1), p.cv.OW, p.cv.div_OW, ow);
+                    off[i] = (oh * p.cv.pix_y + ow * p.cv.pix_x) * 2u + (c & 1) * 16;
+                    kpos[i] = c * 8;
+                } else if constexpr (ROWS) {              // request i: rows 4 i .. 4 i + 3; past the edge the last one again
                     const int r = 4 * i + (lane >> 4), c = (lane & 15) ^ (r & 15);
                     off[i] = (uint32_t)((min(r0 + r, rows - 1) - r0) * ld2) + c * 16;
                     kpos[i] = c * 8;
@@ -63,20 +83,42 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
                     kpos[i] = k;
                 }
             }
-            constexpr int LOW = 3072;                     // a request's immediate offset moves source and destination alike: gemm_ring_kernel
+            constexpr int LOW = 1024 * (RUN - 1);         // a request's immediate offset moves source and destination alike: gemm_ring_kernel
 #pragma unroll
-            for (int i = 0; i < LPW; i++) off[i] += LOW - 1024 * (i & 3);
+            for (int i = 0; i < LPW; i++) off[i] += LOW - 1024 * (i & (RUN - 1));
             const char *org = (IS_A ? reinterpret_cast<const char *>(p.A + bz * p.sA + (long)m0 * p.ldA)
+                                    : PATCH ? reinterpret_cast<const char *>(p.cv.xp + bz * p.cv.img)
                                     : reinterpret_cast<const char *>(p.B + bz * p.sB + (B_KN ? (long)n0 : (long)n0 * p.ldB))) - LOW;
-            const long step = ROWS ? BK * 2 : (long)BK * p.ldB * 2;
-            const uint32_t lds1 = lds0 + (IS_A ? 0 : A_BYTES);
+            const long step = PATCH ? 0 : ROWS ? BK * 2 : (long)BK * p.ldB * 2;
+            const uint32_t lds1 = lds0 + (IS_A ? 0 : A_BYTES) + half * 2048;
+            // PATCH: channel, tap column and byte offset, from the pixel, of the pair of chunks that requests i with i % 2 = t take next
+            const int taps = PATCH ? BK / p.cv.C : 0, rest = PATCH ? BK - taps * p.cv.C : 0, rows_max = PATCH ? (taps + p.cv.KW) / p.cv.KW : 0;
+            const int tap_step = p.cv.tap_x * 2, over_step = (p.cv.tap_x - p.cv.C) * 2, row_step = (p.cv.tap_y - p.cv.KW * p.cv.tap_x) * 2;
+            const int stage_step = taps * tap_step + rest * 2;
+            int ch[2], kw[2];
+            uint32_t at[2] = {0u, 0u};
+            if constexpr (PATCH) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    unsigned c, w;
+                    const unsigned tap = divide(kpos[t] & ~15, p.cv.C, p.cv.div_C, c), kh = divide(tap, p.cv.KW, p.cv.div_KW, w);
+                    ch[t] = c; kw[t] = w;
+                    at[t] = (c + kh * p.cv.tap_y + w * p.cv.tap_x) * 2u;
+                }
+            }
             int next = 0;                                 // the stage of K requested next, and where it goes
             uint32_t stage = 0;
             auto request = [&]() __attribute__((always_inline)) {
                 if ((next + 1) * BK <= p.K) {             // uniform
 #pragma unroll
-                    for (int q = 0; q < LPW; q += 4)
-                        asm volatile("s_mov_b32 m0, %0\n\t"
+                    for (int q = 0; q < LPW; q += RUN)
+                        if constexpr (PATCH)
+                            asm volatile("s_mov_b32 m0, %0\n\t"
+                                         "s_nop 0\n\t"
+                                         "global_load_lds_dwordx4 %1, %3\n\t"
+                                         "global_load_lds_dwordx4 %2, %3 offset:1024" ::"s"(lds1 + stage + q * 2048),
+                                         "v"(off[q] + at[0]), "v"(off[q + 1] + at[1]), "s"(org) : "memory");
+                        else asm volatile("s_mov_b32 m0, %0\n\t"
                                      "s_nop 0\n\t"
                                      "global_load_lds_dwordx4 %1, %5\n\t"
                                      "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
@@ -86,8 +128,24 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
                 } else {                                  // the stage that K ends in: chunks past it come from the zeros
 #pragma unroll
                     for (int i = 0; i < LPW; i++) {
-                        const char *from = next * BK + kpos[i] < p.K ? org + off[i] + 1024 * (i & 3) : reinterpret_cast<const char *>(deep_zero_words);
-                        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds1 + stage + i * 1024) : "memory");
+                        const char *from = next * BK + kpos[i] < p.K ? org + (off[i] + (PATCH ? at[i & 1] : 0u)) + 1024 * (i & (RUN - 1)) : reinterpret_cast<const char *>(deep_zero_words);
+                        const uint32_t to = PATCH ? (i & 1) * 1024 + (i >> 1) * 4096 : i * 1024;
+                        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds1 + stage + to) : "memory");
+                    }
+                }
+                if constexpr (PATCH) {
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        ch[t] += rest;
+                        const bool over = ch[t] >= p.cv.C;
+                        ch[t] -= over ? p.cv.C : 0;
+                        kw[t] += taps + (over ? 1 : 0);
+                        at[t] += stage_step + (over ? over_step : 0);
+                        for (int r = 0; r < rows_max; r++) {      // on to the taps of the next rows
+                            const bool row = kw[t] >= p.cv.KW;
+                            kw[t] -= row ? p.cv.KW : 0;
+                            at[t] += row ? row_step : 0;
+                        }
                     }
                 }
                 org += step;
@@ -120,7 +178,7 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
                 barrier();
             }
         };
-        if (wave == NW + 2) lnf_stats_wave<BM, BN, false, 4>(p, reinterpret_cast<float2v *>(smem + S * STAGE_BYTES), m0, n0, bz, lane, nk, barrier);
+        if (!CONV && wave == NW + 2) lnf_stats_wave<BM, BN, false, 4>(p, reinterpret_cast<float2v *>(smem + S * STAGE_BYTES), m0, n0, bz, lane, nk, barrier);
         else if (wave == NW) load_all(std::true_type{});
         else load_all(std::false_type{});
         return;
@@ -237,6 +295,11 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
 
 constexpr int DEEP_LDS_BYTES = S * 2 * 32 * 128 * 2 + 2 * 32 * 8;       // the stages; rows' and columns' parts of a folded norm
 
+template <int CHAINS>
+int launch_deep_patches(const GemmArgs &a, int64_t nbatch, hipStream_t st) {
+    hipLaunchKernelGGL((gemm_deep_kernel<4, CHAINS, false, true>), dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), dim3(7 * 64), DEEP_LDS_BYTES, st, a);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
 template <int NW, int CHAINS>
 int launch_deep(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st) {
     const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nbatch), block((NW + (a.lnf_stats ? 3 : 2)) * 64);
@@ -253,6 +316,10 @@ int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch
     GemmArgs a = args;
     set_tiles(a, 32, 32);
     a.vec_store = rows_vec16(a);
+    if (a.cv.xp) {
+        if (b_kn || a.cv.img > MI_PATCH_IMAGE_MAX || (int64_t)32 * a.ldA * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+        return a.K > 4096 ? launch_deep_patches<4>(a, nbatch, st) : launch_deep_patches<2>(a, nbatch, st);
+    }
     // per-lane load offsets are 32-bit byte offsets from the tile's origin
     if ((int64_t)32 * a.ldA * 2 >= (1ll << 31) || (int64_t)128 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
     // Past K = 4096 such calls had twelve to twenty chains, as slices of K on the ring; short of it eight are as good as what they had, and
@@ -261,4 +328,7 @@ int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch
     return a.K > 4096 ? launch_deep<4, 4>(a, b_kn, nbatch, st) : launch_deep<4, 2>(a, b_kn, nbatch, st);
 }
 
-int mi_deep_init() { return raise_deep<4, 4>() | raise_deep<4, 2>() | raise_deep<1, 1>(); }
+int mi_deep_init() {
+    return raise_lds(gemm_deep_kernel<4, 2, false, true>, DEEP_LDS_BYTES) | raise_lds(gemm_deep_kernel<4, 4, false, true>, DEEP_LDS_BYTES) |
+           raise_deep<4, 4>() | raise_deep<4, 2>() | raise_deep<1, 1>();
+}

@@ -94,3 +94,43 @@ def test_rows_that_end_between_four_pixels(ctx, Cin, OW, Cout):
             jv.convolution_(ctx, out, torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), bias, (1, 1), (1, 1), (1, 1), 1, act=act)
             want = oracle.conv2d_f16(x, w, None if bias is None else b[1:], (1, 1), (1, 1), (1, 1), 1, act == "relu")
             assert_parity(to_host(out), want, what=f"Cin{Cin} OW{OW} Cout{Cout} {act}")
+
+
+@pytest.mark.parametrize("N,Cin,H,W,Cout,KH,KW,s,p,d,act", [
+    (1, 16, 60, 60, 96, 9, 9, 4, 4, 1, "relu"),            # eight taps a stage, more than a row of them
+    (1, 32, 23, 17, 65, 5, 5, (2, 1), (2, 0), (1, 2), "none"),
+    (2, 48, 13, 11, 96, 5, 3, 1, (1, 2), 1, "relu"),       # taps that end inside a stage, K inside its last one
+    (1, 112, 10, 30, 70, 3, 3, 2, 1, 1, "none"),
+    (1, 128, 8, 33, 32, 3, 3, 1, 1, 1, "none"),            # a tap a stage
+    (1, 144, 31, 14, 144, 3, 3, 1, 1, 1, "none"),
+    (3, 272, 7, 7, 31, 3, 3, 1, 1, 2, "relu"),             # channels and pixels off the tile
+    (2, 192, 64, 3, 96, 3, 3, 1, (0, 1), 1, "none"),       # one output column
+    (1, 256, 5, 5, 256, 3, 3, 1, 1, 1, "none"),
+    (1, 384, 38, 11, 64, 7, 7, 4, 3, 1, "none"),           # two workgroups, 147 stages, four chains a wave
+    (1, 272, 12, 26, 33, 1, 5, 1, (2, 0), 1, "none"),
+    (1, 272, 26, 12, 33, 5, 1, 1, (0, 2), 1, "none"),      # one tap column
+    (1, 256, 30, 112, 64, 3, 3, 1, 1, 1, "relu"),          # 210 workgroups
+])
+def test_patches_of_few_tiles(ctx, N, Cin, H, W, Cout, KH, KW, s, p, d, act):
+    """The patch matrix in 32 x 32 tiles: taps and channels as the stages meet them.  Against 64 bits: products of fp16 values summed in
+    fp32 leave 2^-24 a term of the sum of magnitudes (here below 3e-6 of the largest value), the result's own rounding 2^-11 of it."""
+    import ctypes as C
+
+    import torch
+    import juliavision_amd as jv
+    from juliavision_amd import _lib as L
+    pair = lambda v: v if isinstance(v, tuple) else (v, v)
+    s, p, d = pair(s), pair(p), pair(d)                    # (x, y)
+    assert L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(W, H, Cin, N, KW, KH, Cout, *s, *p, *d, 1, C.byref(C.c_size_t(0)))] == "patch_gemm"
+    x, w = oracle.randn_f16((N, Cin, H, W), 1), oracle.randn_f16((Cout, Cin, KH, KW), 2, 0, 1.0 / np.sqrt(Cin * KH * KW))
+    b = oracle.randn_f16((Cout,), 3, 0, 0.5)
+    want = torch.nn.functional.conv2d(*(torch.from_numpy(a).double() for a in (x, w, b)), s[::-1], p[::-1], d[::-1]).numpy()
+    if act == "relu":
+        want = np.maximum(want, 0)
+    assert -(-Cout // 32) * -(-want[0, 0].size // 32) * N <= 256
+    out = poison(torch.empty(want.shape, dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.convolution_(ctx, out, to_dev(x), to_dev(w), to_dev(b), s, p, d, 1, act=act)
+    torch.cuda.synchronize()
+    got = to_host(out).astype(np.float64)
+    assert np.isfinite(got).all() and (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2.0 ** -24 + 3e-6 * np.abs(want).max()).all()
