@@ -201,7 +201,9 @@ int mi_gemm_f16_batched(void *Y, const void *X, const void *W, const void *bias,
 
 /* Decode-sized T (<= 8; more declines with MI_DECLINE_EXTENT): the
  * bandwidth-bound form.  [K][F] weights: K split across workgroups, fp32
- * partial planes in ws, a reducing epilogue (ws from mi_gemm_f16_workspace).
+ * partial planes in ws, a reducing epilogue (ws from mi_gemm_f16_workspace, which
+ * is asked for whichever kernel runs); or, where that is estimated to be faster,
+ * one launch of 32 x 32 tiles.
  * [F][K] weights: one launch, no workspace.  mi_gemm_f16 takes the same route
  * by itself for T <= 8; this entry forces it.
  * The reference's counterpart is the fp32-only Lava.gemv! path

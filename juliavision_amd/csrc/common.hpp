@@ -204,5 +204,6 @@ int mi_internal_gemm(void *Y, const void *A, const void *B, const void *bias, in
 // Workspace bytes such a call needs (fp32 planes when it splits K); T > 8 rows.
 size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatch);
 // What such a call is estimated to take, in microseconds.
+int mi_internal_layernorm(void *out, float *mean, float *rstd, const void *a, int64_t lda, const void *gamma, const void *beta, int64_t C, int64_t groups, float eps, void *stream);
 double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);      // B a ConvGather: on the kernel that is estimated to be faster
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);

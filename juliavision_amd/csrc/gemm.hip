@@ -1017,6 +1017,9 @@ static bool patches_deep(int64_t T, int64_t K, int64_t F, int64_t nbatch) {
            tile_cost_us(T, F, K, nbatch, DEEP_TILE, 1) < tile_cost_us(T, F, K, nbatch, RING_TILE, 1);
 }
 double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, patches_deep(T, K, F, nbatch) ? DEEP_TILE : RING_TILE, 1); }
+double mi_deep_us(int64_t T, int64_t K, int64_t F) {
+    return ceil_div(T, 32) * ceil_div(F, 32) <= std::min(DEEP_WGS, (int64_t)mi_num_cus()) ? tile_cost_us(T, F, K, 1, DEEP_TILE, 1) : 1e30;
+}
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return plan_tiles(T, F, K, nbatch, nbatch == 1).us; }
 
 // Internal entry used by the convolution path (conv.hip): Y[M x N] = A . B with

@@ -704,6 +704,7 @@ constexpr size_t SKINNY_FK_LDS_MAX = 128 * 1024;    // activations of the [F][K]
 // Up to eight rows; `ws`: the fp32 planes of mi_skinny_splits K-slices ([K][F] weights only).
 int mi_skinny_launch(const GemmArgs &a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st);
 int mi_skinny_splits(int64_t K, int64_t F);
+double mi_deep_us(int64_t T, int64_t K, int64_t F);      // gemm.hip's estimate of gemm_deep_kernel, at most one workgroup a CU; infinite otherwise
 int mi_skinny_init();
 // gemm_pipe.hip: the register-staged pipelined kernel.  `tile` indexes TILE_MODELS (gemm.hip).
 int mi_pipe_launch(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);

@@ -324,8 +324,9 @@ int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch
     if ((int64_t)32 * a.ldA * 2 >= (1ll << 31) || (int64_t)128 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
     // Past K = 4096 such calls had twelve to twenty chains, as slices of K on the ring; short of it eight are as good as what they had, and
     // the second pair of accumulators costs 0.05 to 0.1 us (50 x 3224 -> 992 6.67 | 6.75).
+    // Up to eight rows replace K-slices of [K][F] weights, whose error eight chains exceed from K = 1280 on (9.4e-8 | 9.7e-8, sixteen 8.3e-8).
     if (!split_k) return launch_deep<1, 1>(a, b_kn, nbatch, st);
-    return a.K > 4096 ? launch_deep<4, 4>(a, b_kn, nbatch, st) : launch_deep<4, 2>(a, b_kn, nbatch, st);
+    return a.K > 4096 || (a.M <= 8 && a.K > 768) ? launch_deep<4, 4>(a, b_kn, nbatch, st) : launch_deep<4, 2>(a, b_kn, nbatch, st);
 }
 
 int mi_deep_init() {

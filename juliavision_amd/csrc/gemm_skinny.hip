@@ -572,6 +572,20 @@ int skinny_kper(int64_t K, int64_t F) {
     return (int)kper;
 }
 
+// Whether [K][F] weights run as 32 x 32 tiles with K over the waves of a workgroup (gemm_deep_kernel) instead of K-slices and the launch
+// that sums them.  The tiles are one launch and one trip to memory, their products on the matrix cores; the slices have more loads in
+// flight where a large weight comes from memory.  us, slices | tiles: 384 -> 1536 one row 6.1 | 3.4, eight 9.2 | 3.5; 64 -> 128 4.2 | 3.2,
+// 7.4 | 3.2; 1280 -> 5120 four rows 8.2 | 4.7, from memory 10.0 | 8.5, and one row 6.2 | 6.0, from memory 8.2 | 9.3: hence the megabytes.
+// With a norm in front the rows are normalised into the planes' memory first, by the norm's own kernel, for the bits of the two calls:
+// 384 -> 1536 7.2 | 5.3, 11.4 | 5.5.  That is slower for one or two rows past K = 768 (1032 -> 136 6.4 | 7.6; 768 -> 768 7.1 | 6.2).  Error
+// against 64 bits (fp32 results, 64 <= K <= 1280): 0.76 to 0.96 of the slices'; past that it is theirs that is smaller (1536 -> 384
+// 8.6e-8 | 1.0e-7), so they stay.
+bool kn_on_tiles(int64_t T, int64_t K, int64_t F, size_t planes) {
+    if (K > (T <= 2 ? 768 : 1280) || planes < (size_t)(T * K) * sizeof(half_t)) return false;
+    const double mb = 2e-6 * (double)K * (double)F, rows = T <= 1 ? 0.0 : T <= 2 ? 0.4 : T <= 4 ? 1.3 : 3.4;
+    return mi_deep_us(T, K, F) + 0.25 * std::min(mb, 16.0) < 5.9 + rows + 0.15 * mb + 1.2e-6 * (double)planes;
+}
+
 // few_rows_kernel from five rows on.  us at four rows on the kernels above, at eight on the matrix cores: 1280 -> 5120 5.2 and 6.6, 4096 -> 1024
 // 5.7 and 7.2, 5120 -> 1280 7.6 and 8.4, 1280 -> 51866 27.3 and 26.2, 1536 -> 384 3.2 and 3.8 (the kernels above hold four rows at most).
 constexpr int FEW_ROWS_MIN = 5;
@@ -685,6 +699,16 @@ int mi_skinny_launch(const GemmArgs &a, bool b_kn, void *ws, size_t ws_bytes, hi
         const int kper = skinny_kper(a.K, a.N), nsplit = (int)ceil_div(a.K, kper);
         size_t need = (size_t)nsplit * a.M * a.N * sizeof(float);
         if (!ws || ws_bytes < need || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
+        if (kn_on_tiles(a.M, a.K, a.N, need)) {
+            GemmArgs t = a;
+            if (a.ln_on) {
+                t.ln_on = 0; t.A = reinterpret_cast<const half_t *>(ws); t.ldA = a.K;
+                const int rc = mi_internal_layernorm(ws, nullptr, nullptr, a.A, a.ldA, a.ln_gamma, a.ln_beta, a.K, a.M, a.ln_eps, st);
+                if (rc != MI_OK) return rc;
+            }
+            const int rc = mi_deep_launch(t, true, true, 1, st);
+            if (rc != MI_DECLINE_EXTENT) return rc;      // declined: a row pitch beyond its 32-bit offsets
+        }
         float *part = reinterpret_cast<float *>(ws);
         dim3 grid((unsigned)ceil_div(a.N, SKN_COLS), (unsigned)nsplit);
         if (a.M <= 1)      hipLaunchKernelGGL(skinny_kn_kernel<1>, grid, dim3(256), 0, st, a, part, kper);

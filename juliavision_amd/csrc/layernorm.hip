@@ -9,11 +9,11 @@ namespace {
 // A row of C <= 64 * 8 * NCH halves lives in NCH 16-byte chunks per lane.
 template <int NCH>
 __global__ __launch_bounds__(256) void layernorm_vec_kernel(half_t *out, float *mean, float *rstd, const half_t *a,
-                                                            const half_t *gamma, const half_t *beta, int C, long groups, float eps) {
+                                                            const half_t *gamma, const half_t *beta, int C, long groups, float eps, long lda) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const long g = (long)blockIdx.x * 4 + wave;
     if (g >= groups) return;
-    const half_t *row = a + g * C;
+    const half_t *row = a + g * lda;
     float x[NCH][8];
     float s = 0.0f;
     // gamma and beta are requested together with the row: one trip to memory for the kernel, not two
@@ -70,11 +70,11 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(half_t *out, float *
 
 // Any C, any alignment: the same three passes reading memory each time.
 __global__ __launch_bounds__(256) void layernorm_any_kernel(half_t *out, float *mean, float *rstd, const half_t *a,
-                                                            const half_t *gamma, const half_t *beta, int C, long groups, float eps) {
+                                                            const half_t *gamma, const half_t *beta, int C, long groups, float eps, long lda) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const long g = (long)blockIdx.x * 4 + wave;
     if (g >= groups) return;
-    const half_t *row = a + g * C;
+    const half_t *row = a + g * lda;
     float s = 0.0f;
     for (int i = lane; i < C; i += 64) s += (float)row[i];
     s = wave_sum(s);
@@ -312,6 +312,13 @@ extern "C" {
 
 int mi_layernorm_f16(void *out, float *mean, float *rstd, const void *a, const void *gamma, const void *beta,
                      int64_t C, int64_t groups, float eps, void *stream) {
+    return mi_internal_layernorm(out, mean, rstd, a, C, gamma, beta, C, groups, eps, stream);
+}
+}  // extern "C"
+
+// The rows of `a` at a pitch of lda (a multiple of 8, or C).
+int mi_internal_layernorm(void *out, float *mean, float *rstd, const void *a, int64_t lda, const void *gamma, const void *beta,
+                          int64_t C, int64_t groups, float eps, void *stream) {
     if (!mi_ready()) return MI_ERROR_DEVICE;
     if (!out || !a) return MI_DECLINE_OPERANDS;
     if (C < 1 || C > INT32_MAX || groups < 0) return MI_DECLINE_EXTENT;
@@ -321,13 +328,15 @@ int mi_layernorm_f16(void *out, float *mean, float *rstd, const void *a, const v
     half_t *o = (half_t *)out;
     const half_t *x = (const half_t *)a, *g = (const half_t *)gamma, *b = (const half_t *)beta;
     const bool vec = C % 8 == 0 && aligned_to(a, 16) && aligned_to(out, 16) && (!g || aligned_to(g, 16)) && (!b || aligned_to(b, 16));
-    if (vec && C <= 512)       hipLaunchKernelGGL(layernorm_vec_kernel<1>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps);
-    else if (vec && C <= 1024) hipLaunchKernelGGL(layernorm_vec_kernel<2>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps);
-    else if (vec && C <= 2048) hipLaunchKernelGGL(layernorm_vec_kernel<4>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps);
-    else if (vec && C <= 4096) hipLaunchKernelGGL(layernorm_vec_kernel<8>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps);
-    else                       hipLaunchKernelGGL(layernorm_any_kernel, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps);
+    if (vec && C <= 512)       hipLaunchKernelGGL(layernorm_vec_kernel<1>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps, (long)lda);
+    else if (vec && C <= 1024) hipLaunchKernelGGL(layernorm_vec_kernel<2>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps, (long)lda);
+    else if (vec && C <= 2048) hipLaunchKernelGGL(layernorm_vec_kernel<4>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps, (long)lda);
+    else if (vec && C <= 4096) hipLaunchKernelGGL(layernorm_vec_kernel<8>, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps, (long)lda);
+    else                       hipLaunchKernelGGL(layernorm_any_kernel, grid, block, 0, st, o, mean, rstd, x, g, b, (int)C, (long)groups, eps, (long)lda);
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
 }
+
+extern "C" {
 
 int mi_softmax_f16(void *out, const void *a, int dtype, int64_t n, int64_t rows, float scale, void *stream) {
     if (!mi_ready()) return MI_ERROR_DEVICE;

@@ -84,3 +84,36 @@ def test_rows_of_every_depth_and_width(ctx, T, K, F):
             assert torch.equal(folded, apart)
         else:
             assert_parity(to_host(folded), to_host(apart), what=f"norm T{T} K{K} F{F}")
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 8])
+@pytest.mark.parametrize("K,F", [(8, 64), (64, 24), (72, 8192), (128, 8200), (136, 8), (512, 40), (768, 136), (776, 264), (1280, 72), (1280, 5120), (1288, 64)])
+def test_rows_against_kf_weights(ctx, T, K, F):
+    """[K][F] weights at the ends of the range that runs as 32 x 32 tiles: K of part of a stage, of one and of ten, one column tile and 256 of
+    them.  The rows lie apart in memory.  Error as in test_rows; the norm in front has the bits of the two calls."""
+    import torch
+    import juliavision_amd as jv
+    X, W, b = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K, F), 2), oracle.randn_f16((F,), 3, 0, 0.02)
+    R, g, beta = oracle.randn_f16((T, F), 4), oracle.randn_f16((K,), 5, 1.0, 0.1), oracle.randn_f16((K,), 6, 0, 0.1)
+    held = torch.full((T, K + 24), float("nan"), dtype=torch.float16, device="cuda")
+    dx = held[:, 8:8 + K]
+    dx.copy_(torch.from_numpy(X))
+    w, db = to_dev(W), to_dev(b)
+    new = lambda dt=torch.float16: poison(torch.empty((T, F), dtype=dt, device="cuda"))
+    for epi, res, dt in (("gelu", None, torch.float16), ("none", R, torch.float16), ("relu", None, torch.float32)):
+        out = new(dt)
+        ctx.ws.reset()
+        jv.matmul_(ctx, out, w, dx, db, epi=epi, residual=None if res is None else to_dev(res))
+        assert_parity(to_host(out), oracle.gemm_f16(X, W, b, epi=epi, residual=res), what=f"T{T} K{K} F{F} {epi}")
+    exact = X.astype(np.float64) @ W.astype(np.float64) + b.astype(np.float64)
+    out = new(torch.float32)
+    ctx.ws.reset()
+    jv.matmul_(ctx, out, w, dx, db)
+    assert np.linalg.norm(to_host(out) - exact) <= 2.0 ** -24 * max(8.0, np.sqrt(K)) * np.linalg.norm(exact)
+    h, folded, apart = torch.empty((T, K), dtype=torch.float16, device="cuda"), new(), new()
+    jv.layernorm_(ctx, h, None, None, dx.contiguous(), to_dev(g), to_dev(beta), K, 1e-5)
+    ctx.ws.reset()
+    jv.ln_matmul_(ctx, folded, w, dx, to_dev(g), to_dev(beta), 1e-5, db)
+    ctx.ws.reset()
+    jv.matmul_(ctx, apart, w, h, db)
+    assert torch.equal(folded, apart)
