@@ -38,12 +38,18 @@ namespace {
 // 23 x 300 x 64: 1.48e-7 | 1.45e-7 | 2.7e-4; 63 x 4000 x 64: 2.4e-7 | 2.0e-7 | 3.0e-4; 23 x 300 x 128: 1.66e-7 | 1.58e-7.  Only at head size
 // 72 it is larger, 1.57e-7 | 1.65e-7: there fp32 results stay with the rows kernel (fp16 ones are off by their rounding, 2.1e-4,
 // either way).
+// EARLY: a tile's V is read from LDS ahead of its exponentials, into registers that the others fill behind them, so that the wait for
+// the reads is none.  A wave needs 16 registers more at head size 64 and 24 at 72.  us, late | early: 6 heads x 1370 x 64 11.9 | 11.6, 12 x 4 x
+// 504 x 16 6.95 | 6.7, 2 x 16 x 5 x 3966 x 32 with padding 21.7 | 20.1 (with Q's wait out of the loop), 20 heads x 290 x 64 5.54 | 5.46.  Where the
+// registers cost a wave that the grid has, it is late: 16 x 3644 x 285 x 64 12.6 | 14.7, 5 x 20 x 1085 x 72 79 | 80.  Dense masks take
+// the registers for theirs: 16 x 4 x 77 x 128 6.2 | 6.6.
 // Waves a SIMD that the registers of an instance are budgeted for.
 enum TileMask { NO_MASK, KEYS, DENSE };
-constexpr int tile_waves(int EC, bool F32, int MASK) { return EC == 16 ? 2 : EC == 9 ? (F32 ? 2 : 3) : EC == 8 && F32 ? (MASK == DENSE ? 2 : 3) : MASK == DENSE ? 3 : 4; }
+constexpr bool tile_early(int EC, bool F32, int MASK) { return MASK != DENSE && (F32 || EC != 9); }
+constexpr int tile_waves(int EC, bool F32, int MASK, bool EARLY) { return EC == 8 && !F32 && EARLY ? 3 : EC == 16 ? 2 : EC == 9 ? (F32 ? 2 : 3) : EC == 8 && F32 ? (MASK == DENSE ? 2 : 3) : MASK == DENSE ? 3 : 4; }
 
-template <int EC, int NW, int MASK, bool F32>
-__global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile_kernel(SdpaArgs p) {
+template <int EC, int NW, int MASK, bool F32, bool EARLY = tile_early(EC, F32, MASK)>
+__global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK, EARLY)) void flash_tile_kernel(SdpaArgs p) {
     typedef std::conditional_t<F32, float, half_t> mask_t;
     static_assert(MASK != DENSE || F32, "calls with fp16 probabilities and such a mask run flash_fwd_kernel");
     constexpr int E = EC * 8, KS = (E + 15) / 16, ET = (E + 31) / 32;
@@ -136,6 +142,15 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
         const half8v t = as_half8(qraw[ks]);
 #pragma unroll
         for (int j = 0; j < 8; j++) qf[ks][j] = F32 ? t[j] : (half_t)((float)t[j] * c);
+    }
+    // (F32 does nothing to Q that would wait for it: left to its first use, in the loop, that wait is one for the next K in every turn)
+    if constexpr (F32 && MASK != DENSE) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            u32x4 w = __builtin_bit_cast(u32x4, qf[ks]);
+            asm volatile("" : "+v"(w));
+            qf[ks] = __builtin_bit_cast(half8v, w);
+        }
     }
     float16v o_acc[ET], negm;
 #pragma unroll
@@ -287,6 +302,22 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
         };
         if constexpr (F32) scale();
         else cut();
+        half8v vf[ET][2];
+        auto read_v = [&]() __attribute__((always_inline)) {
+            if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");        // V has landed; the next K may be on its way
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int t = 0; t < ET; t++)
+#pragma unroll
+                for (int bb = 0; bb < 2; bb++) {
+                    const char *vq = vt_lds + ((16 * bb + 4 * hl + vk) * EC + vchunk(t)) * 16 + (lane & 1) * 8;
+                    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)vq);
+                    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq + 8 * EC * 16));
+                    const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    vf[t][bb] = __builtin_bit_cast(half8v, both);
+                }
+        };
+        if constexpr (EARLY) read_v();                            // comes back under the exponentials
         half8v pf[2], lo[2];
         float l_new = l_run;
         probs(sc, pf, lo, l_new);
@@ -327,19 +358,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves(EC, F32, MASK)) void flash_tile
         }
         l_run = l_new;
         if constexpr (MASK == DENSE) { if (more) mask_take(); }
-        if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");        // V has landed; the next K may be on its way
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        half8v vf[ET][2];
-#pragma unroll
-        for (int t = 0; t < ET; t++)
-#pragma unroll
-            for (int bb = 0; bb < 2; bb++) {
-                const char *vq = vt_lds + ((16 * bb + 4 * hl + vk) * EC + vchunk(t)) * 16 + (lane & 1) * 8;
-                const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)vq);
-                const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(vq + 8 * EC * 16));
-                const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                vf[t][bb] = __builtin_bit_cast(half8v, both);
-            }
+        if constexpr (!EARLY) read_v();
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (more) request(false, tile + NW);
 #pragma unroll
@@ -411,28 +430,47 @@ constexpr int tile_lds_bytes() {
     constexpr int part = ((EC * 8 + 31) / 32 * 16 + 2) * 256, tiles = 2 * 32 * EC * 16;
     return NW * (part > tiles ? part : tiles);
 }
+template <int EC, int NW, int MASK, bool F32, bool EARLY>
+int launch_instance(const SdpaArgs &p, int lds, hipStream_t st) {
+    hipLaunchKernelGGL((flash_tile_kernel<EC, NW, MASK, F32, EARLY>), dim3((unsigned)(p.nqb * p.H * p.B)), dim3(NW * 64), lds, st, p);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+}
+template <int EC, int NW, int MASK, bool F32>
+int launch_tiles(const SdpaArgs &p, int lds, hipStream_t st) {
+    constexpr bool early = tile_early(EC, F32, MASK);
+    if constexpr (early && tile_waves(EC, F32, MASK, true) < tile_waves(EC, F32, MASK, false)) {
+        // as long as all waves of the grid find room at once (four SIMDs a CU)
+        if ((int64_t)p.nqb * p.H * p.B * NW > (int64_t)4 * tile_waves(EC, F32, MASK, true) * mi_num_cus()) return launch_instance<EC, NW, MASK, F32, false>(p, lds, st);
+    }
+    return launch_instance<EC, NW, MASK, F32, early>(p, lds, st);
+}
 template <int EC, int NW, bool F32>
 int launch_tiles(const SdpaArgs &p, TileMask mask, hipStream_t st) {
-    const dim3 grid((unsigned)(p.nqb * p.H * p.B));
     const int lds = tile_lds_bytes<EC, NW>();
-    if (mask == KEYS)       hipLaunchKernelGGL((flash_tile_kernel<EC, NW, KEYS, F32>), grid, dim3(NW * 64), lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st, p);
-    else if (mask == DENSE) {
-        if constexpr (F32) hipLaunchKernelGGL((flash_tile_kernel<EC, NW, DENSE, true>), grid, dim3(NW * 64), lds, st, p);
+    if (mask == KEYS) return launch_tiles<EC, NW, KEYS, F32>(p, lds + (int)ceil_div(p.Lk, 32) * 32 * (F32 ? 4 : 2), st);
+    if (mask == DENSE) {
+        if constexpr (F32) return launch_tiles<EC, NW, DENSE, true>(p, lds, st);
         else return MI_DECLINE_BIAS;
     }
-    else                    hipLaunchKernelGGL((flash_tile_kernel<EC, NW, NO_MASK, F32>), grid, dim3(NW * 64), lds, st, p);
-    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERROR_LAUNCH;
+    return launch_tiles<EC, NW, NO_MASK, F32>(p, lds, st);
 }
 template <int EC, bool F32>
 int launch_waves(const SdpaArgs &p, int waves, TileMask mask, hipStream_t st) {
     return waves == 2 ? launch_tiles<EC, 2, F32>(p, mask, st) : waves == 4 ? launch_tiles<EC, 4, F32>(p, mask, st) : launch_tiles<EC, 8, F32>(p, mask, st);
 }
+template <int EC, int NW, int MASK, bool F32>
+int raise_one(int lds) {
+    int bad = 0;
+    if constexpr (tile_early(EC, F32, MASK))
+        bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, MASK, F32, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess;
+    if constexpr (!tile_early(EC, F32, MASK) || tile_waves(EC, F32, MASK, true) < tile_waves(EC, F32, MASK, false))
+        bad |= hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, MASK, F32, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess;
+    return bad;
+}
 template <int EC, int NW, bool F32>
 int raise() {
     const int lds = tile_lds_bytes<EC, NW>();
-    return (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, KEYS, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds + (F32 ? 4 : 2) * MI_SDPA_TILE_KEYMASK_MAX) != hipSuccess) |
-           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, DENSE, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) |
-           (hipFuncSetAttribute(reinterpret_cast<const void *>(flash_tile_kernel<EC, NW, NO_MASK, F32>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess);
+    return raise_one<EC, NW, KEYS, F32>(lds + (F32 ? 4 : 2) * MI_SDPA_TILE_KEYMASK_MAX) | raise_one<EC, NW, DENSE, true>(lds) | raise_one<EC, NW, NO_MASK, F32>(lds);
 }
 template <int EC>
 int raise_all() { return raise<EC, 2, false>() | raise<EC, 4, false>() | raise<EC, 8, false>() | raise<EC, 2, true>() | raise<EC, 4, true>() | raise<EC, 8, true>(); }

@@ -143,3 +143,24 @@ def test_the_plan_names_the_kernel(ctx, B, H, Lq, Lk, E, mask, kernel):
     import juliavision_amd as jv
     q, k, v = (torch.zeros(B, H, L, E, dtype=torch.float16, device="cuda") for L in (Lq, Lk, Lk))
     assert jv.sdpaplan(ctx, q, k, v, q.new_zeros(B, 1, 1, Lk) if mask else None).kernel == kernel
+
+
+@pytest.mark.parametrize("B", [11, 24])
+@pytest.mark.parametrize("mask", [False, True])
+@pytest.mark.parametrize("Lk", [31, 70, 160])
+def test_grids_around_the_waves_that_fit(ctx, B, mask, Lk):
+    """Heads of 64 read V ahead of the exponentials while all waves of the grid fit the registers that takes (880 workgroups of two to four
+    waves here, and 1920), behind them past that.  Probabilities are rounded to fp16 (2^-11 of the result at most), the result once more."""
+    import torch
+    import juliavision_amd as jv
+    q, k, v = (to_dev(oracle.randn_f16((B, 16, L, 64), s, 0, 1.5)) for s, L in ((1, 160), (2, Lk), (3, Lk)))
+    bias = torch.zeros((B, 1, 1, Lk), dtype=torch.float16, device="cuda")
+    for b in range(B if mask else 0):
+        bias[b, ..., Lk - b % Lk:] = torch.finfo(torch.float16).min
+    out = torch.full((B, 16, 160, 64), float("nan"), dtype=torch.float16, device="cuda")
+    ctx.ws.reset()
+    jv.sdpa(ctx, q, k, v, bias if mask else None, None, out=out)
+    s = torch.matmul(q.float(), k.float().transpose(2, 3).contiguous()) / 8.0 + bias.float()
+    want = torch.matmul(torch.softmax(s, -1), v.float())
+    assert ((out.float() - want).norm() / want.norm()).item() <= 2.0 ** -10
+    assert_parity(to_host(out), want.cpu().numpy(), what=f"{B} x 16 heads, {Lk} keys")
