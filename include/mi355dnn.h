@@ -327,7 +327,7 @@ int mi_gemm_f16_plan_caps(const int64_t caps[6], const void *Y, const void *X, c
                           int w_layout, int out_dtype, int64_t nbatch, int64_t sY, int64_t sX, int64_t sW, int *ksplit_out);
 
 /* Which kernel mi_gemm_f16 runs for these extents on the current device (an mi_gemm_kernel), operands and results on 16 bytes with a
- * workspace of the size asked for; folded_norm: mi_lnfold_gemm_f16.  ksplit_out (optional): the slices of K, each on that
+ * workspace of the size asked for, no residual (one may move a call between WIDE and STAGED, which sum in one order); folded_norm: mi_lnfold_gemm_f16.  ksplit_out (optional): the slices of K, each on that
  * kernel.  Never launches, needs no GPU.  (The reference's plans name their kernels: matmul.jl:87-95.) */
 int mi_gemm_f16_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch, int epi, int folded_norm, int *ksplit_out);
 

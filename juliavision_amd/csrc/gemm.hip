@@ -858,6 +858,21 @@ TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_sp
     return e.plan;
 }
 
+// A second look at a call that was given one of the four-wave kernel's tiles.  Against them the 128 x 128 and 64 x 128 tiles are
+// estimated some 9 % too high, and a residual costs the four-wave kernel more: its stores then have no helper waves, and fetch.  The
+// tiles here sum K in one order, so the bits stay.  (Lowered for all calls, these estimates take some from the ring and cost stacks of
+// blocks 2 to 3 %.)  On 45 calls of 72 (M 690 to 7900, N 384 to 4096, K 256 to 2560, half with a residual) 0.94 of the time, 1.02 at worst:
+// 2012 x 1280 -> 1152 15.6 -> 14.0 us, with residual 17.4 -> 14.9; 2791 x 512 -> 4096 with residual 29.3 -> 24.6.
+int settled_tile(int tile, const GemmArgs &a, int64_t nbatch) {
+    if (tile > 1 || a.ag.x || a.K % 64 || a.lnf_stats || a.stats_out || a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH) return tile;
+    double best = 1e30;
+    for (int t = 0; t < 4; t++) {
+        const double us = tile_cost_us(a.M, a.N, a.K, nbatch, t, 1) * (t > 1 ? 0.91 : 1.0) + (t <= 1 && a.residual ? 2.0 : 0.0);
+        if (us < best) { best = us; tile = t; }
+    }
+    return tile;
+}
+
 // Workspace of a planned split: the planes, or the exchanged partials of the peer reduction (never less than the planes,
 // so a launch that cannot take the peer path -- a gathered operand -- falls back to planes in the same workspace).
 size_t plan_workspace_bytes(const TilePlan &tp, int64_t M, int64_t N) {
@@ -984,7 +999,7 @@ int run_gemm(GemmArgs a, bool b_kn, int64_t nbatch, void *ws, size_t ws_bytes, h
         // has its own: the bits are the ones without a GELU.
         if (pipe && split == 1 && !own_order(tp.tile, a.K) && (a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH))
             tp = plan_tiles(a.M, a.N, a.K, nbatch, false, true, deep, lnf);
-        if (pipe) return launch_tile(tp.tile, a, b_kn, nbatch, st);
+        if (pipe) return launch_tile(settled_tile(tp.tile, a, nbatch), a, b_kn, nbatch, st);
         return mi_any_launch(a, b_kn, true, nbatch, st);         // a single tile deep
     }
     return mi_any_launch(a, b_kn, false, nbatch, st);
@@ -1183,6 +1198,11 @@ int mi_gemm_f16_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch, int epi,
     if (tp.split == 1 && !own_order(tp.tile, K) && (epi == MI_EPI_GELU_ERF || epi == MI_EPI_GELU_TANH)) tp = plan_tiles(T, F, K, nbatch, false, true, true, lnf);
     if (ksplit_out) *ksplit_out = tp.split;
     if (tp.peer) return MI_GEMM_KERNEL_EXCHANGE;
+    if (tp.split == 1 && !lnf) {
+        GemmArgs a = {};
+        a.M = (int)T; a.N = (int)F; a.K = (int)K; a.epi = epi;
+        tp.tile = settled_tile(tp.tile, a, nbatch);
+    }
     switch (tp.tile) {
         case 0: case 1: return MI_GEMM_KERNEL_WIDE;
         case RING_TILE: return ceil_div(T, 64) * ceil_div(F, 64) * nbatch * tp.split <= mi_num_cus() ? MI_GEMM_KERNEL_RING : MI_GEMM_KERNEL_RING_SHALLOW;

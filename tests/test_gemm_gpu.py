@@ -546,3 +546,23 @@ def test_gelu_of_infinities_and_nan(ctx):
     torch.cuda.synchronize()
     got = to_host(out)
     assert np.isposinf(got[0]).all() and (got[1] == 0).all() and np.isnan(got[3]).all() and (got[4:] == 0).all()
+
+
+@pytest.mark.parametrize("layout", ["kf", "fk"])
+@pytest.mark.parametrize("T,K,F", [(2114, 1280, 1024), (2500, 512, 2048), (2642, 256, 3072), (1900, 192, 2568)])
+def test_a_residual_moves_no_bit_of_the_product(ctx, T, K, F, layout):
+    """A residual may move a call to another tile: it is still the product as it is without one, rounded, plus the residual, rounded."""
+    import torch
+    import juliavision_amd as jv
+    X, W = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K, F), 2)
+    w = to_dev(W) if layout == "kf" else to_dev(np.ascontiguousarray(W.T)).t()
+    x, b, r = to_dev(X), to_dev(oracle.randn_f16((F,), 3)), to_dev(oracle.randn_f16((T, F), 4))
+    plain, out = (poison(torch.empty((T, F), dtype=torch.float16, device="cuda")) for _ in range(2))
+    for epi in ("none", "relu"):
+        ctx.ws.reset()
+        jv.matmul_(ctx, plain, w, x, b, epi=epi)
+        ctx.ws.reset()
+        jv.matmul_(ctx, out, w, x, b, epi=epi, residual=r)
+        assert torch.equal(out, (plain.float() + r.float()).half())
+        rows = [0, 63, 64, 127, 128, T - 1]
+        assert_parity(to_host(plain)[rows], oracle.gemm_f16(X[rows], W, to_host(b), epi=epi), what=f"T{T} K{K} F{F} {epi} {layout}")

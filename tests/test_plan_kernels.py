@@ -43,6 +43,7 @@ def test_which_kernel_a_gemm_runs():
     for K in (520, 640, 768, 1152, 2304):
         assert kernel(500, K, 504) == "deep" and kernel(500, K, 520) == "ring"      # 256 tiles of 32 x 32, and more
     assert kernel(1500, 1280, 5120, "gelu") == "wide" and kernel(1544, 1288, 1288) == "staged" and kernel(1500, 5120, 1280) == "exchange"
+    assert kernel(2012, 1280, 1152) == kernel(2012, 1280, 1152, "relu") == "staged" and kernel(4510, 2048, 1280) == "wide"
     assert kernel(8, 1280, 1280) == kernel(100, 1284, 64) == "none" and kernel(100, 64, 64) == "one_tile"
     # a GELU moves a call only between tiles that sum K in one order
     for T, K, F in itertools.product((70, 300, 500, 1000, 1370, 3000), (384, 520, 1024, 1536, 2304), (64, 384, 520, 1536, 4096)):
