@@ -102,7 +102,7 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
     // the two sides of one meet the compiler waits for it, and the pieces of a chunk came one trip to memory after the other.
     // What does not exist -- outside the image, past the chunk or past Cin -- reads the tensor's first piece.
     auto patch_in = [&](const Piece &p, int c0) { return p.have && c0 + p.lim < a.Cin; };
-    auto weight_left = [&](const Piece &p, int c0) { return p.have ? min(t.kc, CRS - c0 * taps) - p.lim : 0; };
+    auto weight_left = [&](const Piece &p, int c0) { return p.have ? weight_end(t.kc, CRS, c0 * taps) - p.lim : 0; };
     auto patch_load = [&](const Piece &p, int c0) {
         u32x4 v = zero4;
         if (narrow) {
@@ -211,8 +211,8 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
     };
     const bool one = CHUNKS == 1 || (CHUNKS == 0 && t.nchunk == 1);
     if (one) {
-        // In batches of a few pieces a thread, each one trip to memory.  The pieces that the weight rows' ends cut are cut alike.
-        const int wgone = weight_back(t.kc % 8 ? t.kc % 8 : 8);
+        // In batches of a few pieces a thread, each one trip to memory.
+        const int wend = weight_end(t.kc, CRS, 0), wgone = weight_cut(wend);
         auto stage = [&](auto P_, auto W_) __attribute__((always_inline)) {
             constexpr int P1 = decltype(P_)::value, W1 = decltype(W_)::value;
             for (int d0 = 0, c0 = 0; d0 < t.patch_pieces || c0 < t.weight_pieces; d0 += NT * P1, c0 += NT * W1) {
@@ -235,8 +235,8 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
                     for (int i = 0; i < W1; i++) {
                         if (!short_w) {
                             const u32x4 cut = shifted(wv[i], wgone);
-                            wv[i] = wq[i].lim + 8 > t.kc ? cut : wv[i];
-                            wv[i] = wq[i].have ? wv[i] : zero4;
+                            wv[i] = wq[i].lim + 8 > wend ? cut : wv[i];
+                            wv[i] = wq[i].have && wq[i].lim < wend ? wv[i] : zero4;
                         }
                         if (c0 + tid + i * NT < t.weight_pieces) *weight_lds(0, wq[i].dst) = wv[i];
                     }

@@ -42,6 +42,10 @@ struct TilePlan {
 // the same row, as long as chunk and row have eight halves at all.
 constexpr bool weights_by_element(int kc, int CRS) { return kc < 8 || CRS < 8; }
 constexpr int weight_back(int left) { return left < 8 ? 8 - left : 0; }
+// Where the weights of the chunk from k0 of a row on end: a single chunk, too, may reach past Cin (29 to 31 channels are staged as 32).
+constexpr int weight_end(int kc, int CRS, int k0) { return kc < CRS - k0 ? kc : CRS - k0; }
+// All pieces that such an end cuts are cut alike: by so many halves the load of one was moved back.
+constexpr int weight_cut(int end) { return weight_back(end % 8 ? end % 8 : 8); }
 
 constexpr int LDS_MAX = 160 * 1024;
 

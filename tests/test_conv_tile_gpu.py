@@ -76,6 +76,35 @@ def test_operands_off_sixteen_bytes(ctx, Cin, H, W, Cout, k, s, p, off):
     assert bool(torch.isnan(flat[:off]).all()) and bool(torch.isnan(flat[off + want.size:]).all())
 
 
+@pytest.mark.parametrize("Cin,H,W,Cout,k", [
+    (29, 64, 64, 32, 3), (30, 64, 64, 32, 3), (31, 40, 33, 70, 3), (31, 24, 24, 64, 2),      # staged as 32 channels
+    (61, 20, 20, 32, 3), (62, 20, 20, 32, 3), (63, 20, 17, 33, 2),                           # as 64
+    (29, 64, 5, 32, 3), (31, 40, 7, 40, 3), (62, 40, 5, 33, 2),                              # image rows shorter than a piece
+])
+def test_a_single_chunk_past_the_channels(ctx, Cin, H, W, Cout, k):
+    """A chunk deeper than Cin: the weights that end inside a 16-byte piece, and the pieces behind them, which hold zeros whatever the tensor
+    begins with (an infinity of channel 0 reaches channel 0's results alone)."""
+    import ctypes as C
+
+    import torch
+    import juliavision_amd as jv
+    from juliavision_amd import _lib as L
+    p = k // 2
+    assert L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(W, H, Cin, 1, k, k, Cout, 1, 1, p, p, 1, 1, 1, C.byref(C.c_size_t(0)))] == "tile"
+    x, w, b = oracle.randn_f16((1, Cin, H, W), 1), oracle.randn_f16((Cout, Cin, k, k), 2, 0, 1.0 / np.sqrt(Cin * k * k)), oracle.randn_f16((Cout,), 3, 0, 0.5)
+    outs = []
+    for first in (w[0, 0, 0, 0], np.float16("inf")):
+        w[0, 0, 0, 0] = first
+        out = poison(torch.empty((1, Cout, H + 2 * p - k + 1, W + 2 * p - k + 1), dtype=torch.float16, device="cuda"))
+        ctx.ws.reset()
+        jv.convolution_(ctx, out, to_dev(x), to_dev(w), to_dev(b), (1, 1), (p, p), (1, 1), 1)
+        torch.cuda.synchronize()
+        if not outs:
+            assert_parity(to_host(out), oracle.conv2d_f16(x, w, b, (1, 1), (p, p), (1, 1), 1, False), what=f"conv {Cin},{H},{W}->{Cout} k{k}")
+        outs.append(to_host(out))
+    assert np.array_equal(outs[0][:, 1:], outs[1][:, 1:])
+
+
 @pytest.mark.parametrize("Cin", [3, 24])
 @pytest.mark.parametrize("OW", [1, 2, 3, 5, 6, 7, 18, 37])
 @pytest.mark.parametrize("Cout", [30, 33, 64])
