@@ -149,7 +149,9 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
     auto weight_lds = [&](int buf, int dst) { return reinterpret_cast<u32x4 *>(smem + t.weight_off + buf * t.stage_bytes + dst); };
 
     // The bias is asked for at once, of a single chunk here, of several behind their loop: a load behind a store is waited for
-    // together with the store's acknowledgement (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: a store of 20 300 clocks, 5200 so).
+    // together with the store's acknowledgement (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: a store of 20 300 clocks, 5200 so).  Four channels
+    // at a time, in tiles that end past Cout too: by channel their 64 loads and addresses took 3.5 us of 8 x 512 x 198 x 59 -> 96, 1 x 1 stride 2
+    // (56.2 -> 52.7).
     const int cl = 4 * (lane >> 5);                       // acc[i][4 g + e] of a lane is channel co0 + 32 i + 8 g + cl + e
     const bool all = co0 + CO <= a.Cout;                  // uniform
     half4v bias[TCO][4];
@@ -160,14 +162,24 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
             for (int i = 0; i < TCO; i++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) __builtin_memcpy(&bias[i][g], from + co0 + cl + 32 * i + 8 * g, 8);
+        } else if (a.Cout >= 4) {                         // moved back to end inside; `bias_of` shifts
+#pragma unroll
+            for (int i = 0; i < TCO; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) __builtin_memcpy(&bias[i][g], from + min(co0 + cl + 32 * i + 8 * g, a.Cout - 4), 8);
         } else {
 #pragma unroll
             for (int i = 0; i < TCO; i++)
 #pragma unroll
                 for (int g = 0; g < 4; g++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) bias[i][g][e] = from[min(co0 + 32 * i + 8 * g + cl + e, a.Cout - 1)];
+                    for (int e = 0; e < 4; e++) bias[i][g][e] = i + g == 0 ? from[min(e, a.Cout - 1)] : (half_t)0.0f;
         }
+    };
+    auto bias_of = [&](int i, int g) {
+        const int gone = co0 + 32 * i + 8 * g + cl - (a.Cout - 4);
+        if (all || a.Cout < 4) return bias[i][g];
+        return __builtin_bit_cast(half4v, __builtin_bit_cast(uint64_t, bias[i][g]) >> (gone > 0 ? 16 * (gone & 3) : 0));      // (past Cout, from four on, nothing is stored)
     };
     if (CHUNKS == 1) load_bias();
     float16v acc[TCO];
@@ -362,7 +374,11 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
 #pragma unroll
     for (int i = 0; i < TCO; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][r] += a.bias ? (float)bias[i][r / 4][r % 4] : 0.0f;
+        for (int g = 0; g < 4; g++) {
+            const half4v b = bias_of(i, g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][4 * g + e] += a.bias ? (float)b[e] : 0.0f;
+        }
     // Four lanes, four neighbouring pixels of a row, hold four channels each: they exchange, so that a lane stores four pixels of one
     // channel, eight bytes at any address (by pixel where the row ends between them).
     const int q = lane & 3, left = a.OW - (ox - q);       // pixels of the row from the four's first on

@@ -125,6 +125,21 @@ def test_rows_that_end_between_four_pixels(ctx, Cin, OW, Cout):
             assert_parity(to_host(out), want, what=f"Cin{Cin} OW{OW} Cout{Cout} {act}")
 
 
+@pytest.mark.parametrize("Cin,H,W,k", [(3, 20, 21, 3), (33, 20, 21, 3), (3, 20, 5, 3)])      # a chunk, several, by element
+@pytest.mark.parametrize("Cout", [1, 2, 3, 4, 5, 7, 34, 61, 96, 98, 131])
+def test_bias_of_every_channel(ctx, Cin, H, W, k, Cout):
+    """Weights of zero: each channel is its bias, to the bit, where Cout ends inside four channels, inside a tile and inside four of them."""
+    import torch
+    import juliavision_amd as jv
+    b = torch.arange(1, Cout + 2, dtype=torch.float16, device="cuda")
+    out = torch.full((1, Cout, H, W), float("nan"), dtype=torch.float16, device="cuda")
+    for bias in (b[1:], None):                             # at an odd address
+        ctx.ws.reset()
+        jv.convolution_(ctx, out, to_dev(oracle.randn_f16((1, Cin, H, W), 1)), torch.zeros((Cout, Cin, k, k), dtype=torch.float16, device="cuda"), bias,
+                        (1, 1), (1, 1), (1, 1), 1)
+        assert torch.equal(out, torch.zeros_like(out) if bias is None else bias.view(1, Cout, 1, 1).expand_as(out))
+
+
 @pytest.mark.parametrize("N,Cin,H,W,Cout,KH,KW,s,p,d,act", [
     (1, 16, 60, 60, 96, 9, 9, 4, 4, 1, "relu"),            # eight taps a stage, more than a row of them
     (1, 32, 23, 17, 65, 5, 5, (2, 1), (2, 0), (1, 2), "none"),
