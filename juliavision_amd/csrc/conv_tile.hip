@@ -354,12 +354,24 @@ __global__ __launch_bounds__(PW *KG * 64) void conv_tile_kernel(TileConv t) {
         }
         __syncthreads();
         if (kg > 0) return;
+        auto add = [&](int i, int g) __attribute__((always_inline)) {
 #pragma unroll
-        for (int g = 0; g < KG - 1; g++)
+            for (int r = 0; r < 16; r++) acc[i][r] += part[((g * TCO + i) * 16 + r) * (PW * 64) + pw * 64 + lane];
+        };
+        if constexpr (TCO > 2) {
 #pragma unroll
-            for (int i = 0; i < TCO; i++)
+            for (int i = 0; i < TCO; i++) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][r] += part[((g * TCO + i) * 16 + r) * (PW * 64) + pw * 64 + lane];
+                for (int g = 0; g < KG - 1; g++) add(i, g);
+                // left to the stores, behind their conditions, 192 parts waited in scratch memory (8 x 512 x 198 x 59 -> 96: 52.7 -> 41.4 us)
+                asm volatile("" : "+v"(acc[i]));
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+                for (int i = 0; i < TCO; i++) add(i, g);
+        }
     }
     if (CHUNKS != 1) load_bias();
     const int oy = oy0 + ly, ox = ox0 + lx;
