@@ -271,7 +271,9 @@ Route route_of(const ConvArgs &a) {
     // Patches that do not overlap: their matrix is no larger than the image, and past the K of a single chain (MI_LNA_KMAX) the image
     // and the tokens (mi_conv2d_tokens_f16) of a ViT's patch embedding keep the same bits.
     const bool apart = (a.KH - 1) * a.dy < a.sy && (a.KW - 1) * a.dx < a.sx;
-    if (mi_conv_tile_us(a) * (apart ? 1.25 : 1.03) < staged && !(apart && CRS > 512)) return {MI_CONV_KERNEL_TILE, 0};
+    const bool stageable = patch || PQP * CRSP <= INT32_MAX;      // (the matrix of a very large map is not)
+    const double tile = mi_conv_tile_us(a);
+    if (tile < 1e30 && (!stageable || (tile * (apart ? 1.25 : 1.03) < staged && !(apart && CRS > 512)))) return {MI_CONV_KERNEL_TILE, 0};
     if (patch) return {MI_CONV_KERNEL_PATCH_GEMM, patch_bytes};
     return {MI_CONV_KERNEL_IM2COL_GEMM, round_up((size_t)a.N * PQP * CRSP * 2, 256) + (CRSP != CRS ? round_up((size_t)a.Cout * CRSP * 2, 256) : 0) +
                                             mi_internal_gemm_workspace(a.Cout, CRSP, PQ, a.N)};
