@@ -254,7 +254,7 @@ void im2col_extents(const ConvArgs &a, int64_t &PQP, int64_t &CRSP) {
 
 // What runs, and the scratch it takes.  In one launch where that is estimated to be faster than staging the operand and multiplying
 // it: im2col writes at 0.8 to 1.1 MB/us, slower where it gathers with a stride (1024 x 1024 x 3 -> 144, 7 x 7 stride 4: 43 us
-// staged, 17 us in one launch); the channels-last copy and the weights of the patch form move at some 2 MB/us behind a launch.
+// staged, 15.1 us in one launch); the channels-last copy and the weights of the patch form move at some 2 MB/us behind a launch.
 struct Route { int kernel; size_t scratch; };
 Route route_of(const ConvArgs &a) {
     if (a.groups != 1) return {MI_CONV_KERNEL_DIRECT, 0};
@@ -268,12 +268,9 @@ Route route_of(const ConvArgs &a) {
     const double out_mb = 2e-6 * (double)a.N * a.Cout * PQ;
     const double staged = patch ? 5.9 + 0.5e-6 * (double)patch_bytes + mi_internal_patch_gemm_us(a.Cout, CRS, PQ, a.N) + 0.565 * out_mb
                                 : 2.55 + 0.876 * (3.0 + (a.sx == 1 ? 0.9e-6 : 1.25e-6) * 2.0 * (double)a.N * PQP * CRSP + mi_internal_gemm_us(a.Cout, CRSP, PQ, a.N)) + 0.107 * out_mb;
-    // Patches that do not overlap: their matrix is no larger than the image, and past the K of a single chain (MI_LNA_KMAX) the image
-    // and the tokens (mi_conv2d_tokens_f16) of a ViT's patch embedding keep the same bits.
-    const bool apart = (a.KH - 1) * a.dy < a.sy && (a.KW - 1) * a.dx < a.sx;
     const bool stageable = patch || PQP * CRSP <= INT32_MAX;      // (the matrix of a very large map is not)
     const double tile = mi_conv_tile_us(a);
-    if (tile < 1e30 && (!stageable || (tile * (apart ? 1.25 : 1.03) < staged && !(apart && CRS > 512)))) return {MI_CONV_KERNEL_TILE, 0};
+    if (tile < 1e30 && (tile < staged || !stageable)) return {MI_CONV_KERNEL_TILE, 0};
     if (patch) return {MI_CONV_KERNEL_PATCH_GEMM, patch_bytes};
     return {MI_CONV_KERNEL_IM2COL_GEMM, round_up((size_t)a.N * PQP * CRSP * 2, 256) + (CRSP != CRS ? round_up((size_t)a.Cout * CRSP * 2, 256) : 0) +
                                             mi_internal_gemm_workspace(a.Cout, CRSP, PQ, a.N)};

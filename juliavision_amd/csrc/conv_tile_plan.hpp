@@ -92,25 +92,40 @@ inline bool choose_chunk(TilePlan &t, const ConvShape &a, int co, int nt, int pa
 struct Shape { int pw, kg, tco; };
 constexpr Shape SHAPES[] = {{8, 1, 1}, {8, 1, 2}, {8, 1, 3}, {8, 1, 4}, {8, 1, 5}, {4, 1, 1}, {4, 1, 2}, {4, 1, 3}, {4, 1, 5}, {4, 2, 1}, {4, 2, 2}, {4, 2, 3}, {4, 2, 4}, {2, 4, 1}, {2, 4, 2}, {2, 4, 4}, {2, 2, 1}, {2, 2, 2}};
 
+// Patches that do not overlap: a patch embedding, a strided 1 x 1.
+inline bool patches_apart(const ConvShape &a) { return (a.KH - 1) * a.dy < a.sy && (a.KW - 1) * a.dx < a.sx; }
+// A patch embedding of channels off sixteen, no deeper than MI_LNA_KMAX: its image (mi_conv2d_f16) and its tokens (mi_conv2d_tokens_f16) have the
+// same bits there, those of one chain of sums in the order (ci, kh, kw), which the GEMM over the im2col matrix, unsplit, has either way.
+inline bool keeps_one_chain(const ConvShape &a) {
+    return a.KW == a.sx && a.KH == a.sy && a.px == 0 && a.py == 0 && a.dx == 1 && a.dy == 1 && a.Cin % 16 && (int64_t)a.Cin * a.KH * a.KW <= MI_LNA_KMAX;
+}
 
 // The workgroup shape with the lowest estimate (us), or false where no chunk fits.  Fitted to 130 convolutions in all 18 shapes
 // (2 x 2 to 7 x 7, strides 1, 2 and 4, 3 to 384 channels, 16 to 200 000 pixels): the choice is 3 % above the best shape on average.
-// With the staged routes' estimate (route_of) the choice between one launch and staging is 3.4 % above the best of all of them,
-// 32 % at worst (972 x 23 x 3 -> 96, 2 x 2: 7.4 us, 5.6 in another shape); one launch is the faster in 94 of the 130.
 // A chunk costs its trip to memory and its pieces, a step of a wave its eight gathers and its weight fragments; large outputs 0.1 us a megabyte.
+// Too few steps to split (fewer than two a group) go unsplit: 69 such maps take 0.987 of the time of the shape that is estimated lower.
+// A margin of 3 % goes to the staged routes (route_of; 1.00 to 1.06 choose alike): on 585 overlapping maps the choice between one launch and
+// staging is 1.3 % above the faster, 38 % at worst.
+// Patches apart leave little beside the image and the output, which narrow rectangles read and write a sliver of a line at a time, and share
+// lines across the dies: 4 / TW us a megabyte of output, all of it 1.1 times; past two workgroups a CU, or deeper than MI_LNA_KMAX in channels the
+// patch form takes, twice (2 x 2 over 256 x 256 x 256 -> 64: 45 us, staged 22.6).  844 of them,
+// 1 x 1 to 16 x 16: 1.3 % above the faster, 56 % at worst (1 x 768 x 467 x 73 -> 96, 1 x 1 stride 2: 25.4 us in one launch, 39.4 staged).
 inline bool choose(const ConvShape &a, int cus, TilePlan &t, Shape &best, double &best_us) {
     if ((int64_t)a.Cout * a.Cin * a.KH * a.KW > INT32_MAX / 2) return false;      // 32-bit offsets
+    const bool apart = patches_apart(a), one_chain = keeps_one_chain(a), deep = a.Cin % 16 == 0 && (int64_t)a.Cin * a.KH * a.KW > MI_LNA_KMAX;
     best_us = 1e30;
     TilePlan pick = {};
     for (const Shape &s : SHAPES) {
         TilePlan c = {};
         choose_rectangle(c, a, 32 * s.pw);
         if (!choose_chunk(c, a, 32 * s.tco, s.pw * s.kg * 64, (s.kg - 1) * s.tco * 16 * s.pw * 64 * 4)) continue;
-        if (s.kg > 1 && c.nchunk * c.ksteps < 2 * s.kg) continue;      // (too few steps to split: one chain of sums, as the GEMMs have)
+        if (s.kg > 1 && c.nchunk * c.ksteps < 2 * s.kg) continue;
         const int64_t wgs = (int64_t)c.tiles_x * c.tiles_y * ceil_div(a.Cout, 32 * s.tco) * a.N;
         const double rounds = (double)ceil_div(wgs, cus), steps = (double)c.nchunk * c.ksteps * s.pw / 4.0;
-        const double us = 4.9 + 0.1e-6 * 2.0 * (double)a.N * a.Cout * a.OH * a.OW + rounds * (0.3 + 0.147 * s.tco * s.pw + c.nchunk * (0.836 + 0.417e-3 * (c.patch_pieces + c.weight_pieces)) +
-                                          steps * (0.027 + 0.0096 * s.tco));
+        double us = 4.9 + (apart ? 4.0 / c.TW : 0.1) * 2e-6 * (double)a.N * a.Cout * a.OH * a.OW + rounds * (0.3 + 0.147 * s.tco * s.pw + c.nchunk * (0.836 + 0.417e-3 * (c.patch_pieces + c.weight_pieces)) +
+                                    steps * (0.027 + 0.0096 * s.tco));
+        us *= !apart ? 1.03 : wgs > 2 * cus || deep ? 2.0 : 1.1;
+        if (one_chain && (s.kg > 1 || (c.nchunk > 1 && c.kc % 16))) us += 1e6;
         if (us < best_us) { best_us = us; best = s; pick = c; }
     }
     if (best_us >= 1e30) return false;

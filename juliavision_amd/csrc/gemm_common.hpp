@@ -709,7 +709,6 @@ int mi_skinny_init();
 // gemm_pipe.hip: the register-staged pipelined kernel.  `tile` indexes TILE_MODELS (gemm.hip).
 int mi_pipe_launch(int tile, const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_pipe_launch_ln(bool wide, const GemmArgs &a, bool b_kn, hipStream_t st);
-constexpr int MI_LNA_KMAX = 512;         // deepest K of the layer-norm prologue
 int mi_pipe_init();
 // gemm_ring.hip: small grids of ordinary operands, and patch matrices of a convolution.
 int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);

@@ -110,6 +110,27 @@ def test_conv_writes_tokens_with_the_position_embedding(ctx, N, Cin, H, W, Cout,
     assert bool(torch.isnan(tok[:, 0]).all())                                         # row 0 of each image untouched
 
 
+@pytest.mark.parametrize("N,Cin,H,W,Cout,K", [(4, 3, 182, 262, 64, 4), (1, 5, 60, 64, 30, 3), (2, 1, 137, 173, 512, 8), (4, 3, 214, 244, 32, 7), (8, 24, 400, 390, 32, 4)])
+def test_a_patch_embedding_in_one_launch_has_the_bits_of_its_tokens(ctx, N, Cin, H, W, Cout, K):
+    """Up to 512 taps off sixteen channels the one-launch kernel keeps the GEMM's single chain of sums."""
+    import ctypes as C
+
+    import torch
+    import juliavision_amd as jv
+    from juliavision_amd import _lib as L
+    assert L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(W, H, Cin, N, K, K, Cout, K, K, 0, 0, 1, 1, 1, C.byref(C.c_size_t(0)))] == "tile"
+    x, w, b = to_dev(oracle.randn_f16((N, Cin, H, W), 41)), to_dev(oracle.randn_f16((Cout, Cin, K, K), 42, 0, 0.05)), to_dev(oracle.randn_f16((Cout,), 43, 0, 0.5))
+    OH, OW = H // K, W // K
+    ld = (Cout + 7) // 8 * 8
+    tok = torch.zeros((N, OH * OW, ld), dtype=torch.float16, device="cuda")[:, :, :Cout]
+    chan = poison(torch.empty((N, Cout, OH, OW), dtype=torch.float16, device="cuda"))
+    ctx.ws.reset()
+    jv.convolution_tokens_(ctx, tok, x, w, b, (K, K), (0, 0), (1, 1))
+    ctx.ws.reset()
+    jv.convolution_(ctx, chan, x, w, b, (K, K), (0, 0), (1, 1), 1)
+    assert torch.equal(chan.flatten(2).transpose(1, 2), tok)
+
+
 def test_conv_tokens_declines_misaligned_rows(ctx):
     import torch
     import juliavision_amd as jv
