@@ -204,8 +204,9 @@ int mi_gemm_f16_batched(void *Y, const void *X, const void *W, const void *bias,
  * partial planes in ws, a reducing epilogue (ws from mi_gemm_f16_workspace, which
  * is asked for whichever kernel runs); or, where that is estimated to be faster,
  * one launch of 32 x 32 tiles.
- * [F][K] weights: one launch, no workspace.  mi_gemm_f16 takes the same route
- * by itself for T <= 8; this entry forces it.
+ * [F][K] weights: one launch, no workspace, K up to 65536 at one row,
+ * 32768 at two, 16384 from three on (MI_DECLINE_EXTENT past it).  mi_gemm_f16 takes the
+ * same route by itself for T <= 8 ([F][K]: K <= 8192); this entry forces it.
  * The reference's counterpart is the fp32-only Lava.gemv! path
  * (matmul.jl:108-137) and mm_epilogue_kernel! (matmul.jl:192-217). */
 int mi_gemv_f16(void *Y, const void *X, const void *W, const void *bias, const void *residual,

@@ -608,10 +608,10 @@ void launch_few(const GemmArgs &a, hipStream_t st) {
     hipLaunchKernelGGL((few_rows_kernel<PF, TURNS, LN, false>), dim3((unsigned)wgs), dim3(512), 0, st, a, cols);
 }
 
-// by the 32-deep steps that each of the eight waves takes of K <= 8192
+// by the 32-deep steps that each of the eight waves takes: K <= 16 384, as the caller's bound on LDS says, behind a norm half of it
 int launch_few_k(const GemmArgs &a, hipStream_t st) {
     const int64_t per = ceil_div(ceil_div(a.K, 32), 8);
-    if (per > 32) return MI_DECLINE_EXTENT;
+    if (per > (a.ln_on ? 32 : 64)) return MI_DECLINE_EXTENT;
     if (a.ln_on) {
         if (per <= 2)       launch_few<2, 1, true>(a, st);
         else if (per <= 3)  launch_few<3, 1, true>(a, st);
@@ -637,7 +637,8 @@ int launch_few_k(const GemmArgs &a, hipStream_t st) {
         else if (per <= 16) launch_few<16, 1, false>(a, st);
         else if (per <= 20) launch_few<20, 1, false>(a, st);
         else if (per <= 24) launch_few<12, 2, false>(a, st);
-        else                launch_few<16, 2, false>(a, st);
+        else if (per <= 32) launch_few<16, 2, false>(a, st);
+        else                launch_few<16, 4, false>(a, st);
     }
     return MI_OK;
 }

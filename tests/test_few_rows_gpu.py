@@ -117,3 +117,24 @@ def test_rows_against_kf_weights(ctx, T, K, F):
     ctx.ws.reset()
     jv.matmul_(ctx, apart, w, h, db)
     assert torch.equal(folded, apart)
+
+
+@pytest.mark.parametrize("T,K,F,dt", [(5, 8200, 17, "f16"), (8, 12296, 40, "f16"), (6, 12544, 9, "f32"), (8, 16384, 24, "f32"), (4, 16384, 24, "f16")])
+def test_rows_of_the_deepest_k(ctx, T, K, F, dt):
+    """mi_gemv_f16 takes [F][K] weights as deep as eight rows' share of its bound on LDS lets through, 16 384, at every T; the kernel's
+    rounds end in each of the last two.  Error as in test_rows, and half a step of fp16 where the result is that.  Deeper is declined."""
+    import torch
+    from juliavision_amd import _lib as L
+    X, W, b = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((F, K), 2), oracle.randn_f16((F,), 3, 0, 0.02)
+    out = poison(torch.empty((T, F), dtype=torch.float16 if dt == "f16" else torch.float32, device="cuda"))
+    dx, dw, db = to_dev(X), to_dev(W), to_dev(b)
+
+    def gemv(k):
+        return ctx.lib.mi_gemv_f16(out.data_ptr(), dx.data_ptr(), dw.data_ptr(), db.data_ptr(), None, T, k, F, F, k, k, L.W_FK, L.BIAS_COL,
+                                   L.EPI["none"], L.F16 if dt == "f16" else L.F32, None, 0, ctx.stream)
+    assert gemv(16384 + 8) == L.DECLINE_EXTENT            # nothing is enqueued
+    assert gemv(K) == L.OK
+    torch.cuda.synchronize()
+    exact = X.astype(np.float64) @ W.astype(np.float64).T + b.astype(np.float64)
+    err = np.linalg.norm(to_host(out).astype(np.float64) - exact) / np.linalg.norm(exact)
+    assert err <= 2.0 ** -24 * np.sqrt(K) + (2.0 ** -11 if dt == "f16" else 0.0)
