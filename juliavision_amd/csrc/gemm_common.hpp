@@ -282,12 +282,13 @@ __device__ __forceinline__ void lnf_stats_wave(const GemmArgs &p, float2v *slot,
 // workgroup after its last read of the operand tiles.
 // The column bias of a wave's sub-tile, in the accumulator's order: cb[i][g] covers
 // n = n0 + wn*WTN + 32 i + 8 g + 4 (lane/32) .. +3.  Fetched by the kernels ahead of their last
-// k-step so that the epilogue does not start with a trip to memory.
+// k-step so that the epilogue does not start with a trip to memory; the choices are uniform, no load stands behind a condition
+// of its lane.  Four columns are one load at any address, moved back to end at N where they would pass it: a width off four then has
+// the quad that N ends in shifted, which settle_col_bias undoes where the bias is used.
 template <int TN, int WTN>
 __device__ __forceinline__ void load_col_bias(const GemmArgs &p, half4v (&cb)[TN][4], int n0, int wn, int lane, long bz) {
     const half4v z = {(half_t)0.0f, (half_t)0.0f, (half_t)0.0f, (half_t)0.0f};
-    const int nl = n0 + wn * WTN + 4 * (lane >> 5), last = p.N - 1;
-    // (uniform choices, and columns past the edge re-read the last ones: no load behind a condition of its lane)
+    const int nl = n0 + wn * WTN + 4 * (lane >> 5);
     if (p.bias_mode != MI_BIAS_COL) {
 #pragma unroll
         for (int i = 0; i < TN; i++)
@@ -296,19 +297,31 @@ __device__ __forceinline__ void load_col_bias(const GemmArgs &p, half4v (&cb)[TN
         return;
     }
     const half_t *bias = p.bias + bz * p.sBias;
-    if ((reinterpret_cast<uintptr_t>(bias) & 7) == 0 && p.N % 4 == 0) {
+    if (p.N >= 4) {
 #pragma unroll
         for (int i = 0; i < TN; i++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) cb[i][g] = *reinterpret_cast<const half4v *>(bias + min(nl + 32 * i + 8 * g, p.N - 4));
+            for (int g = 0; g < 4; g++) __builtin_memcpy(&cb[i][g], bias + min(nl + 32 * i + 8 * g, p.N - 4), 8);
     } else {
 #pragma unroll
         for (int i = 0; i < TN; i++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) cb[i][g][e] = bias[min(nl + 32 * i + 8 * g + e, last)];
+                for (int e = 0; e < 4; e++) cb[i][g][e] = bias[min(nl + 32 * i + 8 * g + e, p.N - 1)];
     }
+}
+// nw: the wave's first column.  Only a wave that N ends in has such a quad; quads past N reach nothing.
+template <int TN, int WTN>
+__device__ __forceinline__ void settle_col_bias(const GemmArgs &p, half4v (&cb)[TN][4], int nw, int lane) {
+    if (p.N % 4 == 0 || p.N < 4 || nw + WTN <= p.N) return;       // uniform
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int back = min(max(nw + 32 * i + 8 * g + 4 * (lane >> 5) + 4 - p.N, 0), 3);
+            cb[i][g] = __builtin_bit_cast(half4v, __builtin_bit_cast(uint64_t, cb[i][g]) >> (16 * back));
+        }
 }
 
 // What the store of a folded layer norm carries (by value, so that it stays in registers): (r, r mu) of the lane's rows
@@ -344,7 +357,7 @@ struct LnFoldRegs {
     __device__ __forceinline__ float4v biasp(int i, int g, int, int) const { return b[i][g]; }
 };
 template <int EPI, int TM, int TN, int WTM, int WTN, int NWAVES, int LDS_BYTES, typename LN>
-__device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&cb)[TN][4], char *smem, int m0, int n0, int wm, int wn,
+__device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc)[TN][TM], const half4v (&loaded)[TN][4], char *smem, int m0, int n0, int wm, int wn,
                                                int wave, int lane, long bz, const LN &ln) {
     const int frow = lane & 31;
     const half_t *bias = p.bias ? p.bias + bz * p.sBias : nullptr;
@@ -354,6 +367,12 @@ __device__ __forceinline__ void store_tile_epi(const GemmArgs &p, float16v (&acc
     static_assert(STAGE_BYTES * NWAVES <= LDS_BYTES, "epilogue staging exceeds the operand LDS");
     char *stage = smem + wave * STAGE_BYTES;
     const int hl = lane >> 5;
+    half4v cb[TN][4];
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) cb[i][g] = loaded[i][g];
+    settle_col_bias<TN, WTN>(p, cb, n0 + wn * WTN, lane);
     // Row biases for all of the wave's rows before the first store (store_tile_simple says why).
     float brow_j[TM];
 #pragma unroll

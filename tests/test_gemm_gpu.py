@@ -566,3 +566,26 @@ def test_a_residual_moves_no_bit_of_the_product(ctx, T, K, F, layout):
         assert torch.equal(out, (plain.float() + r.float()).half())
         rows = [0, 63, 64, 127, 128, T - 1]
         assert_parity(to_host(plain)[rows], oracle.gemm_f16(X[rows], W, to_host(b), epi=epi), what=f"T{T} K{K} F{F} {epi} {layout}")
+
+
+@pytest.mark.parametrize("out_f32", [False, True])
+@pytest.mark.parametrize("T,K,runs", [(40, 64, "one_tile"), (70, 520, "deep"), (600, 640, "ring"), (1500, 256, "staged"), (3000, 1280, "wide")])
+def test_column_bias_of_any_width_at_any_address(ctx, T, K, runs, out_f32):
+    """A column bias is loaded by fours, the last four moved back to end with it: widths either side of a quad, of a tile's 32 columns and of
+    its edge, narrower than a quad, at addresses off the load's size, through each kernel.  The product is zero: the bias itself is the result."""
+    import torch
+    import juliavision_amd as jv
+    from juliavision_amd import _lib as L
+    base = {"one_tile": 64, "deep": 96, "ring": 640, "staged": 1024, "wide": 2560}[runs]
+    if runs != "staged":
+        assert L.GEMM_KERNELS[L.load().mi_gemm_f16_kernel(T, K, base, 1, L.EPI["none"], 0, None)] == runs
+    x = torch.zeros((T, K), dtype=torch.float16, device="cuda")
+    w = torch.ones((base + 40, K), dtype=torch.float16, device="cuda")
+    held = torch.arange(1, base + 49, dtype=torch.float32, device="cuda").remainder_(1021).half()
+    for F in [f for f in (1, 2, 3, 4, 5, 6, 7) if runs in ("one_tile", "deep")] + [base - 31, base - 2, base - 1, base, base + 1, base + 2, base + 3, base + 30, base + 33]:
+        for off in (0, 1, 3):
+            b = held[off:off + F]
+            out = poison(torch.empty((T, F), dtype=torch.float32 if out_f32 else torch.float16, device="cuda"))
+            ctx.ws.reset()
+            jv.matmul_(ctx, out, w[:F].t(), x, b)
+            assert torch.equal(out, b.to(out.dtype).expand(T, F)), (F, off)
