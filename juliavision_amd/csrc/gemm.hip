@@ -859,15 +859,28 @@ TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_sp
 }
 
 // A second look at a call that was given one of the four-wave kernel's tiles.  Against them the 128 x 128 and 64 x 128 tiles are
-// estimated some 9 % too high, and a residual costs the four-wave kernel more: its stores then have no helper waves, and fetch.  The
+// estimated too high, and a residual costs the four-wave kernel more: its stores then have no helper waves, and fetch.  The
 // tiles here sum K in one order, so the bits stay.  (Lowered for all calls, these estimates take some from the ring and cost stacks of
-// blocks 2 to 3 %.)  On 45 calls of 72 (M 690 to 7900, N 384 to 4096, K 256 to 2560, half with a residual) 0.94 of the time, 1.02 at worst:
-// 2012 x 1280 -> 1152 15.6 -> 14.0 us, with residual 17.4 -> 14.9; 2791 x 512 -> 4096 with residual 29.3 -> 24.6.
+// blocks 2 to 3 %.)  2012 x 1280 -> 1152 15.6 -> 14.0 us, with residual 17.4 -> 14.9; 2791 x 512 -> 4096 with residual 29.3 -> 24.6.
+//
+// By how much too high: 9 % from K = 256 to 1023, and with a residual below that too (85 calls with one 0.72 to 0.97 of the four-wave
+// tiles' time).  Without one the 128 x 128 tiles are as good as estimated at K = 128 and 192 (35 calls that 9 % moved were 1 to 9 % slower:
+// 4525 x 192 -> 1688 9.7 -> 10.5 us, 1808 x 128 -> 3952 9.3 -> 9.95), the 64 x 128 ones lower (24 calls 0.82 to 0.95).  From K = 1024 on
+// only the 128 x 128 tiles of at most one workgroup a CU are (0.85 to 1.0, one in ten 1.02 to 1.08; with residual 0.81 to 1.0): the others
+// are taken where those pass 256 or 512 by a few (1571 x 1024 -> 2544 15.0 -> 16.0, 3379 x 2048 -> 2360 44 -> 49, with residual 47 -> 52).
+double estimated_high(int tile, const GemmArgs &a, int64_t wgs) {
+    const bool residual = a.residual != nullptr;
+    if (tile <= 1) return 1.0;
+    if (a.K >= 1024) return tile == 2 && wgs <= mi_num_cus() ? (residual ? 0.91 : 0.93) : 1.0;
+    return residual || a.K >= 256 ? 0.91 : tile == 2 ? 0.97 : 0.92;
+}
 int settled_tile(int tile, const GemmArgs &a, int64_t nbatch) {
     if (tile > 1 || a.ag.x || a.K % 64 || a.lnf_stats || a.stats_out || a.epi == MI_EPI_GELU_ERF || a.epi == MI_EPI_GELU_TANH) return tile;
     double best = 1e30;
     for (int t = 0; t < 4; t++) {
-        const double us = tile_cost_us(a.M, a.N, a.K, nbatch, t, 1) * (t > 1 ? 0.91 : 1.0) + (t <= 1 && a.residual ? 2.0 : 0.0);
+        const int64_t wgs = ceil_div(a.M, TILE_MODELS[t].bm) * ceil_div(a.N, TILE_MODELS[t].bn) * nbatch;
+        if (t > 1 && a.K >= 1024 && wgs > 2 * mi_num_cus()) continue;      // (nor does a residual make up for theirs)
+        const double us = tile_cost_us(a.M, a.N, a.K, nbatch, t, 1) * estimated_high(t, a, wgs) + (t <= 1 && a.residual ? 2.0 : 0.0);
         if (us < best) { best = us; tile = t; }
     }
     return tile;

@@ -44,6 +44,9 @@ def test_which_kernel_a_gemm_runs():
         assert kernel(500, K, 504) == "deep" and kernel(500, K, 520) == "ring"      # 256 tiles of 32 x 32, and more
     assert kernel(1500, 1280, 5120, "gelu") == "wide" and kernel(1544, 1288, 1288) == "staged" and kernel(1500, 5120, 1280) == "exchange"
     assert kernel(2012, 1280, 1152) == kernel(2012, 1280, 1152, "relu") == "staged" and kernel(4510, 2048, 1280) == "wide"
+    # past the four-wave tiles' first choice: narrow ones at K of two and three tiles, square ones at a long K
+    assert kernel(6637, 128, 1360) == kernel(7310, 192, 1304) == kernel(3399, 256, 2312) == kernel(3376, 2560, 624) == "staged"
+    assert kernel(1808, 128, 3952) == kernel(2447, 128, 2816) == kernel(4525, 192, 1688) == kernel(1571, 1024, 2544) == "wide"
     assert kernel(8, 1280, 1280) == kernel(100, 1284, 64) == "none" and kernel(100, 64, 64) == "one_tile"
     # a GELU moves a call only between tiles that sum K in one order
     for T, K, F in itertools.product((70, 300, 500, 1000, 1370, 3000), (384, 520, 1024, 1536, 2304), (64, 384, 520, 1536, 4096)):
