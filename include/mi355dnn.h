@@ -321,7 +321,7 @@ int mi_gemm_f16_plan(const void *Y, const void *X, const void *W,
 /* mi_gemm_f16_plan for a device the caller describes: caps are the six values of mi_device_caps (NULL: the current
  * device), of which the planner reads [0] (matrix unit present; without it the tiled MFMA path is not offered) and
  * [5] (compute units, which decide tiles and K-splits).  ksplit_out (optional) receives the number of K-slices the
- * plan would use.  The reference's planners take a DeviceCaps value for the same purpose: tests ask about hardware
+ * plan would use; up to eight rows against [K][F] weights: 1 where they run as 32 x 32 tiles (mi_gemv_f16).  The reference's planners take a DeviceCaps value for the same purpose: tests ask about hardware
  * they do not have (DNNKernels/test/test_flash.jl:328,363,373-377; context.jl:68).  Never launches, needs no GPU. */
 int mi_gemm_f16_plan_caps(const int64_t caps[6], const void *Y, const void *X, const void *W,
                           int64_t T, int64_t K, int64_t F, int64_t ldY, int64_t ldX, int64_t ldW,
@@ -432,6 +432,12 @@ int mi_conv2d_f16_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
                          int64_t KW, int64_t KH, int64_t Cout,
                          int64_t stride_x, int64_t stride_y, int64_t pad_x, int64_t pad_y,
                          int64_t dil_x, int64_t dil_y, int64_t groups, size_t *scratch_out);
+/* Which kernel gathers the patches where that is MI_CONV_KERNEL_PATCH_GEMM: MI_GEMM_KERNEL_DEEP, _RING or _RING_SHALLOW
+ * (an mi_gemm_kernel); MI_GEMM_KERNEL_NONE for the other routes. */
+int mi_conv2d_f16_patch_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N,
+                               int64_t KW, int64_t KH, int64_t Cout,
+                               int64_t stride_x, int64_t stride_y, int64_t pad_x, int64_t pad_y,
+                               int64_t dil_x, int64_t dil_y, int64_t groups);
 /* The same convolution over channels-last tensors: x [N][H][W][Cin], w [Cout][KH][KW][Cin], out [N][OH][OW][Cout]
  * (groups = 1).  An implicit GEMM with nothing staged: out[(n,oh,ow)][Cout] = patch . w^T, the patch matrix gathered
  * from x by the GEMM's own operand loads, the weights read as they lie; split-K planes in ws where the output tiles

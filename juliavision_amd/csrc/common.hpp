@@ -206,4 +206,5 @@ size_t mi_internal_gemm_workspace(int64_t T, int64_t K, int64_t F, int64_t nbatc
 // What such a call is estimated to take, in microseconds.
 int mi_internal_layernorm(void *out, float *mean, float *rstd, const void *a, int64_t lda, const void *gamma, const void *beta, int64_t C, int64_t groups, float eps, void *stream);
 double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);      // B a ConvGather: on the kernel that is estimated to be faster
+int mi_internal_patch_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch);          // that kernel: an mi_gemm_kernel
 double mi_internal_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch);

@@ -322,6 +322,14 @@ int mi_conv2d_f16_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, int64_t
     return r.kernel;
 }
 
+int mi_conv2d_f16_patch_kernel(int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, int64_t KW, int64_t KH, int64_t Cout,
+                               int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy, int64_t groups) {
+    ConvArgs a;
+    if (fill(a, nullptr, nullptr, nullptr, nullptr, Wi, Hi, Cin, N, KW, KH, Cout, sx, sy, px, py, dx, dy, groups, MI_EPI_NONE) != MI_OK) return MI_GEMM_KERNEL_NONE;
+    if (route_of(a).kernel != MI_CONV_KERNEL_PATCH_GEMM) return MI_GEMM_KERNEL_NONE;
+    return mi_internal_patch_kernel(a.Cout, (int64_t)a.Cin * a.KH * a.KW, (int64_t)a.OW * a.OH, a.N);
+}
+
 int mi_conv2d_f16(void *out, const void *x, const void *w, const void *bias,
                   int64_t Wi, int64_t Hi, int64_t Cin, int64_t N, int64_t KW, int64_t KH, int64_t Cout,
                   int64_t sx, int64_t sy, int64_t px, int64_t py, int64_t dx, int64_t dy, int64_t groups, int act,

@@ -1045,6 +1045,10 @@ static bool patches_deep(int64_t T, int64_t K, int64_t F, int64_t nbatch) {
            tile_cost_us(T, F, K, nbatch, DEEP_TILE, 1) < tile_cost_us(T, F, K, nbatch, RING_TILE, 1);
 }
 double mi_internal_patch_gemm_us(int64_t T, int64_t K, int64_t F, int64_t nbatch) { return tile_cost_us(T, F, K, nbatch, patches_deep(T, K, F, nbatch) ? DEEP_TILE : RING_TILE, 1); }
+int mi_internal_patch_kernel(int64_t T, int64_t K, int64_t F, int64_t nbatch) {
+    if (patches_deep(T, K, F, nbatch)) return MI_GEMM_KERNEL_DEEP;
+    return ceil_div(T, 64) * ceil_div(F, 64) * nbatch <= mi_num_cus() ? MI_GEMM_KERNEL_RING : MI_GEMM_KERNEL_RING_SHALLOW;
+}
 double mi_deep_us(int64_t T, int64_t K, int64_t F) {
     return ceil_div(T, 32) * ceil_div(F, 32) <= std::min(DEEP_WGS, (int64_t)mi_num_cus()) ? tile_cost_us(T, F, K, 1, DEEP_TILE, 1) : 1e30;
 }
@@ -1196,7 +1200,7 @@ int mi_gemm_f16_plan_caps(const int64_t caps[6], const void *Y, const void *X, c
     if (ksplit_out) {
         *ksplit_out = 1;
         if (path == MI_GEMM_MFMA && K % 64 == 0 && K >= 128) *ksplit_out = plan_tiles(T, F, K, nbatch < 1 ? 1 : nbatch, true).split;
-        if (path == MI_GEMM_SKINNY && w_layout == MI_W_KF) *ksplit_out = mi_skinny_splits(K, F);
+        if (path == MI_GEMM_SKINNY && w_layout == MI_W_KF) *ksplit_out = mi_skinny_slices(T, K, F, ldX, ldW);
     }
     mi_plan_caps_end();
     return path;

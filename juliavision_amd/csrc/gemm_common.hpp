@@ -723,6 +723,7 @@ constexpr size_t SKINNY_FK_LDS_MAX = 128 * 1024;    // activations of the [F][K]
 // Up to eight rows; `ws`: the fp32 planes of mi_skinny_splits K-slices ([K][F] weights only).
 int mi_skinny_launch(const GemmArgs &a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st);
 int mi_skinny_splits(int64_t K, int64_t F);
+int mi_skinny_slices(int64_t T, int64_t K, int64_t F, int64_t ldA, int64_t ldB);      // those that run: one where the call goes to 32 x 32 tiles
 double mi_deep_us(int64_t T, int64_t K, int64_t F);      // gemm.hip's estimate of gemm_deep_kernel, at most one workgroup a CU; infinite otherwise
 int mi_skinny_init();
 // gemm_pipe.hip: the register-staged pipelined kernel.  `tile` indexes TILE_MODELS (gemm.hip).
@@ -733,6 +734,7 @@ int mi_pipe_init();
 int mi_ring_launch(const GemmArgs &a, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_ring_init();
 // gemm_deep.hip: few output tiles, of ordinary operands (split_k: K over its waves) and of patch matrices (always).
+bool mi_deep_takes(int64_t ldA, int64_t ldB);      // the pitches of ordinary operands
 int mi_deep_launch(const GemmArgs &a, bool split_k, bool b_kn, int64_t nbatch, hipStream_t st);
 int mi_deep_init();
 // gemm_any.hip: the kernels for operands and extents that the others do not take.

@@ -312,6 +312,9 @@ int raise_deep() { return raise_lds(gemm_deep_kernel<NW, CHAINS, true>, DEEP_LDS
 
 }  // namespace
 
+// per-lane load offsets are 32-bit byte offsets from the tile's origin
+bool mi_deep_takes(int64_t ldA, int64_t ldB) { return 32 * ldA * 2 < (1ll << 31) && 128 * ldB * 2 < (1ll << 31); }
+
 int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch, hipStream_t st) {
     GemmArgs a = args;
     set_tiles(a, 32, 32);
@@ -320,8 +323,7 @@ int mi_deep_launch(const GemmArgs &args, bool split_k, bool b_kn, int64_t nbatch
         if (b_kn || a.cv.img > MI_PATCH_IMAGE_MAX || (int64_t)32 * a.ldA * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
         return a.K > 4096 ? launch_deep_patches<4>(a, nbatch, st) : launch_deep_patches<2>(a, nbatch, st);
     }
-    // per-lane load offsets are 32-bit byte offsets from the tile's origin
-    if ((int64_t)32 * a.ldA * 2 >= (1ll << 31) || (int64_t)128 * a.ldB * 2 >= (1ll << 31)) return MI_DECLINE_EXTENT;
+    if (!mi_deep_takes(a.ldA, a.ldB)) return MI_DECLINE_EXTENT;
     // Past K = 4096 such calls had twelve to twenty chains, as slices of K on the ring; short of it eight are as good as what they had, and
     // the second pair of accumulators costs 0.05 to 0.1 us (50 x 3224 -> 992 6.67 | 6.75).
     // Up to eight rows replace K-slices of [K][F] weights, whose error eight chains exceed from K = 1280 on (9.4e-8 | 9.7e-8, sixteen 8.3e-8).

@@ -695,20 +695,24 @@ void launch_fk_k(const GemmArgs &a, hipStream_t st) {
 
 int mi_skinny_splits(int64_t K, int64_t F) { return (int)ceil_div(K, skinny_kper(K, F)); }
 
+static size_t planes_bytes(int64_t T, int64_t K, int64_t F) { return (size_t)mi_skinny_splits(K, F) * T * F * sizeof(float); }
+int mi_skinny_slices(int64_t T, int64_t K, int64_t F, int64_t ldA, int64_t ldB) {
+    return mi_deep_takes(ldA, ldB) && kn_on_tiles(T, K, F, planes_bytes(T, K, F)) ? 1 : mi_skinny_splits(K, F);
+}
+
 int mi_skinny_launch(const GemmArgs &a, bool b_kn, void *ws, size_t ws_bytes, hipStream_t st) {
     if (b_kn) {
         const int kper = skinny_kper(a.K, a.N), nsplit = (int)ceil_div(a.K, kper);
-        size_t need = (size_t)nsplit * a.M * a.N * sizeof(float);
+        const size_t need = planes_bytes(a.M, a.K, a.N);
         if (!ws || ws_bytes < need || !aligned_to(ws, 256)) return MI_DECLINE_WORKSPACE;
-        if (kn_on_tiles(a.M, a.K, a.N, need)) {
+        if (mi_deep_takes(a.ln_on ? a.K : a.ldA, a.ldB) && kn_on_tiles(a.M, a.K, a.N, need)) {
             GemmArgs t = a;
             if (a.ln_on) {
                 t.ln_on = 0; t.A = reinterpret_cast<const half_t *>(ws); t.ldA = a.K;
                 const int rc = mi_internal_layernorm(ws, nullptr, nullptr, a.A, a.ldA, a.ln_gamma, a.ln_beta, a.K, a.M, a.ln_eps, st);
                 if (rc != MI_OK) return rc;
             }
-            const int rc = mi_deep_launch(t, true, true, 1, st);
-            if (rc != MI_DECLINE_EXTENT) return rc;      // declined: a row pitch beyond its 32-bit offsets
+            return mi_deep_launch(t, true, true, 1, st);
         }
         float *part = reinterpret_cast<float *>(ws);
         dim3 grid((unsigned)ceil_div(a.N, SKN_COLS), (unsigned)nsplit);

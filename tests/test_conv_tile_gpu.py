@@ -166,6 +166,7 @@ def test_patches_of_few_tiles(ctx, N, Cin, H, W, Cout, KH, KW, s, p, d, act):
     pair = lambda v: v if isinstance(v, tuple) else (v, v)
     s, p, d = pair(s), pair(p), pair(d)                    # (x, y)
     assert L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(W, H, Cin, N, KW, KH, Cout, *s, *p, *d, 1, C.byref(C.c_size_t(0)))] == "patch_gemm"
+    assert L.GEMM_KERNELS[L.load().mi_conv2d_f16_patch_kernel(W, H, Cin, N, KW, KH, Cout, *s, *p, *d, 1)] == "deep"
     x, w = oracle.randn_f16((N, Cin, H, W), 1), oracle.randn_f16((Cout, Cin, KH, KW), 2, 0, 1.0 / np.sqrt(Cin * KH * KW))
     b = oracle.randn_f16((Cout,), 3, 0, 0.5)
     want = torch.nn.functional.conv2d(*(torch.from_numpy(a).double() for a in (x, w, b)), s[::-1], p[::-1], d[::-1]).numpy()

@@ -90,9 +90,16 @@ def test_rows_of_every_depth_and_width(ctx, T, K, F):
 @pytest.mark.parametrize("K,F", [(8, 64), (64, 24), (72, 8192), (128, 8200), (136, 8), (512, 40), (768, 136), (776, 264), (1280, 72), (1280, 5120), (1288, 64)])
 def test_rows_against_kf_weights(ctx, T, K, F):
     """[K][F] weights at the ends of the range that runs as 32 x 32 tiles: K of part of a stage, of one and of ten, one column tile and 256 of
-    them.  The rows lie apart in memory.  Error as in test_rows; the norm in front has the bits of the two calls."""
+    them; one past each end as slices of K.  The rows lie apart in memory.  Error as in test_rows; the norm in front has the bits of the two calls."""
+    import ctypes as C
+
     import torch
     import juliavision_amd as jv
+    from juliavision_amd import _lib as L
+    slices = C.c_int(0)
+    ctx.lib.mi_gemm_f16_plan_caps(None, 0x10000, 0x20000, 0x30000, T, K, F, F, K + 24, F, L.W_KF, L.F16, 1, 0, 0, 0, C.byref(slices))
+    sliced = K > (768 if T <= 2 else 1280) or F > 8192 or (K, F) == (136, 8)      # (the last: no room for the rows behind a norm)
+    assert (slices.value == 1) == (not sliced)
     X, W, b = oracle.randn_f16((T, K), 1, 0, 1.0 / np.sqrt(K)), oracle.randn_f16((K, F), 2), oracle.randn_f16((F,), 3, 0, 0.02)
     R, g, beta = oracle.randn_f16((T, F), 4), oracle.randn_f16((K,), 5, 1.0, 0.1), oracle.randn_f16((K,), 6, 0, 0.1)
     held = torch.full((T, K + 24), float("nan"), dtype=torch.float16, device="cuda")

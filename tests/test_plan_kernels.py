@@ -56,6 +56,28 @@ def test_which_kernel_a_gemm_runs():
             assert (plain in own) == (gelu in own) and (plain not in own or plain == gelu), (T, K, F)
 
 
+def test_how_rows_against_kf_weights_are_cut():
+    """One slice of K where they run as 32 x 32 tiles, which ask for row pitches below 2^31 bytes a tile."""
+    slices = C.c_int(0)
+
+    def cut(T, K, F, ldX=None, ldW=None):
+        assert L.GEMM_PATHS[L.load().mi_gemm_f16_plan_caps(None, PTR, PTR, PTR, T, K, F, F, ldX or K, ldW or F, L.W_KF, L.F16, 1, 0, 0, 0, C.byref(slices))] == "skinny"
+        return slices.value
+    assert cut(1, 384, 1536) == cut(8, 1280, 5120) == cut(2, 768, 768) == 1
+    assert cut(1, 776, 768) > 1 and cut(8, 1288, 5120) > 1 and cut(4, 128, 8200) > 1
+    assert cut(1, 384, 1536, ldX=2 ** 25 - 8, ldW=2 ** 23 - 8) == 1 and cut(1, 384, 1536, ldX=2 ** 25) > 1 and cut(1, 384, 1536, ldW=2 ** 23) > 1
+
+
+def test_which_kernel_gathers_patches():
+    def kernel(H, W, Cin, Cout, k, s=1, groups=1):
+        args = (W, H, Cin, 1, k, k, Cout, s, s, k // 2, k // 2, 1, 1, groups)
+        conv, gemm = L.CONV_KERNELS[L.load().mi_conv2d_f16_kernel(*args, None)], L.GEMM_KERNELS[L.load().mi_conv2d_f16_patch_kernel(*args)]
+        assert (gemm == "none") == (conv != "patch_gemm")
+        return gemm
+    assert kernel(22, 23, 96, 96, 5) == "deep" and kernel(64, 64, 256, 256, 3) == "ring" and kernel(128, 128, 256, 256, 3) == "ring_shallow"
+    assert kernel(64, 64, 256, 256, 1) == kernel(64, 64, 256, 256, 3, groups=4) == kernel(1024, 1024, 3, 144, 7, 4) == "none"
+
+
 def test_what_the_tiles_do_not_take():
     assert _sdpa(64, 256, 256, 8, 4)[1] == "tiles"
     assert _sdpa(64, 256, 256, 8, 4, q=PTR + 2)[1] == "rows"                       # off 16 bytes
