@@ -7,11 +7,7 @@ namespace {
 // Decode-sized M (<= 8): bandwidth- and latency-bound.  Every weight byte is read once with
 // 16-byte loads, a thread's loads are all issued before the first is used, and the activations
 // (a few KB) are staged in LDS.  Products go through v_dot2_f32_f16: fp16 pairs, fp32 sum.
-//
-// [K][F] weights: a thread owns 8 consecutive columns, 16 threads span 128 columns, the 16 thread
-// rows of a workgroup take interleaved k-pairs.  K is split over workgroups so that the whole chip
-// pulls on HBM; each split writes an fp32 partial plane and skinny_epilogue_kernel sums the planes
-// (the reference's split-K planes + mm_epilogue_kernel!, matmul.jl:192-217).
+
 // Layer-norm statistics of up to MT rows of A, one wave per row, in the summation order of
 // layernorm_vec_kernel (a lane takes the 16-byte chunks lane, lane + 64, ...; butterfly over the wave):
 // the fused result is bit-identical to running that kernel first.  stats[m] = (mean, rstd).
@@ -98,6 +94,10 @@ constexpr int SKN_COLS = 128;      // columns per workgroup
 constexpr int SKN_KMAX = 256;      // deepest k-slice: 16 loads of 16 bytes per thread, all in flight at once
 constexpr int SKN_LOADS = SKN_KMAX / 32;
 
+// [K][F] weights that kn_on_tiles leaves here (K from 1280, of one or two rows from 768, and very wide outputs): a thread owns 8
+// consecutive columns, 16 threads span 128 columns, the 16 thread rows of a workgroup take interleaved k-pairs.  K is split over
+// workgroups so that the whole chip pulls on HBM; each split writes an fp32 partial plane and skinny_epilogue_kernel sums the
+// planes (the reference's split-K planes + mm_epilogue_kernel!, matmul.jl:192-217).
 template <int MT>
 __global__ __launch_bounds__(256) void skinny_kn_kernel(GemmArgs p, float *part, int kper) {
     __shared__ __align__(16) half_t xs[MT][SKN_KMAX];
@@ -269,7 +269,6 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ float lnst[MT][2];
     const int kch = p.K >> 3;
-    const u32x4 z = {0u, 0u, 0u, 0u};
     // what the norm and the staging wait for goes first
     LnRow<PF <= 10 ? PF : 8> lnrow;
     if constexpr (LN) lnrow.request(p, min(wave, p.M - 1), lane);      // (MT is at most the workgroup's four waves)

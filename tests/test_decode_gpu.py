@@ -301,7 +301,8 @@ def test_fill_cross_writes_the_projections_head_major(ctx, B, S, H, E, layout):
 
 @pytest.mark.parametrize("Lk", [70, 700])
 def test_keys_too_far_apart_for_32_bit_offsets(ctx, Lk):
-    """A cache whose keys lie beyond 32-bit byte offsets: the same output and cache bits as the same cache laid out densely."""
+    """A cache whose keys lie beyond 32-bit byte offsets: the same cache bits as in a cache laid out
+    densely, the same output but for the order of its sums (such a cache is read in rounds of four passes)."""
     import torch
     import juliavision_amd as jv
     B, H, E = 1, 2, 16
