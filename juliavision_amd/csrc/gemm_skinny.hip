@@ -607,7 +607,12 @@ void launch_few(const GemmArgs &a, hipStream_t st) {
     hipLaunchKernelGGL((few_rows_kernel<PF, TURNS, LN, false>), dim3((unsigned)wgs), dim3(512), 0, st, a, cols);
 }
 
-// by the 32-deep steps that each of the eight waves takes: K <= 16 384, as the caller's bound on LDS says, behind a norm half of it
+// By the 32-deep steps that each of the eight waves takes: K <= 16 384, as the caller's bound on LDS says, behind a norm half of it.
+// Steps past a wave's share are asked for in vain, and registers decide the waves in flight, so a rung is its kernel.  us of eight rows
+// -> 1280, weights from memory, on its rung | on the next: K 512 2.75 | 2.98, 768 3.02 | 3.26, 1024 3.28 | 3.51, 1280 3.52 | 3.76, 1536 3.78 |
+// 4.38, 2048 4.42 | 4.90, 2560 4.92 | 5.56, 3072 5.58 | 6.72, 4096 6.96 | 7.79, 5120 7.94 | 9.20, 6144 9.28 | 11.4; behind a norm 512 3.72 |
+// 4.04, 768 4.42 | 4.64, 1024 4.73 | 5.29, 1280 5.77 | 6.15, 1536 6.32 | 7.18, 2048 7.68 | 8.46, 3072 9.15 | 11.0, 4096 11.7 | 13.2, 5120 17.1 | 17.6,
+// 6144 19.0 | 20.1 (ten steps at once for K up to 2560 there: 9.01, 8.95 in two rounds of six).
 int launch_few_k(const GemmArgs &a, hipStream_t st) {
     const int64_t per = ceil_div(ceil_div(a.K, 32), 8);
     if (per > (a.ln_on ? 32 : 64)) return MI_DECLINE_EXTENT;
@@ -618,7 +623,6 @@ int launch_few_k(const GemmArgs &a, hipStream_t st) {
         else if (per <= 5)  launch_few<5, 1, true>(a, st);
         else if (per <= 6)  launch_few<6, 1, true>(a, st);
         else if (per <= 8)  launch_few<8, 1, true>(a, st);
-        else if (per <= 10) launch_few<10, 1, true>(a, st);
         else if (per <= 12) launch_few<6, 2, true>(a, st);
         else if (per <= 16) launch_few<8, 2, true>(a, st);
         else if (per <= 20) launch_few<10, 2, true>(a, st);
@@ -679,6 +683,9 @@ int raise_fk() {
     return up(skinny_fk_kernel<MT, PF, 1, false>) | up(skinny_fk_kernel<MT, PF, 1, true>);
 }
 
+// By the 512-column chunks of a row.  us of one row -> 1280 | four rows behind a norm -> 5120, weights from memory, on its rung and on the
+// next: K 512 2.19, 2.32 | 4.61, 4.94; 1024 2.31, 2.40 | 5.48, 5.99; 1536 2.44, 3.10 | 7.4, 12.8; 3072 3.24, 3.38 | 17.2, 18.0; 4096 3.49,
+// 3.81 | 21.8, 22.8; 5120 4.93, 5.09 | 27.1, 35.2.
 template <int MT>
 void launch_fk_k(const GemmArgs &a, hipStream_t st) {
     if (a.K <= 512) launch_fk<MT, 1>(a, st);
