@@ -11,64 +11,76 @@ namespace {
 // Layer-norm statistics of up to MT rows of A, one wave per row, in the summation order of
 // layernorm_vec_kernel (a lane takes the 16-byte chunks lane, lane + 64, ...; butterfly over the wave):
 // the fused result is bit-identical to running that kernel first.  stats[m] = (mean, rstd).
-// In two halves, so that a caller can ask for more in between.  Rows up to NCH * 512 halves stay in registers between the passes; a
-// longer one is read twice.
+// In two halves, so that a caller can ask for more in between (LnRow).  Rows up to NCH * 512 halves stay in registers between the
+// passes; a longer one is read twice.  The two ways share no line but the last: where both led through one body, held and walked
+// rows were live over the choice and took skinny_kn_kernel<8> from 156 registers to 194, a third of its waves (8 rows of 8944 -> 7608
+// 41.6 -> 48.0 us, behind a norm 96 -> 129; 5 of 1464 -> 4248 11.1 -> 13.4).
+__device__ __forceinline__ void ln_stats_done(const GemmArgs &p, float (*stats)[2], int m, int lane, float mu, float s2) {
+    s2 = wave_sum(s2);
+    if (lane == 0) { stats[m][0] = mu; stats[m][1] = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps); }
+}
+__device__ __forceinline__ void ln_stats_walked(const GemmArgs &p, float (*stats)[2], int m, int lane) {
+    float s = 0.0f, s2 = 0.0f;
+    const half_t *row = p.A + (long)m * p.ldA;
+    for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
+        const half8v t = as_half8(ldg16(row + e0));
+#pragma unroll
+        for (int j = 0; j < 8; j++) s += (float)t[j];
+    }
+    s = wave_sum(s);
+    const float mu = s / (float)p.K;
+    for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
+        const half8v t = as_half8(ldg16(row + e0));
+#pragma unroll
+        for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
+    }
+    ln_stats_done(p, stats, m, lane, mu, s2);
+}
 template <int NCH>
 struct LnRow {
     u32x4 raw[NCH];
-    __device__ __forceinline__ void request(const GemmArgs &p, int m, int lane) {
-        if (p.K > NCH * 512) return;                        // uniform
+    __device__ __forceinline__ void load(const GemmArgs &p, int m, int lane) {
         const half_t *row = p.A + (long)m * p.ldA;
 #pragma unroll
         for (int i = 0; i < NCH; i++) raw[i] = ldg16(row + min((lane + 64 * i) * 8, p.K - 8));
     }
-    __device__ __forceinline__ void finish(const GemmArgs &p, float (*stats)[2], int m, int lane) {
-        float s = 0.0f, s2 = 0.0f, mu;
-        if (p.K <= NCH * 512) {
+    __device__ __forceinline__ void held(const GemmArgs &p, float (*stats)[2], int m, int lane) const {
+        float s = 0.0f, s2 = 0.0f;
 #pragma unroll
-            for (int i = 0; i < NCH; i++) {
-                if ((lane + 64 * i) * 8 < p.K) {
-                    const half8v t = as_half8(raw[i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) s += (float)t[j];
-                }
-            }
-            s = wave_sum(s);
-            mu = s / (float)p.K;
-#pragma unroll
-            for (int i = 0; i < NCH; i++) {
-                if ((lane + 64 * i) * 8 < p.K) {
-                    const half8v t = as_half8(raw[i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
-                }
-            }
-        } else {
-            const half_t *row = p.A + (long)m * p.ldA;
-            for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
-                const half8v t = as_half8(ldg16(row + e0));
+        for (int i = 0; i < NCH; i++) {
+            if ((lane + 64 * i) * 8 < p.K) {
+                const half8v t = as_half8(raw[i]);
 #pragma unroll
                 for (int j = 0; j < 8; j++) s += (float)t[j];
             }
-            s = wave_sum(s);
-            mu = s / (float)p.K;
-            for (int e0 = lane * 8; e0 < p.K; e0 += 512) {
-                const half8v t = as_half8(ldg16(row + e0));
+        }
+        s = wave_sum(s);
+        const float mu = s / (float)p.K;
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            if ((lane + 64 * i) * 8 < p.K) {
+                const half8v t = as_half8(raw[i]);
 #pragma unroll
                 for (int j = 0; j < 8; j++) { const float d = (float)t[j] - mu; s2 = fmaf(d, d, s2); }
             }
         }
-        s2 = wave_sum(s2);
-        if (lane == 0) { stats[m][0] = mu; stats[m][1] = 1.0f / sqrtf(s2 / (float)p.K + p.ln_eps); }
+        ln_stats_done(p, stats, m, lane, mu, s2);
+    }
+    __device__ __forceinline__ void request(const GemmArgs &p, int m, int lane) { if (p.K <= NCH * 512) load(p, m, lane); }      // uniform
+    __device__ __forceinline__ void finish(const GemmArgs &p, float (*stats)[2], int m, int lane) const {
+        if (p.K <= NCH * 512) held(p, stats, m, lane);
+        else ln_stats_walked(p, stats, m, lane);
     }
 };
 template <int MT, int NCH = 8, int NWAVES = 4>
 __device__ __forceinline__ void ln_row_stats(const GemmArgs &p, float (*stats)[2], int tid) {
     const int lane = tid & 63, wave = tid >> 6;
     for (int m = wave; m < MT && m < p.M; m += NWAVES) {
-        LnRow<NCH> row;
-        row.request(p, m, lane);
-        row.finish(p, stats, m, lane);
+        if (p.K <= NCH * 512) {
+            LnRow<NCH> row;
+            row.load(p, m, lane);
+            row.held(p, stats, m, lane);
+        } else ln_stats_walked(p, stats, m, lane);
     }
 }
 
