@@ -400,9 +400,15 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
 // re-read its last one: they reach sums that nobody stores).
 // WALK: past one workgroup a CU it goes on to the columns of gridDim.x workgroups further, whose weights it asks for under the current
 // ones' products; the activations stay in registers, normalised once.
+// Steps that a wave may not have, past the rung below in launch_few_k, stand behind uniform branches with nothing on their other side, which
+// nobody waits for (asked for in vain: 8 x 4232 -> 1083 6.95 us, 6.3 so).
+constexpr int few_steps_sure(int steps, bool LN) {
+    return steps == 8 ? 7 : steps == 10 ? 9 : steps == 12 ? (LN ? 9 : 11) : steps == 16 ? 13 : steps == 20 ? 17 : steps == 24 ? 21 : steps == 32 ? 25 : steps == 64 ? 33 : steps;
+}
 template <int PF, int TURNS, bool LN, bool WALK>
 __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
     static_assert(TURNS == 1 || !WALK, "activations in registers");
+    constexpr int SURE = few_steps_sure(PF * TURNS, LN);
     constexpr int NW = 8, NA = 5;
     __shared__ float4v red[WALK ? 2 : 1][NW][64];
     __shared__ float lnst[8][2];
@@ -415,10 +421,12 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
     struct Cols { u32x4 w[PF]; half_t bias, residual; };
     const int om = (tid >> 4) & 7, oc = tid & 15, omc = min(om, p.M - 1);      // outputs: one of each of the first 128 threads
     auto at = [&](int base, int i) { return min((base + i) * 32 + kq * 8, p.K - 8); };
-    auto fetch_w = [&](Cols &c, int n0, int base) {
+    auto fetch_w = [&](Cols &c, int n0, auto TURN) {
+        constexpr int turn = decltype(TURN)::value;
         const half_t *from = p.B + (long)min(n0 + wrow, p.N - 1) * p.ldB;
 #pragma unroll
-        for (int i = 0; i < PF; i++) c.w[i] = ldg16(from + at(base, i));
+        for (int i = 0; i < PF; i++)
+            if (turn * PF + i < SURE || turn * PF + i < per) c.w[i] = ldg16(from + at(s0 + turn * PF, i));
     };
     auto fetch_out = [&](Cols &c, int n0) {
         const int n = min(n0 + min(oc, cols - 1), p.N - 1);
@@ -428,9 +436,12 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
         c.residual = *r;
     };
     u32x4 x[PF], gm[LN ? PF : 1], be[LN ? PF : 1];
-    auto fetch_x = [&](int base) {
+    auto fetch_x = [&](auto TURN) {
+        constexpr int turn = decltype(TURN)::value;
+        const int base = s0 + turn * PF;
 #pragma unroll
         for (int i = 0; i < PF; i++) {
+            if (turn * PF + i >= SURE && turn * PF + i >= per) continue;
             x[i] = ldg16(xrow + at(base, i));
             if constexpr (LN) {
                 gm[i] = ldg16((p.ln_gamma ? p.ln_gamma : p.A) + at(base, i));
@@ -453,9 +464,10 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
     };
     LnRow<(PF * TURNS + 1) / 2 < 8 ? (PF * TURNS + 1) / 2 : 8> lnrow;      // 512 columns are two steps of eight waves
     if constexpr (LN) lnrow.request(p, min(wave, p.M - 1), lane);
-    fetch_x(s0);
+    using I0 = std::integral_constant<int, 0>;
+    fetch_x(I0{});
     Cols cur;
-    fetch_w(cur, nfirst, s0);
+    fetch_w(cur, nfirst, I0{});
     fetch_out(cur, nfirst);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (LN) {
@@ -488,16 +500,16 @@ __global__ __launch_bounds__(512) void few_rows_kernel(GemmArgs p, int cols) {
         const bool more = WALK && p.N - nc > stride;
         if constexpr (WALK) {
             const int nn = more ? nc + stride : p.N - 1;  // (past the end: the last row once more)
-            fetch_w(nxt, nn, s0);
+            fetch_w(nxt, nn, I0{});
             fetch_out(nxt, nn);
         }
 #pragma unroll
         for (int i = 0; i < NA; i++) acc[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-        products(cur, std::integral_constant<int, 0>{});
+        products(cur, I0{});
         auto turn = [&](auto TURN) {
             if constexpr (decltype(TURN)::value < TURNS) {
-                fetch_x(s0 + decltype(TURN)::value * PF);
-                fetch_w(cur, nc, s0 + decltype(TURN)::value * PF);
+                fetch_x(TURN);
+                fetch_w(cur, nc, TURN);
                 normalise();
                 products(cur, TURN);
             }
@@ -620,8 +632,8 @@ void launch_few(const GemmArgs &a, hipStream_t st) {
 }
 
 // By the 32-deep steps that each of the eight waves takes: K <= 16 384, as the caller's bound on LDS says, behind a norm half of it.
-// Steps past a wave's share are asked for in vain, and registers decide the waves in flight, so a rung is its kernel.  us of eight rows
-// -> 1280, weights from memory, on its rung | on the next: K 512 2.75 | 2.98, 768 3.02 | 3.26, 1024 3.28 | 3.51, 1280 3.52 | 3.76, 1536 3.78 |
+// Steps past a wave's share cost the loads' issue, and registers decide the waves in flight, so a rung is its kernel (few_steps_sure: what
+// lies between two).  us of eight rows -> 1280, weights from memory, on its rung | with all steps of the next asked for: K 512 2.75 | 2.98, 768 3.02 | 3.26, 1024 3.28 | 3.51, 1280 3.52 | 3.76, 1536 3.78 |
 // 4.38, 2048 4.42 | 4.90, 2560 4.92 | 5.56, 3072 5.58 | 6.72, 4096 6.96 | 7.79, 5120 7.94 | 9.20, 6144 9.28 | 11.4; behind a norm 512 3.72 |
 // 4.04, 768 4.42 | 4.64, 1024 4.73 | 5.29, 1280 5.77 | 6.15, 1536 6.32 | 7.18, 2048 7.68 | 8.46, 3072 9.15 | 11.0, 4096 11.7 | 13.2, 5120 17.1 | 17.6,
 // 6144 19.0 | 20.1 (ten steps at once for K up to 2560 there: 9.01, 8.95 in two rounds of six).
