@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     half_t *xs = reinterpret_cast<half_t *>(smem);       // [MT][K]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ float lnst[MT][2];
-    const int kch = p.K >> 3;
+    const int kch = p.K >> 3, staged = p.M * kch;         // (rows past M are not: their sums go nowhere)
     // what the norm and the staging wait for goes first
     LnRow<PF <= 10 ? PF : 8> lnrow;
     if constexpr (LN) lnrow.request(p, min(wave, p.M - 1), lane);      // (MT is at most the workgroup's four waves)
@@ -309,26 +309,25 @@ __global__ __launch_bounds__(256) void skinny_fk_kernel(GemmArgs p) {
     for (int i = 0; i < XPF; i++) {
         unsigned ch;
         const int c = tid + 256 * i, m = (int)divide(c, kch, p.div_k8, ch);
-        if (c < MT * kch) {
+        if (c < staged) {
             u32x4 v = xr[i];
             if constexpr (LN) {
-                const int ms = min(m, p.M - 1);
                 const half8v x = as_half8(v), gv = as_half8(gr[i]), bb = as_half8(br[i]);
                 half8v o;
 #pragma unroll
                 for (int j = 0; j < 8; j++)
-                    o[j] = ln_norm1((float)x[j], lnst[ms][0], lnst[ms][1], p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bb[j]);
+                    o[j] = ln_norm1((float)x[j], lnst[m][0], lnst[m][1], p.ln_gamma != nullptr, (float)gv[j], p.ln_beta != nullptr, (float)bb[j]);
                 v = __builtin_bit_cast(u32x4, o);
             }
-            *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;      // (rows past M repeat the last one; their sums go nowhere)
+            *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;
         }
     }
-    for (int c = tid + 256 * XPF; c < MT * kch; c += 256) {
+    for (int c = tid + 256 * XPF; c < staged; c += 256) {
         unsigned ch;
-        const int m = min((int)divide(c, kch, p.div_k8, ch), p.M - 1);
+        const int m = (int)divide(c, kch, p.div_k8, ch);
         u32x4 v = ldg16(p.A + (long)m * p.ldA + ch * 8);
         if constexpr (LN) v = ln_apply8(p, v, lnst[m][0], lnst[m][1], ch * 8);
-        *reinterpret_cast<u32x4 *>(xs + (long)(c / kch) * p.K + ch * 8) = v;
+        *reinterpret_cast<u32x4 *>(xs + (long)m * p.K + ch * 8) = v;
     }
     __syncthreads();
     // A wave walks its columns n .. n + R - 1, then those 4 R gridDim.x further on: once for the widths of a decoder layer
