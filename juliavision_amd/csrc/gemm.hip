@@ -234,6 +234,7 @@ __global__ __launch_bounds__(512) void gemm_w4_kernel(GemmArgs p) {
                                   [](auto) {}, barrier);
     };
     if (wave == 4) {
+        nothing_pending();
         // Per-lane offsets of the tile's 1 KB slots.  A tile that lies inside the operands needs no clamping, and its
         // slots s and s + 2 differ by a constant (eight rows of a K-contiguous operand, 64 / (BN / 8) k-rows of the
         // [K][N] one; the chunk permutation has period two in s): two offsets computed in full, the others one add

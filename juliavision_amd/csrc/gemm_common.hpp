@@ -81,6 +81,11 @@ __device__ __forceinline__ void static_for(F &&f) {
     }
 }
 
+// At the entry of a loader wave, which has asked for nothing.  The branches that part the waves meet again in the compiled code, so that there
+// the compiler takes the matrix waves' loads for pending and waits for each where it next writes that register; between direct-to-LDS
+// requests, which it does not see, such a wait is one for their data, before the next are asked for.  Here it waits for nothing.
+__device__ __forceinline__ void nothing_pending() { __builtin_amdgcn_s_waitcnt(0x0f70); }      // vmcnt(0)
+
 // Kernel arguments come through the scalar cache a 64-byte line at a time: 200 clocks a line in a replayed graph, 550 to 700 where
 // the host has just written them, and the compiler asks for a field where it is first used, so that four or five such trips
 // stood in a row between a launch and its first load.  Naming the fields at the kernel's first line requests them together.

@@ -56,6 +56,7 @@ __global__ __launch_bounds__((NW + 3) * 64, 2) void gemm_deep_kernel(GemmArgs p)
     };
 
     if (__builtin_expect(wave >= NW, 1)) {
+        nothing_pending();
         auto load_all = [&](auto IS_A_) __attribute__((always_inline)) {
             constexpr bool IS_A = decltype(IS_A_)::value, ROWS = IS_A || !B_KN, PATCH = CONV && !IS_A;
             // 1 KB requests of a stage, a run of RUN in a row sharing an LDS address.  PATCH: 2 half + {0, 1, 4, 5}
