@@ -868,11 +868,18 @@ TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool may_sp
 // tiles' time).  Without one the 128 x 128 tiles are as good as estimated at K = 128 and 192 (35 calls that 9 % moved were 1 to 9 % slower:
 // 4525 x 192 -> 1688 9.7 -> 10.5 us, 1808 x 128 -> 3952 9.3 -> 9.95), the 64 x 128 ones lower (24 calls 0.82 to 0.95).  From K = 1024 on
 // only the 128 x 128 tiles of at most one workgroup a CU are (0.85 to 1.0, one in ten 1.02 to 1.08; with residual 0.81 to 1.0): the others
-// are taken where those pass 256 or 512 by a few (1571 x 1024 -> 2544 15.0 -> 16.0, 3379 x 2048 -> 2360 44 -> 49, with residual 47 -> 52).
+// are taken where those pass 256 or 512 by a few (1571 x 1024 -> 2544 15.0 -> 16.0, 3379 x 2048 -> 2360 44 -> 49, with residual 47 -> 52).  The
+// 64 x 128 ones are not from K = 768 on without a residual (1181 x 896 -> 3264 12.7 -> 14.0, 4665 x 896 -> 784 13.1 -> 14.4).
+//
+// What the residual costs the four-wave kernel: 2 us, and 0.6 where it has at most one workgroup a CU and K >= 256, whose tiles
+// are not estimated as much too high (24 such calls, both layouts: 0.97 of the time with 2 us; 6263 x 384 -> 952 15.2 -> 13.6 us,
+// 4942 x 512 -> 1032 14.95 -> 13.4.  60 of more workgroups lose 1 % with 1 us; K = 128 and 192 keep the gain at one workgroup a CU: 3470 x 192
+// -> 1600 10.0 -> 8.65).  With [K][F] weights the same factors hold: 200 calls are 0.4 % above the faster side, 11 % at worst.
 double estimated_high(int tile, const GemmArgs &a, int64_t wgs) {
     const bool residual = a.residual != nullptr;
     if (tile <= 1) return 1.0;
     if (a.K >= 1024) return tile == 2 && wgs <= mi_num_cus() ? (residual ? 0.91 : 0.93) : 1.0;
+    if (tile == 3 && a.K >= 768 && !residual) return 1.0;
     return residual || a.K >= 256 ? 0.91 : tile == 2 ? 0.97 : 0.92;
 }
 int settled_tile(int tile, const GemmArgs &a, int64_t nbatch) {
@@ -881,7 +888,7 @@ int settled_tile(int tile, const GemmArgs &a, int64_t nbatch) {
     for (int t = 0; t < 4; t++) {
         const int64_t wgs = ceil_div(a.M, TILE_MODELS[t].bm) * ceil_div(a.N, TILE_MODELS[t].bn) * nbatch;
         if (t > 1 && a.K >= 1024 && wgs > 2 * mi_num_cus()) continue;      // (nor does a residual make up for theirs)
-        const double us = tile_cost_us(a.M, a.N, a.K, nbatch, t, 1) * estimated_high(t, a, wgs) + (t <= 1 && a.residual ? 2.0 : 0.0);
+        const double us = tile_cost_us(a.M, a.N, a.K, nbatch, t, 1) * estimated_high(t, a, wgs) + (t <= 1 && a.residual ? (a.K >= 256 && wgs <= mi_num_cus() ? 0.6 : 2.0) : 0.0);
         if (us < best) { best = us; tile = t; }
     }
     return tile;
