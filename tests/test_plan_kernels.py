@@ -56,6 +56,12 @@ def test_which_kernel_a_gemm_runs():
             assert (plain in own) == (gelu in own) and (plain not in own or plain == gelu), (T, K, F)
 
 
+@pytest.mark.parametrize("T,K,F,runs", [(1181, 896, 3264, "wide"), (4665, 896, 784, "wide"), (4665, 640, 784, "staged"), (2518, 192, 3552, "staged")])
+def test_narrow_tiles_end_at_k_768(T, K, F, runs):
+    """Two workgroups a CU of 64 x 128 tiles, whose estimate is lowered up to there."""
+    assert L.GEMM_KERNELS[L.load().mi_gemm_f16_kernel(T, K, F, 1, L.EPI["none"], 0, None)] == runs
+
+
 def test_how_rows_against_kf_weights_are_cut():
     """One slice of K where they run as 32 x 32 tiles, which ask for row pitches below 2^31 bytes a tile."""
     slices = C.c_int(0)
